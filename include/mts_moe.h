@@ -387,6 +387,48 @@ int mts_moe_bwd_joint_router(const void* d_out, const void* weighted_act, const 
                              float* d_w_r, void* router_workspace, int64_t router_workspace_bytes,
                              const int32_t* schedule, void* stream);
 
+/* ---- dense operators of the host decoder -----------------------------------
+ * They stand in for the stock operators of the reference's PyTorch backend
+ * (minitrain/kernels/torch_ops.py): RMSNorm, rotary encoding and cross-entropy.
+ *
+ * RMSNorm of sum = x + residual (residual may be NULL: of x itself, `sum` unused), fp32
+ * arithmetic, weight [H] f32; rstd [N] f32 is kept for the backward pass.
+ * mts_rmsnorm_bwd: g_y and g_sum (may be NULL) are the gradients of y and of the sum;
+ * d_sum = g_sum + the norm's share, one rounding; d_weight [H] f32, summed in a fixed order.
+ * Rows: H a multiple of 4, at most 4096 (mts_rmsnorm_supported).                         */
+int mts_rmsnorm_supported(int H);
+int mts_rmsnorm_fwd(const void* x, const void* residual, const float* weight, int64_t N, int H,
+                    float eps, int act_dtype, void* sum, void* y, float* rstd, void* stream);
+int64_t mts_rmsnorm_bwd_workspace_bytes(int64_t N, int H);
+int mts_rmsnorm_bwd(const void* g_y, const void* g_sum, const void* sum, const float* weight,
+                    const float* rstd, int64_t N, int H, int act_dtype, void* d_sum,
+                    float* d_weight, void* workspace, int64_t workspace_bytes, void* stream);
+
+/* Rotary encoding of up to three tensors [B,S,heads,head_dim] in one launch, each with its own
+ * strides in elements (the last dimension is dense).  mode 0: t * cos + rot(t) * sin, each
+ * product rounded to act_dtype; mode 1: the transpose of that map (its gradient); mode 2: copy.
+ * cos and sin are [S, head_dim] in act_dtype.  `tensors` is a host array.                */
+typedef struct {
+    const void* in;
+    void* out;
+    int64_t in_b, in_s, in_h, out_b, out_s, out_h;
+    int mode;
+} MtsRopeTensor;
+int mts_rope(const MtsRopeTensor* tensors, int count, const void* cos, const void* sin, int64_t B,
+             int64_t S, int heads, int head_dim, int act_dtype, void* stream);
+
+/* Mean cross-entropy of logits [N,V] (any of the three types, fp32 arithmetic) over the rows
+ * whose target is not ignore_index.  row_max, row_log_sum [N] and inv_count [1] f32 are kept for
+ * the backward pass (row_loss [N] is scratch): d_logits = (softmax - onehot) * g_loss * inv_count in the logits' type.
+ * A target outside [0, V) makes the loss NaN.                                              */
+int mts_cross_entropy_fwd(const void* logits, const int64_t* targets, int64_t N, int V,
+                          int64_t ignore_index, int dtype, float* row_max, float* row_log_sum,
+                          float* row_loss, float* loss, float* inv_count, void* stream);
+int mts_cross_entropy_bwd(const void* logits, const int64_t* targets, int64_t N, int V,
+                          int64_t ignore_index, int dtype, const float* row_max,
+                          const float* row_log_sum, const float* g_loss, const float* inv_count,
+                          void* d_logits, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -69,7 +69,21 @@ SIGNATURES = {
     "mts_moe_bwd_joint_router_supported": (_i, [_i, _l, _i, _i, _i]),
     "mts_moe_bwd_joint_router": (_i, [_p, _p, _p, _p, _p, _p, _p, _p, _p, _l, _i, _i, _i, _i, _i, _i, _p, _p, _p, _p, _p, _l, _p, _l]
                                  + [_p] * 8 + [_i, _p, _p, _p, _p, _l, _p, _p]),
+    "mts_rmsnorm_supported": (_i, [_i]),
+    "mts_rmsnorm_fwd": (_i, [_p, _p, _p, _l, _i, _c.c_float, _i, _p, _p, _p, _p]),
+    "mts_rmsnorm_bwd_workspace_bytes": (_l, [_l, _i]),
+    "mts_rmsnorm_bwd": (_i, [_p, _p, _p, _p, _p, _l, _i, _i, _p, _p, _p, _l, _p]),
+    "mts_rope": (_i, [_p, _i, _p, _p, _l, _l, _i, _i, _i, _p]),
+    "mts_cross_entropy_fwd": (_i, [_p, _p, _l, _i, _l, _i, _p, _p, _p, _p, _p, _p]),
+    "mts_cross_entropy_bwd": (_i, [_p, _p, _l, _i, _l, _i, _p, _p, _p, _p, _p, _p]),
 }
+
+
+class RopeTensor(_c.Structure):
+    """``MtsRopeTensor``"""
+
+    _fields_ = [("input", _p), ("output", _p), ("in_b", _l), ("in_s", _l), ("in_h", _l), ("out_b", _l), ("out_s", _l), ("out_h", _l), ("mode", _i)]
+
 
 _lib = None
 _lock = threading.Lock()

@@ -5,7 +5,10 @@ Counterpart of the reference's ``TritonOpsBackend``
 that class there is no fallback: an unsupported tensor contract raises.
 """
 
+import torch.nn.functional as F
+
 from minitrain_amd.kernels.dense_ops import DenseTorchOps
+from minitrain_amd.kernels.hip import dense
 from minitrain_amd.kernels.hip.capacity import capacity_mask, is_capacity_mask_supported
 from minitrain_amd.kernels.hip.fused_moe import expert_counts, fused_moe, is_fused_moe_supported
 from minitrain_amd.kernels.hip.moe_layer import moe_layer, moe_layer_violation
@@ -32,6 +35,41 @@ class HipOpsBackend(DenseTorchOps):
 
     def fused_moe(self, x, gate_up_proj, down_proj, top_k_index, top_k_weights):
         return fused_moe(x, gate_up_proj, down_proj, top_k_index, top_k_weights)
+
+    # The decoder's operators around its matrix products: one kernel where the stock operators are a chain of
+    # elementwise and reduction kernels; what the kernels do not take (CPU tensors, other types and layouts) stays stock.
+
+    def rmsnorm(self, x, weight, eps):
+        if dense.is_rmsnorm_supported(x, weight):
+            return dense.rmsnorm(x, weight, eps)
+        return super().rmsnorm(x, weight, eps)
+
+    def add_rmsnorm(self, x, residual, weight, eps):
+        """Extension: ``(x + residual, rmsnorm(x + residual))`` in one pass."""
+        if dense.is_rmsnorm_supported(x, weight, residual):
+            return dense.add_rmsnorm(x, residual, weight, eps)
+        total = x + residual
+        return total, super().rmsnorm(total, weight, eps)
+
+    def rope(self, q, k, cos, sin):
+        if dense.is_rope_supported(q, k, cos, sin):
+            return dense.rope(q, k, cos, sin)
+        return super().rope(q, k, cos, sin)
+
+    def qkv_rope(self, qkv, cos, sin, heads):
+        """Extension: rotated queries and keys and the values ``[B, heads, S, D]`` of a packed projection, or None when
+        the kernel does not take it (the caller then splits the projection and calls ``rope``)."""
+        if not dense.is_qkv_rope_supported(qkv, cos, sin, heads):
+            return None
+        return dense.qkv_rope(qkv, cos, sin, heads)
+
+    def cross_entropy(self, logits, targets):
+        if dense.is_cross_entropy_supported(logits, targets):
+            return dense.cross_entropy(logits, targets)
+        return super().cross_entropy(logits, targets)
+
+    def fused_linear_cross_entropy(self, x, weight, targets):
+        return self.cross_entropy(F.linear(x, weight), targets)
 
     def expert_counts(self, expert_indices, num_experts):
         """Extension: routes per expert (int32 ``[E]``) without a host synchronisation."""

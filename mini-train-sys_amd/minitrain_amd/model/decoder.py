@@ -50,6 +50,20 @@ class RMSNorm(nn.Module):
         return ops.rmsnorm(x, self.weight, self.eps)
 
 
+def is_observed(module: nn.Module) -> bool:
+    """Whether hooks are registered that want the module's own inputs and outputs."""
+    return bool(module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks)
+
+
+def sum_and_norm(norm: RMSNorm, x: torch.Tensor, residual: torch.Tensor | None, ops: OpsBackend):
+    """``(x + residual, norm of it)``, in one pass where the backend offers it; ``residual`` None: of ``x`` itself."""
+    fused = getattr(ops, "add_rmsnorm", None)
+    if residual is not None and fused is not None and not is_observed(norm):
+        return fused(x, residual, norm.weight, norm.eps)
+    x = x if residual is None else x + residual
+    return x, norm(x, ops)
+
+
 class CausalSelfAttention(nn.Module):
     def __init__(self, cfg: ModelConfig) -> None:
         super().__init__()
@@ -62,8 +76,14 @@ class CausalSelfAttention(nn.Module):
 
     def forward(self, x, ops: OpsBackend, rope_cos, rope_sin):
         B, S, H = x.shape
-        q, k, v = (t.view(B, S, self.n_heads, self.head_dim).transpose(1, 2) for t in self.qkv(x).chunk(3, dim=-1))
-        q, k = ops.rope(q, k, rope_cos, rope_sin)
+        qkv = self.qkv(x)
+        packed = getattr(ops, "qkv_rope", None)   # a backend may take the packed projection as it is
+        turned = packed(qkv, rope_cos, rope_sin, self.n_heads) if packed is not None else None
+        if turned is not None:
+            q, k, v = turned
+        else:
+            q, k, v = (t.view(B, S, self.n_heads, self.head_dim).transpose(1, 2) for t in qkv.chunk(3, dim=-1))
+            q, k = ops.rope(q, k, rope_cos, rope_sin)
         ctx = ops.attention(q, k, v, is_causal=True, dropout_p=self.p_drop if self.training else 0.0)
         return self.resid_dropout(self.out(ctx.transpose(1, 2).reshape(B, S, H)))
 
@@ -79,9 +99,15 @@ class TransformerBlock(nn.Module):
         self.ffn = MoEFeedForward(cfg)
 
     def forward(self, x, ops: OpsBackend, rope_cos, rope_sin):
-        x = x + self.attn(self.attn_norm(x, ops), ops, rope_cos, rope_sin)
-        ffn = self.ffn(self.ffn_norm(x, ops), ops)
+        x, ffn = self.residual_forward(x, None, ops, rope_cos, rope_sin)
         return x + ffn.hidden_states, ffn
+
+    def residual_forward(self, x, pending, ops: OpsBackend, rope_cos, rope_sin):
+        """The block without its last sum: ``x`` before it and the feed-forward output, which the norm that follows adds
+        in its own pass; ``pending`` is that output of the block in front (None: ``x`` is complete)."""
+        x, normed = sum_and_norm(self.attn_norm, x, pending, ops)
+        x, normed = sum_and_norm(self.ffn_norm, x, self.attn(normed, ops, rope_cos, rope_sin), ops)
+        return x, self.ffn(normed, ops)
 
 
 class MiniTransformer(nn.Module):
@@ -113,8 +139,14 @@ class MiniTransformer(nn.Module):
         if cos.device != hidden.device or cos.dtype != hidden.dtype:
             raise RuntimeError("RoPE cache must match the residual device and dtype")
         aux, z, per_layer = [], [], {}
+        pending = None
         for block in self.blocks:
-            hidden, ffn = block(hidden, self.ops, cos, sin)
+            if is_observed(block):
+                hidden, ffn = block(hidden if pending is None else hidden + pending, self.ops, cos, sin)
+                pending = None
+            else:
+                hidden, ffn = block.residual_forward(hidden, pending, self.ops, cos, sin)
+                pending = ffn.hidden_states
             aux.append(ffn.router_aux_loss)
             z.append(ffn.router_z_loss)
             for name, value in ffn.router_metrics.items():
@@ -132,7 +164,7 @@ class MiniTransformer(nn.Module):
         metrics["moe/aux_loss"] = self._router_aux.detach()
         metrics["moe/z_loss"] = self._router_z.detach()
         self.last_training_metrics = metrics
-        return self.norm(hidden, self.ops)
+        return sum_and_norm(self.norm, hidden, pending, self.ops)[1]
 
     def forward(self, input_ids: torch.Tensor, targets: torch.Tensor | None = None, use_fused_loss: bool = False):
         hidden = self.hidden_states(input_ids)
