@@ -273,12 +273,14 @@ int mts_moe_combine(const void* y, const void* weights, const void* addend, cons
  * [E,H,I] in the activation dtype, or w2_as_stored = 0, it is the transposed copy [E,I,H]
  * made by mts_moe_stage_weights.  mts_moe_bwd_weights_as_stored(act_dtype, H, I) says
  * whether this entry point and mts_moe_bwd_dx take the stored layout (bf16, H and 2I
- * multiples of 64); otherwise they return MTS_ERR_SHAPE for it.  ds_partial is
+ * multiples of 64); otherwise they return MTS_ERR_SHAPE for it.  fp32 activations take the
+ * stored layout at any widths, asked for as MTS_STORED_F32.  ds_partial is
  * [TK, mts_moe_ds_partials(I)] f32 scratch reduced by mts_moe_bwd_ds (fixed order, no
  * atomics).  weighted_act may be NULL: it is then not written (the caller holds s*a already,
  * see mts_moe_fwd_gateup_swiglu).  schedule may be NULL; otherwise (16-bit activations,
  * mts_moe_bwd_schedule_bytes(E) > 0 bytes, 16-byte aligned) one more block of the launch
  * writes the schedule of mts_moe_bwd_joint there, see mts_moe_bwd_schedule.            */
+#define MTS_STORED_F32 2
 int mts_moe_ds_partials(int I);
 int mts_moe_bwd_weights_as_stored(int act_dtype, int H, int I);
 int mts_moe_bwd_dy1(const void* d_out, const void* w2, int w2_as_stored, const void* pre_act,

@@ -84,8 +84,16 @@ __global__ __launch_bounds__(kThreads) void ds_reduce_kernel(const float* __rest
         const int32_t r = s_rev[n];   // negative: dropped route, no gradient
         float v = 0.f;
         if (r >= 0) {
+            // one add after the other (a fixed order), but 16 loads in flight at a time
             const float* p = part + (int64_t)r * np;
-            for (int j = 0; j < np; ++j) v += p[j];
+            for (int j0 = 0; j0 < np; j0 += 16) {
+                float t[16];
+#pragma unroll
+                for (int j = 0; j < 16; ++j) t[j] = j0 + j < np ? p[j0 + j] : 0.f;
+#pragma unroll
+                for (int j = 0; j < 16; ++j)
+                    if (j0 + j < np) v += t[j];
+            }
         }
         d_w[n] = (OutT)v;
     }

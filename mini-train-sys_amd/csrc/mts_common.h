@@ -83,7 +83,7 @@ int mts_moe_bwd_joint_router_f16(const void* d_out, const void* weighted_act, co
 }
 
 // fp32 GEMM launchers (mts_gemm_f32.hip); epi: 0 plain, 1 SwiGLU, 2 dO*W2 with SwiGLU backward
-int mts_f32_rows(int epi, const float* A, int lda, const int32_t* a_gather, const float* B, int b_rows,
+int mts_f32_rows(int epi, const float* A, int lda, const int32_t* a_gather, const float* B, int b_rows, int b_kmajor,
                  int N, int Kdim, const int32_t* expert_start, int E, int64_t TK, float* C, float* C2,
                  const float* pre_act, const float* route_w, const int32_t* s_scatter, float* ds_part,
                  int np, hipStream_t s);

@@ -2549,7 +2549,7 @@ extern "C" int MTS_GEMM_ENTRY(mts_moe_fwd_gateup_swiglu)(const void* x, const vo
     if (T <= 0 || K < 1) return MTS_ERR_SHAPE;
     if (act_dtype == MTS_F32) {
         if (E < 1 || E > MTS_MAX_MOE_EXPERTS || H < 1 || I < 1 || T * K > 0x7fffffffLL) return MTS_ERR_SHAPE;
-        return mts_f32_rows(1, (const float*)x, H, x_gather, (const float*)w1, 2 * I, I, H, expert_start, E, T * K,
+        return mts_f32_rows(1, (const float*)x, H, x_gather, (const float*)w1, 2 * I, 0, I, H, expert_start, E, T * K,
                             (float*)pre_act, (float*)post_act, nullptr, (const float*)weights, s_scatter, nullptr, 0,
                             (hipStream_t)stream);
     }
@@ -2575,7 +2575,7 @@ extern "C" int MTS_GEMM_ENTRY(mts_moe_fwd_down)(const void* post_act, const void
     if (!post_act || !w2 || !expert_start || !y) return MTS_ERR_NULL;
     if (act_dtype == MTS_F32) {
         if (TK <= 0 || TK > 0x7fffffffLL || E < 1 || E > MTS_MAX_MOE_EXPERTS || H < 1 || I < 1) return MTS_ERR_SHAPE;
-        return mts_f32_rows(0, (const float*)post_act, I, nullptr, (const float*)w2, H, H, I, expert_start, E, TK,
+        return mts_f32_rows(0, (const float*)post_act, I, nullptr, (const float*)w2, H, 0, H, I, expert_start, E, TK,
                             (float*)y, nullptr, nullptr, nullptr, nullptr, nullptr, 0, (hipStream_t)stream);
     }
     if (act_dtype != MTS_GEMM_DTYPE) return MTS_ERR_DTYPE;
@@ -2652,8 +2652,9 @@ extern "C" int MTS_GEMM_ENTRY(mts_moe_bwd_dy1)(const void* d_out, const void* w2
     if (T <= 0 || K < 1) return MTS_ERR_SHAPE;
     if (schedule && (E > kSchedMaxExperts || act_dtype == MTS_F32)) return MTS_ERR_SHAPE;   // see mts_moe_bwd_schedule_bytes
     if (act_dtype == MTS_F32) {
-        if (E < 1 || E > MTS_MAX_MOE_EXPERTS || H < 1 || I < 1 || T * K > 0x7fffffffLL || w2_as_stored) return MTS_ERR_SHAPE;
-        return mts_f32_rows(2, (const float*)d_out, H, x_gather, (const float*)w2t, I, I, H, expert_start, E, T * K,
+        if (E < 1 || E > MTS_MAX_MOE_EXPERTS || H < 1 || I < 1 || T * K > 0x7fffffffLL || (w2_as_stored && w2_as_stored != MTS_STORED_F32))
+            return MTS_ERR_SHAPE;
+        return mts_f32_rows(2, (const float*)d_out, H, x_gather, (const float*)w2t, I, w2_as_stored != 0, I, H, expert_start, E, T * K,
                             (float*)d_pre_act, (float*)weighted_act, (const float*)pre_act, (const float*)weights,
                             s_scatter, ds_partial, mts_moe_ds_partials(I), (hipStream_t)stream);
     }
@@ -2687,9 +2688,10 @@ extern "C" int MTS_GEMM_ENTRY(mts_moe_bwd_dx)(const void* d_pre_act, const void*
 #endif
     if (!d_pre_act || !w1t || !expert_start || !dx_expanded) return MTS_ERR_NULL;
     if (act_dtype == MTS_F32) {
-        if (TK <= 0 || TK > 0x7fffffffLL || E < 1 || E > MTS_MAX_MOE_EXPERTS || H < 1 || I < 1 || w1_as_stored) return MTS_ERR_SHAPE;
-        return mts_f32_rows(0, (const float*)d_pre_act, 2 * I, nullptr, (const float*)w1t, H, H, 2 * I, expert_start, E,
-                            TK, (float*)dx_expanded, nullptr, nullptr, nullptr, nullptr, nullptr, 0,
+        if (TK <= 0 || TK > 0x7fffffffLL || E < 1 || E > MTS_MAX_MOE_EXPERTS || H < 1 || I < 1 || (w1_as_stored && w1_as_stored != MTS_STORED_F32))
+            return MTS_ERR_SHAPE;
+        return mts_f32_rows(0, (const float*)d_pre_act, 2 * I, nullptr, (const float*)w1t, H, w1_as_stored != 0, H, 2 * I,
+                            expert_start, E, TK, (float*)dx_expanded, nullptr, nullptr, nullptr, nullptr, nullptr, 0,
                             (hipStream_t)stream);
     }
     if (act_dtype != MTS_GEMM_DTYPE) return MTS_ERR_DTYPE;

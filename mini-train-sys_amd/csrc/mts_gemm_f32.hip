@@ -1,17 +1,27 @@
-// fp32 variant of the grouped expert GEMMs (activations, weights and accumulation
-// all in fp32, plain FMA): the small debug configuration of the layer and fp32
-// parity checks run through it.  Same contracts and epilogues as the bf16 MFMA
-// kernels; throughput is not a goal here.
+// fp32 variant of the grouped expert GEMMs: activations, weights and accumulation all in fp32, on the fp32 matrix
+// instruction (v_mfma_f32_32x32x2_f32, full fp32 products and sums).  Same contracts and epilogues as the 16-bit kernels.
 //
-// 64x64 output tile per 256-thread block, 16-wide k-steps through LDS, 4x4 outputs
-// per thread.  Row tiles follow the expert segments exactly as in the bf16 path.
+// What bounds it: the instruction's rate, 157 TFLOP/s on the card (64 cycles for 4096 FLOP), a sixteenth of the bf16 rate,
+// so nothing here needs direct-to-LDS loads or specialised waves: tiles of 64 x 64 outputs per block of four waves, 16 of k
+// at a time through two LDS buffers, two more k-tiles in flight in registers, and up to eight blocks per CU.  A tile reads
+// one byte of L2 per 16 FLOP; tiles of 128 rows are no faster at 16 000 rows (101 TFLOP/s over all GEMMs either way) and
+// 12 % slower at 4096, where they leave the CUs unevenly filled.  2048 tokens, 768/1024, 8 experts, top-2: forward and
+// backward of the operator 1776 -> 727 us, 80 TFLOP/s (plain FMA from 64x64 tiles before: 33 TFLOP/s).
+//
+// The k index an operand register stands for is free as long as both operands agree: lanes 0..31 hold k = 8s+0..3 and lanes
+// 32..63 k = 8s+4..7 of four consecutive instructions, so an operand whose rows are k-contiguous is read as one 16-byte
+// LDS load per four instructions, and one whose memory rows are k ("k-major": stored weights in the backward pass, both
+// operands of the weight gradients) as four 4-byte loads, with no transposed copy of anything.
 #include "mts_common.h"
+
+#include <type_traits>
 
 namespace {
 
-constexpr int TB = 64;   // tile rows and columns
-constexpr int TKS = 16;  // k-step
+constexpr int TKS = 16;  // k extent of an LDS tile
+constexpr int BM = 64;   // rows of a tile, and of P columns in the weight gradients
 constexpr int kThreads = 256;
+constexpr int kXcds = 8;
 
 enum Epi32 { E32_PLAIN = 0, E32_SWIGLU = 1, E32_DY1 = 2 };
 
@@ -19,7 +29,7 @@ struct Rows32 {
     const float* A;
     int lda;
     const int32_t* a_gather;
-    const float* B;      // [E][b_rows][Kdim]
+    const float* B;      // [E][b_rows][Kdim], or k-major: [E][Kdim][N]
     int b_rows;
     int N, Kdim;
     const int32_t* expert_start;
@@ -31,123 +41,265 @@ struct Rows32 {
     const int32_t* s_scatter;
     float* ds_part;
     int np;
+    int n_tiles;
 };
 
 __device__ __forceinline__ float sigmoid32(float x) { return 1.0f / (1.0f + expf(-x)); }
 
-template <int EPI>
-__global__ __launch_bounds__(kThreads) void rows_gemm_f32_kernel(Rows32 p) {
-    constexpr int NB = (EPI == E32_SWIGLU) ? 2 : 1;  // B tiles per block (gate and up)
-    __shared__ float As[TKS][TB + 4];
-    __shared__ float Bs[NB][TKS][TB + 4];
-
-    int e = 0, row0 = 0, rend = 0;
-    {
-        int tile = blockIdx.x, seen = 0;
-        bool found = false;
-        for (e = 0; e < p.E; ++e) {
-            const int s0 = p.expert_start[e], s1 = p.expert_start[e + 1];
-            const int nt = (s1 - s0 + TB - 1) / TB;
-            if (tile < seen + nt) {
-                row0 = s0 + (tile - seen) * TB;
-                rend = s1;
-                found = true;
-                break;
-            }
-            seen += nt;
-        }
-        if (!found) return;
+// four consecutive floats at p, of which the first `count` exist (VEC: p is 16-byte aligned and count is 0 or >= 4)
+template <bool VEC>
+__device__ __forceinline__ f32x4 load4(const float* p, int count) {
+    f32x4 v = {};
+    if constexpr (VEC) {
+        if (count > 0) v = *reinterpret_cast<const f32x4*>(p);
+    } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (j < count) v[j] = p[j];
     }
-    const int n0 = blockIdx.y * TB;
-    const int tx = threadIdx.x % 16, ty = threadIdx.x / 16;
+    return v;
+}
 
-    // loader: thread -> (tile row lr, four consecutive k)
-    const int lr = threadIdx.x / 4, lk = (threadIdx.x % 4) * 4;
-    const float* a_ptr = nullptr;
-    if (row0 + lr < rend) {
-        const int64_t src = p.a_gather ? p.a_gather[row0 + lr] : row0 + lr;
-        a_ptr = p.A + src * p.lda;
+// [ROWS][16] tile of k-contiguous rows.  Rows are 20 floats apart in LDS: the 16-byte fragment reads of 16 lanes then
+// start on 16 different groups of four banks.
+template <int ROWS, bool VEC>
+struct RowTile {
+    static constexpr int LD = TKS + 4, TPR = TKS / 4, LOADS = ROWS * TPR / kThreads, SIZE = ROWS * LD;
+    const float* ptr[LOADS];   // this thread's rows, NULL: zeros
+    f32x4 reg[2][LOADS];
+    __device__ __forceinline__ static int row(int p) { return threadIdx.x / TPR + p * (kThreads / TPR); }
+    __device__ __forceinline__ void fetch(int set, int k0, int Kdim) {
+        const int k = k0 + (threadIdx.x % TPR) * 4;
+#pragma unroll
+        for (int p = 0; p < LOADS; ++p) reg[set][p] = load4<VEC>(ptr[p] + k, ptr[p] ? Kdim - k : 0);
+    }
+    __device__ __forceinline__ void commit(int set, float* lds) const {
+#pragma unroll
+        for (int p = 0; p < LOADS; ++p) *reinterpret_cast<f32x4*>(lds + row(p) * LD + (threadIdx.x % TPR) * 4) = reg[set][p];
+    }
+    // k = 8s + 4 * (lane / 32) + 0..3 of row `r0 + lane % 32`
+    __device__ __forceinline__ static f32x4 frag(const float* lds, int r0, int s) {
+        const int lane = threadIdx.x % MTS_WAVE;
+        return *reinterpret_cast<const f32x4*>(lds + (r0 + lane % 32) * LD + s * 8 + (lane / 32) * 4);
+    }
+};
+
+// [16][COLS] tile of k-major rows.  The row length in LDS puts k and k+4, which the two halves of a wave read together,
+// 32 banks apart.
+template <int COLS, bool VEC>
+struct KTile {
+    static constexpr int LD = COLS + 8, LOADS = COLS * TKS / 4 / kThreads, SIZE = TKS * LD, PER_ROW = COLS / 4;
+    const float* base;       // element (k = 0, this thread's first column)
+    int64_t ld;
+    int cols;                // columns from there on that exist
+    f32x4 reg[2][LOADS];
+    __device__ __forceinline__ static int k(int p) { return threadIdx.x / PER_ROW + p * (kThreads / PER_ROW); }
+    __device__ __forceinline__ static int col() { return (threadIdx.x % PER_ROW) * 4; }
+    // rows[p] = memory row of k-row k(p), or < 0: zeros
+    __device__ __forceinline__ void fetch(int set, const int64_t (&rows)[LOADS]) {
+#pragma unroll
+        for (int p = 0; p < LOADS; ++p) reg[set][p] = load4<VEC>(base + rows[p] * ld, rows[p] >= 0 ? cols : 0);
+    }
+    __device__ __forceinline__ void commit(int set, float* lds) const {
+#pragma unroll
+        for (int p = 0; p < LOADS; ++p) *reinterpret_cast<f32x4*>(lds + k(p) * LD + col()) = reg[set][p];
+    }
+    __device__ __forceinline__ static f32x4 frag(const float* lds, int c0, int s) {
+        const int lane = threadIdx.x % MTS_WAVE;
+        const float* q = lds + (s * 8 + (lane / 32) * 4) * LD + c0 + lane % 32;
+        return f32x4{q[0], q[LD], q[2 * LD], q[3 * LD]};
+    }
+};
+
+// one k-tile: MF x NF fragments of 32x32 per wave; a_at / b_at give the first row / column of a fragment in the tile
+template <class AT, class BT, int MF, int NF, class AAt, class BAt>
+__device__ __forceinline__ void mma_tile32(const float* As, const float* Bs, f32x16 (&acc)[MF][NF], AAt a_at, BAt b_at) {
+#pragma unroll
+    for (int s = 0; s < TKS / 8; ++s) {
+        f32x4 a[MF], b[NF];
+#pragma unroll
+        for (int i = 0; i < MF; ++i) a[i] = AT::frag(As, a_at(i), s);
+#pragma unroll
+        for (int i = 0; i < NF; ++i) b[i] = BT::frag(Bs, b_at(i), s);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int mf = 0; mf < MF; ++mf)
+#pragma unroll
+                for (int nf = 0; nf < NF; ++nf)
+                    acc[mf][nf] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[mf][j], b[nf][j], acc[mf][nf], 0, 0, 0);
+    }
+}
+
+// The k loop: two LDS buffers, and two k-tiles in flight in registers behind them (a tile's loads have two tiles' matrix
+// work to arrive in).  fetch(set, t) starts the loads of k-tile t; it is called once for every t in order.
+template <class AT, class BT, int MF, int NF, class AAt, class BAt, class Fetch>
+__device__ __forceinline__ void run_k_tiles(int tiles, AT& a, BT& b, float (*As)[AT::SIZE], float (*Bs)[BT::SIZE], f32x16 (&acc)[MF][NF],
+                                            AAt a_at, BAt b_at, Fetch fetch) {
+    if (tiles <= 0) return;
+    fetch(0, 0);
+    if (tiles > 1) fetch(1, 1);
+    a.commit(0, As[0]);
+    b.commit(0, Bs[0]);
+    __syncthreads();
+    for (int t0 = 0; t0 < tiles; t0 += 2) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int t = t0 + u;
+            if (t >= tiles) break;
+            if (t + 2 < tiles) fetch(u, t + 2);
+            mma_tile32<AT, BT, MF, NF>(As[u], Bs[u], acc, a_at, b_at);
+            if (t + 1 < tiles) {
+                a.commit(1 - u, As[1 - u]);
+                b.commit(1 - u, Bs[1 - u]);
+            }
+            __syncthreads();
+        }
+    }
+}
+
+// The m-tiles of all experts in expert order, 64 experts per round: their number, and expert and rows of tile `tile`
+// (every lane of the wave gets the same answer; tile < 0: only the number is wanted).
+__device__ __forceinline__ int find_m_tile(const int32_t* __restrict__ expert_start, int E, int tile, int& e_out, int& row0, int& rend) {
+    const int lane = threadIdx.x % MTS_WAVE;
+    int seen = 0;
+    for (int e0 = 0; e0 < E; e0 += MTS_WAVE) {
+        const int e = e0 + lane;
+        const int s0 = e < E ? expert_start[e] : 0, s1 = e < E ? expert_start[e + 1] : 0;
+        const int nt = (s1 - s0 + BM - 1) / BM;
+        int upto = nt;
+#pragma unroll
+        for (int o = 1; o < MTS_WAVE; o <<= 1) {
+            const int t = __shfl_up(upto, o, MTS_WAVE);
+            if (lane >= o) upto += t;
+        }
+        const uint64_t mine = __ballot(tile >= seen + upto - nt && tile < seen + upto);
+        if (mine) {
+            const int l = __ffsll((unsigned long long)mine) - 1;
+            e_out = e0 + l;
+            row0 = __shfl(s0, l, MTS_WAVE) + (tile - seen - __shfl(upto - nt, l, MTS_WAVE)) * BM;
+            rend = __shfl(s1, l, MTS_WAVE);
+        }
+        seen += __shfl(upto, MTS_WAVE - 1, MTS_WAVE);
+    }
+    return seen;
+}
+
+// BN counts the columns of the B tile (SwiGLU: gate and up columns side by side, half the outputs)
+template <int BN, int EPI, bool BKM, bool VEC>
+__global__ __launch_bounds__(kThreads) void rows_gemm_f32_kernel(Rows32 p) {
+    constexpr int WAVES_M = 2, WAVES_N = 2;
+    constexpr int MF = BM / WAVES_M / 32, NF = BN / WAVES_N / 32;
+    constexpr int OUT_N = EPI == E32_SWIGLU ? BN / 2 : BN;
+    typedef RowTile<BM, VEC> ATile;
+    typedef typename std::conditional<BKM, KTile<BN, VEC>, RowTile<BN, VEC>>::type BTile;
+    __shared__ __attribute__((aligned(16))) float As[2][ATile::SIZE];
+    __shared__ __attribute__((aligned(16))) float Bs[2][BTile::SIZE];
+    __shared__ float ds_sum[EPI == E32_DY1 ? WAVES_N : 1][BM];
+
+    // block b runs on XCD b % 8: every XCD takes an equal contiguous run of the tiles, columns fastest, so that an expert's
+    // weights stream through one L2 and the blocks that share activation rows are neighbours in time
+    int e = 0, row0 = 0, rend = 0;
+    const int total = find_m_tile(p.expert_start, p.E, -1, e, row0, rend) * p.n_tiles;
+    const int per_xcd = (total + kXcds - 1) / kXcds, slot = blockIdx.x / kXcds;
+    const int tile = (blockIdx.x % kXcds) * per_xcd + slot;
+    if (slot >= per_xcd || tile >= total) return;
+    find_m_tile(p.expert_start, p.E, tile / p.n_tiles, e, row0, rend);
+    const int ny = tile % p.n_tiles, n0 = ny * OUT_N;
+
+    ATile a;
+#pragma unroll
+    for (int q = 0; q < ATile::LOADS; ++q) {
+        const int r = row0 + ATile::row(q);
+        a.ptr[q] = r < rend ? p.A + (int64_t)(p.a_gather ? p.a_gather[r] : r) * p.lda : nullptr;
     }
     const float* Be = p.B + (int64_t)e * p.b_rows * p.Kdim;
-    const float* b_ptr[NB];
+    BTile b;
+    if constexpr (BKM) {
+        b.base = Be + n0 + BTile::col();
+        b.ld = p.N;
+        b.cols = p.N - n0 - BTile::col();
+    } else {
 #pragma unroll
-    for (int h = 0; h < NB; ++h)
-        b_ptr[h] = (n0 + lr < p.N) ? Be + (int64_t)(h * p.N + n0 + lr) * p.Kdim : nullptr;
-
-    float acc[NB][4][4];
-#pragma unroll
-    for (int h = 0; h < NB; ++h)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) acc[h][i][j] = 0.f;
-
-    for (int k0 = 0; k0 < p.Kdim; k0 += TKS) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int k = k0 + lk + q;
-            As[lk + q][lr] = (a_ptr && k < p.Kdim) ? a_ptr[k] : 0.f;
-#pragma unroll
-            for (int h = 0; h < NB; ++h) Bs[h][lk + q][lr] = (b_ptr[h] && k < p.Kdim) ? b_ptr[h][k] : 0.f;
+        for (int q = 0; q < BTile::LOADS; ++q) {
+            const int r = BTile::row(q), half = r / OUT_N, n = n0 + r % OUT_N;
+            b.ptr[q] = n < p.N ? Be + (int64_t)(half * p.N + n) * p.Kdim : nullptr;
         }
-        __syncthreads();
-#pragma unroll
-        for (int k = 0; k < TKS; ++k) {
-            float a[4], b[NB][4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) a[i] = As[k][ty * 4 + i];
-#pragma unroll
-            for (int h = 0; h < NB; ++h)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) b[h][j] = Bs[h][k][tx * 4 + j];
-#pragma unroll
-            for (int h = 0; h < NB; ++h)
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) acc[h][i][j] = fmaf(a[i], b[h][j], acc[h][i][j]);
-        }
-        __syncthreads();
     }
+    auto fetch = [&](int set, int t) {
+        a.fetch(set, t * TKS, p.Kdim);
+        if constexpr (BKM) {
+            int64_t rows[BTile::LOADS];
+#pragma unroll
+            for (int q = 0; q < BTile::LOADS; ++q) rows[q] = t * TKS + BTile::k(q) < p.Kdim ? t * TKS + BTile::k(q) : -1;
+            b.fetch(set, rows);
+        } else b.fetch(set, t * TKS, p.Kdim);
+    };
+
+    const int wave = threadIdx.x / MTS_WAVE, wm = wave / WAVES_N, wn = wave % WAVES_N, lane = threadIdx.x % MTS_WAVE;
+    auto a_at = [&](int mf) { return wm * (BM / WAVES_M) + mf * 32; };
+    auto b_at = [&](int nf) { return EPI == E32_SWIGLU ? nf / (NF / 2) * OUT_N + wn * (OUT_N / WAVES_N) + nf % (NF / 2) * 32 : wn * (BN / WAVES_N) + nf * 32; };
+    f32x16 acc[MF][NF] = {};
+    const int tiles = (p.Kdim + TKS - 1) / TKS;
+    run_k_tiles<ATile, BTile, MF, NF>(tiles, a, b, As, Bs, acc, a_at, b_at, fetch);
 
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int row = row0 + ty * 4 + i;
-        const bool rok = row < rend;
-        float s = 0.f, dsp = 0.f;
-        if (EPI == E32_DY1 && rok) s = p.route_w[p.s_scatter[row]];
-        if (EPI == E32_SWIGLU) s = (rok && p.route_w) ? p.route_w[p.s_scatter[row]] : 1.f;   // post_act may carry the routing weight
+    for (int mf = 0; mf < MF; ++mf)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int n = n0 + tx * 4 + j;
-            if (!rok || n >= p.N) continue;
-            if (EPI == E32_PLAIN) {
-                p.C[(int64_t)row * p.N + n] = acc[0][i][j];
-            } else if (EPI == E32_SWIGLU) {
-                const float g = acc[0][i][j], u = acc[NB - 1][i][j];
-                p.C[(int64_t)row * (2 * p.N) + n] = g;
-                p.C[(int64_t)row * (2 * p.N) + p.N + n] = u;
-                p.C2[(int64_t)row * p.N + n] = g * sigmoid32(g) * u * s;
+        for (int i = 0; i < 16; ++i) {
+            const int r = a_at(mf) + 8 * (i / 4) + 4 * (lane / 32) + i % 4;
+            const int row = row0 + r;
+            const bool rok = row < rend;
+            if constexpr (EPI == E32_PLAIN) {
+#pragma unroll
+                for (int nf = 0; nf < NF; ++nf) {
+                    const int n = n0 + b_at(nf) + lane % 32;
+                    if (rok && n < p.N) p.C[(int64_t)row * p.N + n] = acc[mf][nf][i];
+                }
+            } else if constexpr (EPI == E32_SWIGLU) {
+                const float s = (rok && p.route_w) ? p.route_w[p.s_scatter[row]] : 1.f;   // post_act may carry the routing weight
+#pragma unroll
+                for (int nf = 0; nf < NF / 2; ++nf) {
+                    const int n = n0 + b_at(nf) + lane % 32;
+                    if (!rok || n >= p.N) continue;
+                    const float g = acc[mf][nf][i], u = acc[mf][nf + NF / 2][i];
+                    p.C[(int64_t)row * (2 * p.N) + n] = g;
+                    p.C[(int64_t)row * (2 * p.N) + p.N + n] = u;
+                    p.C2[(int64_t)row * p.N + n] = g * sigmoid32(g) * u * s;
+                }
             } else {
-                const int64_t o = (int64_t)row * (2 * p.N) + n;
-                const float g = p.pre_act[o], u = p.pre_act[o + p.N];
-                const float a = acc[0][i][j];
-                const float sig = sigmoid32(g);
-                const float silu = g * sig;
-                const float y1 = silu * u;
-                dsp += a * y1;
-                if (p.C2) p.C2[(int64_t)row * p.N + n] = s * y1;
-                const float da = a * s;
-                p.C[o] = da * (silu * (1.0f - sig) + sig) * u;
-                p.C[o + p.N] = da * silu;
+                const float s = rok ? p.route_w[p.s_scatter[row]] : 0.f;
+                float dsp = 0.f;
+#pragma unroll
+                for (int nf = 0; nf < NF; ++nf) {
+                    const int n = n0 + b_at(nf) + lane % 32;
+                    if (!rok || n >= p.N) continue;
+                    const int64_t o = (int64_t)row * (2 * p.N) + n;
+                    const float g = p.pre_act[o], u = p.pre_act[o + p.N];
+                    const float v = acc[mf][nf][i];
+                    const float sig = sigmoid32(g);
+                    const float silu = g * sig;
+                    const float y1 = silu * u;
+                    dsp += v * y1;
+                    if (p.C2) p.C2[(int64_t)row * p.N + n] = s * y1;
+                    const float da = v * s;
+                    p.C[o] = da * (silu * (1.0f - sig) + sig) * u;
+                    p.C[o + p.N] = da * silu;
+                }
+#pragma unroll
+                for (int o = 16; o > 0; o >>= 1) dsp += __shfl_xor(dsp, o, 32);
+                if (lane % 32 == 0) ds_sum[wn][r] = dsp;
             }
         }
-        if (EPI == E32_DY1) {
-            // the 16 threads that share `ty` hold the 64 columns of this row
+    if constexpr (EPI == E32_DY1) {   // row sums over the tile's 64 columns
+        __syncthreads();
+        for (int r = threadIdx.x; r < BM; r += kThreads)
+            if (row0 + r < rend) {
+                float v = ds_sum[0][r];
 #pragma unroll
-            for (int o = 8; o > 0; o >>= 1) dsp += __shfl_xor(dsp, o, MTS_WAVE);
-            if (rok && tx == 0) p.ds_part[(int64_t)row * p.np + blockIdx.y] = dsp;
-        }
+                for (int q = 1; q < WAVES_N; ++q) v += ds_sum[q][r];
+                p.ds_part[(int64_t)(row0 + r) * p.np + ny] = v;
+            }
     }
 }
 
@@ -158,89 +310,117 @@ struct Dw32 {
     const int32_t* q_gather;
     int M, N;
     const int32_t* expert_start;
+    int E;
     void* C;
+    int m_tiles, n_tiles;
 };
 
-template <typename OutT>
+// 64 x 64 outputs; the reduction runs over the expert's rows, both operands k-major
+template <typename OutT, bool VEC>
 __global__ __launch_bounds__(kThreads) void dw_gemm_f32_kernel(Dw32 p) {
-    __shared__ float Ps[TKS][TB + 4];
-    __shared__ float Qs[TKS][TB + 4];
-    const int e = blockIdx.z;
-    const int m0 = blockIdx.x * TB, n0 = blockIdx.y * TB;
+    constexpr int BN = 64, MF = BM / 64, NF = 1;
+    typedef KTile<BM, VEC> PT;
+    typedef KTile<BN, VEC> QT;
+    __shared__ __attribute__((aligned(16))) float Ps[2][PT::SIZE];
+    __shared__ __attribute__((aligned(16))) float Qs[2][QT::SIZE];
+    // an XCD takes an equal contiguous run of every expert's tiles, columns fastest: an equal share of the work however
+    // uneven the experts are, and about an eighth of P through its L2
+    const int per_expert = p.m_tiles * p.n_tiles, per_xcd = (per_expert + kXcds - 1) / kXcds;
+    const int slot = blockIdx.x / kXcds, e = slot / per_xcd;
+    const int tile = (blockIdx.x % kXcds) * per_xcd + slot % per_xcd;
+    if (tile >= per_expert || e >= p.E) return;
+    const int m0 = tile / p.n_tiles * BM, n0 = tile % p.n_tiles * BN;
     const int rbeg = p.expert_start[e], rend = p.expert_start[e + 1];
-    const int tx = threadIdx.x % 16, ty = threadIdx.x / 16;
-    const int lk = threadIdx.x / 16, lc = (threadIdx.x % 16) * 4;  // loader: (k row, four columns)
 
-    float acc[4][4];
+    PT a;
+    QT b;
+    a.base = p.P + m0 + PT::col(), a.ld = p.M, a.cols = p.M - m0 - PT::col();
+    b.base = p.Q + n0 + QT::col(), b.ld = p.N, b.cols = p.N - n0 - QT::col();
+    int64_t pr[PT::LOADS], qr[QT::LOADS];   // memory rows of the k-tile to fetch next: read a tile ahead of its data
+    auto locate = [&](int r0) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+        for (int q = 0; q < PT::LOADS; ++q) {
+            const int r = r0 + PT::k(q);
+            pr[q] = r < rend ? (p.p_gather ? p.p_gather[r] : r) : -1;
+        }
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
+        for (int q = 0; q < QT::LOADS; ++q) {
+            const int r = r0 + QT::k(q);
+            qr[q] = r < rend ? (p.q_gather ? p.q_gather[r] : r) : -1;
+        }
+    };
+    const int wave = threadIdx.x / MTS_WAVE, wm = wave / 2, wn = wave % 2, lane = threadIdx.x % MTS_WAVE;
+    auto a_at = [&](int mf) { return wm * (BM / 2) + mf * 32; };
+    auto b_at = [&](int) { return wn * (BN / 2); };
+    f32x16 acc[MF][NF] = {};
+    locate(rbeg);
+    auto fetch = [&](int set, int t) {
+        a.fetch(set, pr);
+        b.fetch(set, qr);
+        locate(rbeg + (t + 1) * TKS);
+    };
+    const int tiles = (rend - rbeg + TKS - 1) / TKS;
+    run_k_tiles<PT, QT, MF, NF>(tiles, a, b, Ps, Qs, acc, a_at, b_at, fetch);
 
-    for (int r0 = rbeg; r0 < rend; r0 += TKS) {
-        const int r = r0 + lk;
-        const bool ok = r < rend;
-        const int64_t ps = ok ? (p.p_gather ? p.p_gather[r] : r) : 0;
-        const int64_t qs = ok ? (p.q_gather ? p.q_gather[r] : r) : 0;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            Ps[lk][lc + q] = (ok && m0 + lc + q < p.M) ? p.P[ps * p.M + m0 + lc + q] : 0.f;
-            Qs[lk][lc + q] = (ok && n0 + lc + q < p.N) ? p.Q[qs * p.N + n0 + lc + q] : 0.f;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int k = 0; k < TKS; ++k) {
-            float a[4], b[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) a[i] = Ps[k][ty * 4 + i];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) b[j] = Qs[k][tx * 4 + j];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
-        }
-        __syncthreads();
-    }
     OutT* C = reinterpret_cast<OutT*>(p.C) + (int64_t)e * p.M * p.N;
+    const int n = n0 + b_at(0) + lane % 32;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int mf = 0; mf < MF; ++mf)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int m = m0 + ty * 4 + i, n = n0 + tx * 4 + j;
-            if (m < p.M && n < p.N) C[(int64_t)m * p.N + n] = (OutT)acc[i][j];
+        for (int i = 0; i < 16; ++i) {
+            const int m = m0 + a_at(mf) + 8 * (i / 4) + 4 * (lane / 32) + i % 4;
+            if (m < p.M && n < p.N) C[(int64_t)m * p.N + n] = (OutT)acc[mf][0][i];
         }
 }
 
 int64_t m_tiles32(int64_t TK, int E) {
-    const int64_t a = (TK + TB - 1) / TB + E - 1;
+    const int64_t a = (TK + BM - 1) / BM + E - 1;
     return a < TK ? a : TK;
 }
 
-}  // namespace
-
-// entry points used by the dispatchers in mts_gemm.hip when act_dtype == MTS_F32
-int mts_f32_rows(int epi, const float* A, int lda, const int32_t* a_gather, const float* B, int b_rows,
-                 int N, int Kdim, const int32_t* expert_start, int E, int64_t TK, float* C, float* C2,
-                 const float* pre_act, const float* route_w, const int32_t* s_scatter, float* ds_part,
-                 int np, hipStream_t s) {
-    Rows32 p = {A, lda, a_gather, B, b_rows, N, Kdim, expert_start, E, C, C2, pre_act, route_w, s_scatter, ds_part, np};
-    dim3 grid((unsigned)m_tiles32(TK, E), (unsigned)((N + TB - 1) / TB));
-    if (epi == E32_PLAIN) rows_gemm_f32_kernel<E32_PLAIN><<<grid, kThreads, 0, s>>>(p);
-    else if (epi == E32_SWIGLU) rows_gemm_f32_kernel<E32_SWIGLU><<<grid, kThreads, 0, s>>>(p);
-    else rows_gemm_f32_kernel<E32_DY1><<<grid, kThreads, 0, s>>>(p);
+template <int EPI, bool BKM>
+int launch_rows(Rows32 p, int64_t TK, bool vec, hipStream_t s) {
+    constexpr int BN = EPI == E32_SWIGLU ? 128 : 64, OUT_N = 64;
+    p.n_tiles = (p.N + OUT_N - 1) / OUT_N;
+    const int64_t blocks = (m_tiles32(TK, p.E) * p.n_tiles + kXcds - 1) / kXcds * kXcds;
+    if (blocks >= (1LL << 31)) return MTS_ERR_SHAPE;
+    const dim3 grid((unsigned)blocks);
+    if (vec) rows_gemm_f32_kernel<BN, EPI, BKM, true><<<grid, kThreads, 0, s>>>(p);
+    else rows_gemm_f32_kernel<BN, EPI, BKM, false><<<grid, kThreads, 0, s>>>(p);
     MTS_CHECK_LAUNCH();
     return MTS_OK;
 }
 
+}  // namespace
+
+// entry points used by the dispatchers in mts_gemm.hip when act_dtype == MTS_F32; b_kmajor: B is [E][Kdim][N]
+int mts_f32_rows(int epi, const float* A, int lda, const int32_t* a_gather, const float* B, int b_rows, int b_kmajor,
+                 int N, int Kdim, const int32_t* expert_start, int E, int64_t TK, float* C, float* C2,
+                 const float* pre_act, const float* route_w, const int32_t* s_scatter, float* ds_part,
+                 int np, hipStream_t s) {
+    Rows32 p = {A, lda, a_gather, B, b_rows, N, Kdim, expert_start, E, C, C2, pre_act, route_w, s_scatter, ds_part, np, 0};
+    // rows that are whole 16-byte groups; others are loaded four bytes at a time
+    const bool vec = lda % 4 == 0 && Kdim % 4 == 0 && (!b_kmajor || N % 4 == 0) && mts_aligned16(A) && mts_aligned16(B);
+    if (epi == E32_SWIGLU) return launch_rows<E32_SWIGLU, false>(p, TK, vec, s);
+    if (epi == E32_PLAIN) return b_kmajor ? launch_rows<E32_PLAIN, true>(p, TK, vec, s) : launch_rows<E32_PLAIN, false>(p, TK, vec, s);
+    return b_kmajor ? launch_rows<E32_DY1, true>(p, TK, vec, s) : launch_rows<E32_DY1, false>(p, TK, vec, s);
+}
+
 int mts_f32_dw(const float* P, const int32_t* p_gather, const float* Q, const int32_t* q_gather, int M,
                int N, const int32_t* expert_start, int E, int grad_dtype, void* C, hipStream_t s) {
-    Dw32 p = {P, p_gather, Q, q_gather, M, N, expert_start, C};
-    dim3 grid((unsigned)((M + TB - 1) / TB), (unsigned)((N + TB - 1) / TB), (unsigned)E);
-    if (grid.y > 65535 || grid.z > 65535) return MTS_ERR_SHAPE;
-    if (grad_dtype == MTS_F32) dw_gemm_f32_kernel<float><<<grid, kThreads, 0, s>>>(p);
-    else if (grad_dtype == MTS_BF16) dw_gemm_f32_kernel<bf16_t><<<grid, kThreads, 0, s>>>(p);
-    else if (grad_dtype == MTS_F16) dw_gemm_f32_kernel<mts_f16_t><<<grid, kThreads, 0, s>>>(p);
+    Dw32 p = {P, p_gather, Q, q_gather, M, N, expert_start, E, C, (M + BM - 1) / BM, (N + 63) / 64};
+    const bool vec = M % 4 == 0 && N % 4 == 0 && mts_aligned16(P) && mts_aligned16(Q);
+    const int64_t blocks = ((int64_t)p.m_tiles * p.n_tiles + kXcds - 1) / kXcds * kXcds * E;
+    if (blocks >= (1LL << 31)) return MTS_ERR_SHAPE;
+    const dim3 grid((unsigned)blocks);
+    auto launch = [&](auto* kind) {
+        typedef typename std::remove_pointer<decltype(kind)>::type OutT;
+        if (vec) dw_gemm_f32_kernel<OutT, true><<<grid, kThreads, 0, s>>>(p);
+        else dw_gemm_f32_kernel<OutT, false><<<grid, kThreads, 0, s>>>(p);
+    };
+    if (grad_dtype == MTS_F32) launch((float*)nullptr);
+    else if (grad_dtype == MTS_BF16) launch((bf16_t*)nullptr);
+    else if (grad_dtype == MTS_F16) launch((mts_f16_t*)nullptr);
     else return MTS_ERR_DTYPE;
     MTS_CHECK_LAUNCH();
     return MTS_OK;

@@ -18,6 +18,7 @@ from minitrain_amd.kernels.hip.switches import SWITCHES
 
 _MAX_EXPERTS = 65534   # MTS_MAX_MOE_EXPERTS
 BLOCK_M_TOKEN = 64
+_STORED_F32 = 2        # MTS_STORED_F32
 
 
 def ensure_contiguous(fn):
@@ -312,6 +313,11 @@ def _stage(lib, w: torch.Tensor, transpose: bool, dtype: torch.dtype, stream: in
     return out
 
 
+def _stored_layout(lib, act: int, H: int, I: int) -> int:
+    """How the backward GEMMs are told that a weight comes as it is stored; 0: they need a transposed copy."""
+    return _STORED_F32 if act == _lib.MTS_F32 else int(lib.mts_moe_bwd_weights_as_stored(act, H, I))
+
+
 class _Saved:
     """What the forward pass leaves for the backward pass (the tensors travel through
     ``ctx.save_for_backward``; the rest are plain attributes)."""
@@ -400,7 +406,7 @@ def moe_forward(x, gate_up_proj, down_proj, weights_flat, routing):
     state.weighted = weighted
     # fp32 parameters under a bf16 activation dtype: the backward GEMMs that read the weights as
     # stored reuse the casts made here (38 MB a layer at the 768/1024 shape) instead of repeating them
-    keep = bool(lib.mts_moe_bwd_weights_as_stored(act, H, I))
+    keep = bool(_stored_layout(lib, act, H, I))
     state.staged = (w1 if keep and w1 is not gate_up_proj else None, w2 if keep and w2 is not down_proj else None)
     return out, tensors, state
 
@@ -459,9 +465,10 @@ def moe_backward(tensors, state, dO, needs, x_addend=None, router_tail=None):
             ev.record(frm)
             main.wait_event(ev)
 
-    # The ring kernels read the weights in their stored layout (bf16, whole 64-wide k-tiles);
-    # other contracts get transposed copies, W1's made on a side stream next to the dO*W2 GEMM.
-    as_stored = bool(lib.mts_moe_bwd_weights_as_stored(act, H, I))
+    # The ring kernels (16-bit types, whole 64-wide k-tiles) and the fp32 kernels read the weights in their
+    # stored layout; other contracts get transposed copies, W1's made on a side stream next to the dO*W2 GEMM.
+    layout = _stored_layout(lib, act, H, I)
+    as_stored = bool(layout)
     w1_bwd = None
     if need_x:
         if as_stored:
@@ -499,7 +506,7 @@ def moe_backward(tensors, state, dO, needs, x_addend=None, router_tail=None):
             schedule = torch.empty(sched_bytes // 4, dtype=torch.int32, device=dev)
     _lib.check(
         lib.mts_moe_bwd_dy1(
-            dO.data_ptr(), w2_bwd.data_ptr(), int(as_stored), pre_act.data_ptr(), weights_flat.data_ptr(),
+            dO.data_ptr(), w2_bwd.data_ptr(), layout, pre_act.data_ptr(), weights_flat.data_ptr(),
             x_gather.data_ptr(),
             s_scatter.data_ptr(), expert_start.data_ptr(), T, K, E, H, I, act, d_pre_act.data_ptr(),
             None if state.weighted else weighted_act.data_ptr(), ds_part.data_ptr(), _lib.ptr(schedule), stream,
@@ -607,7 +614,7 @@ def moe_backward(tensors, state, dO, needs, x_addend=None, router_tail=None):
         dx_expanded = torch.empty(TK, H, dtype=x.dtype, device=dev)
         _lib.check(
             lib.mts_moe_bwd_dx(
-                d_pre_act.data_ptr(), w1_bwd.data_ptr(), int(as_stored), expert_start.data_ptr(), TK, E, H, I,
+                d_pre_act.data_ptr(), w1_bwd.data_ptr(), layout, expert_start.data_ptr(), TK, E, H, I,
                 act, dx_expanded.data_ptr(), stream,
             ),
             "mts_moe_bwd_dx",
