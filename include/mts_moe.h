@@ -241,7 +241,8 @@ int mts_moe_fwd_down(const void* post_act, const void* w2, const int32_t* expert
  * parts go to the XCDs in the same contiguous ranges, so writers and readers of a row share an L2, and
  * a counter per m-tile in `workspace` tells the readers when the rows are complete.
  *   mts_moe_fwd_joint_supported: 1 where the launch exists (bf16 / fp16, H and I multiples of 64, one
- *     expert's W1 no larger than an XCD's L2); elsewhere mts_moe_fwd_gateup_down returns MTS_ERR_SHAPE.
+ *     expert's W1 no larger than two XCD L2s); elsewhere mts_moe_fwd_gateup_down returns MTS_ERR_SHAPE.
+ *   mts_moe_fwd_joint_preferred: 1 where it also has enough rows to be the faster way.
  *   workspace: mts_moe_fwd_joint_workspace_bytes(TK, E) bytes of int32, 16-byte aligned, ALL ZERO on the
  *     first call.  A launch that ran through leaves it all zero, so calls that follow one another on a
  *     stream share one workspace (larger and smaller problems alike); calls that may overlap need one each.
@@ -251,6 +252,7 @@ int mts_moe_fwd_down(const void* post_act, const void* w2, const int32_t* expert
  *     and the workspace must be cleared before it is used again.  Reading the word is the caller's
  *     business (after a synchronisation, or from a copy made on the stream).                          */
 int mts_moe_fwd_joint_supported(int act_dtype, int H, int I);
+int mts_moe_fwd_joint_preferred(int act_dtype, int64_t TK, int E, int H, int I);
 int64_t mts_moe_fwd_joint_workspace_bytes(int64_t TK, int E);
 int mts_moe_fwd_gateup_down(const void* x, const void* w1, const void* w2, const int32_t* x_gather,
                             const int32_t* expert_start, const void* weights,
@@ -272,8 +274,8 @@ int mts_moe_combine(const void* y, const void* weights, const void* addend, cons
  * The weight operand comes in one of two layouts: w2_as_stored = 1, w2 is W2 itself
  * [E,H,I] in the activation dtype, or w2_as_stored = 0, it is the transposed copy [E,I,H]
  * made by mts_moe_stage_weights.  mts_moe_bwd_weights_as_stored(act_dtype, H, I) says
- * whether this entry point and mts_moe_bwd_dx take the stored layout (bf16, H and 2I
- * multiples of 64); otherwise they return MTS_ERR_SHAPE for it.  fp32 activations take the
+ * whether this entry point and mts_moe_bwd_dx take the stored layout (16-bit types, H and 2I each
+ * a multiple of 64 or at least 256); otherwise they return MTS_ERR_SHAPE for it.  fp32 activations take the
  * stored layout at any widths, asked for as MTS_STORED_F32.  ds_partial is
  * [TK, mts_moe_ds_partials(I)] f32 scratch reduced by mts_moe_bwd_ds (fixed order, no
  * atomics).  weighted_act may be NULL: it is then not written (the caller holds s*a already,

@@ -17,7 +17,7 @@
 //
 // Pipelines.  "staged": global -> VGPR -> LDS, two stages, any K that is a multiple
 // of 8.  "ring": global -> LDS directly (buffer_load ... lds), three or four stages,
-// whole k-tiles only, every wave loads and multiplies.  "ws": the same ring with
+// every wave loads and multiplies; lanes behind the end of the last k-tile load zeros.  "ws": the same ring with
 // specialised waves (producers issue the loads, consumers the MFMAs).  LDS rows are
 // XOR-swizzled instead of padded, so fragment reads and tile writes are both
 // bank-conflict free.
@@ -795,7 +795,7 @@ __global__ __launch_bounds__(T::NT) void rows_gemm_kernel(RowsParams p) {
 // MFMAs of tile k and no VGPRs or ds_write instructions are spent on staging.
 // The LDS image of a wave instruction is fixed (lane l lands at byte 16*l), so
 // the swizzle is applied on the global side: lane l fetches the chunk that
-// belongs at its landing slot.  Requires Kdim % BKS == 0.
+// belongs at its landing slot.  Kdim is a multiple of 8.
 // ---------------------------------------------------------------------------
 // A_STAGES_ = STAGES_ + 1: the activation tile has a buffer more than the weight tile (two stages only)
 template <int BM_, int BN_, int WAVES_M_, int WAVES_N_, int BKS_, int STAGES_, int WAVES_PER_EU_ = 1, int A_STAGES_ = STAGES_>
@@ -822,6 +822,28 @@ struct RingTile {
 };
 
 #define MTS_LDS_PTR(p) ((__attribute__((address_space(3))) void*)(p))
+
+// A reduction length that is not a whole number of k-tiles: the last tile's loads leave out what lies behind it.  The
+// offsets of the lanes whose 16-byte chunk (operands with k-contiguous rows) or whose row (k-major weights) is not part
+// of the reduction are put out of range before that tile, the last one they are used for, is issued; the loads then
+// land zeros.  `left`: elements of k in the last tile; first_row: the wave's first row in the tile.
+template <int COUNT, int CHUNKS, int RPI>
+__device__ __forceinline__ void mask_k_chunks(uint32_t (&voff)[COUNT], int first_row, int left) {
+    const int lane = threadIdx.x % MTS_WAVE, slot = lane % CHUNKS;
+#pragma unroll
+    for (int j = 0; j < COUNT; ++j) {
+        const int tr = first_row + j * RPI + lane / CHUNKS;
+        const int chunk = slot ^ (CHUNKS == 8 ? (tr >> 1) & 7 : (tr >> 2) & 3);
+        if (chunk * 8 >= left) voff[j] = kInvalid;
+    }
+}
+template <int COUNT, int CHUNKS_PER_ROW>
+__device__ __forceinline__ void mask_k_rows(uint32_t (&voff)[COUNT], int first_instr, int left) {
+    const int lane = threadIdx.x % MTS_WAVE;
+#pragma unroll
+    for (int j = 0; j < COUNT; ++j)
+        if ((first_instr + j) * (MTS_WAVE / CHUNKS_PER_ROW) + lane / CHUNKS_PER_ROW >= left) voff[j] = kInvalid;
+}
 
 // s_waitcnt vmcnt(N) only (gfx9 encoding: vmcnt = simm16[15:14,3:0], expcnt [6:4], lgkmcnt [11:8])
 template <int N>
@@ -890,9 +912,23 @@ __global__ __launch_bounds__(T::NT, T::WAVES_PER_EU) void rows_gemm_ring_kernel(
         }
     }
 
+    const int nk = (p.Kdim + T::BKS - 1) / T::BKS;
+    const int k_left = p.Kdim % T::BKS;   // of the last tile, 0: all of it
+    auto mask_a = [&](int kt) {
+        if (k_left && kt == nk - 1) mask_k_chunks<T::A_INSTR, T::CHUNKS, T::RPI>(voff_a, wave * T::A_INSTR * T::RPI, k_left);
+    };
+    auto mask_b = [&](int kt) {
+        if (k_left && kt == nk - 1) {
+            if constexpr (BKM) mask_k_rows<T::B_INSTR, CPR_B>(voff_b, wave * T::B_INSTR, k_left);
+            else mask_k_chunks<T::B_INSTR, T::CHUNKS, T::RPI>(voff_b, wave * T::B_INSTR * T::RPI, k_left);
+        }
+    };
+
     // loads of one stage; `part` of `parts` selects a slice so that the refill of a
     // stage can be spread over the k-steps of the tile that is being multiplied
     auto issue = [&](int stage, int kt, int part, int parts) {
+        mask_a(kt);
+        mask_b(kt);
         bf16_t* sa = smem + stage * T::STAGE + wave * T::A_INSTR * 512;
         bf16_t* sb = smem + stage * T::STAGE + T::BM * T::BKS + wave * T::B_INSTR * 512;
         const int soff = kt * T::BKS * 2;
@@ -910,7 +946,6 @@ __global__ __launch_bounds__(T::NT, T::WAVES_PER_EU) void rows_gemm_ring_kernel(
     f32x16 acc[T::MF][T::NF];
     zero_acc<T>(acc);
 
-    const int nk = p.Kdim / T::BKS;
     if constexpr (T::A_STAGES == 3 && S == 2) {
         // The activation tile (rows gathered from anywhere) is fetched two k-tiles ahead into three buffers, the
         // weight tile one ahead into two.  The weight loads of tile kt+1 are issued in the first k-step of tile kt,
@@ -918,6 +953,7 @@ __global__ __launch_bounds__(T::NT, T::WAVES_PER_EU) void rows_gemm_ring_kernel(
         // activation loads in flight.
         static_assert(T::BKS / 16 == 2, "two k-steps per tile");
         auto issue_a = [&](int buf, int kt) {
+            mask_a(kt);
             bf16_t* sa = smem + buf * T::BM * T::BKS + wave * T::A_INSTR * 512;
             const int soff = kt * T::BKS * 2;
 #pragma unroll
@@ -925,6 +961,7 @@ __global__ __launch_bounds__(T::NT, T::WAVES_PER_EU) void rows_gemm_ring_kernel(
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_a, MTS_LDS_PTR(sa + j * 512), 16, (int)voff_a[j], soff, 0, 0);
         };
         auto issue_b = [&](int buf, int kt) {
+            mask_b(kt);
             bf16_t* sb = smem + 3 * T::BM * T::BKS + buf * T::BN * T::BKS + wave * T::B_INSTR * 512;
             const int soff_b = BKM ? kt * T::BKS * p.N * 2 : kt * T::BKS * 2;
 #pragma unroll
@@ -1024,7 +1061,7 @@ __device__ __forceinline__ void rows_gemm_ws_tile(const RowsParams& p, bf16_t* s
     constexpr int S = T::STAGES, L = T::A_INSTR + T::B_INSTR;
     const int n0 = ntile * (SWIGLU ? T::BN / 2 : T::BN);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / MTS_WAVE), lane = threadIdx.x % MTS_WAVE;
-    const int nk = p.Kdim / T::BKS;
+    const int nk = (p.Kdim + T::BKS - 1) / T::BKS;
 
     if (wave >= T::NWAVES) {
         // ------------------------------ producer ------------------------------
@@ -1067,7 +1104,19 @@ __device__ __forceinline__ void rows_gemm_ws_tile(const RowsParams& p, bf16_t* s
                 voff_b[j] = (n < p.N) ? ((uint32_t)grow * (uint32_t)p.Kdim + chunk * 8) * 2u : kInvalid;
             }
         }
+        const int k_left = p.Kdim % T::BKS;   // of the last tile, 0: all of it
+        auto mask_a = [&](int kt) {
+            if (k_left && kt == nk - 1) mask_k_chunks<T::A_INSTR, T::CHUNKS, T::RPI>(voff_a, pw * T::A_INSTR * T::RPI, k_left);
+        };
+        auto mask_b = [&](int kt) {
+            if (k_left && kt == nk - 1) {
+                if constexpr (BKM) mask_k_rows<T::B_INSTR, CPR_B>(voff_b, pw * T::B_INSTR, k_left);
+                else mask_k_chunks<T::B_INSTR, T::CHUNKS, T::RPI>(voff_b, pw * T::B_INSTR * T::RPI, k_left);
+            }
+        };
         auto issue = [&](int stage, int kt) {
+            mask_a(kt);
+            mask_b(kt);
             bf16_t* sa = smem + stage * T::STAGE + pw * T::A_INSTR * 512;
             bf16_t* sb = smem + stage * T::STAGE + T::BM * T::BKS + pw * T::B_INSTR * 512;
             const int soff = kt * T::BKS * 2;
@@ -1085,12 +1134,14 @@ __device__ __forceinline__ void rows_gemm_ws_tile(const RowsParams& p, bf16_t* s
             // tile kt+2, which has two tiles' time to land.  The activation loads of tile kt+1, the youngest in flight,
             // may still be on their way at barrier kt-1... they are waited for one barrier later.
             auto issue_a = [&](int buf, int kt) {
+                mask_a(kt);
                 bf16_t* sa = smem + buf * T::BM * T::BKS + pw * T::A_INSTR * 512;
 #pragma unroll
                 for (int j = 0; j < T::A_INSTR; ++j)
                     __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_a, MTS_LDS_PTR(sa + j * 512), 16, (int)voff_a[j], kt * T::BKS * 2, 0, 0);
             };
             auto issue_b = [&](int buf, int kt) {
+                mask_b(kt);
                 bf16_t* sb = smem + 3 * T::BM * T::BKS + buf * T::BN * T::BKS + pw * T::B_INSTR * 512;
                 const int soff_b = BKM ? kt * T::BKS * p.N * 2 : kt * T::BKS * 2;   // a k-tile of k-major B is BKS memory rows further
 #pragma unroll
@@ -2231,15 +2282,14 @@ int64_t m_tiles(int64_t TK, int E) {
     return a < TK ? a : TK;
 }
 
-// Contiguous ranges of m-tiles per XCD pay off while one expert's weight matrix stays resident in an
-// XCD's 4 MiB L2 next to the streaming operands; larger weights are better streamed by all XCDs at the
-// same time (round-robin deal: one fetch from HBM, the other seven from the Infinity Cache).
-// A comparison run can force one or the other (mts_tuning.h).
+// Contiguous ranges of m-tiles per XCD, whatever the size of an expert's weights: what exceeds half an L2 is walked in
+// groups of column tiles (rows_grid), and the tiles behind the last whole round can be cut in two.  (All XCDs streaming
+// the same weights at the same time, the round-robin deal, costs the operator 4 % at 4096/14336 and 4096 tokens, 8 % at
+// 1024/2048 and 24 576.)  A comparison run can force one or the other (mts_tuning.h).
 constexpr int64_t kL2Bytes = 4 << 20;   // per XCD
-int xcd_ranges_choice(int64_t expert_weight_bytes) {
+int xcd_ranges_choice() {
     const int forced = mts_tuning().xcd_ranges;
-    if (forced >= 0) return forced;
-    return expert_weight_bytes <= kL2Bytes ? 1 : 0;
+    return forced >= 0 ? forced : 1;
 }
 
 // the n-tile groups and the reversed walks of the range mapping, which a comparison run can switch off one by one
@@ -2254,7 +2304,7 @@ dim3 rows_grid(RowsParams& p, int64_t TK) {
     const int per_block = (EPI == EPI_SWIGLU) ? T::BN / 2 : T::BN;
     p.n_tiles = (p.N + per_block - 1) / per_block;
     const int64_t weight_bytes = (int64_t)p.b_rows * p.Kdim * (int64_t)sizeof(bf16_t);
-    p.xcd_ranges = xcd_ranges_choice(weight_bytes);
+    p.xcd_ranges = xcd_ranges_choice();
     p.n_groups = 1;
     if (p.xcd_ranges && (tile_order_mask() & ORDER_GROUPS))
         while (weight_bytes / p.n_groups > kL2Bytes / 2 && p.n_tiles % (2 * p.n_groups) == 0 && p.n_tiles / (2 * p.n_groups) >= 4)
@@ -2265,8 +2315,14 @@ dim3 rows_grid(RowsParams& p, int64_t TK) {
     return dim3((unsigned)((m_groups * p.n_tiles + p.tail_slots / 2 + p.tail_tiles) * kXcds + (p.sched_out ? 1 : 0)));
 }
 
+// The ring and specialised pipelines take whole 64-wide k-tiles, and any other reduction length (a multiple of 8) of at
+// least four of them: the zeros behind the end of the last tile are then at most a fifth of the matrix work, where the
+// staged kernel, which shorter ones are left to, takes up to twice the time per product (6001 tokens of 1000/1368, fp16: down
+// projection 70 -> 44 us, dX and the weight gradients together 330 -> 210 us, no transposed copies of the weights).
+bool rows_pipelined(int Kdim) { return Kdim % 64 == 0 || Kdim >= 256; }
+
 // does launch_rows_any take B in the weights' stored layout for this kind and reduction length?
-bool rows_kmajor_ok(int kind, int Kdim) { return tile_choice(kind) >= 1 && Kdim % 64 == 0; }
+bool rows_kmajor_ok(int kind, int Kdim) { return tile_choice(kind) >= 1 && rows_pipelined(Kdim); }
 
 // b_kmajor: B is [E][Kdim][N] (the weights as stored) instead of the transposed copy [E][N][Kdim];
 // only the ring and specialised kernels read it that way
@@ -2279,8 +2335,7 @@ int launch_rows_any(int kind, RowsParams p, int64_t TK, hipStream_t s, bool b_km
     if (choice == 3 && (EPI != EPI_DY1N || !b_kmajor || (!tile_forced(kind) && p.Kdim > 1024))) choice = 1;
     // the 64-wide variant exists for the GEMMs with a plain or SwiGLU epilogue
     if (choice == 4 && epi_is_dy1(EPI)) choice = 2;
-    // the ring kernels need whole k-tiles; other shapes use the staged kernel
-    if (choice >= 1 && p.Kdim % 64 != 0) choice = 0;
+    if (choice >= 1 && !rows_pipelined(p.Kdim)) choice = 0;
     if (b_kmajor && (choice == 0 || EPI == EPI_SWIGLU)) return MTS_ERR_SHAPE;
     if (choice == 3) {
         if constexpr (EPI == EPI_DY1N) {
@@ -2387,14 +2442,22 @@ int launch_dw_any(int kind, DwParams p, int E, int grad_dtype, void* workspace, 
 }
 
 // gate/up + down as one launch: both on the 256 x 256 tiles with specialised waves, both dealt to the XCDs in
-// contiguous ranges of the same m-tiles (an expert's W1 fits an L2)
+// contiguous ranges of the same m-tiles, and an expert's W1 at most twice an L2 (beyond that the two launches are as
+// fast at 16 384 tokens and faster below)
 bool fwd_joint_ok(int H, int I) {
     const int n_tiles_gu = (I + FwdGuTile::BN / 2 - 1) / (FwdGuTile::BN / 2);
-    return tile_choice(K_GATEUP) == 4 && tile_choice(K_DOWN) == 4 && H % 64 == 0 && I % 64 == 0 &&
-           xcd_ranges_choice((int64_t)2 * I * H * (int64_t)sizeof(bf16_t)) == 1 &&
-           xcd_ranges_choice((int64_t)I * H * (int64_t)sizeof(bf16_t)) == 1 && FwdGuTile::NWAVES * n_tiles_gu <= kReadyCountMax;
+    return tile_choice(K_GATEUP) == 4 && tile_choice(K_DOWN) == 4 && H % 64 == 0 && I % 64 == 0 && xcd_ranges_choice() == 1 &&
+           (int64_t)2 * I * H * (int64_t)sizeof(bf16_t) <= 2 * kL2Bytes && FwdGuTile::NWAVES * n_tiles_gu <= kReadyCountMax;
 }
 int64_t fwd_joint_counters(int64_t TK, int E) { return m_tiles<FwdGuTile>(TK, E); }
+
+// Does the one launch pay at this many rows?  A down tile waits for all gate/up tiles of its rows, which run side by side:
+// with less than two rounds of gate/up tiles over the CUs most of the down part only waits (768/1024, 8 experts: 81 against
+// 45 us for two launches at 4096 rows, 115 against 82 at 13 000, even at 16 384).
+bool fwd_joint_pays(int64_t TK, int E, int I) {
+    const int n_tiles_gu = (I + FwdGuTile::BN / 2 - 1) / (FwdGuTile::BN / 2);
+    return m_tiles<FwdGuTile>(TK, E) * n_tiles_gu >= 2 * kXcds * kCusPerXcd;
+}
 
 int launch_fwd_joint(RowsParams gu, RowsParams down, int64_t TK, int32_t* workspace, hipStream_t s) {
     FwdJointParams q = {};
@@ -2410,7 +2473,8 @@ int launch_fwd_joint(RowsParams gu, RowsParams down, int64_t TK, int32_t* worksp
     const int tail_mtiles = forced >= 0 ? forced : (by_rule > 1 ? by_rule : 1);
     down.tail_tiles = tail_mtiles * down.n_tiles;
     const int n_down = (int)rows_grid<FwdDownTile, EPI_PLAIN>(down, TK).x;
-    if (!gu.xcd_ranges || !down.xcd_ranges || down.n_groups != 1) return MTS_ERR_SHAPE;
+    if (!gu.xcd_ranges || !down.xcd_ranges) return MTS_ERR_SHAPE;
+    down.n_groups = 1;   // its m-tiles become ready one after the other: no second walk through the range
     q.gu = gu;
     q.down = down;
     const int64_t n = fwd_joint_counters(TK, gu.E);
@@ -2593,6 +2657,9 @@ extern "C" int MTS_GEMM_ENTRY(mts_moe_fwd_down)(const void* post_act, const void
 #ifndef MTS_GEMM_F16
 extern "C" int mts_moe_fwd_joint_supported(int act_dtype, int H, int I) {
     return (act_dtype == MTS_BF16 || act_dtype == MTS_F16) && H >= 64 && I >= 64 && fwd_joint_ok(H, I) ? 1 : 0;
+}
+extern "C" int mts_moe_fwd_joint_preferred(int act_dtype, int64_t TK, int E, int H, int I) {
+    return mts_moe_fwd_joint_supported(act_dtype, H, I) && TK > 0 && E >= 1 && fwd_joint_pays(TK, E, I) ? 1 : 0;
 }
 extern "C" int64_t mts_moe_fwd_joint_workspace_bytes(int64_t TK, int E) {
     if (TK <= 0 || E < 1) return 0;

@@ -45,6 +45,7 @@ SIGNATURES = {
     "mts_moe_fwd_gateup_swiglu": (_i, [_p, _p, _p, _p, _p, _p, _l, _i, _i, _i, _i, _i, _p, _p, _p]),
     "mts_moe_fwd_down": (_i, [_p, _p, _p, _l, _i, _i, _i, _i, _p, _p]),
     "mts_moe_fwd_joint_supported": (_i, [_i, _i, _i]),
+    "mts_moe_fwd_joint_preferred": (_i, [_i, _l, _i, _i, _i]),
     "mts_moe_fwd_joint_workspace_bytes": (_l, [_l, _i]),
     "mts_moe_fwd_gateup_down": (_i, [_p] * 7 + [_l, _i, _i, _i, _i, _i, _p, _p, _p, _p, _l, _p]),
     "mts_moe_combine": (_i, [_p, _p, _p, _p, _l, _i, _i, _i, _p, _p]),

@@ -361,7 +361,7 @@ def moe_forward(x, gate_up_proj, down_proj, weights_flat, routing):
     # written again there (TK * I elements held from forward to backward, and as many fewer written).
     weighted = SWITCHES.weighted_post
     y = torch.empty(TK, H, dtype=x.dtype, device=dev)
-    if SWITCHES.joint_fwd and x.dtype != torch.float32 and lib.mts_moe_fwd_joint_supported(act, H, I):
+    if SWITCHES.joint_fwd and lib.mts_moe_fwd_joint_preferred(act, TK, E, H, I):
         # one launch: the down tiles take the CUs as the gate/up tiles leave them
         jw = _joint_forward_workspace(dev)
         jw.before_launch()
@@ -465,7 +465,7 @@ def moe_backward(tensors, state, dO, needs, x_addend=None, router_tail=None):
             ev.record(frm)
             main.wait_event(ev)
 
-    # The ring kernels (16-bit types, whole 64-wide k-tiles) and the fp32 kernels read the weights in their
+    # The ring kernels (16-bit types, widths of whole 64-wide k-tiles or of at least 256) and the fp32 kernels read the weights in their
     # stored layout; other contracts get transposed copies, W1's made on a side stream next to the dO*W2 GEMM.
     layout = _stored_layout(lib, act, H, I)
     as_stored = bool(layout)
