@@ -1,0 +1,813 @@
+// Host path of the `hip` backend: contract checks, allocation and the autograd nodes of the operators, in front of the C ABI
+// of the kernel library (include/mts_moe.h).
+//
+// A layer step is seven to nine launches, 60 to 350 us of kernels at up to 5000 tokens.  Allocating two dozen tensors,
+// marshalling two hundred arguments and passing the interpreter lock between the caller's thread and autograd's took 220 to
+// 360 us in Python (two speeds, from process to process), so that every small call ran at the speed of the host.  Native, a
+// forward pass of 16 tokens takes 51 us instead of 102 and a training step of 512 tokens 161 instead of 220 to 360: what
+// their kernels take.
+//
+// Nothing here synchronises with the GPU.  Every buffer is a torch tensor from the caching allocator; the backward pass of
+// the operator forks two side streams for kernels that do not depend on one another and joins them before it returns.
+#include <ATen/ATen.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+#include <hip/hip_runtime.h>
+#include <pybind11/pybind11.h>
+#include <pybind11/stl.h>
+#include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/utils/pybind.h>
+
+#include <map>
+#include <mutex>
+#include <optional>
+#include <string>
+#include <vector>
+
+#include "mts_moe.h"
+
+namespace {
+
+using at::Tensor;
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+typedef std::optional<Tensor> MaybeTensor;
+
+// ---- small helpers ---------------------------------------------------------------------------------------------------------
+
+void* ptr(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
+template <typename T>
+T* ptr_as(const Tensor& t) { return static_cast<T*>(ptr(t)); }
+
+void check(int code, const char* what) { TORCH_CHECK(code == 0, what, " failed: ", mts_error_string(code), " (code ", code, ")"); }
+
+int dtype_code(at::ScalarType t) {
+    switch (t) {
+        case at::kBFloat16: return MTS_BF16;
+        case at::kHalf: return MTS_F16;
+        case at::kFloat: return MTS_F32;
+        default: TORCH_CHECK(false, "unsupported dtype ", t);
+    }
+}
+int dtype_code(const Tensor& t) { return dtype_code(t.scalar_type()); }
+bool is_activation_type(at::ScalarType t) { return t == at::kBFloat16 || t == at::kHalf || t == at::kFloat; }
+
+void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+Tensor bytes(int64_t n, const Tensor& like) { return at::empty({n > 4 ? n : 4}, like.options().dtype(at::kByte)); }
+Tensor f32(at::IntArrayRef size, const Tensor& like) { return at::empty(size, like.options().dtype(at::kFloat)); }
+Tensor i32(at::IntArrayRef size, const Tensor& like) { return at::empty(size, like.options().dtype(at::kInt)); }
+Tensor like_f32(const Tensor& g) { return g.defined() ? g.to(at::kFloat).contiguous() : g; }
+bool aligned16(const Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; }
+Tensor dense16(const Tensor& t) {   // dense and starting on a 16-byte boundary (a view may start inside an allocation)
+    Tensor d = t.contiguous();
+    return aligned16(d) ? d : d.clone();
+}
+int64_t round4(int64_t n) { return (n + 3) / 4 * 4; }
+
+// ---- contracts ---------------------------------------------------------------------------------------------------------------
+// The first requirement that the arguments miss, or NULL.
+
+constexpr int64_t kMaxExperts = MTS_MAX_MOE_EXPERTS, kMaxTopK = MTS_MAX_TOP_K, kMaxRouterExperts = MTS_MAX_EXPERTS;
+constexpr int64_t k2GiB = 1LL << 31;
+
+const char* expert_violation(const Tensor& x, const Tensor& w1, const Tensor& w2) {
+    if (x.dim() != 2 || w1.dim() != 3 || w2.dim() != 3) return "x is [T,H], gate_up_proj [E,2I,H] and down_proj [E,H,I]";
+    const int64_t T = x.size(0), H = x.size(1), E = w1.size(0), two_i = w1.size(1), I = two_i / 2;
+    if (!x.is_cuda() || !w1.is_cuda() || !w2.is_cuda() || x.device() != w1.device() || x.device() != w2.device()) return "all tensors on one GPU";
+    const auto t = x.scalar_type();
+    if (!is_activation_type(t)) return "activations are bf16, fp16 or fp32";
+    if (T <= 0) return "at least one token";
+    if (E <= 0 || E > kMaxExperts) return "between 1 and 65534 experts";
+    if (two_i % 2 || w1.size(2) != H || w2.size(0) != E || w2.size(1) != H || w2.size(2) != I)
+        return "gate_up_proj is [E,2I,H] and down_proj [E,H,I] for x [T,H]";
+    // expert parameters come in the activation dtype or as fp32 master weights; fp32 activations take 16-bit parameters as
+    // well (widened once per call)
+    auto fits = [&](at::ScalarType p) { return p == at::kFloat || p == t || (t == at::kFloat && is_activation_type(p)); };
+    if (!fits(w1.scalar_type()) || !fits(w2.scalar_type()))
+        return "expert parameters in the activation dtype or fp32 (any of fp32/bf16/fp16 under fp32 activations)";
+    // rows of x and of dO are gathered from anywhere through 32-bit offsets; the [T*K, ...] intermediates are addressed tile
+    // by tile and may be larger
+    if (t != at::kFloat && (T * H * 2 >= k2GiB || 2 * I * H * 2 >= k2GiB)) return "16-bit activations and one expert's weights smaller than 2 GiB each";
+    return nullptr;
+}
+
+const char* routing_violation(const Tensor& x, const Tensor& w1, const Tensor& index, const Tensor& weights) {
+    if (index.dim() != 2) return "top_k_index is [T,K]";
+    const int64_t K = index.size(1);
+    if (!index.is_cuda() || !weights.is_cuda() || index.device() != x.device() || weights.device() != x.device())
+        return "routing tensors on the activations' GPU";
+    if (weights.sizes() != index.sizes() || index.size(0) != x.size(0)) return "top_k_index and top_k_weights are [T,K]";
+    if (K <= 0 || K > std::min<int64_t>(w1.size(0), 32768)) return "1 <= K <= number of experts (at most 32768)";
+    if (x.size(0) * K >= k2GiB) return "fewer than 2^31 routes";
+    if (index.scalar_type() != at::kInt) return "int32 expert indices";
+    if (weights.scalar_type() != x.scalar_type()) return "routing weights in the activation dtype";
+    return nullptr;
+}
+
+const char* fused_moe_violation(const Tensor& x, const Tensor& w1, const Tensor& w2, const Tensor& index, const Tensor& weights) {
+    const char* missed = expert_violation(x, w1, w2);
+    return missed ? missed : routing_violation(x, w1, index, weights);
+}
+
+// The kernels move 16 bytes per lane: rows are whole 16-byte chunks, or zero-padded to that by the caller.
+bool needs_padding(const Tensor& x, const Tensor& w1) {
+    const bool wide = x.scalar_type() == at::kFloat;
+    return x.size(1) % (wide ? 4 : 8) != 0 || (!wide && (w1.size(1) / 2) % 8 != 0);
+}
+
+bool router_logits_supported(const Tensor& x, const Tensor& w) {
+    return x.is_cuda() && w.is_cuda() && x.dim() == 2 && w.dim() == 2 && is_activation_type(x.scalar_type()) && w.scalar_type() == at::kFloat &&
+           x.size(0) > 0 && x.size(1) == w.size(1) && w.size(0) <= 16 && x.size(1) % 4 == 0 && x.size(1) <= 4096 &&
+           w.size(0) * w.size(1) * 4 <= 128 * 1024;   // the projection kernels keep W_r in LDS
+}
+
+const char* layer_violation(const Tensor& x, const Tensor& w_r, const Tensor& w1, const Tensor& w2, int64_t top_k) {
+    if (const char* missed = expert_violation(x, w1, w2)) return missed;
+    const int64_t E = w1.size(0);
+    if (w_r.dim() != 2 || w_r.size(0) != E) return "router weight is [E,H]";
+    if (!router_logits_supported(x, w_r))
+        return "an fp32 router weight on the same GPU, at most 16 experts and a hidden size of at most 4096 (E * H <= 32768)";
+    if (top_k < 1 || top_k > std::min(E, kMaxTopK)) return "1 <= top_k <= min(E, 8)";
+    if (needs_padding(x, w1)) return "hidden and expert widths that are whole 16-byte chunks";
+    if (x.size(0) * top_k >= k2GiB) return "fewer than 2^31 routes";
+    return nullptr;
+}
+
+// ---- options -----------------------------------------------------------------------------------------------------------------
+
+// Comparison switches of the Python side (kernels/hip/switches.py), as they stand when an operator is called.
+enum Switch : int64_t { OVERLAP = 1, JOINT_BWD = 2, JOINT_FWD = 4, TAIL_IN_JOINT = 8, COMBINE_IN_TAIL = 16, JOINT_SCHEDULE = 32, WEIGHTED_POST = 64 };
+
+struct Options {
+    int64_t switches;
+    int64_t dw_workspace_limit;   // row-chunk workspaces of the weight-gradient GEMMs beyond this size are done without
+    bool on(Switch s) const { return (switches & s) != 0; }
+};
+
+// Counters of the joint gate/up + down launch, owned by the Python side (one per device and stream): an object with
+// before_launch(), get(bytes) and after_launch().  Forward passes run under the interpreter lock.
+pybind11::object* joint_workspace_of = nullptr;   // device index -> that object; never destroyed
+
+// ---- streams -----------------------------------------------------------------------------------------------------------------
+
+hipStream_t side_stream(int device, int index) {
+    static std::mutex lock;
+    static std::map<std::pair<int, int>, c10::hip::HIPStream> streams;
+    std::lock_guard<std::mutex> held(lock);
+    auto it = streams.find({device, index});
+    if (it == streams.end()) it = streams.emplace(std::make_pair(device, index), c10::hip::getStreamFromPool(/*isHighPriority=*/false, device)).first;
+    return it->second.stream();
+}
+
+// work enqueued on `to` from here on waits for what `from` holds now
+void order_after(hipStream_t to, hipStream_t from) {
+    if (to == from) return;
+    hipEvent_t ev;
+    TORCH_CHECK(hipEventCreateWithFlags(&ev, hipEventDisableTiming) == hipSuccess, "hipEventCreate failed");
+    const bool ok = hipEventRecord(ev, from) == hipSuccess && hipStreamWaitEvent(to, ev, 0) == hipSuccess;
+    (void)hipEventDestroy(ev);   // released once the recorded work has passed it
+    TORCH_CHECK(ok, "ordering two streams failed");
+}
+
+// ---- experts: forward and backward ---------------------------------------------------------------------------------------------
+
+struct Routing {
+    Tensor expert_start, x_gather, s_scatter, s_reverse;
+};
+
+// Routing metadata of given expert indices, in one int32 allocation (the per-row arrays start on 16-byte boundaries).
+Routing route(const Tensor& index, int64_t E) {
+    const int64_t T = index.size(0), K = index.size(1), TK = T * K, pad = round4(2 * E + 1);
+    Tensor buf = i32({pad + 3 * round4(TK)}, index);
+    Routing r;
+    Tensor counts = buf.narrow(0, 0, E);
+    r.expert_start = buf.narrow(0, E, E + 1);
+    r.s_scatter = buf.narrow(0, pad, TK);
+    r.s_reverse = buf.narrow(0, pad + round4(TK), TK);
+    r.x_gather = buf.narrow(0, pad + 2 * round4(TK), TK);
+    const int64_t ws_bytes = mts_moe_route_workspace_bytes(T, K, E);
+    Tensor ws = bytes(ws_bytes, index);
+    check(mts_moe_route(ptr_as<int32_t>(index), T, K, E, 64, ptr_as<int32_t>(counts), ptr_as<int32_t>(r.expert_start), ptr_as<int32_t>(r.s_scatter),
+                        ptr_as<int32_t>(r.s_reverse), ptr_as<int32_t>(r.x_gather), nullptr, nullptr, nullptr, ptr(ws), ws_bytes, stream_of(index)),
+          "mts_moe_route");
+    return r;
+}
+
+// Copy of an expert weight [E,R,C] in the activation dtype, optionally as [E,C,R].
+Tensor stage(const Tensor& w, bool transpose, at::ScalarType dtype, void* stream) {
+    if (!transpose && w.scalar_type() == dtype) return w;
+    const int64_t E = w.size(0), R = w.size(1), C = w.size(2);
+    Tensor out = at::empty({E, transpose ? C : R, transpose ? R : C}, w.options().dtype(dtype));
+    check(mts_moe_stage_weights(ptr(w), dtype_code(w), ptr(out), dtype_code(dtype), E, R, C, transpose, stream), "mts_moe_stage_weights");
+    return out;
+}
+
+// How the backward GEMMs are told that a weight comes as it is stored; 0: they need a transposed copy.
+int stored_layout(int act, int64_t H, int64_t I) { return act == MTS_F32 ? MTS_STORED_F32 : mts_moe_bwd_weights_as_stored(act, H, I); }
+
+// What the forward pass leaves for the backward pass.  The tensors travel through save_for_backward in this order.
+struct Saved {
+    Tensor x, w1, w2, pre_act, weights, expert_start, x_gather, s_scatter, s_reverse, post_act, staged1, staged2;
+    static constexpr size_t kCount = 12;
+    void append_to(variable_list& v) const {
+        v.insert(v.end(), {x, w1, w2, pre_act, weights, expert_start, x_gather, s_scatter, s_reverse, post_act, staged1, staged2});
+    }
+    explicit Saved(const variable_list& v)
+        : x(v[0]), w1(v[1]), w2(v[2]), pre_act(v[3]), weights(v[4]), expert_start(v[5]), x_gather(v[6]), s_scatter(v[7]), s_reverse(v[8]),
+          post_act(v[9]), staged1(v[10]), staged2(v[11]) {}
+    Saved() = default;
+};
+
+// Gate/up + SwiGLU, down projection and combine for routes that are already sorted.  `weights`: flat, activation dtype.
+Tensor experts_forward(const Tensor& x, const Tensor& w1_in, const Tensor& w2_in, const Tensor& weights, const Routing& r, const Options& opt, Saved& s) {
+    const int64_t T = x.size(0), H = x.size(1), E = w1_in.size(0), I = w1_in.size(1) / 2, TK = weights.numel(), K = TK / T;
+    const auto dtype = x.scalar_type();
+    const int act = dtype_code(dtype);
+    void* stream = stream_of(x);
+    Tensor w1, w2;
+    if (w1_in.scalar_type() == at::kFloat && w2_in.scalar_type() == at::kFloat && dtype != at::kFloat && w1_in.numel() % 8 == 0 && w2_in.numel() % 8 == 0) {
+        // fp32 master weights: both casts in one launch (the backward pass reuses the copies)
+        w1 = at::empty(w1_in.sizes(), x.options());
+        w2 = at::empty(w2_in.sizes(), x.options());
+        check(mts_moe_cast_weights_pair(ptr_as<float>(w1_in), ptr(w1), w1_in.numel(), ptr_as<float>(w2_in), ptr(w2), w2_in.numel(), act, stream),
+              "mts_moe_cast_weights_pair");
+    } else {
+        w1 = stage(w1_in, false, dtype, stream);
+        w2 = stage(w2_in, false, dtype, stream);
+    }
+    // The routing weight is applied where the activation is formed: post_act = s * silu(g) * u.  The down projection then
+    // yields s * y, the combine is a plain sum, and post_act is at the same time the operand of the dW2 GEMM, so it is kept
+    // for the backward pass instead of being written again there.
+    const bool weighted = opt.on(WEIGHTED_POST);
+    Tensor pre_act = at::empty({TK, 2 * I}, x.options()), post_act = at::empty({TK, I}, x.options()), y = at::empty({TK, H}, x.options());
+    void* route_w = weighted ? ptr(weights) : nullptr;
+    int32_t* route_entry = weighted ? ptr_as<int32_t>(r.s_scatter) : nullptr;
+    if (opt.on(JOINT_FWD) && mts_moe_fwd_joint_preferred(act, TK, E, H, I)) {
+        // one launch: the down tiles take the CUs as the gate/up tiles leave them
+        const int64_t need = mts_moe_fwd_joint_workspace_bytes(TK, E);
+        pybind11::object ws = (*joint_workspace_of)((int)x.device().index());
+        ws.attr("before_launch")();
+        Tensor counters = ws.attr("get")(need).cast<Tensor>();
+        check(mts_moe_fwd_gateup_down(ptr(x), ptr(w1), ptr(w2), ptr_as<int32_t>(r.x_gather), ptr_as<int32_t>(r.expert_start), route_w, route_entry, T, K, E, H,
+                                      I, act, ptr(pre_act), ptr(post_act), ptr(y), ptr_as<int32_t>(counters), need, stream),
+              "mts_moe_fwd_gateup_down");
+        ws.attr("after_launch")();
+    } else {
+        check(mts_moe_fwd_gateup_swiglu(ptr(x), ptr(w1), ptr_as<int32_t>(r.x_gather), ptr_as<int32_t>(r.expert_start), route_w, route_entry, T, K, E, H, I,
+                                        act, ptr(pre_act), ptr(post_act), stream),
+              "mts_moe_fwd_gateup_swiglu");
+        check(mts_moe_fwd_down(ptr(post_act), ptr(w2), ptr_as<int32_t>(r.expert_start), TK, E, H, I, act, ptr(y), stream), "mts_moe_fwd_down");
+    }
+    Tensor out = at::empty({T, H}, x.options());
+    check(mts_moe_combine(ptr(y), weighted ? nullptr : ptr(weights), nullptr, ptr_as<int32_t>(r.s_reverse), T, K, H, act, ptr(out), stream), "mts_moe_combine");
+    s.x = x, s.w1 = w1_in, s.w2 = w2_in, s.pre_act = pre_act, s.weights = weights;
+    s.expert_start = r.expert_start, s.x_gather = r.x_gather, s.s_scatter = r.s_scatter, s.s_reverse = r.s_reverse;
+    if (weighted) s.post_act = post_act;
+    if (stored_layout(act, H, I)) {   // the backward GEMMs read the weights as stored: they reuse casts made here
+        if (!w1.is_same(w1_in)) s.staged1 = w1;
+        if (!w2.is_same(w2_in)) s.staged2 = w2;
+    }
+    return out;
+}
+
+struct Needs {
+    bool x, w1, w2, s;
+};
+
+// The router's side of the path from x to the loss, for a caller that owns it (the layer node): its gradient of x is added
+// inside the dX combine, and where the one-launch backward applies its kernels ride in that launch.
+struct RouterTail {
+    Tensor w_r, logits, weights, indices, counts, g_prob_mean, g_z_loss, g_load_balance;
+    bool normalize;
+    Tensor dx_r, dw_r;   // results
+};
+
+struct ExpertGrads {
+    Tensor dx, dw1, dw2, ds;
+};
+
+void router_gradient(const Tensor& x, RouterTail& t, const Tensor& ds) {   // dS and the router's loss terms -> dx_r, dW_r
+    const int64_t T = x.size(0), H = x.size(1), E = t.w_r.size(0), K = t.weights.size(1);
+    const bool narrow = x.scalar_type() != at::kFloat;
+    t.dx_r = at::empty_like(x);
+    t.dw_r = at::empty_like(t.w_r);
+    const int64_t ws_bytes = mts_moe_head_bwd_workspace_bytes(T, H, E);
+    Tensor ws = bytes(ws_bytes, x);
+    check(mts_moe_head_bwd(ptr(x), ptr_as<float>(t.w_r), ptr_as<float>(t.logits), ptr_as<float>(t.weights), ptr_as<int32_t>(t.indices),
+                           ptr_as<int32_t>(t.counts), narrow ? nullptr : ptr_as<float>(ds), narrow ? ptr(ds) : nullptr, ptr_as<float>(t.g_prob_mean),
+                           ptr_as<float>(t.g_z_loss), ptr_as<float>(t.g_load_balance), T, H, E, K, t.normalize, dtype_code(x), ptr(t.dx_r),
+                           ptr_as<float>(t.dw_r), ptr(ws), ws_bytes, stream_of(x)),
+          "mts_moe_head_bwd");
+}
+
+ExpertGrads experts_backward(const Saved& s, Tensor dO, const Needs& need, const Options& opt, RouterTail* tail) {
+    const int64_t T = s.x.size(0), H = s.x.size(1), E = s.w1.size(0), I = s.w1.size(1) / 2, TK = s.weights.numel(), K = TK / T;
+    const auto dtype = s.x.scalar_type();
+    const int act = dtype_code(dtype);
+    dO = dO.to(dtype).contiguous();
+    const int device = s.x.device().index();
+    const hipStream_t main = (hipStream_t)stream_of(s.x);
+    const bool overlap = opt.on(OVERLAP);
+    auto side = [&](int i) { return overlap ? side_stream(device, i) : main; };
+    ExpertGrads g;
+
+    // The ring kernels (16-bit types, widths of whole 64-wide k-tiles or of at least 256) and the fp32 kernels read the
+    // weights in their stored layout; other contracts get transposed copies, W1's made on a side stream next to the dO*W2 GEMM.
+    const int layout = stored_layout(act, H, I);
+    hipStream_t side0 = main;
+    Tensor w1_bwd, w2_bwd;
+    if (need.x) {
+        if (layout) w1_bwd = s.staged1.defined() ? s.staged1 : stage(s.w1, false, dtype, main);
+        else {
+            side0 = side(0);
+            order_after(side0, main);
+            w1_bwd = stage(s.w1, true, dtype, side0);
+        }
+    }
+    w2_bwd = layout && s.staged2.defined() ? s.staged2 : stage(s.w2, !layout, dtype, main);
+
+    const bool weighted = s.post_act.defined();
+    Tensor d_pre_act = at::empty({TK, 2 * I}, s.x.options());
+    Tensor weighted_act = weighted ? s.post_act : at::empty({TK, I}, s.x.options());   // s * silu(g) * u
+    Tensor ds_part = f32({TK, mts_moe_ds_partials(I)}, s.x);
+    // When every gradient is wanted, dW1, dW2, dX and the dS reduction go out as ONE launch whose block order starts the long
+    // weight-gradient tiles first; which XCD runs which of its units and dX tiles follows a table that the dO * W2 launch
+    // writes on the side (uneven routing).
+    const bool joint = opt.on(JOINT_BWD) && need.x && need.w1 && need.w2 && need.s && layout && s.w1.scalar_type() == s.w2.scalar_type() &&
+                       mts_moe_bwd_joint_supported(act, H, I);
+    auto dw_workspace = [&](int which, bool wanted) {
+        const int64_t n = wanted && dtype != at::kFloat ? mts_moe_bwd_dw_workspace_bytes(which, E, H, I) : 0;
+        return n > 0 && n <= opt.dw_workspace_limit ? at::empty({n}, s.x.options().dtype(at::kByte)) : Tensor();
+    };
+    Tensor ws1 = dw_workspace(1, need.w1), ws2 = dw_workspace(2, need.w2), schedule;
+    const int64_t ws1_bytes = ws1.defined() ? ws1.numel() : 0, ws2_bytes = ws2.defined() ? ws2.numel() : 0;
+    if (joint && opt.on(JOINT_SCHEDULE) && ws1.defined() && ws2.defined() && mts_moe_bwd_schedule_bytes(E) > 0)
+        schedule = i32({mts_moe_bwd_schedule_bytes(E) / 4}, s.x);
+    check(mts_moe_bwd_dy1(ptr(dO), ptr(w2_bwd), layout, ptr(s.pre_act), ptr(s.weights), ptr_as<int32_t>(s.x_gather), ptr_as<int32_t>(s.s_scatter),
+                          ptr_as<int32_t>(s.expert_start), T, K, E, H, I, act, ptr(d_pre_act), weighted ? nullptr : ptr(weighted_act),
+                          ptr_as<float>(ds_part), ptr_as<int32_t>(schedule), main),
+          "mts_moe_bwd_dy1");
+
+    Tensor dx_expanded;
+    auto combine_dx = [&]() {
+        if (tail && !tail->dx_r.defined()) router_gradient(s.x, *tail, g.ds);
+        g.dx = at::empty({T, H}, s.x.options());
+        check(mts_moe_combine(ptr(dx_expanded), nullptr, tail ? ptr(tail->dx_r) : nullptr, ptr_as<int32_t>(s.s_reverse), T, K, H, act, ptr(g.dx), main),
+              "mts_moe_combine");
+    };
+
+    if (joint) {
+        g.dw1 = at::empty_like(s.w1);
+        g.dw2 = at::empty_like(s.w2);
+        g.ds = at::empty({T, K}, s.weights.options());
+        dx_expanded = at::empty({TK, H}, s.x.options());
+        const int grad = dtype_code(s.w1);
+        if (tail && opt.on(TAIL_IN_JOINT) && mts_moe_bwd_joint_router_supported(act, T, H, I, E)) {
+            // the router's backward as trailing blocks of the same launch: it needs nothing the launch writes
+            tail->dx_r = at::empty_like(s.x);
+            tail->dw_r = at::empty_like(tail->w_r);
+            if (opt.on(COMBINE_IN_TAIL)) g.dx = at::empty_like(s.x);
+            const int64_t ws_bytes = mts_moe_head_bwd_workspace_bytes(T, H, E);
+            Tensor ws = bytes(ws_bytes, s.x);
+            check(mts_moe_bwd_joint_router(ptr(dO), ptr(weighted_act), ptr(d_pre_act), ptr(s.x), ptr(w1_bwd), ptr_as<int32_t>(s.x_gather),
+                                           ptr_as<int32_t>(s.expert_start), ptr_as<int32_t>(s.s_reverse), ptr_as<float>(ds_part), T, K, E, H, I, act, grad,
+                                           ptr(dx_expanded), ptr(g.dw1), ptr(g.dw2), ptr(g.ds), ptr(ws1), ws1_bytes, ptr(ws2), ws2_bytes,
+                                           ptr_as<float>(tail->w_r), ptr_as<float>(tail->logits), ptr_as<float>(tail->weights),
+                                           ptr_as<int32_t>(tail->indices), ptr_as<int32_t>(tail->counts), ptr_as<float>(tail->g_prob_mean),
+                                           ptr_as<float>(tail->g_z_loss), ptr_as<float>(tail->g_load_balance), tail->normalize, ptr(tail->dx_r), ptr(g.dx),
+                                           ptr_as<float>(tail->dw_r), ptr(ws), ws_bytes, ptr_as<int32_t>(schedule), main),
+                  "mts_moe_bwd_joint_router");
+            if (!g.dx.defined()) combine_dx();
+            return g;
+        }
+        check(mts_moe_bwd_joint(ptr(dO), ptr(weighted_act), ptr(d_pre_act), ptr(s.x), ptr(w1_bwd), ptr_as<int32_t>(s.x_gather),
+                                ptr_as<int32_t>(s.expert_start), ptr_as<int32_t>(s.s_reverse), ptr_as<float>(ds_part), T, K, E, H, I, act, grad,
+                                ptr(dx_expanded), ptr(g.dw1), ptr(g.dw2), ptr(g.ds), ptr(ws1), ws1_bytes, ptr(ws2), ws2_bytes, ptr_as<int32_t>(schedule), main),
+              "mts_moe_bwd_joint");
+        combine_dx();
+        return g;
+    }
+
+    // dW2, dW1 and dX side by side: the two weight-gradient GEMMs have fewer tiles than the chip has CUs
+    const hipStream_t s0 = need.w2 ? side(0) : main, s1 = need.w1 ? side(1) : main;
+    if (need.w2) order_after(s0, main);
+    if (need.w1) order_after(s1, main);
+    // The routing-weight gradient is needed after the join only: it leads one of the side streams (when there is one) so that
+    // dX follows the dO*W2 GEMM directly on the caller's stream; the router's gradient wants it on the caller's stream.
+    if (need.s) {
+        g.ds = at::empty({T, K}, s.weights.options());
+        check(mts_moe_bwd_ds(ptr_as<float>(ds_part), ptr_as<int32_t>(s.s_reverse), TK, I, act, ptr(g.ds), tail ? main : (need.w2 ? s0 : s1)), "mts_moe_bwd_ds");
+    }
+    if (need.w2) {
+        g.dw2 = at::empty_like(s.w2);
+        check(mts_moe_bwd_dw2(ptr(dO), ptr(weighted_act), ptr_as<int32_t>(s.x_gather), ptr_as<int32_t>(s.expert_start), T, K, E, H, I, act,
+                              dtype_code(s.w2), ptr(g.dw2), ptr(ws2), ws2_bytes, s0),
+              "mts_moe_bwd_dw2");
+    }
+    if (need.w1) {
+        g.dw1 = at::empty_like(s.w1);
+        check(mts_moe_bwd_dw1(ptr(d_pre_act), ptr(s.x), ptr_as<int32_t>(s.x_gather), ptr_as<int32_t>(s.expert_start), T, K, E, H, I, act,
+                              dtype_code(s.w1), ptr(g.dw1), ptr(ws1), ws1_bytes, s1),
+              "mts_moe_bwd_dw1");
+    }
+    if (need.x) {
+        if (!layout) order_after(main, side0);   // W1's transposed copy
+        dx_expanded = at::empty({TK, H}, s.x.options());
+        check(mts_moe_bwd_dx(ptr(d_pre_act), ptr(w1_bwd), layout, ptr_as<int32_t>(s.expert_start), TK, E, H, I, act, ptr(dx_expanded), main), "mts_moe_bwd_dx");
+        combine_dx();
+    }
+    // joined before any tensor that the side streams read is released
+    order_after(main, s0);
+    order_after(main, s1);
+    if (need.x && !layout) order_after(main, side0);
+    return g;
+}
+
+// ---- autograd nodes ------------------------------------------------------------------------------------------------------------
+
+struct FusedMoE : torch::autograd::Function<FusedMoE> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& x_, const Tensor& w1_, const Tensor& w2_, const Tensor& index_, const Tensor& weights_,
+                          int64_t switches, int64_t limit) {
+        const Options opt{switches, limit};
+        const Tensor x = x_.contiguous(), w1 = w1_.contiguous(), w2 = w2_.contiguous(), index = index_.contiguous();
+        Saved s;
+        Tensor out = experts_forward(x, w1, w2, weights_.contiguous().view(-1), route(index, w1.size(0)), opt, s);
+        variable_list keep;
+        s.append_to(keep);
+        ctx->save_for_backward(std::move(keep));
+        ctx->saved_data["options"] = std::vector<int64_t>{switches, limit};
+        ctx->set_materialize_grads(false);
+        return out;
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        variable_list result(7);
+        if (!grads[0].defined()) return result;
+        const auto opt = ctx->saved_data["options"].toIntVector();
+        const Saved s(ctx->get_saved_variables());
+        c10::OptionalDeviceGuard guard(s.x.device());
+        const ExpertGrads g = experts_backward(s, grads[0], {ctx->needs_input_grad(0), ctx->needs_input_grad(1), ctx->needs_input_grad(2), ctx->needs_input_grad(4)},
+                                               {opt[0], opt[1]}, nullptr);
+        result[0] = g.dx, result[1] = g.dw1, result[2] = g.dw2, result[4] = g.ds;
+        return result;
+    }
+};
+
+// The whole MoE layer (router projection, post-process, routing metadata, experts, combine) as one node.
+struct MoELayer : torch::autograd::Function<MoELayer> {
+    static variable_list forward(AutogradContext* ctx, const Tensor& x_, const Tensor& w_r_, const Tensor& w1_, const Tensor& w2_, int64_t K, bool normalize,
+                                 int64_t switches, int64_t limit) {
+        const Options opt{switches, limit};
+        const Tensor x = x_.contiguous(), w_r = w_r_.contiguous(), w1 = w1_.contiguous(), w2 = w2_.contiguous();
+        const int64_t T = x.size(0), H = x.size(1), E = w_r.size(0), TK = T * K;
+        const bool narrow = x.scalar_type() != at::kFloat;
+        Tensor logits = f32({T, E}, x), weights = f32({T, K}, x), indices = i32({T, K}, x);
+        Tensor weights_act = narrow ? at::empty({T, K}, x.options()) : weights;
+        Tensor stats = f32({2 * E + 10}, x);   // E mean probabilities, z, entropy, load-balancing term, E + 7 load statistics
+        Tensor prob_mean = stats.narrow(0, 0, E), z_loss = stats.select(0, E), entropy = stats.select(0, E + 1), load_balance = stats.select(0, E + 2),
+               load_stats = stats.narrow(0, E + 3, E + 7);
+        // counts, expert_start and the three permutation arrays in one allocation, each 16-byte aligned
+        const int64_t o1 = round4(E), o2 = o1 + round4(E + 1);
+        Tensor meta = i32({o2 + 3 * round4(TK)}, x);
+        Tensor counts = meta.narrow(0, 0, E);
+        Routing r;
+        r.expert_start = meta.narrow(0, o1, E + 1);
+        r.s_scatter = meta.narrow(0, o2, TK);
+        r.s_reverse = meta.narrow(0, o2 + round4(TK), TK);
+        r.x_gather = meta.narrow(0, o2 + 2 * round4(TK), TK);
+        const int64_t ws_bytes = mts_moe_head_workspace_bytes(T, K, E);
+        Tensor ws = bytes(ws_bytes, x);
+        check(mts_moe_head_fwd(ptr(x), ptr_as<float>(w_r), T, H, E, K, normalize, dtype_code(x), ptr_as<float>(logits), ptr_as<float>(weights),
+                               ptr_as<int32_t>(indices), narrow ? ptr(weights_act) : nullptr, ptr_as<float>(prob_mean), ptr_as<float>(z_loss),
+                               ptr_as<float>(entropy), ptr_as<int32_t>(counts), ptr_as<float>(load_balance), ptr_as<float>(load_stats),
+                               ptr_as<int32_t>(r.expert_start), ptr_as<int32_t>(r.s_scatter), ptr_as<int32_t>(r.s_reverse), ptr_as<int32_t>(r.x_gather),
+                               ptr(ws), ws_bytes, stream_of(x)),
+              "mts_moe_head_fwd");
+        Saved s;
+        Tensor out = experts_forward(x, w1, w2, weights_act.view(-1), r, opt, s);
+        variable_list keep;
+        s.append_to(keep);
+        keep.insert(keep.end(), {w_r, logits, weights, indices, counts});
+        ctx->save_for_backward(std::move(keep));
+        ctx->saved_data["options"] = std::vector<int64_t>{switches, limit, normalize};
+        ctx->mark_non_differentiable({entropy, counts, load_stats, indices, weights});
+        ctx->set_materialize_grads(false);
+        return {out, load_balance, z_loss, prob_mean, entropy, counts, load_stats, indices, weights};
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        const auto o = ctx->saved_data["options"].toIntVector();
+        const variable_list saved = ctx->get_saved_variables();
+        const Saved s(saved);
+        const Tensor* router = &saved[Saved::kCount];
+        c10::OptionalDeviceGuard guard(s.x.device());
+        RouterTail tail{router[0], router[1], router[2], router[3], router[4], like_f32(grads[3]), like_f32(grads[2]), like_f32(grads[1]), o[2] != 0, {}, {}};
+        const bool need_x = ctx->needs_input_grad(0), need_wr = ctx->needs_input_grad(1);
+        const bool wants_router = need_x || need_wr;
+        variable_list result(8);
+        if (grads[0].defined()) {
+            const ExpertGrads g = experts_backward(s, grads[0], {need_x, ctx->needs_input_grad(2), ctx->needs_input_grad(3), wants_router}, {o[0], o[1]},
+                                                   wants_router ? &tail : nullptr);
+            if (wants_router && !tail.dw_r.defined()) router_gradient(s.x, tail, g.ds);   // x needs no gradient: no dX combine
+            result[0] = g.dx, result[2] = g.dw1, result[3] = g.dw2;
+        } else if (wants_router) {   // only the router's loss terms reach this layer
+            router_gradient(s.x, tail, Tensor());
+            if (need_x) result[0] = tail.dx_r;
+        }
+        if (need_wr) result[1] = tail.dw_r;
+        return result;
+    }
+};
+
+struct RouterPostprocess : torch::autograd::Function<RouterPostprocess> {
+    static variable_list forward(AutogradContext* ctx, const Tensor& logits_, int64_t K, bool normalize, int64_t act_dtype) {
+        const Tensor logits = logits_.contiguous();
+        const int64_t T = logits.size(0), E = logits.size(1);
+        const bool cast = act_dtype >= 0;
+        Tensor weights = f32({T, K}, logits), indices = i32({T, K}, logits), counts = i32({E}, logits);
+        Tensor stats = f32({2 * E + 10}, logits);   // E + 3 statistics, E + 7 load statistics
+        Tensor prob_mean = stats.narrow(0, 0, E), z_loss = stats.select(0, E), entropy = stats.select(0, E + 1), load_balance = stats.select(0, E + 2),
+               load_stats = stats.narrow(0, E + 3, E + 7);
+        // the copy of the weights in the activation dtype, written by the same kernel (what the router module otherwise makes
+        // with tensor.to(): one launch forward, one backward)
+        Tensor weights_act;
+        if (cast) weights_act = at::empty({T, K}, logits.options().dtype(act_dtype == MTS_BF16 ? at::kBFloat16 : at::kHalf));
+        const int64_t ws_bytes = mts_router_workspace_bytes(T, E);
+        Tensor ws = bytes(ws_bytes, logits);
+        check(mts_router_fwd(ptr_as<float>(logits), T, E, K, normalize, ptr_as<float>(weights), ptr_as<int32_t>(indices), ptr_as<float>(prob_mean),
+                             ptr_as<float>(z_loss), ptr_as<float>(entropy), ptr_as<int32_t>(counts), ptr_as<float>(load_balance), ptr_as<float>(load_stats),
+                             ptr(weights_act), cast ? (int)act_dtype : 0, ptr(ws), ws_bytes, stream_of(logits)),
+              "mts_router_fwd");
+        ctx->save_for_backward({logits, weights, indices, counts});
+        ctx->saved_data["options"] = std::vector<int64_t>{K, normalize, cast ? act_dtype : 0};
+        ctx->mark_non_differentiable({indices, entropy, counts, load_stats});
+        ctx->set_materialize_grads(false);   // no zero tensors for the outputs that took no part in the loss
+        variable_list out{weights, indices, prob_mean, z_loss, entropy, counts, load_balance, load_stats};
+        if (cast) out.push_back(weights_act);
+        return out;
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        const variable_list s = ctx->get_saved_variables();
+        const auto o = ctx->saved_data["options"].toIntVector();
+        c10::OptionalDeviceGuard guard(s[0].device());
+        const Tensor g_w = like_f32(grads[0]), g_p = like_f32(grads[2]), g_z = like_f32(grads[3]), g_lb = like_f32(grads[6]);
+        const Tensor g_act = grads.size() > 8 && grads[8].defined() ? grads[8].contiguous() : Tensor();   // stays in the activation dtype
+        Tensor g_logits = at::empty_like(s[0]);
+        check(mts_router_bwd(ptr_as<float>(s[0]), ptr_as<float>(s[1]), ptr_as<int32_t>(s[2]), ptr_as<float>(g_w), ptr(g_act), (int)o[2], ptr_as<float>(g_p),
+                             ptr_as<float>(g_z), ptr_as<float>(g_lb), ptr_as<int32_t>(s[3]), s[0].size(0), s[0].size(1), o[0], o[1], ptr_as<float>(g_logits),
+                             stream_of(s[0])),
+              "mts_router_bwd");
+        return {g_logits, Tensor(), Tensor(), Tensor()};
+    }
+};
+
+// logits = float(x) @ W_r^T without the fp32 copy of x; backward gives dx in x's dtype.
+struct RouterLogits : torch::autograd::Function<RouterLogits> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& x_, const Tensor& w_) {
+        const Tensor x = x_.contiguous(), w = w_.contiguous();
+        Tensor logits = f32({x.size(0), w.size(0)}, x);
+        check(mts_router_logits_fwd(ptr(x), ptr_as<float>(w), x.size(0), x.size(1), w.size(0), dtype_code(x), ptr_as<float>(logits), stream_of(x)),
+              "mts_router_logits_fwd");
+        ctx->save_for_backward({x, w});
+        return logits;
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        const variable_list s = ctx->get_saved_variables();
+        c10::OptionalDeviceGuard guard(s[0].device());
+        const Tensor g = like_f32(grads[0]);
+        Tensor dx = at::empty_like(s[0]), dw = at::empty_like(s[1]);
+        const int64_t T = s[0].size(0), H = s[0].size(1), E = s[1].size(0), ws_bytes = mts_router_logits_bwd_workspace_bytes(T, H, E);
+        Tensor ws = bytes(ws_bytes, s[0]);
+        check(mts_router_logits_bwd(ptr_as<float>(g), ptr(s[0]), ptr_as<float>(s[1]), T, H, E, dtype_code(s[0]), ptr(dx), ptr_as<float>(dw), ptr(ws), ws_bytes,
+                                    stream_of(s[0])),
+              "mts_router_logits_bwd");
+        return {dx, dw};
+    }
+};
+
+// ---- the decoder's dense operators -----------------------------------------------------------------------------------------------
+
+bool rmsnorm_supported(const Tensor& x, const Tensor& w, const MaybeTensor& residual) {
+    if (!(x.is_cuda() && w.is_cuda() && is_activation_type(x.scalar_type()) && w.scalar_type() == at::kFloat && w.dim() == 1 && x.dim() >= 1 &&
+          x.size(-1) == w.size(0) && x.numel() > 0 && mts_rmsnorm_supported(x.size(-1))))
+        return false;
+    return !residual || (residual->is_cuda() && residual->scalar_type() == x.scalar_type() && residual->sizes() == x.sizes());
+}
+
+// y, or (x + residual, y) with a residual
+struct RMSNorm : torch::autograd::Function<RMSNorm> {
+    static variable_list forward(AutogradContext* ctx, const Tensor& x_, const MaybeTensor& residual_, const Tensor& w_, double eps) {
+        const Tensor x = dense16(x_), w = dense16(w_);
+        const int64_t H = x.size(-1), N = x.numel() / H;
+        Tensor residual, total = x, y = at::empty_like(x), rstd = f32({N}, x);
+        if (residual_) {
+            residual = dense16(*residual_);
+            total = at::empty_like(x);
+        }
+        check(mts_rmsnorm_fwd(ptr(x), ptr(residual), ptr_as<float>(w), N, H, eps, dtype_code(x), residual_ ? ptr(total) : nullptr, ptr(y), ptr_as<float>(rstd),
+                              stream_of(x)),
+              "mts_rmsnorm_fwd");
+        ctx->save_for_backward({total, w, rstd});
+        ctx->set_materialize_grads(false);
+        if (residual_) return {total, y};
+        return {y};
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        const variable_list s = ctx->get_saved_variables();
+        const bool with_sum = grads.size() == 2;
+        Tensor g_sum = with_sum ? grads[0] : Tensor(), g_y = grads.back();
+        if (!g_y.defined()) return {g_sum, with_sum ? g_sum : Tensor(), Tensor(), Tensor()};   // only the residual stream goes on
+        c10::OptionalDeviceGuard guard(s[0].device());
+        const int64_t H = s[0].size(-1), N = s[0].numel() / H, ws_bytes = mts_rmsnorm_bwd_workspace_bytes(N, H);
+        g_y = dense16(g_y);
+        if (g_sum.defined()) g_sum = dense16(g_sum);
+        Tensor d_sum = at::empty_like(s[0]), dw = at::empty_like(s[1]), ws = bytes(ws_bytes, s[0]);
+        check(mts_rmsnorm_bwd(ptr(g_y), ptr(g_sum), ptr(s[0]), ptr_as<float>(s[1]), ptr_as<float>(s[2]), N, H, dtype_code(s[0]), ptr(d_sum), ptr_as<float>(dw),
+                              ptr(ws), ws_bytes, stream_of(s[0])),
+              "mts_rmsnorm_bwd");
+        return {d_sum, with_sum ? d_sum : Tensor(), dw, Tensor()};
+    }
+};
+
+enum RopeMode { TURN = 0, TURN_BACK = 1, COPY = 2 };
+
+bool rope_table_fits(const Tensor& t, const Tensor& like, int64_t S, int64_t D) {
+    return t.is_cuda() && t.scalar_type() == like.scalar_type() && t.dim() == 2 && t.size(0) == S && t.size(1) == D && t.is_contiguous() && !t.requires_grad();
+}
+bool rope_supported(const Tensor& q, const Tensor& k, const Tensor& cos, const Tensor& sin) {
+    if (!(q.is_cuda() && k.is_cuda() && q.dim() == 4 && q.sizes() == k.sizes() && q.scalar_type() == k.scalar_type() && is_activation_type(q.scalar_type()) &&
+          q.numel() > 0))
+        return false;
+    const int64_t S = q.size(2), D = q.size(3);
+    return D % 2 == 0 && q.size(0) * S < k2GiB && rope_table_fits(cos, q, S, D) && rope_table_fits(sin, q, S, D);
+}
+bool qkv_rope_supported(const Tensor& qkv, const Tensor& cos, const Tensor& sin, int64_t heads) {
+    if (!(qkv.is_cuda() && qkv.dim() == 3 && is_activation_type(qkv.scalar_type()) && qkv.numel() > 0 && qkv.size(2) % (3 * heads) == 0)) return false;
+    const int64_t S = qkv.size(1), D = qkv.size(2) / (3 * heads);
+    return D % 2 == 0 && qkv.size(0) * S < k2GiB && rope_table_fits(cos, qkv, S, D) && rope_table_fits(sin, qkv, S, D);
+}
+
+struct RopeJob {
+    Tensor in, out;   // [B, heads, S, D], any strides but a dense last dimension
+    int mode;
+};
+void launch_rope(const std::vector<RopeJob>& jobs, const Tensor& cos, const Tensor& sin) {
+    MtsRopeTensor array[3];
+    for (size_t i = 0; i < jobs.size(); ++i) {
+        const Tensor &a = jobs[i].in, &b = jobs[i].out;
+        array[i] = {ptr(a), ptr(b), a.stride(0), a.stride(2), a.stride(1), b.stride(0), b.stride(2), b.stride(1), jobs[i].mode};
+    }
+    const Tensor& t = jobs[0].in;
+    check(mts_rope(array, (int)jobs.size(), ptr(cos), ptr(sin), t.size(0), t.size(2), t.size(1), t.size(3), dtype_code(t), stream_of(t)), "mts_rope");
+}
+Tensor dense_rows(const Tensor& t) { return t.stride(-1) == 1 ? t : t.contiguous(); }
+// [B, S, heads, D] in memory, as the projection that queries and keys are views of
+Tensor heads_inside(const Tensor& like, int64_t B, int64_t heads, int64_t S, int64_t D) { return at::empty({B, S, heads, D}, like.options()).transpose(1, 2); }
+
+struct Rope : torch::autograd::Function<Rope> {
+    static variable_list turn(const Tensor& q_, const Tensor& k_, const Tensor& cos, const Tensor& sin, int mode) {
+        const Tensor q = dense_rows(q_), k = dense_rows(k_);
+        Tensor a = heads_inside(q, q.size(0), q.size(1), q.size(2), q.size(3)), b = heads_inside(q, q.size(0), q.size(1), q.size(2), q.size(3));
+        launch_rope({{q, a, mode}, {k, b, mode}}, cos, sin);
+        return {a, b};
+    }
+    static variable_list forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& cos, const Tensor& sin) {
+        ctx->save_for_backward({cos, sin});
+        return turn(q, k, cos, sin, TURN);
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        const variable_list s = ctx->get_saved_variables();
+        c10::OptionalDeviceGuard guard(s[0].device());
+        const variable_list g = turn(grads[0], grads[1], s[0], s[1], TURN_BACK);
+        return {g[0], g[1], Tensor(), Tensor()};
+    }
+};
+
+// Packed projection [B, S, 3 * heads * D] to rotated queries, rotated keys and values [B, heads, S, D].  The values stay where
+// they are; the backward launch writes the gradient of the projection in one piece.
+struct QkvRope : torch::autograd::Function<QkvRope> {
+    static variable_list forward(AutogradContext* ctx, const Tensor& qkv_, const Tensor& cos, const Tensor& sin, int64_t heads) {
+        const Tensor qkv = qkv_.contiguous();
+        const int64_t B = qkv.size(0), S = qkv.size(1), D = qkv.size(2) / (3 * heads);
+        const Tensor parts = qkv.view({B, S, 3, heads, D});
+        Tensor q = heads_inside(qkv, B, heads, S, D), k = heads_inside(qkv, B, heads, S, D);
+        launch_rope({{parts.select(2, 0).transpose(1, 2), q, TURN}, {parts.select(2, 1).transpose(1, 2), k, TURN}}, cos, sin);
+        ctx->save_for_backward({cos, sin});
+        ctx->saved_data["heads"] = heads;
+        ctx->set_materialize_grads(false);
+        return {q, k, parts.select(2, 2).transpose(1, 2)};
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        const variable_list s = ctx->get_saved_variables();
+        const Tensor* first = nullptr;
+        int given = 0;
+        for (const Tensor& g : grads)
+            if (g.defined()) {
+                ++given;
+                first = &g;
+            }
+        if (!first) return variable_list(4);
+        c10::OptionalDeviceGuard guard(s[0].device());
+        const int64_t B = first->size(0), heads = first->size(1), S = first->size(2), D = first->size(3);
+        // zeros where a part took no part in the loss
+        Tensor out = given == 3 ? at::empty({B, S, 3, heads, D}, first->options()) : at::zeros({B, S, 3, heads, D}, first->options());
+        std::vector<RopeJob> jobs;
+        for (int i = 0; i < 3; ++i)
+            if (grads[i].defined()) jobs.push_back({dense_rows(grads[i]), out.select(2, i).transpose(1, 2), i < 2 ? TURN_BACK : COPY});
+        launch_rope(jobs, s[0], s[1]);
+        return {out.view({B, S, 3 * heads * D}), Tensor(), Tensor(), Tensor()};
+    }
+};
+
+constexpr int64_t kIgnoreIndex = -100;   // torch's default
+
+bool cross_entropy_supported(const Tensor& logits, const Tensor& targets) {
+    return logits.is_cuda() && targets.is_cuda() && logits.dim() == 2 && targets.dim() == 1 && is_activation_type(logits.scalar_type()) &&
+           targets.scalar_type() == at::kLong && logits.size(0) == targets.size(0) && logits.size(0) > 0 && logits.size(0) < k2GiB && logits.size(1) > 0 &&
+           logits.size(1) < k2GiB;
+}
+
+// mean cross-entropy without an fp32 copy of the logits
+struct CrossEntropy : torch::autograd::Function<CrossEntropy> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& logits_, const Tensor& targets_) {
+        const Tensor logits = dense16(logits_), targets = targets_.contiguous();
+        const int64_t N = logits.size(0), V = logits.size(1);
+        Tensor rows = f32({3, N}, logits), scalars = f32({2}, logits);   // per row: maximum, log of the sum, loss; loss, 1 / count
+        float* row = ptr_as<float>(rows);
+        float* scalar = ptr_as<float>(scalars);
+        check(mts_cross_entropy_fwd(ptr(logits), ptr_as<int64_t>(targets), N, V, kIgnoreIndex, dtype_code(logits), row, row + N, row + 2 * N, scalar, scalar + 1,
+                                    stream_of(logits)),
+              "mts_cross_entropy_fwd");
+        ctx->save_for_backward({logits, targets, rows, scalars});
+        return scalars.select(0, 0);
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        const variable_list s = ctx->get_saved_variables();
+        c10::OptionalDeviceGuard guard(s[0].device());
+        const int64_t N = s[0].size(0), V = s[0].size(1);
+        const Tensor g = like_f32(grads[0]);
+        Tensor d = at::empty_like(s[0]);
+        const float* row = ptr_as<float>(s[2]);
+        check(mts_cross_entropy_bwd(ptr(s[0]), ptr_as<int64_t>(s[1]), N, V, kIgnoreIndex, dtype_code(s[0]), row, row + N, ptr_as<float>(g),
+                                    ptr_as<float>(s[3]) + 1, ptr(d), stream_of(s[0])),
+              "mts_cross_entropy_bwd");
+        return {d, Tensor()};
+    }
+};
+
+}  // namespace
+
+PYBIND11_MODULE(_host, m) {
+    namespace py = pybind11;
+    m.def("set_joint_workspace", [](py::object f) { joint_workspace_of = new py::object(std::move(f)); });
+    m.def("fused_moe_violation", &fused_moe_violation);
+    m.def("layer_violation", &layer_violation);
+    m.def("needs_padding", &needs_padding);
+    m.def("router_logits_supported", &router_logits_supported);
+    m.def("route", [](const Tensor& index, int64_t E) {
+        const Routing r = route(index.contiguous(), E);
+        return std::make_tuple(r.expert_start, r.x_gather, r.s_scatter, r.s_reverse);
+    });
+    m.def("fused_moe", [](const Tensor& x, const Tensor& w1, const Tensor& w2, const Tensor& index, const Tensor& weights, int64_t switches, int64_t limit) {
+        c10::OptionalDeviceGuard guard(x.device());
+        return FusedMoE::apply(x, w1, w2, index, weights, switches, limit);
+    });
+    m.def("moe_layer", [](const Tensor& x, const Tensor& w_r, const Tensor& w1, const Tensor& w2, int64_t top_k, bool normalize, int64_t switches, int64_t limit) {
+        c10::OptionalDeviceGuard guard(x.device());
+        const variable_list v = MoELayer::apply(x, w_r, w1, w2, top_k, normalize, switches, limit);
+        return std::make_tuple(v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], v[8]);
+    });
+    m.def("router_postprocess", [](const Tensor& logits, int64_t top_k, bool normalize, int64_t act_dtype) {
+        c10::OptionalDeviceGuard guard(logits.device());
+        return RouterPostprocess::apply(logits, top_k, normalize, act_dtype);
+    });
+    m.def("router_logits", [](const Tensor& x, const Tensor& w) {
+        c10::OptionalDeviceGuard guard(x.device());
+        return RouterLogits::apply(x, w);
+    });
+    m.def("rmsnorm_supported", &rmsnorm_supported);
+    m.def("rmsnorm", [](const Tensor& x, const Tensor& w, double eps) {
+        c10::OptionalDeviceGuard guard(x.device());
+        return RMSNorm::apply(x, MaybeTensor(), w, eps)[0];
+    });
+    m.def("add_rmsnorm", [](const Tensor& x, const Tensor& residual, const Tensor& w, double eps) {
+        c10::OptionalDeviceGuard guard(x.device());
+        const variable_list v = RMSNorm::apply(x, MaybeTensor(residual), w, eps);
+        return std::make_tuple(v[0], v[1]);
+    });
+    m.def("rope_supported", &rope_supported);
+    m.def("rope", [](const Tensor& q, const Tensor& k, const Tensor& cos, const Tensor& sin) {
+        c10::OptionalDeviceGuard guard(q.device());
+        const variable_list v = Rope::apply(q, k, cos, sin);
+        return std::make_tuple(v[0], v[1]);
+    });
+    m.def("qkv_rope_supported", &qkv_rope_supported);
+    m.def("qkv_rope", [](const Tensor& qkv, const Tensor& cos, const Tensor& sin, int64_t heads) {
+        c10::OptionalDeviceGuard guard(qkv.device());
+        const variable_list v = QkvRope::apply(qkv, cos, sin, heads);
+        return std::make_tuple(v[0], v[1], v[2]);
+    });
+    m.def("cross_entropy_supported", &cross_entropy_supported);
+    m.def("cross_entropy", [](const Tensor& logits, const Tensor& targets) {
+        c10::OptionalDeviceGuard guard(logits.device());
+        return CrossEntropy::apply(logits, targets);
+    });
+}

@@ -80,13 +80,9 @@ SIGNATURES = {
 }
 
 
-class RopeTensor(_c.Structure):
-    """``MtsRopeTensor``"""
-
-    _fields_ = [("input", _p), ("output", _p), ("in_b", _l), ("in_s", _l), ("in_h", _l), ("out_b", _l), ("out_s", _l), ("out_h", _l), ("mode", _i)]
-
-
 _lib = None
+_host = None
+_joint_workspace = None
 _lock = threading.Lock()
 
 
@@ -113,6 +109,30 @@ def load():
                 fn.argtypes = args
             _lib = lib
     return _lib
+
+
+def host():
+    """The native host path (``csrc/host/mts_host.cpp``): contract checks, allocations and autograd nodes."""
+    global _host
+    if _host is None:
+        load()
+        try:
+            from minitrain_amd.lib import _host as module
+        except ImportError as err:
+            raise MtsError(f"lib/_host.so does not load ({err}): build it with `python -m minitrain_amd.build` "
+                           "(there is no fallback for the hip backend)") from err
+        if _joint_workspace is not None:
+            module.set_joint_workspace(_joint_workspace)
+        _host = module
+    return _host
+
+
+def set_joint_workspace(provider) -> None:
+    """``provider(device_index)``: the counters of the joint gate/up + down launch on the current stream of a device."""
+    global _joint_workspace
+    _joint_workspace = provider
+    if _host is not None:
+        _host.set_joint_workspace(provider)
 
 
 def check(code: int, what: str) -> None:

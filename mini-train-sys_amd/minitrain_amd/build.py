@@ -1,6 +1,7 @@
-"""Compile the gfx950 HIP sources into ``lib/libmts_moe.so`` with hipcc.
+"""Compile the gfx950 HIP sources into ``lib/libmts_moe.so`` with hipcc, and the host path in front of them
+(``csrc/host``, against torch's C++ interface) into ``lib/_host.so`` with the host compiler.
 
-``python -m minitrain_amd.build`` (or ``build_library()``) always recompiles.  The
+``python -m minitrain_amd.build`` (or ``build_library()``) always recompiles both.  The
 library is linked against the HIP runtime by soname only, with no run path, so a
 process that has already imported torch resolves it to the runtime torch loaded.
 """
@@ -12,6 +13,7 @@ import re
 import shutil
 import subprocess
 import sys
+import sysconfig
 import tempfile
 
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
@@ -19,6 +21,8 @@ CSRC = os.path.join(os.path.dirname(PKG_DIR), "csrc")
 INCLUDE = os.path.join(os.path.dirname(os.path.dirname(PKG_DIR)), "include")
 LIB_DIR = os.path.join(PKG_DIR, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libmts_moe.so")
+HOST_SOURCE = os.path.join(CSRC, "host", "mts_host.cpp")
+HOST_PATH = os.path.join(LIB_DIR, "_host.so")
 SOURCES = ("mts_router.hip", "mts_router_linear.hip", "mts_route.hip", "mts_capacity.hip", "mts_combine.hip", "mts_dense.hip", "mts_gemm.hip", "mts_gemm_f16.hip", "mts_gemm_f32.hip", "mts_probe.hip", "mts_tuning.hip")
 
 FLAGS = [
@@ -40,6 +44,25 @@ def find_hipcc() -> str:
     raise RuntimeError("hipcc not found; set HIPCC or install ROCm")
 
 
+def host_compile_command(obj: str) -> list[str]:
+    import torch
+
+    root = os.path.dirname(torch.__file__)
+    includes = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"), "/opt/rocm/include",
+                sysconfig.get_paths()["include"]]
+    return [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{INCLUDE}",
+            *[a for i in includes for a in ("-isystem", i)], "-c", HOST_SOURCE, "-o", obj]
+
+
+def host_link_command(obj: str, out: str) -> list[str]:
+    import torch
+
+    # the kernel library is found beside the module; torch's libraries are in the process before either is opened
+    return [os.environ.get("CXX", "g++"), "-shared", obj, "-o", out, f"-L{os.path.join(os.path.dirname(torch.__file__), 'lib')}", "-ltorch",
+            "-ltorch_cpu", "-ltorch_hip", "-ltorch_python", "-lc10", "-lc10_hip", f"-L{LIB_DIR}", "-lmts_moe", "-Wl,-rpath,$ORIGIN"]
+
+
 def build_library(verbose: bool = False, resource_report: bool = False, out: str | None = None,
                   defines: tuple = ()) -> str:
     """Compile every source (one hipcc process each, side by side) and link the shared library."""
@@ -52,6 +75,10 @@ def build_library(verbose: bool = False, resource_report: bool = False, out: str
         if resource_report:
             base.append("-Rpass-analysis=kernel-resource-usage")
         procs = []
+        # with another output path (a variant of the kernels) the host path stays as it is
+        host_obj = os.path.join(objdir, "mts_host.o") if out == LIB_PATH else None
+        if host_obj:
+            procs.append((host_obj, subprocess.Popen(host_compile_command(host_obj), stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True)))
         for src in SOURCES:
             obj = os.path.join(objdir, src.replace(".hip", ".o"))
             procs.append((obj, subprocess.Popen(base + ["-c", os.path.join(CSRC, src), "-o", obj],
@@ -67,15 +94,20 @@ def build_library(verbose: bool = False, resource_report: bool = False, out: str
             _, err = proc.communicate()
             stderr += err
             if proc.returncode != 0:
-                failure = f"hipcc failed ({proc.returncode}):\n{_quiet(err)}"
+                failure = f"compiling failed ({proc.returncode}):\n{_quiet(err)}"
         if failure is not None:
             raise RuntimeError(failure)
         tmp = out + ".tmp"
-        link = subprocess.run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", *[o for o, _ in procs], "-o", tmp],
-                              capture_output=True, text=True)
+        link = subprocess.run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", *[o for o, _ in procs if o != host_obj],
+                               "-o", tmp], capture_output=True, text=True)
         if link.returncode != 0:
             raise RuntimeError(f"link failed ({link.returncode}):\n{_quiet(link.stderr)}")
         os.replace(tmp, out)
+        if host_obj:
+            link = subprocess.run(host_link_command(host_obj, HOST_PATH + ".tmp"), capture_output=True, text=True)
+            if link.returncode != 0:
+                raise RuntimeError(f"link of the host path failed ({link.returncode}):\n{link.stderr}")
+            os.replace(HOST_PATH + ".tmp", HOST_PATH)
     finally:
         shutil.rmtree(objdir, ignore_errors=True)
     if resource_report:

@@ -11,7 +11,7 @@ from minitrain_amd.kernels.dense_ops import DenseTorchOps
 from minitrain_amd.kernels.hip import dense
 from minitrain_amd.kernels.hip.capacity import capacity_mask, is_capacity_mask_supported
 from minitrain_amd.kernels.hip.fused_moe import expert_counts, fused_moe, is_fused_moe_supported
-from minitrain_amd.kernels.hip.moe_layer import moe_layer, moe_layer_violation
+from minitrain_amd.kernels.hip.moe_layer import moe_layer, moe_layer_violation, run_moe_layer
 from minitrain_amd.kernels.hip.switches import SWITCHES
 from minitrain_amd.kernels.hip.router import (
     is_router_logits_supported,
@@ -93,7 +93,7 @@ class HipOpsBackend(DenseTorchOps):
         caller then composes the layer from ``router_postprocess`` and ``fused_moe``."""
         if not self.offers_moe_layer or moe_layer_violation(x, router_weight, gate_up_proj, down_proj, top_k) is not None:
             return None
-        return moe_layer(x, router_weight, gate_up_proj, down_proj, top_k, normalize=normalize)
+        return run_moe_layer(x, router_weight, gate_up_proj, down_proj, top_k, normalize)
 
     def router_logits(self, hidden_states, weight):
         """Extension beyond the reference's operator interface: the router projection in fp32

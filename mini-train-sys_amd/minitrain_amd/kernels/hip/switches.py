@@ -41,6 +41,11 @@ class Switches:
     router_cast: bool
     layer_node: bool
 
+    def mask(self) -> int:
+        """The fields that the native host path reads, as its bit mask (``Switch`` in csrc/host/mts_host.cpp)."""
+        return (self.overlap | self.joint_bwd << 1 | self.joint_fwd << 2 | self.tail_in_joint << 3 | self.combine_in_tail << 4
+                | self.joint_schedule << 5 | self.weighted_post << 6)
+
 
 SWITCHES = Switches(
     overlap=not _off("MTS_NO_OVERLAP"),
