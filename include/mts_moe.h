@@ -194,6 +194,30 @@ int mts_moe_capacity_mask(const int32_t* top_k_index, const float* top_k_weights
                           int32_t* accepted_counts, void* workspace, int64_t workspace_bytes,
                           void* stream);
 
+/* The same selection for routes that already have a permutation (counts, expert_start and s_scatter of
+ * mts_moe_head_fwd or mts_moe_route, every route in it): the compacted permutation of the kept routes in
+ * one launch, as mts_moe_route would make it of the kept_index above.  kept_reverse is -1 for a dropped
+ * route, kept_start[E] the number of kept routes.                                              */
+int64_t mts_moe_capacity_compact_workspace_bytes(int64_t T, int K);
+int mts_moe_capacity_compact(const float* top_k_weights, const int32_t* counts,
+                             const int32_t* expert_start, const int32_t* s_scatter, int64_t T, int K,
+                             int E, int64_t capacity, int32_t* accepted_counts, int32_t* kept_start,
+                             int32_t* kept_scatter, int32_t* kept_reverse, int32_t* kept_gather,
+                             void* workspace, int64_t workspace_bytes, void* stream);
+
+/* What the router module does with the weights under a capacity limit (minitrain/model/moe_router.py:
+ * 92-110): zero for dropped routes, with `normalize` divided by the sum of a token's kept weights
+ * (weights_out [T,K] in act_dtype), and the load metrics of the accepted routes in the layout of
+ * mts_router_fwd's load_stats.  _bwd: the gradient of weights_out (act_dtype) -> that of
+ * top_k_weights (f32).                                                                         */
+int mts_moe_capacity_weights_fwd(const float* top_k_weights, const int32_t* kept_reverse,
+                                 const int32_t* accepted_counts, const float* entropy, int64_t T, int K,
+                                 int E, int normalize, int act_dtype, void* weights_out,
+                                 float* load_stats, void* stream);
+int mts_moe_capacity_weights_bwd(const void* g_weights, const float* top_k_weights,
+                                 const int32_t* kept_reverse, int64_t T, int K, int normalize,
+                                 int act_dtype, float* g_top_k_weights, void* stream);
+
 /* ---- weight staging -----------------------------------------------------
  * src [E,R,C] of src_dtype -> dst of dst_dtype, [E,R,C] (transpose=0) or [E,C,R]
  * (transpose=1).  Stands in for the in-kernel weight casts of the reference
@@ -377,6 +401,9 @@ int mts_moe_bwd_joint(const void* d_out, const void* weighted_act, const void* d
  * the launch of partial sums (two routes per token) or as one more launch behind it.  mts_moe_bwd_joint_router_supported()
  * says whether the shapes allow it (those of mts_moe_bwd_joint, E <= 8, H a multiple of 4 whose
  * dW_r sums fit the block's LDS).                                                       */
+/* MTS_NORMALIZE_KEPT in `normalize`: the expert weights were those of mts_moe_capacity_weights_fwd (zero for
+ * routes whose s_reverse is negative, renormalised if bit 0 is set too); their gradient is taken back to `weights`. */
+#define MTS_NORMALIZE_KEPT 2
 int mts_moe_bwd_joint_router_supported(int act_dtype, int64_t T, int H, int I, int E);
 int mts_moe_bwd_joint_router(const void* d_out, const void* weighted_act, const void* d_pre_act,
                              const void* x, const void* w1, const int32_t* x_gather,

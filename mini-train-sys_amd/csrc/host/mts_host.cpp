@@ -279,7 +279,8 @@ struct Needs {
 struct RouterTail {
     Tensor w_r, logits, weights, indices, counts, g_prob_mean, g_z_loss, g_load_balance;
     bool normalize;
-    Tensor dx_r, dw_r;   // results
+    Tensor kept_reverse;   // defined: the weights were limited to the routes it gives a row, and renormalised
+    Tensor dx_r, dw_r;     // results
 };
 
 struct ExpertGrads {
@@ -291,10 +292,18 @@ void router_gradient(const Tensor& x, RouterTail& t, const Tensor& ds) {   // dS
     const bool narrow = x.scalar_type() != at::kFloat;
     t.dx_r = at::empty_like(x);
     t.dw_r = at::empty_like(t.w_r);
+    Tensor g_w = narrow ? Tensor() : ds, g_w_act = narrow ? ds : Tensor();
+    if (t.kept_reverse.defined() && ds.defined()) {
+        g_w = at::empty_like(t.weights);
+        g_w_act = Tensor();
+        check(mts_moe_capacity_weights_bwd(ptr(ds), ptr_as<float>(t.weights), ptr_as<int32_t>(t.kept_reverse), T, K, t.normalize, dtype_code(ds),
+                                           ptr_as<float>(g_w), stream_of(x)),
+              "mts_moe_capacity_weights_bwd");
+    }
     const int64_t ws_bytes = mts_moe_head_bwd_workspace_bytes(T, H, E);
     Tensor ws = bytes(ws_bytes, x);
     check(mts_moe_head_bwd(ptr(x), ptr_as<float>(t.w_r), ptr_as<float>(t.logits), ptr_as<float>(t.weights), ptr_as<int32_t>(t.indices),
-                           ptr_as<int32_t>(t.counts), narrow ? nullptr : ptr_as<float>(ds), narrow ? ptr(ds) : nullptr, ptr_as<float>(t.g_prob_mean),
+                           ptr_as<int32_t>(t.counts), ptr_as<float>(g_w), ptr(g_w_act), ptr_as<float>(t.g_prob_mean),
                            ptr_as<float>(t.g_z_loss), ptr_as<float>(t.g_load_balance), T, H, E, K, t.normalize, dtype_code(x), ptr(t.dx_r),
                            ptr_as<float>(t.dw_r), ptr(ws), ws_bytes, stream_of(x)),
           "mts_moe_head_bwd");
@@ -374,7 +383,8 @@ ExpertGrads experts_backward(const Saved& s, Tensor dO, const Needs& need, const
                                            ptr(dx_expanded), ptr(g.dw1), ptr(g.dw2), ptr(g.ds), ptr(ws1), ws1_bytes, ptr(ws2), ws2_bytes,
                                            ptr_as<float>(tail->w_r), ptr_as<float>(tail->logits), ptr_as<float>(tail->weights),
                                            ptr_as<int32_t>(tail->indices), ptr_as<int32_t>(tail->counts), ptr_as<float>(tail->g_prob_mean),
-                                           ptr_as<float>(tail->g_z_loss), ptr_as<float>(tail->g_load_balance), tail->normalize, ptr(tail->dx_r), ptr(g.dx),
+                                           ptr_as<float>(tail->g_z_loss), ptr_as<float>(tail->g_load_balance),
+                                           (tail->normalize ? 1 : 0) | (tail->kept_reverse.defined() ? MTS_NORMALIZE_KEPT : 0), ptr(tail->dx_r), ptr(g.dx),
                                            ptr_as<float>(tail->dw_r), ptr(ws), ws_bytes, ptr_as<int32_t>(schedule), main),
                   "mts_moe_bwd_joint_router");
             if (!g.dx.defined()) combine_dx();
@@ -454,14 +464,15 @@ struct FusedMoE : torch::autograd::Function<FusedMoE> {
 
 // The whole MoE layer (router projection, post-process, routing metadata, experts, combine) as one node.
 struct MoELayer : torch::autograd::Function<MoELayer> {
+    // capacity >= 0: an expert accepts at most that many routes; the others get no row
     static variable_list forward(AutogradContext* ctx, const Tensor& x_, const Tensor& w_r_, const Tensor& w1_, const Tensor& w2_, int64_t K, bool normalize,
-                                 int64_t switches, int64_t limit) {
+                                 int64_t capacity, int64_t switches, int64_t limit) {
         const Options opt{switches, limit};
         const Tensor x = x_.contiguous(), w_r = w_r_.contiguous(), w1 = w1_.contiguous(), w2 = w2_.contiguous();
         const int64_t T = x.size(0), H = x.size(1), E = w_r.size(0), TK = T * K;
-        const bool narrow = x.scalar_type() != at::kFloat;
+        const bool narrow = x.scalar_type() != at::kFloat, limited = capacity >= 0;
         Tensor logits = f32({T, E}, x), weights = f32({T, K}, x), indices = i32({T, K}, x);
-        Tensor weights_act = narrow ? at::empty({T, K}, x.options()) : weights;
+        Tensor weights_act = narrow || limited ? at::empty({T, K}, x.options()) : weights;
         Tensor stats = f32({2 * E + 10}, x);   // E mean probabilities, z, entropy, load-balancing term, E + 7 load statistics
         Tensor prob_mean = stats.narrow(0, 0, E), z_loss = stats.select(0, E), entropy = stats.select(0, E + 1), load_balance = stats.select(0, E + 2),
                load_stats = stats.narrow(0, E + 3, E + 7);
@@ -477,18 +488,35 @@ struct MoELayer : torch::autograd::Function<MoELayer> {
         const int64_t ws_bytes = mts_moe_head_workspace_bytes(T, K, E);
         Tensor ws = bytes(ws_bytes, x);
         check(mts_moe_head_fwd(ptr(x), ptr_as<float>(w_r), T, H, E, K, normalize, dtype_code(x), ptr_as<float>(logits), ptr_as<float>(weights),
-                               ptr_as<int32_t>(indices), narrow ? ptr(weights_act) : nullptr, ptr_as<float>(prob_mean), ptr_as<float>(z_loss),
-                               ptr_as<float>(entropy), ptr_as<int32_t>(counts), ptr_as<float>(load_balance), ptr_as<float>(load_stats),
+                               ptr_as<int32_t>(indices), narrow && !limited ? ptr(weights_act) : nullptr, ptr_as<float>(prob_mean), ptr_as<float>(z_loss),
+                               ptr_as<float>(entropy), ptr_as<int32_t>(counts), ptr_as<float>(load_balance), limited ? nullptr : ptr_as<float>(load_stats),
                                ptr_as<int32_t>(r.expert_start), ptr_as<int32_t>(r.s_scatter), ptr_as<int32_t>(r.s_reverse), ptr_as<int32_t>(r.x_gather),
                                ptr(ws), ws_bytes, stream_of(x)),
               "mts_moe_head_fwd");
+        if (limited) {
+            const Routing every = r;
+            Tensor kept = i32({o2 + 3 * round4(TK)}, x), accepted = kept.narrow(0, 0, E);
+            r.expert_start = kept.narrow(0, o1, E + 1);
+            r.s_scatter = kept.narrow(0, o2, TK);
+            r.s_reverse = kept.narrow(0, o2 + round4(TK), TK);
+            r.x_gather = kept.narrow(0, o2 + 2 * round4(TK), TK);
+            const int64_t keys_bytes = mts_moe_capacity_compact_workspace_bytes(T, K);
+            Tensor keys = bytes(keys_bytes, x);
+            check(mts_moe_capacity_compact(ptr_as<float>(weights), ptr_as<int32_t>(counts), ptr_as<int32_t>(every.expert_start), ptr_as<int32_t>(every.s_scatter),
+                                           T, K, E, capacity, ptr_as<int32_t>(accepted), ptr_as<int32_t>(r.expert_start), ptr_as<int32_t>(r.s_scatter),
+                                           ptr_as<int32_t>(r.s_reverse), ptr_as<int32_t>(r.x_gather), ptr(keys), keys_bytes, stream_of(x)),
+                  "mts_moe_capacity_compact");
+            check(mts_moe_capacity_weights_fwd(ptr_as<float>(weights), ptr_as<int32_t>(r.s_reverse), ptr_as<int32_t>(accepted), ptr_as<float>(entropy), T, K, E,
+                                               normalize, dtype_code(x), ptr(weights_act), ptr_as<float>(load_stats), stream_of(x)),
+                  "mts_moe_capacity_weights_fwd");
+        }
         Saved s;
         Tensor out = experts_forward(x, w1, w2, weights_act.view(-1), r, opt, s);
         variable_list keep;
         s.append_to(keep);
         keep.insert(keep.end(), {w_r, logits, weights, indices, counts});
         ctx->save_for_backward(std::move(keep));
-        ctx->saved_data["options"] = std::vector<int64_t>{switches, limit, normalize};
+        ctx->saved_data["options"] = std::vector<int64_t>{switches, limit, normalize, limited};
         ctx->mark_non_differentiable({entropy, counts, load_stats, indices, weights});
         ctx->set_materialize_grads(false);
         return {out, load_balance, z_loss, prob_mean, entropy, counts, load_stats, indices, weights};
@@ -499,10 +527,11 @@ struct MoELayer : torch::autograd::Function<MoELayer> {
         const Saved s(saved);
         const Tensor* router = &saved[Saved::kCount];
         c10::OptionalDeviceGuard guard(s.x.device());
-        RouterTail tail{router[0], router[1], router[2], router[3], router[4], like_f32(grads[3]), like_f32(grads[2]), like_f32(grads[1]), o[2] != 0, {}, {}};
+        RouterTail tail{router[0], router[1], router[2], router[3], router[4], like_f32(grads[3]), like_f32(grads[2]), like_f32(grads[1]), o[2] != 0,
+                        o[3] ? s.s_reverse : Tensor(), {}, {}};
         const bool need_x = ctx->needs_input_grad(0), need_wr = ctx->needs_input_grad(1);
         const bool wants_router = need_x || need_wr;
-        variable_list result(8);
+        variable_list result(9);
         if (grads[0].defined()) {
             const ExpertGrads g = experts_backward(s, grads[0], {need_x, ctx->needs_input_grad(2), ctx->needs_input_grad(3), wants_router}, {o[0], o[1]},
                                                    wants_router ? &tail : nullptr);
@@ -770,9 +799,10 @@ PYBIND11_MODULE(_host, m) {
         c10::OptionalDeviceGuard guard(x.device());
         return FusedMoE::apply(x, w1, w2, index, weights, switches, limit);
     });
-    m.def("moe_layer", [](const Tensor& x, const Tensor& w_r, const Tensor& w1, const Tensor& w2, int64_t top_k, bool normalize, int64_t switches, int64_t limit) {
+    m.def("moe_layer", [](const Tensor& x, const Tensor& w_r, const Tensor& w1, const Tensor& w2, int64_t top_k, bool normalize, int64_t capacity, int64_t switches,
+                          int64_t limit) {
         c10::OptionalDeviceGuard guard(x.device());
-        const variable_list v = MoELayer::apply(x, w_r, w1, w2, top_k, normalize, switches, limit);
+        const variable_list v = MoELayer::apply(x, w_r, w1, w2, top_k, normalize, capacity, switches, limit);
         return std::make_tuple(v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], v[8]);
     });
     m.def("router_postprocess", [](const Tensor& logits, int64_t top_k, bool normalize, int64_t act_dtype) {

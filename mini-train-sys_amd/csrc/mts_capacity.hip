@@ -8,6 +8,7 @@
 // 32-bit keys (four passes of 8 bits, histogram in LDS), and a last pass in segment order
 // ranks the entries that tie with that weight.
 #include "mts_common.h"
+#include "mts_router_row.h"
 
 namespace {
 
@@ -41,28 +42,81 @@ __device__ __forceinline__ void count_digit(uint32_t* hist, bool count, uint32_t
     if (count) atomicAdd(&hist[d], 1u);
 }
 
+// Where the answer for position i of an expert's segment (entry `entry`) goes.  MaskOut: 1/0 and the expert index or -1 per
+// entry.  CompactOut: the compacted permutation, in which the kept entries of an expert keep their order; `rank` counts the
+// kept entries in front of this one.
+struct MaskOut {
+    static constexpr bool kRanked = false;
+    uint8_t* keep;
+    int32_t* kept_index;   // may be NULL
+    int e;
+    __device__ __forceinline__ void put(int32_t entry, bool kept, uint32_t) const {
+        keep[entry] = kept ? 1 : 0;
+        if (kept_index) kept_index[entry] = kept ? e : -1;
+    }
+};
+struct CompactOut {
+    static constexpr bool kRanked = true;
+    int32_t* s_scatter;
+    int32_t* s_reverse;
+    int32_t* x_gather;
+    int first, K;          // first row of the expert's kept entries
+    __device__ __forceinline__ void put(int32_t entry, bool kept, uint32_t rank) const {
+        const int row = first + (int)rank;
+        s_reverse[entry] = kept ? row : -1;
+        if (kept) {
+            s_scatter[row] = entry;
+            x_gather[row] = entry / K;
+        }
+    }
+};
+
+// exclusive scan, in place, of one word per (slice, wave) in segment order; called by one wave
+__device__ __forceinline__ void scan_table(uint32_t* table, int lane) {
+    constexpr int PER_LANE = kRegKeys * kSelWaves / MTS_WAVE;
+    uint32_t v[PER_LANE], sum = 0;
+#pragma unroll
+    for (int j = 0; j < PER_LANE; ++j) {
+        v[j] = table[lane * PER_LANE + j];
+        sum += v[j];
+    }
+    uint32_t incl = sum;
+#pragma unroll
+    for (int o = 1; o < MTS_WAVE; o <<= 1) {
+        const uint32_t up = __shfl_up(incl, o, MTS_WAVE);
+        if (lane >= o) incl += up;
+    }
+    uint32_t run = incl - sum;
+#pragma unroll
+    for (int j = 0; j < PER_LANE; ++j) {
+        table[lane * PER_LANE + j] = run;
+        run += v[j];
+    }
+}
+
 // REGS: the segment has at most kRegKeys keys per thread and they stay in registers; otherwise
 // they are written to `kseg` in the first pass and read back in the later ones (the same thread
 // touches kseg[i] in every pass).  Position i of the segment belongs to thread i % kSelThreads.
-template <bool REGS>
+template <bool REGS, class Out>
 __device__ __forceinline__ void select_segment(const float* __restrict__ w, const int32_t* __restrict__ seg,
-                                               uint32_t* __restrict__ kseg, int n, int e, uint32_t capacity,
-                                               uint8_t* __restrict__ keep, int32_t* __restrict__ kept_index,
+                                               uint32_t* __restrict__ kseg, int n, uint32_t capacity, const Out& out,
                                                uint32_t* hist, uint32_t* chosen, uint32_t* wave_ties,
-                                               uint32_t* tie_table) {
+                                               uint32_t* tie_table, uint32_t* kept_table) {
     const int tid = threadIdx.x, lane = tid % MTS_WAVE, wave = tid / MTS_WAVE;
     uint32_t kr[REGS ? kRegKeys : 1];
     if (REGS) {
         int32_t entry[kRegKeys];
+        // (slices behind the segment's end are skipped by the whole block, here and below)
 #pragma unroll
         for (int u = 0; u < kRegKeys; ++u) {
             const int i = tid + u * kSelThreads;
-            entry[u] = i < n ? seg[i] : 0;
+            if (u * kSelThreads < n) entry[u] = i < n ? seg[i] : 0;
         }
 #pragma unroll
         for (int u = 0; u < kRegKeys; ++u) {
             const int i = tid + u * kSelThreads;
-            kr[u] = i < n ? order_key(w[entry[u]]) : 0u;
+            kr[u] = 0u;
+            if (u * kSelThreads < n) kr[u] = i < n ? order_key(w[entry[u]]) : 0u;
         }
     } else {
         for (int i0 = tid; i0 < n; i0 += kUnroll * kSelThreads) {
@@ -150,63 +204,42 @@ __device__ __forceinline__ void select_segment(const float* __restrict__ w, cons
     // prefix is now the key of the capacity-th largest weight; `need` of the entries with
     // exactly that key are kept, the earliest in segment order (= ascending entry)
     const uint64_t lt = lanemask_lt();
-    uint32_t carry = 0;
-    auto rank_block = [&](int i, uint32_t k) {   // one block-wide slice of kSelThreads positions
-        const bool in = i < n;
-        const bool tie = in && k == prefix;
-        const uint64_t b = __ballot(tie);
-        if (lane == 0) wave_ties[wave] = (uint32_t)__popcll(b);
-        __syncthreads();
-        uint32_t before = carry, total = 0;
-#pragma unroll
-        for (int j = 0; j < kSelWaves; ++j) {
-            const uint32_t c = wave_ties[j];
-            if (j < wave) before += c;
-            total += c;
-        }
-        if (in) {
-            const uint32_t rank = before + (uint32_t)__popcll(b & lt);
-            const bool kp = k > prefix || (tie && rank < need);
-            const int32_t entry = seg[i];
-            keep[entry] = kp ? 1 : 0;
-            if (kept_index) kept_index[entry] = kp ? e : -1;
-        }
-        carry += total;
-        __syncthreads();
-    };
     if (REGS) {
         // all slices at once: ties per (slice, wave) to LDS, one exclusive scan over that table in
         // segment order, then every thread ranks and writes its entries with the loads of their
-        // entry numbers in flight together (a barrier per slice would expose one L2 round trip each)
+        // entry numbers in flight together (a barrier per slice would expose one L2 round trip each);
+        // the compacted permutation counts the kept entries the same way
 #pragma unroll
         for (int u = 0; u < kRegKeys; ++u) {
             const int i = tid + u * kSelThreads;
-            const uint64_t b = __ballot(i < n && kr[u] == prefix);
+            uint64_t b = 0;
+            if (u * kSelThreads < n) b = __ballot(i < n && kr[u] == prefix);
             if (lane == 0) tie_table[u * kSelWaves + wave] = (uint32_t)__popcll(b);
         }
         __syncthreads();
-        if (wave == 0) {
-            constexpr int PER_LANE = kRegKeys * kSelWaves / MTS_WAVE;
-            uint32_t v[PER_LANE], sum = 0;
+        if (wave == 0) scan_table(tie_table, lane);
+        __syncthreads();
+        uint32_t kept_mask = 0;   // bit u: this thread's position of slice u is kept
 #pragma unroll
-            for (int j = 0; j < PER_LANE; ++j) {
-                v[j] = tie_table[lane * PER_LANE + j];
-                sum += v[j];
+        for (int u = 0; u < kRegKeys; ++u) {
+            bool kept = false;
+            if (u * kSelThreads < n) {
+                const int i = tid + u * kSelThreads;
+                const bool tie = i < n && kr[u] == prefix;
+                const uint32_t rank = tie_table[u * kSelWaves + wave] + (uint32_t)__popcll(__ballot(tie) & lt);
+                kept = i < n && (kr[u] > prefix || (tie && rank < need));
+                kept_mask |= (kept ? 1u : 0u) << u;
             }
-            uint32_t incl = sum;
-#pragma unroll
-            for (int o = 1; o < MTS_WAVE; o <<= 1) {
-                const uint32_t up = __shfl_up(incl, o, MTS_WAVE);
-                if (lane >= o) incl += up;
-            }
-            uint32_t run = incl - sum;
-#pragma unroll
-            for (int j = 0; j < PER_LANE; ++j) {
-                tie_table[lane * PER_LANE + j] = run;
-                run += v[j];
+            if constexpr (Out::kRanked) {
+                const uint64_t b = __ballot(kept);
+                if (lane == 0) kept_table[u * kSelWaves + wave] = (uint32_t)__popcll(b);
             }
         }
-        __syncthreads();
+        if constexpr (Out::kRanked) {
+            __syncthreads();
+            if (wave == 0) scan_table(kept_table, lane);
+            __syncthreads();
+        }
         constexpr int BATCH = 8;
 #pragma unroll
         for (int u0 = 0; u0 < kRegKeys; u0 += BATCH) {
@@ -220,53 +253,164 @@ __device__ __forceinline__ void select_segment(const float* __restrict__ w, cons
 #pragma unroll
             for (int j = 0; j < BATCH; ++j) {
                 const int u = u0 + j;
-                const int i = tid + u * kSelThreads;
-                const bool tie = i < n && kr[u] == prefix;
-                const uint64_t b = __ballot(tie);
-                const uint32_t rank = tie_table[u * kSelWaves + wave] + (uint32_t)__popcll(b & lt);
-                if (i < n) {
-                    const bool kp = kr[u] > prefix || (tie && rank < need);
-                    keep[entry[j]] = kp ? 1 : 0;
-                    if (kept_index) kept_index[entry[j]] = kp ? e : -1;
-                }
+                const bool kept = (kept_mask >> u) & 1u;
+                uint32_t rank = 0;
+                if constexpr (Out::kRanked) rank = kept_table[u * kSelWaves + wave] + (uint32_t)__popcll(__ballot(kept) & lt);
+                if (tid + u * kSelThreads < n) out.put(entry[j], kept, rank);
             }
         }
     } else {
-        for (int base = 0; base < n; base += kSelThreads) {
+        uint32_t carry = 0, kept_carry = 0;
+        for (int base = 0; base < n; base += kSelThreads) {   // one block-wide slice of kSelThreads positions
             const int i = base + tid;
-            rank_block(i, i < n ? kseg[i] : 0u);
+            const bool in = i < n;
+            const uint32_t k = in ? kseg[i] : 0u;
+            const bool tie = in && k == prefix;
+            auto count_before = [&](bool flag, uint32_t& running) {   // flags of the segment in front of this position
+                const uint64_t b = __ballot(flag);
+                if (lane == 0) wave_ties[wave] = (uint32_t)__popcll(b);
+                __syncthreads();
+                uint32_t before = running, total = 0;
+#pragma unroll
+                for (int j = 0; j < kSelWaves; ++j) {
+                    const uint32_t c = wave_ties[j];
+                    if (j < wave) before += c;
+                    total += c;
+                }
+                running += total;
+                __syncthreads();
+                return before + (uint32_t)__popcll(b & lt);
+            };
+            const uint32_t tie_rank = count_before(tie, carry);
+            const bool kept = in && (k > prefix || (tie && tie_rank < need));
+            uint32_t rank = 0;
+            if constexpr (Out::kRanked) rank = count_before(kept, kept_carry);
+            if (in) out.put(seg[i], kept, rank);
         }
     }
 }
+
+// one expert's segment: everything, nothing, or the selection
+template <class Out>
+__device__ __forceinline__ void select_expert(const float* __restrict__ w, const int32_t* __restrict__ seg, uint32_t* __restrict__ keys, int n,
+                                              int64_t capacity, const Out& out) {
+    __shared__ uint32_t hist[256];
+    __shared__ uint32_t chosen[2];          // prefix, number still to take inside it
+    __shared__ uint32_t wave_ties[kSelWaves];
+    __shared__ uint32_t tie_table[kRegKeys * kSelWaves];   // ties per (slice of kSelThreads positions, wave)
+    __shared__ uint32_t kept_table[Out::kRanked ? kRegKeys * kSelWaves : 1];
+    const bool all = (int64_t)n <= capacity, none = capacity <= 0;
+    if (all || none) {   // block-uniform
+        for (int i = threadIdx.x; i < n; i += kSelThreads) out.put(seg[i], !none, (uint32_t)i);
+        return;
+    }
+    if (n <= kRegKeys * kSelThreads)
+        select_segment<true>(w, seg, (uint32_t*)nullptr, n, (uint32_t)capacity, out, hist, chosen, wave_ties, tie_table, kept_table);
+    else
+        select_segment<false>(w, seg, keys, n, (uint32_t)capacity, out, hist, chosen, wave_ties, tie_table, kept_table);
+}
+
+__device__ __forceinline__ int32_t accepted_of(int n, int64_t capacity) { return capacity <= 0 ? 0 : ((int64_t)n <= capacity ? n : (int32_t)capacity); }
 
 __global__ __launch_bounds__(kSelThreads) void capacity_select_kernel(
     const float* __restrict__ w, const int32_t* __restrict__ s_scatter,
     const int32_t* __restrict__ counts, const int32_t* __restrict__ expert_start, int64_t capacity,
     uint32_t* __restrict__ keys, uint8_t* __restrict__ keep, int32_t* __restrict__ kept_index,
     int32_t* __restrict__ accepted) {
-    __shared__ uint32_t hist[256];
-    __shared__ uint32_t chosen[2];          // prefix, number still to take inside it
-    __shared__ uint32_t wave_ties[kSelWaves];
-    __shared__ uint32_t tie_table[kRegKeys * kSelWaves];   // ties per (slice of kSelThreads positions, wave)
-    const int e = blockIdx.x;
-    const int tid = threadIdx.x;
-    const int n = counts[e];
-    const int32_t* seg = s_scatter + expert_start[e];
-    const bool all = (int64_t)n <= capacity, none = capacity <= 0;
-    if (tid == 0) accepted[e] = none ? 0 : (all ? n : (int32_t)capacity);
-    if (all || none) {   // block-uniform
-        for (int i = tid; i < n; i += kSelThreads) {
-            const int32_t entry = seg[i];
-            keep[entry] = none ? 0 : 1;
-            if (kept_index) kept_index[entry] = none ? -1 : e;
-        }
-        return;
+    const int e = blockIdx.x, n = counts[e], first = expert_start[e];
+    if (threadIdx.x == 0) accepted[e] = accepted_of(n, capacity);
+    select_expert(w, s_scatter + first, keys + first, n, capacity, MaskOut{keep, kept_index, e});
+}
+
+// The same selection as a compacted permutation: how many routes every expert accepts is known from the counts alone, so
+// every block knows where its expert's kept rows start.  24 576 x 2 routes over 8 experts, half of them over the limit: 39 us
+// on eight blocks (four counting passes of about 5 us over up to 12 000 keys, then scattered stores), in place of the
+// routing metadata twice (25 us), the mask (34 us) and its application.
+__global__ __launch_bounds__(kSelThreads) void capacity_compact_kernel(
+    const float* __restrict__ w, const int32_t* __restrict__ s_scatter, const int32_t* __restrict__ counts,
+    const int32_t* __restrict__ expert_start, int E, int K, int64_t capacity, uint32_t* __restrict__ keys, int32_t* __restrict__ accepted,
+    int32_t* __restrict__ kept_start, int32_t* __restrict__ kept_scatter, int32_t* __restrict__ kept_reverse, int32_t* __restrict__ kept_gather) {
+    __shared__ int32_t in_front[kSelWaves];
+    const int e = blockIdx.x, tid = threadIdx.x, n = counts[e], first = expert_start[e];
+    int32_t v = tid < e ? accepted_of(counts[tid], capacity) : 0;   // at most 1024 experts: one per thread
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, MTS_WAVE);
+    if (tid % MTS_WAVE == 0) in_front[tid / MTS_WAVE] = v;
+    __syncthreads();
+    int32_t kept_first = 0;
+#pragma unroll
+    for (int j = 0; j < kSelWaves; ++j) kept_first += in_front[j];
+    if (tid == 0) {
+        const int32_t a = accepted_of(n, capacity);
+        accepted[e] = a;
+        kept_start[e] = kept_first;
+        if (e == E - 1) kept_start[E] = kept_first + a;
     }
-    if (n <= kRegKeys * kSelThreads)
-        select_segment<true>(w, seg, nullptr, n, e, (uint32_t)capacity, keep, kept_index, hist, chosen, wave_ties, tie_table);
-    else
-        select_segment<false>(w, seg, keys + expert_start[e], n, e, (uint32_t)capacity, keep, kept_index, hist,
-                              chosen, wave_ties, tie_table);
+    select_expert(w, s_scatter + first, keys + first, n, capacity, CompactOut{kept_scatter, kept_reverse, kept_gather, kept_first, K});
+}
+
+// Weights under a capacity limit: those of dropped routes become zero, a token's others are renormalised (a token may lose
+// every route).  One thread per token; block 0 also writes the load statistics of the accepted routes, in the layout of
+// mts_router_fwd's.
+constexpr float kSmallest = 1.1920929e-07f;   // fp32 epsilon: the least sum that is divided by
+constexpr int kWeightThreads = 256;
+template <typename ET>
+__global__ __launch_bounds__(kWeightThreads) void capacity_weights_kernel(const float* __restrict__ w, const int32_t* __restrict__ kept_reverse,
+                                                                          const int32_t* __restrict__ accepted, const float* __restrict__ entropy,
+                                                                          int64_t T, int K, int E, int normalize, ET* __restrict__ out,
+                                                                          float* __restrict__ load_stats) {
+    for (int64_t t = (int64_t)blockIdx.x * kWeightThreads + threadIdx.x; t < T; t += (int64_t)gridDim.x * kWeightThreads) {
+        float total = 0.f;
+        for (int k = 0; k < K; ++k) total += kept_reverse[t * K + k] >= 0 ? w[t * K + k] : 0.f;
+        const float div = normalize && total > 0.f ? (total > kSmallest ? total : kSmallest) : 1.f;
+        for (int k = 0; k < K; ++k) out[t * K + k] = (ET)((kept_reverse[t * K + k] >= 0 ? w[t * K + k] : 0.f) / div);
+    }
+    if (blockIdx.x != 0 || threadIdx.x >= MTS_WAVE) return;
+    const int lane = threadIdx.x;
+    const float routes = (float)((double)T * K), scale = (float)E;
+    float most = -1.f, least = INFINITY, sum = 0.f, dead = 0.f;
+    for (int e = lane; e < E; e += MTS_WAVE) {
+        const float a = (float)accepted[e];
+        load_stats[e] = a / routes;
+        most = fmaxf(most, a);
+        least = fminf(least, a);
+        sum += a;
+        dead += a == 0.f ? 1.f : 0.f;
+    }
+    sum = wave_sum(sum), dead = wave_sum(dead);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        most = fmaxf(most, __shfl_xor(most, o, MTS_WAVE));
+        least = fminf(least, __shfl_xor(least, o, MTS_WAVE));
+    }
+    const float mean = sum / routes / scale;
+    float dev = 0.f;
+    for (int e = lane; e < E; e += MTS_WAVE) {
+        const float d = (float)accepted[e] / routes - mean;
+        dev += d * d;
+    }
+    dev = wave_sum(dev);
+    if (lane == 0) {
+        float* s = load_stats + E;
+        s[0] = most;
+        s[1] = least;
+        s[2] = sqrtf(dev / scale) * scale;
+        s[3] = most / routes * scale;
+        s[4] = dead;
+        s[5] = 1.0f - sum / routes;
+        s[6] = *entropy / (E > 1 ? logf(scale) : 1.0f);
+    }
+}
+
+// the gradient of those weights, which arrives in the activation dtype, taken back to the unlimited weights
+template <typename ET>
+__global__ __launch_bounds__(kWeightThreads) void capacity_weights_bwd_kernel(const ET* __restrict__ g, const float* __restrict__ w,
+                                                                              const int32_t* __restrict__ kept_reverse, int64_t T, int K,
+                                                                              int normalize, float* __restrict__ g_w) {
+    for (int64_t t = (int64_t)blockIdx.x * kWeightThreads + threadIdx.x; t < T; t += (int64_t)gridDim.x * kWeightThreads) {
+        const mts_router::KeptWeights kw(w + t * K, kept_reverse + t * K, K, normalize, [&](int k) { return (float)g[t * K + k]; });
+        for (int k = 0; k < K; ++k) g_w[t * K + k] = kw.gradient(k, (float)g[t * K + k]);
+    }
 }
 
 // entries whose index is negative on input belong to no segment: they read as dropped
@@ -321,6 +465,61 @@ extern "C" int mts_moe_capacity_mask(const int32_t* top_k_index, const float* to
     MTS_CHECK_LAUNCH();
     capacity_select_kernel<<<E, kSelThreads, 0, (hipStream_t)stream>>>(
         top_k_weights, s_scatter, counts, expert_start, capacity, keys, keep, kept_index, accepted_counts);
+    MTS_CHECK_LAUNCH();
+    return MTS_OK;
+}
+
+extern "C" int64_t mts_moe_capacity_compact_workspace_bytes(int64_t T, int K) { return align256(T * K * 4); }
+
+extern "C" int mts_moe_capacity_compact(const float* top_k_weights, const int32_t* counts, const int32_t* expert_start, const int32_t* s_scatter,
+                                        int64_t T, int K, int E, int64_t capacity, int32_t* accepted_counts, int32_t* kept_start,
+                                        int32_t* kept_scatter, int32_t* kept_reverse, int32_t* kept_gather, void* workspace,
+                                        int64_t workspace_bytes, void* stream) {
+    if (!top_k_weights || !counts || !expert_start || !s_scatter || !accepted_counts || !kept_start || !kept_scatter || !kept_reverse ||
+        !kept_gather || !workspace)
+        return MTS_ERR_NULL;
+    if (T <= 0 || K < 1 || E < 1 || E > MTS_MAX_EXPERTS || T * (int64_t)K > 0x7fffffffLL) return MTS_ERR_SHAPE;
+    if (workspace_bytes < mts_moe_capacity_compact_workspace_bytes(T, K)) return MTS_ERR_WORKSPACE;
+    capacity_compact_kernel<<<E, kSelThreads, 0, (hipStream_t)stream>>>(top_k_weights, s_scatter, counts, expert_start, E, K, capacity,
+                                                                        (uint32_t*)workspace, accepted_counts, kept_start, kept_scatter,
+                                                                        kept_reverse, kept_gather);
+    MTS_CHECK_LAUNCH();
+    return MTS_OK;
+}
+
+extern "C" int mts_moe_capacity_weights_fwd(const float* top_k_weights, const int32_t* kept_reverse, const int32_t* accepted_counts,
+                                            const float* entropy, int64_t T, int K, int E, int normalize, int act_dtype, void* weights_out,
+                                            float* load_stats, void* stream) {
+    if (!top_k_weights || !kept_reverse || !accepted_counts || !entropy || !weights_out || !load_stats) return MTS_ERR_NULL;
+    if (T <= 0 || K < 1 || E < 1 || T * (int64_t)K > 0x7fffffffLL) return MTS_ERR_SHAPE;
+    const int64_t want = (T + kWeightThreads - 1) / kWeightThreads;
+    const dim3 grid((unsigned)(want < 1024 ? want : 1024));
+    hipStream_t s = (hipStream_t)stream;
+    if (act_dtype == MTS_BF16)
+        capacity_weights_kernel<bf16_t><<<grid, kWeightThreads, 0, s>>>(top_k_weights, kept_reverse, accepted_counts, entropy, T, K, E, normalize, (bf16_t*)weights_out, load_stats);
+    else if (act_dtype == MTS_F16)
+        capacity_weights_kernel<mts_f16_t><<<grid, kWeightThreads, 0, s>>>(top_k_weights, kept_reverse, accepted_counts, entropy, T, K, E, normalize, (mts_f16_t*)weights_out, load_stats);
+    else if (act_dtype == MTS_F32)
+        capacity_weights_kernel<float><<<grid, kWeightThreads, 0, s>>>(top_k_weights, kept_reverse, accepted_counts, entropy, T, K, E, normalize, (float*)weights_out, load_stats);
+    else return MTS_ERR_DTYPE;
+    MTS_CHECK_LAUNCH();
+    return MTS_OK;
+}
+
+extern "C" int mts_moe_capacity_weights_bwd(const void* g_weights, const float* top_k_weights, const int32_t* kept_reverse, int64_t T, int K,
+                                            int normalize, int act_dtype, float* g_top_k_weights, void* stream) {
+    if (!g_weights || !top_k_weights || !kept_reverse || !g_top_k_weights) return MTS_ERR_NULL;
+    if (T <= 0 || K < 1 || T * (int64_t)K > 0x7fffffffLL) return MTS_ERR_SHAPE;
+    const int64_t want = (T + kWeightThreads - 1) / kWeightThreads;
+    const dim3 grid((unsigned)(want < 1024 ? want : 1024));
+    hipStream_t s = (hipStream_t)stream;
+    if (act_dtype == MTS_BF16)
+        capacity_weights_bwd_kernel<bf16_t><<<grid, kWeightThreads, 0, s>>>((const bf16_t*)g_weights, top_k_weights, kept_reverse, T, K, normalize, g_top_k_weights);
+    else if (act_dtype == MTS_F16)
+        capacity_weights_bwd_kernel<mts_f16_t><<<grid, kWeightThreads, 0, s>>>((const mts_f16_t*)g_weights, top_k_weights, kept_reverse, T, K, normalize, g_top_k_weights);
+    else if (act_dtype == MTS_F32)
+        capacity_weights_bwd_kernel<float><<<grid, kWeightThreads, 0, s>>>((const float*)g_weights, top_k_weights, kept_reverse, T, K, normalize, g_top_k_weights);
+    else return MTS_ERR_DTYPE;
     MTS_CHECK_LAUNCH();
     return MTS_OK;
 }

@@ -2961,7 +2961,7 @@ extern "C" int MTS_GEMM_ENTRY(mts_moe_bwd_joint_router)(
     q.r_col_threads = g.col_threads;
     q.r_dx = (bf16_t*)dx_router; q.r_part = (float*)router_workspace; q.r_dw = d_w_r;
     q.c_out = (bf16_t*)dx; q.c_K = K;
-    q.rg = {logits, weights, indices, counts, nullptr, nullptr, g_prob_mean, g_z_loss, g_load_balance, act_dtype, K, normalize,
-            ds_partial, s_reverse, q.np};
+    q.rg = {logits, weights, indices, counts, nullptr, nullptr, g_prob_mean, g_z_loss, g_load_balance, act_dtype, K, normalize & 1,
+            ds_partial, s_reverse, q.np, (normalize & MTS_NORMALIZE_KEPT) != 0};
     return launch_bwd_joint(q, E, grad_dtype, workspace1, workspace1_bytes, workspace2, workspace2_bytes, schedule, (hipStream_t)stream);
 }

@@ -76,6 +76,7 @@ struct RouterGradIn {
     const float* ds_part;
     const int32_t* s_reverse;
     int np;
+    int kept_only;   // the weights were limited to the routes that s_reverse gives a row, and renormalised (KeptWeights)
 };
 constexpr int kChainRows = 256;   // most rows a block of the chained kernel takes (their logit gradients sit in LDS)
 
@@ -124,8 +125,14 @@ __device__ __forceinline__ void router_logits_bwd_block(const float* __restrict_
                 }
                 return v;
             };
-            row_logit_gradient<EP, 1>(r, gp, gz, rg.K, rg.normalize, 0, rg.weights + row * rg.K, rg.indices + row * rg.K,
-                                      grad_w, o);
+            if (rg.kept_only) {
+                const KeptWeights kw(rg.weights + row * rg.K, rg.s_reverse + row * rg.K, rg.K, rg.normalize, grad_w);
+                row_logit_gradient<EP, 1>(r, gp, gz, rg.K, rg.normalize, 0, rg.weights + row * rg.K, rg.indices + row * rg.K,
+                                          [&](int k) { return kw.gradient(k, grad_w(k)); }, o);
+            } else {
+                row_logit_gradient<EP, 1>(r, gp, gz, rg.K, rg.normalize, 0, rg.weights + row * rg.K, rg.indices + row * rg.K,
+                                          grad_w, o);
+            }
 #pragma unroll
             for (int e = 0; e < EP; ++e) dl_lds[(row - b0) * EP + e] = e < E ? o[e] : 0.f;
         }

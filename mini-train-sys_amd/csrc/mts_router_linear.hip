@@ -854,7 +854,7 @@ extern "C" int mts_moe_head_bwd(const void* x, const float* w_r, const float* lo
     const size_t lds = (size_t)E * shape.cols_per_block * sizeof(float);
     float* part = (float*)workspace;
     RouterGradIn rg = {logits, weights, indices, counts, g_weights, g_weights_act, g_prob_mean, g_z_loss, g_load_balance,
-                       act_dtype, K, normalize, nullptr, nullptr, 0};
+                       act_dtype, K, normalize, nullptr, nullptr, 0, 0};
 #define MTS_CHAIN(XT, EP)                                                                                        \
     do {                                                                                                         \
         if (allow_lds(router_logits_bwd_kernel<XT, EP, false, true>, lds, kChainRows * EP * sizeof(float)) != hipSuccess) \

@@ -10,6 +10,26 @@
 
 namespace mts_router {
 
+// A token's routing weights under a capacity limit: routes without a row (kept_reverse < 0) weigh nothing and the others are
+// divided by their sum.  What a gradient of the result is for the weights it was formed from; `g_of(k)`: that gradient.
+struct KeptWeights {
+    const int32_t* kept;
+    float scale = 1.f, dot = 0.f;   // 1 / sum, and sum_j g_j w'_j
+    template <class G>
+    __device__ __forceinline__ KeptWeights(const float* w, const int32_t* kept_reverse, int K, int normalize, G g_of) : kept(kept_reverse) {
+        if (!normalize) return;
+        float total = 0.f;
+        for (int k = 0; k < K; ++k) total += kept[k] >= 0 ? w[k] : 0.f;
+        if (!(total > 0.f)) return;
+        constexpr float smallest = 1.1920929e-07f;   // below it the forward pass divides by this constant
+        scale = 1.f / (total > smallest ? total : smallest);
+        if (total > smallest)
+            for (int k = 0; k < K; ++k) dot += kept[k] >= 0 ? g_of(k) * w[k] * scale : 0.f;
+    }
+    __device__ __forceinline__ float gradient(int k, float g) const { return kept[k] >= 0 ? (g - dot) * scale : 0.f; }
+};
+
+
 constexpr float kLogFloor = -20.72326583694641f;  // log(1e-9): the entropy clamps p at 1e-9
 
 template <int G>

@@ -40,6 +40,10 @@ SIGNATURES = {
     "mts_moe_route_static": (_i, [_p, _l, _i, _i, _i, _p, _p, _p, _p, _p, _p, _p, _p, _p]),
     "mts_moe_capacity_workspace_bytes": (_l, [_l, _i, _i]),
     "mts_moe_capacity_mask": (_i, [_p, _p, _l, _i, _i, _l, _p, _p, _p, _p, _l, _p]),
+    "mts_moe_capacity_compact_workspace_bytes": (_l, [_l, _i]),
+    "mts_moe_capacity_compact": (_i, [_p] * 4 + [_l, _i, _i, _l] + [_p] * 6 + [_l, _p]),
+    "mts_moe_capacity_weights_fwd": (_i, [_p, _p, _p, _p, _l, _i, _i, _i, _i, _p, _p, _p]),
+    "mts_moe_capacity_weights_bwd": (_i, [_p, _p, _p, _l, _i, _i, _i, _p, _p]),
     "mts_moe_stage_weights": (_i, [_p, _i, _p, _i, _i, _l, _l, _i, _p]),
     "mts_moe_cast_weights_pair": (_i, [_p, _p, _l, _p, _p, _l, _i, _p]),
     "mts_moe_fwd_gateup_swiglu": (_i, [_p, _p, _p, _p, _p, _p, _l, _i, _i, _i, _i, _i, _p, _p, _p]),

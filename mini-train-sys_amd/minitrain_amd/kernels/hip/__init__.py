@@ -87,13 +87,16 @@ class HipOpsBackend(DenseTorchOps):
     # call that module)
     offers_moe_layer = SWITCHES.layer_node
 
-    def moe_layer(self, x, router_weight, gate_up_proj, down_proj, top_k, *, normalize):
+    # moe_layer takes a capacity limit
+    limits_moe_layer = True
+
+    def moe_layer(self, x, router_weight, gate_up_proj, down_proj, top_k, *, normalize, capacity=None):
         """Extension: router projection, post-process, routing metadata and the experts as one autograd
         node (see ``kernels/hip/moe_layer.py``).  Returns None when the contract is not supported; the
         caller then composes the layer from ``router_postprocess`` and ``fused_moe``."""
         if not self.offers_moe_layer or moe_layer_violation(x, router_weight, gate_up_proj, down_proj, top_k) is not None:
             return None
-        return run_moe_layer(x, router_weight, gate_up_proj, down_proj, top_k, normalize)
+        return run_moe_layer(x, router_weight, gate_up_proj, down_proj, top_k, normalize, capacity)
 
     def router_logits(self, hidden_states, weight):
         """Extension beyond the reference's operator interface: the router projection in fp32

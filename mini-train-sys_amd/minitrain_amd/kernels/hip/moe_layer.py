@@ -25,17 +25,20 @@ def moe_layer_violation(x, router_weight, gate_up_proj, down_proj, top_k: int):
     return _lib.host().layer_violation(x, router_weight, gate_up_proj, down_proj, top_k)
 
 
-def moe_layer(x, router_weight, gate_up_proj, down_proj, top_k: int, *, normalize: bool):
+def moe_layer(x, router_weight, gate_up_proj, down_proj, top_k: int, *, normalize: bool, capacity: int | None = None):
     """``(hidden, load_balance_loss, z_loss, probability_per_expert, entropy, expert_counts, load_stats,
     expert_indices, expert_weights)`` of one MoE layer on ``x [T,H]``; the first four are differentiable.
+    With ``capacity`` an expert accepts its that many most confident routes (the rule of ``capacity_mask``): the others get
+    no row, a token's kept weights are renormalised with ``normalize``, and ``load_stats`` describes the accepted routes;
+    ``expert_counts``, ``expert_indices`` and ``expert_weights`` stay those of the unlimited routing.
     The autograd node is native (``csrc/host/mts_host.cpp``)."""
     missed = moe_layer_violation(x, router_weight, gate_up_proj, down_proj, top_k)
     if missed is not None:
         raise RuntimeError(f"Unsupported tensor contract for the hip MoE layer: it requires {missed}")
-    return run_moe_layer(x, router_weight, gate_up_proj, down_proj, top_k, normalize)
+    return run_moe_layer(x, router_weight, gate_up_proj, down_proj, top_k, normalize, capacity)
 
 
-def run_moe_layer(x, router_weight, gate_up_proj, down_proj, top_k: int, normalize: bool):
+def run_moe_layer(x, router_weight, gate_up_proj, down_proj, top_k: int, normalize: bool, capacity: int | None):
     """:func:`moe_layer` for arguments that are known to fit the contract."""
-    return _lib.host().moe_layer(x, router_weight, gate_up_proj, down_proj, top_k, normalize, SWITCHES.mask(),
-                                 dw_workspace_limit(x, gate_up_proj))
+    return _lib.host().moe_layer(x, router_weight, gate_up_proj, down_proj, top_k, normalize, -1 if capacity is None else capacity,
+                                 SWITCHES.mask(), dw_workspace_limit(x, gate_up_proj))
