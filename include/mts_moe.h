@@ -107,6 +107,17 @@ int mts_router_logits_bwd(const float* dlogits, const void* x, const float* w_r,
                           int H, int E, int act_dtype, void* dx, float* d_w_r,
                           void* workspace, int64_t workspace_bytes, void* stream);
 
+/* The same projection and backward for any number of experts up to MTS_MAX_EXPERTS, H a multiple of 4
+ * (fp32 matrix instruction; 16-bit activations are widened on load).  The entry points above are the
+ * faster ones where they apply.                                                               */
+int mts_router_wide_supported(int H, int E);
+int mts_router_wide_fwd(const void* x, const float* w_r, int64_t T, int H, int E, int act_dtype,
+                        float* logits, void* stream);
+int64_t mts_router_wide_bwd_workspace_bytes(int64_t T, int H, int E);
+int mts_router_wide_bwd(const float* dlogits, const void* x, const float* w_r, int64_t T, int H, int E,
+                        int act_dtype, void* dx, float* d_w_r, void* workspace,
+                        int64_t workspace_bytes, void* stream);
+
 /* ---- the layer's head in two launches ---------------------------------------
  * mts_router_logits_fwd + mts_router_fwd + mts_moe_route as one chain (router projection,
  * post-process and routing metadata of minitrain/model/moe_router.py:64-90 and

@@ -115,10 +115,13 @@ bool needs_padding(const Tensor& x, const Tensor& w1) {
     return x.size(1) % (wide ? 4 : 8) != 0 || (!wide && (w1.size(1) / 2) % 8 != 0);
 }
 
+// Up to 16 experts the projection kernels keep W_r in LDS; more take the kernels on the fp32 matrix instruction.
+constexpr int64_t kFewExperts = 16;
 bool router_logits_supported(const Tensor& x, const Tensor& w) {
     return x.is_cuda() && w.is_cuda() && x.dim() == 2 && w.dim() == 2 && is_activation_type(x.scalar_type()) && w.scalar_type() == at::kFloat &&
-           x.size(0) > 0 && x.size(1) == w.size(1) && w.size(0) <= 16 && x.size(1) % 4 == 0 && x.size(1) <= 4096 &&
-           w.size(0) * w.size(1) * 4 <= 128 * 1024;   // the projection kernels keep W_r in LDS
+           x.size(0) > 0 && x.size(1) == w.size(1) &&
+           (w.size(0) <= kFewExperts ? x.size(1) % 4 == 0 && x.size(1) <= 4096 && w.size(0) * w.size(1) * 4 <= 128 * 1024
+                                     : mts_router_wide_supported(x.size(1), w.size(0)));
 }
 
 const char* layer_violation(const Tensor& x, const Tensor& w_r, const Tensor& w1, const Tensor& w2, int64_t top_k) {
@@ -126,7 +129,7 @@ const char* layer_violation(const Tensor& x, const Tensor& w_r, const Tensor& w1
     const int64_t E = w1.size(0);
     if (w_r.dim() != 2 || w_r.size(0) != E) return "router weight is [E,H]";
     if (!router_logits_supported(x, w_r))
-        return "an fp32 router weight on the same GPU, at most 16 experts and a hidden size of at most 4096 (E * H <= 32768)";
+        return "an fp32 router weight on the same GPU, at most 1024 experts, and up to 16 of them a hidden size of at most 4096 (E * H <= 32768)";
     if (top_k < 1 || top_k > std::min(E, kMaxTopK)) return "1 <= top_k <= min(E, 8)";
     if (needs_padding(x, w1)) return "hidden and expert widths that are whole 16-byte chunks";
     if (x.size(0) * top_k >= k2GiB) return "fewer than 2^31 routes";
@@ -287,6 +290,24 @@ struct ExpertGrads {
     Tensor dx, dw1, dw2, ds;
 };
 
+void router_projection_forward(const Tensor& x, const Tensor& w, const Tensor& logits) {
+    const int64_t T = x.size(0), H = x.size(1), E = w.size(0);
+    if (E > kFewExperts)
+        check(mts_router_wide_fwd(ptr(x), ptr_as<float>(w), T, H, E, dtype_code(x), ptr_as<float>(logits), stream_of(x)), "mts_router_wide_fwd");
+    else
+        check(mts_router_logits_fwd(ptr(x), ptr_as<float>(w), T, H, E, dtype_code(x), ptr_as<float>(logits), stream_of(x)), "mts_router_logits_fwd");
+}
+
+void router_projection_backward(const Tensor& g, const Tensor& x, const Tensor& w, const Tensor& dx, const Tensor& dw) {
+    const int64_t T = x.size(0), H = x.size(1), E = w.size(0);
+    const bool wide = E > kFewExperts;
+    const int64_t ws_bytes = wide ? mts_router_wide_bwd_workspace_bytes(T, H, E) : mts_router_logits_bwd_workspace_bytes(T, H, E);
+    Tensor ws = bytes(ws_bytes, x);
+    check((wide ? mts_router_wide_bwd : mts_router_logits_bwd)(ptr_as<float>(g), ptr(x), ptr_as<float>(w), T, H, E, dtype_code(x), ptr(dx), ptr_as<float>(dw),
+                                                               ptr(ws), ws_bytes, stream_of(x)),
+          wide ? "mts_router_wide_bwd" : "mts_router_logits_bwd");
+}
+
 void router_gradient(const Tensor& x, RouterTail& t, const Tensor& ds) {   // dS and the router's loss terms -> dx_r, dW_r
     const int64_t T = x.size(0), H = x.size(1), E = t.w_r.size(0), K = t.weights.size(1);
     const bool narrow = x.scalar_type() != at::kFloat;
@@ -299,6 +320,15 @@ void router_gradient(const Tensor& x, RouterTail& t, const Tensor& ds) {   // dS
         check(mts_moe_capacity_weights_bwd(ptr(ds), ptr_as<float>(t.weights), ptr_as<int32_t>(t.kept_reverse), T, K, t.normalize, dtype_code(ds),
                                            ptr_as<float>(g_w), stream_of(x)),
               "mts_moe_capacity_weights_bwd");
+    }
+    if (E > kFewExperts) {
+        Tensor g_logits = at::empty_like(t.logits);
+        check(mts_router_bwd(ptr_as<float>(t.logits), ptr_as<float>(t.weights), ptr_as<int32_t>(t.indices), ptr_as<float>(g_w), ptr(g_w_act),
+                             narrow ? dtype_code(x) : 0, ptr_as<float>(t.g_prob_mean), ptr_as<float>(t.g_z_loss), ptr_as<float>(t.g_load_balance),
+                             ptr_as<int32_t>(t.counts), T, E, K, t.normalize, ptr_as<float>(g_logits), stream_of(x)),
+              "mts_router_bwd");
+        router_projection_backward(g_logits, x, t.w_r, t.dx_r, t.dw_r);
+        return;
     }
     const int64_t ws_bytes = mts_moe_head_bwd_workspace_bytes(T, H, E);
     Tensor ws = bytes(ws_bytes, x);
@@ -485,14 +515,26 @@ struct MoELayer : torch::autograd::Function<MoELayer> {
         r.s_scatter = meta.narrow(0, o2, TK);
         r.s_reverse = meta.narrow(0, o2 + round4(TK), TK);
         r.x_gather = meta.narrow(0, o2 + 2 * round4(TK), TK);
-        const int64_t ws_bytes = mts_moe_head_workspace_bytes(T, K, E);
-        Tensor ws = bytes(ws_bytes, x);
-        check(mts_moe_head_fwd(ptr(x), ptr_as<float>(w_r), T, H, E, K, normalize, dtype_code(x), ptr_as<float>(logits), ptr_as<float>(weights),
-                               ptr_as<int32_t>(indices), narrow && !limited ? ptr(weights_act) : nullptr, ptr_as<float>(prob_mean), ptr_as<float>(z_loss),
-                               ptr_as<float>(entropy), ptr_as<int32_t>(counts), ptr_as<float>(load_balance), limited ? nullptr : ptr_as<float>(load_stats),
-                               ptr_as<int32_t>(r.expert_start), ptr_as<int32_t>(r.s_scatter), ptr_as<int32_t>(r.s_reverse), ptr_as<int32_t>(r.x_gather),
-                               ptr(ws), ws_bytes, stream_of(x)),
-              "mts_moe_head_fwd");
+        if (E > kFewExperts) {   // the chained head is written for few experts
+            router_projection_forward(x, w_r, logits);
+            const int64_t ws_bytes = mts_router_workspace_bytes(T, E);
+            Tensor ws = bytes(ws_bytes, x);
+            check(mts_router_fwd(ptr_as<float>(logits), T, E, K, normalize, ptr_as<float>(weights), ptr_as<int32_t>(indices), ptr_as<float>(prob_mean),
+                                 ptr_as<float>(z_loss), ptr_as<float>(entropy), ptr_as<int32_t>(counts), ptr_as<float>(load_balance),
+                                 limited ? nullptr : ptr_as<float>(load_stats), narrow && !limited ? ptr(weights_act) : nullptr, narrow ? dtype_code(x) : 0,
+                                 ptr(ws), ws_bytes, stream_of(x)),
+                  "mts_router_fwd");
+            r = route(indices, E);
+        } else {
+            const int64_t ws_bytes = mts_moe_head_workspace_bytes(T, K, E);
+            Tensor ws = bytes(ws_bytes, x);
+            check(mts_moe_head_fwd(ptr(x), ptr_as<float>(w_r), T, H, E, K, normalize, dtype_code(x), ptr_as<float>(logits), ptr_as<float>(weights),
+                                   ptr_as<int32_t>(indices), narrow && !limited ? ptr(weights_act) : nullptr, ptr_as<float>(prob_mean), ptr_as<float>(z_loss),
+                                   ptr_as<float>(entropy), ptr_as<int32_t>(counts), ptr_as<float>(load_balance), limited ? nullptr : ptr_as<float>(load_stats),
+                                   ptr_as<int32_t>(r.expert_start), ptr_as<int32_t>(r.s_scatter), ptr_as<int32_t>(r.s_reverse), ptr_as<int32_t>(r.x_gather),
+                                   ptr(ws), ws_bytes, stream_of(x)),
+                  "mts_moe_head_fwd");
+        }
         if (limited) {
             const Routing every = r;
             Tensor kept = i32({o2 + 3 * round4(TK)}, x), accepted = kept.narrow(0, 0, E);
@@ -593,8 +635,7 @@ struct RouterLogits : torch::autograd::Function<RouterLogits> {
     static Tensor forward(AutogradContext* ctx, const Tensor& x_, const Tensor& w_) {
         const Tensor x = x_.contiguous(), w = w_.contiguous();
         Tensor logits = f32({x.size(0), w.size(0)}, x);
-        check(mts_router_logits_fwd(ptr(x), ptr_as<float>(w), x.size(0), x.size(1), w.size(0), dtype_code(x), ptr_as<float>(logits), stream_of(x)),
-              "mts_router_logits_fwd");
+        router_projection_forward(x, w, logits);
         ctx->save_for_backward({x, w});
         return logits;
     }
@@ -603,11 +644,7 @@ struct RouterLogits : torch::autograd::Function<RouterLogits> {
         c10::OptionalDeviceGuard guard(s[0].device());
         const Tensor g = like_f32(grads[0]);
         Tensor dx = at::empty_like(s[0]), dw = at::empty_like(s[1]);
-        const int64_t T = s[0].size(0), H = s[0].size(1), E = s[1].size(0), ws_bytes = mts_router_logits_bwd_workspace_bytes(T, H, E);
-        Tensor ws = bytes(ws_bytes, s[0]);
-        check(mts_router_logits_bwd(ptr_as<float>(g), ptr(s[0]), ptr_as<float>(s[1]), T, H, E, dtype_code(s[0]), ptr(dx), ptr_as<float>(dw), ptr(ws), ws_bytes,
-                                    stream_of(s[0])),
-              "mts_router_logits_bwd");
+        router_projection_backward(g, s[0], s[1], dx, dw);
         return {dx, dw};
     }
 };

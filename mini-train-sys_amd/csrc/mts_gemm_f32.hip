@@ -7,21 +7,18 @@
 // one byte of L2 per 16 FLOP; tiles of 128 rows are no faster at 16 000 rows (101 TFLOP/s over all GEMMs either way) and
 // 12 % slower at 4096, where they leave the CUs unevenly filled.  2048 tokens, 768/1024, 8 experts, top-2: forward and
 // backward of the operator 1776 -> 727 us, 80 TFLOP/s (plain FMA from 64x64 tiles before: 33 TFLOP/s).
-//
-// The k index an operand register stands for is free as long as both operands agree: lanes 0..31 hold k = 8s+0..3 and lanes
-// 32..63 k = 8s+4..7 of four consecutive instructions, so an operand whose rows are k-contiguous is read as one 16-byte
-// LDS load per four instructions, and one whose memory rows are k ("k-major": stored weights in the backward pass, both
-// operands of the weight gradients) as four 4-byte loads, with no transposed copy of anything.
-#include "mts_common.h"
+#include "mts_f32_tiles.h"
 
 #include <type_traits>
 
 namespace {
 
-constexpr int TKS = 16;  // k extent of an LDS tile
+using namespace mts_f32;
+
 constexpr int BM = 64;   // rows of a tile, and of P columns in the weight gradients
-constexpr int kThreads = 256;
+constexpr int kThreads = kTileThreads;
 constexpr int kXcds = 8;
+constexpr int TKS = 16;  // k extent of an LDS tile
 
 enum Epi32 { E32_PLAIN = 0, E32_SWIGLU = 1, E32_DY1 = 2 };
 
@@ -45,118 +42,6 @@ struct Rows32 {
 };
 
 __device__ __forceinline__ float sigmoid32(float x) { return 1.0f / (1.0f + expf(-x)); }
-
-// four consecutive floats at p, of which the first `count` exist (VEC: p is 16-byte aligned and count is 0 or >= 4)
-template <bool VEC>
-__device__ __forceinline__ f32x4 load4(const float* p, int count) {
-    f32x4 v = {};
-    if constexpr (VEC) {
-        if (count > 0) v = *reinterpret_cast<const f32x4*>(p);
-    } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            if (j < count) v[j] = p[j];
-    }
-    return v;
-}
-
-// [ROWS][16] tile of k-contiguous rows.  Rows are 20 floats apart in LDS: the 16-byte fragment reads of 16 lanes then
-// start on 16 different groups of four banks.
-template <int ROWS, bool VEC>
-struct RowTile {
-    static constexpr int LD = TKS + 4, TPR = TKS / 4, LOADS = ROWS * TPR / kThreads, SIZE = ROWS * LD;
-    const float* ptr[LOADS];   // this thread's rows, NULL: zeros
-    f32x4 reg[2][LOADS];
-    __device__ __forceinline__ static int row(int p) { return threadIdx.x / TPR + p * (kThreads / TPR); }
-    __device__ __forceinline__ void fetch(int set, int k0, int Kdim) {
-        const int k = k0 + (threadIdx.x % TPR) * 4;
-#pragma unroll
-        for (int p = 0; p < LOADS; ++p) reg[set][p] = load4<VEC>(ptr[p] + k, ptr[p] ? Kdim - k : 0);
-    }
-    __device__ __forceinline__ void commit(int set, float* lds) const {
-#pragma unroll
-        for (int p = 0; p < LOADS; ++p) *reinterpret_cast<f32x4*>(lds + row(p) * LD + (threadIdx.x % TPR) * 4) = reg[set][p];
-    }
-    // k = 8s + 4 * (lane / 32) + 0..3 of row `r0 + lane % 32`
-    __device__ __forceinline__ static f32x4 frag(const float* lds, int r0, int s) {
-        const int lane = threadIdx.x % MTS_WAVE;
-        return *reinterpret_cast<const f32x4*>(lds + (r0 + lane % 32) * LD + s * 8 + (lane / 32) * 4);
-    }
-};
-
-// [16][COLS] tile of k-major rows.  The row length in LDS puts k and k+4, which the two halves of a wave read together,
-// 32 banks apart.
-template <int COLS, bool VEC>
-struct KTile {
-    static constexpr int LD = COLS + 8, LOADS = COLS * TKS / 4 / kThreads, SIZE = TKS * LD, PER_ROW = COLS / 4;
-    const float* base;       // element (k = 0, this thread's first column)
-    int64_t ld;
-    int cols;                // columns from there on that exist
-    f32x4 reg[2][LOADS];
-    __device__ __forceinline__ static int k(int p) { return threadIdx.x / PER_ROW + p * (kThreads / PER_ROW); }
-    __device__ __forceinline__ static int col() { return (threadIdx.x % PER_ROW) * 4; }
-    // rows[p] = memory row of k-row k(p), or < 0: zeros
-    __device__ __forceinline__ void fetch(int set, const int64_t (&rows)[LOADS]) {
-#pragma unroll
-        for (int p = 0; p < LOADS; ++p) reg[set][p] = load4<VEC>(base + rows[p] * ld, rows[p] >= 0 ? cols : 0);
-    }
-    __device__ __forceinline__ void commit(int set, float* lds) const {
-#pragma unroll
-        for (int p = 0; p < LOADS; ++p) *reinterpret_cast<f32x4*>(lds + k(p) * LD + col()) = reg[set][p];
-    }
-    __device__ __forceinline__ static f32x4 frag(const float* lds, int c0, int s) {
-        const int lane = threadIdx.x % MTS_WAVE;
-        const float* q = lds + (s * 8 + (lane / 32) * 4) * LD + c0 + lane % 32;
-        return f32x4{q[0], q[LD], q[2 * LD], q[3 * LD]};
-    }
-};
-
-// one k-tile: MF x NF fragments of 32x32 per wave; a_at / b_at give the first row / column of a fragment in the tile
-template <class AT, class BT, int MF, int NF, class AAt, class BAt>
-__device__ __forceinline__ void mma_tile32(const float* As, const float* Bs, f32x16 (&acc)[MF][NF], AAt a_at, BAt b_at) {
-#pragma unroll
-    for (int s = 0; s < TKS / 8; ++s) {
-        f32x4 a[MF], b[NF];
-#pragma unroll
-        for (int i = 0; i < MF; ++i) a[i] = AT::frag(As, a_at(i), s);
-#pragma unroll
-        for (int i = 0; i < NF; ++i) b[i] = BT::frag(Bs, b_at(i), s);
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int mf = 0; mf < MF; ++mf)
-#pragma unroll
-                for (int nf = 0; nf < NF; ++nf)
-                    acc[mf][nf] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[mf][j], b[nf][j], acc[mf][nf], 0, 0, 0);
-    }
-}
-
-// The k loop: two LDS buffers, and two k-tiles in flight in registers behind them (a tile's loads have two tiles' matrix
-// work to arrive in).  fetch(set, t) starts the loads of k-tile t; it is called once for every t in order.
-template <class AT, class BT, int MF, int NF, class AAt, class BAt, class Fetch>
-__device__ __forceinline__ void run_k_tiles(int tiles, AT& a, BT& b, float (*As)[AT::SIZE], float (*Bs)[BT::SIZE], f32x16 (&acc)[MF][NF],
-                                            AAt a_at, BAt b_at, Fetch fetch) {
-    if (tiles <= 0) return;
-    fetch(0, 0);
-    if (tiles > 1) fetch(1, 1);
-    a.commit(0, As[0]);
-    b.commit(0, Bs[0]);
-    __syncthreads();
-    for (int t0 = 0; t0 < tiles; t0 += 2) {
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const int t = t0 + u;
-            if (t >= tiles) break;
-            if (t + 2 < tiles) fetch(u, t + 2);
-            mma_tile32<AT, BT, MF, NF>(As[u], Bs[u], acc, a_at, b_at);
-            if (t + 1 < tiles) {
-                a.commit(1 - u, As[1 - u]);
-                b.commit(1 - u, Bs[1 - u]);
-            }
-            __syncthreads();
-        }
-    }
-}
 
 // The m-tiles of all experts in expert order, 64 experts per round: their number, and expert and rows of tile `tile`
 // (every lane of the wave gets the same answer; tile < 0: only the number is wanted).
@@ -191,8 +76,8 @@ __global__ __launch_bounds__(kThreads) void rows_gemm_f32_kernel(Rows32 p) {
     constexpr int WAVES_M = 2, WAVES_N = 2;
     constexpr int MF = BM / WAVES_M / 32, NF = BN / WAVES_N / 32;
     constexpr int OUT_N = EPI == E32_SWIGLU ? BN / 2 : BN;
-    typedef RowTile<BM, VEC> ATile;
-    typedef typename std::conditional<BKM, KTile<BN, VEC>, RowTile<BN, VEC>>::type BTile;
+    typedef RowTile<float, BM, TKS, VEC> ATile;
+    typedef typename std::conditional<BKM, KTile<float, BN, TKS, VEC>, RowTile<float, BN, TKS, VEC>>::type BTile;
     __shared__ __attribute__((aligned(16))) float As[2][ATile::SIZE];
     __shared__ __attribute__((aligned(16))) float Bs[2][BTile::SIZE];
     __shared__ float ds_sum[EPI == E32_DY1 ? WAVES_N : 1][BM];
@@ -241,7 +126,7 @@ __global__ __launch_bounds__(kThreads) void rows_gemm_f32_kernel(Rows32 p) {
     auto b_at = [&](int nf) { return EPI == E32_SWIGLU ? nf / (NF / 2) * OUT_N + wn * (OUT_N / WAVES_N) + nf % (NF / 2) * 32 : wn * (BN / WAVES_N) + nf * 32; };
     f32x16 acc[MF][NF] = {};
     const int tiles = (p.Kdim + TKS - 1) / TKS;
-    run_k_tiles<ATile, BTile, MF, NF>(tiles, a, b, As, Bs, acc, a_at, b_at, fetch);
+    run_k_tiles<ATile, BTile, TKS / 8, MF, NF>(tiles, a, b, As, Bs, acc, a_at, b_at, fetch);
 
 #pragma unroll
     for (int mf = 0; mf < MF; ++mf)
@@ -319,8 +204,8 @@ struct Dw32 {
 template <typename OutT, bool VEC>
 __global__ __launch_bounds__(kThreads) void dw_gemm_f32_kernel(Dw32 p) {
     constexpr int BN = 64, MF = BM / 64, NF = 1;
-    typedef KTile<BM, VEC> PT;
-    typedef KTile<BN, VEC> QT;
+    typedef KTile<float, BM, TKS, VEC> PT;
+    typedef KTile<float, BN, TKS, VEC> QT;
     __shared__ __attribute__((aligned(16))) float Ps[2][PT::SIZE];
     __shared__ __attribute__((aligned(16))) float Qs[2][QT::SIZE];
     // an XCD takes an equal contiguous run of every expert's tiles, columns fastest: an equal share of the work however
@@ -360,7 +245,7 @@ __global__ __launch_bounds__(kThreads) void dw_gemm_f32_kernel(Dw32 p) {
         locate(rbeg + (t + 1) * TKS);
     };
     const int tiles = (rend - rbeg + TKS - 1) / TKS;
-    run_k_tiles<PT, QT, MF, NF>(tiles, a, b, Ps, Qs, acc, a_at, b_at, fetch);
+    run_k_tiles<PT, QT, TKS / 8, MF, NF>(tiles, a, b, Ps, Qs, acc, a_at, b_at, fetch);
 
     OutT* C = reinterpret_cast<OutT*>(p.C) + (int64_t)e * p.M * p.N;
     const int n = n0 + b_at(0) + lane % 32;

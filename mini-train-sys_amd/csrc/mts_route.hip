@@ -166,8 +166,7 @@ __device__ __forceinline__ void scatter_place(const int (&ev)[kSteps], int K, in
     const uint64_t lt = lanemask_lt();
     if (EW <= kFewExperts) {   // wave-uniform
         // A window of few experts: one ballot per expert ranks the 64 entries of a step, and the next free rows
-        // stay in registers from step to step (the same positions as the loop over the experts present below:
-        // entries of one expert in lane order).
+        // stay in registers from step to step (the same positions as below: entries of one expert in lane order).
         int32_t nx[kFewExperts];
 #pragma unroll
         for (int x = 0; x < kFewExperts; ++x) nx[x] = x < EW ? next[x] : 0;
@@ -201,15 +200,17 @@ __device__ __forceinline__ void scatter_place(const int (&ev)[kSteps], int K, in
         const int e = ev[s];
         const bool valid = e >= 0;
         int pos = -1;
-        uint64_t todo = __ballot(valid);
-        while (todo) {
-            int leader = __ffsll((unsigned long long)todo) - 1;
-            int el = __shfl(e, leader, MTS_WAVE);
-            uint64_t same = __ballot(e == el);
-            int first = next[el];  // every lane reads before the leader updates
-            if (e == el) pos = first + __popcll(same & lt);
-            if (lane == leader) next[el] = first + __popcll(same);
-            todo &= ~same;
+        // the lanes with the same expert: one ballot per bit of the id
+        uint64_t same = __ballot(valid);
+#pragma unroll 1
+        for (int bit = 0; (1 << bit) < EW; ++bit) {
+            const uint64_t set = __ballot((e >> bit) & 1);
+            same &= ((e >> bit) & 1) ? set : ~set;
+        }
+        if (valid) {
+            const int first = next[e];   // every lane reads before the first of its group updates
+            pos = first + __popcll(same & lt);
+            if ((same & lt) == 0) next[e] = first + __popcll(same);
         }
         if (e >= -1 && n < cend) s_reverse[n] = pos;
         if (valid) {
