@@ -83,8 +83,8 @@ class HipOpsBackend(DenseTorchOps):
         return capacity_mask(expert_indices, expert_weights, num_experts, capacity)
 
     # a comparison switch keeps the layer on the three separate operators (switches.py); an instance may also set
-    # this attribute to False, e.g. to have forward hooks on the router module fire (the one-node path does not
-    # call that module)
+    # this attribute to False (the one-node path does not call the router module; the block does not take it when that
+    # module has hooks or a forward of its own)
     offers_moe_layer = SWITCHES.layer_node
 
     # moe_layer takes a capacity limit

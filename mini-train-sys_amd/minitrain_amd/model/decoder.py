@@ -13,7 +13,7 @@ import math
 import torch
 from torch import nn
 
-from minitrain_amd.model.blocks import MoEFeedForward
+from minitrain_amd.model.blocks import MoEFeedForward, runs_as_written
 from minitrain_amd.model.config import ModelConfig
 from minitrain_amd.model.ops import OpsBackend
 
@@ -50,15 +50,10 @@ class RMSNorm(nn.Module):
         return ops.rmsnorm(x, self.weight, self.eps)
 
 
-def is_observed(module: nn.Module) -> bool:
-    """Whether hooks are registered that want the module's own inputs and outputs."""
-    return bool(module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks)
-
-
 def sum_and_norm(norm: RMSNorm, x: torch.Tensor, residual: torch.Tensor | None, ops: OpsBackend):
     """``(x + residual, norm of it)``, in one pass where the backend offers it; ``residual`` None: of ``x`` itself."""
     fused = getattr(ops, "add_rmsnorm", None)
-    if residual is not None and fused is not None and not is_observed(norm):
+    if residual is not None and fused is not None and runs_as_written(norm, RMSNorm):
         return fused(x, residual, norm.weight, norm.eps)
     x = x if residual is None else x + residual
     return x, norm(x, ops)
@@ -141,12 +136,12 @@ class MiniTransformer(nn.Module):
         aux, z, per_layer = [], [], {}
         pending = None
         for block in self.blocks:
-            if is_observed(block):
-                hidden, ffn = block(hidden if pending is None else hidden + pending, self.ops, cos, sin)
-                pending = None
-            else:
+            if runs_as_written(block, TransformerBlock):
                 hidden, ffn = block.residual_forward(hidden, pending, self.ops, cos, sin)
                 pending = ffn.hidden_states
+            else:
+                hidden, ffn = block(hidden if pending is None else hidden + pending, self.ops, cos, sin)
+                pending = None
             aux.append(ffn.router_aux_loss)
             z.append(ffn.router_z_loss)
             for name, value in ffn.router_metrics.items():
