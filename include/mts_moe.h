@@ -46,6 +46,10 @@ extern "C" {
 #define MTS_MAX_MOE_EXPERTS 65534     /* routing metadata and the grouped GEMMs (the reference's
                                          limit, minitrain/kernels/triton/fused_moe.py:55-70)      */
 #define MTS_MAX_TOP_K 8
+/* one launch holds fewer than 2^32 threads */
+#define MTS_MAX_NORM_ROWS (1LL << 26)   /* 64 threads a row  */
+#define MTS_MAX_LOSS_ROWS (1LL << 23)   /* 512 threads a row */
+#define MTS_MAX_ROPE_PAIRS ((1LL << 32) - 256)
 
 int mts_version(void);
 const char* mts_error_string(int code);

@@ -10,7 +10,10 @@
 // Nothing here synchronises with the GPU.  Every buffer is a torch tensor from the caching allocator; the backward pass of
 // the operator forks two side streams for kernels that do not depend on one another and joins them before it returns.
 #include <ATen/ATen.h>
+#include <ATen/PythonTorchFunctionTLS.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime.h>
 #include <pybind11/pybind11.h>
@@ -61,6 +64,23 @@ bool aligned16(const Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr(
 Tensor dense16(const Tensor& t) {   // dense and starting on a 16-byte boundary (a view may start inside an allocation)
     Tensor d = t.contiguous();
     return aligned16(d) ? d : d.clone();
+}
+// Whether a kernel may be run on the tensors' memory in the place of stock operators: not where those are looked at by a
+// function transform (vmap, grad, forward mode), a trace, a dispatch mode or a subclass.
+bool nobody_looks() {
+    using c10::DispatchKey;
+    return !c10::impl::tls_is_dispatch_key_included(DispatchKey::FuncTorchDynamicLayerFrontMode) &&
+           !c10::impl::tls_is_dispatch_key_included(DispatchKey::Tracer) && !c10::impl::TorchDispatchModeTLS::any_modes_set() &&
+           !at::impl::torch_function_mode_enabled();
+}
+bool is_plain(const Tensor& t) {
+    static const c10::DispatchKeySet wrapped({c10::DispatchKey::Python, c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
+                                              c10::DispatchKey::Functionalize, c10::DispatchKey::Conjugate, c10::DispatchKey::Negative});
+    return !t.key_set().has_any(wrapped) && !t._fw_grad(/*level=*/0).defined();
+}
+template <typename... Ts>
+bool all_plain(const Ts&... t) {
+    return nobody_looks() && (is_plain(t) && ...);
 }
 int64_t round4(int64_t n) { return (n + 3) / 4 * 4; }
 
@@ -118,8 +138,8 @@ bool needs_padding(const Tensor& x, const Tensor& w1) {
 // Up to 16 experts the projection kernels keep W_r in LDS; more take the kernels on the fp32 matrix instruction.
 constexpr int64_t kFewExperts = 16;
 bool router_logits_supported(const Tensor& x, const Tensor& w) {
-    return x.is_cuda() && w.is_cuda() && x.dim() == 2 && w.dim() == 2 && is_activation_type(x.scalar_type()) && w.scalar_type() == at::kFloat &&
-           x.size(0) > 0 && x.size(1) == w.size(1) &&
+    return all_plain(x, w) && x.is_cuda() && w.is_cuda() && x.dim() == 2 && w.dim() == 2 && is_activation_type(x.scalar_type()) &&
+           w.scalar_type() == at::kFloat && x.size(0) > 0 && x.size(1) == w.size(1) &&
            (w.size(0) <= kFewExperts ? x.size(1) % 4 == 0 && x.size(1) <= 4096 && w.size(0) * w.size(1) * 4 <= 128 * 1024
                                      : mts_router_wide_supported(x.size(1), w.size(0)));
 }
@@ -632,8 +652,7 @@ struct RouterPostprocess : torch::autograd::Function<RouterPostprocess> {
 
 // logits = float(x) @ W_r^T without the fp32 copy of x; backward gives dx in x's dtype.
 struct RouterLogits : torch::autograd::Function<RouterLogits> {
-    static Tensor forward(AutogradContext* ctx, const Tensor& x_, const Tensor& w_) {
-        const Tensor x = x_.contiguous(), w = w_.contiguous();
+    static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w) {   // dense
         Tensor logits = f32({x.size(0), w.size(0)}, x);
         router_projection_forward(x, w, logits);
         ctx->save_for_backward({x, w});
@@ -643,6 +662,7 @@ struct RouterLogits : torch::autograd::Function<RouterLogits> {
         const variable_list s = ctx->get_saved_variables();
         c10::OptionalDeviceGuard guard(s[0].device());
         const Tensor g = like_f32(grads[0]);
+        if (at::GradMode::is_enabled()) return {g.matmul(s[1]).to(s[0].scalar_type()), g.t().matmul(s[0].to(at::kFloat))};   // differentiable
         Tensor dx = at::empty_like(s[0]), dw = at::empty_like(s[1]);
         router_projection_backward(g, s[0], s[1], dx, dw);
         return {dx, dw};
@@ -651,27 +671,30 @@ struct RouterLogits : torch::autograd::Function<RouterLogits> {
 
 // ---- the decoder's dense operators -----------------------------------------------------------------------------------------------
 
+// Each gives way to stock operators where all_plain() does not hold, and computes a gradient that is itself to be
+// differentiated (create_graph) with them.
+
 bool rmsnorm_supported(const Tensor& x, const Tensor& w, const MaybeTensor& residual) {
-    if (!(x.is_cuda() && w.is_cuda() && is_activation_type(x.scalar_type()) && w.scalar_type() == at::kFloat && w.dim() == 1 && x.dim() >= 1 &&
-          x.size(-1) == w.size(0) && x.numel() > 0 && mts_rmsnorm_supported(x.size(-1))))
+    if (!(all_plain(x, w) && (!residual || is_plain(*residual)) && x.is_cuda() && w.is_cuda() && is_activation_type(x.scalar_type()) && w.scalar_type() == at::kFloat && w.dim() == 1 && x.dim() >= 1 &&
+          x.size(-1) == w.size(0) && x.numel() > 0 && x.numel() / x.size(-1) < MTS_MAX_NORM_ROWS && mts_rmsnorm_supported(x.size(-1))))
         return false;
     return !residual || (residual->is_cuda() && residual->scalar_type() == x.scalar_type() && residual->sizes() == x.sizes());
 }
 
 // y, or (x + residual, y) with a residual
 struct RMSNorm : torch::autograd::Function<RMSNorm> {
-    static variable_list forward(AutogradContext* ctx, const Tensor& x_, const MaybeTensor& residual_, const Tensor& w_, double eps) {
-        const Tensor x = dense16(x_), w = dense16(w_);
+    static variable_list forward(AutogradContext* ctx, const Tensor& x, const MaybeTensor& residual_, const Tensor& w, double eps) {   // dense16
         const int64_t H = x.size(-1), N = x.numel() / H;
         Tensor residual, total = x, y = at::empty_like(x), rstd = f32({N}, x);
         if (residual_) {
-            residual = dense16(*residual_);
+            residual = *residual_;
             total = at::empty_like(x);
         }
         check(mts_rmsnorm_fwd(ptr(x), ptr(residual), ptr_as<float>(w), N, H, eps, dtype_code(x), residual_ ? ptr(total) : nullptr, ptr(y), ptr_as<float>(rstd),
                               stream_of(x)),
               "mts_rmsnorm_fwd");
         ctx->save_for_backward({total, w, rstd});
+        ctx->saved_data["eps"] = eps;
         ctx->set_materialize_grads(false);
         if (residual_) return {total, y};
         return {y};
@@ -683,6 +706,14 @@ struct RMSNorm : torch::autograd::Function<RMSNorm> {
         if (!g_y.defined()) return {g_sum, with_sum ? g_sum : Tensor(), Tensor(), Tensor()};   // only the residual stream goes on
         c10::OptionalDeviceGuard guard(s[0].device());
         const int64_t H = s[0].size(-1), N = s[0].numel() / H, ws_bytes = mts_rmsnorm_bwd_workspace_bytes(N, H);
+        if (at::GradMode::is_enabled()) {
+            const Tensor v = s[0].to(at::kFloat), r = at::rsqrt(v.square().mean(-1, true) + ctx->saved_data["eps"].toDouble()), n = v * r;
+            const Tensor gy = g_y.to(at::kFloat), gw = gy * s[1];
+            Tensor d = r * (gw - n * (gw * n).mean(-1, true));
+            if (g_sum.defined()) d = d + g_sum.to(at::kFloat);
+            d = d.to(s[0].scalar_type());
+            return {d, with_sum ? d : Tensor(), (gy * n).reshape({N, H}).sum(0), Tensor()};
+        }
         g_y = dense16(g_y);
         if (g_sum.defined()) g_sum = dense16(g_sum);
         Tensor d_sum = at::empty_like(s[0]), dw = at::empty_like(s[1]), ws = bytes(ws_bytes, s[0]);
@@ -693,33 +724,33 @@ struct RMSNorm : torch::autograd::Function<RMSNorm> {
     }
 };
 
-enum RopeMode { TURN = 0, TURN_BACK = 1, COPY = 2 };
+enum RopeMode : int64_t { TURN = 0, TURN_BACK = 1, COPY = 2 };
 
 bool rope_table_fits(const Tensor& t, const Tensor& like, int64_t S, int64_t D) {
     return t.is_cuda() && t.scalar_type() == like.scalar_type() && t.dim() == 2 && t.size(0) == S && t.size(1) == D && t.is_contiguous() && !t.requires_grad();
 }
 bool rope_supported(const Tensor& q, const Tensor& k, const Tensor& cos, const Tensor& sin) {
-    if (!(q.is_cuda() && k.is_cuda() && q.dim() == 4 && q.sizes() == k.sizes() && q.scalar_type() == k.scalar_type() && is_activation_type(q.scalar_type()) &&
+    if (!(all_plain(q, k, cos, sin) && q.is_cuda() && k.is_cuda() && q.dim() == 4 && q.sizes() == k.sizes() && q.scalar_type() == k.scalar_type() && is_activation_type(q.scalar_type()) &&
           q.numel() > 0))
         return false;
     const int64_t S = q.size(2), D = q.size(3);
-    return D % 2 == 0 && q.size(0) * S < k2GiB && rope_table_fits(cos, q, S, D) && rope_table_fits(sin, q, S, D);
+    return D % 2 == 0 && q.numel() / 2 < MTS_MAX_ROPE_PAIRS && rope_table_fits(cos, q, S, D) && rope_table_fits(sin, q, S, D);
 }
 bool qkv_rope_supported(const Tensor& qkv, const Tensor& cos, const Tensor& sin, int64_t heads) {
-    if (!(qkv.is_cuda() && qkv.dim() == 3 && is_activation_type(qkv.scalar_type()) && qkv.numel() > 0 && qkv.size(2) % (3 * heads) == 0)) return false;
+    if (!(all_plain(qkv, cos, sin) && qkv.is_cuda() && qkv.dim() == 3 && is_activation_type(qkv.scalar_type()) && qkv.numel() > 0 && qkv.size(2) % (3 * heads) == 0)) return false;
     const int64_t S = qkv.size(1), D = qkv.size(2) / (3 * heads);
-    return D % 2 == 0 && qkv.size(0) * S < k2GiB && rope_table_fits(cos, qkv, S, D) && rope_table_fits(sin, qkv, S, D);
+    return D % 2 == 0 && qkv.numel() / 6 < MTS_MAX_ROPE_PAIRS && rope_table_fits(cos, qkv, S, D) && rope_table_fits(sin, qkv, S, D);
 }
 
 struct RopeJob {
     Tensor in, out;   // [B, heads, S, D], any strides but a dense last dimension
-    int mode;
+    int64_t mode;
 };
 void launch_rope(const std::vector<RopeJob>& jobs, const Tensor& cos, const Tensor& sin) {
     MtsRopeTensor array[3];
     for (size_t i = 0; i < jobs.size(); ++i) {
         const Tensor &a = jobs[i].in, &b = jobs[i].out;
-        array[i] = {ptr(a), ptr(b), a.stride(0), a.stride(2), a.stride(1), b.stride(0), b.stride(2), b.stride(1), jobs[i].mode};
+        array[i] = {ptr(a), ptr(b), a.stride(0), a.stride(2), a.stride(1), b.stride(0), b.stride(2), b.stride(1), (int)jobs[i].mode};
     }
     const Tensor& t = jobs[0].in;
     check(mts_rope(array, (int)jobs.size(), ptr(cos), ptr(sin), t.size(0), t.size(2), t.size(1), t.size(3), dtype_code(t), stream_of(t)), "mts_rope");
@@ -729,21 +760,23 @@ Tensor dense_rows(const Tensor& t) { return t.stride(-1) == 1 ? t : t.contiguous
 Tensor heads_inside(const Tensor& like, int64_t B, int64_t heads, int64_t S, int64_t D) { return at::empty({B, S, heads, D}, like.options()).transpose(1, 2); }
 
 struct Rope : torch::autograd::Function<Rope> {
-    static variable_list turn(const Tensor& q_, const Tensor& k_, const Tensor& cos, const Tensor& sin, int mode) {
+    static variable_list turn(const Tensor& q_, const Tensor& k_, const Tensor& cos, const Tensor& sin, int64_t mode) {
         const Tensor q = dense_rows(q_), k = dense_rows(k_);
         Tensor a = heads_inside(q, q.size(0), q.size(1), q.size(2), q.size(3)), b = heads_inside(q, q.size(0), q.size(1), q.size(2), q.size(3));
         launch_rope({{q, a, mode}, {k, b, mode}}, cos, sin);
         return {a, b};
     }
-    static variable_list forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& cos, const Tensor& sin) {
+    static variable_list forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& cos, const Tensor& sin, int64_t mode) {
         ctx->save_for_backward({cos, sin});
-        return turn(q, k, cos, sin, TURN);
+        ctx->saved_data["back"] = mode == TURN ? (int64_t)TURN_BACK : (int64_t)TURN;
+        return turn(q, k, cos, sin, mode);
     }
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
         const variable_list s = ctx->get_saved_variables();
         c10::OptionalDeviceGuard guard(s[0].device());
-        const variable_list g = turn(grads[0], grads[1], s[0], s[1], TURN_BACK);
-        return {g[0], g[1], Tensor(), Tensor()};
+        const int64_t back = ctx->saved_data["back"].toInt();   // each turn is the other's gradient
+        const variable_list g = at::GradMode::is_enabled() ? Rope::apply(grads[0], grads[1], s[0], s[1], back) : turn(grads[0], grads[1], s[0], s[1], back);
+        return {g[0], g[1], Tensor(), Tensor(), Tensor()};
     }
 };
 
@@ -773,6 +806,12 @@ struct QkvRope : torch::autograd::Function<QkvRope> {
         if (!first) return variable_list(4);
         c10::OptionalDeviceGuard guard(s[0].device());
         const int64_t B = first->size(0), heads = first->size(1), S = first->size(2), D = first->size(3);
+        if (at::GradMode::is_enabled()) {
+            auto part = [&](int i) { return grads[i].defined() ? grads[i] : at::zeros_like(*first); };
+            const variable_list qk = Rope::apply(part(0), part(1), s[0], s[1], (int64_t)TURN_BACK);
+            return {at::stack({qk[0].transpose(1, 2), qk[1].transpose(1, 2), part(2).transpose(1, 2)}, 2).view({B, S, 3 * heads * D}), Tensor(), Tensor(),
+                    Tensor()};
+        }
         // zeros where a part took no part in the loss
         Tensor out = given == 3 ? at::empty({B, S, 3, heads, D}, first->options()) : at::zeros({B, S, 3, heads, D}, first->options());
         std::vector<RopeJob> jobs;
@@ -786,15 +825,14 @@ struct QkvRope : torch::autograd::Function<QkvRope> {
 constexpr int64_t kIgnoreIndex = -100;   // torch's default
 
 bool cross_entropy_supported(const Tensor& logits, const Tensor& targets) {
-    return logits.is_cuda() && targets.is_cuda() && logits.dim() == 2 && targets.dim() == 1 && is_activation_type(logits.scalar_type()) &&
-           targets.scalar_type() == at::kLong && logits.size(0) == targets.size(0) && logits.size(0) > 0 && logits.size(0) < k2GiB && logits.size(1) > 0 &&
+    return all_plain(logits, targets) && logits.is_cuda() && targets.is_cuda() && logits.dim() == 2 && targets.dim() == 1 && is_activation_type(logits.scalar_type()) &&
+           targets.scalar_type() == at::kLong && logits.size(0) == targets.size(0) && logits.size(0) > 0 && logits.size(0) < MTS_MAX_LOSS_ROWS && logits.size(1) > 0 &&
            logits.size(1) < k2GiB;
 }
 
 // mean cross-entropy without an fp32 copy of the logits
 struct CrossEntropy : torch::autograd::Function<CrossEntropy> {
-    static Tensor forward(AutogradContext* ctx, const Tensor& logits_, const Tensor& targets_) {
-        const Tensor logits = dense16(logits_), targets = targets_.contiguous();
+    static Tensor forward(AutogradContext* ctx, const Tensor& logits, const Tensor& targets) {   // dense16, dense
         const int64_t N = logits.size(0), V = logits.size(1);
         Tensor rows = f32({3, N}, logits), scalars = f32({2}, logits);   // per row: maximum, log of the sum, loss; loss, 1 / count
         float* row = ptr_as<float>(rows);
@@ -810,6 +848,11 @@ struct CrossEntropy : torch::autograd::Function<CrossEntropy> {
         c10::OptionalDeviceGuard guard(s[0].device());
         const int64_t N = s[0].size(0), V = s[0].size(1);
         const Tensor g = like_f32(grads[0]);
+        if (at::GradMode::is_enabled()) {
+            const Tensor t = s[1].unsqueeze(1), hit = at::arange(V, s[1].options()).unsqueeze(0).eq(t);
+            const Tensor p = at::softmax(s[0].to(at::kFloat), 1) - hit.to(at::kFloat);
+            return {at::where(t.eq(kIgnoreIndex), at::zeros({}, p.options()), p * (g * s[3].select(0, 1))).to(s[0].scalar_type()), Tensor()};
+        }
         Tensor d = at::empty_like(s[0]);
         const float* row = ptr_as<float>(s[2]);
         check(mts_cross_entropy_bwd(ptr(s[0]), ptr_as<int64_t>(s[1]), N, V, kIgnoreIndex, dtype_code(s[0]), row, row + N, ptr_as<float>(g),
@@ -848,22 +891,22 @@ PYBIND11_MODULE(_host, m) {
     });
     m.def("router_logits", [](const Tensor& x, const Tensor& w) {
         c10::OptionalDeviceGuard guard(x.device());
-        return RouterLogits::apply(x, w);
+        return RouterLogits::apply(x.contiguous(), w.contiguous());
     });
     m.def("rmsnorm_supported", &rmsnorm_supported);
     m.def("rmsnorm", [](const Tensor& x, const Tensor& w, double eps) {
         c10::OptionalDeviceGuard guard(x.device());
-        return RMSNorm::apply(x, MaybeTensor(), w, eps)[0];
+        return RMSNorm::apply(dense16(x), MaybeTensor(), dense16(w), eps)[0];
     });
     m.def("add_rmsnorm", [](const Tensor& x, const Tensor& residual, const Tensor& w, double eps) {
         c10::OptionalDeviceGuard guard(x.device());
-        const variable_list v = RMSNorm::apply(x, MaybeTensor(residual), w, eps);
+        const variable_list v = RMSNorm::apply(dense16(x), MaybeTensor(dense16(residual)), dense16(w), eps);
         return std::make_tuple(v[0], v[1]);
     });
     m.def("rope_supported", &rope_supported);
     m.def("rope", [](const Tensor& q, const Tensor& k, const Tensor& cos, const Tensor& sin) {
         c10::OptionalDeviceGuard guard(q.device());
-        const variable_list v = Rope::apply(q, k, cos, sin);
+        const variable_list v = Rope::apply(q, k, cos, sin, (int64_t)TURN);
         return std::make_tuple(v[0], v[1]);
     });
     m.def("qkv_rope_supported", &qkv_rope_supported);
@@ -875,6 +918,6 @@ PYBIND11_MODULE(_host, m) {
     m.def("cross_entropy_supported", &cross_entropy_supported);
     m.def("cross_entropy", [](const Tensor& logits, const Tensor& targets) {
         c10::OptionalDeviceGuard guard(logits.device());
-        return CrossEntropy::apply(logits, targets);
+        return CrossEntropy::apply(dense16(logits), targets.contiguous());
     });
 }

@@ -247,7 +247,8 @@ struct RopeArgs {
     RopeTensor<ET> t[3];
     const ET* cos;
     const ET* sin;
-    int B, S, heads, D;
+    int64_t B, S;
+    int heads, D;
 };
 
 // The products are rounded to the activation dtype before they are added, as separate elementwise operators leave them.
@@ -256,14 +257,14 @@ __global__ __launch_bounds__(256) void rope_kernel(RopeArgs<ET> a) {
     typedef __attribute__((ext_vector_type(VEC))) ET vec;
     const RopeTensor<ET>& t = a.t[blockIdx.y];
     const int half = a.D / 2, chunks = half / VEC;
-    const int64_t total = (int64_t)a.B * a.S * a.heads * chunks;
+    const int64_t total = a.B * a.S * a.heads * chunks;
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= total) return;
     const int c = (int)(i % chunks) * VEC;
     const int64_t rest = i / chunks;
     const int h = (int)(rest % a.heads);
     const int64_t tok = rest / a.heads;
-    const int s = (int)(tok % a.S);
+    const int64_t s = tok % a.S;
     const int64_t b = tok / a.S;
     const ET* in = t.in + b * t.in_b + s * t.in_s + h * t.in_h + c;
     ET* out = t.out + b * t.out_b + s * t.out_s + h * t.out_h + c;
@@ -273,8 +274,8 @@ __global__ __launch_bounds__(256) void rope_kernel(RopeArgs<ET> a) {
         *reinterpret_cast<vec*>(out + half) = v2;
         return;
     }
-    const ET* cs = a.cos + (int64_t)s * a.D + c;
-    const ET* sn = a.sin + (int64_t)s * a.D + c;
+    const ET* cs = a.cos + s * a.D + c;
+    const ET* sn = a.sin + s * a.D + c;
     const vec c1 = *reinterpret_cast<const vec*>(cs), c2 = *reinterpret_cast<const vec*>(cs + half);
     const vec s1 = *reinterpret_cast<const vec*>(sn), s2 = *reinterpret_cast<const vec*>(sn + half);
     vec o1, o2;
@@ -310,7 +311,7 @@ int launch_rope(const MtsRopeTensor* tensors, int count, const void* cos, const 
     fits(cos, 0, 0, 0);
     fits(sin, 0, 0, 0);
     a.cos = (const ET*)cos, a.sin = (const ET*)sin;
-    a.B = (int)B, a.S = (int)S, a.heads = heads, a.D = D;
+    a.B = B, a.S = S, a.heads = heads, a.D = D;
     const int64_t total = B * S * heads * (D / 2 / vec);
     const dim3 grid((unsigned)((total + 255) / 256), count);
     if (vec == 8) {
@@ -511,7 +512,7 @@ extern "C" int mts_rmsnorm_supported(int H) { return H > 0 && H % 4 == 0 && norm
 extern "C" int mts_rmsnorm_fwd(const void* x, const void* residual, const float* weight, int64_t N, int H, float eps, int act_dtype, void* sum,
                                void* y, float* rstd, void* stream) {
     if (!x || !weight || !y || !rstd || (residual && !sum)) return MTS_ERR_NULL;
-    if (N <= 0 || !mts_rmsnorm_supported(H)) return MTS_ERR_SHAPE;
+    if (N <= 0 || N >= MTS_MAX_NORM_ROWS || !mts_rmsnorm_supported(H)) return MTS_ERR_SHAPE;
     if (!dense_dtype_ok(act_dtype)) return MTS_ERR_DTYPE;
     if (!mts_aligned16(x) || !mts_aligned16(residual) || !mts_aligned16(weight) || !mts_aligned16(sum) || !mts_aligned16(y)) return MTS_ERR_ALIGN;
     hipStream_t st = (hipStream_t)stream;
@@ -529,7 +530,7 @@ extern "C" int64_t mts_rmsnorm_bwd_workspace_bytes(int64_t N, int H) { return (i
 extern "C" int mts_rmsnorm_bwd(const void* g_y, const void* g_sum, const void* sum, const float* weight, const float* rstd, int64_t N, int H,
                                int act_dtype, void* d_sum, float* d_weight, void* workspace, int64_t workspace_bytes, void* stream) {
     if (!g_y || !sum || !weight || !rstd || !d_sum || !d_weight || !workspace) return MTS_ERR_NULL;
-    if (N <= 0 || !mts_rmsnorm_supported(H)) return MTS_ERR_SHAPE;
+    if (N <= 0 || N >= MTS_MAX_NORM_ROWS || !mts_rmsnorm_supported(H)) return MTS_ERR_SHAPE;
     if (!dense_dtype_ok(act_dtype)) return MTS_ERR_DTYPE;
     if (workspace_bytes < mts_rmsnorm_bwd_workspace_bytes(N, H)) return MTS_ERR_WORKSPACE;
     if (!mts_aligned16(g_y) || !mts_aligned16(g_sum) || !mts_aligned16(sum) || !mts_aligned16(weight) || !mts_aligned16(d_sum) ||
@@ -550,8 +551,8 @@ extern "C" int mts_rmsnorm_bwd(const void* g_y, const void* g_sum, const void* s
 extern "C" int mts_rope(const MtsRopeTensor* tensors, int count, const void* cos, const void* sin, int64_t B, int64_t S, int heads, int head_dim,
                         int act_dtype, void* stream) {
     if (!tensors || !cos || !sin) return MTS_ERR_NULL;
-    if (count < 1 || count > 3 || B <= 0 || S <= 0 || heads <= 0 || head_dim <= 0 || head_dim % 2 || B * S >= (1LL << 31)) return MTS_ERR_SHAPE;
-    if (B * S * heads * (head_dim / 2) / 256 >= (1LL << 31)) return MTS_ERR_SHAPE;
+    if (count < 1 || count > 3 || B <= 0 || S <= 0 || heads <= 0 || head_dim <= 0 || head_dim % 2) return MTS_ERR_SHAPE;
+    if (B * S * heads * (head_dim / 2) >= MTS_MAX_ROPE_PAIRS) return MTS_ERR_SHAPE;
     for (int i = 0; i < count; ++i) {
         if (!tensors[i].in || !tensors[i].out) return MTS_ERR_NULL;
         if (tensors[i].mode < ROPE_TURN || tensors[i].mode > ROPE_COPY) return MTS_ERR_SHAPE;
@@ -568,7 +569,7 @@ extern "C" int mts_rope(const MtsRopeTensor* tensors, int count, const void* cos
 extern "C" int mts_cross_entropy_fwd(const void* logits, const int64_t* targets, int64_t N, int V, int64_t ignore_index, int dtype, float* row_max,
                                      float* row_log_sum, float* row_loss, float* loss, float* inv_count, void* stream) {
     if (!logits || !targets || !row_max || !row_log_sum || !row_loss || !loss || !inv_count) return MTS_ERR_NULL;
-    if (N <= 0 || N >= (1LL << 31) || V <= 0) return MTS_ERR_SHAPE;
+    if (N <= 0 || N >= MTS_MAX_LOSS_ROWS || V <= 0) return MTS_ERR_SHAPE;
     if (!dense_dtype_ok(dtype)) return MTS_ERR_DTYPE;
     if (!mts_aligned16(logits)) return MTS_ERR_ALIGN;
     hipStream_t st = (hipStream_t)stream;
@@ -585,7 +586,7 @@ extern "C" int mts_cross_entropy_fwd(const void* logits, const int64_t* targets,
 extern "C" int mts_cross_entropy_bwd(const void* logits, const int64_t* targets, int64_t N, int V, int64_t ignore_index, int dtype, const float* row_max,
                                      const float* row_log_sum, const float* g_loss, const float* inv_count, void* d_logits, void* stream) {
     if (!logits || !targets || !row_max || !row_log_sum || !g_loss || !inv_count || !d_logits) return MTS_ERR_NULL;
-    if (N <= 0 || N >= (1LL << 31) || V <= 0) return MTS_ERR_SHAPE;
+    if (N <= 0 || N >= MTS_MAX_LOSS_ROWS || V <= 0) return MTS_ERR_SHAPE;
     if (!dense_dtype_ok(dtype)) return MTS_ERR_DTYPE;
     if (!mts_aligned16(logits) || !mts_aligned16(d_logits)) return MTS_ERR_ALIGN;
     hipStream_t st = (hipStream_t)stream;

@@ -39,6 +39,10 @@ class HipOpsBackend(DenseTorchOps):
     # The decoder's operators around its matrix products: one kernel where the stock operators are a chain of
     # elementwise and reduction kernels; what the kernels do not take (CPU tensors, other types and layouts) stays stock.
 
+    def _is_own(self, name) -> bool:
+        """Whether an operator is this class's, so that a fused form may stand in for it."""
+        return getattr(getattr(self, name), "__func__", None) is _OWN[name]
+
     def rmsnorm(self, x, weight, eps):
         if dense.is_rmsnorm_supported(x, weight):
             return dense.rmsnorm(x, weight, eps)
@@ -46,10 +50,10 @@ class HipOpsBackend(DenseTorchOps):
 
     def add_rmsnorm(self, x, residual, weight, eps):
         """Extension: ``(x + residual, rmsnorm(x + residual))`` in one pass."""
-        if dense.is_rmsnorm_supported(x, weight, residual):
+        if self._is_own("rmsnorm") and dense.is_rmsnorm_supported(x, weight, residual):
             return dense.add_rmsnorm(x, residual, weight, eps)
         total = x + residual
-        return total, super().rmsnorm(total, weight, eps)
+        return total, self.rmsnorm(total, weight, eps)
 
     def rope(self, q, k, cos, sin):
         if dense.is_rope_supported(q, k, cos, sin):
@@ -59,7 +63,7 @@ class HipOpsBackend(DenseTorchOps):
     def qkv_rope(self, qkv, cos, sin, heads):
         """Extension: rotated queries and keys and the values ``[B, heads, S, D]`` of a packed projection, or None when
         the kernel does not take it (the caller then splits the projection and calls ``rope``)."""
-        if not dense.is_qkv_rope_supported(qkv, cos, sin, heads):
+        if not self._is_own("rope") or not dense.is_qkv_rope_supported(qkv, cos, sin, heads):
             return None
         return dense.qkv_rope(qkv, cos, sin, heads)
 
@@ -106,6 +110,8 @@ class HipOpsBackend(DenseTorchOps):
             return None
         return router_logits(hidden_states, weight)
 
+
+_OWN = {name: getattr(HipOpsBackend, name) for name in ("rmsnorm", "rope")}
 
 __all__ = [
     "HipOpsBackend",

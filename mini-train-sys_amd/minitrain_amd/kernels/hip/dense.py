@@ -8,11 +8,19 @@ everything else (CPU tensors, other dtypes or layouts) to the stock operators.  
 are native (``csrc/host/mts_host.cpp``).
 """
 
+import torch
+from torch.overrides import has_torch_function
+
 from minitrain_amd import _lib
 
 
+def _may_replace(*tensors) -> bool:
+    """The stock operators stay where a compiler traces them or a subclass wants to see them."""
+    return not torch.compiler.is_compiling() and not has_torch_function(tensors)
+
+
 def is_rmsnorm_supported(x, weight, residual=None) -> bool:
-    return _lib.host().rmsnorm_supported(x, weight, residual)
+    return _may_replace(x, weight, residual) and _lib.host().rmsnorm_supported(x, weight, residual)
 
 
 def rmsnorm(x, weight, eps: float):
@@ -25,7 +33,7 @@ def add_rmsnorm(x, residual, weight, eps: float):
 
 
 def is_rope_supported(q, k, cos, sin) -> bool:
-    return _lib.host().rope_supported(q, k, cos, sin)
+    return _may_replace(q, k, cos, sin) and _lib.host().rope_supported(q, k, cos, sin)
 
 
 def rope(q, k, cos, sin):
@@ -33,7 +41,7 @@ def rope(q, k, cos, sin):
 
 
 def is_qkv_rope_supported(qkv, cos, sin, heads: int) -> bool:
-    return _lib.host().qkv_rope_supported(qkv, cos, sin, heads)
+    return _may_replace(qkv, cos, sin) and _lib.host().qkv_rope_supported(qkv, cos, sin, heads)
 
 
 def qkv_rope(qkv, cos, sin, heads: int):
@@ -42,7 +50,7 @@ def qkv_rope(qkv, cos, sin, heads: int):
 
 
 def is_cross_entropy_supported(logits, targets) -> bool:
-    return _lib.host().cross_entropy_supported(logits, targets)
+    return _may_replace(logits, targets) and _lib.host().cross_entropy_supported(logits, targets)
 
 
 def cross_entropy(logits, targets):

@@ -1,0 +1,126 @@
+"""The decoder's dense operators where something other than a plain first-order pass wants their gradients: function
+transforms, forward mode, dispatch modes and gradients of gradients give what the stock operators give (GPU, fp32)."""
+
+import pytest
+import torch
+
+from minitrain_amd.kernels.dense_ops import DenseTorchOps
+from minitrain_amd.kernels.hip import HipOpsBackend, dense
+from tests.helpers import hip_backend
+
+pytestmark = pytest.mark.gpu
+
+STOCK = DenseTorchOps()
+TOL = dict(rtol=2e-5, atol=2e-5)   # fp32 sums of at most 64 terms of order one, in another order
+
+
+def _operands(name):
+    g = torch.Generator().manual_seed(5)
+    r = lambda *shape: torch.randn(*shape, generator=g).cuda()
+    if name == "rmsnorm":
+        return (r(6, 64), 1 + 0.1 * r(64)), lambda ops, x, w: ops.rmsnorm(x, w, 1e-5)
+    if name == "add_rmsnorm":
+        def both(ops, x, residual, w):
+            if hasattr(ops, "add_rmsnorm"):
+                return torch.cat(ops.add_rmsnorm(x, residual, w, 1e-5))
+            return torch.cat((x + residual, ops.rmsnorm(x + residual, w, 1e-5)))
+        return (r(6, 64), r(6, 64), 1 + 0.1 * r(64)), both
+    if name == "cross_entropy":
+        targets = torch.tensor([1, 0, -100, 6, 3, 3], device="cuda")
+        return (r(6, 7),), lambda ops, x: ops.cross_entropy(x, targets)
+    angle = r(5, 8)
+    cos, sin = angle.cos(), angle.sin()
+    if name == "rope":
+        return (r(2, 3, 5, 8), r(2, 3, 5, 8)), lambda ops, q, k: torch.stack(ops.rope(q, k, cos, sin))
+
+    def packed(ops, qkv):
+        if hasattr(ops, "qkv_rope"):
+            turned = ops.qkv_rope(qkv, cos, sin, 3)
+            if turned is not None:
+                return torch.stack(turned)
+        q, k, v = (t.view(2, 5, 3, 8).transpose(1, 2) for t in qkv.chunk(3, dim=-1))
+        return torch.stack((*ops.rope(q, k, cos, sin), v))
+    return (r(2, 5, 72),), packed
+
+
+NAMES = ["rmsnorm", "add_rmsnorm", "cross_entropy", "rope", "qkv_rope"]
+
+
+@pytest.mark.parametrize("name", NAMES)
+def test_gradients_of_gradients(name):
+    print(name, flush=True)
+    operands, f = _operands(name)
+    results = []
+    for ops in (hip_backend(), STOCK):
+        leaves = [t.clone().requires_grad_(True) for t in operands]
+        out = f(ops, *leaves)
+        seed = torch.linspace(-1, 1, out.numel(), device="cuda").reshape(out.shape).requires_grad_(True)
+        first = torch.autograd.grad((out.square() * seed).sum(), leaves, create_graph=True)
+        second = torch.autograd.grad(sum((t * t).sum() for t in first), [*leaves, seed])
+        results.append([*first, *second])
+    for got, want in zip(*results):
+        torch.testing.assert_close(got, want, rtol=2e-4, atol=2e-4)   # products of up to five factors of order one to ten
+
+
+@pytest.mark.parametrize("name", NAMES)
+def test_function_transforms(name):
+    print(name, flush=True)
+    operands, f = _operands(name)
+    ops = hip_backend()
+    tangents = tuple(torch.ones_like(t) for t in operands)
+    got, want = (torch.func.jvp(lambda *a: f(o, *a), operands, tangents) for o in (ops, STOCK))
+    torch.testing.assert_close(got, want, **TOL)
+    got, want = (torch.func.grad(lambda *a: f(o, *a).square().sum())(*operands) for o in (ops, STOCK))
+    torch.testing.assert_close(got, want, rtol=1e-4, atol=1e-4)
+    stacked = torch.stack([operands[0], 2 * operands[0]])
+    got, want = (torch.func.vmap(lambda x: f(o, x, *operands[1:]))(stacked) for o in (ops, STOCK))
+    torch.testing.assert_close(got, want, **TOL)
+
+
+@pytest.mark.parametrize("name", NAMES)
+def test_modes_see_the_stock_operators(name):
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    print(name, flush=True)
+    operands, f = _operands(name)
+
+    class Seen(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return func(*args, **(kwargs or {}))
+
+    runs = []
+    for ops in (hip_backend(), STOCK):
+        seen = []
+        with Seen():
+            f(ops, *operands)
+        runs.append(seen)
+    assert runs[0] == runs[1]
+
+
+def test_more_rows_than_one_launch_takes():
+    """A launch holds fewer than 2^32 threads; the predicates look at sizes only (tensors of one element, expanded)."""
+    one = torch.ones(1, 1, device="cuda")
+    w = torch.ones(4, device="cuda")
+    assert dense.is_rmsnorm_supported(one.expand(2**26 - 1, 4), w) and not dense.is_rmsnorm_supported(one.expand(2**26, 4), w)
+    targets = torch.zeros(1, dtype=torch.long, device="cuda")
+    for rows, fits in ((2**23 - 1, True), (2**23, False)):
+        assert dense.is_cross_entropy_supported(one.expand(rows, 4), targets.expand(rows)) is fits
+    table = torch.ones(2**20, 2, device="cuda")
+    for batch, fits in ((2**12 - 1, True), (2**12, False)):
+        assert dense.is_qkv_rope_supported(one.view(1, 1, 1).expand(batch, 2**20, 6), table, table, 1) is fits
+
+
+def test_overridden_operator_is_called():
+    class Doubled(HipOpsBackend):
+        def rmsnorm(self, x, weight, eps):
+            return 2 * super().rmsnorm(x, weight, eps)
+
+        def rope(self, q, k, cos, sin):
+            return k, q
+
+    (x, r, w), _ = _operands("add_rmsnorm")
+    ops = Doubled()
+    torch.testing.assert_close(ops.add_rmsnorm(x, r, w, 1e-5)[1], 2 * STOCK.rmsnorm(x + r, w, 1e-5), **TOL)
+    (qkv,), _ = _operands("qkv_rope")
+    assert ops.qkv_rope(qkv, torch.ones(5, 8, device="cuda"), torch.ones(5, 8, device="cuda"), 3) is None
