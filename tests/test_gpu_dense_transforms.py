@@ -23,7 +23,8 @@ def _operands(name):
         def both(ops, x, residual, w):
             if hasattr(ops, "add_rmsnorm"):
                 return torch.cat(ops.add_rmsnorm(x, residual, w, 1e-5))
-            return torch.cat((x + residual, ops.rmsnorm(x + residual, w, 1e-5)))
+            total = x + residual
+            return torch.cat((total, ops.rmsnorm(total, w, 1e-5)))
         return (r(6, 64), r(6, 64), 1 + 0.1 * r(64)), both
     if name == "cross_entropy":
         targets = torch.tensor([1, 0, -100, 6, 3, 3], device="cuda")
