@@ -475,6 +475,25 @@ int mts_cross_entropy_bwd(const void* logits, const int64_t* targets, int64_t N,
                           const float* row_log_sum, const float* g_loss, const float* inv_count,
                           void* d_logits, void* stream);
 
+/* Scaled dot-product attention of heads of 64 elements, bf16 or fp16, queries and keys of the
+ * same length; causal != 0: query i sees keys 0..i.  Tensors are [B,heads,S,64], dense in the last
+ * dimension, 16-byte aligned, other strides multiples of 8 elements.  fp32 scores, sums and
+ * accumulation; probabilities and score gradients enter their products in act_dtype.
+ * lse [B*heads*S] f32 is kept for the backward pass (log2 of a row's sum of exponentials); delta
+ * [B*heads*S] f32 is scratch.  The gradients are summed in a fixed order.                  */
+typedef struct {
+    void* data;
+    int64_t batch_stride, head_stride, row_stride;   /* elements */
+} MtsHeads;
+int mts_attention_supported(int64_t B, int heads, int64_t S, int head_dim);
+int mts_attention_fwd(const MtsHeads* q, const MtsHeads* k, const MtsHeads* v, int64_t B, int heads,
+                      int64_t S, int causal, int act_dtype, const MtsHeads* out, float* lse,
+                      void* stream);
+int mts_attention_bwd(const MtsHeads* q, const MtsHeads* k, const MtsHeads* v, const MtsHeads* out,
+                      const MtsHeads* d_out, const float* lse, int64_t B, int heads, int64_t S,
+                      int causal, int act_dtype, const MtsHeads* dq, const MtsHeads* dk,
+                      const MtsHeads* dv, float* delta, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

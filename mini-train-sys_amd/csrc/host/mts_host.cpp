@@ -11,6 +11,7 @@
 // the operator forks two side streams for kernels that do not depend on one another and joins them before it returns.
 #include <ATen/ATen.h>
 #include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/autocast_mode.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
@@ -21,6 +22,7 @@
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/utils/pybind.h>
 
+#include <cmath>
 #include <map>
 #include <mutex>
 #include <optional>
@@ -822,6 +824,56 @@ struct QkvRope : torch::autograd::Function<QkvRope> {
     }
 };
 
+bool heads_fit(const Tensor& t) {   // as the kernels read them
+    return t.stride(3) == 1 && t.stride(0) % 8 == 0 && t.stride(1) % 8 == 0 && t.stride(2) % 8 == 0 && aligned16(t);
+}
+bool attention_supported(const Tensor& q, const Tensor& k, const Tensor& v) {
+    if (!(all_plain(q, k, v) && q.is_cuda() && k.device() == q.device() && v.device() == q.device() && q.dim() == 4 && k.sizes() == q.sizes() &&
+          v.sizes() == q.sizes() && (q.scalar_type() == at::kBFloat16 || q.scalar_type() == at::kHalf) && k.scalar_type() == q.scalar_type() &&
+          v.scalar_type() == q.scalar_type() && mts_attention_supported(q.size(0), q.size(1), q.size(2), q.size(3))))
+        return false;
+    // what the caller has chosen for the stock operator stays chosen: another type, another implementation
+    if (at::autocast::is_autocast_enabled(at::kCUDA) && at::autocast::get_autocast_dtype(at::kCUDA) != q.scalar_type()) return false;
+    return at::globalContext().userEnabledFlashSDP() && heads_fit(q) && heads_fit(k) && heads_fit(v);
+}
+
+struct Attention : torch::autograd::Function<Attention> {
+    static MtsHeads view(const Tensor& t) { return {ptr(t), t.stride(0), t.stride(1), t.stride(2)}; }
+    static Tensor forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, bool causal) {
+        const int64_t B = q.size(0), heads = q.size(1), S = q.size(2);
+        Tensor out = heads_inside(q, B, heads, S, q.size(3)), lse = f32({B * heads * S}, q);
+        const MtsHeads vq = view(q), vk = view(k), vv = view(v), vo = view(out);
+        check(mts_attention_fwd(&vq, &vk, &vv, B, heads, S, causal, dtype_code(q), &vo, ptr_as<float>(lse), stream_of(q)), "mts_attention_fwd");
+        ctx->save_for_backward({q, k, v, out, lse});
+        ctx->saved_data["causal"] = causal;
+        return out;
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        const variable_list s = ctx->get_saved_variables();
+        const Tensor &q = s[0], &k = s[1], &v = s[2];
+        c10::OptionalDeviceGuard guard(q.device());
+        const bool causal = ctx->saved_data["causal"].toBool();
+        const int64_t B = q.size(0), heads = q.size(1), S = q.size(2), D = q.size(3);
+        if (at::GradMode::is_enabled()) {   // a gradient that is itself to be differentiated: written out, in fp32
+            const double scale = 1.0 / std::sqrt((double)D);
+            const Tensor qf = q.to(at::kFloat), kf = k.to(at::kFloat), vf = v.to(at::kFloat), g = grads[0].to(at::kFloat);
+            Tensor score = at::matmul(qf, kf.transpose(2, 3).contiguous()) * scale;
+            if (causal) score = score.masked_fill(at::ones({S, S}, q.options().dtype(at::kBool)).triu(1), -INFINITY);
+            const Tensor p = at::softmax(score, -1), dp = at::matmul(g, vf.transpose(2, 3).contiguous());
+            const Tensor ds = p * (dp - (dp * p).sum(-1, true)) * scale;
+            const auto t = q.scalar_type();
+            return {at::matmul(ds, kf).to(t), at::matmul(ds.transpose(2, 3).contiguous(), qf).to(t), at::matmul(p.transpose(2, 3).contiguous(), g).to(t), Tensor()};
+        }
+        const Tensor g = heads_fit(grads[0]) ? grads[0] : dense16(grads[0]);
+        Tensor dq = heads_inside(q, B, heads, S, D), dk = heads_inside(q, B, heads, S, D), dv = heads_inside(q, B, heads, S, D), delta = at::empty_like(s[4]);
+        const MtsHeads vq = view(q), vk = view(k), vv = view(v), vo = view(s[3]), vg = view(g), vdq = view(dq), vdk = view(dk), vdv = view(dv);
+        check(mts_attention_bwd(&vq, &vk, &vv, &vo, &vg, ptr_as<float>(s[4]), B, heads, S, causal, dtype_code(q), &vdq, &vdk, &vdv, ptr_as<float>(delta),
+                                stream_of(q)),
+              "mts_attention_bwd");
+        return {dq, dk, dv, Tensor()};
+    }
+};
+
 constexpr int64_t kIgnoreIndex = -100;   // torch's default
 
 bool cross_entropy_supported(const Tensor& logits, const Tensor& targets) {
@@ -914,6 +966,11 @@ PYBIND11_MODULE(_host, m) {
         c10::OptionalDeviceGuard guard(qkv.device());
         const variable_list v = QkvRope::apply(qkv, cos, sin, heads);
         return std::make_tuple(v[0], v[1], v[2]);
+    });
+    m.def("attention_supported", &attention_supported);
+    m.def("attention", [](const Tensor& q, const Tensor& k, const Tensor& v, bool causal) {
+        c10::OptionalDeviceGuard guard(q.device());
+        return Attention::apply(q, k, v, causal);
     });
     m.def("cross_entropy_supported", &cross_entropy_supported);
     m.def("cross_entropy", [](const Tensor& logits, const Tensor& targets) {

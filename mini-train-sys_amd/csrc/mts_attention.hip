@@ -1,0 +1,483 @@
+// Attention of the decoder for heads of 64 elements, forward and backward, causal or not, without materialised scores.
+//
+// Every product runs on v_mfma_f32_32x32x16 and is laid out so that no score changes lanes.  An accumulator of that
+// instruction holds, for column n = lane % 32, the rows 8 * (i / 4) + 4 * (lane / 32) + i % 4; its 16 x n operand wants
+// 8 values of k per lane.  Which k those are is free as long as the other operand agrees, so eight consecutive
+// accumulator registers serve as an operand as they are, and the other one is read from LDS with rows
+// krow0 + 4 * (lane / 32) + {0..3, 8..11} by the transposing load.  The scores are therefore formed transposed (keys x
+// queries) where they are summed over the keys (output, dQ), and as queries x keys where they are summed over the queries
+// (dK, dV): the operand that a wave owns stays in registers, the other one streams through LDS in tiles of 64 rows.
+//
+// The vector pipe bounds it: for 32 x 64 scores the forward pass issues 512 cycles of MFMA and about 1000 of exponentials (a
+// quarter of the rate), maxima, sums and conversions.  bf16, causal, 12 heads of 64, 1024 rows, against the stock operator:
+// batch 8: 33 us forward (79) and 127 backward (308); batch 24: 75 us (515 TFLOP/s; 168) and 311 (435 TFLOP/s of the seven
+// products that two separate kernels form, so that each gradient is summed by one block in a fixed order; 844).
+#include "mts_common.h"
+
+namespace {
+
+typedef __attribute__((ext_vector_type(4))) short s16x4;
+typedef __attribute__((ext_vector_type(8))) short s16x8;
+
+template <typename ET>
+struct Mma;
+template <>
+struct Mma<bf16_t> {
+    typedef bf16x8 frag;
+    typedef bf16x4 quad;
+    static __device__ __forceinline__ f32x16 mul(frag a, frag b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0); }
+};
+template <>
+struct Mma<mts_f16_t> {
+    typedef mts_f16x8 frag;
+    typedef mts_f16x4 quad;
+    static __device__ __forceinline__ f32x16 mul(frag a, frag b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0); }
+};
+
+constexpr int kHead = 64;               // elements of a head
+constexpr int kTile = 64;               // rows of a streamed tile
+constexpr int kWaves = 4;
+constexpr int kThreads = kWaves * MTS_WAVE;
+constexpr int kOwn = 32 * kWaves;       // rows a block owns, 32 a wave
+constexpr int kTileElems = kTile * kHead;
+constexpr float kLog2e = 1.4426950408889634f;
+
+// [B, heads, S, 64], dense in the last dimension, strides in elements
+template <typename T>
+struct Heads {
+    T* p;
+    int64_t b, h, s;
+    __device__ __forceinline__ T* row0(int64_t bh, int heads) const { return p + (bh / heads) * b + (bh % heads) * h; }
+};
+
+// 16-byte chunk of a row, exchanged so that 16 consecutive rows of one chunk (row fragments) and 4 rows of four chunks
+// (transposed fragments) both fall on all 64 banks
+__device__ __forceinline__ int chunk_off(int row, int chunk) { return row * kHead + ((chunk ^ (((row >> 1) & 1) << 2 | ((row >> 2) & 3))) << 3); }
+
+// rows row0 + lane % 32, elements 16 * ks + 8 * (lane / 32) + 0..7
+template <typename ET>
+__device__ __forceinline__ typename Mma<ET>::frag row_frag(const ET* tile, int row0, int ks) {
+    const int lane = threadIdx.x % MTS_WAVE;
+    return *reinterpret_cast<const typename Mma<ET>::frag*>(tile + chunk_off(row0 + lane % 32, 2 * ks + lane / 32));
+}
+
+// columns col0 + lane % 32, rows krow0 + 4 * (lane / 32) + {0..3, 8..11}
+template <typename ET>
+__device__ __forceinline__ typename Mma<ET>::frag column_frag(const ET* tile, int krow0, int col0) {
+    const int lane = threadIdx.x % MTS_WAVE;
+    const int col = col0 + 16 * ((lane / 16) % 2) + 4 * (lane % 4);
+    s16x4 h[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        const ET* src = tile + chunk_off(krow0 + 8 * q + 4 * (lane / 32) + (lane % 16) / 4, col / 8) + col % 8;
+        h[q] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(src));
+    }
+    const s16x8 v = {h[0][0], h[0][1], h[0][2], h[0][3], h[1][0], h[1][1], h[1][2], h[1][3]};
+    return __builtin_bit_cast(typename Mma<ET>::frag, v);
+}
+
+// A tile on its way from memory to LDS through registers, so that its latency is covered by the tile before it; rows behind
+// the end arrive as zeros.
+template <typename ET>
+struct TileCopy {
+    u32x4 reg[kTileElems / 8 / kThreads];
+    __device__ __forceinline__ void fetch(const ET* head, int64_t stride, int row0, int S) {
+#pragma unroll
+        for (int i = 0; i < (int)(sizeof(reg) / 16); ++i) {
+            const int row = row0 + (threadIdx.x + i * kThreads) / 8, c = threadIdx.x % 8;
+            reg[i] = row < S ? *reinterpret_cast<const u32x4*>(head + row * stride + c * 8) : u32x4{};
+        }
+    }
+    __device__ __forceinline__ void commit(ET* tile) const {
+#pragma unroll
+        for (int i = 0; i < (int)(sizeof(reg) / 16); ++i)
+            *reinterpret_cast<u32x4*>(tile + chunk_off((threadIdx.x + i * kThreads) / 8, threadIdx.x % 8)) = reg[i];
+    }
+};
+
+// the 32 rows a wave owns, as an operand that stays in registers (row row, elements 16 * ks + 8 * (lane / 32) + 0..7)
+template <typename ET>
+__device__ __forceinline__ void own_frags(const ET* row, typename Mma<ET>::frag (&f)[4]) {
+    const int lane = threadIdx.x % MTS_WAVE;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) f[ks] = *reinterpret_cast<const typename Mma<ET>::frag*>(row + 16 * ks + 8 * (lane / 32));
+}
+
+template <typename ET>
+__device__ __forceinline__ typename Mma<ET>::frag narrowed(const f32x16& v, int t) {
+    typename Mma<ET>::frag f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) f[j] = (ET)v[8 * t + j];
+    return f;
+}
+
+// transposed accumulators (64 x 32: two tiles) to the row of this lane's column
+template <typename ET>
+__device__ __forceinline__ void store_row(ET* row, const f32x16 (&acc)[2], float scale) {
+    const int lane = threadIdx.x % MTS_WAVE;
+#pragma unroll
+    for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            typename Mma<ET>::quad o;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) o[r] = (ET)(acc[dt][4 * g + r] * scale);
+            *reinterpret_cast<typename Mma<ET>::quad*>(row + 32 * dt + 8 * g + 4 * (lane / 32)) = o;
+        }
+}
+
+// Blocks of one head on one XCD (its keys and values, or queries and gradients, are read by all of them); `order` counts the
+// blocks of a head, the same for all heads before the next, so that the longest of a causal pass start first.
+struct Where {
+    int64_t bh;
+    int order;
+    __device__ __forceinline__ Where(int64_t BH) {
+        const int64_t j = blockIdx.x / 8, per = (BH + 7) / 8;
+        order = (int)(j / per);
+        bh = (j % per) * 8 + blockIdx.x % 8;
+    }
+};
+
+template <typename ET>
+struct AttnArgs {
+    Heads<const ET> q, k, v, o, dO;
+    Heads<ET> out, dq, dk, dv;
+    float *lse, *delta;   // [BH, S]: log2 of the row's sum of exponentials; sum of dO * O
+    int64_t BH;
+    int heads, S, blocks;
+    float scale;
+};
+
+template <typename ET, bool CAUSAL>
+__global__ __launch_bounds__(kThreads, 3) void attention_fwd_kernel(AttnArgs<ET> a) {
+    typedef typename Mma<ET>::frag frag;
+    __shared__ __align__(16) ET lds[2][2][kTileElems];
+    const Where at(a.BH);
+    if (at.bh >= a.BH) return;
+    const int lane = threadIdx.x % MTS_WAVE, wave = threadIdx.x / MTS_WAVE, half = lane / 32;
+    const int S = a.S, q0 = (CAUSAL ? a.blocks - 1 - at.order : at.order) * kOwn, first = q0 + 32 * wave, row = first + lane % 32;
+    const ET *k = a.k.row0(at.bh, a.heads), *v = a.v.row0(at.bh, a.heads);
+    frag q[4];
+    own_frags<ET>(a.q.row0(at.bh, a.heads) + min(row, S - 1) * a.q.s, q);
+    const float sc = a.scale * kLog2e;
+    float top = -INFINITY, sum = 0.f;
+    f32x16 acc[2] = {};
+    const int end = CAUSAL ? min(S, q0 + kOwn) : S, tiles = (end + kTile - 1) / kTile;
+    TileCopy<ET> kc, vc;
+    kc.fetch(k, a.k.s, 0, S);
+    vc.fetch(v, a.v.s, 0, S);
+    kc.commit(lds[0][0]);
+    vc.commit(lds[0][1]);
+    __syncthreads();
+    for (int t = 0; t < tiles; ++t) {
+        const int kv0 = t * kTile;
+        const ET *kt = lds[t & 1][0], *vt = lds[t & 1][1];
+        if (t + 1 < tiles) {
+            kc.fetch(k, a.k.s, kv0 + kTile, S);
+            vc.fetch(v, a.v.s, kv0 + kTile, S);
+        }
+        if (!CAUSAL || kv0 <= first + 31) {
+            f32x16 s[2] = {};
+#pragma unroll
+            for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+                for (int m = 0; m < 2; ++m) s[m] = Mma<ET>::mul(row_frag(kt, 32 * m, ks), q[ks], s[m]);
+            if (kv0 + kTile > S || (CAUSAL && kv0 + kTile - 1 > first)) {
+                const int last = CAUSAL ? min(row, S - 1) : S - 1;
+#pragma unroll
+                for (int m = 0; m < 2; ++m)
+#pragma unroll
+                    for (int i = 0; i < 16; ++i)
+                        if (kv0 + 32 * m + 8 * (i / 4) + 4 * half + i % 4 > last) s[m][i] = -INFINITY;
+            }
+            float hi = s[0][0];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) hi = fmaxf(hi, fmaxf(s[0][i], s[1][i]));
+            hi = fmaxf(hi, __shfl_xor(hi, 32, MTS_WAVE));
+            if (__any(hi > top)) {
+                const float next = fmaxf(top, hi), keep = next == top ? 1.f : __builtin_amdgcn_exp2f((top - next) * sc);
+                top = next;
+                sum *= keep;
+#pragma unroll
+                for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) acc[dt][i] *= keep;
+            }
+            const float base = top == -INFINITY ? 0.f : -top * sc;   // nothing but -inf so far: every exponential is zero
+#pragma unroll
+            for (int m = 0; m < 2; ++m)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    s[m][i] = __builtin_amdgcn_exp2f(fmaf(s[m][i], sc, base));
+                    sum += s[m][i];
+                }
+#pragma unroll
+            for (int m = 0; m < 2; ++m)
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    const frag p = narrowed<ET>(s[m], u);
+#pragma unroll
+                    for (int dt = 0; dt < 2; ++dt) acc[dt] = Mma<ET>::mul(column_frag(vt, 32 * m + 16 * u, 32 * dt), p, acc[dt]);
+                }
+        }
+        if (t + 1 < tiles) {
+            kc.commit(lds[(t + 1) & 1][0]);
+            vc.commit(lds[(t + 1) & 1][1]);
+        }
+        __syncthreads();
+    }
+    sum += __shfl_xor(sum, 32, MTS_WAVE);
+    if (row >= S) return;
+    store_row(a.out.row0(at.bh, a.heads) + row * a.out.s, acc, 1.f / sum);
+    if (half == 0) a.lse[at.bh * S + row] = top * sc + log2f(sum);
+}
+
+// dQ of 128 queries; also delta, which the other kernel reads.
+template <typename ET, bool CAUSAL>
+__global__ __launch_bounds__(kThreads, 2) void attention_dq_kernel(AttnArgs<ET> a) {
+    typedef typename Mma<ET>::frag frag;
+    __shared__ __align__(16) ET lds[2][2][kTileElems];
+    const Where at(a.BH);
+    if (at.bh >= a.BH) return;
+    const int lane = threadIdx.x % MTS_WAVE, wave = threadIdx.x / MTS_WAVE, half = lane / 32;
+    const int S = a.S, q0 = (CAUSAL ? a.blocks - 1 - at.order : at.order) * kOwn, first = q0 + 32 * wave, row = first + lane % 32;
+    const int64_t from = min(row, S - 1);
+    const ET *k = a.k.row0(at.bh, a.heads), *v = a.v.row0(at.bh, a.heads);
+    frag q[4], g[4];
+    own_frags<ET>(a.q.row0(at.bh, a.heads) + from * a.q.s, q);
+    own_frags<ET>(a.dO.row0(at.bh, a.heads) + from * a.dO.s, g);
+    float delta = 0.f;
+    {
+        frag o[4];
+        own_frags<ET>(a.o.row0(at.bh, a.heads) + from * a.o.s, o);
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) delta += (float)o[ks][j] * (float)g[ks][j];
+        delta += __shfl_xor(delta, 32, MTS_WAVE);
+        if (half == 0 && row < S) a.delta[at.bh * S + row] = delta;
+    }
+    const float sc = a.scale * kLog2e, lse = a.lse[at.bh * S + from];
+    f32x16 acc[2] = {};
+    const int end = CAUSAL ? min(S, q0 + kOwn) : S, tiles = (end + kTile - 1) / kTile;
+    TileCopy<ET> kc, vc;
+    kc.fetch(k, a.k.s, 0, S);
+    vc.fetch(v, a.v.s, 0, S);
+    kc.commit(lds[0][0]);
+    vc.commit(lds[0][1]);
+    __syncthreads();
+    for (int t = 0; t < tiles; ++t) {
+        const int kv0 = t * kTile;
+        const ET *kt = lds[t & 1][0], *vt = lds[t & 1][1];
+        if (t + 1 < tiles) {
+            kc.fetch(k, a.k.s, kv0 + kTile, S);
+            vc.fetch(v, a.v.s, kv0 + kTile, S);
+        }
+#pragma unroll
+        for (int m = 0; m < 2; ++m) {
+            const int kvm = kv0 + 32 * m;
+            if (CAUSAL && kvm > first + 31) continue;
+            f32x16 s = {}, d = {};
+#pragma unroll
+            for (int ks = 0; ks < 4; ++ks) {
+                s = Mma<ET>::mul(row_frag(kt, 32 * m, ks), q[ks], s);
+                d = Mma<ET>::mul(row_frag(vt, 32 * m, ks), g[ks], d);
+            }
+#pragma unroll
+            for (int i = 0; i < 16; ++i) s[i] = __builtin_amdgcn_exp2f(fmaf(s[i], sc, -lse));
+            if (kvm + 32 > S || (CAUSAL && kvm + 31 > first)) {
+                const int last = CAUSAL ? min(row, S - 1) : S - 1;
+#pragma unroll
+                for (int i = 0; i < 16; ++i)
+                    if (kvm + 8 * (i / 4) + 4 * half + i % 4 > last) s[i] = 0.f;
+            }
+#pragma unroll
+            for (int i = 0; i < 16; ++i) s[i] *= d[i] - delta;
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const frag ds = narrowed<ET>(s, u);
+#pragma unroll
+                for (int dt = 0; dt < 2; ++dt) acc[dt] = Mma<ET>::mul(column_frag(kt, 32 * m + 16 * u, 32 * dt), ds, acc[dt]);
+            }
+        }
+        if (t + 1 < tiles) {
+            kc.commit(lds[(t + 1) & 1][0]);
+            vc.commit(lds[(t + 1) & 1][1]);
+        }
+        __syncthreads();
+    }
+    if (row < S) store_row(a.dq.row0(at.bh, a.heads) + row * a.dq.s, acc, a.scale);
+}
+
+// dK and dV of 128 keys.
+template <typename ET, bool CAUSAL>
+__global__ __launch_bounds__(kThreads, 2) void attention_dkdv_kernel(AttnArgs<ET> a) {
+    typedef typename Mma<ET>::frag frag;
+    __shared__ __align__(16) ET lds[2][2][kTileElems];
+    __shared__ __align__(16) float stats[2][2][kTile];
+    const Where at(a.BH);
+    if (at.bh >= a.BH) return;
+    const int lane = threadIdx.x % MTS_WAVE, wave = threadIdx.x / MTS_WAVE, half = lane / 32;
+    const int S = a.S, first = at.order * kOwn + 32 * wave, row = first + lane % 32;
+    const int64_t from = min(row, S - 1);
+    const ET *q = a.q.row0(at.bh, a.heads), *g = a.dO.row0(at.bh, a.heads);
+    const float *lse = a.lse + at.bh * S, *delta = a.delta + at.bh * S;
+    frag k[4], v[4];
+    own_frags<ET>(a.k.row0(at.bh, a.heads) + from * a.k.s, k);
+    own_frags<ET>(a.v.row0(at.bh, a.heads) + from * a.v.s, v);
+    const float sc = a.scale * kLog2e;
+    f32x16 dk[2] = {}, dv[2] = {};
+    const int t0 = CAUSAL ? at.order * kOwn / kTile : 0, tiles = (S + kTile - 1) / kTile;
+    TileCopy<ET> qc, gc;
+    float stat = 0.f;
+    auto fetch = [&](int t) {
+        qc.fetch(q, a.q.s, t * kTile, S);
+        gc.fetch(g, a.dO.s, t * kTile, S);
+        if (threadIdx.x < 2 * kTile) {   // queries behind the end: the exponential of -inf
+            const int r = t * kTile + threadIdx.x % kTile;
+            stat = threadIdx.x < kTile ? (r < S ? lse[r] : INFINITY) : (r < S ? delta[r] : 0.f);
+        }
+    };
+    auto commit = [&](int buf) {
+        qc.commit(lds[buf][0]);
+        gc.commit(lds[buf][1]);
+        if (threadIdx.x < 2 * kTile) stats[buf][threadIdx.x / kTile][threadIdx.x % kTile] = stat;
+    };
+    fetch(t0);
+    commit(t0 & 1);
+    __syncthreads();
+    for (int t = t0; t < tiles; ++t) {
+        const ET *qt = lds[t & 1][0], *gt = lds[t & 1][1];
+        if (t + 1 < tiles) fetch(t + 1);
+#pragma unroll
+        for (int m = 0; m < 2; ++m) {
+            const int qm = t * kTile + 32 * m;
+            if (CAUSAL && qm + 31 < first) continue;
+            f32x16 s = {}, d = {};
+#pragma unroll
+            for (int ks = 0; ks < 4; ++ks) {
+                s = Mma<ET>::mul(row_frag(qt, 32 * m, ks), k[ks], s);
+                d = Mma<ET>::mul(row_frag(gt, 32 * m, ks), v[ks], d);
+            }
+            const float *l = stats[t & 1][0] + 32 * m + 4 * half, *dl = stats[t & 1][1] + 32 * m + 4 * half;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const f32x4 l4 = *reinterpret_cast<const f32x4*>(l + 8 * j);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) s[4 * j + r] = __builtin_amdgcn_exp2f(fmaf(s[4 * j + r], sc, -l4[r]));
+            }
+            if (CAUSAL && qm < first + 31) {
+#pragma unroll
+                for (int i = 0; i < 16; ++i)
+                    if (qm + 8 * (i / 4) + 4 * half + i % 4 < row) s[i] = 0.f;
+            }
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const frag p = narrowed<ET>(s, u);
+#pragma unroll
+                for (int dt = 0; dt < 2; ++dt) dv[dt] = Mma<ET>::mul(column_frag(gt, 32 * m + 16 * u, 32 * dt), p, dv[dt]);
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const f32x4 d4 = *reinterpret_cast<const f32x4*>(dl + 8 * j);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) s[4 * j + r] *= d[4 * j + r] - d4[r];
+            }
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const frag ds = narrowed<ET>(s, u);
+#pragma unroll
+                for (int dt = 0; dt < 2; ++dt) dk[dt] = Mma<ET>::mul(column_frag(qt, 32 * m + 16 * u, 32 * dt), ds, dk[dt]);
+            }
+        }
+        if (t + 1 < tiles) commit((t + 1) & 1);
+        __syncthreads();
+    }
+    if (row >= S) return;
+    store_row(a.dk.row0(at.bh, a.heads) + row * a.dk.s, dk, a.scale);
+    store_row(a.dv.row0(at.bh, a.heads) + row * a.dv.s, dv, 1.f);
+}
+
+template <typename T>
+Heads<T> heads_of(const MtsHeads& t) {
+    return {(T*)t.data, t.batch_stride, t.head_stride, t.row_stride};
+}
+
+bool heads_ok(const MtsHeads& t) {
+    return t.data && mts_aligned16(t.data) && t.batch_stride % 8 == 0 && t.head_stride % 8 == 0 && t.row_stride % 8 == 0;
+}
+
+int attention_shape(const MtsHeads* const* tensors, int count, int64_t B, int heads, int64_t S, int act_dtype) {
+    for (int i = 0; i < count; ++i) {
+        if (!tensors[i] || !tensors[i]->data) return MTS_ERR_NULL;
+        if (!heads_ok(*tensors[i])) return MTS_ERR_ALIGN;
+    }
+    if (act_dtype != MTS_BF16 && act_dtype != MTS_F16) return MTS_ERR_DTYPE;
+    if (!mts_attention_supported(B, heads, S, kHead)) return MTS_ERR_SHAPE;
+    return MTS_OK;
+}
+
+template <typename ET>
+AttnArgs<ET> attention_args(const MtsHeads* q, const MtsHeads* k, const MtsHeads* v, int64_t B, int heads, int64_t S) {
+    AttnArgs<ET> a = {};
+    a.q = heads_of<const ET>(*q), a.k = heads_of<const ET>(*k), a.v = heads_of<const ET>(*v);
+    a.BH = B * heads, a.heads = heads, a.S = (int)S, a.blocks = (int)((S + kOwn - 1) / kOwn);
+    a.scale = 0.125f;   // 1 / sqrt(64)
+    return a;
+}
+
+template <typename ET>
+dim3 attention_grid(const AttnArgs<ET>& a) { return dim3((unsigned)((a.BH + 7) / 8 * 8 * a.blocks)); }
+
+template <typename ET>
+int attention_fwd(const MtsHeads* q, const MtsHeads* k, const MtsHeads* v, int64_t B, int heads, int64_t S, int causal, const MtsHeads* out, float* lse,
+                  hipStream_t st) {
+    AttnArgs<ET> a = attention_args<ET>(q, k, v, B, heads, S);
+    a.out = heads_of<ET>(*out), a.lse = lse;
+    if (causal) attention_fwd_kernel<ET, true><<<attention_grid(a), kThreads, 0, st>>>(a);
+    else attention_fwd_kernel<ET, false><<<attention_grid(a), kThreads, 0, st>>>(a);
+    MTS_CHECK_LAUNCH();
+    return MTS_OK;
+}
+
+template <typename ET>
+int attention_bwd(const MtsHeads* q, const MtsHeads* k, const MtsHeads* v, const MtsHeads* out, const MtsHeads* d_out, const float* lse, int64_t B,
+                  int heads, int64_t S, int causal, const MtsHeads* dq, const MtsHeads* dk, const MtsHeads* dv, float* delta, hipStream_t st) {
+    AttnArgs<ET> a = attention_args<ET>(q, k, v, B, heads, S);
+    a.o = heads_of<const ET>(*out), a.dO = heads_of<const ET>(*d_out);
+    a.dq = heads_of<ET>(*dq), a.dk = heads_of<ET>(*dk), a.dv = heads_of<ET>(*dv);
+    a.lse = const_cast<float*>(lse), a.delta = delta;
+    if (causal) attention_dq_kernel<ET, true><<<attention_grid(a), kThreads, 0, st>>>(a);
+    else attention_dq_kernel<ET, false><<<attention_grid(a), kThreads, 0, st>>>(a);
+    MTS_CHECK_LAUNCH();
+    if (causal) attention_dkdv_kernel<ET, true><<<attention_grid(a), kThreads, 0, st>>>(a);
+    else attention_dkdv_kernel<ET, false><<<attention_grid(a), kThreads, 0, st>>>(a);
+    MTS_CHECK_LAUNCH();
+    return MTS_OK;
+}
+
+}  // namespace
+
+extern "C" int mts_attention_supported(int64_t B, int heads, int64_t S, int head_dim) {
+    if (B <= 0 || heads <= 0 || S <= 0 || head_dim != kHead || S > (1 << 24) || B >= (1LL << 31)) return 0;
+    return (B * heads + 7) / 8 * 8 * ((S + kOwn - 1) / kOwn) * kThreads < (1LL << 32);
+}
+
+extern "C" int mts_attention_fwd(const MtsHeads* q, const MtsHeads* k, const MtsHeads* v, int64_t B, int heads, int64_t S, int causal, int act_dtype,
+                                 const MtsHeads* out, float* lse, void* stream) {
+    const MtsHeads* all[] = {q, k, v, out};
+    if (!lse) return MTS_ERR_NULL;
+    if (int e = attention_shape(all, 4, B, heads, S, act_dtype)) return e;
+    if (act_dtype == MTS_BF16) return attention_fwd<bf16_t>(q, k, v, B, heads, S, causal, out, lse, (hipStream_t)stream);
+    return attention_fwd<mts_f16_t>(q, k, v, B, heads, S, causal, out, lse, (hipStream_t)stream);
+}
+
+extern "C" int mts_attention_bwd(const MtsHeads* q, const MtsHeads* k, const MtsHeads* v, const MtsHeads* out, const MtsHeads* d_out, const float* lse,
+                                 int64_t B, int heads, int64_t S, int causal, int act_dtype, const MtsHeads* dq, const MtsHeads* dk, const MtsHeads* dv,
+                                 float* delta, void* stream) {
+    const MtsHeads* all[] = {q, k, v, out, d_out, dq, dk, dv};
+    if (!lse || !delta) return MTS_ERR_NULL;
+    if (int e = attention_shape(all, 8, B, heads, S, act_dtype)) return e;
+    if (act_dtype == MTS_BF16) return attention_bwd<bf16_t>(q, k, v, out, d_out, lse, B, heads, S, causal, dq, dk, dv, delta, (hipStream_t)stream);
+    return attention_bwd<mts_f16_t>(q, k, v, out, d_out, lse, B, heads, S, causal, dq, dk, dv, delta, (hipStream_t)stream);
+}

@@ -67,6 +67,11 @@ class HipOpsBackend(DenseTorchOps):
             return None
         return dense.qkv_rope(qkv, cos, sin, heads)
 
+    def attention(self, q, k, v, *, is_causal, dropout_p):
+        if not dropout_p and dense.is_attention_supported(q, k, v):
+            return dense.attention(q, k, v, is_causal)
+        return super().attention(q, k, v, is_causal=is_causal, dropout_p=dropout_p)
+
     def cross_entropy(self, logits, targets):
         if dense.is_cross_entropy_supported(logits, targets):
             return dense.cross_entropy(logits, targets)

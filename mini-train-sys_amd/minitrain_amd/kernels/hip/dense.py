@@ -1,4 +1,4 @@
-"""The decoder's operators around its matrix products: RMSNorm, rotary encoding and cross-entropy.
+"""The decoder's operators around its matrix products: RMSNorm, rotary encoding, attention and cross-entropy.
 
 Each stands in for a chain of stock elementwise and reduction kernels
 (minitrain/kernels/torch_ops.py of the reference) that reads and writes the activations several
@@ -47,6 +47,15 @@ def is_qkv_rope_supported(qkv, cos, sin, heads: int) -> bool:
 def qkv_rope(qkv, cos, sin, heads: int):
     """Rotated queries, rotated keys and values ``[B, heads, S, D]`` of the packed projection ``[B, S, 3 * heads * D]``"""
     return _lib.host().qkv_rope(qkv, cos, sin, heads)
+
+
+def is_attention_supported(q, k, v) -> bool:
+    return _may_replace(q, k, v) and _lib.host().attention_supported(q, k, v)
+
+
+def attention(q, k, v, is_causal: bool):
+    """``F.scaled_dot_product_attention(q, k, v, is_causal=is_causal)``"""
+    return _lib.host().attention(q, k, v, is_causal)
 
 
 def is_cross_entropy_supported(logits, targets) -> bool:
