@@ -299,6 +299,19 @@ int mts_moe_fwd_gateup_down(const void* x, const void* w1, const void* w2, const
                             int act_dtype, void* pre_act, void* post_act, void* y,
                             int32_t* workspace, int64_t workspace_bytes, void* stream);
 
+/* Both forward GEMMs for few rows per expert, bound by reading the weights: w1 and w2 of
+ * act_dtype or MTS_F32 (rounded to act_dtype as they are read).  Results as those of
+ * mts_moe_fwd_gateup_swiglu and mts_moe_fwd_down; any number of rows is correct.           */
+int mts_moe_fwd_few_rows_supported(int act_dtype, int weight_dtype, int64_t T, int64_t TK, int E,
+                                   int H, int I);
+int mts_moe_fwd_few_rows_preferred(int act_dtype, int weight_dtype, int64_t T, int64_t TK, int E,
+                                   int H, int I);
+int mts_moe_fwd_few_rows(const void* x, const void* w1, const void* w2, int weight_dtype,
+                         const int32_t* x_gather, const int32_t* expert_start,
+                         const void* weights, const int32_t* s_scatter, int64_t T, int K, int E,
+                         int H, int I, int act_dtype, void* pre_act, void* post_act, void* y,
+                         void* stream);
+
 /* Replaces _token_gather_weighted_sum_kernel (fused_moe_kernels.py:451-498):
  * out[t] = addend[t] + sum_k w[t,k] * y[s_reverse[t*K+k]]  (fp32 sum, one rounding);
  * weights == NULL gives the unweighted sum used for dx; addend [T,H] (act_dtype) may be NULL

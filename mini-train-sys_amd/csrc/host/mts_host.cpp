@@ -161,13 +161,18 @@ const char* layer_violation(const Tensor& x, const Tensor& w_r, const Tensor& w1
 // ---- options -----------------------------------------------------------------------------------------------------------------
 
 // Comparison switches of the Python side (kernels/hip/switches.py), as they stand when an operator is called.
-enum Switch : int64_t { OVERLAP = 1, JOINT_BWD = 2, JOINT_FWD = 4, TAIL_IN_JOINT = 8, COMBINE_IN_TAIL = 16, JOINT_SCHEDULE = 32, WEIGHTED_POST = 64 };
+enum Switch : int64_t { OVERLAP = 1, JOINT_BWD = 2, JOINT_FWD = 4, TAIL_IN_JOINT = 8, COMBINE_IN_TAIL = 16, JOINT_SCHEDULE = 32, WEIGHTED_POST = 64, NO_BACKWARD = 1 << 20 };
 
 struct Options {
     int64_t switches;
     int64_t dw_workspace_limit;   // row-chunk workspaces of the weight-gradient GEMMs beyond this size are done without
     bool on(Switch s) const { return (switches & s) != 0; }
 };
+
+template <typename... Ts>
+int64_t no_backward(const Ts&... t) {
+    return at::GradMode::is_enabled() && (t.requires_grad() || ...) ? 0 : NO_BACKWARD;
+}
 
 // Counters of the joint gate/up + down launch, owned by the Python side (one per device and stream): an object with
 // before_launch(), get(bytes) and after_launch().  Forward passes run under the interpreter lock.
@@ -249,8 +254,16 @@ Tensor experts_forward(const Tensor& x, const Tensor& w1_in, const Tensor& w2_in
     const auto dtype = x.scalar_type();
     const int act = dtype_code(dtype);
     void* stream = stream_of(x);
+    const bool weighted = opt.on(WEIGHTED_POST);
     Tensor w1, w2;
-    if (w1_in.scalar_type() == at::kFloat && w2_in.scalar_type() == at::kFloat && dtype != at::kFloat && w1_in.numel() % 8 == 0 && w2_in.numel() % 8 == 0) {
+    // with few rows the kernels read the weights once and round fp32 ones themselves; a backward pass wants the rounded copies
+    const bool masters = w1_in.scalar_type() == at::kFloat && w2_in.scalar_type() == at::kFloat && dtype != at::kFloat;
+    const bool few_masters = masters && opt.on(NO_BACKWARD) && mts_moe_fwd_few_rows_preferred(act, MTS_F32, T, TK, E, H, I);
+    const bool few = few_masters || mts_moe_fwd_few_rows_preferred(act, act, T, TK, E, H, I);
+    if (few_masters) {
+        w1 = w1_in;
+        w2 = w2_in;
+    } else if (masters && w1_in.numel() % 8 == 0 && w2_in.numel() % 8 == 0) {
         // fp32 master weights: both casts in one launch (the backward pass reuses the copies)
         w1 = at::empty(w1_in.sizes(), x.options());
         w2 = at::empty(w2_in.sizes(), x.options());
@@ -263,11 +276,14 @@ Tensor experts_forward(const Tensor& x, const Tensor& w1_in, const Tensor& w2_in
     // The routing weight is applied where the activation is formed: post_act = s * silu(g) * u.  The down projection then
     // yields s * y, the combine is a plain sum, and post_act is at the same time the operand of the dW2 GEMM, so it is kept
     // for the backward pass instead of being written again there.
-    const bool weighted = opt.on(WEIGHTED_POST);
     Tensor pre_act = at::empty({TK, 2 * I}, x.options()), post_act = at::empty({TK, I}, x.options()), y = at::empty({TK, H}, x.options());
     void* route_w = weighted ? ptr(weights) : nullptr;
     int32_t* route_entry = weighted ? ptr_as<int32_t>(r.s_scatter) : nullptr;
-    if (opt.on(JOINT_FWD) && mts_moe_fwd_joint_preferred(act, TK, E, H, I)) {
+    if (few) {
+        check(mts_moe_fwd_few_rows(ptr(x), ptr(w1), ptr(w2), dtype_code(w1), ptr_as<int32_t>(r.x_gather), ptr_as<int32_t>(r.expert_start), route_w, route_entry,
+                                   T, K, E, H, I, act, ptr(pre_act), ptr(post_act), ptr(y), stream),
+              "mts_moe_fwd_few_rows");
+    } else if (opt.on(JOINT_FWD) && mts_moe_fwd_joint_preferred(act, TK, E, H, I)) {
         // one launch: the down tiles take the CUs as the gate/up tiles leave them
         const int64_t need = mts_moe_fwd_joint_workspace_bytes(TK, E);
         pybind11::object ws = (*joint_workspace_of)((int)x.device().index());
@@ -929,12 +945,12 @@ PYBIND11_MODULE(_host, m) {
     });
     m.def("fused_moe", [](const Tensor& x, const Tensor& w1, const Tensor& w2, const Tensor& index, const Tensor& weights, int64_t switches, int64_t limit) {
         c10::OptionalDeviceGuard guard(x.device());
-        return FusedMoE::apply(x, w1, w2, index, weights, switches, limit);
+        return FusedMoE::apply(x, w1, w2, index, weights, switches | no_backward(x, w1, w2, weights), limit);
     });
     m.def("moe_layer", [](const Tensor& x, const Tensor& w_r, const Tensor& w1, const Tensor& w2, int64_t top_k, bool normalize, int64_t capacity, int64_t switches,
                           int64_t limit) {
         c10::OptionalDeviceGuard guard(x.device());
-        const variable_list v = MoELayer::apply(x, w_r, w1, w2, top_k, normalize, capacity, switches, limit);
+        const variable_list v = MoELayer::apply(x, w_r, w1, w2, top_k, normalize, capacity, switches | no_backward(x, w_r, w1, w2), limit);
         return std::make_tuple(v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], v[8]);
     });
     m.def("router_postprocess", [](const Tensor& logits, int64_t top_k, bool normalize, int64_t act_dtype) {
