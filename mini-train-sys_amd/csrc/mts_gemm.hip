@@ -2029,6 +2029,7 @@ typedef WsTile<256, 256, 2, 4, 64, 3, 4, 3> WsDeep;        // three activation b
 typedef WsTile<128, 256, 2, 4, 64, 3, 4, 3> WsDeepHalf;    // activation rows the launch before it has written (-4 %; nothing for gate/up and dX)
 typedef WsTile<128, 256, 2, 4, 64, 2, 4, 3> WsWideHalf;    // half-height tiles of the last round: the same waves take 64x64 each,
 typedef WsTile<128, 256, 4, 2, 64, 2, 4, 3> WsWideGuHalf;  // and for gate/up 32x128 each       // the same waves on two buffers of 64-wide k-tiles (whole cache lines per row)
+typedef WsTile<128, 128, 4, 2, 64, 4, 4, 3> WsSmall;      // a quarter of the tile and twice the k-tiles in flight: where the large ones are too few
 typedef DwWsTile<256, 256, 2, 4, 32, 4, 4> DwWsLarge;     // same shape for the weight-gradient GEMMs
 typedef DwWsTile<256, 256, 2, 4, 64, 2, 4> DwWsWide;      // two buffers of 64 rows: half the barriers per row
 typedef DwWsWide JointDwTile;                             // the weight-gradient tile of the joint backward launch
@@ -2072,10 +2073,10 @@ struct BwdJointParams {
 
 static_assert(WsWide::BM == kSchedDxRows, "the schedule counts dX tiles of this height");
 typedef WsWide JointDxTile;   // dX reads d_pre_act row-major: whole lines per row with 64-wide k-tiles (a third buffer gains nothing here)
-template <typename OutT>
+template <typename OutT, class DxTile>
 __global__ __launch_bounds__(WsLarge::NT, WsLarge::WAVES_PER_EU) void bwd_joint_kernel(BwdJointParams q) {
-    static_assert(WsLarge::NT == JointDwTile::NT && JointDxTile::NT == WsLarge::NT, "one block shape");
-    constexpr int ROWS_LDS = ws_lds_elems<JointDxTile, EPI_PLAIN>();
+    static_assert(WsLarge::NT == JointDwTile::NT && DxTile::NT == WsLarge::NT, "one block shape");
+    constexpr int ROWS_LDS = ws_lds_elems<DxTile, EPI_PLAIN>();
     constexpr int LDS_ELEMS = ROWS_LDS > JointDwTile::LDS_ELEMS ? ROWS_LDS : JointDwTile::LDS_ELEMS;
     static_assert(LDS_ELEMS * 2 <= 160 * 1024, "LDS capacity");
     __shared__ __attribute__((aligned(1024))) bf16_t smem[LDS_ELEMS];
@@ -2091,7 +2092,7 @@ __global__ __launch_bounds__(WsLarge::NT, WsLarge::WAVES_PER_EU) void bwd_joint_
     }
     b -= q.n_dw2;
     if (b < q.n_dx) {
-        rows_gemm_ws_block<JointDxTile, EPI_PLAIN, true>(q.dx, smem, b);   // W1 as stored: [E][2I][H]
+        rows_gemm_ws_block<DxTile, EPI_PLAIN, true>(q.dx, smem, b);   // W1 as stored: [E][2I][H]
         return;
     }
     b -= q.n_dx;
@@ -2244,7 +2245,7 @@ typedef MtsGemmKind Kind;
 constexpr Kind K_GATEUP = MTS_K_GATEUP, K_DOWN = MTS_K_DOWN, K_DY1 = MTS_K_DY1, K_DX = MTS_K_DX, K_DW2 = MTS_K_DW2, K_DW1 = MTS_K_DW1;
 constexpr int K_COUNT = MTS_K_COUNT;
 // rows_gemm: 0 StagedSmall, 1 RingTwoPerCu, 2 WsLarge, 3 RingThreePerCu (dY1 without the weighted_act output
-// only), 4 WsWide (no SwiGLU backward: gate/up, down and dX; dY1 falls back to 2);
+// only), 4 WsWide (no SwiGLU backward: gate/up, down and dX; dY1 falls back to 2), 5 WsSmall (few rows: small_tiles_pay);
 // dw_gemm: 0 StagedSmall, 2 DwWsLarge, 4 DwWsWide (the same output tiles, so one workspace layout).
 // Defaults are the choices with the shortest LAYER STEP measured on the 24576-token, 768/1024, 8-expert layer.
 // The chip runs this step against its power limit, so a kernel's own duration is not the whole story: what
@@ -2321,6 +2322,21 @@ dim3 rows_grid(RowsParams& p, int64_t TK) {
 // projection 70 -> 44 us, dX and the weight gradients together 330 -> 210 us, no transposed copies of the weights).
 bool rows_pipelined(int Kdim) { return Kdim % 64 == 0 || Kdim >= 256; }
 
+// Tiles of 128 x 128 where one for every CU is enough.  A 256 x 256 tile waits a microsecond for every k-tile, and with few
+// rows the chip has a fraction of its CUs in such tiles (512 tokens, 768/1024, 8 experts: 64 blocks of gate/up, 24 of down and
+// dX).  The kernels at that width, 256 x 256 against 128 x 128 (in brackets: how many of the latter), us:
+//   gate/up  512 tokens 19.4 / 14.8 (192), 1024 tokens 21.9 / 23.5 (320);   down  2048 tokens 17.6 / 13.2 (216), 4096 tokens 20.5 / 23.1 (408);
+//   dO*W2 (192 x 128 ring blocks there)  1024 tokens 25.6 / 16.0 (160), 2048 tokens 27.2 / 28.1 (288);
+//   joint backward launch  192 tokens 49 / 27, 512 tokens 58 / 37, 1024 tokens 65 / 52 (120), 2048 tokens 62 / 68 (216): dX shares the CUs
+//   with the weight gradients (in front of them instead of behind: 512 tokens 44).
+// The count is that of routes spread evenly: half a tile more per expert than whole ones.
+bool small_tiles_pay(int kind, int64_t TK, int E, int N) {
+    const int per_block = kind == K_GATEUP ? WsSmall::BN / 2 : WsSmall::BN;
+    const int64_t present = TK < E ? TK : E, spread = TK / WsSmall::BM + E / 2;
+    const int64_t tiles = (spread > present ? spread : present) * ((N + per_block - 1) / per_block);
+    return tiles <= (kind == K_DX ? 160 : 256);
+}
+
 // does launch_rows_any take B in the weights' stored layout for this kind and reduction length?
 bool rows_kmajor_ok(int kind, int Kdim) { return tile_choice(kind) >= 1 && rows_pipelined(Kdim); }
 
@@ -2331,6 +2347,7 @@ int launch_rows_any(int kind, RowsParams p, int64_t TK, hipStream_t s, bool b_km
     p.reverse = ((kind == K_DOWN && (tile_order_mask() & ORDER_DOWN)) || (kind == K_DY1 && (tile_order_mask() & ORDER_DY1)) ||
                  (kind == K_DX && (tile_order_mask() & ORDER_DX))) ? 1 : 0;
     int choice = tile_choice(kind);
+    if (!tile_forced(kind) && small_tiles_pay(kind, TK, p.E, p.N)) choice = 5;
     // three blocks per CU hold two stages each: for short reductions, and for the epilogue that fits beside them
     if (choice == 3 && (EPI != EPI_DY1N || !b_kmajor || (!tile_forced(kind) && p.Kdim > 1024))) choice = 1;
     // the 64-wide variant exists for the GEMMs with a plain or SwiGLU epilogue
@@ -2341,6 +2358,14 @@ int launch_rows_any(int kind, RowsParams p, int64_t TK, hipStream_t s, bool b_km
         if constexpr (EPI == EPI_DY1N) {
             const dim3 grid = rows_grid<RingThreePerCu, EPI>(p, TK);
             rows_gemm_ring_kernel<RingThreePerCu, EPI, true><<<grid, RingThreePerCu::NT, 0, s>>>(p);
+        }
+    } else if (choice == 5) {
+        const dim3 grid = rows_grid<WsSmall, EPI>(p, TK);
+        if constexpr (EPI != EPI_SWIGLU) {
+            if (b_kmajor) rows_gemm_ws_kernel<WsSmall, EPI, true><<<grid, WsSmall::NT, 0, s>>>(p);
+            else rows_gemm_ws_kernel<WsSmall, EPI><<<grid, WsSmall::NT, 0, s>>>(p);
+        } else {
+            rows_gemm_ws_kernel<WsSmall, EPI><<<grid, WsSmall::NT, 0, s>>>(p);
         }
     } else if (choice == 1) {
         const dim3 grid = rows_grid<RingTwoPerCu, EPI>(p, TK);
@@ -2535,7 +2560,8 @@ int launch_bwd_joint(BwdJointParams q, int E, int grad_dtype, void* ws1, int64_t
         q.dw2.part = nullptr;
     }
     q.dx.reverse = (tile_order_mask() & ORDER_DX) ? 1 : 0;
-    q.n_dx = (int)rows_grid<JointDxTile, EPI_PLAIN>(q.dx, q.dx.TK).x;
+    const bool small_dx = tile_forced(K_DX) ? tile_choice(K_DX) == 5 : small_tiles_pay(K_DX, q.dx.TK, E, q.dx.N);
+    q.n_dx = (int)(small_dx ? rows_grid<WsSmall, EPI_PLAIN>(q.dx, q.dx.TK) : rows_grid<JointDxTile, EPI_PLAIN>(q.dx, q.dx.TK)).x;
     // With both workspaces (row chunks on) and a schedule from the caller (written by the dO*W2 launch), units and dX
     // tiles go to the XCDs as the table says.
     if (schedule && own_dw2 && q.dw1.part && q.dw2.part && E <= kSchedMaxExperts && mts_tuning().joint_schedule) {
@@ -2544,7 +2570,7 @@ int launch_bwd_joint(BwdJointParams q, int E, int grad_dtype, void* ws1, int64_t
         schedule_shape(q.dx.TK, E, slots, cap);
         q.dw1.sched = q.dw2.sched = schedule;
         q.dw1.sched_slots = q.dw2.sched_slots = slots;
-        if (q.dx.xcd_ranges) {
+        if (q.dx.xcd_ranges && !small_dx) {
             q.dx.sched = schedule;
             q.dx.n_groups = 1;
             q.n_dx = cap * q.dx.n_tiles * kXcds;
@@ -2553,8 +2579,13 @@ int launch_bwd_joint(BwdJointParams q, int E, int grad_dtype, void* ws1, int64_t
     const int64_t want = (q.entries + WsLarge::NT * 4 - 1) / (WsLarge::NT * 4);
     q.n_ds = (int)(want < 64 ? want : 64);
     const dim3 grid((unsigned)(q.n_dw1 + q.n_dw2 + q.n_dx + q.n_ds + q.n_router));
-    if (grad_dtype == MTS_GEMM_DTYPE) bwd_joint_kernel<bf16_t><<<grid, WsLarge::NT, 0, s>>>(q);
-    else bwd_joint_kernel<float><<<grid, WsLarge::NT, 0, s>>>(q);
+    if (small_dx) {
+        if (grad_dtype == MTS_GEMM_DTYPE) bwd_joint_kernel<bf16_t, WsSmall><<<grid, WsLarge::NT, 0, s>>>(q);
+        else bwd_joint_kernel<float, WsSmall><<<grid, WsLarge::NT, 0, s>>>(q);
+    } else {
+        if (grad_dtype == MTS_GEMM_DTYPE) bwd_joint_kernel<bf16_t, JointDxTile><<<grid, WsLarge::NT, 0, s>>>(q);
+        else bwd_joint_kernel<float, JointDxTile><<<grid, WsLarge::NT, 0, s>>>(q);
+    }
     MTS_CHECK_LAUNCH();
     if (q.dw1.part && (q.dw2.part || !own_dw2) && 2 * E <= 65535) {
         const int t = q.dw1.tiles_per_expert > q.dw2.tiles_per_expert ? q.dw1.tiles_per_expert : q.dw2.tiles_per_expert;

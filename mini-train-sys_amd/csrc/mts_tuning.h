@@ -3,7 +3,7 @@
 // every launcher reads: no launcher looks at the environment, and nothing is written after load, so calls from
 // several host threads see the same values without synchronisation.
 //
-//   MTS_TILE_GATEUP / _DOWN / _DY1 / _DX / _DW1 / _DW2 = 0..4   tile family of that GEMM instead of the default
+//   MTS_TILE_GATEUP / _DOWN / _DY1 / _DX / _DW1 / _DW2 = 0..5   tile family of that GEMM instead of the default
 //   MTS_XCD_RANGES = 0 | 1        round-robin deal of the m-tiles | contiguous ranges per XCD, whatever the weights' size
 //   MTS_NO_TILE_ORDER = 1         no n-tile groups, no reversed walks of an XCD's range
 //   MTS_TILE_ORDER = mask         those one by one (bit 0 groups, 1 down reversed, 2 dY1 reversed, 3 dX reversed)

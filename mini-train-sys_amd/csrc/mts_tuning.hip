@@ -17,7 +17,7 @@ MtsTuning read_environment() {
     for (int k = 0; k < MTS_K_COUNT; ++k) {
         const char* s = getenv(kTileEnv[k]);
         const int c = s && *s ? atoi(s) : -1;
-        t.tile[k] = (c >= 0 && c <= 4) ? c : -1;
+        t.tile[k] = (c >= 0 && c <= 5) ? c : -1;
     }
     const char* ranges = getenv("MTS_XCD_RANGES");
     t.xcd_ranges = ranges && *ranges ? (atoi(ranges) != 0) : -1;

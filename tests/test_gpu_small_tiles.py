@@ -1,0 +1,45 @@
+"""Grouped GEMMs with few rows per expert on 128 x 128 tiles: the operator's results and gradients against fp64 (GPU).
+
+Tolerance, relative to the largest value: 2^-7 (bf16) and 2^-10 (fp16), two half-ulp roundings of the intermediates that enter
+the last product and one of its result."""
+
+import pytest
+import torch
+
+from minitrain_amd.kernels.hip.fused_moe import fused_moe
+
+pytestmark = pytest.mark.gpu
+
+TOL = {torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10}
+
+
+@pytest.mark.parametrize("rows,E,H,I", [
+    ((127, 128, 129), 3, 256, 256), ((256, 0, 1), 3, 128, 192), ((300, 50), 2, 712, 328), ((95, 400, 96, 33, 0, 64), 6, 768, 512), ((1,), 1, 320, 1368)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("params", ["same", "fp32"])
+def test_small_tiles(rows, E, H, I, dtype, params):
+    """One row to three tiles of an expert and one more or less, experts without rows, widths that are not whole tiles."""
+    print(f"small tiles rows={rows} H={H} I={I} {dtype} {params}", flush=True)
+    g = torch.Generator().manual_seed(sum(rows) + H)
+    T = sum(rows)
+    pt = torch.float32 if params == "fp32" else dtype
+    idx = torch.repeat_interleave(torch.arange(E), torch.tensor(rows))[torch.randperm(T, generator=g)].int()[:, None].cuda()
+    x, grad = (torch.randn(T, H, generator=g).to(dtype).cuda() for _ in range(2))
+    w1, w2 = (torch.randn(E, 2 * I, H, generator=g) * H ** -0.5).to(pt).cuda(), (torch.randn(E, H, I, generator=g) * I ** -0.5).to(pt).cuda()
+    s = (0.5 + torch.rand(T, 1, generator=g)).to(dtype).cuda()
+    leaves = [t.requires_grad_(True) for t in (x, w1, w2, s)]
+    out = fused_moe(x, w1, w2, idx, s)
+    out.backward(grad)
+    # the weights enter the products in the activation dtype
+    wide = [x.detach().double(), w1.detach().to(dtype).double(), w2.detach().to(dtype).double(), s.detach().double()]
+    wide = [t.requires_grad_(True) for t in wide]
+    parts = []
+    for e in range(E):
+        at = (idx[:, 0] == e).nonzero()[:, 0]
+        gate, up = (wide[0][at] @ wide[1][e].T).chunk(2, dim=1)
+        parts.append((at, ((torch.nn.functional.silu(gate) * up) @ wide[2][e].T) * wide[3][at]))
+    want = torch.zeros(T, H, dtype=torch.float64, device="cuda").index_copy(0, torch.cat([p[0] for p in parts]), torch.cat([p[1] for p in parts]))
+    want.backward(grad.double())
+    for what, got, ref in [("out", out.detach(), want.detach())] + [(n, a.grad, b.grad) for n, a, b in zip(("dx", "dw1", "dw2", "ds"), leaves, wide)]:
+        err, scale = float((got.double() - ref).abs().max()), float(ref.abs().max())
+        assert err <= TOL[dtype] * scale, (what, err, scale)
