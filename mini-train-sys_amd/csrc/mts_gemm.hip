@@ -2349,7 +2349,11 @@ int launch_rows_any(int kind, RowsParams p, int64_t TK, hipStream_t s, bool b_km
     int choice = tile_choice(kind);
     if (!tile_forced(kind) && small_tiles_pay(kind, TK, p.E, p.N)) choice = 5;
     // three blocks per CU hold two stages each: for short reductions, and for the epilogue that fits beside them
-    if (choice == 3 && (EPI != EPI_DY1N || !b_kmajor || (!tile_forced(kind) && p.Kdim > 1024))) choice = 1;
+    if (choice == 3 && (EPI != EPI_DY1N || !b_kmajor)) choice = 1;
+    // longer ones go to the specialised waves, whose k-loop is the better one and whose epilogue then weighs less (the operator,
+    // forward and backward, on two blocks per CU / on these, us: 4096 tokens 4096/14336 9464 / 9147, 16 384 tokens 2048/2048 2471 / 2437,
+    // 6000 tokens 2048/1024 580 / 567; 1024/2048 668 / 638 to 646 / 652 in turn, 24 576 tokens of 768/1024 855 / 873)
+    if (choice == 3 && !tile_forced(kind) && p.Kdim > 1024) choice = 2;
     // the 64-wide variant exists for the GEMMs with a plain or SwiGLU epilogue
     if (choice == 4 && epi_is_dy1(EPI)) choice = 2;
     if (choice >= 1 && !rows_pipelined(p.Kdim)) choice = 0;
