@@ -10,7 +10,7 @@
 //
 // The vector pipe bounds it: for 32 x 64 scores the forward pass issues 512 cycles of MFMA and about 1000 of exponentials (a
 // quarter of the rate), maxima, sums and conversions.  bf16, causal, 12 heads of 64, 1024 rows, against the stock operator:
-// batch 8: 33 us forward (79) and 127 backward (308); batch 24: 75 us (515 TFLOP/s; 168) and 311 (435 TFLOP/s of the seven
+// batch 8: 31 us forward (79) and 121 backward (308); batch 24: 72 us (534 TFLOP/s; 168) and 304 (445 TFLOP/s of the seven
 // products that two separate kernels form, so that each gradient is summed by one block in a fixed order; 844).
 #include "mts_common.h"
 
@@ -40,6 +40,7 @@ constexpr int kWaves = 4;
 constexpr int kThreads = kWaves * MTS_WAVE;
 constexpr int kOwn = 32 * kWaves;       // rows a block owns, 32 a wave
 constexpr int kTileElems = kTile * kHead;
+constexpr int kCusPerXcd = 32;
 constexpr float kLog2e = 1.4426950408889634f;
 
 // [B, heads, S, 64], dense in the last dimension, strides in elements
@@ -127,12 +128,17 @@ __device__ __forceinline__ void store_row(ET* row, const f32x16 (&acc)[2], float
 }
 
 // Blocks of one head on one XCD (its keys and values, or queries and gradients, are read by all of them); `order` counts the
-// blocks of a head, the same for all heads before the next, so that the longest of a causal pass start first.
+// blocks of a head, the same for all heads before the next, so that the longest of a causal pass start first.  Every other
+// round of an XCD's 32 CUs is dealt backwards, so that a CU that took the longest block of one takes the shortest of the next
+// (batch 8: 33 -> 31 us forward, 127 -> 121 backward; 24: 75 -> 72 and 311 -> 304).
 struct Where {
     int64_t bh;
     int order;
     __device__ __forceinline__ Where(int64_t BH) {
-        const int64_t j = blockIdx.x / 8, per = (BH + 7) / 8;
+        const int64_t per = (BH + 7) / 8, total = gridDim.x / 8;
+        int64_t j = blockIdx.x / 8;
+        const int64_t round = j / kCusPerXcd;
+        if (round % 2 && (round + 1) * kCusPerXcd <= total) j = (2 * round + 1) * kCusPerXcd - 1 - j;
         order = (int)(j / per);
         bh = (j % per) * 8 + blockIdx.x % 8;
     }
