@@ -253,7 +253,8 @@ int mts_moe_cast_weights_pair(const float* w1, void* w1_out, int64_t n1, const f
 /* ---- forward ------------------------------------------------------------
  * Replaces _fused_up_proj_swiglu_kernel (fused_moe_kernels.py:264-367):
  * for every row r (token x_gather[r], expert e): [g;u] = W1[e] x ; a = silu(g)*u.
- * x [T,H], w1 [E,2I,H], pre_act [TK,2I], post_act [TK,I], all of act_dtype
+ * x [T,H], w1 [E,2I,H], pre_act [TK,2I], post_act [TK,I], all of act_dtype; pre_act may be NULL for
+ * the 16-bit types (here and in the entry points below): it is kept for a backward pass only
  * (MTS_BF16, MTS_F16: MFMA kernels, H and I multiples of 8; MTS_F32: plain fp32 kernels).
  * weights (flat [T*K], act_dtype) and s_scatter (row -> entry) are optional as a pair.  With
  * them post_act[r] = s_r * silu(g) * u, s_r = weights[s_scatter[r]] (fp32 product, one

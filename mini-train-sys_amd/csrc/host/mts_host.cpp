@@ -161,7 +161,7 @@ const char* layer_violation(const Tensor& x, const Tensor& w_r, const Tensor& w1
 // ---- options -----------------------------------------------------------------------------------------------------------------
 
 // Comparison switches of the Python side (kernels/hip/switches.py), as they stand when an operator is called.
-enum Switch : int64_t { OVERLAP = 1, JOINT_BWD = 2, JOINT_FWD = 4, TAIL_IN_JOINT = 8, COMBINE_IN_TAIL = 16, JOINT_SCHEDULE = 32, WEIGHTED_POST = 64, NO_BACKWARD = 1 << 20 };
+enum Switch : int64_t { OVERLAP = 1, JOINT_BWD = 2, JOINT_FWD = 4, TAIL_IN_JOINT = 8, COMBINE_IN_TAIL = 16, JOINT_SCHEDULE = 32, WEIGHTED_POST = 64, NO_BACKWARD = 1 << 20 /* set here: nothing that this call computes will be differentiated */ };
 
 struct Options {
     int64_t switches;
@@ -276,7 +276,8 @@ Tensor experts_forward(const Tensor& x, const Tensor& w1_in, const Tensor& w2_in
     // The routing weight is applied where the activation is formed: post_act = s * silu(g) * u.  The down projection then
     // yields s * y, the combine is a plain sum, and post_act is at the same time the operand of the dW2 GEMM, so it is kept
     // for the backward pass instead of being written again there.
-    Tensor pre_act = at::empty({TK, 2 * I}, x.options()), post_act = at::empty({TK, I}, x.options()), y = at::empty({TK, H}, x.options());
+    Tensor pre_act, post_act = at::empty({TK, I}, x.options()), y = at::empty({TK, H}, x.options());
+    if (!opt.on(NO_BACKWARD) || dtype == at::kFloat) pre_act = at::empty({TK, 2 * I}, x.options());
     void* route_w = weighted ? ptr(weights) : nullptr;
     int32_t* route_entry = weighted ? ptr_as<int32_t>(r.s_scatter) : nullptr;
     if (few) {

@@ -189,9 +189,11 @@ __global__ __launch_bounds__(kThreads) void few_rows_kernel(FewRows p) {
                 g[r] = (ET)v[0][r], u[r] = (ET)v[1][r];
                 a[r] = (ET)(v[0][r] * __builtin_amdgcn_rcpf(1.0f + __expf(-v[0][r])) * v[1][r] * s);
             }
-            ET* pre = (ET*)p.C + (int64_t)row * 2 * p.N + n;
-            *reinterpret_cast<quad*>(pre) = g;
-            *reinterpret_cast<quad*>(pre + p.N) = u;
+            if (p.C) {
+                ET* pre = (ET*)p.C + (int64_t)row * 2 * p.N + n;
+                *reinterpret_cast<quad*>(pre) = g;
+                *reinterpret_cast<quad*>(pre + p.N) = u;
+            }
             *reinterpret_cast<quad*>((ET*)p.C2 + (int64_t)row * p.N + n) = a;
         } else {
             quad y;
@@ -253,7 +255,7 @@ extern "C" int mts_moe_fwd_few_rows_preferred(int act_dtype, int weight_dtype, i
 extern "C" int mts_moe_fwd_few_rows(const void* x, const void* w1, const void* w2, int weight_dtype, const int32_t* x_gather, const int32_t* expert_start,
                                     const void* weights, const int32_t* s_scatter, int64_t T, int K, int E, int H, int I, int act_dtype, void* pre_act,
                                     void* post_act, void* y, void* stream) {
-    if (!x || !w1 || !w2 || !x_gather || !expert_start || !pre_act || !post_act || !y) return MTS_ERR_NULL;
+    if (!x || !w1 || !w2 || !x_gather || !expert_start || !post_act || !y) return MTS_ERR_NULL;
     if ((weights != nullptr) != (s_scatter != nullptr)) return MTS_ERR_NULL;
     if (K < 1 || !mts_moe_fwd_few_rows_supported(act_dtype, weight_dtype, T, T * K, E, H, I)) return MTS_ERR_SHAPE;
     if (!mts_aligned16(x) || !mts_aligned16(w1) || !mts_aligned16(w2) || !mts_aligned16(pre_act) || !mts_aligned16(post_act) || !mts_aligned16(y))

@@ -425,7 +425,7 @@ __device__ __forceinline__ void rows_epilogue(const RowsParams& p, f32x16 (&acc)
     const int64_t left = rend - row0;
     const int64_t ldc = EPI == EPI_PLAIN ? N : 2 * N;
     const bool has_c2 = EPI == EPI_SWIGLU || EPI == EPI_DY1;
-    const __amdgpu_buffer_rsrc_t rs_c = make_rsrc(p.C + (int64_t)row0 * ldc, left * ldc * 2);
+    const __amdgpu_buffer_rsrc_t rs_c = make_rsrc(p.C ? p.C + (int64_t)row0 * ldc : nullptr, p.C ? left * ldc * 2 : 0);
     const __amdgpu_buffer_rsrc_t rs_c2 = make_rsrc(has_c2 ? p.C2 + (int64_t)row0 * N : nullptr, has_c2 ? left * (int64_t)N * 2 : 0);
     const __amdgpu_buffer_rsrc_t rs_pre = make_rsrc(DY1 ? p.pre_act + (int64_t)row0 * 2 * N : nullptr, DY1 ? left * (int64_t)N * 4 : 0);
     const int rrel = rend - row0;   // rows of the tile that exist
@@ -484,12 +484,16 @@ __device__ __forceinline__ void rows_epilogue(const RowsParams& p, f32x16 (&acc)
                         a[q] = g[q] * sigmoidf_(g[q]) * u[q] * s;
                     }
                     const int o = ml * LDW + f * 32 + 8 * j + nq;
-                    stage4(buf0 + o, g[0], g[1], g[2], g[3]);
-                    stage4(buf1 + o, u[0], u[1], u[2], u[3]);
+                    if (p.C) {
+                        stage4(buf0 + o, g[0], g[1], g[2], g[3]);
+                        stage4(buf1 + o, u[0], u[1], u[2], u[3]);
+                    }
                     stage4(buf2 + o, a[0], a[1], a[2], a[3]);
                 }
-            flush_tile<COLS>(buf0, rs_c, 2 * N, ncol0, rowg0, rrel, ncol0, p.N);
-            flush_tile<COLS>(buf1, rs_c, 2 * N, N + ncol0, rowg0, rrel, ncol0, p.N);
+            if (p.C) {   // no backward pass wants them: two thirds of what the epilogue stages and writes
+                flush_tile<COLS>(buf0, rs_c, 2 * N, ncol0, rowg0, rrel, ncol0, p.N);
+                flush_tile<COLS>(buf1, rs_c, 2 * N, N + ncol0, rowg0, rrel, ncol0, p.N);
+            }
             flush_tile<COLS>(buf2, rs_c2, N, ncol0, rowg0, rrel, ncol0, p.N);
         } else {  // dY1
             const int row = row0 + rowg0 + ml;
@@ -2643,7 +2647,7 @@ extern "C" int MTS_GEMM_ENTRY(mts_moe_fwd_gateup_swiglu)(const void* x, const vo
 #ifndef MTS_GEMM_F16
     if (act_dtype == MTS_F16) return mts_moe_fwd_gateup_swiglu_f16(x, w1, x_gather, expert_start, weights, s_scatter, T, K, E, H, I, act_dtype, pre_act, post_act, stream);
 #endif
-    if (!x || !w1 || !x_gather || !expert_start || !pre_act || !post_act) return MTS_ERR_NULL;
+    if (!x || !w1 || !x_gather || !expert_start || (!pre_act && act_dtype == MTS_F32) || !post_act) return MTS_ERR_NULL;
     if ((weights != nullptr) != (s_scatter != nullptr)) return MTS_ERR_NULL;   // the routing weight needs the row -> entry map
     if (T <= 0 || K < 1) return MTS_ERR_SHAPE;
     if (act_dtype == MTS_F32) {
@@ -2709,7 +2713,7 @@ extern "C" int MTS_GEMM_ENTRY(mts_moe_fwd_gateup_down)(const void* x, const void
 #ifndef MTS_GEMM_F16
     if (act_dtype == MTS_F16) return mts_moe_fwd_gateup_down_f16(x, w1, w2, x_gather, expert_start, weights, s_scatter, T, K, E, H, I, act_dtype, pre_act, post_act, y, workspace, workspace_bytes, stream);
 #endif
-    if (!x || !w1 || !w2 || !x_gather || !expert_start || !pre_act || !post_act || !y || !workspace) return MTS_ERR_NULL;
+    if (!x || !w1 || !w2 || !x_gather || !expert_start || !post_act || !y || !workspace) return MTS_ERR_NULL;
     if ((weights != nullptr) != (s_scatter != nullptr)) return MTS_ERR_NULL;
     if (T <= 0 || K < 1) return MTS_ERR_SHAPE;
     if (act_dtype != MTS_GEMM_DTYPE) return MTS_ERR_DTYPE;

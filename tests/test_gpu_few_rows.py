@@ -73,11 +73,14 @@ def test_few_rows(T, K, E, H, I, dtype, weight_dtype, weighted):
         assert got[rows:].isnan().all()   # rows behind the last expert's are left alone
 
 
-def test_layer_with_and_without_a_backward_pass():
-    """fp32 weights are read as they are where no backward pass follows, and as rounded copies where one does: the same result."""
-    print("layer, few rows, master weights", flush=True)
+@pytest.mark.parametrize("T", [24, 700, 20000])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_layer_with_and_without_a_backward_pass(T, dtype):
+    """Where no backward pass follows the pre-activations are not kept and few rows read fp32 weights as they are: the same result
+    as with one, for few rows, small tiles and the joint launch."""
+    print(f"layer, master weights, T={T} {dtype}", flush=True)
     g = torch.Generator().manual_seed(2)
-    x = torch.randn(24, 256, generator=g).bfloat16().cuda()
+    x = torch.randn(T, 256, generator=g).to(dtype).cuda()
     w_r, w1, w2 = ((torch.randn(*s, generator=g) * 0.05).cuda().requires_grad_(True) for s in ((8, 256), (8, 512, 256), (8, 256, 256)))
     trained = moe_layer(x, w_r, w1, w2, 2, normalize=True)[0]
     with torch.no_grad():
