@@ -489,6 +489,14 @@ int mts_cross_entropy_bwd(const void* logits, const int64_t* targets, int64_t N,
                           const float* row_log_sum, const float* g_loss, const float* inv_count,
                           void* d_logits, void* stream);
 
+/* Weight gradient of a dense projection y = x W^T: dw [N,K] f32 = g^T x, g [T,N] and x [T,K] dense
+ * bf16 or fp16, fp32 sums in a fixed order.  N and K multiples of 8, at most 32 tiles of 256 x 256,
+ * T at least 1024 (mts_linear_dw_supported).                                               */
+int mts_linear_dw_supported(int act_dtype, int64_t T, int N, int K);
+int64_t mts_linear_dw_workspace_bytes(int64_t T, int N, int K);
+int mts_linear_dw(const void* g, const void* x, int64_t T, int N, int K, int act_dtype, float* dw,
+                  void* workspace, int64_t workspace_bytes, void* stream);
+
 /* Scaled dot-product attention of heads of 64 elements, bf16 or fp16, queries and keys of the
  * same length; causal != 0: query i sees keys 0..i.  Tensors are [B,heads,S,64], dense in the last
  * dimension, 16-byte aligned, other strides multiples of 8 elements.  fp32 scores, sums and

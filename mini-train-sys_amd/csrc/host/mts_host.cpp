@@ -841,6 +841,43 @@ struct QkvRope : torch::autograd::Function<QkvRope> {
     }
 };
 
+// A projection under autocast: the product is the library's, the gradient of its fp32 weight is summed in fp32 here.
+bool linear_supported(const Tensor& x, const Tensor& w) {
+    if (!(at::GradMode::is_enabled() && w.requires_grad() && all_plain(x, w) && x.is_cuda() && w.device() == x.device() && x.dim() >= 2 && w.dim() == 2 &&
+          w.scalar_type() == at::kFloat && (x.scalar_type() == at::kBFloat16 || x.scalar_type() == at::kHalf) && x.size(-1) == w.size(1) && x.numel() > 0))
+        return false;
+    if (!at::autocast::is_autocast_enabled(at::kCUDA) || at::autocast::get_autocast_dtype(at::kCUDA) != x.scalar_type()) return false;
+    return mts_linear_dw_supported(dtype_code(x), x.numel() / x.size(-1), w.size(0), w.size(1));
+}
+
+struct Linear : torch::autograd::Function<Linear> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w) {
+        const Tensor rounded = w.to(x.scalar_type());
+        ctx->save_for_backward({x, w, rounded});
+        return at::linear(x, rounded);
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        const variable_list s = ctx->get_saved_variables();
+        const Tensor &x = s[0], &w = s[1], &rounded = s[2];
+        c10::OptionalDeviceGuard guard(x.device());
+        const int64_t N = w.size(0), K = w.size(1), T = x.numel() / K;
+        if (at::GradMode::is_enabled()) {   // to be differentiated itself
+            const Tensor g = grads[0].reshape({T, N}), wide = g.to(at::kFloat);
+            return {at::matmul(g, w.to(x.scalar_type())).view(x.sizes()), at::matmul(wide.t().contiguous(), x.reshape({T, K}).to(at::kFloat))};
+        }
+        const Tensor g = dense16(grads[0].reshape({T, N})), in = dense16(x.reshape({T, K}));
+        Tensor dx, dw;
+        if (ctx->needs_input_grad(0)) dx = at::matmul(g, rounded).view(x.sizes());
+        if (ctx->needs_input_grad(1)) {
+            dw = f32({N, K}, x);
+            const int64_t ws_bytes = mts_linear_dw_workspace_bytes(T, N, K);
+            Tensor ws = ws_bytes ? bytes(ws_bytes, x) : Tensor();
+            check(mts_linear_dw(ptr(g), ptr(in), T, N, K, dtype_code(x), ptr_as<float>(dw), ptr(ws), ws_bytes, stream_of(x)), "mts_linear_dw");
+        }
+        return {dx, dw};
+    }
+};
+
 bool heads_fit(const Tensor& t) {   // as the kernels read them
     return t.stride(3) == 1 && t.stride(0) % 8 == 0 && t.stride(1) % 8 == 0 && t.stride(2) % 8 == 0 && aligned16(t);
 }
@@ -983,6 +1020,11 @@ PYBIND11_MODULE(_host, m) {
         c10::OptionalDeviceGuard guard(qkv.device());
         const variable_list v = QkvRope::apply(qkv, cos, sin, heads);
         return std::make_tuple(v[0], v[1], v[2]);
+    });
+    m.def("linear_supported", &linear_supported);
+    m.def("linear", [](const Tensor& x, const Tensor& w) {
+        c10::OptionalDeviceGuard guard(x.device());
+        return Linear::apply(x, w);
     });
     m.def("attention_supported", &attention_supported);
     m.def("attention", [](const Tensor& q, const Tensor& k, const Tensor& v, bool causal) {

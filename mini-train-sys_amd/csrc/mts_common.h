@@ -61,6 +61,7 @@ int mts_moe_bwd_dx_f16(const void* d_pre_act, const void* w1, int w1_as_stored, 
 int mts_moe_bwd_dw2_f16(const void* d_out, const void* weighted_act, const int32_t* x_gather,
                         const int32_t* expert_start, int64_t T, int K, int E, int H, int I, int act_dtype,
                         int grad_dtype, void* d_w2, void* workspace, int64_t workspace_bytes, void* stream);
+int mts_linear_dw_tiles_f16(const void* g, const void* x, int64_t T, int N, int K, float* part, void* stream);
 int mts_moe_bwd_dw1_f16(const void* d_pre_act, const void* x, const int32_t* x_gather, const int32_t* expert_start,
                         int64_t T, int K, int E, int H, int I, int act_dtype, int grad_dtype, void* d_w1,
                         void* workspace, int64_t workspace_bytes, void* stream);

@@ -1304,6 +1304,7 @@ struct DwParams {
     int E, n_tiles, tiles_per_expert;  // set by the launcher
     const int32_t* sched;   // the unit table of the joint backward launch's schedule (which units an XCD runs), or NULL:
     int sched_slots;        // unit u runs on XCD u % 8; sched_slots: table entries per XCD
+    int segment_rows;       // not 0: no experts, E segments of this many of the TK rows
 };
 
 // ---------------------------------------------------------------------------
@@ -1336,6 +1337,13 @@ __device__ __forceinline__ int dw_chunks(const DwParams& p, int count, int share
 
 // every lane of the calling wave gets the same answer
 __device__ __forceinline__ bool locate_dw_unit(const DwParams& p, int unit, DwUnit& u) {
+    if (p.segment_rows) {
+        const int64_t first = (int64_t)unit * p.segment_rows;
+        u.e = unit, u.slot = -1;
+        u.rbeg = (int)(first < p.TK ? first : p.TK);
+        u.rend = (int)(first + p.segment_rows < p.TK ? first + p.segment_rows : p.TK);
+        return unit < p.E;
+    }
     const int lane = threadIdx.x % MTS_WAVE;
     const int share = dw_share(p);
     int seen = 0, seen_slots = 0;
@@ -2868,6 +2876,88 @@ extern "C" int MTS_GEMM_ENTRY(mts_moe_bwd_dw1)(const void* d_pre_act, const void
     p.M = 2 * I; p.N = H; p.TK = T * K; p.expert_start = expert_start; p.C = d_w1;
     return launch_dw_any(K_DW1, p, E, grad_dtype, workspace, workspace_bytes, (hipStream_t)stream);
 }
+
+// ---------------------------------------------------------------------------
+// Weight gradient of a dense projection, dW [N,K] = g^T x over T rows, in fp32.  A projection of a decoder has few tiles
+// (768 x 768: 9 of 256 x 256) and a long reduction, so the rows are cut into segments, a multiple of the XCDs and as many as keep
+// an XCD's 32 CUs in one round; a segment's tiles run on one XCD, and a second kernel adds the segments' partial results
+// in their order.  24 576 rows: 768 x 768 166 -> 46 us (36 and the sum), 2304 x 768 194 -> 97 us against the library's products, which
+// the widening of their 16-bit results follows; both gradients of the projection 193 -> 83 and 288 -> 206, and no slower
+// down to 1024 rows (89 -> 70), the least that is measured.
+// ---------------------------------------------------------------------------
+namespace {
+constexpr int kLinearTiles = 32;   // CUs of an XCD
+struct LinearSplit {
+    int tiles, segments, rows;
+};
+LinearSplit linear_split(int64_t T, int N, int K) {
+    LinearSplit s;
+    s.tiles = ((N + DwWsWide::BM - 1) / DwWsWide::BM) * ((K + DwWsWide::BN - 1) / DwWsWide::BN);
+    const int64_t most = kXcds * (kLinearTiles / s.tiles > 0 ? kLinearTiles / s.tiles : 1);
+    const int64_t rows = ((T + most - 1) / most + DwWsWide::BKS - 1) / DwWsWide::BKS * DwWsWide::BKS;
+    s.rows = (int)rows;
+    s.segments = (int)((T + rows - 1) / rows);
+    return s;
+}
+
+#ifndef MTS_GEMM_F16
+__global__ __launch_bounds__(256) void linear_dw_sum_kernel(const f32x4* __restrict__ part, int segments, int64_t quads, f32x4* __restrict__ dw) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= quads) return;
+    f32x4 sum = part[i];
+#pragma unroll 8
+    for (int s = 1; s < segments; ++s) {
+        const f32x4 v = part[(int64_t)s * quads + i];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) sum[j] += v[j];
+    }
+    dw[i] = sum;
+}
+#endif
+}  // namespace
+
+#ifdef MTS_GEMM_F16
+extern "C" int mts_linear_dw_tiles_f16(const void* g, const void* x, int64_t T, int N, int K, float* part, void* stream) {
+#else
+static int linear_dw_tiles(const void* g, const void* x, int64_t T, int N, int K, float* part, void* stream) {
+#endif
+    const LinearSplit split = linear_split(T, N, K);
+    DwParams p = {};
+    p.P = (const bf16_t*)g; p.p_rows = T;
+    p.Q = (const bf16_t*)x; p.q_rows = T;
+    p.M = N; p.N = K; p.TK = T; p.C = part; p.segment_rows = split.rows;
+    const dim3 grid = dw_grid<DwWsWide>(p, split.segments, split.segments);
+    dw_gemm_ws_kernel<DwWsWide, float><<<grid, DwWsWide::NT, 0, (hipStream_t)stream>>>(p);
+    MTS_CHECK_LAUNCH();
+    return MTS_OK;
+}
+
+#ifndef MTS_GEMM_F16
+extern "C" int mts_linear_dw_supported(int act_dtype, int64_t T, int N, int K) {
+    if ((act_dtype != MTS_BF16 && act_dtype != MTS_F16) || N < 8 || K < 8 || N % 8 || K % 8 || T < 1024 || T > 0x7fffffffLL) return 0;
+    return (int64_t)N * K < (1LL << 30) && linear_split(T, N, K).tiles <= kLinearTiles;
+}
+extern "C" int64_t mts_linear_dw_workspace_bytes(int64_t T, int N, int K) {
+    const int segments = linear_split(T, N, K).segments;
+    return segments > 1 ? (int64_t)segments * N * K * 4 : 0;
+}
+extern "C" int mts_linear_dw(const void* g, const void* x, int64_t T, int N, int K, int act_dtype, float* dw, void* workspace, int64_t workspace_bytes,
+                             void* stream) {
+    if (!g || !x || !dw) return MTS_ERR_NULL;
+    if (act_dtype != MTS_BF16 && act_dtype != MTS_F16) return MTS_ERR_DTYPE;
+    if (!mts_linear_dw_supported(act_dtype, T, N, K)) return MTS_ERR_SHAPE;
+    const int segments = linear_split(T, N, K).segments;
+    if (segments > 1 && (!workspace || workspace_bytes < mts_linear_dw_workspace_bytes(T, N, K))) return MTS_ERR_WORKSPACE;
+    if (!mts_aligned16(g) || !mts_aligned16(x) || !mts_aligned16(dw) || !mts_aligned16(workspace)) return MTS_ERR_ALIGN;
+    float* part = segments > 1 ? (float*)workspace : dw;
+    const int rc = act_dtype == MTS_F16 ? mts_linear_dw_tiles_f16(g, x, T, N, K, part, stream) : linear_dw_tiles(g, x, T, N, K, part, stream);
+    if (rc || segments == 1) return rc;
+    const int64_t quads = (int64_t)N * K / 4;
+    linear_dw_sum_kernel<<<dim3((unsigned)((quads + 255) / 256)), 256, 0, (hipStream_t)stream>>>((const f32x4*)part, segments, quads, (f32x4*)dw);
+    MTS_CHECK_LAUNCH();
+    return MTS_OK;
+}
+#endif
 
 #ifndef MTS_GEMM_F16
 extern "C" int mts_moe_bwd_joint_supported(int act_dtype, int H, int I) {

@@ -67,6 +67,12 @@ class HipOpsBackend(DenseTorchOps):
             return None
         return dense.qkv_rope(qkv, cos, sin, heads)
 
+    def linear(self, x, weight):
+        """Extension: ``F.linear(x, weight)``, or None where the caller's own does as well."""
+        if not dense.is_linear_supported(x, weight):
+            return None
+        return dense.linear(x, weight)
+
     def attention(self, q, k, v, *, is_causal, dropout_p):
         if not dropout_p and dense.is_attention_supported(q, k, v):
             return dense.attention(q, k, v, is_causal)

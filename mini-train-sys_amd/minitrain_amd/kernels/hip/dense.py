@@ -49,6 +49,15 @@ def qkv_rope(qkv, cos, sin, heads: int):
     return _lib.host().qkv_rope(qkv, cos, sin, heads)
 
 
+def is_linear_supported(x, weight) -> bool:
+    return _may_replace(x, weight) and _lib.host().linear_supported(x, weight)
+
+
+def linear(x, weight):
+    """``F.linear(x, weight)`` under autocast, with the gradient of the fp32 ``weight`` summed in fp32"""
+    return _lib.host().linear(x, weight)
+
+
 def is_attention_supported(q, k, v) -> bool:
     return _may_replace(q, k, v) and _lib.host().attention_supported(q, k, v)
 

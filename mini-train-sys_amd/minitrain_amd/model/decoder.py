@@ -59,6 +59,13 @@ def sum_and_norm(norm: RMSNorm, x: torch.Tensor, residual: torch.Tensor | None, 
     return x, norm(x, ops)
 
 
+def project(linear: nn.Linear, x: torch.Tensor, ops: OpsBackend) -> torch.Tensor:
+    """``linear(x)``, by the backend's own operator where it has one for these operands."""
+    own = getattr(ops, "linear", None)
+    y = own(x, linear.weight) if own is not None and runs_as_written(linear, nn.Linear) and linear.bias is None else None
+    return linear(x) if y is None else y
+
+
 class CausalSelfAttention(nn.Module):
     def __init__(self, cfg: ModelConfig) -> None:
         super().__init__()
@@ -71,7 +78,7 @@ class CausalSelfAttention(nn.Module):
 
     def forward(self, x, ops: OpsBackend, rope_cos, rope_sin):
         B, S, H = x.shape
-        qkv = self.qkv(x)
+        qkv = project(self.qkv, x, ops)
         packed = getattr(ops, "qkv_rope", None)   # a backend may take the packed projection as it is
         turned = packed(qkv, rope_cos, rope_sin, self.n_heads) if packed is not None else None
         if turned is not None:
@@ -80,7 +87,7 @@ class CausalSelfAttention(nn.Module):
             q, k, v = (t.view(B, S, self.n_heads, self.head_dim).transpose(1, 2) for t in qkv.chunk(3, dim=-1))
             q, k = ops.rope(q, k, rope_cos, rope_sin)
         ctx = ops.attention(q, k, v, is_causal=True, dropout_p=self.p_drop if self.training else 0.0)
-        return self.resid_dropout(self.out(ctx.transpose(1, 2).reshape(B, S, H)))
+        return self.resid_dropout(project(self.out, ctx.transpose(1, 2).reshape(B, S, H), ops))
 
 
 class TransformerBlock(nn.Module):

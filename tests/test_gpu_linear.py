@@ -1,0 +1,48 @@
+"""Projection under autocast with the weight gradient summed in fp32, against fp64 products of the rounded operands (GPU).
+
+The sum of T products of order one in fp32, in segments: an error of at most sqrt(T) * 2^-24 of its own size with margin, 1e-5
+of the largest value for the lengths here.  The other results carry one 16-bit rounding (2^-8, 2^-11)."""
+
+import pytest
+import torch
+
+from minitrain_amd.kernels.hip import dense
+from tests.helpers import hip_backend
+
+pytestmark = pytest.mark.gpu
+
+ULP = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}
+
+
+@pytest.mark.parametrize("T,N,K", [(1024, 8, 8), (1025, 256, 256), (1600, 264, 248), (4099, 768, 768), (2000, 2304, 768), (9000, 1032, 40), (1500, 1000, 2048)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_linear(T, N, K, dtype):
+    """Segments of one k-tile and of several, the last one partly filled, widths that are not whole tiles, one tile and 32."""
+    print(f"linear T={T} N={N} K={K} {dtype}", flush=True)
+    g = torch.Generator().manual_seed(T)
+    x = torch.randn(T, K, generator=g).to(dtype).cuda().requires_grad_(True)
+    w = (torch.randn(N, K, generator=g) * K ** -0.5).cuda().requires_grad_(True)
+    grad = torch.randn(T, N, generator=g).to(dtype).cuda()
+    with torch.autocast("cuda", dtype=dtype):
+        y = hip_backend().linear(x, w)
+    assert y is not None and y.dtype == dtype
+    y.backward(grad)
+    wide = w.detach().to(dtype).double()
+    for got, want, tol, what in ((y.detach(), x.detach().double() @ wide.T, ULP[dtype], "y"), (x.grad, grad.double() @ wide, ULP[dtype], "dx"),
+                                 (w.grad, grad.double().T @ x.detach().double(), 1e-5, "dw")):
+        err, scale = float((got.double() - want).abs().max()), float(want.abs().max())
+        assert err <= tol * scale, (what, err, scale)
+    assert w.grad.dtype == torch.float32
+
+
+def test_other_calls_stay_stock():
+    x = torch.randn(2, 1024, 64, device="cuda", dtype=torch.bfloat16)
+    w = torch.randn(64, 64, device="cuda", requires_grad=True)
+    assert not dense.is_linear_supported(x, w)   # without autocast the types do not go together
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert dense.is_linear_supported(x, w)
+        assert not dense.is_linear_supported(x[:, :8], w) and not dense.is_linear_supported(x, w.detach()) and not dense.is_linear_supported(x.float(), w)
+        with torch.no_grad():
+            assert not dense.is_linear_supported(x, w)
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert not dense.is_linear_supported(x, w)
