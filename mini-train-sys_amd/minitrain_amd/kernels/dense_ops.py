@@ -1,8 +1,8 @@
-"""The six operators that stay on stock PyTorch-ROCm.
+"""The six operators outside the MoE path on stock PyTorch-ROCm.
 
-The `hip` backend replaces only the two MoE operators; like the reference's
-Triton backend (minitrain/kernels/triton/__init__.py:36) it inherits the rest
-from a plain PyTorch class.  This base class deliberately has NO
+Like the reference's Triton backend (minitrain/kernels/triton/__init__.py:36) the `hip`
+backend inherits them from a plain PyTorch class; where a kernel of its own takes a call
+(``kernels/hip/dense.py``) it stands in.  This base class deliberately has NO
 ``router_postprocess`` and NO ``fused_moe``: there is nothing for the MoE path to
 fall back to.
 """

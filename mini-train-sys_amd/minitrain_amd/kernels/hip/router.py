@@ -69,7 +69,7 @@ def is_router_logits_supported(hidden_states: torch.Tensor, weight: torch.Tensor
 
 
 def router_logits(hidden_states: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
-    """fp32 router logits of ``hidden_states`` [T,H] (bf16 or fp32) and ``weight`` [E,H] (fp32).
+    """fp32 router logits of ``hidden_states`` [T,H] (bf16, fp16 or fp32) and ``weight`` [E,H] (fp32).
 
     Stands in for ``F.linear(hidden_states.float(), weight.float())`` of the reference's
     TopKRouter.forward (minitrain/model/moe_router.py:64-76).
@@ -77,7 +77,7 @@ def router_logits(hidden_states: torch.Tensor, weight: torch.Tensor) -> torch.Te
 
     if not is_router_logits_supported(hidden_states, weight):
         raise RuntimeError(
-            "hip router_logits requires 2D bf16/fp32 activations and a 2D fp32 weight on the GPU with "
-            "at most 16 experts and a hidden size that is a multiple of 4 and at most 4096 (E * H <= 32768)"
+            "hip router_logits requires 2D bf16/fp16/fp32 activations and a 2D fp32 weight on the GPU with at most 1024 experts, "
+            "and up to 16 of them a hidden size that is a multiple of 4 and at most 4096 (E * H <= 32768)"
         )
     return _lib.host().router_logits(hidden_states, weight)
