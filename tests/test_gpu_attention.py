@@ -65,6 +65,40 @@ def test_large_scores_and_rows_without_a_finite_score():
     assert out[0, 0, :4].isnan().all() and out[0, 0, 4:].isfinite().all() and out[0, 1].isfinite().all()
 
 
+def _layouts():
+    g = torch.Generator().manual_seed(9)
+    r = lambda *shape: torch.randn(*shape, generator=g).bfloat16().cuda()
+    yield "heads in front", [r(3, 2, 70, 64).transpose(0, 1) for _ in range(3)]
+    yield "rows in front", [r(70, 2, 3, 64).permute(1, 2, 0, 3) for _ in range(3)]
+    yield "one batch for all", [r(1, 3, 70, 64).expand(2, 3, 70, 64) for _ in range(3)]
+    yield "one head for all keys and values", [r(2, 3, 70, 64), r(2, 1, 70, 64).expand(2, 3, 70, 64), r(2, 1, 70, 64).expand(2, 3, 70, 64)]
+    yield "every other row", [r(2, 3, 140, 64)[:, :, ::2] for _ in range(3)]
+    yield "part of a wider row", [r(2, 3, 70, 136)[..., 8:72] for _ in range(3)]
+
+
+@pytest.mark.parametrize("which", range(6))
+@pytest.mark.parametrize("grad_layout", ["dense", "one value", "rows in front", "misaligned"])
+def test_layouts(which, grad_layout):
+    """Every order of the outer dimensions, strides of zero, rows apart; gradients as reductions and slices leave them."""
+    name, (q, k, v) = list(_layouts())[which]
+    print(f"attention, {name}, gradient {grad_layout}", flush=True)
+    assert dense.is_attention_supported(q, k, v)
+    leaves = [t.detach().requires_grad_(True) for t in (q, k, v)]
+    ref = [t.detach().double().requires_grad_(True) for t in (q, k, v)]
+    g = torch.Generator().manual_seed(10)
+    grad = {"dense": lambda: torch.randn(2, 3, 70, 64, generator=g), "one value": lambda: torch.ones(()).expand(2, 3, 70, 64),
+            "rows in front": lambda: torch.randn(70, 3, 2, 64, generator=g).permute(2, 1, 0, 3),
+            "misaligned": lambda: torch.randn(2, 3, 70, 65, generator=g)}[grad_layout]().bfloat16().cuda()
+    grad = grad[..., 1:] if grad_layout == "misaligned" else grad
+    out = hip_backend().attention(*leaves, is_causal=True, dropout_p=0.0)
+    out.backward(grad)
+    want = _written_out(*ref, True)
+    want.backward(grad.double())
+    _close(out.detach(), want.detach(), TOL[torch.bfloat16], "out")
+    for got, w, what in zip(leaves, ref, ("dq", "dk", "dv")):
+        _close(got.grad, w.grad, 2 * TOL[torch.bfloat16], what)
+
+
 def test_other_layouts_types_and_choices_stay_stock():
     ops, stock = hip_backend(), DenseTorchOps()
     q = torch.randn(1, 2, 40, 64, device="cuda", dtype=torch.bfloat16)

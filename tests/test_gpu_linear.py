@@ -35,6 +35,27 @@ def test_linear(T, N, K, dtype):
     assert w.grad.dtype == torch.float32
 
 
+@pytest.mark.parametrize("layout", ["sequence first", "every other row", "part of a wider row", "misaligned", "gradient of one value"])
+def test_layouts(layout):
+    """Operands and gradients that are not dense or not aligned go through a copy: the same sums."""
+    print(f"linear, {layout}", flush=True)
+    g = torch.Generator().manual_seed(3)
+    r = lambda *shape: torch.randn(*shape, generator=g).bfloat16().cuda()
+    x = {"sequence first": lambda: r(600, 2, 64).transpose(0, 1), "every other row": lambda: r(2, 1200, 64)[:, ::2], "misaligned": lambda: r(2, 600, 65)[..., 1:],
+         "part of a wider row": lambda: r(2, 600, 128)[..., 32:96], "gradient of one value": lambda: r(2, 600, 64)}[layout]()
+    w = torch.randn(72, 64, generator=g).cuda().requires_grad_(True)
+    x = x.detach().requires_grad_(True)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        y = hip_backend().linear(x, w)
+    grad = torch.ones((), device="cuda", dtype=torch.bfloat16).expand(2, 600, 72) if layout == "gradient of one value" else r(2, 72, 600).transpose(1, 2)
+    y.backward(grad)
+    wide = w.detach().bfloat16().double()
+    for got, want, tol, what in ((y.detach(), x.detach().double() @ wide.T, ULP[torch.bfloat16], "y"), (x.grad, grad.double() @ wide, ULP[torch.bfloat16], "dx"),
+                                 (w.grad, grad.double().reshape(-1, 72).T @ x.detach().double().reshape(-1, 64), 1e-5, "dw")):
+        err, scale = float((got.double() - want).abs().max()), float(want.abs().max())
+        assert got.shape == want.shape and err <= tol * scale, (what, err, scale)
+
+
 def test_other_calls_stay_stock():
     x = torch.randn(2, 1024, 64, device="cuda", dtype=torch.bfloat16)
     w = torch.randn(64, 64, device="cuda", requires_grad=True)
