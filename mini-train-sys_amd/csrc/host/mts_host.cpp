@@ -329,6 +329,9 @@ struct ExpertGrads {
     Tensor dx, dw1, dw2, ds;
 };
 
+// The projection of many experts stands in for a library product that takes any alignment.
+Tensor dense_router_operand(const Tensor& t, int64_t E) { return E > kFewExperts ? dense16(t) : t.contiguous(); }
+
 void router_projection_forward(const Tensor& x, const Tensor& w, const Tensor& logits) {
     const int64_t T = x.size(0), H = x.size(1), E = w.size(0);
     if (E > kFewExperts)
@@ -537,7 +540,8 @@ struct MoELayer : torch::autograd::Function<MoELayer> {
     static variable_list forward(AutogradContext* ctx, const Tensor& x_, const Tensor& w_r_, const Tensor& w1_, const Tensor& w2_, int64_t K, bool normalize,
                                  int64_t capacity, int64_t switches, int64_t limit) {
         const Options opt{switches, limit};
-        const Tensor x = x_.contiguous(), w_r = w_r_.contiguous(), w1 = w1_.contiguous(), w2 = w2_.contiguous();
+        const Tensor x = dense_router_operand(x_, w_r_.size(0)), w_r = dense_router_operand(w_r_, w_r_.size(0));
+        const Tensor w1 = w1_.contiguous(), w2 = w2_.contiguous();
         const int64_t T = x.size(0), H = x.size(1), E = w_r.size(0), TK = T * K;
         const bool narrow = x.scalar_type() != at::kFloat, limited = capacity >= 0;
         Tensor logits = f32({T, E}, x), weights = f32({T, K}, x), indices = i32({T, K}, x);
@@ -997,7 +1001,7 @@ PYBIND11_MODULE(_host, m) {
     });
     m.def("router_logits", [](const Tensor& x, const Tensor& w) {
         c10::OptionalDeviceGuard guard(x.device());
-        return RouterLogits::apply(x.contiguous(), w.contiguous());
+        return RouterLogits::apply(dense_router_operand(x, w.size(0)), dense_router_operand(w, w.size(0)));
     });
     m.def("rmsnorm_supported", &rmsnorm_supported);
     m.def("rmsnorm", [](const Tensor& x, const Tensor& w, double eps) {

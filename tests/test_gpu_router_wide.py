@@ -27,6 +27,27 @@ def test_wide_projection(T, H, E, dtype):
     assert_close_scaled(b.grad, go.double().T @ x.double(), 1e-5, "dW")
 
 
+def _misaligned(t):
+    """A dense copy that starts one element behind a 16-byte boundary."""
+    return torch.empty(t.numel() + 8, dtype=t.dtype, device="cuda")[1:1 + t.numel()].copy_(t.flatten()).view(t.shape)
+
+
+def test_operands_that_start_anywhere():
+    """The library product that this projection stands in for takes any alignment."""
+    print("wide projection, misaligned", flush=True)
+    ops = hip_backend()
+    x, w_r, w1, w2, g = (t.cuda() for t in O.make_inputs(3, 100, 64, 24, 32))
+    results = []
+    for place in (lambda t: t.clone(), _misaligned):
+        leaves = [place(x).requires_grad_(True), place(w_r).requires_grad_(True), w1.clone().requires_grad_(True), w2.clone().requires_grad_(True)]
+        out = ops.moe_layer(*leaves, 4, normalize=True)[0]
+        out.backward(g)
+        logits = ops.router_logits(leaves[0], leaves[1])
+        results.append([out.detach(), logits.detach(), *(t.grad for t in leaves)])
+    for a, b in zip(*results):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("T,H,E,I,K,capacity", [(500, 128, 24, 64, 2, None), (1000, 256, 64, 128, 4, None), (300, 64, 130, 64, 8, None), (1000, 128, 32, 64, 4, 60)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_layer_node_of_many_experts(T, H, E, I, K, capacity, dtype):
