@@ -121,14 +121,13 @@ __global__ __launch_bounds__(kThreads) void router_fwd_kernel(
     }
 }
 
-// 16 waves: a column of the partials per wave and round (66 columns at 64 experts: 35 us on four waves)
 constexpr int kStatsThreads = 1024;
 __global__ __launch_bounds__(kStatsThreads) void router_stats_kernel(
     const float* __restrict__ partial, const int32_t* __restrict__ partial_counts, int nblocks, int E,
     float inv_t, float inv_routes, float* __restrict__ prob_mean, float* __restrict__ z_loss,
     float* __restrict__ entropy, int32_t* __restrict__ counts, float* __restrict__ load_balance,
     float* __restrict__ load_stats) {
-    stats_block<kStatsThreads / MTS_WAVE>(partial, partial_counts, nblocks, E, inv_t, inv_routes, prob_mean, z_loss, entropy,
+    stats_block<kStatsThreads>(partial, partial_counts, nblocks, E, inv_t, inv_routes, prob_mean, z_loss, entropy,
                                      counts, load_balance, load_stats, threadIdx.x / MTS_WAVE);
 }
 

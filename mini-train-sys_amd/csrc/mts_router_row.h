@@ -259,38 +259,47 @@ __device__ __forceinline__ void stats_finalize(const StatsShared& sh, int wave, 
     }
 }
 
-// mean of column i of the partials over nblocks blocks: lanes stride over the blocks, the lane sums
-// meet in a fixed shuffle tree
-__device__ __forceinline__ float stats_column_mean(const float* __restrict__ partial, int nblocks, int E, int i,
-                                                   float inv_t) {
-    const int lane = threadIdx.x % MTS_WAVE;
-    float v = 0.f;
-    for (int b = lane; b < nblocks; b += MTS_WAVE) v += partial[(int64_t)b * (E + 2) + i];
-    return wave_sum(v) * inv_t;
-}
-
-// The whole reduction by one block of NWAVES waves: wave w takes columns w, w + NWAVES, ...
-template <int NWAVES>
+// The whole reduction by one block: neighbouring threads take neighbouring columns of the partials, sets of them every
+// (sets)th row, and the sets' sums are added in order.  (A column per wave, a row per lane, asks for a line per value: 17 us for
+// 256 rows of 66 columns, this 9.)
+template <int THREADS>
 __device__ __forceinline__ void stats_block(
     const float* __restrict__ partial, const int32_t* __restrict__ partial_counts, int nblocks, int E,
     float inv_t, float inv_routes, float* __restrict__ prob_mean, float* __restrict__ z_loss,
     float* __restrict__ entropy, int32_t* __restrict__ counts, float* __restrict__ load_balance,
     float* __restrict__ load_stats, int wave) {
     __shared__ StatsShared sh;
-    const int lane = threadIdx.x % MTS_WAVE;
-    for (int i = wave; i < E + 2; i += NWAVES) {
-        const float v = stats_column_mean(partial, nblocks, E, i, inv_t);
-        int c = 0;
-        if (i < E) {
-            for (int b = lane; b < nblocks; b += MTS_WAVE) c += partial_counts[(int64_t)b * E + i];
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, MTS_WAVE);
+    __shared__ float set_sum[THREADS];
+    __shared__ int32_t set_count[THREADS];
+    int width = 16;
+    while (width < E + 2 && width < THREADS) width <<= 1;
+    const int sets = THREADS / width, set = threadIdx.x / width;
+    for (int i0 = 0; i0 < E + 2; i0 += width) {
+        const int i = i0 + threadIdx.x % width;
+        float v = 0.f;
+        int32_t c = 0;
+        if (i < E + 2) {
+#pragma unroll 8
+            for (int b = set; b < nblocks; b += sets) {
+                v += partial[(int64_t)b * (E + 2) + i];
+                c += i < E ? partial_counts[(int64_t)b * E + i] : 0;
+            }
         }
-        if (lane == 0) stats_column(sh, i, v, c, E, inv_routes, prob_mean, z_loss, entropy, counts);
+        set_sum[threadIdx.x] = v;
+        set_count[threadIdx.x] = c;
+        __syncthreads();
+        if (set == 0 && i < E + 2) {
+#pragma unroll 8
+            for (int k = 1; k < sets; ++k) {
+                v += set_sum[k * width + threadIdx.x];
+                c += set_count[k * width + threadIdx.x];
+            }
+            stats_column(sh, i, v * inv_t, c, E, inv_routes, prob_mean, z_loss, entropy, counts);
+        }
+        __syncthreads();
     }
     if (!load_balance && !load_stats) return;   // block-uniform
-    __syncthreads();
-    stats_finalize(sh, wave, 0, 1 % NWAVES, E, load_balance, load_stats);
+    stats_finalize(sh, wave, 0, 1, E, load_balance, load_stats);
 }
 
 }  // namespace mts_router
