@@ -26,11 +26,11 @@ __device__ __forceinline__ uint32_t order_key(float w) {
 
 // One pass of the select over the keys of a thread: counts the digit at `shift` of the keys
 // whose higher digits equal `prefix`.  Router weights share their leading bits, so most lanes
-// of a wave hit the same bin in the first passes: the two most common digits of a wave are
-// added once per wave.
-__device__ __forceinline__ void count_digit(uint32_t* hist, bool count, uint32_t d, int lane) {
+// of a wave hit the same bin in the first pass (`crowded`), where the two most common digits of a wave are
+// added once per wave; the digits behind it are mantissa bits, spread over the bins (all passes that way: 38 us for 49 152 routes to 8 experts, this 33).
+__device__ __forceinline__ void count_digit(uint32_t* hist, bool count, uint32_t d, int lane, bool crowded) {
 #pragma unroll
-    for (int r = 0; r < 2; ++r) {
+    for (int r = 0; crowded && r < 2; ++r) {
         const uint64_t todo = __ballot(count);
         if (!todo) break;
         const int leader = __ffsll((unsigned long long)todo) - 1;
@@ -145,7 +145,7 @@ __device__ __forceinline__ void select_segment(const float* __restrict__ w, cons
             for (int u = 0; u < kRegKeys; ++u) {
                 const int i = tid + u * kSelThreads;
                 const bool count = i < n && (pass == 0 || (kr[u] >> (shift + 8)) == prefix);
-                if (u * kSelThreads < n) count_digit(hist, count, (kr[u] >> shift) & 255u, lane);
+                if (u * kSelThreads < n) count_digit(hist, count, (kr[u] >> shift) & 255u, lane, pass == 0);
             }
         } else {
             for (int i0 = tid; i0 < n; i0 += kUnroll * kSelThreads) {
@@ -159,7 +159,7 @@ __device__ __forceinline__ void select_segment(const float* __restrict__ w, cons
                 for (int u = 0; u < kUnroll; ++u) {
                     const int i = i0 + u * kSelThreads;
                     const bool count = i < n && (pass == 0 || (k[u] >> (shift + 8)) == prefix);
-                    count_digit(hist, count, (k[u] >> shift) & 255u, lane);
+                    count_digit(hist, count, (k[u] >> shift) & 255u, lane, pass == 0);
                 }
             }
         }
