@@ -12,6 +12,9 @@
 // quarter of the rate), maxima, sums and conversions.  bf16, causal, 12 heads of 64, 1024 rows, against the stock operator:
 // batch 8: 31 us forward (79) and 121 backward (308); batch 24: 72 us (534 TFLOP/s; 168) and 304 (445 TFLOP/s of the seven
 // products that two separate kernels form, so that each gradient is summed by one block in a fixed order; 844).
+//
+// Error against fp64 (2-norm, bf16, 24 heads x 1024): output 2.0e-3, dQ 2.5e-3, dK 2.4e-3, dV 2.3e-3, the stock operator's to
+// three digits; likewise at 200 and 777 rows, for scores three times as far apart, and in fp16.
 #include "mts_common.h"
 
 namespace {
