@@ -779,8 +779,11 @@ void launch_rope(const std::vector<RopeJob>& jobs, const Tensor& cos, const Tens
     check(mts_rope(array, (int)jobs.size(), ptr(cos), ptr(sin), t.size(0), t.size(2), t.size(1), t.size(3), dtype_code(t), stream_of(t)), "mts_rope");
 }
 Tensor dense_rows(const Tensor& t) { return t.stride(-1) == 1 ? t : t.contiguous(); }
-// [B, S, heads, D] in memory, as the projection that queries and keys are views of
-Tensor heads_inside(const Tensor& like, int64_t B, int64_t heads, int64_t S, int64_t D) { return at::empty({B, S, heads, D}, like.options()).transpose(1, 2); }
+// [B, S, heads, D] in memory, as the projection that queries and keys are views of.  A tensor of its own: autograd lets nobody
+// change the view that a node returns.
+Tensor heads_inside(const Tensor& like, int64_t B, int64_t heads, int64_t S, int64_t D) {
+    return at::empty_strided({B, heads, S, D}, {S * heads * D, D, heads * D, 1}, like.options());
+}
 
 struct Rope : torch::autograd::Function<Rope> {
     static variable_list turn(const Tensor& q_, const Tensor& k_, const Tensor& cos, const Tensor& sin, int64_t mode) {
@@ -944,14 +947,15 @@ bool cross_entropy_supported(const Tensor& logits, const Tensor& targets) {
 struct CrossEntropy : torch::autograd::Function<CrossEntropy> {
     static Tensor forward(AutogradContext* ctx, const Tensor& logits, const Tensor& targets) {   // dense16, dense
         const int64_t N = logits.size(0), V = logits.size(1);
-        Tensor rows = f32({3, N}, logits), scalars = f32({2}, logits);   // per row: maximum, log of the sum, loss; loss, 1 / count
+        // per row: maximum, log of the sum, loss; then 1 / count.  The loss is a tensor of its own, which the caller may change
+        // (no view) and which is not kept.
+        Tensor rows = f32({3 * N + 1}, logits), loss = f32({}, logits);
         float* row = ptr_as<float>(rows);
-        float* scalar = ptr_as<float>(scalars);
-        check(mts_cross_entropy_fwd(ptr(logits), ptr_as<int64_t>(targets), N, V, kIgnoreIndex, dtype_code(logits), row, row + N, row + 2 * N, scalar, scalar + 1,
-                                    stream_of(logits)),
+        check(mts_cross_entropy_fwd(ptr(logits), ptr_as<int64_t>(targets), N, V, kIgnoreIndex, dtype_code(logits), row, row + N, row + 2 * N,
+                                    ptr_as<float>(loss), row + 3 * N, stream_of(logits)),
               "mts_cross_entropy_fwd");
-        ctx->save_for_backward({logits, targets, rows, scalars});
-        return scalars.select(0, 0);
+        ctx->save_for_backward({logits, targets, rows});
+        return loss;
     }
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
         const variable_list s = ctx->get_saved_variables();
@@ -961,12 +965,12 @@ struct CrossEntropy : torch::autograd::Function<CrossEntropy> {
         if (at::GradMode::is_enabled()) {
             const Tensor t = s[1].unsqueeze(1), hit = at::arange(V, s[1].options()).unsqueeze(0).eq(t);
             const Tensor p = at::softmax(s[0].to(at::kFloat), 1) - hit.to(at::kFloat);
-            return {at::where(t.eq(kIgnoreIndex), at::zeros({}, p.options()), p * (g * s[3].select(0, 1))).to(s[0].scalar_type()), Tensor()};
+            return {at::where(t.eq(kIgnoreIndex), at::zeros({}, p.options()), p * (g * s[2].select(0, 3 * N))).to(s[0].scalar_type()), Tensor()};
         }
         Tensor d = at::empty_like(s[0]);
         const float* row = ptr_as<float>(s[2]);
         check(mts_cross_entropy_bwd(ptr(s[0]), ptr_as<int64_t>(s[1]), N, V, kIgnoreIndex, dtype_code(s[0]), row, row + N, ptr_as<float>(g),
-                                    ptr_as<float>(s[3]) + 1, ptr(d), stream_of(s[0])),
+                                    row + 3 * N, ptr(d), stream_of(s[0])),
               "mts_cross_entropy_bwd");
         return {d, Tensor()};
     }

@@ -123,3 +123,30 @@ def test_cross_entropy_without_valid_targets_and_outside_the_vocabulary():
     logits = torch.randn(3, 9, device="cuda")
     assert torch.isnan(ops.cross_entropy(logits, torch.full((3,), -100, device="cuda")))
     assert torch.isnan(ops.cross_entropy(logits, torch.tensor([0, 9, 1], device="cuda")))
+
+
+def test_results_may_be_changed_in_place():
+    """The loss, rotated queries and keys and the attention's result are tensors of their own, as the stock operators' are."""
+    print("results changed in place", flush=True)
+    g = torch.Generator().manual_seed(2)
+    logits, targets = torch.randn(6, 9, generator=g).bfloat16().cuda(), torch.randint(0, 9, (6,), generator=g).cuda()
+    q, k, v = (torch.randn(2, 3, 5, 64, generator=g).bfloat16().cuda() for _ in range(3))
+    angle = torch.rand(5, 64, generator=g) * 6.3
+    cos, sin = angle.cos().bfloat16().cuda(), angle.sin().bfloat16().cuda()
+    got = []
+    for ops in (hip_backend(), STOCK):
+        a, b, c = (t.clone().requires_grad_(True) for t in (logits, q, k))
+        loss = ops.cross_entropy(a, targets)
+        loss.detach().mul_(3)   # as a logged copy that is reduced over ranks
+        loss /= 3
+        rotated = ops.rope(b, c, cos, sin)
+        for t in rotated:
+            t *= 2
+        torch.autograd.backward((loss, *rotated), (torch.ones_like(loss), q, k))
+        got.append([loss.detach(), *(t.detach() for t in rotated), a.grad, b.grad, c.grad])
+    for i, (a, b) in enumerate(zip(*got)):
+        _close(a, b, 1e-6 if i == 0 else ULP[torch.bfloat16], i)
+    packed = torch.cat([t.transpose(1, 2).reshape(2, 5, -1) for t in (q, k, v)], -1).requires_grad_(True)
+    out = hip_backend().attention(*(t.detach().requires_grad_(True) for t in (q, k, v)), is_causal=True, dropout_p=0.0)
+    for t in (*hip_backend().qkv_rope(packed, cos, sin, 3)[:2], out):
+        t *= 2
