@@ -69,20 +69,28 @@ Tensor dense16(const Tensor& t) {   // dense and starting on a 16-byte boundary 
 }
 // Whether a kernel may be run on the tensors' memory in the place of stock operators: not where those are looked at by a
 // function transform (vmap, grad, forward mode), a trace, a dispatch mode or a subclass.
-bool nobody_looks() {
+bool nobody_dispatches() {
     using c10::DispatchKey;
     return !c10::impl::tls_is_dispatch_key_included(DispatchKey::FuncTorchDynamicLayerFrontMode) &&
-           !c10::impl::tls_is_dispatch_key_included(DispatchKey::Tracer) && !c10::impl::TorchDispatchModeTLS::any_modes_set() &&
-           !at::impl::torch_function_mode_enabled();
+           !c10::impl::tls_is_dispatch_key_included(DispatchKey::Tracer) && !c10::impl::TorchDispatchModeTLS::any_modes_set();
 }
 bool is_plain(const Tensor& t) {
-    static const c10::DispatchKeySet wrapped({c10::DispatchKey::Python, c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
-                                              c10::DispatchKey::Functionalize, c10::DispatchKey::Conjugate, c10::DispatchKey::Negative});
+    using c10::DispatchKey;
+    static const c10::DispatchKeySet wrapped({DispatchKey::Python, DispatchKey::Batched, DispatchKey::FuncTorchBatched, DispatchKey::FuncTorchGradWrapper,
+                                              DispatchKey::Functionalize, DispatchKey::Conjugate, DispatchKey::Negative, DispatchKey::ZeroTensor});
     return !t.key_set().has_any(wrapped) && !t._fw_grad(/*level=*/0).defined();
 }
 template <typename... Ts>
 bool all_plain(const Ts&... t) {
-    return nobody_looks() && (is_plain(t) && ...);
+    return nobody_dispatches() && !at::impl::torch_function_mode_enabled() && (is_plain(t) && ...);
+}
+// Whether a backward pass is written out in stock operators: its gradients are themselves to be differentiated (create_graph),
+// they come batched or wrapped (is_grads_batched, vmap over autograd.grad), or somebody looks on.
+bool written_out(const variable_list& grads) {
+    if (at::GradMode::is_enabled() || !nobody_dispatches()) return true;
+    for (const Tensor& g : grads)
+        if (g.defined() && !is_plain(g)) return true;
+    return false;
 }
 int64_t round4(int64_t n) { return (n + 3) / 4 * 4; }
 
@@ -684,8 +692,11 @@ struct RouterLogits : torch::autograd::Function<RouterLogits> {
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
         const variable_list s = ctx->get_saved_variables();
         c10::OptionalDeviceGuard guard(s[0].device());
+        if (written_out(grads)) {
+            const Tensor wide = grads[0].to(at::kFloat);
+            return {wide.matmul(s[1]).to(s[0].scalar_type()), wide.t().matmul(s[0].to(at::kFloat))};
+        }
         const Tensor g = like_f32(grads[0]);
-        if (at::GradMode::is_enabled()) return {g.matmul(s[1]).to(s[0].scalar_type()), g.t().matmul(s[0].to(at::kFloat))};   // differentiable
         Tensor dx = at::empty_like(s[0]), dw = at::empty_like(s[1]);
         router_projection_backward(g, s[0], s[1], dx, dw);
         return {dx, dw};
@@ -694,8 +705,8 @@ struct RouterLogits : torch::autograd::Function<RouterLogits> {
 
 // ---- the decoder's dense operators -----------------------------------------------------------------------------------------------
 
-// Each gives way to stock operators where all_plain() does not hold, and computes a gradient that is itself to be
-// differentiated (create_graph) with them.
+// Each gives way to stock operators where all_plain() does not hold, and computes its gradients with them where
+// written_out() says so.
 
 bool rmsnorm_supported(const Tensor& x, const Tensor& w, const MaybeTensor& residual) {
     if (!(all_plain(x, w) && (!residual || is_plain(*residual)) && x.is_cuda() && w.is_cuda() && is_activation_type(x.scalar_type()) && w.scalar_type() == at::kFloat && w.dim() == 1 && x.dim() >= 1 &&
@@ -729,7 +740,7 @@ struct RMSNorm : torch::autograd::Function<RMSNorm> {
         if (!g_y.defined()) return {g_sum, with_sum ? g_sum : Tensor(), Tensor(), Tensor()};   // only the residual stream goes on
         c10::OptionalDeviceGuard guard(s[0].device());
         const int64_t H = s[0].size(-1), N = s[0].numel() / H, ws_bytes = mts_rmsnorm_bwd_workspace_bytes(N, H);
-        if (at::GradMode::is_enabled()) {
+        if (written_out(grads)) {
             const Tensor v = s[0].to(at::kFloat), r = at::rsqrt(v.square().mean(-1, true) + ctx->saved_data["eps"].toDouble()), n = v * r;
             const Tensor gy = g_y.to(at::kFloat), gw = gy * s[1];
             Tensor d = r * (gw - n * (gw * n).mean(-1, true));
@@ -785,6 +796,12 @@ Tensor heads_inside(const Tensor& like, int64_t B, int64_t heads, int64_t S, int
     return at::empty_strided({B, heads, S, D}, {S * heads * D, D, heads * D, 1}, like.options());
 }
 
+// the gradient of a turn in stock operators: the pairs turned back
+Tensor turned_back(const Tensor& g, const Tensor& cos, const Tensor& sin) {
+    const variable_list h = (g * sin).chunk(2, -1);
+    return g * cos + at::cat({h[1], -h[0]}, -1);
+}
+
 struct Rope : torch::autograd::Function<Rope> {
     static variable_list turn(const Tensor& q_, const Tensor& k_, const Tensor& cos, const Tensor& sin, int64_t mode) {
         const Tensor q = dense_rows(q_), k = dense_rows(k_);
@@ -792,17 +809,16 @@ struct Rope : torch::autograd::Function<Rope> {
         launch_rope({{q, a, mode}, {k, b, mode}}, cos, sin);
         return {a, b};
     }
-    static variable_list forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& cos, const Tensor& sin, int64_t mode) {
+    static variable_list forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& cos, const Tensor& sin) {
         ctx->save_for_backward({cos, sin});
-        ctx->saved_data["back"] = mode == TURN ? (int64_t)TURN_BACK : (int64_t)TURN;
-        return turn(q, k, cos, sin, mode);
+        return turn(q, k, cos, sin, TURN);
     }
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
         const variable_list s = ctx->get_saved_variables();
         c10::OptionalDeviceGuard guard(s[0].device());
-        const int64_t back = ctx->saved_data["back"].toInt();   // each turn is the other's gradient
-        const variable_list g = at::GradMode::is_enabled() ? Rope::apply(grads[0], grads[1], s[0], s[1], back) : turn(grads[0], grads[1], s[0], s[1], back);
-        return {g[0], g[1], Tensor(), Tensor(), Tensor()};
+        if (written_out(grads)) return {turned_back(grads[0], s[0], s[1]), turned_back(grads[1], s[0], s[1]), Tensor(), Tensor()};
+        const variable_list g = turn(grads[0], grads[1], s[0], s[1], TURN_BACK);
+        return {g[0], g[1], Tensor(), Tensor()};
     }
 };
 
@@ -832,11 +848,9 @@ struct QkvRope : torch::autograd::Function<QkvRope> {
         if (!first) return variable_list(4);
         c10::OptionalDeviceGuard guard(s[0].device());
         const int64_t B = first->size(0), heads = first->size(1), S = first->size(2), D = first->size(3);
-        if (at::GradMode::is_enabled()) {
-            auto part = [&](int i) { return grads[i].defined() ? grads[i] : at::zeros_like(*first); };
-            const variable_list qk = Rope::apply(part(0), part(1), s[0], s[1], (int64_t)TURN_BACK);
-            return {at::stack({qk[0].transpose(1, 2), qk[1].transpose(1, 2), part(2).transpose(1, 2)}, 2).view({B, S, 3 * heads * D}), Tensor(), Tensor(),
-                    Tensor()};
+        if (written_out(grads)) {
+            auto part = [&](int i) { return (!grads[i].defined() ? at::zeros_like(*first) : i < 2 ? turned_back(grads[i], s[0], s[1]) : grads[i]).transpose(1, 2); };
+            return {at::stack({part(0), part(1), part(2)}, 2).reshape({B, S, 3 * heads * D}), Tensor(), Tensor(), Tensor()};
         }
         // zeros where a part took no part in the loss
         Tensor out = given == 3 ? at::empty({B, S, 3, heads, D}, first->options()) : at::zeros({B, S, 3, heads, D}, first->options());
@@ -868,7 +882,7 @@ struct Linear : torch::autograd::Function<Linear> {
         const Tensor &x = s[0], &w = s[1], &rounded = s[2];
         c10::OptionalDeviceGuard guard(x.device());
         const int64_t N = w.size(0), K = w.size(1), T = x.numel() / K;
-        if (at::GradMode::is_enabled()) {   // to be differentiated itself
+        if (written_out(grads)) {
             const Tensor g = grads[0].reshape({T, N}), wide = g.to(at::kFloat);
             return {at::matmul(g, w.to(x.scalar_type())).view(x.sizes()), at::matmul(wide.t().contiguous(), x.reshape({T, K}).to(at::kFloat))};
         }
@@ -915,7 +929,7 @@ struct Attention : torch::autograd::Function<Attention> {
         c10::OptionalDeviceGuard guard(q.device());
         const bool causal = ctx->saved_data["causal"].toBool();
         const int64_t B = q.size(0), heads = q.size(1), S = q.size(2), D = q.size(3);
-        if (at::GradMode::is_enabled()) {   // a gradient that is itself to be differentiated: written out, in fp32
+        if (written_out(grads)) {   // in fp32
             const double scale = 1.0 / std::sqrt((double)D);
             const Tensor qf = q.to(at::kFloat), kf = k.to(at::kFloat), vf = v.to(at::kFloat), g = grads[0].to(at::kFloat);
             Tensor score = at::matmul(qf, kf.transpose(2, 3).contiguous()) * scale;
@@ -961,12 +975,13 @@ struct CrossEntropy : torch::autograd::Function<CrossEntropy> {
         const variable_list s = ctx->get_saved_variables();
         c10::OptionalDeviceGuard guard(s[0].device());
         const int64_t N = s[0].size(0), V = s[0].size(1);
-        const Tensor g = like_f32(grads[0]);
-        if (at::GradMode::is_enabled()) {
+        if (written_out(grads)) {
+            const Tensor g = grads[0].to(at::kFloat);
             const Tensor t = s[1].unsqueeze(1), hit = at::arange(V, s[1].options()).unsqueeze(0).eq(t);
             const Tensor p = at::softmax(s[0].to(at::kFloat), 1) - hit.to(at::kFloat);
             return {at::where(t.eq(kIgnoreIndex), at::zeros({}, p.options()), p * (g * s[2].select(0, 3 * N))).to(s[0].scalar_type()), Tensor()};
         }
+        const Tensor g = like_f32(grads[0]);
         Tensor d = at::empty_like(s[0]);
         const float* row = ptr_as<float>(s[2]);
         check(mts_cross_entropy_bwd(ptr(s[0]), ptr_as<int64_t>(s[1]), N, V, kIgnoreIndex, dtype_code(s[0]), row, row + N, ptr_as<float>(g),
@@ -1020,7 +1035,7 @@ PYBIND11_MODULE(_host, m) {
     m.def("rope_supported", &rope_supported);
     m.def("rope", [](const Tensor& q, const Tensor& k, const Tensor& cos, const Tensor& sin) {
         c10::OptionalDeviceGuard guard(q.device());
-        const variable_list v = Rope::apply(q, k, cos, sin, (int64_t)TURN);
+        const variable_list v = Rope::apply(q, k, cos, sin);
         return std::make_tuple(v[0], v[1]);
     });
     m.def("qkv_rope_supported", &qkv_rope_supported);

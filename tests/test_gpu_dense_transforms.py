@@ -125,3 +125,45 @@ def test_overridden_operator_is_called():
     torch.testing.assert_close(ops.add_rmsnorm(x, r, w, 1e-5)[1], 2 * STOCK.rmsnorm(x + r, w, 1e-5), **TOL)
     (qkv,), _ = _operands("qkv_rope")
     assert ops.qkv_rope(qkv, torch.ones(5, 8, device="cuda"), torch.ones(5, 8, device="cuda"), 3) is None
+
+
+def _more_operands(name):
+    """The operators that take 16-bit operands only, and the projection of many experts."""
+    if name in NAMES:
+        return _operands(name)
+    g = torch.Generator().manual_seed(6)
+    r = lambda *shape: torch.randn(*shape, generator=g).cuda()
+    if name == "attention":
+        return tuple(r(2, 3, 9, 64).bfloat16() for _ in range(3)), lambda ops, q, k, v: ops.attention(q, k, v, is_causal=True, dropout_p=0.0)
+    if name == "linear":
+        def project(ops, x, w):
+            with torch.autocast("cuda", dtype=torch.bfloat16):
+                y = ops.linear(x, w) if hasattr(ops, "linear") else None
+                return torch.nn.functional.linear(x, w) if y is None else y
+        return (r(2, 520, 64).bfloat16(), r(72, 64) / 8), project
+    return (r(37, 64), r(24, 64) / 8), lambda ops, x, w: ops.router_logits(x, w)
+
+
+# relative to the largest value: fp32 sums of at most 64 terms, or one rounding to bf16 of results whose sums carry others
+SCALED_TOL = {torch.float32: 2e-5, torch.bfloat16: 2.0 ** -6}
+
+
+@pytest.mark.parametrize("name", [*NAMES, "attention", "linear", "router_logits"])
+@pytest.mark.parametrize("how", ["is_grads_batched", "vmap"])
+def test_batched_gradients(name, how):
+    """Several gradients of one result in a call, as a vectorised jacobian takes them, against one call for each."""
+    print(name, how, flush=True)
+    operands, f = _more_operands(name)
+    leaves = [t.clone().requires_grad_(True) for t in operands]
+    out = f(hip_backend(), *leaves)
+    seeds = torch.randn(3, *out.shape, generator=torch.Generator().manual_seed(7)).to(out.dtype).cuda()
+    if how == "vmap":
+        got = torch.func.vmap(lambda s: torch.autograd.grad(out, leaves, s, retain_graph=True))(seeds)
+    else:
+        got = torch.autograd.grad(out, leaves, seeds, retain_graph=True, is_grads_batched=True)
+    each = [torch.autograd.grad(out, leaves, s, retain_graph=True) for s in seeds]
+    for i, (a, leaf) in enumerate(zip(got, leaves)):
+        want = torch.stack([e[i] for e in each])
+        assert a.dtype == leaf.dtype and a.shape == want.shape
+        err, scale = float((a.float() - want.float()).abs().max()), float(want.float().abs().max())
+        assert err <= SCALED_TOL[leaf.dtype] * scale, (i, err, scale)
