@@ -696,7 +696,7 @@ struct RouterLogits : torch::autograd::Function<RouterLogits> {
             const Tensor wide = grads[0].to(at::kFloat);
             return {wide.matmul(s[1]).to(s[0].scalar_type()), wide.t().matmul(s[0].to(at::kFloat))};
         }
-        const Tensor g = like_f32(grads[0]);
+        const Tensor g = dense_router_operand(grads[0].to(at::kFloat), s[1].size(0));
         Tensor dx = at::empty_like(s[0]), dw = at::empty_like(s[1]);
         router_projection_backward(g, s[0], s[1], dx, dw);
         return {dx, dw};

@@ -48,6 +48,22 @@ def test_operands_that_start_anywhere():
         assert torch.equal(a, b)
 
 
+def test_gradient_that_starts_anywhere():
+    """Logits of two batches joined: the second part's gradient is a dense slice of the joined one."""
+    print("wide projection, misaligned gradient", flush=True)
+    ops = hip_backend()
+    x, w = torch.randn(5, 64, device="cuda", requires_grad=True), torch.randn(18, 64, device="cuda", requires_grad=True)
+    seed = torch.randn(10, 18, device="cuda")
+    for rows in (3, 5):   # 54 and 90 elements in front of the slice
+        joined = torch.cat((ops.router_logits(x[:rows], w), ops.router_logits(x, w)))
+        got = torch.autograd.grad(joined, (x, w), seed[:rows + 5])
+        first, second = seed[:rows].double(), seed[rows:rows + 5].double()
+        dx = second @ w.double()
+        dx[:rows] += first @ w.double()
+        assert_close_scaled(got[0], dx, 1e-5, "dx")
+        assert_close_scaled(got[1], first.T @ x[:rows].double() + second.T @ x.double(), 1e-5, "dW")
+
+
 @pytest.mark.parametrize("T,H,E,I,K,capacity", [(500, 128, 24, 64, 2, None), (1000, 256, 64, 128, 4, None), (300, 64, 130, 64, 8, None), (1000, 128, 32, 64, 4, 60)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_layer_node_of_many_experts(T, H, E, I, K, capacity, dtype):
