@@ -92,6 +92,10 @@ bool written_out(const variable_list& grads) {
         if (g.defined() && !is_plain(g)) return true;
     return false;
 }
+template <typename... Ts>
+bool on_one_gpu(const Tensor& first, const Ts&... others) {
+    return first.is_cuda() && ((others.device() == first.device()) && ...);
+}
 int64_t round4(int64_t n) { return (n + 3) / 4 * 4; }
 
 // ---- contracts ---------------------------------------------------------------------------------------------------------------
@@ -103,7 +107,7 @@ constexpr int64_t k2GiB = 1LL << 31;
 const char* expert_violation(const Tensor& x, const Tensor& w1, const Tensor& w2) {
     if (x.dim() != 2 || w1.dim() != 3 || w2.dim() != 3) return "x is [T,H], gate_up_proj [E,2I,H] and down_proj [E,H,I]";
     const int64_t T = x.size(0), H = x.size(1), E = w1.size(0), two_i = w1.size(1), I = two_i / 2;
-    if (!x.is_cuda() || !w1.is_cuda() || !w2.is_cuda() || x.device() != w1.device() || x.device() != w2.device()) return "all tensors on one GPU";
+    if (!on_one_gpu(x, w1, w2)) return "all tensors on one GPU";
     const auto t = x.scalar_type();
     if (!is_activation_type(t)) return "activations are bf16, fp16 or fp32";
     if (T <= 0) return "at least one token";
@@ -124,8 +128,7 @@ const char* expert_violation(const Tensor& x, const Tensor& w1, const Tensor& w2
 const char* routing_violation(const Tensor& x, const Tensor& w1, const Tensor& index, const Tensor& weights) {
     if (index.dim() != 2) return "top_k_index is [T,K]";
     const int64_t K = index.size(1);
-    if (!index.is_cuda() || !weights.is_cuda() || index.device() != x.device() || weights.device() != x.device())
-        return "routing tensors on the activations' GPU";
+    if (!on_one_gpu(x, index, weights)) return "routing tensors on the activations' GPU";
     if (weights.sizes() != index.sizes() || index.size(0) != x.size(0)) return "top_k_index and top_k_weights are [T,K]";
     if (K <= 0 || K > std::min<int64_t>(w1.size(0), 32768)) return "1 <= K <= number of experts (at most 32768)";
     if (x.size(0) * K >= k2GiB) return "fewer than 2^31 routes";
@@ -148,7 +151,7 @@ bool needs_padding(const Tensor& x, const Tensor& w1) {
 // Up to 16 experts the projection kernels keep W_r in LDS; more take the kernels on the fp32 matrix instruction.
 constexpr int64_t kFewExperts = 16;
 bool router_logits_supported(const Tensor& x, const Tensor& w) {
-    return all_plain(x, w) && x.is_cuda() && w.is_cuda() && x.dim() == 2 && w.dim() == 2 && is_activation_type(x.scalar_type()) &&
+    return all_plain(x, w) && on_one_gpu(x, w) && x.dim() == 2 && w.dim() == 2 && is_activation_type(x.scalar_type()) &&
            w.scalar_type() == at::kFloat && x.size(0) > 0 && x.size(1) == w.size(1) &&
            (w.size(0) <= kFewExperts ? x.size(1) % 4 == 0 && x.size(1) <= 4096 && w.size(0) * w.size(1) * 4 <= 128 * 1024
                                      : mts_router_wide_supported(x.size(1), w.size(0)));
@@ -709,10 +712,10 @@ struct RouterLogits : torch::autograd::Function<RouterLogits> {
 // written_out() says so.
 
 bool rmsnorm_supported(const Tensor& x, const Tensor& w, const MaybeTensor& residual) {
-    if (!(all_plain(x, w) && (!residual || is_plain(*residual)) && x.is_cuda() && w.is_cuda() && is_activation_type(x.scalar_type()) && w.scalar_type() == at::kFloat && w.dim() == 1 && x.dim() >= 1 &&
-          x.size(-1) == w.size(0) && x.numel() > 0 && x.numel() / x.size(-1) < MTS_MAX_NORM_ROWS && mts_rmsnorm_supported(x.size(-1))))
+    if (!(all_plain(x, w) && (!residual || is_plain(*residual)) && on_one_gpu(x, w) && is_activation_type(x.scalar_type()) &&
+          w.scalar_type() == at::kFloat && w.dim() == 1 && x.dim() >= 1 && x.size(-1) == w.size(0) && x.numel() > 0 && x.numel() / x.size(-1) < MTS_MAX_NORM_ROWS && mts_rmsnorm_supported(x.size(-1))))
         return false;
-    return !residual || (residual->is_cuda() && residual->scalar_type() == x.scalar_type() && residual->sizes() == x.sizes());
+    return !residual || (on_one_gpu(x, *residual) && residual->scalar_type() == x.scalar_type() && residual->sizes() == x.sizes());
 }
 
 // y, or (x + residual, y) with a residual
@@ -761,11 +764,11 @@ struct RMSNorm : torch::autograd::Function<RMSNorm> {
 enum RopeMode : int64_t { TURN = 0, TURN_BACK = 1, COPY = 2 };
 
 bool rope_table_fits(const Tensor& t, const Tensor& like, int64_t S, int64_t D) {
-    return t.is_cuda() && t.scalar_type() == like.scalar_type() && t.dim() == 2 && t.size(0) == S && t.size(1) == D && t.is_contiguous() && !t.requires_grad();
+    return on_one_gpu(like, t) && t.scalar_type() == like.scalar_type() && t.dim() == 2 && t.size(0) == S && t.size(1) == D && t.is_contiguous() && !t.requires_grad();
 }
 bool rope_supported(const Tensor& q, const Tensor& k, const Tensor& cos, const Tensor& sin) {
-    if (!(all_plain(q, k, cos, sin) && q.is_cuda() && k.is_cuda() && q.dim() == 4 && q.sizes() == k.sizes() && q.scalar_type() == k.scalar_type() && is_activation_type(q.scalar_type()) &&
-          q.numel() > 0))
+    if (!(all_plain(q, k, cos, sin) && on_one_gpu(q, k) && q.dim() == 4 && q.sizes() == k.sizes() && q.scalar_type() == k.scalar_type() &&
+          is_activation_type(q.scalar_type()) && q.numel() > 0))
         return false;
     const int64_t S = q.size(2), D = q.size(3);
     return D % 2 == 0 && q.numel() / 2 < MTS_MAX_ROPE_PAIRS && rope_table_fits(cos, q, S, D) && rope_table_fits(sin, q, S, D);
@@ -864,7 +867,7 @@ struct QkvRope : torch::autograd::Function<QkvRope> {
 
 // A projection under autocast: the product is the library's, the gradient of its fp32 weight is summed in fp32 here.
 bool linear_supported(const Tensor& x, const Tensor& w) {
-    if (!(at::GradMode::is_enabled() && w.requires_grad() && all_plain(x, w) && x.is_cuda() && w.device() == x.device() && x.dim() >= 2 && w.dim() == 2 &&
+    if (!(at::GradMode::is_enabled() && w.requires_grad() && all_plain(x, w) && on_one_gpu(x, w) && x.dim() >= 2 && w.dim() == 2 &&
           w.scalar_type() == at::kFloat && (x.scalar_type() == at::kBFloat16 || x.scalar_type() == at::kHalf) && x.size(-1) == w.size(1) && x.numel() > 0))
         return false;
     if (!at::autocast::is_autocast_enabled(at::kCUDA) || at::autocast::get_autocast_dtype(at::kCUDA) != x.scalar_type()) return false;
@@ -903,7 +906,7 @@ bool heads_fit(const Tensor& t) {   // as the kernels read them
     return t.stride(3) == 1 && t.stride(0) % 8 == 0 && t.stride(1) % 8 == 0 && t.stride(2) % 8 == 0 && aligned16(t);
 }
 bool attention_supported(const Tensor& q, const Tensor& k, const Tensor& v) {
-    if (!(all_plain(q, k, v) && q.is_cuda() && k.device() == q.device() && v.device() == q.device() && q.dim() == 4 && k.sizes() == q.sizes() &&
+    if (!(all_plain(q, k, v) && on_one_gpu(q, k, v) && q.dim() == 4 && k.sizes() == q.sizes() &&
           v.sizes() == q.sizes() && (q.scalar_type() == at::kBFloat16 || q.scalar_type() == at::kHalf) && k.scalar_type() == q.scalar_type() &&
           v.scalar_type() == q.scalar_type() && mts_attention_supported(q.size(0), q.size(1), q.size(2), q.size(3))))
         return false;
@@ -952,8 +955,8 @@ struct Attention : torch::autograd::Function<Attention> {
 constexpr int64_t kIgnoreIndex = -100;   // torch's default
 
 bool cross_entropy_supported(const Tensor& logits, const Tensor& targets) {
-    return all_plain(logits, targets) && logits.is_cuda() && targets.is_cuda() && logits.dim() == 2 && targets.dim() == 1 && is_activation_type(logits.scalar_type()) &&
-           targets.scalar_type() == at::kLong && logits.size(0) == targets.size(0) && logits.size(0) > 0 && logits.size(0) < MTS_MAX_LOSS_ROWS && logits.size(1) > 0 &&
+    return all_plain(logits, targets) && on_one_gpu(logits, targets) && logits.dim() == 2 && targets.dim() == 1 &&
+           is_activation_type(logits.scalar_type()) && targets.scalar_type() == at::kLong && logits.size(0) == targets.size(0) && logits.size(0) > 0 && logits.size(0) < MTS_MAX_LOSS_ROWS && logits.size(1) > 0 &&
            logits.size(1) < k2GiB;
 }
 
