@@ -107,9 +107,10 @@ class HipOpsBackend(DenseTorchOps):
 
     def moe_layer(self, x, router_weight, gate_up_proj, down_proj, top_k, *, normalize, capacity=None):
         """Extension: router projection, post-process, routing metadata and the experts as one autograd
-        node (see ``kernels/hip/moe_layer.py``).  Returns None when the contract is not supported; the
-        caller then composes the layer from ``router_postprocess`` and ``fused_moe``."""
-        if not self.offers_moe_layer or moe_layer_violation(x, router_weight, gate_up_proj, down_proj, top_k) is not None:
+        node (see ``kernels/hip/moe_layer.py``).  Returns None when the contract is not supported or one of the
+        operators that it stands for is overridden; the caller then composes the layer from them."""
+        operators = _OF_LAYER if capacity is None else _OF_LIMITED_LAYER
+        if not self.offers_moe_layer or not all(map(self._is_own, operators)) or moe_layer_violation(x, router_weight, gate_up_proj, down_proj, top_k) is not None:
             return None
         return run_moe_layer(x, router_weight, gate_up_proj, down_proj, top_k, normalize, capacity)
 
@@ -122,7 +123,9 @@ class HipOpsBackend(DenseTorchOps):
         return router_logits(hidden_states, weight)
 
 
-_OWN = {name: getattr(HipOpsBackend, name) for name in ("rmsnorm", "rope")}
+_OF_LAYER = ("router_logits", "router_postprocess", "fused_moe")
+_OF_LIMITED_LAYER = (*_OF_LAYER, "capacity_mask")
+_OWN = {name: getattr(HipOpsBackend, name) for name in ("rmsnorm", "rope", *_OF_LIMITED_LAYER)}
 
 __all__ = [
     "HipOpsBackend",

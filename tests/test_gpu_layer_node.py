@@ -270,6 +270,34 @@ def test_block_uses_the_layer_node_and_falls_back_when_it_must():
         torch.testing.assert_close(one.router_metrics[key].float(), three.router_metrics[key].float(), rtol=2e-5, atol=2e-6)
 
 
+@pytest.mark.parametrize("name,experts,factor", [("router_logits", 24, None), ("router_postprocess", 8, None), ("fused_moe", 24, None), ("fused_moe", 8, 1.0),
+                                                 ("capacity_mask", 8, 1.0)])
+@pytest.mark.parametrize("how", ["subclass", "instance"])
+def test_overridden_operator_is_called(name, experts, factor, how):
+    """A backend whose operator is not the class's own gets the layer composed, with that operator called."""
+    print(f"overridden {name}, {how}, {experts} experts, capacity factor {factor}", flush=True)
+    from minitrain_amd.kernels.hip import HipOpsBackend
+    from minitrain_amd.model.blocks import MoEFeedForward
+    from minitrain_amd.model.config import ModelConfig
+
+    calls = []
+    own = getattr(HipOpsBackend, name)
+
+    def counted(self, *args, **kwargs):
+        calls.append(1)
+        return own(self, *args, **kwargs)
+
+    if how == "subclass":
+        ops = type("Counted", (HipOpsBackend,), {name: counted})()
+    else:
+        ops = HipOpsBackend()
+        setattr(ops, name, lambda *args, **kwargs: counted(ops, *args, **kwargs))
+    cfg = ModelConfig(hidden_size=64, n_heads=1, intermediate_size=64, num_experts=experts, experts_per_token=2, expert_capacity_factor=factor)
+    block = MoEFeedForward(cfg).cuda()
+    block(torch.randn(40, 64, device="cuda"), ops)
+    assert calls == [1]
+
+
 def test_layer_step_replayed_from_a_graph():
     """Forward and backward of the layer node captured into one graph and replayed, with eager steps and
     synchronisations between the replays: outputs and all four gradients equal the eager step's, bit for bit.  No
