@@ -981,8 +981,10 @@ struct CrossEntropy : torch::autograd::Function<CrossEntropy> {
         if (written_out(grads)) {
             const Tensor g = grads[0].to(at::kFloat);
             const Tensor t = s[1].unsqueeze(1), hit = at::arange(V, s[1].options()).unsqueeze(0).eq(t);
-            const Tensor p = at::softmax(s[0].to(at::kFloat), 1) - hit.to(at::kFloat);
-            return {at::where(t.eq(kIgnoreIndex), at::zeros({}, p.options()), p * (g * s[2].select(0, 3 * N))).to(s[0].scalar_type()), Tensor()};
+            const Tensor p = at::softmax(s[0].to(at::kFloat), 1) - hit.to(at::kFloat), none = at::zeros({}, p.options());
+            const Tensor ignored = t.eq(kIgnoreIndex), outside = t.lt(0).logical_or(t.ge(V)).logical_and(ignored.logical_not());
+            const Tensor scale = g * s[2].select(0, 3 * N) + at::where(outside, at::full({}, NAN, p.options()), none);
+            return {at::where(ignored, none, p * scale).to(s[0].scalar_type()), Tensor()};
         }
         const Tensor g = like_f32(grads[0]);
         Tensor d = at::empty_like(s[0]);

@@ -457,7 +457,7 @@ __global__ __launch_bounds__(kCeMeanThreads) void cross_entropy_mean_kernel(cons
     }
 }
 
-// d_logits = (softmax - onehot) * g / count, zero where the target is ignored
+// d_logits = (softmax - onehot) * g / count, zero where the target is ignored, NaN as the loss where it is outside the vocabulary
 template <typename ET>
 __global__ __launch_bounds__(kCeThreads) void cross_entropy_bwd_kernel(const ET* __restrict__ logits, const int64_t* __restrict__ targets, int V,
                                                                        int64_t ignore, const float* __restrict__ row_max,
@@ -470,7 +470,7 @@ __global__ __launch_bounds__(kCeThreads) void cross_entropy_bwd_kernel(const ET*
     const ET* p = logits + row * V;
     ET* d = d_logits + row * V;
     const CeRow<ET> r(p, V);
-    const float scale = target == ignore ? 0.f : *g * *inv_count;
+    const float scale = target == ignore ? 0.f : ((target < 0 || target >= V) ? NAN : *g * *inv_count);
     // maximum and logarithm of the sum apart: their sum would carry the rounding of a large maximum into every probability
     const float hi = row_max[row], base = row_log_sum[row] * kLog2e;
     const int t = (int)target;

@@ -125,6 +125,19 @@ def test_cross_entropy_without_valid_targets_and_outside_the_vocabulary():
     assert torch.isnan(ops.cross_entropy(logits, torch.tensor([0, 9, 1], device="cuda")))
 
 
+@pytest.mark.parametrize("create_graph", [False, True])
+def test_gradient_of_targets_outside_the_vocabulary(create_graph):
+    """NaN in the rows whose loss is NaN (2^32 + 1 has the low bits of a target inside), what they were in the others."""
+    print(f"targets outside the vocabulary, create_graph={create_graph}", flush=True)
+    logits = torch.randn(5, 9, device="cuda", requires_grad=True)
+    targets = torch.tensor([0, 9, -100, 2 ** 32 + 1, -1], device="cuda")
+    d, = torch.autograd.grad(hip_backend().cross_entropy(logits, targets), logits, create_graph=create_graph)
+    assert d[[1, 3, 4]].isnan().all() and not d[2].any()
+    want = torch.softmax(logits[0].detach(), 0)
+    want[0] -= 1
+    _close(d[0], want / 4, 1e-5, "row inside", scale=0.25)
+
+
 def test_results_may_be_changed_in_place():
     """The loss, rotated queries and keys and the attention's result are tensors of their own, as the stock operators' are."""
     print("results changed in place", flush=True)
