@@ -877,17 +877,19 @@ bool linear_supported(const Tensor& x, const Tensor& w) {
 struct Linear : torch::autograd::Function<Linear> {
     static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w) {
         const Tensor rounded = w.to(x.scalar_type());
-        ctx->save_for_backward({x, w, rounded});
+        ctx->save_for_backward({x, rounded});
+        ctx->saved_data["weight"] = w;   // not kept as it is now: the caller may change it before the backward pass, as under stock autocast
         return at::linear(x, rounded);
     }
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
         const variable_list s = ctx->get_saved_variables();
-        const Tensor &x = s[0], &w = s[1], &rounded = s[2];
+        const Tensor &x = s[0], &rounded = s[1];
         c10::OptionalDeviceGuard guard(x.device());
-        const int64_t N = w.size(0), K = w.size(1), T = x.numel() / K;
+        const int64_t N = rounded.size(0), K = rounded.size(1), T = x.numel() / K;
         if (written_out(grads)) {
             const Tensor g = grads[0].reshape({T, N}), wide = g.to(at::kFloat);
-            return {at::matmul(g, w.to(x.scalar_type())).view(x.sizes()), at::matmul(wide.t().contiguous(), x.reshape({T, K}).to(at::kFloat))};
+            const Tensor now = ctx->saved_data["weight"].toTensor().to(x.scalar_type());   // for its derivative; the value is that of the forward pass
+            return {at::matmul(g, rounded + (now - now.detach())).view(x.sizes()), at::matmul(wide.t().contiguous(), x.reshape({T, K}).to(at::kFloat))};
         }
         const Tensor g = dense16(grads[0].reshape({T, N})), in = dense16(x.reshape({T, K}));
         Tensor dx, dw;

@@ -56,6 +56,43 @@ def test_layouts(layout):
         assert got.shape == want.shape and err <= tol * scale, (what, err, scale)
 
 
+@pytest.mark.parametrize("create_graph", [False, True])
+def test_weight_changed_before_the_backward_pass(create_graph):
+    """As under stock autocast, which keeps the rounded copy: the gradients are those of the weight of the forward pass."""
+    print(f"linear, weight changed in place, create_graph={create_graph}", flush=True)
+    g = torch.Generator().manual_seed(4)
+    x, w = torch.randn(2, 600, 64, generator=g).bfloat16().cuda().requires_grad_(True), torch.randn(72, 64, generator=g).cuda().requires_grad_(True)
+    grad = torch.randn(2, 600, 72, generator=g).bfloat16().cuda()
+    got = []
+    for f in (lambda: hip_backend().linear(x, w), lambda: torch.nn.functional.linear(x, w)):
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            y = f()
+        with torch.no_grad():
+            w.mul_(2)
+        got.append(torch.autograd.grad(y, (x, w), grad, create_graph=create_graph))
+        with torch.no_grad():
+            w.div_(2)
+    for (a, b), tol in zip(zip(*got), (1e-6, ULP[torch.bfloat16])):   # the same product; the stock gradient of w is rounded to bf16
+        a, b = a.detach(), b.detach()
+        assert a.dtype == b.dtype and float((a.float() - b.float()).abs().max()) <= tol * float(b.float().abs().max())
+
+
+def test_gradient_of_a_gradient():
+    """Second derivatives against fp64 products of the rounded operands: a handful of bf16 roundings."""
+    print("linear, second derivative", flush=True)
+    g = torch.Generator().manual_seed(5)
+    x, w = torch.randn(1100, 64, generator=g).bfloat16().cuda().requires_grad_(True), (torch.randn(72, 64, generator=g) / 8).bfloat16().float().cuda().requires_grad_(True)
+    wide = [t.detach().double().requires_grad_(True) for t in (x, w)]
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        y = hip_backend().linear(x, w)
+    results = []
+    for out, leaves in ((y, (x, w)), (wide[0] @ wide[1].T, wide)):
+        first = torch.autograd.grad(out.float().square().sum() if out is y else out.square().sum(), leaves, create_graph=True)
+        results.append(torch.autograd.grad(sum(t.to(out.dtype if out is not y else torch.float32).square().sum() for t in first), leaves))
+    for got, want in zip(*results):
+        assert float((got.double() - want).abs().max()) <= 2.0 ** -6 * float(want.abs().max())
+
+
 def test_other_calls_stay_stock():
     x = torch.randn(2, 1024, 64, device="cuda", dtype=torch.bfloat16)
     w = torch.randn(64, 64, device="cuda", requires_grad=True)
