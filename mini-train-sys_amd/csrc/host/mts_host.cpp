@@ -210,6 +210,31 @@ void order_after(hipStream_t to, hipStream_t from) {
     TORCH_CHECK(ok, "ordering two streams failed");
 }
 
+// Side streams that work has been forked onto.  The caller's stream waits for them before what they read and write is released,
+// also where an error (a refused call, memory that runs out) leaves the function: the allocator knows the caller's stream only.
+class Forked {
+    hipStream_t main_, streams_[2] = {};
+    int n_ = 0;
+
+  public:
+    explicit Forked(hipStream_t main) : main_(main) {}
+    Forked(const Forked&) = delete;
+    void fork(hipStream_t s) {
+        if (s == main_) return;
+        if (s != streams_[0] && s != streams_[1]) streams_[n_++] = s;
+        order_after(s, main_);
+    }
+    void join() {
+        while (n_) order_after(main_, streams_[--n_]);
+    }
+    ~Forked() {
+        try {
+            join();
+        } catch (...) {   // on top of the error that is under way
+        }
+    }
+};
+
 // ---- experts: forward and backward ---------------------------------------------------------------------------------------------
 
 struct Routing {
@@ -402,26 +427,27 @@ ExpertGrads experts_backward(const Saved& s, Tensor dO, const Needs& need, const
     const bool overlap = opt.on(OVERLAP);
     auto side = [&](int i) { return overlap ? side_stream(device, i) : main; };
     ExpertGrads g;
+    Tensor w1_bwd, w2_bwd, d_pre_act, weighted_act, ds_part, ws1, ws2, schedule, dx_expanded;
+    Forked forked(main);   // behind everything that the side streams touch: joined first
 
     // The ring kernels (16-bit types, widths of whole 64-wide k-tiles or of at least 256) and the fp32 kernels read the
     // weights in their stored layout; other contracts get transposed copies, W1's made on a side stream next to the dO*W2 GEMM.
     const int layout = stored_layout(act, H, I);
     hipStream_t side0 = main;
-    Tensor w1_bwd, w2_bwd;
     if (need.x) {
         if (layout) w1_bwd = s.staged1.defined() ? s.staged1 : stage(s.w1, false, dtype, main);
         else {
             side0 = side(0);
-            order_after(side0, main);
+            forked.fork(side0);
             w1_bwd = stage(s.w1, true, dtype, side0);
         }
     }
     w2_bwd = layout && s.staged2.defined() ? s.staged2 : stage(s.w2, !layout, dtype, main);
 
     const bool weighted = s.post_act.defined();
-    Tensor d_pre_act = at::empty({TK, 2 * I}, s.x.options());
-    Tensor weighted_act = weighted ? s.post_act : at::empty({TK, I}, s.x.options());   // s * silu(g) * u
-    Tensor ds_part = f32({TK, mts_moe_ds_partials(I)}, s.x);
+    d_pre_act = at::empty({TK, 2 * I}, s.x.options());
+    weighted_act = weighted ? s.post_act : at::empty({TK, I}, s.x.options());   // s * silu(g) * u
+    ds_part = f32({TK, mts_moe_ds_partials(I)}, s.x);
     // When every gradient is wanted, dW1, dW2, dX and the dS reduction go out as ONE launch whose block order starts the long
     // weight-gradient tiles first; which XCD runs which of its units and dX tiles follows a table that the dO * W2 launch
     // writes on the side (uneven routing).
@@ -431,7 +457,8 @@ ExpertGrads experts_backward(const Saved& s, Tensor dO, const Needs& need, const
         const int64_t n = wanted && dtype != at::kFloat ? mts_moe_bwd_dw_workspace_bytes(which, E, H, I) : 0;
         return n > 0 && n <= opt.dw_workspace_limit ? at::empty({n}, s.x.options().dtype(at::kByte)) : Tensor();
     };
-    Tensor ws1 = dw_workspace(1, need.w1), ws2 = dw_workspace(2, need.w2), schedule;
+    ws1 = dw_workspace(1, need.w1);
+    ws2 = dw_workspace(2, need.w2);
     const int64_t ws1_bytes = ws1.defined() ? ws1.numel() : 0, ws2_bytes = ws2.defined() ? ws2.numel() : 0;
     if (joint && opt.on(JOINT_SCHEDULE) && ws1.defined() && ws2.defined() && mts_moe_bwd_schedule_bytes(E) > 0)
         schedule = i32({mts_moe_bwd_schedule_bytes(E) / 4}, s.x);
@@ -440,7 +467,6 @@ ExpertGrads experts_backward(const Saved& s, Tensor dO, const Needs& need, const
                           ptr_as<float>(ds_part), ptr_as<int32_t>(schedule), main),
           "mts_moe_bwd_dy1");
 
-    Tensor dx_expanded;
     auto combine_dx = [&]() {
         if (tail && !tail->dx_r.defined()) router_gradient(s.x, *tail, g.ds);
         g.dx = at::empty({T, H}, s.x.options());
@@ -483,8 +509,8 @@ ExpertGrads experts_backward(const Saved& s, Tensor dO, const Needs& need, const
 
     // dW2, dW1 and dX side by side: the two weight-gradient GEMMs have fewer tiles than the chip has CUs
     const hipStream_t s0 = need.w2 ? side(0) : main, s1 = need.w1 ? side(1) : main;
-    if (need.w2) order_after(s0, main);
-    if (need.w1) order_after(s1, main);
+    if (need.w2) forked.fork(s0);
+    if (need.w1) forked.fork(s1);
     // The routing-weight gradient is needed after the join only: it leads one of the side streams (when there is one) so that
     // dX follows the dO*W2 GEMM directly on the caller's stream; the router's gradient wants it on the caller's stream.
     if (need.s) {
@@ -509,10 +535,7 @@ ExpertGrads experts_backward(const Saved& s, Tensor dO, const Needs& need, const
         check(mts_moe_bwd_dx(ptr(d_pre_act), ptr(w1_bwd), layout, ptr_as<int32_t>(s.expert_start), TK, E, H, I, act, ptr(dx_expanded), main), "mts_moe_bwd_dx");
         combine_dx();
     }
-    // joined before any tensor that the side streams read is released
-    order_after(main, s0);
-    order_after(main, s1);
-    if (need.x && !layout) order_after(main, side0);
+    forked.join();
     return g;
 }
 

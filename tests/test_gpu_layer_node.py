@@ -340,3 +340,22 @@ def test_layer_step_replayed_from_a_graph():
         assert torch.equal(got_out, want_out), replay
         for a, b in zip(got_grads, want_grads):
             assert torch.equal(a, b), replay
+
+
+def test_side_streams_are_joined_where_the_backward_pass_raises():
+    """A gradient that the kernels refuse (dense, off a 16-byte boundary), at widths whose backward pass has forked a side
+    stream by then: a capture ends only if that stream has been joined."""
+    print("side streams after an error", flush=True)
+    ops = hip_backend()
+    x, w1, w2 = (torch.randn(*shape, device="cuda", dtype=torch.bfloat16, requires_grad=True) for shape in ((20, 72), (4, 80, 72), (4, 72, 40)))
+    index = torch.randint(0, 4, (20, 2), device="cuda", dtype=torch.int32)
+    weights = torch.rand(20, 2, device="cuda", dtype=torch.bfloat16)
+    seed = torch.empty(20 * 72 + 8, device="cuda", dtype=torch.bfloat16)[1:1 + 20 * 72].view(20, 72)
+    ops.fused_moe(x, w1, w2, index, weights).sum().backward()   # nothing is set up inside the capture
+    torch.cuda.synchronize()
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.graph(torch.cuda.CUDAGraph(), stream=stream):
+        out = ops.fused_moe(x, w1, w2, index, weights)
+        with pytest.raises(RuntimeError, match="aligned"):
+            torch.autograd.grad(out, (x, w1, w2), seed)
