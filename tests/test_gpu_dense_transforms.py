@@ -3,6 +3,7 @@ transforms, forward mode, dispatch modes and gradients of gradients give what th
 
 import pytest
 import torch
+from torch.utils._python_dispatch import TorchDispatchMode
 
 from minitrain_amd.kernels.dense_ops import DenseTorchOps
 from minitrain_amd.kernels.hip import HipOpsBackend, dense
@@ -80,8 +81,6 @@ def test_function_transforms(name):
 
 @pytest.mark.parametrize("name", NAMES)
 def test_modes_see_the_stock_operators(name):
-    from torch.utils._python_dispatch import TorchDispatchMode
-
     print(name, flush=True)
     operands, f = _operands(name)
 
@@ -167,3 +166,72 @@ def test_batched_gradients(name, how):
         assert a.dtype == leaf.dtype and a.shape == want.shape
         err, scale = float((a.float() - want.float()).abs().max()), float(want.float().abs().max())
         assert err <= SCALED_TOL[leaf.dtype] * scale, (i, err, scale)
+
+
+class Through(TorchDispatchMode):
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        return func(*args, **(kwargs or {}))
+
+
+def _predicates():
+    from minitrain_amd.kernels.hip import is_router_logits_supported
+    from minitrain_amd.kernels.hip.moe_layer import moe_layer_violation
+
+    def linear(x, w):
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            return dense.is_linear_supported(x, w)
+
+    def layer(w_r, *operands):
+        return moe_layer_violation(operands[0], w_r, *operands[1:], 2) is None
+
+    r = lambda *shape: torch.randn(*shape, device="cuda")
+    yield "attention", dense.is_attention_supported, [r(2, 3, 9, 64).bfloat16() for _ in range(3)]
+    yield "linear", linear, [r(2, 520, 64).bfloat16(), r(72, 64).requires_grad_(True)]
+    yield "router_logits", is_router_logits_supported, [r(37, 64), r(24, 64)]
+    yield "moe_layer", layer, [r(4, 64), r(37, 64), r(4, 128, 64), r(4, 64, 64)]
+
+
+@pytest.mark.parametrize("which", range(4))
+def test_kernels_stay_out_where_somebody_looks(which):
+    """The operators that take 16-bit operands only and the layer as one node: not under a transform, a mode or with duals."""
+    import torch.autograd.forward_ad as fwd
+
+    name, takes, operands = list(_predicates())[which]
+    print(name, flush=True)
+    assert takes(*operands)
+    answers = []
+
+    def look(first, *others):
+        answers.append(takes(first, *others))
+        return first.sum()
+
+    first, others = operands[0], operands[1:]
+    torch.func.grad(look)(first, *others)
+    torch.func.jvp(lambda x: look(x, *others), (first,), (torch.ones_like(first),))
+    torch.func.vmap(lambda x: look(x, *others))(torch.stack([first, first]))
+    with Through():
+        look(*operands)
+    with torch.device("cuda"):
+        look(*operands)
+    with fwd.dual_level():
+        look(fwd.make_dual(first, torch.ones_like(first)), *others)
+    assert answers == [False] * 6
+
+
+def test_moe_operators_refuse_transforms():
+    """The two MoE operators have no stock form: they raise under a transform and work under a mode."""
+    print("MoE operators under transforms", flush=True)
+    ops = hip_backend()
+    r = lambda *shape: torch.randn(*shape, device="cuda")
+    x, w1, w2, logits = r(37, 64), r(4, 128, 64), r(4, 64, 64), r(37, 4)
+    route = ops.router_postprocess(logits, 2, normalize=True)
+    experts = lambda x: ops.fused_moe(x, w1, w2, route.expert_indices, route.expert_weights)
+    weights = lambda l: ops.router_postprocess(l, 2, normalize=True).expert_weights
+    for f, operand in ((experts, x), (weights, logits)):
+        for transformed in (lambda: torch.func.grad(lambda t: f(t).sum())(operand), lambda: torch.func.vmap(f)(operand.expand(2, *operand.shape)),
+                            lambda: torch.func.jvp(f, (operand,), (torch.ones_like(operand),))):
+            with pytest.raises(RuntimeError):
+                transformed()
+        plain = f(operand)
+        with Through():
+            assert torch.equal(f(operand), plain)

@@ -244,8 +244,8 @@ def test_layer_node_partial_gradients():
 
 
 def test_block_uses_the_layer_node_and_falls_back_when_it_must():
-    """MoEFeedForward takes the one-node path when the backend offers it; with a capacity limit (or a
-    backend without the hook) it composes the layer from the router module and fused_moe."""
+    """MoEFeedForward takes the one-node path when the backend offers it; otherwise it composes the layer from the router
+    module and fused_moe."""
     print("block path selection", flush=True)
     from minitrain_amd.model.blocks import MoEFeedForward
     from minitrain_amd.model.config import ModelConfig
