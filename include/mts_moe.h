@@ -255,7 +255,7 @@ int mts_moe_cast_weights_pair(const float* w1, void* w1_out, int64_t n1, const f
  * for every row r (token x_gather[r], expert e): [g;u] = W1[e] x ; a = silu(g)*u.
  * x [T,H], w1 [E,2I,H], pre_act [TK,2I], post_act [TK,I], all of act_dtype; pre_act may be NULL for
  * the 16-bit types (here and in the entry points below): it is kept for a backward pass only
- * (MTS_BF16, MTS_F16: MFMA kernels, H and I multiples of 8; MTS_F32: plain fp32 kernels).
+ * (MTS_BF16, MTS_F16: H and I multiples of 8; MTS_F32: the fp32 matrix instruction).
  * weights (flat [T*K], act_dtype) and s_scatter (row -> entry) are optional as a pair.  With
  * them post_act[r] = s_r * silu(g) * u, s_r = weights[s_scatter[r]] (fp32 product, one
  * rounding): the down projection then yields s_r * y[r], the combine is the unweighted sum
@@ -390,7 +390,7 @@ int mts_moe_bwd_dw1(const void* d_pre_act, const void* x, const int32_t* x_gathe
  * results are bit-identical to those calls.  The block index orders the work: the
  * weight-gradient tiles, which are the long ones, start first and the dX tiles fill the
  * CUs as they come free.  mts_moe_bwd_joint_supported() says whether the shapes allow it
- * (16-bit activations, 2I a multiple of 64); both weight gradients have grad_dtype.
+ * (16-bit activations, 2I a multiple of 64 or at least 256); both weight gradients have grad_dtype.
  * workspace1 / workspace2: as for mts_moe_bwd_dw1 / mts_moe_bwd_dw2 (may be NULL).
  * d_w2 == NULL (then weighted_act and workspace2 may be NULL too): dW2 is left to a call of
  * mts_moe_bwd_dw2, which does not depend on mts_moe_bwd_dy1.
@@ -480,7 +480,7 @@ int mts_rope(const MtsRopeTensor* tensors, int count, const void* cos, const voi
 /* Mean cross-entropy of logits [N,V] (any of the three types, fp32 arithmetic) over the rows
  * whose target is not ignore_index.  row_max, row_log_sum [N] and inv_count [1] f32 are kept for
  * the backward pass (row_loss [N] is scratch): d_logits = (softmax - onehot) * g_loss * inv_count in the logits' type.
- * A target outside [0, V) makes the loss NaN.                                              */
+ * A target outside [0, V) makes the loss and the gradient of its row NaN.                    */
 int mts_cross_entropy_fwd(const void* logits, const int64_t* targets, int64_t N, int V,
                           int64_t ignore_index, int dtype, float* row_max, float* row_log_sum,
                           float* row_loss, float* loss, float* inv_count, void* stream);

@@ -323,8 +323,8 @@ __global__ __launch_bounds__(kSelThreads) void capacity_select_kernel(
 }
 
 // The same selection as a compacted permutation: how many routes every expert accepts is known from the counts alone, so
-// every block knows where its expert's kept rows start.  24 576 x 2 routes over 8 experts, half of them over the limit: 39 us
-// on eight blocks (four counting passes of about 5 us over up to 12 000 keys, then scattered stores), in place of the
+// every block knows where its expert's kept rows start.  24 576 x 2 routes over 8 experts, half of them over the limit: 31 to 33 us
+// on eight blocks (four counting passes over up to 12 000 keys, then scattered stores), in place of the
 // routing metadata twice (25 us), the mask (34 us) and its application.
 __global__ __launch_bounds__(kSelThreads) void capacity_compact_kernel(
     const float* __restrict__ w, const int32_t* __restrict__ s_scatter, const int32_t* __restrict__ counts,

@@ -574,7 +574,7 @@ __device__ __forceinline__ void rows_epilogue(const RowsParams& p, f32x16 (&acc)
 // it works its way through one expert after the other, the expert's weights are
 // fetched into that L2 once and every m-tile of the range finds them there, and the
 // j-th block of an XCD computes n-tile j % n_tiles of the range's m-tile j / n_tiles,
-// so all column tiles of an m-tile (same activation rows) run side by side.  The
+// so all column tiles of an m-tile (same activation rows) run side by side.
 // Two refinements of the range mapping (measured together: 1.5 % of the layer step).  n_groups: where an
 // expert's weights take more than half an L2, the n-tiles are walked in groups - all m-tiles of the range for
 // the first group of weight columns, then for the next - so that a group's weights stay in the L2 next to the

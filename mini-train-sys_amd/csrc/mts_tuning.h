@@ -19,7 +19,7 @@ enum MtsGemmKind { MTS_K_GATEUP = 0, MTS_K_DOWN, MTS_K_DY1, MTS_K_DX, MTS_K_DW2,
 
 struct MtsTuning {
     int tile[MTS_K_COUNT];      // forced tile family per GEMM, -1: the launcher's own choice
-    int xcd_ranges;             // -1: by the size of one expert's weights
+    int xcd_ranges;             // -1: the launcher's own choice (ranges)
     int tile_order_mask;        // ORDER_* bits
     bool tail_split;
     bool mfma_router;

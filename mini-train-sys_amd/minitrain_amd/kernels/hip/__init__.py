@@ -39,9 +39,13 @@ class HipOpsBackend(DenseTorchOps):
     # The decoder's operators around its matrix products: one kernel where the stock operators are a chain of
     # elementwise and reduction kernels; what the kernels do not take (CPU tensors, other types and layouts) stays stock.
 
-    def _is_own(self, name) -> bool:
-        """Whether an operator is this class's, so that a fused form may stand in for it."""
-        return getattr(getattr(self, name), "__func__", None) is _OWN[name]
+    def _are_own(self, names) -> bool:
+        """Whether these operators are this class's, so that a fused form may stand in for them."""
+        cls, instance = type(self), self.__dict__
+        for name in names:
+            if name in instance or getattr(cls, name) is not _OWN[name]:
+                return False
+        return True
 
     def rmsnorm(self, x, weight, eps):
         if dense.is_rmsnorm_supported(x, weight):
@@ -50,7 +54,7 @@ class HipOpsBackend(DenseTorchOps):
 
     def add_rmsnorm(self, x, residual, weight, eps):
         """Extension: ``(x + residual, rmsnorm(x + residual))`` in one pass."""
-        if self._is_own("rmsnorm") and dense.is_rmsnorm_supported(x, weight, residual):
+        if self._are_own(("rmsnorm",)) and dense.is_rmsnorm_supported(x, weight, residual):
             return dense.add_rmsnorm(x, residual, weight, eps)
         total = x + residual
         return total, self.rmsnorm(total, weight, eps)
@@ -63,7 +67,7 @@ class HipOpsBackend(DenseTorchOps):
     def qkv_rope(self, qkv, cos, sin, heads):
         """Extension: rotated queries and keys and the values ``[B, heads, S, D]`` of a packed projection, or None when
         the kernel does not take it (the caller then splits the projection and calls ``rope``)."""
-        if not self._is_own("rope") or not dense.is_qkv_rope_supported(qkv, cos, sin, heads):
+        if not self._are_own(("rope",)) or not dense.is_qkv_rope_supported(qkv, cos, sin, heads):
             return None
         return dense.qkv_rope(qkv, cos, sin, heads)
 
@@ -110,7 +114,7 @@ class HipOpsBackend(DenseTorchOps):
         node (see ``kernels/hip/moe_layer.py``).  Returns None when the contract is not supported or one of the
         operators that it stands for is overridden; the caller then composes the layer from them."""
         operators = _OF_LAYER if capacity is None else _OF_LIMITED_LAYER
-        if not self.offers_moe_layer or not all(map(self._is_own, operators)) or moe_layer_violation(x, router_weight, gate_up_proj, down_proj, top_k) is not None:
+        if not self.offers_moe_layer or not self._are_own(operators) or moe_layer_violation(x, router_weight, gate_up_proj, down_proj, top_k) is not None:
             return None
         return run_moe_layer(x, router_weight, gate_up_proj, down_proj, top_k, normalize, capacity)
 

@@ -88,7 +88,7 @@ def test_contract_violations_are_reported_before_any_launch():
     assert lib.mts_moe_bwd_dw_workspace_bytes(2, 8, 768, 1024) == 2 * 8 * (3 * 4) * 256 * 256 * 4
     assert lib.mts_moe_bwd_dw1(fake, fake, fake, fake, 256, 2, 4, 64, 128, _lib.MTS_BF16, _lib.MTS_BF16, fake, fake, 16,
                                None) == WORKSPACE
-    # dW1 + dW2 + dX + dS as one launch: 16-bit activations with whole 64-wide k-tiles of 2I only
+    # dW1 + dW2 + dX + dS as one launch: 16-bit activations, 2I a multiple of 64 or at least 256
     assert lib.mts_moe_bwd_joint_supported(_lib.MTS_BF16, 768, 1024) == 1
     assert lib.mts_moe_bwd_joint_supported(_lib.MTS_F16, 64, 128) == 1
     assert lib.mts_moe_bwd_joint_supported(_lib.MTS_F32, 768, 1024) == 0

@@ -510,8 +510,8 @@ def test_reference_sweep_sizes(T):
 
 def test_mixtral_class_widths():
     """H = 4096, I = 14336 (the reference's `mixtral_7b` benchmark profile, moe_runner.py:53): one expert's weights
-    are 224 MiB, far more than an XCD's L2, so the row-tiled GEMMs deal their tiles round-robin over the XCDs, and
-    the reduction of dO*W2 is longer than the three-blocks-per-CU kernel takes, so it runs on the two-block ring.
+    are 224 MiB, far more than an XCD's L2, so the row-tiled GEMMs walk their column tiles in groups, and the
+    reduction of dO*W2 is longer than the three-blocks-per-CU kernel takes, so it runs on the specialised waves.
     Checked against the CPU oracle on sampled tokens (forward, dX, dS) and on slices of one expert's dW1 / dW2
     (float64 sums over the expert's routes), and through the reference's acceptance rule on the whole operator."""
     print("moe mixtral-class widths", flush=True)
