@@ -1,10 +1,10 @@
-// Tiles of fp32 products on v_mfma_f32_32x32x2_f32, shared by the fp32 expert GEMMs (mts_gemm_f32.hip) and the router
-// projection of many experts (mts_router_wide.hip): loaders, fragment reads and the k loop of a block of four waves.
+// Tiles of fp32 products on v_mfma_f32_32x32x2_f32 for the router projection of many experts (mts_router_wide.hip):
+// loaders, fragment reads and the k loop of a block of four waves.
 //
 // The k index an operand register stands for is free as long as both operands agree: lanes 0..31 hold k = 8s+0..3 and lanes
 // 32..63 k = 8s+4..7 of four consecutive instructions, so an operand whose rows are k-contiguous is read as one 16-byte
-// LDS load per four instructions, and one whose memory rows are k ("k-major": stored weights in the backward pass, both
-// operands of the weight gradients) as four 4-byte loads, with no transposed copy of anything.
+// LDS load per four instructions, and one whose memory rows are k ("k-major": the weights in the backward pass, both
+// operands of the weight gradient) as four 4-byte loads, with no transposed copy of anything.
 #pragma once
 
 #include "mts_common.h"

@@ -1,24 +1,35 @@
-// fp32 variant of the grouped expert GEMMs: activations, weights and accumulation all in fp32, on the fp32 matrix
-// instruction (v_mfma_f32_32x32x2_f32, full fp32 products and sums).  Same contracts and epilogues as the 16-bit kernels.
+// fp32 variant of the grouped expert GEMMs: activations, weights and results in fp32.  Same contracts and epilogues as the
+// 16-bit kernels.
 //
-// What bounds it: the instruction's rate, 157 TFLOP/s on the card (64 cycles for 4096 FLOP), a sixteenth of the bf16 rate,
-// so nothing here needs direct-to-LDS loads or specialised waves: tiles of 64 x 64 outputs per block of four waves, 16 of k
-// at a time through two LDS buffers, two more k-tiles in flight in registers, and up to eight blocks per CU.  A tile reads
-// one byte of L2 per 16 FLOP; tiles of 128 rows are no faster at 16 000 rows (101 TFLOP/s over all GEMMs either way) and
-// 12 % slower at 4096, where they leave the CUs unevenly filled.  2048 tokens, 768/1024, 8 experts, top-2: forward and
-// backward of the operator 1776 -> 727 us, 80 TFLOP/s (plain FMA from 64x64 tiles before: 33 TFLOP/s).
-#include "mts_f32_tiles.h"
+// An fp32 value is the exact sum of three bf16 ones (x = x0 + x1 + x2, each the rest rounded to nearest: mts_split3.h), a
+// product of two bf16 values is exact in fp32, and the bf16 matrix instruction adds in fp32 at 16 times the rate of the fp32
+// one.  A product is therefore taken as x0*y0 + x0*y1 + x1*y0 + x1*y1 + x0*y2 + x2*y0; the three terms left out are below
+// 2^-26 of it, a quarter of an fp32 rounding.  k-tiles that hold a value whose split is not exact (infinite, NaN, below 2^-60 or
+// from 2^127 on, but not zero) are multiplied by the fp32 instruction instead.
+//
+// What bounds it: on paper the matrix pipes (six instructions of 32 cycles for a 32 x 32 x 16 product: 417 TFLOP/s at 2.4 GHz, 2.7 times the fp32
+// instruction), in fact the vector unit that splits: a value costs about 8 vector instructions, each 4.9 cycles of a SIMD, and a wave alone
+// issues one in 8.  Hence half of a block's waves load and split while the other half multiply (in step, a block's two phases would add
+// up), tiles as large as two blocks of a CU can be (128 x 128, 16 of k, two LDS tiles: each value is split once per 128 outputs), and
+// loads that never depend on a branch.  2048 tokens, 768/1024, 8 experts, top-2, us before (fp32 instruction) and now: gate/up 178 -> 112, down
+// 90 -> 60, dO*W2 95 -> 90, dX 167 -> 96, dW1 146 -> 87, dW2 76 -> 57; 8192 tokens: 588 -> 397, 282 -> 172, 298 -> 227, 498 -> 324, 512 -> 303, 266 -> 177.
+// Relative error against fp64 over all five results of the operator: 4.1e-7..1.02e-6 where the fp32 instruction had 4.3e-7..1.18e-6,
+// smaller for each at every size (fewer roundings of a sum: 6 per 16 products instead of 8).
+#include "mts_split3.h"
 
 #include <type_traits>
 
 namespace {
 
-using namespace mts_f32;
+using namespace mts_split3;
 
-constexpr int BM = 64;   // rows of a tile, and of P columns in the weight gradients
-constexpr int kThreads = kTileThreads;
 constexpr int kXcds = 8;
-constexpr int TKS = 16;  // k extent of an LDS tile
+
+// Tiles of 128 x 128 where about 160 of them come together: below that the CUs they leave idle cost more than the smaller tiles'
+// splitting of every value twice as often.  us, 64 x 64 / 128 x 128 tiles, top-2, 8 experts of 768/1024: gate/up 32 / 39 at 256 tokens (128 tiles),
+// 47 / 42 at 512 (192); down 45 / 49 at 1024 (120), 76 / 60 at 2048 (216); dX 81 / 85 and 129 / 95 there.  Weight gradients, whose tiles do not
+// depend on the rows: dW1 15.2 / 14.5 at 64 tokens, 114 / 87 at 2048.
+bool large_tiles(int64_t rows, int64_t cols, int units) { return (rows + 64 * (int64_t)units) * cols >= 160 * 128 * 128; }
 
 enum Epi32 { E32_PLAIN = 0, E32_SWIGLU = 1, E32_DY1 = 2 };
 
@@ -45,6 +56,7 @@ __device__ __forceinline__ float sigmoid32(float x) { return 1.0f / (1.0f + expf
 
 // The m-tiles of all experts in expert order, 64 experts per round: their number, and expert and rows of tile `tile`
 // (every lane of the wave gets the same answer; tile < 0: only the number is wanted).
+template <int BM>
 __device__ __forceinline__ int find_m_tile(const int32_t* __restrict__ expert_start, int E, int tile, int& e_out, int& row0, int& rend) {
     const int lane = threadIdx.x % MTS_WAVE;
     int seen = 0;
@@ -71,120 +83,148 @@ __device__ __forceinline__ int find_m_tile(const int32_t* __restrict__ expert_st
 }
 
 // BN counts the columns of the B tile (SwiGLU: gate and up columns side by side, half the outputs)
-template <int BN, int EPI, bool BKM, bool VEC>
-__global__ __launch_bounds__(kThreads) void rows_gemm_f32_kernel(Rows32 p) {
+template <int BM, int BN, int EPI, bool BKM, bool VEC>
+__global__ __launch_bounds__(kThreads, 4) void rows_gemm_f32_kernel(Rows32 p) {
     constexpr int WAVES_M = 2, WAVES_N = 2;
     constexpr int MF = BM / WAVES_M / 32, NF = BN / WAVES_N / 32;
-    constexpr int OUT_N = EPI == E32_SWIGLU ? BN / 2 : BN;
-    typedef RowTile<float, BM, TKS, VEC> ATile;
-    typedef typename std::conditional<BKM, KTile<float, BN, TKS, VEC>, RowTile<float, BN, TKS, VEC>>::type BTile;
-    __shared__ __attribute__((aligned(16))) float As[2][ATile::SIZE];
-    __shared__ __attribute__((aligned(16))) float Bs[2][BTile::SIZE];
+    constexpr int OUT_N = EPI == E32_SWIGLU ? BN / 2 : BN, SLOT = 64, SLOTS = OUT_N / SLOT;
+    static_assert(OUT_N % SLOT == 0, "partial row sums cover 64 columns each");
+    typedef RowPlanes<BM, VEC> ATile;
+    typedef typename std::conditional<BKM, KPlanes<BN, VEC>, RowPlanes<BN, VEC>>::type BTile;
+    __shared__ __attribute__((aligned(16))) bf16_t As[2 * ATile::SIZE];
+    __shared__ __attribute__((aligned(16))) bf16_t Bs[2 * BTile::SIZE];
     __shared__ float ds_sum[EPI == E32_DY1 ? WAVES_N : 1][BM];
+    __shared__ float row_weight[EPI == E32_PLAIN ? 1 : BM];
+    __shared__ int special;
 
     // block b runs on XCD b % 8: every XCD takes an equal contiguous run of the tiles, columns fastest, so that an expert's
     // weights stream through one L2 and the blocks that share activation rows are neighbours in time
     int e = 0, row0 = 0, rend = 0;
-    const int total = find_m_tile(p.expert_start, p.E, -1, e, row0, rend) * p.n_tiles;
+    const int total = find_m_tile<BM>(p.expert_start, p.E, -1, e, row0, rend) * p.n_tiles;
     const int per_xcd = (total + kXcds - 1) / kXcds, slot = blockIdx.x / kXcds;
     const int tile = (blockIdx.x % kXcds) * per_xcd + slot;
     if (slot >= per_xcd || tile >= total) return;
-    find_m_tile(p.expert_start, p.E, tile / p.n_tiles, e, row0, rend);
+    find_m_tile<BM>(p.expert_start, p.E, tile / p.n_tiles, e, row0, rend);
     const int ny = tile % p.n_tiles, n0 = ny * OUT_N;
 
-    ATile a;
-#pragma unroll
-    for (int q = 0; q < ATile::LOADS; ++q) {
-        const int r = row0 + ATile::row(q);
-        a.ptr[q] = r < rend ? p.A + (int64_t)(p.a_gather ? p.a_gather[r] : r) * p.lda : nullptr;
+    if constexpr (EPI != E32_PLAIN) {   // the k loop's barriers stand between these and the epilogue
+        const int r = row0 + threadIdx.x;
+        if (threadIdx.x < BM) row_weight[threadIdx.x] = p.route_w && r < rend ? p.route_w[p.s_scatter[r]] : 1.f;
     }
-    const float* Be = p.B + (int64_t)e * p.b_rows * p.Kdim;
-    BTile b;
-    if constexpr (BKM) {
-        b.base = Be + n0 + BTile::col();
-        b.ld = p.N;
-        b.cols = p.N - n0 - BTile::col();
-    } else {
-#pragma unroll
-        for (int q = 0; q < BTile::LOADS; ++q) {
-            const int r = BTile::row(q), half = r / OUT_N, n = n0 + r % OUT_N;
-            b.ptr[q] = n < p.N ? Be + (int64_t)(half * p.N + n) * p.Kdim : nullptr;
-        }
-    }
-    auto fetch = [&](int set, int t) {
-        a.fetch(set, t * TKS, p.Kdim);
-        if constexpr (BKM) {
-            int64_t rows[BTile::LOADS];
-#pragma unroll
-            for (int q = 0; q < BTile::LOADS; ++q) rows[q] = t * TKS + BTile::k(q) < p.Kdim ? t * TKS + BTile::k(q) : -1;
-            b.fetch(set, rows);
-        } else b.fetch(set, t * TKS, p.Kdim);
-    };
-
+    if (threadIdx.x == 0) special = 0;
+    const int tiles = (p.Kdim + TK - 1) / TK;
+    f32x16 acc[MF][NF] = {};
     const int wave = threadIdx.x / MTS_WAVE, wm = wave / WAVES_N, wn = wave % WAVES_N, lane = threadIdx.x % MTS_WAVE;
     auto a_at = [&](int mf) { return wm * (BM / WAVES_M) + mf * 32; };
     auto b_at = [&](int nf) { return EPI == E32_SWIGLU ? nf / (NF / 2) * OUT_N + wn * (OUT_N / WAVES_N) + nf % (NF / 2) * 32 : wn * (BN / WAVES_N) + nf * 32; };
-    f32x16 acc[MF][NF] = {};
-    const int tiles = (p.Kdim + TKS - 1) / TKS;
-    run_k_tiles<ATile, BTile, TKS / 8, MF, NF>(tiles, a, b, As, Bs, acc, a_at, b_at, fetch);
-
+    if (threadIdx.x >= kLoaders) {
+        ATile a;
 #pragma unroll
-    for (int mf = 0; mf < MF; ++mf)
+        for (int q = 0; q < ATile::LOADS; ++q) {
+            const int r = row0 + ATile::row(q) < rend ? row0 + ATile::row(q) : rend - 1;
+            a.ptr[q] = p.A + (int64_t)(p.a_gather ? p.a_gather[r] : r) * p.lda;
+        }
+        const float* Be = p.B + (int64_t)e * p.b_rows * p.Kdim;
+        BTile b;
+        if constexpr (BKM) {
+            b.base = Be + n0;
+            b.ld = p.N;
+            b.cols = p.N - n0;
+        } else {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int r = a_at(mf) + 8 * (i / 4) + 4 * (lane / 32) + i % 4;
-            const int row = row0 + r;
-            const bool rok = row < rend;
-            if constexpr (EPI == E32_PLAIN) {
-#pragma unroll
-                for (int nf = 0; nf < NF; ++nf) {
-                    const int n = n0 + b_at(nf) + lane % 32;
-                    if (rok && n < p.N) p.C[(int64_t)row * p.N + n] = acc[mf][nf][i];
-                }
-            } else if constexpr (EPI == E32_SWIGLU) {
-                const float s = (rok && p.route_w) ? p.route_w[p.s_scatter[row]] : 1.f;   // post_act may carry the routing weight
-#pragma unroll
-                for (int nf = 0; nf < NF / 2; ++nf) {
-                    const int n = n0 + b_at(nf) + lane % 32;
-                    if (!rok || n >= p.N) continue;
-                    const float g = acc[mf][nf][i], u = acc[mf][nf + NF / 2][i];
-                    p.C[(int64_t)row * (2 * p.N) + n] = g;
-                    p.C[(int64_t)row * (2 * p.N) + p.N + n] = u;
-                    p.C2[(int64_t)row * p.N + n] = g * sigmoid32(g) * u * s;
-                }
-            } else {
-                const float s = rok ? p.route_w[p.s_scatter[row]] : 0.f;
-                float dsp = 0.f;
-#pragma unroll
-                for (int nf = 0; nf < NF; ++nf) {
-                    const int n = n0 + b_at(nf) + lane % 32;
-                    if (!rok || n >= p.N) continue;
-                    const int64_t o = (int64_t)row * (2 * p.N) + n;
-                    const float g = p.pre_act[o], u = p.pre_act[o + p.N];
-                    const float v = acc[mf][nf][i];
-                    const float sig = sigmoid32(g);
-                    const float silu = g * sig;
-                    const float y1 = silu * u;
-                    dsp += v * y1;
-                    if (p.C2) p.C2[(int64_t)row * p.N + n] = s * y1;
-                    const float da = v * s;
-                    p.C[o] = da * (silu * (1.0f - sig) + sig) * u;
-                    p.C[o + p.N] = da * silu;
-                }
-#pragma unroll
-                for (int o = 16; o > 0; o >>= 1) dsp += __shfl_xor(dsp, o, 32);
-                if (lane % 32 == 0) ds_sum[wn][r] = dsp;
+            for (int q = 0; q < BTile::LOADS; ++q) {
+                const int r = BTile::row(q), half = r / OUT_N, n = n0 + r % OUT_N < p.N ? n0 + r % OUT_N : p.N - 1;
+                b.ptr[q] = Be + (int64_t)(half * p.N + n) * p.Kdim;
             }
         }
-    if constexpr (EPI == E32_DY1) {   // row sums over the tile's 64 columns
-        __syncthreads();
-        for (int r = threadIdx.x; r < BM; r += kThreads)
-            if (row0 + r < rend) {
-                float v = ds_sum[0][r];
+        auto fetch = [&](int set, int t) {
+            a.fetch(set, t * TK, p.Kdim);
+            if constexpr (BKM) {
+                int64_t rows[BTile::LOADS];
 #pragma unroll
-                for (int q = 1; q < WAVES_N; ++q) v += ds_sum[q][r];
-                p.ds_part[(int64_t)(row0 + r) * p.np + ny] = v;
+                for (int q = 0; q < BTile::LOADS; ++q) rows[q] = t * TK + BTile::k(q) < p.Kdim ? t * TK + BTile::k(q) : p.Kdim - 1;
+                b.fetch(set, rows);
+            } else b.fetch(set, t * TK, p.Kdim);
+        };
+        load_k_tiles(p.Kdim, a, b, As, Bs, (LdsWord*)&special, fetch);
+    } else multiply_k_tiles<ATile, BTile>(tiles, As, Bs, (LdsWord*)&special, acc, a_at, b_at);
+
+    if (threadIdx.x < kLoaders) {
+#pragma unroll
+        for (int mf = 0; mf < MF; ++mf)
+#pragma unroll
+            for (int i4 = 0; i4 < 16; i4 += 4) {
+                const int r0 = a_at(mf) + 8 * (i4 / 4) + 4 * (lane / 32);   // the lane's four rows from here on
+                float g[NF][4], u[NF][4];
+                if constexpr (EPI == E32_DY1) {   // all loads of the four rows ahead of their use; the ones that do not exist read others
+#pragma unroll
+                    for (int nf = 0; nf < NF; ++nf)
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            const int row = row0 + r0 + j < rend ? row0 + r0 + j : rend - 1, n = n0 + b_at(nf) + lane % 32;
+                            const float* src = p.pre_act + (int64_t)row * (2 * p.N) + (n < p.N ? n : 0);
+                            g[nf][j] = src[0], u[nf][j] = src[p.N];
+                        }
+                }
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int r = r0 + j, row = row0 + r, i = i4 + j;
+                    const bool rok = row < rend;
+                    if constexpr (EPI == E32_PLAIN) {
+#pragma unroll
+                        for (int nf = 0; nf < NF; ++nf) {
+                            const int n = n0 + b_at(nf) + lane % 32;
+                            if (rok && n < p.N) p.C[(int64_t)row * p.N + n] = acc[mf][nf][i];
+                        }
+                    } else if constexpr (EPI == E32_SWIGLU) {
+                        const float s = row_weight[r];   // post_act may carry the routing weight
+#pragma unroll
+                        for (int nf = 0; nf < NF / 2; ++nf) {
+                            const int n = n0 + b_at(nf) + lane % 32;
+                            const float gate = acc[mf][nf][i], up = acc[mf][nf + NF / 2][i];
+                            const float y = gate * sigmoid32(gate) * up * s;
+                            if (!rok || n >= p.N) continue;
+                            p.C[(int64_t)row * (2 * p.N) + n] = gate;
+                            p.C[(int64_t)row * (2 * p.N) + p.N + n] = up;
+                            p.C2[(int64_t)row * p.N + n] = y;
+                        }
+                    } else {
+                        const float s = row_weight[r];
+                        float dsp = 0.f;
+#pragma unroll
+                        for (int nf = 0; nf < NF; ++nf) {
+                            const int n = n0 + b_at(nf) + lane % 32;
+                            const int64_t o = (int64_t)row * (2 * p.N) + n;
+                            const float v = acc[mf][nf][i];
+                            const float sig = sigmoid32(g[nf][j]);
+                            const float silu = g[nf][j] * sig;
+                            const float y1 = silu * u[nf][j];
+                            const float da = v * s, dg = da * (silu * (1.0f - sig) + sig) * u[nf][j];
+                            if (!rok || n >= p.N) continue;
+                            dsp += v * y1;
+                            if (p.C2) p.C2[(int64_t)row * p.N + n] = s * y1;
+                            p.C[o] = dg;
+                            p.C[o + p.N] = da * silu;
+                        }
+#pragma unroll
+                        for (int o = 16; o > 0; o >>= 1) dsp += __shfl_xor(dsp, o, 32);
+                        if (lane % 32 == 0) ds_sum[wn][r] = dsp;
+                    }
+                }
             }
+    }
+    if constexpr (EPI == E32_DY1) {   // row sums over 64 columns each: of one wave, or of the two that share them
+        constexpr int PER = WAVES_N / SLOTS;
+        __syncthreads();
+        for (int i = threadIdx.x; i < BM * SLOTS; i += kThreads) {
+            const int r = i % BM, slot = i / BM, at = ny * SLOTS + slot;
+            if (row0 + r < rend && at < p.np) {
+                float v = ds_sum[slot * PER][r];
+#pragma unroll
+                for (int q = 1; q < PER; ++q) v += ds_sum[slot * PER + q][r];
+                p.ds_part[(int64_t)(row0 + r) * p.np + at] = v;
+            }
+        }
     }
 }
 
@@ -200,14 +240,15 @@ struct Dw32 {
     int m_tiles, n_tiles;
 };
 
-// 64 x 64 outputs; the reduction runs over the expert's rows, both operands k-major
-template <typename OutT, bool VEC>
-__global__ __launch_bounds__(kThreads) void dw_gemm_f32_kernel(Dw32 p) {
-    constexpr int BN = 64, MF = BM / 64, NF = 1;
-    typedef KTile<float, BM, TKS, VEC> PT;
-    typedef KTile<float, BN, TKS, VEC> QT;
-    __shared__ __attribute__((aligned(16))) float Ps[2][PT::SIZE];
-    __shared__ __attribute__((aligned(16))) float Qs[2][QT::SIZE];
+// BM x BN outputs; the reduction runs over the expert's rows, both operands k-major
+template <int BM, int BN, typename OutT, bool VEC>
+__global__ __launch_bounds__(kThreads, 4) void dw_gemm_f32_kernel(Dw32 p) {
+    constexpr int MF = BM / 64, NF = BN / 64;
+    typedef KPlanes<BM, VEC> PT;
+    typedef KPlanes<BN, VEC> QT;
+    __shared__ __attribute__((aligned(16))) bf16_t Ps[2 * PT::SIZE];
+    __shared__ __attribute__((aligned(16))) bf16_t Qs[2 * QT::SIZE];
+    __shared__ int special;
     // an XCD takes an equal contiguous run of every expert's tiles, columns fastest: an equal share of the work however
     // uneven the experts are, and about an eighth of P through its L2
     const int per_expert = p.m_tiles * p.n_tiles, per_xcd = (per_expert + kXcds - 1) / kXcds;
@@ -217,63 +258,83 @@ __global__ __launch_bounds__(kThreads) void dw_gemm_f32_kernel(Dw32 p) {
     const int m0 = tile / p.n_tiles * BM, n0 = tile % p.n_tiles * BN;
     const int rbeg = p.expert_start[e], rend = p.expert_start[e + 1];
 
-    PT a;
-    QT b;
-    a.base = p.P + m0 + PT::col(), a.ld = p.M, a.cols = p.M - m0 - PT::col();
-    b.base = p.Q + n0 + QT::col(), b.ld = p.N, b.cols = p.N - n0 - QT::col();
-    int64_t pr[PT::LOADS], qr[QT::LOADS];   // memory rows of the k-tile to fetch next: read a tile ahead of its data
-    auto locate = [&](int r0) {
-#pragma unroll
-        for (int q = 0; q < PT::LOADS; ++q) {
-            const int r = r0 + PT::k(q);
-            pr[q] = r < rend ? (p.p_gather ? p.p_gather[r] : r) : -1;
-        }
-#pragma unroll
-        for (int q = 0; q < QT::LOADS; ++q) {
-            const int r = r0 + QT::k(q);
-            qr[q] = r < rend ? (p.q_gather ? p.q_gather[r] : r) : -1;
-        }
-    };
+    if (threadIdx.x == 0) special = 0;
+    const int tiles = (rend - rbeg + TK - 1) / TK;
     const int wave = threadIdx.x / MTS_WAVE, wm = wave / 2, wn = wave % 2, lane = threadIdx.x % MTS_WAVE;
     auto a_at = [&](int mf) { return wm * (BM / 2) + mf * 32; };
-    auto b_at = [&](int) { return wn * (BN / 2); };
+    auto b_at = [&](int nf) { return wn * (BN / 2) + nf * 32; };
     f32x16 acc[MF][NF] = {};
-    locate(rbeg);
-    auto fetch = [&](int set, int t) {
-        a.fetch(set, pr);
-        b.fetch(set, qr);
-        locate(rbeg + (t + 1) * TKS);
-    };
-    const int tiles = (rend - rbeg + TKS - 1) / TKS;
-    run_k_tiles<PT, QT, TKS / 8, MF, NF>(tiles, a, b, Ps, Qs, acc, a_at, b_at, fetch);
+    if (threadIdx.x >= kLoaders) {
+        PT a;
+        QT b;
+        a.base = p.P + m0, a.ld = p.M, a.cols = p.M - m0;
+        b.base = p.Q + n0, b.ld = p.N, b.cols = p.N - n0;
+        // Memory rows of the k-tiles, read two tiles ahead: loads return in order, so a row read one tile ahead would be waited
+        // for together with the data of the tile in front of it.  An operand that is not gathered reads some index and drops it.
+        int pi[2][PT::LOADS], qi[2][QT::LOADS];
+        auto locate = [&](int set, int r0) {
+#pragma unroll
+            for (int q = 0; q < PT::LOADS; ++q) pi[set][q] = *(p.p_gather ? p.p_gather + min(r0 + PT::k(q), rend - 1) : p.expert_start);
+#pragma unroll
+            for (int q = 0; q < QT::LOADS; ++q) qi[set][q] = *(p.q_gather ? p.q_gather + min(r0 + QT::k(q), rend - 1) : p.expert_start);
+        };
+        if (rbeg < rend) {
+            locate(0, rbeg);
+            locate(1, rbeg + TK);
+        }
+        auto fetch = [&](int set, int t) {   // set is t % 2
+            const int r0 = rbeg + t * TK;
+            int64_t pr[PT::LOADS], qr[QT::LOADS];
+#pragma unroll
+            for (int q = 0; q < PT::LOADS; ++q) pr[q] = p.p_gather ? pi[set][q] : min(r0 + PT::k(q), rend - 1);
+#pragma unroll
+            for (int q = 0; q < QT::LOADS; ++q) qr[q] = p.q_gather ? qi[set][q] : min(r0 + QT::k(q), rend - 1);
+            a.fetch(set, pr);
+            b.fetch(set, qr);
+            locate(set, r0 + 2 * TK);
+        };
+        load_k_tiles(rend - rbeg, a, b, Ps, Qs, (LdsWord*)&special, fetch);
+        return;
+    }
+    multiply_k_tiles<PT, QT>(tiles, Ps, Qs, (LdsWord*)&special, acc, a_at, b_at);
 
     OutT* C = reinterpret_cast<OutT*>(p.C) + (int64_t)e * p.M * p.N;
-    const int n = n0 + b_at(0) + lane % 32;
 #pragma unroll
     for (int mf = 0; mf < MF; ++mf)
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
             const int m = m0 + a_at(mf) + 8 * (i / 4) + 4 * (lane / 32) + i % 4;
-            if (m < p.M && n < p.N) C[(int64_t)m * p.N + n] = (OutT)acc[mf][0][i];
+#pragma unroll
+            for (int nf = 0; nf < NF; ++nf) {
+                const int n = n0 + b_at(nf) + lane % 32;
+                if (m < p.M && n < p.N) C[(int64_t)m * p.N + n] = (OutT)acc[mf][nf][i];
+            }
         }
 }
 
-int64_t m_tiles32(int64_t TK, int E) {
-    const int64_t a = (TK + BM - 1) / BM + E - 1;
-    return a < TK ? a : TK;
+int64_t m_tiles32(int64_t rows, int E, int bm) {
+    const int64_t a = (rows + bm - 1) / bm + E - 1;
+    return a < rows ? a : rows;
+}
+
+template <int BM, int BN, int EPI, bool BKM>
+int launch_rows_tile(Rows32 p, int64_t rows, bool vec, hipStream_t s) {
+    constexpr int OUT_N = EPI == E32_SWIGLU ? BN / 2 : BN;
+    p.n_tiles = (p.N + OUT_N - 1) / OUT_N;
+    const int64_t blocks = (m_tiles32(rows, p.E, BM) * p.n_tiles + kXcds - 1) / kXcds * kXcds;
+    if (blocks >= (1LL << 31)) return MTS_ERR_SHAPE;
+    const dim3 grid((unsigned)blocks);
+    if (vec) rows_gemm_f32_kernel<BM, BN, EPI, BKM, true><<<grid, kThreads, 0, s>>>(p);
+    else rows_gemm_f32_kernel<BM, BN, EPI, BKM, false><<<grid, kThreads, 0, s>>>(p);
+    MTS_CHECK_LAUNCH();
+    return MTS_OK;
 }
 
 template <int EPI, bool BKM>
-int launch_rows(Rows32 p, int64_t TK, bool vec, hipStream_t s) {
-    constexpr int BN = EPI == E32_SWIGLU ? 128 : 64, OUT_N = 64;
-    p.n_tiles = (p.N + OUT_N - 1) / OUT_N;
-    const int64_t blocks = (m_tiles32(TK, p.E) * p.n_tiles + kXcds - 1) / kXcds * kXcds;
-    if (blocks >= (1LL << 31)) return MTS_ERR_SHAPE;
-    const dim3 grid((unsigned)blocks);
-    if (vec) rows_gemm_f32_kernel<BN, EPI, BKM, true><<<grid, kThreads, 0, s>>>(p);
-    else rows_gemm_f32_kernel<BN, EPI, BKM, false><<<grid, kThreads, 0, s>>>(p);
-    MTS_CHECK_LAUNCH();
-    return MTS_OK;
+int launch_rows(const Rows32& p, int64_t rows, bool vec, hipStream_t s) {
+    constexpr int SMALL_N = EPI == E32_SWIGLU ? 128 : 64;
+    if (large_tiles(rows, EPI == E32_SWIGLU ? 2 * p.N : p.N, p.E)) return launch_rows_tile<128, 128, EPI, BKM>(p, rows, vec, s);
+    return launch_rows_tile<64, SMALL_N, EPI, BKM>(p, rows, vec, s);
 }
 
 }  // namespace
@@ -293,15 +354,19 @@ int mts_f32_rows(int epi, const float* A, int lda, const int32_t* a_gather, cons
 
 int mts_f32_dw(const float* P, const int32_t* p_gather, const float* Q, const int32_t* q_gather, int M,
                int N, const int32_t* expert_start, int E, int grad_dtype, void* C, hipStream_t s) {
-    Dw32 p = {P, p_gather, Q, q_gather, M, N, expert_start, E, C, (M + BM - 1) / BM, (N + 63) / 64};
+    const bool large = large_tiles((int64_t)E * M, N, 0);
+    const int bt = large ? 128 : 64;
+    Dw32 p = {P, p_gather, Q, q_gather, M, N, expert_start, E, C, (M + bt - 1) / bt, (N + bt - 1) / bt};
     const bool vec = M % 4 == 0 && N % 4 == 0 && mts_aligned16(P) && mts_aligned16(Q);
     const int64_t blocks = ((int64_t)p.m_tiles * p.n_tiles + kXcds - 1) / kXcds * kXcds * E;
     if (blocks >= (1LL << 31)) return MTS_ERR_SHAPE;
     const dim3 grid((unsigned)blocks);
     auto launch = [&](auto* kind) {
         typedef typename std::remove_pointer<decltype(kind)>::type OutT;
-        if (vec) dw_gemm_f32_kernel<OutT, true><<<grid, kThreads, 0, s>>>(p);
-        else dw_gemm_f32_kernel<OutT, false><<<grid, kThreads, 0, s>>>(p);
+        if (large && vec) dw_gemm_f32_kernel<128, 128, OutT, true><<<grid, kThreads, 0, s>>>(p);
+        else if (large) dw_gemm_f32_kernel<128, 128, OutT, false><<<grid, kThreads, 0, s>>>(p);
+        else if (vec) dw_gemm_f32_kernel<64, 64, OutT, true><<<grid, kThreads, 0, s>>>(p);
+        else dw_gemm_f32_kernel<64, 64, OutT, false><<<grid, kThreads, 0, s>>>(p);
     };
     if (grad_dtype == MTS_F32) launch((float*)nullptr);
     else if (grad_dtype == MTS_BF16) launch((bf16_t*)nullptr);

@@ -1,8 +1,9 @@
-"""fp32 activations through the fp32 matrix-instruction GEMMs at the edges of their tiles, against the oracle in fp64."""
+"""fp32 activations through the fp32 GEMMs at the edges of their tiles, against the oracle in fp64."""
 
 import pytest
 import torch
 
+from minitrain_amd import _lib
 from tests.helpers import assert_close_scaled, hip_moe_grads, oracle_moe_grads, routed_case
 
 pytestmark = pytest.mark.gpu
@@ -13,6 +14,8 @@ pytestmark = pytest.mark.gpu
     (257, 64, 4, 130, 2),     # I not a multiple of 4: rows loaded four bytes at a time; column tiles with a remainder
     (129, 36, 70, 24, 2),     # more experts than a wave holds
     (512, 132, 8, 200, 2),    # wider than a column tile, with a remainder of four
+    (1500, 520, 3, 1032, 2),  # tiles of 128 x 128 in every GEMM, the last k-tile half empty
+    (1300, 513, 2, 1031, 2),  # the same at odd widths
     (33, 64, 2, 64, 1), (1, 4, 1, 1, 1)])
 @pytest.mark.parametrize("wdtype", [torch.float32, torch.bfloat16])
 def test_fp32_gemms(T, H, E, I, K, wdtype):
@@ -26,3 +29,61 @@ def test_fp32_gemms(T, H, E, I, K, wdtype):
     assert_close_scaled(out, ref_out, 1e-5, "out")
     for name, a, b in zip(("dx", "dW1", "dW2", "dS"), grads, ref_grads):
         assert_close_scaled(a, b, 2.0 ** -8 if a.dtype == torch.bfloat16 else 1e-5, name)
+
+
+def _down(act, w2, starts):
+    y = torch.empty(act.shape[0], w2.shape[1], device="cuda")
+    es = torch.tensor(starts, dtype=torch.int32, device="cuda")
+    _lib.check(_lib.load().mts_moe_fwd_down(act.data_ptr(), w2.data_ptr(), es.data_ptr(), act.shape[0], w2.shape[0], w2.shape[1], act.shape[1], _lib.MTS_F32,
+                                            y.data_ptr(), torch.cuda.current_stream().cuda_stream), "down")
+    return y.cpu()
+
+
+def _dw2(d_out, act, starts):
+    T, H = d_out.shape
+    dw = torch.empty(len(starts) - 1, H, act.shape[1], device="cuda")
+    es = torch.tensor(starts, dtype=torch.int32, device="cuda")
+    gather = torch.arange(T, dtype=torch.int32, device="cuda")
+    _lib.check(_lib.load().mts_moe_bwd_dw2(d_out.data_ptr(), act.data_ptr(), gather.data_ptr(), es.data_ptr(), T, 1, len(starts) - 1, H, act.shape[1], _lib.MTS_F32,
+                                           _lib.MTS_F32, dw.data_ptr(), None, 0, torch.cuda.current_stream().cuda_stream), "dw2")
+    return dw.cpu()
+
+
+@pytest.mark.parametrize("R,H,I", [(90, 72, 100), (2700, 1100, 260)])   # both tile sizes
+def test_values_that_three_bf16_terms_do_not_hold(R, H, I):
+    """Infinities, NaN, the largest and the smallest numbers, denormal ones among them, in single rows and at any place of the
+    reduction: what plain products of these values give, and nothing in the other rows.  1e-5 as above; a value is scaled so that its products are
+    ordinary numbers."""
+    print(f"special fp32 values R={R} H={H} I={I}", flush=True)
+    torch.manual_seed(R)
+    starts = [0, R // 3, R // 3, R]
+    act, w2 = torch.randn(R, I), torch.randn(3, H, I) * 0.05
+    act[3, 5], act[R - 1, I - 1], act[40, 0] = float("inf"), float("-inf"), float("nan")
+    act[7] *= 2.0 ** -135
+    act[8] *= 2.0 ** -70
+    act[9, 40] = 3.4e38
+    big = w2 * 2.0 ** 90
+    big[:, :, 40] = 0.0   # the largest number meets zero there, where its rounding up would give NaN
+    got, got_big = _down(act.cuda(), w2.cuda(), starts), _down(act.cuda(), big.cuda(), starts)
+    expert = (torch.arange(R) >= starts[2]).long() * 2
+    for w, y in ((w2, got), (big, got_big)):
+        want = torch.einsum("ri,rhi->rh", act.double(), w.double()[expert]).float()
+        for r in range(R):
+            a, b = y[r], want[r]
+            if r in (3, 40, R - 1):
+                assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.isinf(), b.isinf()) and torch.equal(a[a.isinf()], b[b.isinf()]), r
+            elif not (r in (7, 8) and w is w2):
+                assert_close_scaled(a, b, 1e-5, f"row {r}")
+    # weight gradient: a column of d_out is a row of the result
+    d_out, act = torch.randn(R, H), torch.randn(R, I)
+    d_out[1, 2], d_out[R - 2, 50], act[5, 9] = float("inf"), float("nan"), 2.0 ** -140
+    d_out[R // 3:, 4] *= 2.0 ** -90
+    act[R // 3:] *= 2.0 ** 80
+    dw = _dw2(d_out.cuda(), act.cuda(), starts)
+    assert not dw[1].any()
+    for e, (lo, hi) in ((0, (0, starts[1])), (2, (starts[2], R))):
+        want = (d_out[lo:hi].double().t() @ act[lo:hi].double()).float()
+        for h in range(H):
+            assert torch.equal(dw[e, h].isnan(), want[h].isnan()), h
+            if want[h].isfinite().all():
+                assert_close_scaled(dw[e, h], want[h], 1e-5, f"column {h}")
