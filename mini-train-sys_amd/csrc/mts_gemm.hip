@@ -115,6 +115,30 @@ struct Tile {
     static_assert((BM * 8) % NT == 0 && (BN * 8) % NT == 0, "loader split");
 };
 
+// Division by a number the host knows, for the block-uniform index arithmetic in front of a tile: a multiplication and a correction on the
+// scalar unit, where the compiler's sequence is some twenty vector instructions, each of which costs a lone wave eight cycles.
+struct Divider {
+    uint32_t d, inverse;   // floor(2^32 / d): the product is the quotient or one less
+    void set(int by) { d = (uint32_t)by, inverse = by > 1 ? (uint32_t)((1ull << 32) / (uint32_t)by) : 0xffffffffu; }
+    __device__ __forceinline__ int quotient(int x, int& rest) const {
+        uint32_t q = __umulhi((uint32_t)x, inverse), r = (uint32_t)x - q * d;
+        if (r >= d) ++q, r -= d;
+        rest = (int)r;
+        return (int)q;
+    }
+};
+
+// inclusive sum over the wave's lanes, on the vector unit alone (a shuffle goes through LDS: a hundred cycles for each of six)
+__device__ __forceinline__ int wave_scan(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);   // one lane up within a row of 16, then 2, 4, 8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);   // the last lane of rows 0 and 2 to rows 1 and 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);   // lane 31 to rows 2 and 3
+    return v;
+}
+
 // EPI_DY1N: the dO*W2 epilogue without the weighted_act output (the caller kept the forward
 // pass's post_act, which already carries the routing weight)
 enum Epilogue { EPI_PLAIN = 0, EPI_SWIGLU = 1, EPI_DY1 = 2, EPI_DY1N = 3 };
@@ -139,7 +163,8 @@ struct RowsParams {
     float* ds_part;            // DY1: [TK][np]
     int np;
     int64_t TK;                // rows of every output
-    int n_tiles;               // column tiles per m-tile (set by the launcher)
+    int n_tiles;               // column tiles per m-tile (set by the launcher, like by_n_tiles and by_group)
+    Divider by_n_tiles, by_group;   // by n_tiles and by the tiles of a group
     int xcd_ranges;            // block -> tile mapping: 1 = every XCD takes a contiguous range of m-tiles
     int n_groups;              // with xcd_ranges: the n-tiles are walked in this many groups, all m-tiles of the range per group
     int reverse;               // with xcd_ranges: the range's m-tiles are walked from the last to the first
@@ -586,12 +611,14 @@ __device__ __forceinline__ void rows_epilogue(const RowsParams& p, f32x16 (&acc)
 // xcd + 8*(j / n_tiles): all eight L2s then stream the same expert's weights at the
 // same time and each of them again for every group of m-tiles.
 // ---------------------------------------------------------------------------
-constexpr int kXcds = 8;
+constexpr int kXcds = 8, kCusPerXcd = 32;
 
 // The expert that owns m-tile `tile` is found with one vector load: lane l reads
 // expert_start[l] and [l+1], a wave scan turns tile counts into tile offsets, and a
-// ballot picks the first expert whose offset range contains the tile (63 experts per
-// round; more experts take more rounds).
+// ballot picks the first expert whose offset range contains the tile (up to 64 experts; more take a round of shuffles
+// for every 64).  A tile is a few microseconds of work behind this, so it is kept short: the scan and the divisions as above, the
+// answer read out of its lane straight into scalar registers.  With shuffles and the compiler's divisions it took 1.8 us of a tile's time
+// (a weight-gradient tile of two k-tiles 12.9 -> 11.1 us); the layer of 24 576 tokens 877 -> 868 us, 4096 tokens of 4096/14336 -1.4 %.
 // mtile: the m-tile's index in expert order, -1 where the block has none; a block that has the empty half of a cut tile
 // (the tile's rows end in the other half) gets the index and the answer false.
 template <int BM>
@@ -600,90 +627,92 @@ __device__ __forceinline__ bool find_rows_tile(const RowsParams& p, int b, int& 
     mtile = -1;
     // up to 64 experts: lane l reads expert_start[l] and [l + 1] once, for the count of m-tiles and for the search
     const bool in_regs = p.E <= MTS_WAVE;
-    const int lane_ = threadIdx.x % MTS_WAVE;
-    const int w0 = in_regs && lane_ < p.E ? p.expert_start[lane_] : 0;
-    const int w1 = in_regs && lane_ < p.E ? p.expert_start[lane_ + 1] : 0;
+    const int lane = threadIdx.x % MTS_WAVE;
+    const int w0 = in_regs && lane < p.E ? p.expert_start[lane] : 0;
+    const int w1 = in_regs && lane < p.E ? p.expert_start[lane + 1] : 0;
+    const int wnt = (w1 - w0 + BM - 1) / BM, wincl = wave_scan(wnt);   // in_regs: the lane's m-tiles, and those up to its last one
     const int xcd = b % kXcds;
     int j = b / kXcds;
-    const int lane = threadIdx.x % MTS_WAVE;
-    int tile = xcd + kXcds * (j / p.n_tiles);
-    ntile = j % p.n_tiles;
+    int k = p.by_n_tiles.quotient(j, ntile);
+    int tile = xcd + kXcds * k;
     parts = 1;      // pieces the tile is cut into: this block computes piece `part`
     int part = 0;
     if (p.xcd_ranges && p.sched) {
         // the XCD's range of m-tiles comes from the table (n-tile groups and cut tiles are not combined with it); a block
         // the table leaves without work finds that out with one load
         const int my = p.sched[kXcds + xcd];
-        int k = j / p.n_tiles;
         if (k >= my) return false;
         if (p.reverse) k = my - 1 - k;
         tile = p.sched[xcd] + k;
     } else if (p.xcd_ranges) {
         // m-tiles of the launch: the first (total % 8) XCDs take one more than the others
-        int mine = 0;
-        if (in_regs) mine = (w1 - w0 + BM - 1) / BM;
-        else
-            for (int le = lane; le < p.E; le += MTS_WAVE) mine += (p.expert_start[le + 1] - p.expert_start[le] + BM - 1) / BM;
+        int all = __builtin_amdgcn_readlane(wincl, MTS_WAVE - 1);
+        if (!in_regs) {
+            for (int le = lane; le < p.E; le += MTS_WAVE) all += (p.expert_start[le + 1] - p.expert_start[le] + BM - 1) / BM;
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1) mine += __shfl_xor(mine, o, MTS_WAVE);
-        const int per = mine / kXcds, rem = mine % kXcds;
+            for (int o = 32; o > 0; o >>= 1) all += __shfl_xor(all, o, MTS_WAVE);
+        }
+        const int per = all / kXcds, rem = all % kXcds;
         const int my = per + (xcd < rem ? 1 : 0);
         if (p.tail_slots > 0 || p.tail_tiles > 0) {
             // the blocks behind the last whole round of this XCD: two per tile, the upper and the lower half (cutting
             // into four where a quarter of the slots is filled gains another 0.15 % of the layer step: not done)
             const int total = my * p.n_tiles;
-            const int whole = p.tail_tiles > 0 ? (total > p.tail_tiles ? total - p.tail_tiles : 0) : total / p.tail_slots * p.tail_slots;
-            const int cut = p.tail_tiles > 0 || 2 * (total - whole) <= p.tail_slots ? 2 : 1;
-            if (cut > 1 && j >= whole) {
-                parts = cut;
-                part = (j - whole) % cut;
-                j = whole + (j - whole) / cut;
-                ntile = j % p.n_tiles;
+            const int whole = p.tail_tiles > 0 ? (total > p.tail_tiles ? total - p.tail_tiles : 0) : total / kCusPerXcd * kCusPerXcd;
+            if ((p.tail_tiles > 0 || 2 * (total - whole) <= kCusPerXcd) && j >= whole) {
+                parts = 2;
+                part = (j - whole) % 2;
+                j = whole + (j - whole) / 2;
+                k = p.by_n_tiles.quotient(j, ntile);
             }
         }
-        int k = j / p.n_tiles;
         if (p.n_groups > 1 && my > 0) {
-            const int npg = p.n_tiles / p.n_groups;   // n-tiles per group (n_tiles is a multiple of n_groups)
-            const int g = j / (my * npg);
+            // group g of the columns, m-tile k of the range, column r of the group: j = (g * my + k) * npg + r
+            const int gk = p.by_group.quotient(j, ntile), g = gk / my;
             if (g >= p.n_groups) return false;
-            const int r = j - g * my * npg;
-            k = r / npg;
-            ntile = g * npg + r % npg;
+            k = gk - g * my;
+            ntile += g * (int)p.by_group.d;
         }
         if (k >= my) return false;
         if (p.reverse) k = my - 1 - k;
         tile = xcd * per + (xcd < rem ? xcd : rem) + k;
     }
-    int seen = 0;
-    for (int e0 = 0; e0 < p.E; e0 += MTS_WAVE) {
-        const int le = e0 + lane;
-        const int s0 = in_regs ? w0 : (le < p.E ? p.expert_start[le] : 0);
-        const int s1 = in_regs ? w1 : (le < p.E ? p.expert_start[le + 1] : 0);
-        const int nt = (s1 - s0 + BM - 1) / BM;
-        int incl = nt;
-#pragma unroll
-        for (int o = 1; o < MTS_WAVE; o <<= 1) {
-            const int up = __shfl_up(incl, o, MTS_WAVE);
-            if (lane >= o) incl += up;
-        }
-        const uint64_t hit = __ballot(tile < seen + incl);
+    bool found = false;
+    if (in_regs) {
+        const uint64_t hit = __ballot(tile < wincl);
         if (hit) {
             const int w = __ffsll((unsigned long long)hit) - 1;
-            const int first = seen + __shfl(incl, w, MTS_WAVE) - __shfl(nt, w, MTS_WAVE);
-            e = e0 + w;
-            row0 = __shfl(s0, w, MTS_WAVE) + (tile - first) * BM;
-            rend = __shfl(s1, w, MTS_WAVE);
-            mtile = tile;
-            if (parts > 1) {
-                row0 += part * (BM / parts);
-                if (row0 + BM / parts < rend) rend = row0 + BM / parts;
-                return row0 < rend;
-            }
-            return true;
+            e = w;
+            row0 = __builtin_amdgcn_readlane(w0, w) + (tile - __builtin_amdgcn_readlane(wincl - wnt, w)) * BM;
+            rend = __builtin_amdgcn_readlane(w1, w);
+            found = true;
         }
-        seen += __shfl(incl, MTS_WAVE - 1, MTS_WAVE);
+    } else {
+        int seen = 0;
+        for (int e0 = 0; e0 < p.E && !found; e0 += MTS_WAVE) {
+            const int le = e0 + lane;
+            const int s0 = le < p.E ? p.expert_start[le] : 0;
+            const int s1 = le < p.E ? p.expert_start[le + 1] : 0;
+            const int nt = (s1 - s0 + BM - 1) / BM, incl = wave_scan(nt);
+            const uint64_t hit = __ballot(tile < seen + incl);
+            if (hit) {
+                const int w = __ffsll((unsigned long long)hit) - 1;
+                e = e0 + w;
+                row0 = __shfl(s0, w, MTS_WAVE) + (tile - seen - __shfl(incl - nt, w, MTS_WAVE)) * BM;
+                rend = __shfl(s1, w, MTS_WAVE);
+                found = true;
+            }
+            seen += __shfl(incl, MTS_WAVE - 1, MTS_WAVE);
+        }
     }
-    return false;
+    if (!found) return false;
+    mtile = tile;
+    if (parts > 1) {
+        row0 += part * (BM / parts);
+        if (row0 + BM / parts < rend) rend = row0 + BM / parts;
+        return row0 < rend;
+    }
+    return true;
 }
 
 // The answer is the same in every lane, and the compiler is told so behind the search loop: descriptors
@@ -1302,6 +1331,7 @@ struct DwParams {
     void* C;  // [E][M][N], bf16 or f32
     float* part;   // fp32 tile partials of experts whose rows are split over several blocks, or null
     int E, n_tiles, tiles_per_expert;  // set by the launcher
+    Divider by_n_tiles, by_tiles;      // by n_tiles and tiles_per_expert
     const int32_t* sched;   // the unit table of the joint backward launch's schedule (which units an XCD runs), or NULL:
     int sched_slots;        // unit u runs on XCD u % 8; sched_slots: table entries per XCD
     int segment_rows;       // not 0: no experts, E segments of this many of the TK rows
@@ -1344,6 +1374,13 @@ __device__ __forceinline__ bool locate_dw_unit(const DwParams& p, int unit, DwUn
         u.rend = (int)(first + p.segment_rows < p.TK ? first + p.segment_rows : p.TK);
         return unit < p.E;
     }
+    if (p.part == nullptr) {   // no row chunks: unit u is expert u
+        if (unit >= p.E) return false;
+        u.e = unit, u.slot = -1;
+        u.rbeg = p.expert_start[unit];
+        u.rend = p.expert_start[unit + 1];
+        return true;
+    }
     const int lane = threadIdx.x % MTS_WAVE;
     const int share = dw_share(p);
     int seen = 0, seen_slots = 0;
@@ -1353,31 +1390,23 @@ __device__ __forceinline__ bool locate_dw_unit(const DwParams& p, int unit, DwUn
         const int s1 = le < p.E ? p.expert_start[le + 1] : 0;
         const int nc = le < p.E ? dw_chunks(p, s1 - s0, share) : 0;
         const int ns = nc > 1 ? nc : 0;
-        int incl = nc, sincl = ns;
-#pragma unroll
-        for (int o = 1; o < MTS_WAVE; o <<= 1) {
-            const int up = __shfl_up(incl, o, MTS_WAVE), sup = __shfl_up(sincl, o, MTS_WAVE);
-            if (lane >= o) {
-                incl += up;
-                sincl += sup;
-            }
-        }
+        const int incl = wave_scan(nc), sincl = wave_scan(ns);
         const uint64_t hit = __ballot(le < p.E && unit < seen + incl);
         if (hit) {
-            const int w = __ffsll((unsigned long long)hit) - 1;
-            const int ncw = __shfl(nc, w, MTS_WAVE);
-            const int c = unit - (seen + __shfl(incl, w, MTS_WAVE) - ncw);
-            const int b = __shfl(s0, w, MTS_WAVE), e = __shfl(s1, w, MTS_WAVE);
+            const int w = __builtin_amdgcn_readfirstlane(__ffsll((unsigned long long)hit) - 1);
+            const int ncw = __builtin_amdgcn_readlane(nc, w);
+            const int c = unit - (seen + __builtin_amdgcn_readlane(incl, w) - ncw);
+            const int b = __builtin_amdgcn_readlane(s0, w), e = __builtin_amdgcn_readlane(s1, w);
             const int per = ((e - b + ncw - 1) / ncw + 31) / 32 * 32;
             const int r0 = b + c * per;
             u.e = e0 + w;
             u.rbeg = r0 < e ? r0 : e;
             u.rend = r0 + per < e ? r0 + per : e;
-            u.slot = ncw > 1 ? seen_slots + __shfl(sincl, w, MTS_WAVE) - __shfl(ns, w, MTS_WAVE) + c : -1;
+            u.slot = ncw > 1 ? seen_slots + __builtin_amdgcn_readlane(sincl - ns, w) + c : -1;
             return true;
         }
-        seen += __shfl(incl, MTS_WAVE - 1, MTS_WAVE);
-        seen_slots += __shfl(sincl, MTS_WAVE - 1, MTS_WAVE);
+        seen += __builtin_amdgcn_readlane(incl, MTS_WAVE - 1);
+        seen_slots += __builtin_amdgcn_readlane(sincl, MTS_WAVE - 1);
     }
     return false;
 }
@@ -1786,34 +1815,6 @@ struct DwWsTile {
     static_assert(LDS_ELEMS * 2 <= 160 * 1024, "LDS capacity");
 };
 
-// the work of block `block` of a launch; `smem` holds T::LDS_ELEMS elements, 1 KiB aligned
-template <class T, typename OutT>
-__device__ __forceinline__ void dw_gemm_ws_block(const DwParams& p, bf16_t* smem, int block) {
-    constexpr int S = T::STAGES, L = T::A_INSTR + T::B_INSTR;
-    // all tiles of a unit (an expert, or a row chunk of an over-full one) run on one XCD
-    const int xcd = block % kXcds, jb = block / kXcds;
-    DwUnit unit;
-    if (p.sched) {
-        const int k = jb / p.tiles_per_expert;
-        if (k >= p.sched[kSchedCounts + xcd]) return;
-        const int32_t* u = p.sched + kSchedUnits + (xcd * p.sched_slots + k) * 4;
-        unit.e = u[0]; unit.rbeg = u[1]; unit.rend = u[2]; unit.slot = u[3];
-    } else if (!locate_dw_unit(p, xcd + kXcds * (jb / p.tiles_per_expert), unit)) {
-        return;
-    }
-    const int e = __builtin_amdgcn_readfirstlane(unit.e);
-    const int rbeg = __builtin_amdgcn_readfirstlane(unit.rbeg), rend = __builtin_amdgcn_readfirstlane(unit.rend);
-    const int slot = __builtin_amdgcn_readfirstlane(unit.slot);
-    const int tile = jb % p.tiles_per_expert;
-    const int m0 = (tile / p.n_tiles) * T::BM, n0 = (tile % p.n_tiles) * T::BN;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / MTS_WAVE), lane = threadIdx.x % MTS_WAVE;
-    const int nk = (rend - rbeg + T::BKS - 1) / T::BKS;
-
-    if (wave >= T::NWAVES) {
-        // ------------------------------ producer ------------------------------
-        // The producer's own instruction count bounds the fill rate (a wave issues roughly one
-        // instruction per 4-8 clocks), so everything that does not change from tile to tile is
-        // computed once.  An operand that is read in place gets a descriptor that starts at the
 // Accumulators -> the tile at C (leading dimension ldc, rows x cols of it exist).  The MFMAs take the Q fragment first, so a lane holds runs of four
 // consecutive columns of one row; 32 x 64 slabs go through the wave's part of `stage` and out in 16-byte pieces, whole 128-byte lines
 // per row.  An element a lane and store, with an address and a bounds check each, took 3.4 us a tile; now 1.7 (a tile of 1024 rows at
@@ -1858,6 +1859,34 @@ __device__ __forceinline__ void dw_epilogue(f32x16 (&acc)[T::MF][T::NF], bf16_t*
     }
 }
 
+// the work of block `block` of a launch; `smem` holds T::LDS_ELEMS elements, 1 KiB aligned
+template <class T, typename OutT>
+__device__ __forceinline__ void dw_gemm_ws_block(const DwParams& p, bf16_t* smem, int block) {
+    constexpr int S = T::STAGES, L = T::A_INSTR + T::B_INSTR;
+    // all tiles of a unit (an expert, or a row chunk of an over-full one) run on one XCD
+    const int xcd = block % kXcds, jb = block / kXcds;
+    DwUnit unit;
+    int tile, tile_n;
+    const int k = p.by_tiles.quotient(jb, tile);
+    if (p.sched) {
+        if (k >= p.sched[kSchedCounts + xcd]) return;
+        const int32_t* u = p.sched + kSchedUnits + (xcd * p.sched_slots + k) * 4;
+        unit.e = u[0]; unit.rbeg = u[1]; unit.rend = u[2]; unit.slot = u[3];
+    } else if (!locate_dw_unit(p, xcd + kXcds * k, unit)) {
+        return;
+    }
+    const int e = __builtin_amdgcn_readfirstlane(unit.e);
+    const int rbeg = __builtin_amdgcn_readfirstlane(unit.rbeg), rend = __builtin_amdgcn_readfirstlane(unit.rend);
+    const int slot = __builtin_amdgcn_readfirstlane(unit.slot);
+    const int m0 = p.by_n_tiles.quotient(tile, tile_n) * T::BM, n0 = tile_n * T::BN;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / MTS_WAVE), lane = threadIdx.x % MTS_WAVE;
+    const int nk = (rend - rbeg + T::BKS - 1) / T::BKS;
+
+    if (wave >= T::NWAVES) {
+        // ------------------------------ producer ------------------------------
+        // The producer's own instruction count bounds the fill rate (a wave issues roughly one
+        // instruction per 4-8 clocks), so everything that does not change from tile to tile is
+        // computed once.  An operand that is read in place gets a descriptor that starts at the
         // tile's first row and ends at the expert's last row, rebuilt with scalar instructions
         // per tile: the per-lane offsets are constants and rows past the expert's end read as
         // zeros.  A gathered operand takes its row indices through the scalar cache, fetched
@@ -1901,9 +1930,8 @@ __device__ __forceinline__ void dw_epilogue(f32x16 (&acc)[T::MF][T::NF], bf16_t*
                 if (gath_q) s_buffer_load8(rs_gq, (r0 + pw * ROWS_B + 8 * h) * 4, idx_b[2 * h], idx_b[2 * h + 1]);
             }
         };
-        auto issue = [&](int stage, int r0) {
+        auto issue_p = [&](int stage, int r0) {
             bf16_t* sa = smem + stage * T::STAGE + pw * T::A_INSTR * 512;
-            bf16_t* sb = smem + stage * T::STAGE + T::BKS * T::BM + pw * T::B_INSTR * 512;
             const int left = rend - r0;   // rows of the expert from this tile on
             if (gath_p) {
 #pragma unroll
@@ -1919,6 +1947,10 @@ __device__ __forceinline__ void dw_epilogue(f32x16 (&acc)[T::MF][T::NF], bf16_t*
                 for (int j = 0; j < T::A_INSTR; ++j)
                     __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, MTS_LDS_PTR(sa + j * 512), 16, (int)fix_a[j], 0, 0, 0);
             }
+        };
+        auto issue_q = [&](int stage, int r0) {
+            bf16_t* sb = smem + stage * T::STAGE + T::BKS * T::BM + pw * T::B_INSTR * 512;
+            const int left = rend - r0;
             if (gath_q) {
 #pragma unroll
                 for (int j = 0; j < T::B_INSTR; ++j) {
@@ -1934,12 +1966,22 @@ __device__ __forceinline__ void dw_epilogue(f32x16 (&acc)[T::MF][T::NF], bf16_t*
                     __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, MTS_LDS_PTR(sb + j * 512), 16, (int)fix_b[j], 0, 0, 0);
             }
         };
+        auto issue = [&](int stage, int r0) {
+            issue_p(stage, r0);
+            issue_q(stage, r0);
+        };
+        auto issue_first = [&]() {   // the operand that is read in place does not wait for the row indices of the other
+            if (!gath_p) issue_p(0, rbeg);
+            if (!gath_q) issue_q(0, rbeg);
+            fetch_index(rbeg);
+            if (gath_p) issue_p(0, rbeg);
+            if (gath_q) issue_q(0, rbeg);
+        };
 
         if constexpr (S == 2) {
             // Two buffers of wide tiles: barrier kt tells the consumers that tile kt has landed and
             // the producers that tile kt-1 is consumed, whose buffer then takes tile kt+1.
-            fetch_index(rbeg);
-            issue(0, rbeg);
+            issue_first();
             if (1 < nk) fetch_index(rbeg + T::BKS);
             for (int kt = 0; kt < nk; ++kt) {
                 wait_vmcnt<0>();
@@ -2336,8 +2378,12 @@ int xcd_ranges_choice() {
 enum { ORDER_GROUPS = 1, ORDER_DOWN = 2, ORDER_DY1 = 4, ORDER_DX = 8, ORDER_ALL = 15 };
 int tile_order_mask() { return mts_tuning().tile_order_mask; }
 
-constexpr int kCusPerXcd = 32;
 bool tail_split_on() { return mts_tuning().tail_split; }
+
+void set_dividers(RowsParams& p) {
+    p.by_n_tiles.set(p.n_tiles);
+    p.by_group.set(p.n_groups > 1 ? p.n_tiles / p.n_groups : p.n_tiles);   // n_tiles is a multiple of n_groups
+}
 
 template <class T, int EPI>
 dim3 rows_grid(RowsParams& p, int64_t TK) {
@@ -2349,6 +2395,7 @@ dim3 rows_grid(RowsParams& p, int64_t TK) {
     if (p.xcd_ranges && (tile_order_mask() & ORDER_GROUPS))
         while (weight_bytes / p.n_groups > kL2Bytes / 2 && p.n_tiles % (2 * p.n_groups) == 0 && p.n_tiles / (2 * p.n_groups) >= 4)
             p.n_groups *= 2;
+    set_dividers(p);
     const int64_t m_groups = (m_tiles<T>(TK, p.E) + kXcds - 1) / kXcds;
     if (!p.xcd_ranges) p.tail_slots = 0;
     // tiles that are cut in two add at most tail_slots / 2 blocks per XCD; one more block writes the schedule (dO*W2 only)
@@ -2456,6 +2503,8 @@ dim3 dw_grid(DwParams& p, int E, int units) {
     p.E = E;
     p.n_tiles = (p.N + T::BN - 1) / T::BN;
     p.tiles_per_expert = ((p.M + T::BM - 1) / T::BM) * p.n_tiles;
+    p.by_n_tiles.set(p.n_tiles);
+    p.by_tiles.set(p.tiles_per_expert);
     return dim3((unsigned)(((units + kXcds - 1) / kXcds) * kXcds * p.tiles_per_expert));
 }
 
