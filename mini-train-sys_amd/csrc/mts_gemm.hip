@@ -426,11 +426,32 @@ __device__ __forceinline__ void flush_tile(const bf16_t* buf, __amdgpu_buffer_rs
     }
 }
 
+// Routing weight of each of the lane's rows (dY1; SwiGLU when post_act carries the weight), for the epilogue: asked for ahead of the k loop,
+// the two dependent loads of all rows in two batches.
+template <class T, int EPI>
+__device__ __forceinline__ void load_row_weights(const RowsParams& p, int row0, int rend, int wm, float (&srow)[T::MF]) {
+    if constexpr (EPI != EPI_PLAIN) {
+        if (epi_is_dy1(EPI) || p.route_w != nullptr) {
+            int entry[T::MF];
+#pragma unroll
+            for (int mf = 0; mf < T::MF; ++mf) {
+                const int row = row0 + wm * T::WM + mf * 32 + (int)(threadIdx.x % 32);
+                entry[mf] = p.s_scatter[row < rend ? row : rend - 1];   // rows that do not exist are not stored
+            }
+#pragma unroll
+            for (int mf = 0; mf < T::MF; ++mf) srow[mf] = (float)p.route_w[entry[mf]];
+            return;
+        }
+    }
+#pragma unroll
+    for (int mf = 0; mf < T::MF; ++mf) srow[mf] = 1.f;
+}
+
 // PREFETCH (dY1): the pre-activations of slab mf+1 are loaded into registers before the
 // arithmetic of slab mf (32 more registers: for the kernels that have them to spare).
 template <class T, int EPI, bool PREFETCH = false>
 __device__ __forceinline__ void rows_epilogue(const RowsParams& p, f32x16 (&acc)[T::MF][T::NF], bf16_t* smem,
-                                              int row0, int rend, int n0, int wm, int wn) {
+                                              int row0, int rend, int n0, int wm, int wn, const float (&srow)[T::MF]) {
     typedef EpiShape<T, EPI> ES;
     constexpr int COLS = ES::COLS, LDW = ES::LDW;
     constexpr bool DY1 = epi_is_dy1(EPI), WACT = (EPI == EPI_DY1);
@@ -455,9 +476,6 @@ __device__ __forceinline__ void rows_epilogue(const RowsParams& p, f32x16 (&acc)
     const __amdgpu_buffer_rsrc_t rs_pre = make_rsrc(DY1 ? p.pre_act + (int64_t)row0 * 2 * N : nullptr, DY1 ? left * (int64_t)N * 4 : 0);
     const int rrel = rend - row0;   // rows of the tile that exist
 
-    // routing weight of each of the lane's rows (dY1; SwiGLU when post_act carries the weight): two
-    // dependent loads, issued for all rows up front
-    float srow[T::MF];
     // dY1: gate and up pre-activations of one 32 x COLS slab of the wave's tile, row-contiguous
     // 16-byte loads held in registers; the loads of slab mf+1 are issued before the arithmetic of
     // slab mf so that their latency is covered
@@ -474,15 +492,7 @@ __device__ __forceinline__ void rows_epilogue(const RowsParams& p, f32x16 (&acc)
             uv[it] = buf_load16(rs_pre, po == kInvalid ? kInvalid : po + N * 2u);
         }
     };
-    if (DY1 || EPI == EPI_SWIGLU) {
-        const bool weighted = DY1 || p.route_w != nullptr;
-#pragma unroll
-        for (int mf = 0; mf < T::MF; ++mf) {
-            const int row = row0 + wm * T::WM + mf * 32 + ml;
-            srow[mf] = !weighted ? 1.f : (row < rend ? (float)p.route_w[p.s_scatter[row]] : 0.f);
-        }
-        if (DY1 && PREFETCH) load_pre(0);
-    }
+    if (DY1 && PREFETCH) load_pre(0);
 #pragma unroll
     for (int mf = 0; mf < T::MF; ++mf) {
         const int rowg0 = wm * T::WM + mf * 32;   // first row of the slab, counted from row0
@@ -715,6 +725,19 @@ __device__ __forceinline__ bool find_rows_tile(const RowsParams& p, int b, int& 
     return true;
 }
 
+// Source rows of the tile rows `row`: all index loads under one branch (a branch per load, which is what a choice per row compiles to,
+// is a round trip to the cache per load).
+template <int N>
+__device__ __forceinline__ void gather_rows(const int32_t* __restrict__ gather, int row0, int rend, const int (&row)[N], int (&src)[N]) {
+    if (gather) {
+#pragma unroll
+        for (int j = 0; j < N; ++j) src[j] = gather[row[j] < rend ? row[j] : rend - 1];   // keep the load in range
+    } else {
+#pragma unroll
+        for (int j = 0; j < N; ++j) src[j] = row[j] - row0;
+    }
+}
+
 // The answer is the same in every lane, and the compiler is told so behind the search loop: descriptors
 // and LDS addresses built from these values then stay in scalar registers (a buffer instruction whose
 // descriptor sits in vector registers is wrapped in a loop over its distinct values).
@@ -768,13 +791,13 @@ __global__ __launch_bounds__(T::NT) void rows_gemm_kernel(RowsParams p) {
     lb.rsrc = make_rsrc(p.B + (int64_t)e * p.b_rows * p.Kdim, (int64_t)p.b_rows * p.Kdim * 2);
     {
         const int r = threadIdx.x / 8;
+        int row[la.LOADS], src[la.LOADS];
 #pragma unroll
-        for (int q = 0; q < la.LOADS; ++q) {
-            int row = row0 + q * (T::NT / 8) + r;
-            int lrow = row < rend ? row : rend - 1;          // keep the index load in range
-            int src = p.a_gather ? p.a_gather[lrow] : lrow - row0;
-            la.voff[q] = row < rend ? ((uint32_t)src * (uint32_t)p.lda + la.chunk * 8) * 2u : kInvalid;
-        }
+        for (int q = 0; q < la.LOADS; ++q) row[q] = row0 + q * (T::NT / 8) + r;
+        gather_rows(p.a_gather, row0, rend, row, src);
+#pragma unroll
+        for (int q = 0; q < la.LOADS; ++q)
+            la.voff[q] = row[q] < rend ? ((uint32_t)src[q] * (uint32_t)p.lda + la.chunk * 8) * 2u : kInvalid;
 #pragma unroll
         for (int q = 0; q < lb.LOADS; ++q) {
             int br = q * (T::NT / 8) + r;  // row inside the B tile
@@ -793,6 +816,8 @@ __global__ __launch_bounds__(T::NT) void rows_gemm_kernel(RowsParams p) {
 
     const int wave = threadIdx.x / MTS_WAVE, lane = threadIdx.x % MTS_WAVE;
     const int wm = wave / T::WAVES_N, wn = wave % T::WAVES_N;
+    float srow[T::MF];
+    load_row_weights<T, EPI>(p, row0, rend, wm, srow);
     f32x16 acc[T::MF][T::NF];
     zero_acc<T>(acc);
 
@@ -818,7 +843,7 @@ __global__ __launch_bounds__(T::NT) void rows_gemm_kernel(RowsParams p) {
         __syncthreads();
     }
 
-    rows_epilogue<T, EPI>(p, acc, smem, row0, rend, n0, wm, wn);
+    rows_epilogue<T, EPI>(p, acc, smem, row0, rend, n0, wm, wn, srow);
 }
 
 // ---------------------------------------------------------------------------
@@ -912,16 +937,19 @@ __global__ __launch_bounds__(T::NT, T::WAVES_PER_EU) void rows_gemm_ring_kernel(
     const __amdgpu_buffer_rsrc_t rs_b =
         make_rsrc(p.B + (int64_t)e * p.b_rows * p.Kdim, (int64_t)p.b_rows * p.Kdim * 2);
     uint32_t voff_a[T::A_INSTR], voff_b[T::B_INSTR];
+    float srow[T::MF];
     {
         const int slot = lane % T::CHUNKS, rin = lane / T::CHUNKS;
+        int row[T::A_INSTR], src[T::A_INSTR];
+#pragma unroll
+        for (int j = 0; j < T::A_INSTR; ++j) row[j] = row0 + (wave * T::A_INSTR + j) * T::RPI + rin;
+        gather_rows(p.a_gather, row0, rend, row, src);
+        load_row_weights<T, EPI>(p, row0, rend, wm, srow);
 #pragma unroll
         for (int j = 0; j < T::A_INSTR; ++j) {
-            const int tr = (wave * T::A_INSTR + j) * T::RPI + rin;   // row inside the A tile
+            const int tr = row[j] - row0;   // row inside the A tile
             const int chunk = slot ^ (T::CHUNKS == 8 ? (tr >> 1) & 7 : (tr >> 2) & 3);
-            const int row = row0 + tr;
-            const int lrow = row < rend ? row : rend - 1;
-            const int src = p.a_gather ? p.a_gather[lrow] : lrow - row0;
-            voff_a[j] = row < rend ? ((uint32_t)src * (uint32_t)p.lda + chunk * 8) * 2u : kInvalid;
+            voff_a[j] = row[j] < rend ? ((uint32_t)src[j] * (uint32_t)p.lda + chunk * 8) * 2u : kInvalid;
         }
 #pragma unroll
         for (int j = 0; j < T::B_INSTR; ++j) {
@@ -1019,7 +1047,7 @@ __global__ __launch_bounds__(T::NT, T::WAVES_PER_EU) void rows_gemm_ring_kernel(
             abuf = abuf == 2 ? 0 : abuf + 1;
         }
         __builtin_amdgcn_s_barrier();  // every wave is done reading the buffers before they are reused
-        rows_epilogue<T, EPI, true>(p, acc, smem, row0, rend, n0, wm, wn);
+        rows_epilogue<T, EPI, true>(p, acc, smem, row0, rend, n0, wm, wn, srow);
         return;
     }
 #pragma unroll
@@ -1047,7 +1075,7 @@ __global__ __launch_bounds__(T::NT, T::WAVES_PER_EU) void rows_gemm_ring_kernel(
         stage = stage + 1 == S ? 0 : stage + 1;
     }
     __builtin_amdgcn_s_barrier();  // every wave is done reading the ring before it is reused
-    rows_epilogue<T, EPI, true>(p, acc, smem, row0, rend, n0, wm, wn);
+    rows_epilogue<T, EPI, true>(p, acc, smem, row0, rend, n0, wm, wn, srow);
 }
 
 // ---------------------------------------------------------------------------
@@ -1108,15 +1136,10 @@ __device__ __forceinline__ void rows_gemm_ws_tile(const RowsParams& p, bf16_t* s
         const int slot = lane % T::CHUNKS, rin = lane / T::CHUNKS;
         constexpr int CPR_B = T::BN / 8, RPI_B = MTS_WAVE / CPR_B;   // k-major B: chunks per tile row, rows per instruction
         static_assert(!BKM || (EPI != EPI_SWIGLU && T::BKS / RPI_B / T::PRODUCERS == T::B_INSTR), "k-major B loader split");
+        int row[T::A_INSTR], src[T::A_INSTR];
 #pragma unroll
-        for (int j = 0; j < T::A_INSTR; ++j) {
-            const int tr = (pw * T::A_INSTR + j) * T::RPI + rin;
-            const int chunk = slot ^ (T::CHUNKS == 8 ? (tr >> 1) & 7 : (tr >> 2) & 3);
-            const int row = row0 + tr;
-            const int lrow = row < rend ? row : rend - 1;
-            const int src = p.a_gather ? p.a_gather[lrow] : lrow - row0;
-            voff_a[j] = row < rend ? ((uint32_t)src * (uint32_t)p.lda + chunk * 8) * 2u : kInvalid;
-        }
+        for (int j = 0; j < T::A_INSTR; ++j) row[j] = row0 + (pw * T::A_INSTR + j) * T::RPI + rin;
+        gather_rows(p.a_gather, row0, rend, row, src);   // on their way while the weights' offsets are worked out
 #pragma unroll
         for (int j = 0; j < T::B_INSTR; ++j) {
             if constexpr (BKM) {
@@ -1137,6 +1160,14 @@ __device__ __forceinline__ void rows_gemm_ws_tile(const RowsParams& p, bf16_t* s
                 voff_b[j] = (n < p.N) ? ((uint32_t)grow * (uint32_t)p.Kdim + chunk * 8) * 2u : kInvalid;
             }
         }
+        auto offsets_a = [&]() {
+#pragma unroll
+            for (int j = 0; j < T::A_INSTR; ++j) {
+                const int tr = row[j] - row0;
+                const int chunk = slot ^ (T::CHUNKS == 8 ? (tr >> 1) & 7 : (tr >> 2) & 3);
+                voff_a[j] = row[j] < rend ? ((uint32_t)src[j] * (uint32_t)p.lda + chunk * 8) * 2u : kInvalid;
+            }
+        };
         const int k_left = p.Kdim % T::BKS;   // of the last tile, 0: all of it
         auto mask_a = [&](int kt) {
             if (k_left && kt == nk - 1) mask_k_chunks<T::A_INSTR, T::CHUNKS, T::RPI>(voff_a, pw * T::A_INSTR * T::RPI, k_left);
@@ -1147,42 +1178,36 @@ __device__ __forceinline__ void rows_gemm_ws_tile(const RowsParams& p, bf16_t* s
                 else mask_k_chunks<T::B_INSTR, T::CHUNKS, T::RPI>(voff_b, pw * T::B_INSTR * T::RPI, k_left);
             }
         };
-        auto issue = [&](int stage, int kt) {
+        auto tile_a = [&](bf16_t* sa, int kt) {
             mask_a(kt);
-            mask_b(kt);
-            bf16_t* sa = smem + stage * T::STAGE + pw * T::A_INSTR * 512;
-            bf16_t* sb = smem + stage * T::STAGE + T::BM * T::BKS + pw * T::B_INSTR * 512;
-            const int soff = kt * T::BKS * 2;
-            const int soff_b = BKM ? kt * T::BKS * p.N * 2 : soff;   // a k-tile of k-major B is BKS memory rows further
+            const int soff_a = kt * T::BKS * 2;
 #pragma unroll
             for (int j = 0; j < T::A_INSTR; ++j)
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_a, MTS_LDS_PTR(sa + j * 512), 16, (int)voff_a[j], soff, 0, 0);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_a, MTS_LDS_PTR(sa + j * 512), 16, (int)voff_a[j], soff_a, 0, 0);
+        };
+        auto tile_b = [&](bf16_t* sb, int kt) {
+            mask_b(kt);
+            const int soff_b = BKM ? kt * T::BKS * p.N * 2 : kt * T::BKS * 2;   // a k-tile of k-major B is BKS memory rows further
 #pragma unroll
             for (int j = 0; j < T::B_INSTR; ++j)
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_b, MTS_LDS_PTR(sb + j * 512), 16, (int)voff_b[j], soff_b, 0, 0);
+        };
+        auto stage_b = [&](int stage, int kt) { tile_b(smem + stage * T::STAGE + T::BM * T::BKS + pw * T::B_INSTR * 512, kt); };
+        auto stage_a = [&](int stage, int kt) { tile_a(smem + stage * T::STAGE + pw * T::A_INSTR * 512, kt); };
+        auto issue = [&](int stage, int kt) {
+            stage_a(stage, kt);
+            stage_b(stage, kt);
         };
         if constexpr (S == 3) {
             // Three buffers for the activation tile, two for the weight tile.  Barrier kt says that tile kt has landed
             // and that tile kt-1 has been consumed: its weight buffer then takes tile kt+1 and its activation buffer
             // tile kt+2, which has two tiles' time to land.  The activation loads of tile kt+1, the youngest in flight,
             // may still be on their way at barrier kt-1... they are waited for one barrier later.
-            auto issue_a = [&](int buf, int kt) {
-                mask_a(kt);
-                bf16_t* sa = smem + buf * T::BM * T::BKS + pw * T::A_INSTR * 512;
-#pragma unroll
-                for (int j = 0; j < T::A_INSTR; ++j)
-                    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_a, MTS_LDS_PTR(sa + j * 512), 16, (int)voff_a[j], kt * T::BKS * 2, 0, 0);
-            };
-            auto issue_b = [&](int buf, int kt) {
-                mask_b(kt);
-                bf16_t* sb = smem + 3 * T::BM * T::BKS + buf * T::BN * T::BKS + pw * T::B_INSTR * 512;
-                const int soff_b = BKM ? kt * T::BKS * p.N * 2 : kt * T::BKS * 2;   // a k-tile of k-major B is BKS memory rows further
-#pragma unroll
-                for (int j = 0; j < T::B_INSTR; ++j)
-                    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_b, MTS_LDS_PTR(sb + j * 512), 16, (int)voff_b[j], soff_b, 0, 0);
-            };
+            auto issue_a = [&](int buf, int kt) { tile_a(smem + buf * T::BM * T::BKS + pw * T::A_INSTR * 512, kt); };
+            auto issue_b = [&](int buf, int kt) { tile_b(smem + 3 * T::BM * T::BKS + buf * T::BN * T::BKS + pw * T::B_INSTR * 512, kt); };
             // in this order the loads that the first barrier does not wait for are still the youngest
             issue_b(0, 0);
+            offsets_a();
             rows_ready(0);
             issue_a(0, 0);
             if (nk > 1) issue_a(1, 1);
@@ -1201,7 +1226,9 @@ __device__ __forceinline__ void rows_gemm_ws_tile(const RowsParams& p, bf16_t* s
         if constexpr (S == 2) {
             // Two buffers of 64-wide k-tiles (a row contributes a whole 128-byte line per load): barrier kt says
             // that tile kt has landed and that tile kt-1 has been consumed, whose buffer then takes tile kt+1.
-            issue(0, 0);
+            stage_b(0, 0);   // the weights do not wait for the row indices
+            offsets_a();
+            stage_a(0, 0);
             for (int kt = 0; kt < nk; ++kt) {
                 wait_vmcnt<0>();
                 __builtin_amdgcn_s_barrier();
@@ -1213,8 +1240,11 @@ __device__ __forceinline__ void rows_gemm_ws_tile(const RowsParams& p, bf16_t* s
         // Barrier kt tells the consumers that tiles kt and kt+1 have landed (they read the first
         // fragments of tile kt+1 behind the last MFMAs of tile kt) and tells the producers that
         // every consumer is done with tile kt-1, whose stage then takes tile kt-1+S.
+        stage_b(0, 0);
+        offsets_a();
+        stage_a(0, 0);
 #pragma unroll
-        for (int s = 0; s < S; ++s)
+        for (int s = 1; s < S; ++s)
             if (s < nk) issue(s, s);
         int stage = S - 1;   // stage of tile kt-1
         for (int kt = 0; kt < nk; ++kt) {
@@ -1232,6 +1262,8 @@ __device__ __forceinline__ void rows_gemm_ws_tile(const RowsParams& p, bf16_t* s
 
     // -------------------------------- consumer --------------------------------
     const int wm = wave / T::WAVES_N, wn = wave % T::WAVES_N;
+    float srow[T::MF];
+    load_row_weights<T, EPI>(p, row0, rend, wm, srow);
     f32x16 acc[T::MF][T::NF];
     zero_acc<T>(acc);
     FragPipe<T, SWIGLU, T::BKS, BKM> pipe;
@@ -1250,7 +1282,7 @@ __device__ __forceinline__ void rows_gemm_ws_tile(const RowsParams& p, bf16_t* s
             pipe.template step<false>(KSTEPS - 1, acc, cur, cur_b, 0);
         }
         __builtin_amdgcn_s_barrier();       // every wave is done with the buffers before the epilogue reuses them
-        rows_epilogue<T, EPI>(p, acc, smem, row0, rend, n0, wm, wn);
+        rows_epilogue<T, EPI>(p, acc, smem, row0, rend, n0, wm, wn, srow);
         return;
     }
     if constexpr (S == 2) {
@@ -1263,7 +1295,7 @@ __device__ __forceinline__ void rows_gemm_ws_tile(const RowsParams& p, bf16_t* s
             pipe.template step<false>(KSTEPS - 1, acc, cur, 0);
         }
         __builtin_amdgcn_s_barrier();       // every wave is done with the buffers before the epilogue reuses them
-        rows_epilogue<T, EPI>(p, acc, smem, row0, rend, n0, wm, wn);
+        rows_epilogue<T, EPI>(p, acc, smem, row0, rend, n0, wm, wn, srow);
         return;
     }
     __builtin_amdgcn_s_barrier();   // tiles 0 and 1 are visible
@@ -1281,7 +1313,7 @@ __device__ __forceinline__ void rows_gemm_ws_tile(const RowsParams& p, bf16_t* s
         // tile it is the barrier that frees the ring for the epilogue
         __builtin_amdgcn_s_barrier();
     }
-    rows_epilogue<T, EPI>(p, acc, smem, row0, rend, n0, wm, wn);
+    rows_epilogue<T, EPI>(p, acc, smem, row0, rend, n0, wm, wn, srow);
 }
 
 // the work of block `block` of a launch; `smem` holds ws_lds_elems<T, EPI>() elements, 1 KiB aligned.
