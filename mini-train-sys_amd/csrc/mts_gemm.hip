@@ -638,8 +638,7 @@ __device__ __forceinline__ bool find_rows_tile(const RowsParams& p, int b, int& 
     // up to 64 experts: lane l reads expert_start[l] and [l + 1] once, for the count of m-tiles and for the search
     const bool in_regs = p.E <= MTS_WAVE;
     const int lane = threadIdx.x % MTS_WAVE;
-    const int w0 = in_regs && lane < p.E ? p.expert_start[lane] : 0;
-    const int w1 = in_regs && lane < p.E ? p.expert_start[lane + 1] : 0;
+    const int w0 = p.expert_start[min(lane, p.E)], w1 = p.expert_start[min(lane + 1, p.E)];   // equal behind the last expert
     const int wnt = (w1 - w0 + BM - 1) / BM, wincl = wave_scan(wnt);   // in_regs: the lane's m-tiles, and those up to its last one
     const int xcd = b % kXcds;
     int j = b / kXcds;
@@ -656,11 +655,13 @@ __device__ __forceinline__ bool find_rows_tile(const RowsParams& p, int b, int& 
         tile = p.sched[xcd] + k;
     } else if (p.xcd_ranges) {
         // m-tiles of the launch: the first (total % 8) XCDs take one more than the others
-        int all = __builtin_amdgcn_readlane(wincl, MTS_WAVE - 1);
-        if (!in_regs) {
-            for (int le = lane; le < p.E; le += MTS_WAVE) all += (p.expert_start[le + 1] - p.expert_start[le] + BM - 1) / BM;
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) all += __shfl_xor(all, o, MTS_WAVE);
+        int all;
+        if (in_regs) {
+            all = __builtin_amdgcn_readlane(wincl, MTS_WAVE - 1);
+        } else {
+            int mine = 0;
+            for (int le = lane; le < p.E; le += MTS_WAVE) mine += (p.expert_start[le + 1] - p.expert_start[le] + BM - 1) / BM;
+            all = __builtin_amdgcn_readlane(wave_scan(mine), MTS_WAVE - 1);
         }
         const int per = all / kXcds, rem = all % kXcds;
         const int my = per + (xcd < rem ? 1 : 0);
@@ -708,11 +709,11 @@ __device__ __forceinline__ bool find_rows_tile(const RowsParams& p, int b, int& 
             if (hit) {
                 const int w = __ffsll((unsigned long long)hit) - 1;
                 e = e0 + w;
-                row0 = __shfl(s0, w, MTS_WAVE) + (tile - seen - __shfl(incl - nt, w, MTS_WAVE)) * BM;
-                rend = __shfl(s1, w, MTS_WAVE);
+                row0 = __builtin_amdgcn_readlane(s0, w) + (tile - seen - __builtin_amdgcn_readlane(incl - nt, w)) * BM;
+                rend = __builtin_amdgcn_readlane(s1, w);
                 found = true;
             }
-            seen += __shfl(incl, MTS_WAVE - 1, MTS_WAVE);
+            seen += __builtin_amdgcn_readlane(incl, MTS_WAVE - 1);
         }
     }
     if (!found) return false;
