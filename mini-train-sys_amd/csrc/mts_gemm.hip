@@ -426,6 +426,21 @@ __device__ __forceinline__ void flush_tile(const bf16_t* buf, __amdgpu_buffer_rs
     }
 }
 
+// SwiGLU backward of one value: g and u are 16-bit elements of a word (high: the upper ones), a its gradient before the routing weight s
+__device__ __forceinline__ void swiglu_backward(uint32_t gw, uint32_t uw, bool high, float a, float s, float& dg, float& du, float& ds, float* y = nullptr) {
+    const float g = elem_bits_to_f32(high ? gw >> 16 : gw & 0xffffu);
+    const float u = elem_bits_to_f32(high ? uw >> 16 : uw & 0xffffu);
+    const float sig = sigmoidf_(g);
+    const float silu = g * sig;
+    const float y1 = silu * u;
+    ds += a * y1;
+    if (y) *y = y1;
+    const float da = a * s;
+    // d silu/dg * u = (sig + silu (1 - sig)) u = y1 + sig (u - y1)
+    dg = da * __builtin_fmaf(sig, u - y1, y1);
+    du = da * silu;
+}
+
 // Routing weight of each of the lane's rows (dY1; SwiGLU when post_act carries the weight), for the epilogue: asked for ahead of the k loop,
 // the two dependent loads of all rows in two batches.
 template <class T, int EPI>
@@ -568,19 +583,9 @@ __device__ __forceinline__ void rows_epilogue(const RowsParams& p, f32x16 (&acc)
                     float wa[4], dg[4], du[4];
 #pragma unroll
                     for (int q = 0; q < 4; ++q) {
-                        const uint32_t gw = q < 2 ? gr.x : gr.y, uw = q < 2 ? ur.x : ur.y;
-                        const float g = elem_bits_to_f32((q & 1) ? gw >> 16 : gw & 0xffffu);
-                        const float u = elem_bits_to_f32((q & 1) ? uw >> 16 : uw & 0xffffu);
-                        const float a = acc[mf][nf][4 * j + q];
-                        const float sig = sigmoidf_(g);
-                        const float silu = g * sig;
-                        const float y1 = silu * u;
-                        dsp += a * y1;
+                        float y1;
+                        swiglu_backward(q < 2 ? gr.x : gr.y, q < 2 ? ur.x : ur.y, q & 1, acc[mf][nf][4 * j + q], s, dg[q], du[q], dsp, &y1);
                         wa[q] = s * y1;
-                        const float da = a * s;
-                        // d silu/dg * u = (sig + silu (1 - sig)) u = y1 + sig (u - y1)
-                        dg[q] = da * __builtin_fmaf(sig, u - y1, y1);
-                        du[q] = da * silu;
                     }
                     if (WACT) stage4(buf0 + o, wa[0], wa[1], wa[2], wa[3]);
                     stage4(bufg + o, dg[0], dg[1], dg[2], dg[3]);
@@ -1113,6 +1118,83 @@ constexpr int ws_lds_elems() {
     return T::LDS_ELEMS > EpiShape<T, EPI>::ELEMS ? T::LDS_ELEMS : EpiShape<T, EPI>::ELEMS;
 }
 
+// ---------------------------------------------------------------------------
+// dO*W2 on two buffers of 64-wide k-tiles: the pre-activations reach the epilogue through the buffers that the k loop leaves free,
+// loaded by the producer waves, slab by slab (32 rows of every consumer wave's tile: 64 KiB of gate and up for eight waves, a buffer).
+// Slab 0 lands while the last k-tile is multiplied, slab m + 1 while slab m is worked on; d_gate and d_up replace the values they come from and
+// leave in whole lines.  (Loaded by the consumer waves themselves, whose registers hold no more than a slab in flight beside the
+// accumulators, every slab waits for memory.)
+// A slab of a wave: gate [32][64], then up; the 16-byte chunks of a row are dealt as in a k-tile of that width.
+// ---------------------------------------------------------------------------
+template <class T>
+struct PreSlabs {
+    static constexpr int PER_WAVE = 2 * 32 * 64, SIZE = T::NWAVES * PER_WAVE;   // elements
+    // a slab of every wave fits the buffer that the last k-tile is not in; else (tiles of half the height, whose block has the LDS of a whole
+    // one) the slabs wait for the end of the k loop
+    static constexpr bool EARLY = SIZE <= T::STAGE;
+    static_assert(T::WN == 64, "a wave's slab is 64 columns wide");
+    __device__ __forceinline__ static bf16_t* place(bf16_t* smem, int nk, int mf) { return EARLY ? smem + ((nk + mf) & 1) * T::STAGE : smem + (mf & 1) * SIZE; }
+    __device__ __forceinline__ static int at(int r, int chunk) { return r * 64 + ((chunk ^ (r >> 1 & 7)) << 3); }
+};
+
+// the part of producer wave pw in slab mf
+template <class T>
+__device__ __forceinline__ void load_pre_slab(const RowsParams& p, __amdgpu_buffer_rsrc_t rs_pre, bf16_t* buf, int mf, int rrel, int n0, int pw) {
+    constexpr int WAVES = T::NWAVES / T::PRODUCERS;
+    const int lane = threadIdx.x % MTS_WAVE, rin = lane / 8, slot = lane % 8;
+    const uint32_t N = (uint32_t)p.N;
+#pragma unroll
+    for (int q = 0; q < WAVES; ++q) {
+        const int w = pw * WAVES + q, first = w / T::WAVES_N * T::WM + mf * 32, ncol0 = n0 + w % T::WAVES_N * 64;
+        bf16_t* dst = buf + w * PreSlabs<T>::PER_WAVE;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int r = i * 8 + rin, col = ncol0 + ((slot ^ (r >> 1 & 7)) << 3);
+            // columns behind the last one read zeros, and so do rows behind the expert's end: the descriptor ends there
+            const uint32_t off = first + r < rrel && col < p.N ? ((uint32_t)(first + r) * 2u * N + (uint32_t)col) * 2u : kInvalid;
+            const uint32_t off_up = off == kInvalid ? kInvalid : off + N * 2u;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_pre, MTS_LDS_PTR(dst + i * 512), 16, (int)off, 0, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_pre, MTS_LDS_PTR(dst + 2048 + i * 512), 16, (int)off_up, 0, 0, 0);
+        }
+    }
+}
+
+// slab mf of consumer wave (wm, wn): `buf` holds it
+template <class T>
+__device__ __forceinline__ void dy1_slab(const RowsParams& p, f32x16 (&acc)[T::NF], __amdgpu_buffer_rsrc_t rs_c, bf16_t* buf, int mf, int row0, int rend,
+                                         int n0, int wm, int wn, float s) {
+    const int lane = threadIdx.x % MTS_WAVE, ml = lane % 32, half = lane / 32;
+    bf16_t* gate = buf + (wm * T::WAVES_N + wn) * PreSlabs<T>::PER_WAVE;
+    bf16_t* up = gate + 2048;
+    float dsp = 0.f;
+#pragma unroll
+    for (int nf = 0; nf < T::NF; ++nf)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int o = PreSlabs<T>::at(ml, nf * 4 + j) + 4 * half;
+            const uint2 gr = *reinterpret_cast<const uint2*>(gate + o), ur = *reinterpret_cast<const uint2*>(up + o);
+            float dg[4], du[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) swiglu_backward(q < 2 ? gr.x : gr.y, q < 2 ? ur.x : ur.y, q & 1, acc[nf][4 * j + q], s, dg[q], du[q], dsp);
+            stage4(gate + o, dg[0], dg[1], dg[2], dg[3]);
+            stage4(up + o, du[0], du[1], du[2], du[3]);
+        }
+    dsp += __shfl_xor(dsp, 32, MTS_WAVE);
+    const int first = wm * T::WM + mf * 32, ncol0 = n0 + wn * 64;
+    if (lane < 32 && row0 + first + ml < rend && ncol0 / 64 < p.np) p.ds_part[(int64_t)(row0 + first + ml) * p.np + ncol0 / 64] = dsp;
+    const int c = lane % 8;
+    const uint32_t N = (uint32_t)p.N;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int r = i * 8 + lane / 8;
+        const u32x4 g16 = *reinterpret_cast<const u32x4*>(gate + PreSlabs<T>::at(r, c)), u16 = *reinterpret_cast<const u32x4*>(up + PreSlabs<T>::at(r, c));
+        const bool ok = row0 + first + r < rend && ncol0 + c * 8 < p.N;
+        const uint32_t off = ok ? ((uint32_t)(first + r) * 2u * N + (uint32_t)(ncol0 + c * 8)) * 2u : kInvalid;
+        __builtin_amdgcn_raw_buffer_store_b128(g16, rs_c, (int)off, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b128(u16, rs_c, (int)(ok ? off + N * 2u : kInvalid), 0, 0);
+    }
+}
+
 // one output tile: rows [row0, rend) of expert e (at most T::BM of them), column tile ntile
 // `rows_ready` runs in the producer waves of a tile on three activation buffers, behind the first loads of the weights and
 // in front of the first loads of the activation rows (a launch whose rows are written by other blocks of the same launch).
@@ -1121,6 +1203,7 @@ __device__ __forceinline__ void rows_gemm_ws_tile(const RowsParams& p, bf16_t* s
                                                   RowsReady rows_ready = RowsReady()) {
     constexpr bool SWIGLU = (EPI == EPI_SWIGLU);
     constexpr int S = T::STAGES, L = T::A_INSTR + T::B_INSTR;
+    constexpr bool DY_PIPE = EPI == EPI_DY1N && S == 2;
     const int n0 = ntile * (SWIGLU ? T::BN / 2 : T::BN);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / MTS_WAVE), lane = threadIdx.x % MTS_WAVE;
     const int nk = (p.Kdim + T::BKS - 1) / T::BKS;
@@ -1235,6 +1318,17 @@ __device__ __forceinline__ void rows_gemm_ws_tile(const RowsParams& p, bf16_t* s
                 __builtin_amdgcn_s_barrier();
                 if (kt + 1 < nk) issue((kt + 1) & 1, kt + 1);
             }
+            if constexpr (DY_PIPE) {
+                const __amdgpu_buffer_rsrc_t rs_pre = make_rsrc(p.pre_act + (int64_t)row0 * 2 * p.N, (int64_t)(rend - row0) * p.N * 4);
+                if constexpr (!PreSlabs<T>::EARLY) __builtin_amdgcn_s_barrier();
+#pragma unroll
+                for (int mf = 0; mf < T::MF; ++mf) {
+                    load_pre_slab<T>(p, rs_pre, PreSlabs<T>::place(smem, nk, mf), mf, rend - row0, n0, pw);
+                    wait_vmcnt<0>();
+                    __builtin_amdgcn_s_barrier();   // slab mf has landed, slab mf-1 (before slab 0: the last k-tile) is done with
+                }
+                return;
+            }
             __builtin_amdgcn_s_barrier();       // matches the consumers' barrier behind the last tile
             return;
         }
@@ -1295,6 +1389,17 @@ __device__ __forceinline__ void rows_gemm_ws_tile(const RowsParams& p, bf16_t* s
             for (int ks = 0; ks < KSTEPS - 1; ++ks) pipe.step(ks, acc, cur, ks + 1);
             pipe.template step<false>(KSTEPS - 1, acc, cur, 0);
         }
+        if constexpr (DY_PIPE) {
+            const __amdgpu_buffer_rsrc_t rs_c = make_rsrc(p.C + (int64_t)row0 * 2 * p.N, (int64_t)(rend - row0) * p.N * 4);
+            if constexpr (!PreSlabs<T>::EARLY) __builtin_amdgcn_s_barrier();
+#pragma unroll
+            for (int mf = 0; mf < T::MF; ++mf) {
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // what this wave read of the buffer it leaves is in its registers
+                __builtin_amdgcn_s_barrier();
+                dy1_slab<T>(p, acc[mf], rs_c, PreSlabs<T>::place(smem, nk, mf), mf, row0, rend, n0, wm, wn, srow[mf]);
+            }
+            return;
+        }
         __builtin_amdgcn_s_barrier();       // every wave is done with the buffers before the epilogue reuses them
         rows_epilogue<T, EPI>(p, acc, smem, row0, rend, n0, wm, wn, srow);
         return;
@@ -1333,6 +1438,7 @@ template <class T, int EPI, bool BKM, class TH = T>
 __device__ __forceinline__ void rows_gemm_ws_block(const RowsParams& p, bf16_t* smem, int block) {
     static_assert(TH::NT == T::NT && TH::BN == T::BN && (TH::BM == T::BM || 2 * TH::BM == T::BM), "half tile shape");
     static_assert(ws_lds_elems<TH, EPI>() <= ws_lds_elems<T, EPI>(), "the half tile fits the same LDS");
+    static_assert(EPI != EPI_DY1N || T::STAGES != 2 || 2 * TH::NWAVES * 4096 <= ws_lds_elems<T, EPI>(), "two slabs of the half tile fit it");
     int e, row0, rend, ntile, parts;
     if (!locate_rows_tile<T::BM>(p, block, e, row0, rend, ntile, parts)) return;
     rows_gemm_ws_run<T, EPI, BKM, TH>(p, smem, e, row0, rend, ntile, parts);
@@ -2359,7 +2465,7 @@ typedef MtsGemmKind Kind;
 constexpr Kind K_GATEUP = MTS_K_GATEUP, K_DOWN = MTS_K_DOWN, K_DY1 = MTS_K_DY1, K_DX = MTS_K_DX, K_DW2 = MTS_K_DW2, K_DW1 = MTS_K_DW1;
 constexpr int K_COUNT = MTS_K_COUNT;
 // rows_gemm: 0 StagedSmall, 1 RingTwoPerCu, 2 WsLarge, 3 RingThreePerCu (dY1 without the weighted_act output
-// only), 4 WsWide (no SwiGLU backward: gate/up, down and dX; dY1 falls back to 2), 5 WsSmall (few rows: small_tiles_pay);
+// only), 4 WsWide (dY1 that writes weighted_act or reads transposed weights falls back to 2), 5 WsSmall (few rows: small_tiles_pay);
 // dw_gemm: 0 StagedSmall, 2 DwWsLarge, 4 DwWsWide (the same output tiles, so one workspace layout).
 // Defaults are the choices with the shortest LAYER STEP measured on the 24576-token, 768/1024, 8-expert layer.
 // The chip runs this step against its power limit, so a kernel's own duration is not the whole story: what
@@ -2469,12 +2575,17 @@ int launch_rows_any(int kind, RowsParams p, int64_t TK, hipStream_t s, bool b_km
     if (!tile_forced(kind) && small_tiles_pay(kind, TK, p.E, p.N)) choice = 5;
     // three blocks per CU hold two stages each: for short reductions, and for the epilogue that fits beside them
     if (choice == 3 && (EPI != EPI_DY1N || !b_kmajor)) choice = 1;
-    // longer ones go to the specialised waves, whose k-loop is the better one and whose epilogue then weighs less (the operator,
-    // forward and backward, on two blocks per CU / on these, us: 4096 tokens 4096/14336 9464 / 9147, 16 384 tokens 2048/2048 2471 / 2437,
-    // 6000 tokens 2048/1024 580 / 567; 1024/2048 668 / 638 to 646 / 652 in turn, 24 576 tokens of 768/1024 855 / 873)
-    if (choice == 3 && !tile_forced(kind) && p.Kdim > 1024) choice = 2;
+    // longer ones, and launches of more than about a round of 256 x 256 tiles, go to the specialised waves: a third less L2 traffic per product and
+    // pre-activations that land during the k loop.  The kernel, three blocks per CU / this, us (tiles): 24 576 tokens of 768/1024 150.0 / 140.6
+    // (800), 8192 of 1024/512 with 64 experts, top-4, 64.0 / 54.4 (320), 24 576 of 2048/1024 266 / 226 (WsLarge 240), 5003 of 768/1024 31.7 / 33.2
+    // (172), 6001 of 1000/1368 with even experts 61.5 / 66.0 (306), uneven ones the operator's call 553 / 533.  In the layer step, which the power limit
+    // holds, what it gains is 1 % at 20 000 and 40 000 tokens and nothing at 24 576.
+    if (choice == 3 && !tile_forced(kind)) {
+        const int64_t tiles = (TK / WsWide::BM + p.E / 2) * ((p.N + WsWide::BN - 1) / WsWide::BN);
+        if (p.Kdim > 1024 || tiles >= 300) choice = 4;
+    }
     // the 64-wide variant exists for the GEMMs with a plain or SwiGLU epilogue
-    if (choice == 4 && epi_is_dy1(EPI)) choice = 2;
+    if (choice == 4 && epi_is_dy1(EPI) && (EPI != EPI_DY1N || !b_kmajor)) choice = 2;
     if (choice >= 1 && !rows_pipelined(p.Kdim)) choice = 0;
     if (b_kmajor && (choice == 0 || EPI == EPI_SWIGLU)) return MTS_ERR_SHAPE;
     if (choice == 3) {
@@ -2499,7 +2610,11 @@ int launch_rows_any(int kind, RowsParams p, int64_t TK, hipStream_t s, bool b_km
             rows_gemm_ring_kernel<RingTwoPerCu, EPI><<<grid, RingTwoPerCu::NT, 0, s>>>(p);
         }
     } else if (choice == 4) {
-        if constexpr (!epi_is_dy1(EPI)) {
+        if constexpr (EPI == EPI_DY1N) {
+            if (tail_split_on()) p.tail_slots = kCusPerXcd;
+            const dim3 grid = rows_grid<WsWide, EPI>(p, TK);
+            rows_gemm_ws_kernel<WsWide, EPI, true, WsWideHalf><<<grid, WsWide::NT, 0, s>>>(p);
+        } else if constexpr (!epi_is_dy1(EPI)) {
             // The tiles are few and long: 6.25 (gate/up) and 2.34 (down) per CU at the 24576-token layer.  The ones
             // behind the last whole round of an XCD's 32 CUs are cut in two where they would leave more than half
             // of the CUs idle (gate/up -3 %, down -4 %).

@@ -14,6 +14,8 @@ pytestmark = pytest.mark.gpu
     (257, 320, 3, 680, 1),      # ragged I only
     (129, 712, 5, 128, 3),      # ragged H only, 2I the shortest that is taken
     (64, 1080, 4, 1288, 2),     # a reduction of more than 1024 in dO*W2 (two blocks per CU)
+    (4500, 1096, 8, 520, 2),    # dO*W2 on 256 x 256 tiles, every tile cut in two, rows, columns and k-tiles with a remainder
+    (12000, 1032, 4, 264, 2),   # the same, whole tiles
     (1, 504, 2, 504, 1)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_ragged_widths(T, H, E, I, K, dtype):

@@ -23,6 +23,8 @@ CONFIGURATIONS = {
     "staged kernels, separate launches": dict(MTS_TILE_GATEUP="0", MTS_TILE_DOWN="0", MTS_TILE_DY1="0", MTS_TILE_DX="0",
                                               MTS_TILE_DW1="0", MTS_TILE_DW2="0", MTS_NO_JOINT_BWD="1", MTS_NO_OVERLAP="1"),
     "specialised waves for dY1, round-robin tiles": dict(MTS_TILE_DY1="2", MTS_XCD_RANGES="0", MTS_NO_TILE_ORDER="1"),
+    "64-wide k-tiles for dY1": dict(MTS_TILE_DY1="4"),
+    "64-wide k-tiles for dY1, every tile whole": dict(MTS_TILE_DY1="4", MTS_NO_TAIL_SPLIT="1"),
     "four stages of 32-wide k-tiles, separate launches": dict(MTS_TILE_GATEUP="2", MTS_TILE_DOWN="2", MTS_TILE_DX="2",
                                                               MTS_TILE_DW1="2", MTS_TILE_DW2="2", MTS_NO_JOINT_BWD="1"),
     "64-wide k-tiles for dX and the weight gradients on their own, every tile whole": dict(MTS_NO_JOINT_BWD="1",
