@@ -202,7 +202,7 @@ __global__ __launch_bounds__(kThreads, 3) void attention_fwd_kernel(AttnArgs<ET>
             float hi = s[0][0];
 #pragma unroll
             for (int i = 0; i < 16; ++i) hi = fmaxf(hi, fmaxf(s[0][i], s[1][i]));
-            hi = fmaxf(hi, __shfl_xor(hi, 32, MTS_WAVE));
+            hi = lane_pair<32>(hi, [](float a, float b) { return fmaxf(a, b); });
             if (__any(hi > top)) {
                 const float next = fmaxf(top, hi), keep = next == top ? 1.f : __builtin_amdgcn_exp2f((top - next) * sc);
                 top = next;
@@ -235,7 +235,7 @@ __global__ __launch_bounds__(kThreads, 3) void attention_fwd_kernel(AttnArgs<ET>
         }
         __syncthreads();
     }
-    sum += __shfl_xor(sum, 32, MTS_WAVE);
+    sum = lane_pair<32>(sum, LaneSum());
     if (row >= S) return;
     store_row(a.out.row0(at.bh, a.heads) + row * a.out.s, acc, 1.f / sum);
     if (half == 0) a.lse[at.bh * S + row] = top * sc + log2f(sum);
@@ -263,7 +263,7 @@ __global__ __launch_bounds__(kThreads, 2) void attention_dq_kernel(AttnArgs<ET> 
         for (int ks = 0; ks < 4; ++ks)
 #pragma unroll
             for (int j = 0; j < 8; ++j) delta += (float)o[ks][j] * (float)g[ks][j];
-        delta += __shfl_xor(delta, 32, MTS_WAVE);
+        delta = lane_pair<32>(delta, LaneSum());
         if (half == 0 && row < S) a.delta[at.bh * S + row] = delta;
     }
     const float sc = a.scale * kLog2e, lse = a.lse[at.bh * S + from];

@@ -333,8 +333,7 @@ __global__ __launch_bounds__(kSelThreads) void capacity_compact_kernel(
     __shared__ int32_t in_front[kSelWaves];
     const int e = blockIdx.x, tid = threadIdx.x, n = counts[e], first = expert_start[e];
     int32_t v = tid < e ? accepted_of(counts[tid], capacity) : 0;   // at most 1024 experts: one per thread
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, MTS_WAVE);
+    v = wave_sum(v);
     if (tid % MTS_WAVE == 0) in_front[tid / MTS_WAVE] = v;
     __syncthreads();
     int32_t kept_first = 0;
@@ -378,11 +377,8 @@ __global__ __launch_bounds__(kWeightThreads) void capacity_weights_kernel(const 
         dead += a == 0.f ? 1.f : 0.f;
     }
     sum = wave_sum(sum), dead = wave_sum(dead);
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        most = fmaxf(most, __shfl_xor(most, o, MTS_WAVE));
-        least = fminf(least, __shfl_xor(least, o, MTS_WAVE));
-    }
+    most = lane_reduce<32, 1>(most, [](float a, float b) { return fmaxf(a, b); });
+    least = lane_reduce<32, 1>(least, [](float a, float b) { return fminf(a, b); });
     const float mean = sum / routes / scale;
     float dev = 0.f;
     for (int e = lane; e < E; e += MTS_WAVE) {

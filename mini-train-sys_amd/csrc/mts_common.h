@@ -29,9 +29,70 @@ __device__ __forceinline__ float bf16_bits_to_f32(uint32_t bits16) {
     return __uint_as_float(bits16 << 16);
 }
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, MTS_WAVE);
+// The value of lane ^ O, on the vector unit (a shuffle goes through LDS: a hundred cycles of latency); O < 16.
+template <int O>
+__device__ __forceinline__ uint32_t lane_xor_bits(uint32_t v) {
+    static_assert(O == 8 || O == 4 || O == 2 || O == 1, "within a row of 16 lanes");
+    if constexpr (O == 8) return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x128, 0xf, 0xf, true);   // rotate the row by 8
+    else if constexpr (O == 4) {   // lanes 0..3 and 8..11 of a row from four lanes up, the others from four lanes down
+        const int up = __builtin_amdgcn_update_dpp((int)v, (int)v, 0x104, 0xf, 0x5, false);
+        return (uint32_t)__builtin_amdgcn_update_dpp(up, (int)v, 0x114, 0xf, 0xa, false);
+    } else if constexpr (O == 2) return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4e, 0xf, 0xf, true);
+    else return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xb1, 0xf, 0xf, true);
+}
+
+// op(value of this lane, value of lane ^ O) for a commutative op
+template <int O, typename V, class Op>
+__device__ __forceinline__ V lane_pair(V v, Op op) {
+    static_assert(sizeof(V) == 4, "one register");
+    const uint32_t bits = __builtin_bit_cast(uint32_t, v);
+    if constexpr (O == 32) {
+        const auto r = __builtin_amdgcn_permlane32_swap(bits, bits, false, false);
+        return op(__builtin_bit_cast(V, (uint32_t)r[0]), __builtin_bit_cast(V, (uint32_t)r[1]));
+    } else if constexpr (O == 16) {
+        const auto r = __builtin_amdgcn_permlane16_swap(bits, bits, false, false);
+        return op(__builtin_bit_cast(V, (uint32_t)r[0]), __builtin_bit_cast(V, (uint32_t)r[1]));
+    } else return op(v, __builtin_bit_cast(V, lane_xor_bits<O>(bits)));
+}
+
+// the value of lane ^ O
+template <int O, typename V>
+__device__ __forceinline__ V lane_other(V v) {
+    static_assert(sizeof(V) == 4, "one register");
+    const uint32_t bits = __builtin_bit_cast(uint32_t, v);
+    if constexpr (O >= 16) {   // the swap leaves the lower lanes' values in the first register and the upper ones' in the second
+        const bool upper = threadIdx.x & O;
+        if constexpr (O == 32) {
+            const auto r = __builtin_amdgcn_permlane32_swap(bits, bits, false, false);
+            return __builtin_bit_cast(V, (uint32_t)(upper ? r[0] : r[1]));
+        } else {
+            const auto r = __builtin_amdgcn_permlane16_swap(bits, bits, false, false);
+            return __builtin_bit_cast(V, (uint32_t)(upper ? r[0] : r[1]));
+        }
+    } else return __builtin_bit_cast(V, lane_xor_bits<O>(bits));
+}
+
+// op over lanes that agree but for the bits from `LOW` up to FROM, widest distance first
+template <int FROM, int LOW, typename V, class Op>
+__device__ __forceinline__ V lane_reduce(V v, Op op) {
+    if constexpr (FROM >= LOW && FROM > 0) return lane_reduce<FROM / 2, LOW>(lane_pair<FROM>(v, op), op);
+    else return v;
+}
+struct LaneSum {
+    template <typename V>
+    __device__ __forceinline__ V operator()(V a, V b) const { return a + b; }
+};
+__device__ __forceinline__ float wave_sum(float v) { return lane_reduce<32, 1>(v, LaneSum()); }
+__device__ __forceinline__ int32_t wave_sum(int32_t v) { return lane_reduce<32, 1>(v, LaneSum()); }
+
+// inclusive sum over the wave's lanes
+__device__ __forceinline__ int wave_scan(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);   // one lane up within a row of 16, then 2, 4, 8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);   // the last lane of rows 0 and 2 to rows 1 and 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);   // lane 31 to rows 2 and 3
     return v;
 }
 

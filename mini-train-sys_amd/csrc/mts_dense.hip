@@ -359,6 +359,14 @@ struct MaxSum {
     }
 };
 
+template <int O, class Acc>
+__device__ __forceinline__ void merge_lanes(Acc& acc) {
+    if constexpr (O > 0) {
+        acc.merge(lane_other<O>(acc.m), lane_other<O>(acc.s));
+        merge_lanes<O / 2>(acc);
+    }
+}
+
 template <typename ET>
 __global__ __launch_bounds__(kCeThreads) void cross_entropy_fwd_kernel(const ET* __restrict__ logits, const int64_t* __restrict__ targets, int V,
                                                                        int64_t ignore, float* __restrict__ row_max, float* __restrict__ row_log_sum,
@@ -412,8 +420,7 @@ __global__ __launch_bounds__(kCeThreads) void cross_entropy_fwd_kernel(const ET*
         take(x);
     }
     nan |= acc.s != acc.s;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) acc.merge(__shfl_xor(acc.m, o, MTS_WAVE), __shfl_xor(acc.s, o, MTS_WAVE));
+    merge_lanes<32>(acc);
     __shared__ float ms[kCeThreads / MTS_WAVE], ss[kCeThreads / MTS_WAVE];
     const int any_nan = __syncthreads_or(nan);
     if (threadIdx.x % MTS_WAVE == 0) {

@@ -79,21 +79,16 @@ __device__ __forceinline__ bool find_tile(const int32_t* start, int E, int m, in
         const int e = min(e0 + lane, E - 1);
         const int s = start[e], t = e0 + lane < E ? start[e + 1] : s;
         const int own = (t - s + rows - 1) / rows;
-        int upto = own;
-#pragma unroll
-        for (int o = 1; o < MTS_WAVE; o <<= 1) {
-            const int v = __shfl_up(upto, o, MTS_WAVE);
-            if (lane >= o) upto += v;
-        }
+        const int upto = wave_scan(own);
         const uint64_t behind = __ballot(upto > m);
         if (behind) {
             const int l = __ffsll((unsigned long long)behind) - 1;
-            expert = __builtin_amdgcn_readfirstlane(e0 + l);
-            row0 = __builtin_amdgcn_readfirstlane(__shfl(s, l, MTS_WAVE) + (m - __shfl(upto - own, l, MTS_WAVE)) * rows);
-            end = __builtin_amdgcn_readfirstlane(__shfl(t, l, MTS_WAVE));
+            expert = e0 + l;
+            row0 = __builtin_amdgcn_readlane(s, l) + (m - __builtin_amdgcn_readlane(upto - own, l)) * rows;
+            end = __builtin_amdgcn_readlane(t, l);
             return true;
         }
-        m -= __shfl(upto, MTS_WAVE - 1, MTS_WAVE);
+        m -= __builtin_amdgcn_readlane(upto, MTS_WAVE - 1);
     }
     return false;
 }

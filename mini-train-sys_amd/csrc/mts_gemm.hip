@@ -128,17 +128,6 @@ struct Divider {
     }
 };
 
-// inclusive sum over the wave's lanes, on the vector unit alone (a shuffle goes through LDS: a hundred cycles for each of six)
-__device__ __forceinline__ int wave_scan(int v) {
-    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);   // one lane up within a row of 16, then 2, 4, 8
-    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);   // the last lane of rows 0 and 2 to rows 1 and 3
-    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);   // lane 31 to rows 2 and 3
-    return v;
-}
-
 // EPI_DY1N: the dO*W2 epilogue without the weighted_act output (the caller kept the forward
 // pass's post_act, which already carries the routing weight)
 enum Epilogue { EPI_PLAIN = 0, EPI_SWIGLU = 1, EPI_DY1 = 2, EPI_DY1N = 3 };
@@ -591,7 +580,7 @@ __device__ __forceinline__ void rows_epilogue(const RowsParams& p, f32x16 (&acc)
                     stage4(bufg + o, dg[0], dg[1], dg[2], dg[3]);
                     stage4(bufu + o, du[0], du[1], du[2], du[3]);
                 }
-            dsp += __shfl_xor(dsp, 32, MTS_WAVE);
+            dsp = lane_pair<32>(dsp, LaneSum());
             // one partial per 64 output columns, whatever the tile shape: a wave that
             // covers 128 columns writes its sum to the first slot and 0 to the second
             if (rok && lane < 32) {
@@ -1179,7 +1168,7 @@ __device__ __forceinline__ void dy1_slab(const RowsParams& p, f32x16 (&acc)[T::N
             stage4(gate + o, dg[0], dg[1], dg[2], dg[3]);
             stage4(up + o, du[0], du[1], du[2], du[3]);
         }
-    dsp += __shfl_xor(dsp, 32, MTS_WAVE);
+    dsp = lane_pair<32>(dsp, LaneSum());
     const int first = wm * T::WM + mf * 32, ncol0 = n0 + wn * 64;
     if (lane < 32 && row0 + first + ml < rend && ncol0 / 64 < p.np) p.ds_part[(int64_t)(row0 + first + ml) * p.np + ncol0 / 64] = dsp;
     const int c = lane % 8;
@@ -1711,8 +1700,7 @@ __device__ __forceinline__ void dw_chunk_sum_expert(const DwParams& p, int e) {
         const int c = dw_chunks(p, p.expert_start[le + 1] - p.expert_start[le], share);
         before += c > 1 ? c : 0;
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) before += __shfl_xor(before, o, MTS_WAVE);
+    before = wave_sum(before);
     constexpr int PER_TILE = BM * BN / 4;
     const int64_t tile_stride = (int64_t)BM * BN;
     const int64_t items = (int64_t)p.tiles_per_expert * PER_TILE;

@@ -64,20 +64,15 @@ __device__ __forceinline__ int find_m_tile(const int32_t* __restrict__ expert_st
         const int e = e0 + lane;
         const int s0 = e < E ? expert_start[e] : 0, s1 = e < E ? expert_start[e + 1] : 0;
         const int nt = (s1 - s0 + BM - 1) / BM;
-        int upto = nt;
-#pragma unroll
-        for (int o = 1; o < MTS_WAVE; o <<= 1) {
-            const int t = __shfl_up(upto, o, MTS_WAVE);
-            if (lane >= o) upto += t;
-        }
+        const int upto = wave_scan(nt);
         const uint64_t mine = __ballot(tile >= seen + upto - nt && tile < seen + upto);
         if (mine) {
             const int l = __ffsll((unsigned long long)mine) - 1;
             e_out = e0 + l;
-            row0 = __shfl(s0, l, MTS_WAVE) + (tile - seen - __shfl(upto - nt, l, MTS_WAVE)) * BM;
-            rend = __shfl(s1, l, MTS_WAVE);
+            row0 = __builtin_amdgcn_readlane(s0, l) + (tile - seen - __builtin_amdgcn_readlane(upto - nt, l)) * BM;
+            rend = __builtin_amdgcn_readlane(s1, l);
         }
-        seen += __shfl(upto, MTS_WAVE - 1, MTS_WAVE);
+        seen += __builtin_amdgcn_readlane(upto, MTS_WAVE - 1);
     }
     return seen;
 }

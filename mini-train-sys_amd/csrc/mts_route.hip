@@ -77,14 +77,9 @@ __device__ __forceinline__ void route_scan_block(
         for (int64_t c0 = 0; c0 < n_chunks; c0 += MTS_WAVE) {
             int64_t c = c0 + lane;
             int32_t v = (c < n_chunks) ? cnt[c * E + e] : 0;
-            int32_t incl = v;
-#pragma unroll
-            for (int o = 1; o < MTS_WAVE; o <<= 1) {
-                int32_t up = __shfl_up(incl, o, MTS_WAVE);
-                if (lane >= o) incl += up;
-            }
+            const int32_t incl = wave_scan(v);
             if (c < n_chunks) cnt[c * E + e] = carry + incl - v;
-            carry += __shfl(incl, MTS_WAVE - 1, MTS_WAVE);
+            carry += __builtin_amdgcn_readlane(incl, MTS_WAVE - 1);
         }
         if (lane == 0) total[e] = carry;
     }
@@ -95,24 +90,15 @@ __device__ __forceinline__ void route_scan_block(
             int e = eb + lane;
             int32_t v = (e < E) ? total[e] : 0;
             int32_t tv = (v + block_m - 1) / block_m;
-            int32_t incl = v, tincl = tv;
-#pragma unroll
-            for (int o = 1; o < MTS_WAVE; o <<= 1) {
-                int32_t up = __shfl_up(incl, o, MTS_WAVE);
-                int32_t tup = __shfl_up(tincl, o, MTS_WAVE);
-                if (lane >= o) {
-                    incl += up;
-                    tincl += tup;
-                }
-            }
+            const int32_t incl = wave_scan(v), tincl = wave_scan(tv);
             if (e < E) {
                 start[e] = carry + incl - v;
                 tile_off[e] = tcarry + tincl - tv;
                 counts[e] = v;
                 expert_start[e] = carry + incl - v;
             }
-            carry += __shfl(incl, MTS_WAVE - 1, MTS_WAVE);
-            tcarry += __shfl(tincl, MTS_WAVE - 1, MTS_WAVE);
+            carry += __builtin_amdgcn_readlane(incl, MTS_WAVE - 1);
+            tcarry += __builtin_amdgcn_readlane(tincl, MTS_WAVE - 1);
         }
         if (lane == 0) {
             start[E] = carry;
@@ -159,11 +145,25 @@ __device__ __forceinline__ void scatter_load(int (&ev)[kSteps], const int32_t* _
     }
 }
 
+// Division of an entry (below 2^31) by the routes per token: a multiplication and a correction for each, one division for all
+struct TokenOf {
+    uint32_t K, inverse;
+    __device__ __forceinline__ explicit TokenOf(int k) : K((uint32_t)k), inverse(0xffffffffu / (uint32_t)k) {}
+    __device__ __forceinline__ uint32_t operator()(uint32_t n) const {
+        const uint32_t q = __umulhi(n, inverse);   // the quotient or one less
+        return n - q * K >= K ? q + 1 : q;
+    }
+};
+
+// LDS the compiler knows as LDS: through a generic pointer every access would wait for the global ones in flight
+typedef volatile __attribute__((address_space(3))) int32_t* LdsRows;
+
 __device__ __forceinline__ void scatter_place(const int (&ev)[kSteps], int K, int EW, int64_t base, int64_t cend,
-                                              volatile int32_t* next, int32_t* __restrict__ s_scatter,
+                                              LdsRows next, int32_t* __restrict__ s_scatter,
                                               int32_t* __restrict__ s_reverse, int32_t* __restrict__ x_gather) {
     const int lane = threadIdx.x % MTS_WAVE;
     const uint64_t lt = lanemask_lt();
+    const TokenOf by_K(K);
     if (EW <= kFewExperts) {   // wave-uniform
         // A window of few experts: one ballot per expert ranks the 64 entries of a step, and the next free rows
         // stay in registers from step to step (the same positions as below: entries of one expert in lane order).
@@ -185,7 +185,7 @@ __device__ __forceinline__ void scatter_place(const int (&ev)[kSteps], int K, in
             if (e >= -1 && n < cend) s_reverse[n] = pos;
             if (e >= 0) {
                 s_scatter[pos] = (int32_t)n;
-                x_gather[pos] = (int32_t)(n / K);
+                x_gather[pos] = (int32_t)by_K((uint32_t)n);
             }
         }
 #pragma unroll
@@ -215,14 +215,14 @@ __device__ __forceinline__ void scatter_place(const int (&ev)[kSteps], int K, in
         if (e >= -1 && n < cend) s_reverse[n] = pos;
         if (valid) {
             s_scatter[pos] = (int32_t)n;
-            x_gather[pos] = (int32_t)(n / K);
+            x_gather[pos] = (int32_t)by_K((uint32_t)n);
         }
     }
 }
 
 // `first` holds the ids of the chunk's first kSteps x 64 entries already (scatter_load at cbeg)
 __device__ __forceinline__ void scatter_chunk(int (&first)[kSteps], const int32_t* __restrict__ idx, int K, int E, int e0,
-                                              int EW, int64_t cbeg, int64_t cend, volatile int32_t* next,
+                                              int EW, int64_t cbeg, int64_t cend, LdsRows next,
                                               int32_t* __restrict__ s_scatter, int32_t* __restrict__ s_reverse,
                                               int32_t* __restrict__ x_gather) {
     scatter_place(first, K, EW, cbeg, cend, next, s_scatter, s_reverse, x_gather);
@@ -248,7 +248,7 @@ __global__ __launch_bounds__(kThreads) void route_scatter_kernel(
     const int64_t cend = cbeg + chunk_len < TK ? cbeg + chunk_len : TK;
     int first[kSteps];
     scatter_load(first, idx, E, e0, EW, cbeg, cend);   // in flight with the counter loads below
-    volatile int32_t* next = lds + wave * EW;
+    LdsRows next = (LdsRows)(lds + wave * EW);
     for (int e = lane; e < EW; e += MTS_WAVE) next[e] = expert_start[e] + cnt[chunk * EW + e];
     scatter_chunk(first, idx, K, E, e0, EW, cbeg, cend, next, s_scatter, s_reverse, x_gather);
 }
@@ -313,12 +313,7 @@ __global__ __launch_bounds__(kThreads) void head_scatter_kernel(
 #pragma unroll
         for (int e = 0; e < kFinishMaxE; ++e) {
             if (e < E) {   // block-uniform
-                int32_t t = total[e], b = before[e];
-#pragma unroll
-                for (int o = 32; o > 0; o >>= 1) {
-                    t += __shfl_xor(t, o, MTS_WAVE);
-                    b += __shfl_xor(b, o, MTS_WAVE);
-                }
+                const int32_t t = wave_sum(total[e]), b = wave_sum(before[e]);
                 if (lane == 0) {
                     sums[wave][e] = t;
                     sums[wave][kFinishMaxE + e] = b;
@@ -336,13 +331,8 @@ __global__ __launch_bounds__(kThreads) void head_scatter_kernel(
                 bsum += sums[w][kFinishMaxE + lane];
             }
         }
-        int32_t incl = t;
-#pragma unroll
-        for (int o = 1; o < kFinishMaxE; o <<= 1) {
-            const int32_t up = __shfl_up(incl, o, MTS_WAVE);
-            if (lane >= o) incl += up;
-        }
-        volatile int32_t* next = next_rows[wave];
+        const int32_t incl = wave_scan(t);
+        LdsRows next = (LdsRows)next_rows[wave];
         if (lane < E) next[lane] = incl - t + bsum + own;
         scatter_chunk(first_ids, idx, K, E, 0, E, cbeg, cend, next, s_scatter, s_reverse, x_gather);
         return;
@@ -378,8 +368,7 @@ __global__ __launch_bounds__(kThreads) void head_scatter_kernel(
                 c += totv[q][u];
             }
             v = wave_sum(v);
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, MTS_WAVE);
+            c = wave_sum(c);
             if (lane == 0) {
                 if (i < E) total_s[i] = c;
                 mts_router::stats_column(sh, i, v * inv_t, c, E, inv_routes, prob_mean, z_loss, entropy, counts);
@@ -389,12 +378,7 @@ __global__ __launch_bounds__(kThreads) void head_scatter_kernel(
     __syncthreads();
     if (wave == kWaves - 1) {   // exclusive scan of the routes per expert: one lane per expert
         const int32_t v = lane < E ? total_s[lane] : 0;
-        int32_t incl = v;
-#pragma unroll
-        for (int o = 1; o < MTS_WAVE; o <<= 1) {
-            const int32_t up = __shfl_up(incl, o, MTS_WAVE);
-            if (lane >= o) incl += up;
-        }
+        const int32_t incl = wave_scan(v);
         if (lane < E) expert_start[lane] = incl - v;
         if (lane == E - 1) expert_start[E] = incl;
     }

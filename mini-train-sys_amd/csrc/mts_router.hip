@@ -77,17 +77,11 @@ __global__ __launch_bounds__(kThreads) void router_fwd_kernel(
 
     // wave: sum lanes that hold the same experts (same g)
 #pragma unroll
-    for (int j = 0; j < EP; ++j) {
-#pragma unroll
-        for (int o = 32; o >= G; o >>= 1) psum[j] += __shfl_xor(psum[j], o, MTS_WAVE);
-    }
+    for (int j = 0; j < EP; ++j) psum[j] = lane_reduce<32, G>(psum[j], LaneSum());
     zsum = wave_sum(zsum);
     hsum = wave_sum(hsum);
 #pragma unroll
-    for (int j = 0; j < EP; ++j) {
-#pragma unroll
-        for (int o = 32; o >= G; o >>= 1) csum[j] += __shfl_xor(csum[j], o, MTS_WAVE);
-    }
+    for (int j = 0; j < EP; ++j) csum[j] = lane_reduce<32, G>(csum[j], LaneSum());
 
     __shared__ float red[kThreads / MTS_WAVE][EP * G + 2];
     __shared__ int32_t cred[kThreads / MTS_WAVE][EP * G];

@@ -28,12 +28,12 @@ __device__ __forceinline__ void reduce_scatter(float (&v)[NV], int lane, int& id
             for (int i = 0; i < N / 2; ++i) {
                 const float send = up ? v[i] : v[i + N / 2];
                 const float keep = up ? v[i + N / 2] : v[i];
-                v[i] = keep + __shfl_xor(send, O, MTS_WAVE);
+                v[i] = keep + lane_other<O>(send);
             }
             idx += up ? N / 2 : 0;
             reduce_scatter<NV, N / 2, O / 2>(v, lane, idx);
         } else {
-            v[0] += __shfl_xor(v[0], O, MTS_WAVE);
+            v[0] = lane_pair<O>(v[0], LaneSum());
             reduce_scatter<NV, 1, O / 2>(v, lane, idx);
         }
     }
@@ -122,31 +122,67 @@ inline bool mma_projection_ok(int H, int E, int act_dtype) {
 template <int NT>
 struct MmaWeights {
     f32x4 v[kStageBatch];
+    // expert and first column of the thread's piece u: a multiplication for the division, exact for the few thousand pieces there are
+    static __device__ __forceinline__ int place(int i, int quads, float inv, int& k) {
+        const int e = (int)(((float)i + 0.5f) * inv);
+        k = (i - e * quads) * 4;
+        return e;
+    }
     __device__ __forceinline__ void load(const float* __restrict__ w, int H, int E, int batch) {
         const int quads = H / 4;
+        const float inv = 1.0f / (float)quads;
 #pragma unroll
         for (int u = 0; u < kStageBatch; ++u) {
-            const int i = threadIdx.x + (batch * kStageBatch + u) * NT;
-            const int e = i / quads, k = (i % quads) * 4;
-            const f32x4 z = {0.f, 0.f, 0.f, 0.f};
-            v[u] = (i < 8 * quads && e < E) ? *reinterpret_cast<const f32x4*>(w + (int64_t)e * H + k) : z;
+            int k;
+            const int e = place(threadIdx.x + (batch * kStageBatch + u) * NT, quads, inv, k);
+            const f32x4 z = {0.f, 0.f, 0.f, 0.f}, t = *reinterpret_cast<const f32x4*>(w + (int64_t)(e < E ? e : E - 1) * H + k);
+            v[u] = e < E ? t : z;
         }
     }
     __device__ __forceinline__ void split(bf16_t* wb, int H, int batch) const {
         const int quads = H / 4, stride = mma_lds_stride(H);
+        const float inv = 1.0f / (float)quads;
         if (batch == 0) {   // the row of zeros that stands in for the M rows no term maps to
             const bf16x4 z = {};
             for (int k = threadIdx.x * 4; k < H; k += NT * 4) *reinterpret_cast<bf16x4*>(wb + kMmaTerms * 8 * stride + k) = z;
         }
+        uint32_t largest = 0;
 #pragma unroll
+        for (int u = 0; u < kStageBatch; ++u)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) largest = max(largest, __float_as_uint(v[u][q]) & 0x7fffffffu);
+        if (__ballot(largest >= 0x7f000000u) == 0) {   // every weight of the wave is below 2^127: rounding is all there is to a term
+#pragma unroll
+            for (int u = 0; u < kStageBatch; ++u) {
+                const int i = threadIdx.x + (batch * kStageBatch + u) * NT;
+                if (i >= 8 * quads) continue;
+                int k;
+                const int e = place(i, quads, inv, k);
+                f32x4 r = v[u];
+#pragma unroll
+                for (int t = 0; t < 3; ++t) {
+                    uint2 h;   // two values rounded to bf16 in one register each
+                    asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(h.x) : "v"(r[0]), "v"(r[1]));
+                    asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(h.y) : "v"(r[2]), "v"(r[3]));
+                    *reinterpret_cast<uint2*>(wb + (t * 8 + e) * stride + k) = h;
+                    r -= f32x4{__uint_as_float(h.x << 16), __uint_as_float(h.x & 0xffff0000u), __uint_as_float(h.y << 16), __uint_as_float(h.y & 0xffff0000u)};   // exact
+                }
+            }
+            return;
+        }
+#pragma unroll 1
         for (int u = 0; u < kStageBatch; ++u) {
             const int i = threadIdx.x + (batch * kStageBatch + u) * NT;
             if (i >= 8 * quads) continue;
-            const int e = i / quads, k = (i % quads) * 4;
+            int k;
+            const int e = place(i, quads, inv, k);
             bf16x4 t0, t1, t2;
+            f32x4 piece = v[0];
+#pragma unroll
+            for (int q = 1; q < kStageBatch; ++q) piece = u == q ? v[q] : piece;
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                const float a = v[u][q];
+                const float a = piece[q];
                 bf16_t h = (bf16_t)a;
                 // A NaN or infinite weight is carried by the first term alone (inf - inf would turn an infinite weight
                 // into NaN logits where the fp32 dot product gives inf); a finite weight that rounds up to infinity
@@ -489,8 +525,6 @@ __global__ __launch_bounds__(kFwdThreads, MMA ? 2 : 1) void router_head_kernel(
                         if (act_dtype == MTS_BF16) reinterpret_cast<bf16_t*>(weights_act)[row * K + k] = (bf16_t)wk;
                         else reinterpret_cast<mts_f16_t*>(weights_act)[row * K + k] = (mts_f16_t)wk;
                     }
-#pragma unroll
-                    for (int e = 0; e < EP; ++e) csum[e] += e == sel_e[k] ? 1 : 0;
                 }
             }
 #pragma unroll
@@ -501,6 +535,12 @@ __global__ __launch_bounds__(kFwdThreads, MMA ? 2 : 1) void router_head_kernel(
             }
             zsum += rs.L * rs.L;
         }
+        // routes per expert: one ballot each, the sums in scalar registers
+#pragma unroll
+        for (int k = 0; k < MTS_MAX_TOP_K; ++k)
+            if (k < K)
+#pragma unroll
+                for (int e = 0; e < EP; ++e) csum[e] += (int)__popcll(__ballot(live && e == sel_e[k]));
         pass_base = parked_to;
         __builtin_amdgcn_wave_barrier();
     }
@@ -510,8 +550,6 @@ __global__ __launch_bounds__(kFwdThreads, MMA ? 2 : 1) void router_head_kernel(
 #pragma unroll
     for (int e = 0; e < EP; ++e) {
         psum[e] = wave_sum(psum[e]);
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) csum[e] += __shfl_xor(csum[e], o, MTS_WAVE);
     }
     zsum = wave_sum(zsum);
     hsum = wave_sum(hsum);

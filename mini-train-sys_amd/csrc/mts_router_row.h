@@ -33,16 +33,10 @@ struct KeptWeights {
 constexpr float kLogFloor = -20.72326583694641f;  // log(1e-9): the entropy clamps p at 1e-9
 
 template <int G>
-__device__ __forceinline__ float group_sum(float v) {
-#pragma unroll
-    for (int o = G / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, MTS_WAVE);
-    return v;
-}
+__device__ __forceinline__ float group_sum(float v) { return lane_reduce<G / 2, 1>(v, LaneSum()); }
 template <int G>
 __device__ __forceinline__ float group_max(float v) {
-#pragma unroll
-    for (int o = G / 2; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, MTS_WAVE));
-    return v;
+    return lane_reduce<G / 2, 1>(v, [](float a, float b) { return fmaxf(a, b); });
 }
 
 template <int EP, int G>
@@ -95,6 +89,17 @@ __device__ __forceinline__ void load_row(const float* __restrict__ logits, int64
 }
 
 
+// the larger value of the lanes that share a row, and its expert; the lower expert where two are equal
+template <int O>
+__device__ __forceinline__ void best_of_lanes(float& bv, int& be) {
+    if constexpr (O > 0) {
+        const float ov = lane_other<O>(bv);
+        const int oe = lane_other<O>(be);
+        if (ov > bv || (ov == bv && oe < be)) bv = ov, be = oe;
+        best_of_lanes<O / 2>(bv, be);
+    }
+}
+
 // K rounds of arg-max over the logits of a row (ties to the lower expert index).  `taken` has a
 // bit per slot j of this lane (expert j*G + g); sel_e / sel_p get the expert and its softmax
 // probability per rank, mass the sum of the selected probabilities.
@@ -122,15 +127,7 @@ __device__ __forceinline__ void select_top_k(const RowState<EP, G>& r, int E, in
                     be = e;
                 }
             }
-#pragma unroll
-            for (int o = G / 2; o > 0; o >>= 1) {
-                float ov = __shfl_xor(bv, o, MTS_WAVE);
-                int oe = __shfl_xor(be, o, MTS_WAVE);
-                if (ov > bv || (ov == bv && oe < be)) {
-                    bv = ov;
-                    be = oe;
-                }
-            }
+            best_of_lanes<G / 2>(bv, be);
             if (be % G == g) taken |= 1u << (be / G);
             float pk = expf(bv - r.m) / r.s;
             sel_p[k] = pk;
@@ -234,12 +231,9 @@ __device__ __forceinline__ void stats_finalize(const StatsShared& sh, int wave, 
         }
         sum = wave_sum(sum);
         dead = wave_sum(dead);
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            hi = fmaxf(hi, __shfl_xor(hi, o, MTS_WAVE));
-            most = max(most, __shfl_xor(most, o, MTS_WAVE));
-            fewest = min(fewest, __shfl_xor(fewest, o, MTS_WAVE));
-        }
+        hi = lane_reduce<32, 1>(hi, [](float a, float b) { return fmaxf(a, b); });
+        most = lane_reduce<32, 1>(most, [](int a, int b) { return max(a, b); });
+        fewest = lane_reduce<32, 1>(fewest, [](int a, int b) { return min(a, b); });
         const float mean = sum / (float)E;
         float var = 0.f;
         for (int e = lane; e < E; e += MTS_WAVE) {
