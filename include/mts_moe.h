@@ -488,6 +488,11 @@ int mts_cross_entropy_bwd(const void* logits, const int64_t* targets, int64_t N,
                           int64_t ignore_index, int dtype, const float* row_max,
                           const float* row_log_sum, const float* g_loss, const float* inv_count,
                           void* d_logits, void* stream);
+/* the same with rows of d_logits pitch elements apart (at least V, a multiple of 8; the rest is left as it is) */
+int mts_cross_entropy_bwd_pitched(const void* logits, const int64_t* targets, int64_t N, int V,
+                                  int64_t ignore_index, int dtype, const float* row_max,
+                                  const float* row_log_sum, const float* g_loss, const float* inv_count,
+                                  void* d_logits, int64_t pitch, void* stream);
 
 /* Weight gradient of a dense projection y = x W^T: dw [N,K] f32 = g^T x, g [T,N] and x [T,K] dense
  * bf16 or fp16, fp32 sums in a fixed order.  N and K multiples of 8, at most 32 tiles of 256 x 256,
@@ -496,6 +501,16 @@ int mts_linear_dw_supported(int act_dtype, int64_t T, int N, int K);
 int64_t mts_linear_dw_workspace_bytes(int64_t T, int N, int K);
 int mts_linear_dw(const void* g, const void* x, int64_t T, int N, int K, int act_dtype, float* dw,
                   void* workspace, int64_t workspace_bytes, void* stream);
+/* Both gradients where they have tiles for whole rounds of the chip: dw as above, and
+ * dx [T,K] = g W of act_dtype, w [N,K] the rounded weight.  Rows of g are ldg elements apart (a multiple
+ * of 8, at least N; what lies between them is not used), N is any number, K a multiple of 8.
+ * which: 0 dx, 1 dw.                                                                        */
+int mts_linear_rounds_supported(int act_dtype, int64_t T, int N, int K, int64_t ldg);
+int64_t mts_linear_rounds_workspace_bytes(int which, int64_t T, int N, int K);
+int mts_linear_dw_rounds(const void* g, int64_t ldg, const void* x, int64_t T, int N, int K, int act_dtype,
+                         float* dw, void* workspace, int64_t workspace_bytes, void* stream);
+int mts_linear_dx_rounds(const void* g, int64_t ldg, const void* w, int64_t T, int N, int K, int act_dtype,
+                         void* dx, void* workspace, int64_t workspace_bytes, void* stream);
 
 /* Scaled dot-product attention of heads of 64 elements, bf16 or fp16, queries and keys of the
  * same length; causal != 0: query i sees keys 0..i.  Tensors are [B,heads,S,64], dense in the last

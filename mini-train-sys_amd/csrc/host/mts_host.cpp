@@ -891,16 +891,49 @@ struct QkvRope : torch::autograd::Function<QkvRope> {
     }
 };
 
+// The projection on a vocabulary: both gradients are this framework's, over whole rounds of tiles (mts_linear_dx_rounds).  They are ahead
+// of the library's from 128 rows on (768 wide, us, dX and dW, here / library: 24 576 rows of 50 257 1610 / 2577 and 1520 / 2199, 4096 rows
+// 279 / 555 and 278 / 375, 512 rows 69 / 197 and 58 / 67; 1024 rows of 8192 31 / 44 and 26 / 25), and dX no longer where a projection
+// is less than eight times as wide as its input (12 288 rows of 2304 48 / 45, 8192 rows of 4096 -> 12 288 612 / 594).
+constexpr int64_t kLinearRoundsRows = 128;
+bool linear_in_rounds(const Tensor& x, int64_t T, int64_t N, int64_t K) {
+    return T >= kLinearRoundsRows && N >= 8 * K && N < k2GiB && mts_linear_rounds_supported(dtype_code(x), T, N, K, (N + 7) / 8 * 8);
+}
+// rows that mts_linear_dx_rounds and mts_linear_dw_rounds read in place
+bool rows_fit(const Tensor& g) { return g.stride(1) == 1 && g.stride(0) >= g.size(1) && g.stride(0) % 8 == 0 && aligned16(g); }
+
 // A projection under autocast: the product is the library's, the gradient of its fp32 weight is summed in fp32 here.
 bool linear_supported(const Tensor& x, const Tensor& w) {
     if (!(at::GradMode::is_enabled() && w.requires_grad() && all_plain(x, w) && on_one_gpu(x, w) && x.dim() >= 2 && w.dim() == 2 &&
           w.scalar_type() == at::kFloat && (x.scalar_type() == at::kBFloat16 || x.scalar_type() == at::kHalf) && x.size(-1) == w.size(1) && x.numel() > 0))
         return false;
     if (!at::autocast::is_autocast_enabled(at::kCUDA) || at::autocast::get_autocast_dtype(at::kCUDA) != x.scalar_type()) return false;
-    return mts_linear_dw_supported(dtype_code(x), x.numel() / x.size(-1), w.size(0), w.size(1));
+    const int64_t T = x.numel() / x.size(-1), N = w.size(0), K = w.size(1);
+    return linear_in_rounds(x, T, N, K) || mts_linear_dw_supported(dtype_code(x), T, N, K);
 }
 
 struct Linear : torch::autograd::Function<Linear> {
+    static variable_list in_rounds(AutogradContext* ctx, const Tensor& g, const Tensor& x, const Tensor& rounded, int64_t T, int64_t N, int64_t K) {
+        Tensor dx, dw;
+        auto workspace = [&](int which, int64_t& size) {
+            size = mts_linear_rounds_workspace_bytes(which, T, N, K);
+            return size ? bytes(size, x) : Tensor();
+        };
+        int64_t size = 0;
+        if (ctx->needs_input_grad(0)) {
+            const Tensor w = dense16(rounded), ws = workspace(0, size);
+            dx = at::empty({T, K}, x.options());
+            check(mts_linear_dx_rounds(ptr(g), g.stride(0), ptr(w), T, N, K, dtype_code(x), ptr(dx), ptr(ws), size, stream_of(x)), "mts_linear_dx_rounds");
+            dx = dx.view(x.sizes());
+        }
+        if (ctx->needs_input_grad(1)) {
+            const Tensor in = dense16(x.reshape({T, K})), ws = workspace(1, size);
+            dw = f32({N, K}, x);
+            check(mts_linear_dw_rounds(ptr(g), g.stride(0), ptr(in), T, N, K, dtype_code(x), ptr_as<float>(dw), ptr(ws), size, stream_of(x)),
+                  "mts_linear_dw_rounds");
+        }
+        return {dx, dw};
+    }
     static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w) {
         const Tensor rounded = w.to(x.scalar_type());
         ctx->save_for_backward({x, rounded});
@@ -912,10 +945,24 @@ struct Linear : torch::autograd::Function<Linear> {
         const Tensor &x = s[0], &rounded = s[1];
         c10::OptionalDeviceGuard guard(x.device());
         const int64_t N = rounded.size(0), K = rounded.size(1), T = x.numel() / K;
+        const bool rounds = linear_in_rounds(x, T, N, K);
         if (written_out(grads)) {
-            const Tensor g = grads[0].reshape({T, N}), wide = g.to(at::kFloat);
+            const Tensor g = grads[0].reshape({T, N});
             const Tensor now = ctx->saved_data["weight"].toTensor().to(x.scalar_type());   // for its derivative; the value is that of the forward pass
-            return {at::matmul(g, rounded + (now - now.detach())).view(x.sizes()), at::matmul(wide.t().contiguous(), x.reshape({T, K}).to(at::kFloat))};
+            const Tensor dx = at::matmul(g, rounded + (now - now.detach())).view(x.sizes());
+            // an fp32 copy of the gradient of as many logits would be larger than all else: stock autocast's product there
+            if (rounds) return {dx, at::matmul(g.t(), x.reshape({T, K})).to(at::kFloat)};
+            return {dx, at::matmul(g.to(at::kFloat).t().contiguous(), x.reshape({T, K}).to(at::kFloat))};
+        }
+        if (rounds) {
+            const Tensor g = grads[0].reshape({T, N});
+            if (rows_fit(g) && mts_linear_rounds_supported(dtype_code(x), T, N, K, g.stride(0))) return in_rounds(ctx, g, x, rounded, T, N, K);
+            if (!mts_linear_dw_supported(dtype_code(x), T, N, K)) {   // rows at odd places: a copy costs more than it gives
+                Tensor dx, dw;
+                if (ctx->needs_input_grad(0)) dx = at::matmul(g, rounded).view(x.sizes());
+                if (ctx->needs_input_grad(1)) dw = at::matmul(g.t(), x.reshape({T, K})).to(at::kFloat);
+                return {dx, dw};
+            }
         }
         const Tensor g = dense16(grads[0].reshape({T, N})), in = dense16(x.reshape({T, K}));
         Tensor dx, dw;
@@ -988,9 +1035,24 @@ bool cross_entropy_supported(const Tensor& logits, const Tensor& targets) {
            logits.size(1) < k2GiB;
 }
 
+// Whether the logits come, through views at most, from a projection whose gradients read rows of any pitch (Linear::in_rounds)
+bool logits_of_rounds(const Tensor& logits) {
+    if (!at::GradMode::is_enabled() || !logits.requires_grad() || logits.scalar_type() == at::kFloat) return false;
+    std::shared_ptr<torch::autograd::Node> fn = logits.grad_fn();
+    for (int depth = 0; fn && depth < 4; ++depth) {
+        if (dynamic_cast<torch::autograd::CppNode<Linear>*>(fn.get())) return true;
+        const std::string name = fn->name();
+        if ((name != "ViewBackward0" && name != "UnsafeViewBackward0" && name != "ReshapeAliasBackward0") || fn->num_outputs() != 1) return false;
+        fn = fn->next_edge(0).function;
+    }
+    return false;
+}
+
 // mean cross-entropy without an fp32 copy of the logits
 struct CrossEntropy : torch::autograd::Function<CrossEntropy> {
-    static Tensor forward(AutogradContext* ctx, const Tensor& logits, const Tensor& targets) {   // dense16, dense
+    // dense16, dense; `pitched`: the rows of the gradient start on 128 bytes
+    static Tensor forward(AutogradContext* ctx, const Tensor& logits, const Tensor& targets, bool pitched) {
+        ctx->saved_data["pitched"] = pitched;
         const int64_t N = logits.size(0), V = logits.size(1);
         // per row: maximum, log of the sum, loss; then 1 / count.  The loss is a tensor of its own, which the caller may change
         // (no view) and which is not kept.
@@ -1012,15 +1074,23 @@ struct CrossEntropy : torch::autograd::Function<CrossEntropy> {
             const Tensor p = at::softmax(s[0].to(at::kFloat), 1) - hit.to(at::kFloat), none = at::zeros({}, p.options());
             const Tensor ignored = t.eq(kIgnoreIndex), outside = t.lt(0).logical_or(t.ge(V)).logical_and(ignored.logical_not());
             const Tensor scale = g * s[2].select(0, 3 * N) + at::where(outside, at::full({}, NAN, p.options()), none);
-            return {at::where(ignored, none, p * scale).to(s[0].scalar_type()), Tensor()};
+            return {at::where(ignored, none, p * scale).to(s[0].scalar_type()), Tensor(), Tensor()};
         }
         const Tensor g = like_f32(grads[0]);
-        Tensor d = at::empty_like(s[0]);
         const float* row = ptr_as<float>(s[2]);
+        if (ctx->saved_data["pitched"].toBool() && V % 8) {
+            const int64_t pitch = (V + 63) / 64 * 64;
+            Tensor rows = at::empty({N, pitch}, s[0].options());
+            check(mts_cross_entropy_bwd_pitched(ptr(s[0]), ptr_as<int64_t>(s[1]), N, V, kIgnoreIndex, dtype_code(s[0]), row, row + N, ptr_as<float>(g),
+                                                row + 3 * N, ptr(rows), pitch, stream_of(s[0])),
+                  "mts_cross_entropy_bwd_pitched");
+            return {rows.narrow(1, 0, V), Tensor(), Tensor()};
+        }
+        Tensor d = at::empty_like(s[0]);
         check(mts_cross_entropy_bwd(ptr(s[0]), ptr_as<int64_t>(s[1]), N, V, kIgnoreIndex, dtype_code(s[0]), row, row + N, ptr_as<float>(g),
                                     row + 3 * N, ptr(d), stream_of(s[0])),
               "mts_cross_entropy_bwd");
-        return {d, Tensor()};
+        return {d, Tensor(), Tensor()};
     }
 };
 
@@ -1090,6 +1160,7 @@ PYBIND11_MODULE(_host, m) {
     m.def("cross_entropy_supported", &cross_entropy_supported);
     m.def("cross_entropy", [](const Tensor& logits, const Tensor& targets) {
         c10::OptionalDeviceGuard guard(logits.device());
-        return CrossEntropy::apply(dense16(logits), targets.contiguous());
+        const Tensor dense = dense16(logits);
+        return CrossEntropy::apply(dense, targets.contiguous(), logits_of_rounds(dense));
     });
 }

@@ -464,19 +464,23 @@ __global__ __launch_bounds__(kCeMeanThreads) void cross_entropy_mean_kernel(cons
     }
 }
 
-// d_logits = (softmax - onehot) * g / count, zero where the target is ignored, NaN as the loss where it is outside the vocabulary
-template <typename ET>
+// d_logits = (softmax - onehot) * g / count, zero where the target is ignored, NaN as the loss where it is outside the vocabulary.
+// PITCHED: rows of d_logits start on 16 bytes, pitch elements apart, whatever V is (the projection's gradients read them so); the 16-byte
+// pieces then follow the output and are read from wherever they lie in the logits.  Memory-bound either way: 24 576 rows of 50 257 949 us dense,
+// 900 pitched (5.5 TB/s).
+template <typename ET, bool PITCHED>
 __global__ __launch_bounds__(kCeThreads) void cross_entropy_bwd_kernel(const ET* __restrict__ logits, const int64_t* __restrict__ targets, int V,
                                                                        int64_t ignore, const float* __restrict__ row_max,
                                                                        const float* __restrict__ row_log_sum, const float* __restrict__ g,
-                                                                       const float* __restrict__ inv_count, ET* __restrict__ d_logits) {
+                                                                       const float* __restrict__ inv_count, ET* __restrict__ d_logits, int64_t pitch) {
     constexpr int W = CeRow<ET>::W, UN = 4;
     typedef __attribute__((ext_vector_type(W))) ET vec;
+    typedef __attribute__((ext_vector_type(W), aligned(PITCHED ? sizeof(ET) : 16))) ET in_vec;
     const int64_t row = blockIdx.x;
     const int64_t target = targets[row];
     const ET* p = logits + row * V;
-    ET* d = d_logits + row * V;
-    const CeRow<ET> r(p, V);
+    ET* d = d_logits + row * (PITCHED ? pitch : V);
+    const CeRow<ET> r(PITCHED ? d : p, V);
     const float scale = target == ignore ? 0.f : ((target < 0 || target >= V) ? NAN : *g * *inv_count);
     // maximum and logarithm of the sum apart: their sum would carry the rounding of a large maximum into every probability
     const float hi = row_max[row], base = row_log_sum[row] * kLog2e;
@@ -490,7 +494,7 @@ __global__ __launch_bounds__(kCeThreads) void cross_entropy_bwd_kernel(const ET*
         const int c = r.head + r.vecs * W + threadIdx.x;
         d[c] = grad((float)p[c], c);
     }
-    const vec* body = reinterpret_cast<const vec*>(p + r.head);
+    const in_vec* body = reinterpret_cast<const in_vec*>(p + r.head);
     vec* out = reinterpret_cast<vec*>(d + r.head);
     int i = threadIdx.x;
     for (; i < r.vecs; i += UN * kCeThreads) {
@@ -590,20 +594,32 @@ extern "C" int mts_cross_entropy_fwd(const void* logits, const int64_t* targets,
     return MTS_OK;
 }
 
-extern "C" int mts_cross_entropy_bwd(const void* logits, const int64_t* targets, int64_t N, int V, int64_t ignore_index, int dtype, const float* row_max,
-                                     const float* row_log_sum, const float* g_loss, const float* inv_count, void* d_logits, void* stream) {
+template <bool PITCHED>
+static int cross_entropy_bwd(const void* logits, const int64_t* targets, int64_t N, int V, int64_t ignore_index, int dtype, const float* row_max,
+                             const float* row_log_sum, const float* g_loss, const float* inv_count, void* d_logits, int64_t pitch, void* stream) {
     if (!logits || !targets || !row_max || !row_log_sum || !g_loss || !inv_count || !d_logits) return MTS_ERR_NULL;
-    if (N <= 0 || N >= MTS_MAX_LOSS_ROWS || V <= 0) return MTS_ERR_SHAPE;
+    if (N <= 0 || N >= MTS_MAX_LOSS_ROWS || V <= 0 || (PITCHED && (pitch < V || pitch % 8))) return MTS_ERR_SHAPE;
     if (!dense_dtype_ok(dtype)) return MTS_ERR_DTYPE;
     if (!mts_aligned16(logits) || !mts_aligned16(d_logits)) return MTS_ERR_ALIGN;
     hipStream_t st = (hipStream_t)stream;
     const dim3 grid((unsigned)N), block(kCeThreads);
     if (dtype == MTS_BF16)
-        cross_entropy_bwd_kernel<bf16_t><<<grid, block, 0, st>>>((const bf16_t*)logits, targets, V, ignore_index, row_max, row_log_sum, g_loss, inv_count, (bf16_t*)d_logits);
+        cross_entropy_bwd_kernel<bf16_t, PITCHED><<<grid, block, 0, st>>>((const bf16_t*)logits, targets, V, ignore_index, row_max, row_log_sum, g_loss, inv_count,
+                                                                          (bf16_t*)d_logits, pitch);
     else if (dtype == MTS_F16)
-        cross_entropy_bwd_kernel<mts_f16_t><<<grid, block, 0, st>>>((const mts_f16_t*)logits, targets, V, ignore_index, row_max, row_log_sum, g_loss, inv_count, (mts_f16_t*)d_logits);
+        cross_entropy_bwd_kernel<mts_f16_t, PITCHED><<<grid, block, 0, st>>>((const mts_f16_t*)logits, targets, V, ignore_index, row_max, row_log_sum, g_loss, inv_count,
+                                                                             (mts_f16_t*)d_logits, pitch);
     else
-        cross_entropy_bwd_kernel<float><<<grid, block, 0, st>>>((const float*)logits, targets, V, ignore_index, row_max, row_log_sum, g_loss, inv_count, (float*)d_logits);
+        cross_entropy_bwd_kernel<float, PITCHED><<<grid, block, 0, st>>>((const float*)logits, targets, V, ignore_index, row_max, row_log_sum, g_loss, inv_count,
+                                                                         (float*)d_logits, pitch);
     MTS_CHECK_LAUNCH();
     return MTS_OK;
+}
+extern "C" int mts_cross_entropy_bwd(const void* logits, const int64_t* targets, int64_t N, int V, int64_t ignore_index, int dtype, const float* row_max,
+                                     const float* row_log_sum, const float* g_loss, const float* inv_count, void* d_logits, void* stream) {
+    return cross_entropy_bwd<false>(logits, targets, N, V, ignore_index, dtype, row_max, row_log_sum, g_loss, inv_count, d_logits, V, stream);
+}
+extern "C" int mts_cross_entropy_bwd_pitched(const void* logits, const int64_t* targets, int64_t N, int V, int64_t ignore_index, int dtype, const float* row_max,
+                                             const float* row_log_sum, const float* g_loss, const float* inv_count, void* d_logits, int64_t pitch, void* stream) {
+    return cross_entropy_bwd<true>(logits, targets, N, V, ignore_index, dtype, row_max, row_log_sum, g_loss, inv_count, d_logits, pitch, stream);
 }

@@ -130,7 +130,8 @@ struct Divider {
 
 // EPI_DY1N: the dO*W2 epilogue without the weighted_act output (the caller kept the forward
 // pass's post_act, which already carries the routing weight)
-enum Epilogue { EPI_PLAIN = 0, EPI_SWIGLU = 1, EPI_DY1 = 2, EPI_DY1N = 3 };
+// EPI_SPLIT: the product of a part of k as an fp32 tile (part), or of all of it in C (part == NULL)
+enum Epilogue { EPI_PLAIN = 0, EPI_SWIGLU = 1, EPI_DY1 = 2, EPI_DY1N = 3, EPI_SPLIT = 4 };
 constexpr bool epi_is_dy1(int epi) { return epi == EPI_DY1 || epi == EPI_DY1N; }
 
 struct RowsParams {
@@ -164,6 +165,7 @@ struct RowsParams {
     const int32_t* sched;      // with xcd_ranges: the m-tile range of every XCD (first[8], count[8]) from the schedule of the joint
                                // backward launch, or NULL: equal ranges
     int32_t* sched_out;        // dO*W2 launch: one more block writes the schedule of the joint backward launch here (NULL: none)
+    float* part;               // EPI_SPLIT: the tile's place among the partial results
     int sched_slots, sched_dx_cap;
 };
 
@@ -386,7 +388,7 @@ __device__ __forceinline__ void zero_acc(f32x16 (&acc)[T::MF][T::NF]) {
 template <class T, int EPI>
 struct EpiShape {
     static constexpr int COLS = (EPI == EPI_SWIGLU) ? T::WN / 2 : T::WN;  // contiguous columns per staged tile
-    static constexpr int NBUF = (EPI == EPI_PLAIN) ? 1 : (EPI == EPI_DY1N ? 2 : 3);
+    static constexpr int NBUF = (EPI == EPI_PLAIN || EPI == EPI_SPLIT) ? 1 : (EPI == EPI_DY1N ? 2 : 3);
     static constexpr int LDW = COLS + 8;
     static constexpr int ELEMS = T::NWAVES * NBUF * 32 * LDW;
 };
@@ -434,7 +436,7 @@ __device__ __forceinline__ void swiglu_backward(uint32_t gw, uint32_t uw, bool h
 // the two dependent loads of all rows in two batches.
 template <class T, int EPI>
 __device__ __forceinline__ void load_row_weights(const RowsParams& p, int row0, int rend, int wm, float (&srow)[T::MF]) {
-    if constexpr (EPI != EPI_PLAIN) {
+    if constexpr (EPI != EPI_PLAIN && EPI != EPI_SPLIT) {
         if (epi_is_dy1(EPI) || p.route_w != nullptr) {
             int entry[T::MF];
 #pragma unroll
@@ -1184,6 +1186,50 @@ __device__ __forceinline__ void dy1_slab(const RowsParams& p, f32x16 (&acc)[T::N
     }
 }
 
+// Accumulators -> the tile at C (leading dimension ldc, rows x cols of it exist).  The MFMAs take the Q fragment first, so a lane holds runs of four
+// consecutive columns of one row; 32 x 64 slabs go through the wave's part of `stage` and out in 16-byte pieces, whole 128-byte lines
+// per row.  An element a lane and store, with an address and a bounds check each, took 3.4 us a tile; now 1.7 (a tile of 1024 rows at
+// 4096/14336 36.0 -> 34.5 us, of 512 rows at 1024/512 22.0 -> 20.4).
+template <class T, typename OutT>
+__device__ __forceinline__ void dw_epilogue(f32x16 (&acc)[T::MF][T::NF], bf16_t* stage, OutT* C, int ldc, int rows, int cols, int wm, int wn) {
+    static_assert(T::WN == 64 && T::NWAVES * 32 * T::WN * sizeof(float) <= (size_t)T::BKS * (T::BM + T::BN) * (T::STAGES == 2 ? 2 : 8), "staging area");
+    const int wave = threadIdx.x / MTS_WAVE, lane = threadIdx.x % MTS_WAVE;
+    const int ml = lane % 32, half = lane / 32;
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(C, (int64_t)(rows < T::BM ? rows : T::BM) * ldc * (int64_t)sizeof(OutT));
+    const int col0 = wn * T::WN;
+#pragma unroll
+    for (int mf = 0; mf < T::MF; ++mf) {
+        const int row0 = wm * T::WM + mf * 32;
+        if constexpr (sizeof(OutT) == 2) {
+            constexpr int LDW = T::WN + 8;
+            bf16_t* buf = stage + wave * 32 * LDW;
+#pragma unroll
+            for (int nf = 0; nf < T::NF; ++nf)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    stage4(buf + ml * LDW + nf * 32 + 8 * j + 4 * half, acc[mf][nf][4 * j], acc[mf][nf][4 * j + 1], acc[mf][nf][4 * j + 2],
+                           acc[mf][nf][4 * j + 3]);
+            flush_tile<T::WN>(buf, rs, (uint32_t)ldc, (uint32_t)col0, row0, rows, col0, cols);
+        } else {   // 16-byte groups of a row change places by the row, so that neither direction piles up on a bank
+            float* buf = reinterpret_cast<float*>(stage) + wave * 32 * T::WN;
+#pragma unroll
+            for (int nf = 0; nf < T::NF; ++nf)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const f32x4 v = {acc[mf][nf][4 * j], acc[mf][nf][4 * j + 1], acc[mf][nf][4 * j + 2], acc[mf][nf][4 * j + 3]};
+                    *reinterpret_cast<f32x4*>(buf + ml * T::WN + (((nf * 8 + 2 * j + half) ^ (ml & 15)) << 2)) = v;
+                }
+#pragma unroll
+            for (int it = 0; it < 8; ++it) {
+                const int r = it * 4 + lane / 16, g = lane % 16;
+                const u32x4 v = *reinterpret_cast<const u32x4*>(buf + r * T::WN + ((g ^ (r & 15)) << 2));
+                const bool ok = row0 + r < rows && col0 + g * 4 < cols;
+                __builtin_amdgcn_raw_buffer_store_b128(v, rs, ok ? (int)(((uint32_t)(row0 + r) * (uint32_t)ldc + (uint32_t)(col0 + g * 4)) * 4u) : (int)kInvalid, 0, 0);
+            }
+        }
+    }
+}
+
 // one output tile: rows [row0, rend) of expert e (at most T::BM of them), column tile ntile
 // `rows_ready` runs in the producer waves of a tile on three activation buffers, behind the first loads of the weights and
 // in front of the first loads of the activation rows (a launch whose rows are written by other blocks of the same launch).
@@ -1251,6 +1297,16 @@ __device__ __forceinline__ void rows_gemm_ws_tile(const RowsParams& p, bf16_t* s
                 else mask_k_chunks<T::B_INSTR, T::CHUNKS, T::RPI>(voff_b, pw * T::B_INSTR * T::RPI, k_left);
             }
         };
+        auto clear_past_k = [&](bf16_t* sa) {
+            const bf16_t zero = (bf16_t)0.f;
+#pragma unroll
+            for (int j = 0; j < T::A_INSTR; ++j) {
+                const int tr = row[j] - row0;
+                if ((slot ^ (T::CHUNKS == 8 ? (tr >> 1) & 7 : (tr >> 2) & 3)) == k_left / 8)
+                    for (int i = k_left % 8; i < 8; ++i) sa[j * 512 + lane * 8 + i] = zero;
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        };
         auto tile_a = [&](bf16_t* sa, int kt) {
             mask_a(kt);
             const int soff_a = kt * T::BKS * 2;
@@ -1304,6 +1360,9 @@ __device__ __forceinline__ void rows_gemm_ws_tile(const RowsParams& p, bf16_t* s
             stage_a(0, 0);
             for (int kt = 0; kt < nk; ++kt) {
                 wait_vmcnt<0>();
+                if constexpr (EPI == EPI_SPLIT) {   // what follows the last k in its chunk is not the operand's (the others end with a chunk)
+                    if (k_left % 8 && kt == nk - 1) clear_past_k(smem + (kt & 1) * T::STAGE + pw * T::A_INSTR * 512);
+                }
                 __builtin_amdgcn_s_barrier();
                 if (kt + 1 < nk) issue((kt + 1) & 1, kt + 1);
             }
@@ -1390,7 +1449,12 @@ __device__ __forceinline__ void rows_gemm_ws_tile(const RowsParams& p, bf16_t* s
             return;
         }
         __builtin_amdgcn_s_barrier();       // every wave is done with the buffers before the epilogue reuses them
-        rows_epilogue<T, EPI>(p, acc, smem, row0, rend, n0, wm, wn, srow);
+        if constexpr (EPI == EPI_SPLIT) {
+            if (p.part) dw_epilogue<T>(acc, smem, p.part, T::BN, T::BM, T::BN, wm, wn);
+            else dw_epilogue<T>(acc, smem, p.C + (int64_t)row0 * p.N + n0, p.N, rend - row0, p.N - n0, wm, wn);
+        } else {
+            rows_epilogue<T, EPI>(p, acc, smem, row0, rend, n0, wm, wn, srow);
+        }
         return;
     }
     __builtin_amdgcn_s_barrier();   // tiles 0 and 1 are visible
@@ -1463,6 +1527,7 @@ struct DwParams {
     const int32_t* sched;   // the unit table of the joint backward launch's schedule (which units an XCD runs), or NULL:
     int sched_slots;        // unit u runs on XCD u % 8; sched_slots: table entries per XCD
     int segment_rows;       // not 0: no experts, E segments of this many of the TK rows
+    int p_pad;              // elements between the rows of P (0: dense), with a P that is read in place
 };
 
 // ---------------------------------------------------------------------------
@@ -1942,70 +2007,11 @@ struct DwWsTile {
     static_assert(LDS_ELEMS * 2 <= 160 * 1024, "LDS capacity");
 };
 
-// Accumulators -> the tile at C (leading dimension ldc, rows x cols of it exist).  The MFMAs take the Q fragment first, so a lane holds runs of four
-// consecutive columns of one row; 32 x 64 slabs go through the wave's part of `stage` and out in 16-byte pieces, whole 128-byte lines
-// per row.  An element a lane and store, with an address and a bounds check each, took 3.4 us a tile; now 1.7 (a tile of 1024 rows at
-// 4096/14336 36.0 -> 34.5 us, of 512 rows at 1024/512 22.0 -> 20.4).
+// the tile at (m0, n0) over rows [rbeg, rend): to `part` as a whole fp32 tile, or (part == NULL) to C, the tile's first element.
+// `smem` holds T::LDS_ELEMS elements, 1 KiB aligned
 template <class T, typename OutT>
-__device__ __forceinline__ void dw_epilogue(f32x16 (&acc)[T::MF][T::NF], bf16_t* stage, OutT* C, int ldc, int rows, int cols, int wm, int wn) {
-    static_assert(T::WN == 64 && T::NWAVES * 32 * T::WN * sizeof(float) <= (size_t)T::BKS * (T::BM + T::BN) * (T::STAGES == 2 ? 2 : 8), "staging area");
-    const int wave = threadIdx.x / MTS_WAVE, lane = threadIdx.x % MTS_WAVE;
-    const int ml = lane % 32, half = lane / 32;
-    const __amdgpu_buffer_rsrc_t rs = make_rsrc(C, (int64_t)(rows < T::BM ? rows : T::BM) * ldc * (int64_t)sizeof(OutT));
-    const int col0 = wn * T::WN;
-#pragma unroll
-    for (int mf = 0; mf < T::MF; ++mf) {
-        const int row0 = wm * T::WM + mf * 32;
-        if constexpr (sizeof(OutT) == 2) {
-            constexpr int LDW = T::WN + 8;
-            bf16_t* buf = stage + wave * 32 * LDW;
-#pragma unroll
-            for (int nf = 0; nf < T::NF; ++nf)
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    stage4(buf + ml * LDW + nf * 32 + 8 * j + 4 * half, acc[mf][nf][4 * j], acc[mf][nf][4 * j + 1], acc[mf][nf][4 * j + 2],
-                           acc[mf][nf][4 * j + 3]);
-            flush_tile<T::WN>(buf, rs, (uint32_t)ldc, (uint32_t)col0, row0, rows, col0, cols);
-        } else {   // 16-byte groups of a row change places by the row, so that neither direction piles up on a bank
-            float* buf = reinterpret_cast<float*>(stage) + wave * 32 * T::WN;
-#pragma unroll
-            for (int nf = 0; nf < T::NF; ++nf)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const f32x4 v = {acc[mf][nf][4 * j], acc[mf][nf][4 * j + 1], acc[mf][nf][4 * j + 2], acc[mf][nf][4 * j + 3]};
-                    *reinterpret_cast<f32x4*>(buf + ml * T::WN + (((nf * 8 + 2 * j + half) ^ (ml & 15)) << 2)) = v;
-                }
-#pragma unroll
-            for (int it = 0; it < 8; ++it) {
-                const int r = it * 4 + lane / 16, g = lane % 16;
-                const u32x4 v = *reinterpret_cast<const u32x4*>(buf + r * T::WN + ((g ^ (r & 15)) << 2));
-                const bool ok = row0 + r < rows && col0 + g * 4 < cols;
-                __builtin_amdgcn_raw_buffer_store_b128(v, rs, ok ? (int)(((uint32_t)(row0 + r) * (uint32_t)ldc + (uint32_t)(col0 + g * 4)) * 4u) : (int)kInvalid, 0, 0);
-            }
-        }
-    }
-}
-
-// the work of block `block` of a launch; `smem` holds T::LDS_ELEMS elements, 1 KiB aligned
-template <class T, typename OutT>
-__device__ __forceinline__ void dw_gemm_ws_block(const DwParams& p, bf16_t* smem, int block) {
+__device__ __forceinline__ void dw_gemm_ws_tile(const DwParams& p, bf16_t* smem, int rbeg, int rend, int m0, int n0, float* part, OutT* C) {
     constexpr int S = T::STAGES, L = T::A_INSTR + T::B_INSTR;
-    // all tiles of a unit (an expert, or a row chunk of an over-full one) run on one XCD
-    const int xcd = block % kXcds, jb = block / kXcds;
-    DwUnit unit;
-    int tile, tile_n;
-    const int k = p.by_tiles.quotient(jb, tile);
-    if (p.sched) {
-        if (k >= p.sched[kSchedCounts + xcd]) return;
-        const int32_t* u = p.sched + kSchedUnits + (xcd * p.sched_slots + k) * 4;
-        unit.e = u[0]; unit.rbeg = u[1]; unit.rend = u[2]; unit.slot = u[3];
-    } else if (!locate_dw_unit(p, xcd + kXcds * k, unit)) {
-        return;
-    }
-    const int e = __builtin_amdgcn_readfirstlane(unit.e);
-    const int rbeg = __builtin_amdgcn_readfirstlane(unit.rbeg), rend = __builtin_amdgcn_readfirstlane(unit.rend);
-    const int slot = __builtin_amdgcn_readfirstlane(unit.slot);
-    const int m0 = p.by_n_tiles.quotient(tile, tile_n) * T::BM, n0 = tile_n * T::BN;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / MTS_WAVE), lane = threadIdx.x % MTS_WAVE;
     const int nk = (rend - rbeg + T::BKS - 1) / T::BKS;
 
@@ -2026,7 +2032,8 @@ __device__ __forceinline__ void dw_gemm_ws_block(const DwParams& p, bf16_t* smem
         static_assert(T::RPI_A == 2 && T::RPI_B == 2 && T::CPR_A == T::CPR_B, "two rows per wave instruction");
         static_assert(ROWS_A == ROWS_B && (ROWS_A == 8 || ROWS_A == 16), "index fetch layout: 8 or 16 rows per producer wave");
         const bool upper = lane >= T::CPR_A;
-        const uint32_t ld_a = (uint32_t)p.M * 2u, ld_b = (uint32_t)p.N * 2u;   // row pitch in bytes
+        const int ldp = p.M + p.p_pad;
+        const uint32_t ld_a = (uint32_t)ldp * 2u, ld_b = (uint32_t)p.N * 2u;   // row pitch in bytes
         uint32_t col_a[T::A_INSTR], col_b[T::B_INSTR], fix_a[T::A_INSTR], fix_b[T::B_INSTR];
         int rin_a[T::A_INSTR], rin_b[T::B_INSTR];
 #pragma unroll
@@ -2069,7 +2076,7 @@ __device__ __forceinline__ void dw_gemm_ws_block(const DwParams& p, bf16_t* smem
                     __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_p, MTS_LDS_PTR(sa + j * 512), 16, (int)off, 0, 0, 0);
                 }
             } else {
-                const __amdgpu_buffer_rsrc_t rs = make_rsrc(p.P + (int64_t)r0 * p.M, (int64_t)left * p.M * 2);
+                const __amdgpu_buffer_rsrc_t rs = make_rsrc(p.P + (int64_t)r0 * ldp, (int64_t)left * ldp * 2);
 #pragma unroll
                 for (int j = 0; j < T::A_INSTR; ++j)
                     __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, MTS_LDS_PTR(sa + j * 512), 16, (int)fix_a[j], 0, 0, 0);
@@ -2208,13 +2215,32 @@ __device__ __forceinline__ void dw_gemm_ws_block(const DwParams& p, bf16_t* smem
 
     // LDS that nothing reads or lands in any more: with two buffers the one that the last k-tile is not in
     bf16_t* stage = S == 2 ? smem + (nk & 1) * T::STAGE : smem;
-    if (slot >= 0) {   // a row chunk: the whole fp32 tile goes to the unit's slot of the workspace
-        float* part = p.part + ((int64_t)slot * p.tiles_per_expert + tile) * (int64_t)(T::BM * T::BN);
-        dw_epilogue<T>(acc, stage, part, T::BN, T::BM, T::BN, wm, wn);
+    if (part) dw_epilogue<T>(acc, stage, part, T::BN, T::BM, T::BN, wm, wn);
+    else dw_epilogue<T>(acc, stage, C, p.N, p.M - m0, p.N - n0, wm, wn);
+}
+
+// the work of block `block` of a launch
+template <class T, typename OutT>
+__device__ __forceinline__ void dw_gemm_ws_block(const DwParams& p, bf16_t* smem, int block) {
+    // all tiles of a unit (an expert, or a row chunk of an over-full one) run on one XCD
+    const int xcd = block % kXcds, jb = block / kXcds;
+    DwUnit unit;
+    int tile, tile_n;
+    const int k = p.by_tiles.quotient(jb, tile);
+    if (p.sched) {
+        if (k >= p.sched[kSchedCounts + xcd]) return;
+        const int32_t* u = p.sched + kSchedUnits + (xcd * p.sched_slots + k) * 4;
+        unit.e = u[0]; unit.rbeg = u[1]; unit.rend = u[2]; unit.slot = u[3];
+    } else if (!locate_dw_unit(p, xcd + kXcds * k, unit)) {
         return;
     }
-    OutT* C = reinterpret_cast<OutT*>(p.C) + (int64_t)e * p.M * p.N + (int64_t)m0 * p.N + n0;
-    dw_epilogue<T>(acc, stage, C, p.N, p.M - m0, p.N - n0, wm, wn);
+    const int e = __builtin_amdgcn_readfirstlane(unit.e);
+    const int rbeg = __builtin_amdgcn_readfirstlane(unit.rbeg), rend = __builtin_amdgcn_readfirstlane(unit.rend);
+    const int slot = __builtin_amdgcn_readfirstlane(unit.slot);
+    const int m0 = p.by_n_tiles.quotient(tile, tile_n) * T::BM, n0 = tile_n * T::BN;
+    // a row chunk: the whole fp32 tile goes to the unit's slot of the workspace
+    float* part = slot >= 0 ? p.part + ((int64_t)slot * p.tiles_per_expert + tile) * (int64_t)(T::BM * T::BN) : nullptr;
+    dw_gemm_ws_tile<T, OutT>(p, smem, rbeg, rend, m0, n0, part, reinterpret_cast<OutT*>(p.C) + (int64_t)e * p.M * p.N + (int64_t)m0 * p.N + n0);
 }
 
 template <class T, typename OutT>
@@ -3126,7 +3152,150 @@ __global__ __launch_bounds__(256) void linear_dw_sum_kernel(const f32x4* __restr
     dw[i] = sum;
 }
 #endif
+// Many tiles (the vocabulary's projection): whole rounds of the chip's CUs, and the tiles behind the last of them cut over the reduction so
+// that they make a round of short blocks, whose fp32 tiles a second kernel adds in their order.  A block costs its k-tiles and about six
+// more (its start, its epilogue); an XCD's blocks are neighbouring tiles, which share the operand that is read once.
+// Bound by the matrix units at the clock they are held to.  24 576 rows, a vocabulary of 50 257, 768 wide: 288 tiles of dX are 1.13 rounds of
+// 786 k-tiles, 591 of dW 2.31 of 384, which left to whole tiles are two and three rounds of time; cut they cost 885 and 896 k-tiles,
+// 1415 and 1476 us (1.34 and 1.29 PFLOP/s), the library's products 2260 and 2030 and a widening copy of 27.
+constexpr int kChipCus = kXcds * kCusPerXcd, kLinearMaxParts = 16, kLinearMaxUnits = 3 * kChipCus;
+struct LinearRounds {
+    int k_tiles, whole, rest, parts, per_part, per_xcd;   // tiles left whole, tiles that are cut, parts of those, k-tiles of a part, parts an XCD
+    Divider by_rest, by_n_tiles;
+};
+LinearRounds linear_rounds(int64_t m_tiles, int n_tiles, int64_t k) {
+    LinearRounds r = {};
+    const int tiles = (int)(m_tiles * n_tiles);
+    r.k_tiles = (int)((k + WsWide::BKS - 1) / WsWide::BKS);
+    r.rest = tiles % kChipCus;
+    r.whole = tiles - r.rest;
+    float best = 0.f;
+    for (int s = 1; s <= kLinearMaxParts && s <= r.k_tiles && (s == 1 || r.rest * s <= kLinearMaxUnits); ++s) {
+        const int per = (r.k_tiles + s - 1) / s, parts = (r.k_tiles + per - 1) / per;   // no part is empty
+        const float cost = (float)((r.rest * parts + kChipCus - 1) / kChipCus * (per + 6)) + (parts > 1 ? 4.f + 0.1f * (float)(r.rest * parts) : 0.f);
+        if (s == 1 || cost < best) best = cost, r.parts = parts, r.per_part = per;
+    }
+    r.per_xcd = (r.rest * r.parts + kXcds - 1) / kXcds;
+    r.by_rest.set(r.rest > 0 ? r.rest : 1);
+    r.by_n_tiles.set(n_tiles);
+    return r;
+}
+int linear_blocks(const LinearRounds& r) { return r.whole + r.per_xcd * kXcds; }
+int64_t linear_part_bytes(const LinearRounds& r) { return r.parts > 1 ? (int64_t)r.rest * r.parts * WsWide::BM * WsWide::BN * 4 : 0; }
+
+struct LinearUnit {
+    int m0, n0, k0, k_len;   // k_len: whole k-tiles, the last one may be ragged
+    int slot;                // of the partial results, -1: none
+};
+__device__ __forceinline__ bool locate_linear_unit(const LinearRounds& r, int block, LinearUnit& u) {
+    const int xcd = block % kXcds;
+    int tile, k_tile = 0, k_tiles = r.k_tiles;
+    u.slot = -1;
+    if (block < r.whole) {
+        tile = xcd * (r.whole / kXcds) + block / kXcds;
+    } else {
+        const int i = xcd * r.per_xcd + (block - r.whole) / kXcds;
+        if (i >= r.rest * r.parts) return false;
+        k_tile = r.by_rest.quotient(i, tile) * r.per_part;
+        k_tiles = k_tiles - k_tile < r.per_part ? k_tiles - k_tile : r.per_part;
+        tile += r.whole;
+        if (r.parts > 1) u.slot = i;
+    }
+    int n_tile;
+    u.m0 = r.by_n_tiles.quotient(tile, n_tile) * WsWide::BM;
+    u.n0 = n_tile * WsWide::BN;
+    u.k0 = k_tile * WsWide::BKS;
+    u.k_len = k_tiles * WsWide::BKS;
+    return true;
+}
+static_assert(WsWide::BM == DwWsWide::BM && WsWide::BN == DwWsWide::BN && WsWide::BKS == DwWsWide::BKS, "one division for both gradients");
+
+__global__ __launch_bounds__(DwWsWide::NT) void linear_dw_rounds_kernel(DwParams p, LinearRounds r) {
+    __shared__ __attribute__((aligned(1024))) bf16_t smem[DwWsWide::LDS_ELEMS];
+    LinearUnit u;
+    if (!locate_linear_unit(r, blockIdx.x, u)) return;
+    const int rend = u.k0 + u.k_len < p.TK ? u.k0 + u.k_len : (int)p.TK;
+    float* part = u.slot >= 0 ? p.part + (int64_t)u.slot * (DwWsWide::BM * DwWsWide::BN) : nullptr;
+    dw_gemm_ws_tile<DwWsWide, float>(p, smem, u.k0, rend, u.m0, u.n0, part, (float*)p.C + (int64_t)u.m0 * p.N + u.n0);
+}
+
+__global__ __launch_bounds__(WsWide::NT, WsWide::WAVES_PER_EU) void linear_dx_rounds_kernel(RowsParams p, LinearRounds r) {
+    __shared__ __attribute__((aligned(1024))) bf16_t smem[ws_lds_elems<WsWide, EPI_SPLIT>()];
+    LinearUnit u;
+    if (!locate_linear_unit(r, blockIdx.x, u)) return;
+    p.A += u.k0;
+    p.B += (int64_t)u.k0 * p.N;
+    p.Kdim = u.k_len < p.Kdim - u.k0 ? u.k_len : p.Kdim - u.k0;
+    p.part = u.slot >= 0 ? p.part + (int64_t)u.slot * (WsWide::BM * WsWide::BN) : nullptr;
+    const int rend = u.m0 + WsWide::BM < p.TK ? u.m0 + WsWide::BM : (int)p.TK;
+    rows_gemm_ws_tile<WsWide, EPI_SPLIT, true>(p, smem, 0, u.m0, rend, u.n0 / WsWide::BN);
+}
+
+// the parts of the tiles that were cut -> C [rows, cols]
+template <typename OutT>
+__global__ __launch_bounds__(256) void linear_tile_sum_kernel(const f32x4* __restrict__ part, LinearRounds r, int64_t rows, int cols, OutT* __restrict__ C) {
+    constexpr int QUADS = WsWide::BM * WsWide::BN / 4, PER_ROW = WsWide::BN / 4;
+    const int rest = blockIdx.x / (QUADS / 256), q = blockIdx.x % (QUADS / 256) * 256 + threadIdx.x;
+    int n_tile;
+    const int64_t row = (int64_t)r.by_n_tiles.quotient(r.whole + rest, n_tile) * WsWide::BM + q / PER_ROW;
+    const int col = n_tile * WsWide::BN + q % PER_ROW * 4;
+    if (row >= rows || col >= cols) return;
+    part += (int64_t)rest * QUADS + q;
+    f32x4 sum = part[0];
+#pragma unroll 4
+    for (int s = 1; s < r.parts; ++s) {
+        const f32x4 v = part[(int64_t)s * r.rest * QUADS];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) sum[j] += v[j];
+    }
+    OutT* c = C + row * cols + col;
+    if constexpr (sizeof(OutT) == 4) *reinterpret_cast<f32x4*>(c) = sum;
+    else stage4(c, sum[0], sum[1], sum[2], sum[3]);
+}
+template <typename OutT>
+int launch_linear_tile_sum(const float* part, const LinearRounds& r, int64_t rows, int cols, OutT* C, hipStream_t s) {
+    if (r.parts == 1) return MTS_OK;
+    linear_tile_sum_kernel<OutT><<<dim3((unsigned)(r.rest * (WsWide::BM * WsWide::BN / 4 / 256))), 256, 0, s>>>((const f32x4*)part, r, rows, cols, C);
+    MTS_CHECK_LAUNCH();
+    return MTS_OK;
+}
+LinearRounds linear_dw_rounds(int64_t T, int N, int K) {
+    return linear_rounds((N + DwWsWide::BM - 1) / DwWsWide::BM, (K + DwWsWide::BN - 1) / DwWsWide::BN, T);
+}
+LinearRounds linear_dx_rounds(int64_t T, int N, int K) {
+    return linear_rounds((T + WsWide::BM - 1) / WsWide::BM, (K + WsWide::BN - 1) / WsWide::BN, N);
+}
 }  // namespace
+
+#ifdef MTS_GEMM_F16
+extern "C" int mts_linear_dw_rounds_f16(const void* g, int64_t ldg, const void* x, int64_t T, int N, int K, float* dw, float* part, void* stream) {
+#else
+static int linear_dw_rounds_launch(const void* g, int64_t ldg, const void* x, int64_t T, int N, int K, float* dw, float* part, void* stream) {
+#endif
+    const LinearRounds r = linear_dw_rounds(T, N, K);
+    DwParams p = {};
+    p.P = (const bf16_t*)g; p.p_rows = T; p.p_pad = (int)(ldg - N);
+    p.Q = (const bf16_t*)x; p.q_rows = T;
+    p.M = N; p.N = K; p.TK = T; p.C = dw; p.part = part;
+    linear_dw_rounds_kernel<<<dim3((unsigned)linear_blocks(r)), DwWsWide::NT, 0, (hipStream_t)stream>>>(p, r);
+    MTS_CHECK_LAUNCH();
+    return launch_linear_tile_sum(part, r, N, K, dw, (hipStream_t)stream);
+}
+
+#ifdef MTS_GEMM_F16
+extern "C" int mts_linear_dx_rounds_f16(const void* g, int64_t ldg, const void* w, int64_t T, int N, int K, void* dx, float* part, void* stream) {
+#else
+static int linear_dx_rounds_launch(const void* g, int64_t ldg, const void* w, int64_t T, int N, int K, void* dx, float* part, void* stream) {
+#endif
+    const LinearRounds r = linear_dx_rounds(T, N, K);
+    RowsParams p = {};
+    p.A = (const bf16_t*)g; p.a_rows = T; p.lda = (int)ldg;
+    p.B = (const bf16_t*)w; p.b_rows = K; p.N = K; p.Kdim = N;
+    p.C = (bf16_t*)dx; p.TK = T; p.part = part;
+    linear_dx_rounds_kernel<<<dim3((unsigned)linear_blocks(r)), WsWide::NT, 0, (hipStream_t)stream>>>(p, r);
+    MTS_CHECK_LAUNCH();
+    return launch_linear_tile_sum(part, r, T, K, (bf16_t*)dx, (hipStream_t)stream);
+}
 
 #ifdef MTS_GEMM_F16
 extern "C" int mts_linear_dw_tiles_f16(const void* g, const void* x, int64_t T, int N, int K, float* part, void* stream) {
@@ -3168,6 +3337,39 @@ extern "C" int mts_linear_dw(const void* g, const void* x, int64_t T, int N, int
     linear_dw_sum_kernel<<<dim3((unsigned)((quads + 255) / 256)), 256, 0, (hipStream_t)stream>>>((const f32x4*)part, segments, quads, (f32x4*)dw);
     MTS_CHECK_LAUNCH();
     return MTS_OK;
+}
+
+// both gradients over whole rounds of tiles: what the kernels can address
+static int linear_rounds_shape(int64_t T, int N, int K, int64_t ldg) {
+    return T >= 1 && T < (1LL << 30) && N >= 1 && K >= 8 && K % 8 == 0 && (int64_t)N * K < (1LL << 30) && ldg >= N && ldg % 8 == 0 && ldg < (1 << 22);
+}
+extern "C" int mts_linear_rounds_supported(int act_dtype, int64_t T, int N, int K, int64_t ldg) {
+    return (act_dtype == MTS_BF16 || act_dtype == MTS_F16) && linear_rounds_shape(T, N, K, ldg);
+}
+extern "C" int64_t mts_linear_rounds_workspace_bytes(int which, int64_t T, int N, int K) {
+    return linear_part_bytes(which ? linear_dw_rounds(T, N, K) : linear_dx_rounds(T, N, K));
+}
+extern "C" int mts_linear_dw_rounds(const void* g, int64_t ldg, const void* x, int64_t T, int N, int K, int act_dtype, float* dw, void* workspace,
+                                    int64_t workspace_bytes, void* stream) {
+    if (!g || !x || !dw) return MTS_ERR_NULL;
+    if (act_dtype != MTS_BF16 && act_dtype != MTS_F16) return MTS_ERR_DTYPE;
+    if (!linear_rounds_shape(T, N, K, ldg)) return MTS_ERR_SHAPE;
+    const int64_t need = mts_linear_rounds_workspace_bytes(1, T, N, K);
+    if (need && (!workspace || workspace_bytes < need)) return MTS_ERR_WORKSPACE;
+    if (!mts_aligned16(g) || !mts_aligned16(x) || !mts_aligned16(dw) || !mts_aligned16(workspace)) return MTS_ERR_ALIGN;
+    return act_dtype == MTS_F16 ? mts_linear_dw_rounds_f16(g, ldg, x, T, N, K, dw, (float*)workspace, stream)
+                                : linear_dw_rounds_launch(g, ldg, x, T, N, K, dw, (float*)workspace, stream);
+}
+extern "C" int mts_linear_dx_rounds(const void* g, int64_t ldg, const void* w, int64_t T, int N, int K, int act_dtype, void* dx, void* workspace,
+                                    int64_t workspace_bytes, void* stream) {
+    if (!g || !w || !dx) return MTS_ERR_NULL;
+    if (act_dtype != MTS_BF16 && act_dtype != MTS_F16) return MTS_ERR_DTYPE;
+    if (!linear_rounds_shape(T, N, K, ldg)) return MTS_ERR_SHAPE;
+    const int64_t need = mts_linear_rounds_workspace_bytes(0, T, N, K);
+    if (need && (!workspace || workspace_bytes < need)) return MTS_ERR_WORKSPACE;
+    if (!mts_aligned16(g) || !mts_aligned16(w) || !mts_aligned16(dx) || !mts_aligned16(workspace)) return MTS_ERR_ALIGN;
+    return act_dtype == MTS_F16 ? mts_linear_dx_rounds_f16(g, ldg, w, T, N, K, dx, (float*)workspace, stream)
+                                : linear_dx_rounds_launch(g, ldg, w, T, N, K, dx, (float*)workspace, stream);
 }
 #endif
 

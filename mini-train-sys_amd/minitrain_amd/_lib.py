@@ -90,10 +90,15 @@ SIGNATURES = {
     "mts_linear_dw_supported": (_i, [_i, _l, _i, _i]),
     "mts_linear_dw_workspace_bytes": (_l, [_l, _i, _i]),
     "mts_linear_dw": (_i, [_p, _p, _l, _i, _i, _i, _p, _p, _l, _p]),
+    "mts_linear_rounds_supported": (_i, [_i, _l, _i, _i, _l]),
+    "mts_linear_rounds_workspace_bytes": (_l, [_i, _l, _i, _i]),
+    "mts_linear_dw_rounds": (_i, [_p, _l, _p, _l, _i, _i, _i, _p, _p, _l, _p]),
+    "mts_linear_dx_rounds": (_i, [_p, _l, _p, _l, _i, _i, _i, _p, _p, _l, _p]),
     "mts_attention_supported": (_i, [_l, _i, _l, _i]),
     "mts_attention_fwd": (_i, [_p, _p, _p, _l, _i, _l, _i, _i, _p, _p, _p]),
     "mts_attention_bwd": (_i, [_p, _p, _p, _p, _p, _p, _l, _i, _l, _i, _i, _p, _p, _p, _p, _p]),
     "mts_cross_entropy_bwd": (_i, [_p, _p, _l, _i, _l, _i, _p, _p, _p, _p, _p, _p]),
+    "mts_cross_entropy_bwd_pitched": (_i, [_p, _p, _l, _i, _l, _i, _p, _p, _p, _p, _p, _l, _p]),
 }
 
 

@@ -88,7 +88,8 @@ class HipOpsBackend(DenseTorchOps):
         return super().cross_entropy(logits, targets)
 
     def fused_linear_cross_entropy(self, x, weight, targets):
-        return self.cross_entropy(F.linear(x, weight), targets)
+        logits = self.linear(x, weight)
+        return self.cross_entropy(F.linear(x, weight) if logits is None else logits, targets)
 
     def expert_counts(self, expert_indices, num_experts):
         """Extension: routes per expert (int32 ``[E]``) without a host synchronisation."""

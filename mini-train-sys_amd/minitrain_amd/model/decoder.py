@@ -178,7 +178,7 @@ class MiniTransformer(nn.Module):
             )
             output = hidden
         else:
-            output = self.lm_head(hidden)
+            output = project(self.lm_head, hidden, self.ops)
             lm_loss = self.ops.cross_entropy(output.reshape(-1, output.size(-1)), targets.reshape(-1))
         weighted_aux = self.cfg.router_aux_loss_coef * self._router_aux
         weighted_z = self.cfg.router_z_loss_coef * self._router_z

@@ -35,6 +35,69 @@ def test_linear(T, N, K, dtype):
     assert w.grad.dtype == torch.float32
 
 
+@pytest.mark.parametrize("T,N,K,pad", [(128, 64, 8, 0), (131, 67, 8, 5), (300, 1003, 120, 21), (1025, 2112, 264, 0), (520, 9001, 1000, 7), (66000, 67, 8, 61), (66000, 64, 8, 8),
+                                       (130, 66001, 8, 7)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_linear_in_rounds(T, N, K, pad, dtype):
+    """Outputs of at least eight times the input's width: reductions of one k-tile and of many, cut and whole, with every remainder of the
+    16-byte chunks; more tiles than the chip has CUs; rows of the gradient that are further apart, with NaN between them."""
+    print(f"linear in rounds T={T} N={N} K={K} pad={pad} {dtype}", flush=True)
+    g = torch.Generator().manual_seed(T)
+    x = torch.randn(T, K, generator=g).to(dtype).cuda().requires_grad_(True)
+    w = (torch.randn(N, K, generator=g) * K ** -0.5).cuda().requires_grad_(True)
+    rows = torch.full((T, N + pad), float("nan"), dtype=dtype, device="cuda")
+    grad = rows[:, :N]
+    grad.copy_(torch.randn(T, N, generator=g))
+    with torch.autocast("cuda", dtype=dtype):
+        y = hip_backend().linear(x, w)
+    y.backward(grad)
+    wide = w.detach().to(dtype).double()
+    for got, want, tol, what in ((x.grad, grad.double() @ wide, ULP[dtype], "dx"), (w.grad, grad.double().T @ x.detach().double(), 1e-5, "dw")):
+        err, scale = float((got.double() - want).abs().max()), float(want.abs().max())
+        assert err <= tol * scale, (what, err, scale)
+    assert w.grad.dtype == torch.float32
+
+
+@pytest.mark.parametrize("N", [64, 67])
+@pytest.mark.parametrize("layout", ["dense", "every other column", "misaligned", "gradient of one value"])
+def test_gradients_in_other_layouts_in_rounds(layout, N):
+    """What the kernels read in place and what they do not: the same products (those of the library are rounded to 16 bits)."""
+    print(f"linear in rounds, {layout}, {N} columns", flush=True)
+    g = torch.Generator().manual_seed(6)
+    r = lambda *shape: torch.randn(*shape, generator=g).bfloat16().cuda()
+    grad = {"dense": lambda: r(200, N), "every other column": lambda: r(200, 2 * N)[:, ::2], "misaligned": lambda: r(200, 80)[:, 1:N + 1],
+            "gradient of one value": lambda: torch.ones((), device="cuda", dtype=torch.bfloat16).expand(200, N)}[layout]()
+    x, w = r(200, 8).requires_grad_(True), torch.randn(N, 8, generator=g).cuda().requires_grad_(True)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        y = hip_backend().linear(x, w)
+    y.backward(grad)
+    for got, want in ((x.grad, grad.double() @ w.detach().bfloat16().double()), (w.grad, grad.double().T @ x.detach().double())):
+        assert float((got.double() - want).abs().max()) <= ULP[torch.bfloat16] * float(want.abs().max())
+
+
+@pytest.mark.parametrize("rows,V", [(130, 64), (200, 1003), (129, 50257)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_loss_on_a_projection(rows, V, dtype):
+    """The gradient of the logits of a projection has rows that start on 16 bytes, with the values that a leaf's has."""
+    print(f"loss on a projection {rows}x{V} {dtype}", flush=True)
+    g = torch.Generator().manual_seed(V)
+    x, w = torch.randn(1, rows, 8, generator=g).to(dtype).cuda().requires_grad_(True), torch.randn(V, 8, generator=g).cuda().requires_grad_(True)
+    targets = torch.randint(0, V, (rows,), generator=g).cuda()
+    targets[1] = -100
+    ops = hip_backend()
+    with torch.autocast("cuda", dtype=dtype):
+        logits = ops.linear(x, w)
+        seen = []
+        logits.register_hook(seen.append)
+        ops.cross_entropy(logits.reshape(-1, V), targets).backward()
+    leaf = logits.detach().view(-1, V).requires_grad_(True)
+    ops.cross_entropy(leaf, targets).backward()
+    assert torch.equal(seen[0].view(-1, V), leaf.grad) and leaf.grad.is_contiguous()
+    assert seen[0].stride(1) % 8 == 0 and logits.is_contiguous()
+    for got, want, tol in ((x.grad[0], leaf.grad.double() @ w.detach().to(dtype).double(), ULP[dtype]), (w.grad, leaf.grad.double().T @ x.detach()[0].double(), 1e-5)):
+        assert float((got.double() - want).abs().max()) <= tol * float(want.abs().max())
+
+
 @pytest.mark.parametrize("layout", ["sequence first", "every other row", "part of a wider row", "misaligned", "gradient of one value"])
 def test_layouts(layout):
     """Operands and gradients that are not dense or not aligned go through a copy: the same sums."""
