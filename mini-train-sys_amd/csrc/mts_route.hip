@@ -57,8 +57,10 @@ __global__ __launch_bounds__(kThreads) void route_hist_kernel(const int32_t* __r
     }
 }
 
-// One block.  Wave w owns experts w, w+nw, ...: exclusive scan over chunks in
-// groups of 64, then an exclusive scan of the totals over experts.
+// One block.  A column of threads for every expert, `width` columns at a time, and in a column `sets` threads that take a run of chunks
+// each: their counters in batches of eight loads, whole lines a row; the runs' sums meet in LDS.  Then an exclusive scan of the totals over
+// experts.  (A wave that walked an expert's chunks by lanes waited for a strided load and a store for every 64 chunks of every expert: 11 us
+// for 128 chunks of 64 experts, now 4.8.)
 // E: experts of this window; counts / expert_start point at the window's first expert, whose id is e0.
 // For e0 > 0 the rows and tiles used by the earlier windows are read from expert_start[0] (the
 // sentinel the pass before wrote) and tile_count[0].
@@ -72,18 +74,45 @@ __device__ __forceinline__ void route_scan_block(
     __shared__ int32_t tile_off[MTS_MAX_EXPERTS + 1];
     const int wave = threadIdx.x / MTS_WAVE, lane = threadIdx.x % MTS_WAVE;
     const int nw = blockDim.x / MTS_WAVE;
-    for (int e = wave; e < E; e += nw) {
-        int32_t carry = 0;
-        for (int64_t c0 = 0; c0 < n_chunks; c0 += MTS_WAVE) {
-            int64_t c = c0 + lane;
-            int32_t v = (c < n_chunks) ? cnt[c * E + e] : 0;
-            const int32_t incl = wave_scan(v);
-            if (c < n_chunks) cnt[c * E + e] = carry + incl - v;
-            carry += __builtin_amdgcn_readlane(incl, MTS_WAVE - 1);
+    constexpr int kBatch = 8;
+    __shared__ int32_t run_sum[1024];
+    int width = 16;
+    while (width < E && width < (int)blockDim.x) width <<= 1;
+    const int sets = blockDim.x / width, set = threadIdx.x / width;
+    const int64_t per = (n_chunks + sets - 1) / sets, c0 = set * per < n_chunks ? set * per : n_chunks;
+    const int64_t c1 = c0 + per < n_chunks ? c0 + per : n_chunks;
+    for (int eb = 0; eb < E; eb += width) {
+        const int e = eb + threadIdx.x % width;
+        int32_t* column = cnt + (e < E ? e : E - 1);
+        int32_t v[kBatch];
+        auto load = [&](int64_t c) {   // zeros behind the run
+#pragma unroll
+            for (int i = 0; i < kBatch; ++i) v[i] = column[(c + i < n_chunks ? c + i : n_chunks - 1) * E];
+#pragma unroll
+            for (int i = 0; i < kBatch; ++i) v[i] = c + i < c1 ? v[i] : 0;
+        };
+        int32_t sum = 0;
+        for (int64_t c = c0; c < c1; c += kBatch) {
+            load(c);
+#pragma unroll
+            for (int i = 0; i < kBatch; ++i) sum += v[i];
         }
-        if (lane == 0) total[e] = carry;
+        run_sum[threadIdx.x] = sum;
+        __syncthreads();
+        int32_t before = 0;
+#pragma unroll 8
+        for (int k = 0; k < set; ++k) before += run_sum[k * width + threadIdx.x % width];
+        if (set == sets - 1 && e < E) total[e] = before + sum;
+        for (int64_t c = c0; c < c1; c += kBatch) {
+            if (per > kBatch) load(c);   // a run of one batch is still there
+#pragma unroll
+            for (int i = 0; i < kBatch; ++i) {
+                if (e < E && c + i < c1) column[(c + i) * E] = before;
+                before += v[i];
+            }
+        }
+        __syncthreads();
     }
-    __syncthreads();
     if (wave == 0) {
         int32_t carry = e0 > 0 ? expert_start[0] : 0, tcarry = (e0 > 0 && tile_count) ? tile_count[0] : 0;
         for (int eb = 0; eb < E; eb += MTS_WAVE) {

@@ -272,13 +272,27 @@ __device__ __forceinline__ void stats_block(
         const int i = i0 + threadIdx.x % width;
         float v = 0.f;
         int32_t c = 0;
-        if (i < E + 2) {
-#pragma unroll 8
-            for (int b = set; b < nblocks; b += sets) {
-                v += partial[(int64_t)b * (E + 2) + i];
-                c += i < E ? partial_counts[(int64_t)b * E + i] : 0;
+        // sixteen rows in flight, whatever the lane: a load that some lanes skip waits for the ones before it
+        const float* p = partial + (i < E + 2 ? i : E + 1);
+        const int32_t* pc = partial_counts + (i < E ? i : E - 1);
+        constexpr int kBatch = 16;
+        for (int b0 = set; b0 < nblocks; b0 += kBatch * sets) {
+            float vb[kBatch];
+            int32_t cb[kBatch];
+#pragma unroll
+            for (int k = 0; k < kBatch; ++k) {
+                const int64_t b = b0 + k * sets < nblocks ? b0 + k * sets : nblocks - 1;
+                vb[k] = p[b * (E + 2)];
+                cb[k] = pc[b * E];
+            }
+#pragma unroll
+            for (int k = 0; k < kBatch; ++k) {
+                const bool there = b0 + k * sets < nblocks;
+                v = there ? v + vb[k] : v;
+                c += there ? cb[k] : 0;
             }
         }
+        if (i >= E) c = 0;
         set_sum[threadIdx.x] = v;
         set_count[threadIdx.x] = c;
         __syncthreads();

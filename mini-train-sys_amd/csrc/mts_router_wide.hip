@@ -4,10 +4,11 @@
 // mts_router_linear.hip.)
 //
 // What bounds it: 2*T*H*E FLOP each way at the instruction's 157 TFLOP/s (7 us for 8192 x 1024 x 64, where x is 17 MB, 4 us),
-// so what matters is that every SIMD has a share: forward, 32 rows x 64 experts per block with k dealt to its four waves;
-// dW_r, whose outputs fill 16 blocks only, the rows cut into chunks and the partial sums added in chunk order.
-// 8192 x 1024, 64 experts, bf16: 23 us forward, 20 + 20 + 6 us backward (the library's fp32 products with a widened copy of x
-// and a narrowed dx took 24 and 110 us).
+// so what matters is that every SIMD has a share: forward, 32 rows x 64 experts per block with k dealt to its eight waves;
+// dW_r, whose outputs fill 16 blocks only, the rows cut into chunks and the partial sums added in chunk order; dx in the same launch, so that
+// the blocks of either fill the CUs that the other leaves.  Loads never depend on a branch (mts_f32_tiles.h).
+// 8192 x 1024, 64 experts, bf16: 15.8 us forward, 29 + 5.5 backward; 22 and 19 + 17 + 6 with branches at the loads, four waves, 2-byte stores
+// of dx and a launch each.  16 384 x 2048, 128 experts: 124 -> 95 and 210 -> 188.
 #include "mts_f32_tiles.h"
 
 #include <type_traits>
@@ -16,17 +17,21 @@ namespace {
 
 using namespace mts_f32;
 
-constexpr int kThreads = kTileThreads;
+constexpr int kThreads = 256, kLogitsThreads = 512;
+constexpr int kBwdLds = 2 * (64 * 20 + 16 * 72);   // floats: the two buffers of dx
 
-// 32 rows x 64 experts; wave w multiplies k-steps 2w and 2w+1 of every 64-wide k-tile, the four sums meet in LDS
+// 32 rows x 64 experts; wave w multiplies k-step w of every 64-wide k-tile, the eight sums meet in LDS.  Two waves of a SIMD: one reads its
+// fragments while the other multiplies (four waves of two k-steps each: 19.9 us for 8192 x 1024 x 64 where this takes 15.8).
 template <typename XT>
-__global__ __launch_bounds__(kThreads) void wide_logits_kernel(const XT* __restrict__ x, const float* __restrict__ w, int64_t T, int H, int E,
-                                                               float* __restrict__ logits) {
-    constexpr int BM = 32, BN = 64, TKS = 64, STEPS = TKS / 8 / 4;
-    typedef RowTile<XT, BM, TKS, true> AT;
-    typedef RowTile<float, BN, TKS, true> BT;
-    __shared__ __attribute__((aligned(16))) float As[2][AT::SIZE];
-    __shared__ __attribute__((aligned(16))) float Bs[2][BT::SIZE];
+__global__ __launch_bounds__(kLogitsThreads) void wide_logits_kernel(const XT* __restrict__ x, const float* __restrict__ w, int64_t T, int H, int E,
+                                                                     float* __restrict__ logits) {
+    constexpr int BM = 32, BN = 64, TKS = 64, WAVES = kLogitsThreads / MTS_WAVE, STEPS = TKS / 8 / WAVES;
+    typedef RowTile<XT, BM, TKS, true, kLogitsThreads> AT;
+    typedef RowTile<float, BN, TKS, true, kLogitsThreads> BT;
+    constexpr int TILES = 2 * (AT::SIZE + BT::SIZE), SUMS = WAVES * BM * BN;
+    __shared__ __attribute__((aligned(16))) float lds[TILES > SUMS ? TILES : SUMS];
+    float(*As)[AT::SIZE] = reinterpret_cast<float(*)[AT::SIZE]>(lds);
+    float(*Bs)[BT::SIZE] = reinterpret_cast<float(*)[BT::SIZE]>(lds + 2 * AT::SIZE);
     const int64_t row0 = (int64_t)blockIdx.x * BM;
     const int e0 = blockIdx.y * BN;
     AT a;
@@ -34,12 +39,12 @@ __global__ __launch_bounds__(kThreads) void wide_logits_kernel(const XT* __restr
 #pragma unroll
     for (int q = 0; q < AT::LOADS; ++q) {
         const int64_t r = row0 + AT::row(q);
-        a.ptr[q] = r < T ? x + r * H : nullptr;
+        a.ptr[q] = x + (r < T ? r : T - 1) * H;
     }
 #pragma unroll
     for (int q = 0; q < BT::LOADS; ++q) {
         const int e = e0 + BT::row(q);
-        b.ptr[q] = e < E ? w + (int64_t)e * H : nullptr;
+        b.ptr[q] = w + (int64_t)(e < E ? e : E - 1) * H;
     }
     const int wave = threadIdx.x / MTS_WAVE, lane = threadIdx.x % MTS_WAVE;
     f32x16 acc[1][2] = {};
@@ -47,102 +52,143 @@ __global__ __launch_bounds__(kThreads) void wide_logits_kernel(const XT* __restr
         a.fetch(set, t * TKS, H);
         b.fetch(set, t * TKS, H);
     };
-    run_k_tiles<AT, BT, STEPS, 1, 2>((H + TKS - 1) / TKS, a, b, As, Bs, acc, [](int) { return 0; }, [](int nf) { return nf * 32; }, fetch, wave * STEPS);
-    // the waves' sums, in wave order
-    float* sums = &Bs[0][0];   // [32][64]
-    static_assert(2 * BT::SIZE >= BM * BN, "the sums fit the weight buffers");
-#pragma unroll 1
-    for (int k = 0; k < 4; ++k) {
-        if (wave == k) {
+    run_k_tiles<AT, BT, TKS, STEPS, 1, 2, true>(H, a, b, As, Bs, acc, [](int) { return 0; }, [](int nf) { return nf * 32; }, fetch, wave * STEPS);
+    // a lane holds runs of four experts of row lane % 32; the groups of four of a row are dealt by the row
+    const int ml = lane % 32;
+    float* mine = lds + wave * BM * BN + ml * BN;
 #pragma unroll
-            for (int nf = 0; nf < 2; ++nf)
+    for (int nf = 0; nf < 2; ++nf)
 #pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    float* s = sums + (8 * (i / 4) + 4 * (lane / 32) + i % 4) * BN + nf * 32 + lane % 32;
-                    *s = k ? *s + acc[0][nf][i] : acc[0][nf][i];
-                }
+        for (int j = 0; j < 4; ++j) {
+            const f32x4 v = {acc[0][nf][4 * j], acc[0][nf][4 * j + 1], acc[0][nf][4 * j + 2], acc[0][nf][4 * j + 3]};
+            *reinterpret_cast<f32x4*>(mine + (((nf * 8 + 2 * j + lane / 32) ^ (ml & 15)) << 2)) = v;
         }
-        __syncthreads();
+    __syncthreads();
+    static_assert(BM * BN / 4 == kLogitsThreads, "four sums a thread");
+    const int m = threadIdx.x / (BN / 4), g = threadIdx.x % (BN / 4);
+    const int64_t r = row0 + m;
+    const float* part = lds + m * BN + ((g ^ (m & 15)) << 2);
+    f32x4 sum = *reinterpret_cast<const f32x4*>(part);
+#pragma unroll
+    for (int k = 1; k < WAVES; ++k) {   // in wave order
+        const f32x4 v = *reinterpret_cast<const f32x4*>(part + k * BM * BN);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) sum[j] += v[j];
     }
-    for (int i = threadIdx.x; i < BM * BN; i += kThreads) {
-        const int64_t r = row0 + i / BN;
-        const int e = e0 + i % BN;
-        if (r < T && e < E) logits[r * E + e] = sums[i];
+    if (r >= T) return;
+    float* out = logits + r * E + e0 + 4 * g;
+    if (E % 4 == 0) {
+        if (e0 + 4 * g < E) *reinterpret_cast<f32x4*>(out) = sum;
+    } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (e0 + 4 * g + j < E) out[j] = sum[j];
     }
 }
 
 // dx[t,h] = sum_e dlogits[t,e] * w_r[e,h], 64 x 64 per block
 template <typename XT, bool VEC>
-__global__ __launch_bounds__(kThreads) void wide_dx_kernel(const float* __restrict__ dl, const float* __restrict__ w, int64_t T, int H, int E,
-                                                           XT* __restrict__ dx) {
+__device__ __forceinline__ void wide_dx_block(const float* __restrict__ dl, const float* __restrict__ w, int64_t T, int H, int E, XT* __restrict__ dx,
+                                              unsigned block, float* lds) {
     constexpr int BM = 64, BN = 64, TKS = 16;
     typedef RowTile<float, BM, TKS, VEC> AT;
     typedef KTile<float, BN, TKS, true> BT;
-    __shared__ __attribute__((aligned(16))) float As[2][AT::SIZE];
-    __shared__ __attribute__((aligned(16))) float Bs[2][BT::SIZE];
+    constexpr int LDO = BN + 16 / (int)sizeof(XT), PER16 = 16 / (int)sizeof(XT);
+    float(*As)[AT::SIZE] = reinterpret_cast<float(*)[AT::SIZE]>(lds);
+    float(*Bs)[BT::SIZE] = reinterpret_cast<float(*)[BT::SIZE]>(lds + 2 * AT::SIZE);
+    XT* staged = reinterpret_cast<XT*>(lds);
+    static_assert(2 * (AT::SIZE + BT::SIZE) <= kBwdLds && BM * LDO * sizeof(XT) <= kBwdLds * sizeof(float), "LDS of a block");
     const int n_tiles = (H + BN - 1) / BN;
-    const int64_t row0 = (int64_t)(blockIdx.x / n_tiles) * BM;
-    const int n0 = blockIdx.x % n_tiles * BN;
+    const int64_t row0 = (int64_t)(block / n_tiles) * BM;
+    const int n0 = block % n_tiles * BN;
     AT a;
     BT b;
 #pragma unroll
     for (int q = 0; q < AT::LOADS; ++q) {
         const int64_t r = row0 + AT::row(q);
-        a.ptr[q] = r < T ? dl + r * E : nullptr;
+        a.ptr[q] = dl + (r < T ? r : T - 1) * E;
     }
-    b.base = w + n0 + BT::col(), b.ld = H, b.cols = H - n0 - BT::col();
+    b.base = w + n0, b.ld = H, b.cols = H - n0;
     const int wave = threadIdx.x / MTS_WAVE, lane = threadIdx.x % MTS_WAVE, wm = wave / 2, wn = wave % 2;
     f32x16 acc[1][1] = {};
     auto fetch = [&](int set, int t) {
         a.fetch(set, t * TKS, E);
         int64_t rows[BT::LOADS];
 #pragma unroll
-        for (int q = 0; q < BT::LOADS; ++q) rows[q] = t * TKS + BT::k(q) < E ? t * TKS + BT::k(q) : -1;
+        for (int q = 0; q < BT::LOADS; ++q) rows[q] = t * TKS + BT::k(q) < E ? t * TKS + BT::k(q) : E - 1;
         b.fetch(set, rows);
     };
-    run_k_tiles<AT, BT, TKS / 8, 1, 1>((E + TKS - 1) / TKS, a, b, As, Bs, acc, [&](int) { return wm * 32; }, [&](int) { return wn * 32; }, fetch);
-    const int n = n0 + wn * 32 + lane % 32;
+    run_k_tiles<AT, BT, TKS, TKS / 8, 1, 1, true>(E, a, b, As, Bs, acc, [&](int) { return wm * 32; }, [&](int) { return wn * 32; }, fetch);
+    // through LDS (the k loop ends with a barrier) into stores of 16 bytes
+    typedef __attribute__((ext_vector_type(4))) XT quad;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const int64_t r = row0 + wm * 32 + 8 * (i / 4) + 4 * (lane / 32) + i % 4;
-        if (r < T && n < H) dx[r * H + n] = (XT)acc[0][0][i];
+    for (int j = 0; j < 4; ++j) {
+        const quad v = {(XT)acc[0][0][4 * j], (XT)acc[0][0][4 * j + 1], (XT)acc[0][0][4 * j + 2], (XT)acc[0][0][4 * j + 3]};
+        *reinterpret_cast<quad*>(staged + (wm * 32 + lane % 32) * LDO + wn * 32 + 8 * j + 4 * (lane / 32)) = v;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = threadIdx.x; i < BM * BN / PER16; i += kThreads) {
+        const int m = i / (BN / PER16), c = i % (BN / PER16) * PER16;
+        const int64_t r = row0 + m;
+        if (r >= T || n0 + c >= H) continue;
+        const XT* from = staged + m * LDO + c;
+        XT* to = dx + r * H + n0 + c;
+        if (H % PER16 == 0) *reinterpret_cast<u32x4*>(to) = *reinterpret_cast<const u32x4*>(from);
+        else {   // rows start on four elements
+            *reinterpret_cast<quad*>(to) = *reinterpret_cast<const quad*>(from);
+            if (PER16 > 4 && n0 + c + 4 < H) *reinterpret_cast<quad*>(to + PER16 - 4) = *reinterpret_cast<const quad*>(from + PER16 - 4);
+        }
     }
 }
 
 // partial dW_r[e,h] over one chunk of rows, 64 x 64 per block
 template <typename XT, bool VEC>
-__global__ __launch_bounds__(kThreads) void wide_dw_kernel(const float* __restrict__ dl, const XT* __restrict__ x, int64_t T, int H, int E,
-                                                           int64_t rows_per_chunk, float* __restrict__ part) {
+__device__ __forceinline__ void wide_dw_block(const float* __restrict__ dl, const XT* __restrict__ x, int64_t T, int H, int E, int64_t rows_per_chunk,
+                                              float* __restrict__ part, unsigned tile, unsigned chunk, float* lds) {
     constexpr int BM = 64, BN = 64, TKS = 16;
     typedef KTile<float, BM, TKS, VEC> PT;
     typedef KTile<XT, BN, TKS, true> QT;
-    __shared__ __attribute__((aligned(16))) float Ps[2][PT::SIZE];
-    __shared__ __attribute__((aligned(16))) float Qs[2][QT::SIZE];
-    const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-    const int64_t r0 = (int64_t)blockIdx.z * rows_per_chunk, r1 = r0 + rows_per_chunk < T ? r0 + rows_per_chunk : T;
+    float(*Ps)[PT::SIZE] = reinterpret_cast<float(*)[PT::SIZE]>(lds);
+    float(*Qs)[QT::SIZE] = reinterpret_cast<float(*)[QT::SIZE]>(lds + 2 * PT::SIZE);
+    static_assert(2 * (PT::SIZE + QT::SIZE) <= kBwdLds, "LDS of a block");
+    const unsigned n_tiles = (unsigned)((H + BN - 1) / BN);
+    const int m0 = tile / n_tiles * BM, n0 = tile % n_tiles * BN;
+    const int64_t r0 = (int64_t)chunk * rows_per_chunk, r1 = r0 + rows_per_chunk < T ? r0 + rows_per_chunk : T;
     PT a;
     QT b;
-    a.base = dl + m0 + PT::col(), a.ld = E, a.cols = E - m0 - PT::col();
-    b.base = x + n0 + QT::col(), b.ld = H, b.cols = H - n0 - QT::col();
+    a.base = dl + m0, a.ld = E, a.cols = E - m0;
+    b.base = x + n0, b.ld = H, b.cols = H - n0;
     const int wave = threadIdx.x / MTS_WAVE, lane = threadIdx.x % MTS_WAVE, wm = wave / 2, wn = wave % 2;
     f32x16 acc[1][1] = {};
     auto fetch = [&](int set, int t) {
         int64_t pr[PT::LOADS], qr[QT::LOADS];
 #pragma unroll
-        for (int q = 0; q < PT::LOADS; ++q) pr[q] = r0 + t * TKS + PT::k(q) < r1 ? r0 + t * TKS + PT::k(q) : -1;
+        for (int q = 0; q < PT::LOADS; ++q) pr[q] = r0 + t * TKS + PT::k(q) < r1 ? r0 + t * TKS + PT::k(q) : r1 - 1;
 #pragma unroll
-        for (int q = 0; q < QT::LOADS; ++q) qr[q] = r0 + t * TKS + QT::k(q) < r1 ? r0 + t * TKS + QT::k(q) : -1;
+        for (int q = 0; q < QT::LOADS; ++q) qr[q] = r0 + t * TKS + QT::k(q) < r1 ? r0 + t * TKS + QT::k(q) : r1 - 1;
         a.fetch(set, pr);
         b.fetch(set, qr);
     };
-    run_k_tiles<PT, QT, TKS / 8, 1, 1>((int)((r1 - r0 + TKS - 1) / TKS), a, b, Ps, Qs, acc, [&](int) { return wm * 32; }, [&](int) { return wn * 32; }, fetch);
-    float* out = part + (int64_t)blockIdx.z * E * H;
+    run_k_tiles<PT, QT, TKS, TKS / 8, 1, 1>((int)(r1 - r0), a, b, Ps, Qs, acc, [&](int) { return wm * 32; }, [&](int) { return wn * 32; }, fetch);
+    float* out = part + (int64_t)chunk * E * H;
     const int n = n0 + wn * 32 + lane % 32;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
         const int m = m0 + wm * 32 + 8 * (i / 4) + 4 * (lane / 32) + i % 4;
         if (m < E && n < H) out[(int64_t)m * H + n] = acc[0][0][i];
     }
+}
+
+// Both gradients, the longer blocks of dW_r first.
+template <typename XT, bool VEC>
+__global__ __launch_bounds__(kThreads) void wide_bwd_kernel(const float* __restrict__ dl, const XT* __restrict__ x, const float* __restrict__ w, int64_t T, int H,
+                                                            int E, int64_t rows_per_chunk, unsigned dw_tiles, unsigned chunks, XT* __restrict__ dx,
+                                                            float* __restrict__ part) {
+    __shared__ __attribute__((aligned(16))) float lds[kBwdLds];
+    const unsigned dw_blocks = dw_tiles * chunks;
+    if (blockIdx.x < dw_blocks) wide_dw_block<XT, VEC>(dl, x, T, H, E, rows_per_chunk, part, blockIdx.x % dw_tiles, blockIdx.x / dw_tiles, lds);
+    else wide_dx_block<XT, VEC>(dl, w, T, H, E, dx, blockIdx.x - dw_blocks, lds);
 }
 
 // Rows are cut into as many chunks as make about two blocks per CU, of at least 64 rows.
@@ -161,7 +207,7 @@ WideChunks wide_chunks(int64_t T, int H, int E) {
 
 int wide_check(const void* x, const float* w_r, int64_t T, int H, int E, int act_dtype) {
     if (!x || !w_r) return MTS_ERR_NULL;
-    if (!mts_router_wide_supported(H, E) || T <= 0 || (T + 63) / 64 * ((H + 63) / 64) >= (1LL << 31)) return MTS_ERR_SHAPE;
+    if (!mts_router_wide_supported(H, E) || T <= 0 || (T + 63) / 64 * ((H + 63) / 64) >= (1LL << 31) - (1 << 20)) return MTS_ERR_SHAPE;
     if (act_dtype != MTS_BF16 && act_dtype != MTS_F16 && act_dtype != MTS_F32) return MTS_ERR_DTYPE;
     if (!mts_aligned16(x) || !mts_aligned16(w_r)) return MTS_ERR_ALIGN;
     return MTS_OK;
@@ -177,9 +223,9 @@ extern "C" int mts_router_wide_fwd(const void* x, const float* w_r, int64_t T, i
     if (!logits) return MTS_ERR_NULL;
     const dim3 grid((unsigned)((T + 31) / 32), (unsigned)((E + 63) / 64));
     hipStream_t s = (hipStream_t)stream;
-    if (act_dtype == MTS_BF16) wide_logits_kernel<bf16_t><<<grid, kThreads, 0, s>>>((const bf16_t*)x, w_r, T, H, E, logits);
-    else if (act_dtype == MTS_F16) wide_logits_kernel<mts_f16_t><<<grid, kThreads, 0, s>>>((const mts_f16_t*)x, w_r, T, H, E, logits);
-    else wide_logits_kernel<float><<<grid, kThreads, 0, s>>>((const float*)x, w_r, T, H, E, logits);
+    if (act_dtype == MTS_BF16) wide_logits_kernel<bf16_t><<<grid, kLogitsThreads, 0, s>>>((const bf16_t*)x, w_r, T, H, E, logits);
+    else if (act_dtype == MTS_F16) wide_logits_kernel<mts_f16_t><<<grid, kLogitsThreads, 0, s>>>((const mts_f16_t*)x, w_r, T, H, E, logits);
+    else wide_logits_kernel<float><<<grid, kLogitsThreads, 0, s>>>((const float*)x, w_r, T, H, E, logits);
     MTS_CHECK_LAUNCH();
     return MTS_OK;
 }
@@ -198,19 +244,14 @@ extern "C" int mts_router_wide_bwd(const float* dlogits, const void* x, const fl
     if (!mts_aligned16(dlogits) || !mts_aligned16(dx) || !mts_aligned16(d_w_r) || !mts_aligned16(workspace)) return MTS_ERR_ALIGN;
     hipStream_t s = (hipStream_t)stream;
     const bool vec = E % 4 == 0;
-    const dim3 grid_dx((unsigned)((T + 63) / 64 * ((H + 63) / 64)));
     const WideChunks c = wide_chunks(T, H, E);
-    const dim3 grid_dw((unsigned)((H + 63) / 64), (unsigned)((E + 63) / 64), (unsigned)c.count);
+    const unsigned dw_tiles = (unsigned)((H + 63) / 64 * ((E + 63) / 64));
+    const dim3 grid((unsigned)(dw_tiles * c.count + (T + 63) / 64 * ((H + 63) / 64)));
     float* part = (float*)workspace;
     auto launch = [&](auto* kind) {
         typedef typename std::remove_pointer<decltype(kind)>::type XT;
-        if (vec) {
-            wide_dx_kernel<XT, true><<<grid_dx, kThreads, 0, s>>>(dlogits, w_r, T, H, E, (XT*)dx);
-            wide_dw_kernel<XT, true><<<grid_dw, kThreads, 0, s>>>(dlogits, (const XT*)x, T, H, E, c.rows, part);
-        } else {
-            wide_dx_kernel<XT, false><<<grid_dx, kThreads, 0, s>>>(dlogits, w_r, T, H, E, (XT*)dx);
-            wide_dw_kernel<XT, false><<<grid_dw, kThreads, 0, s>>>(dlogits, (const XT*)x, T, H, E, c.rows, part);
-        }
+        if (vec) wide_bwd_kernel<XT, true><<<grid, kThreads, 0, s>>>(dlogits, (const XT*)x, w_r, T, H, E, c.rows, dw_tiles, (unsigned)c.count, (XT*)dx, part);
+        else wide_bwd_kernel<XT, false><<<grid, kThreads, 0, s>>>(dlogits, (const XT*)x, w_r, T, H, E, c.rows, dw_tiles, (unsigned)c.count, (XT*)dx, part);
     };
     if (act_dtype == MTS_BF16) launch((bf16_t*)nullptr);
     else if (act_dtype == MTS_F16) launch((mts_f16_t*)nullptr);

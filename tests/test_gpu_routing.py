@@ -63,6 +63,13 @@ def test_against_oracle(T, E, K):
     _compare(idx, E)
 
 
+@pytest.mark.parametrize("T,E,K", [(65536, 16, 2), (65537, 16, 2), (10000, 100, 2), (2048, 65, 8), (40000, 513, 1)])
+def test_runs_of_chunks(T, E, K):
+    """The scan's threads take runs of chunks: whole batches of loads, one chunk more, runs that are empty, a column of threads per expert."""
+    print(f"routing T={T} E={E} K={K}", flush=True)
+    _compare(np.random.default_rng(T).integers(0, E, (T, K)).astype(np.int32), E)
+
+
 @pytest.mark.parametrize("T,E,K,dropped", [(700, 1025, 2, False), (5000, 3000, 4, True), (300, 65534, 2, False),
                                            (4097, 2048, 8, True)])
 def test_more_experts_than_one_window(T, E, K, dropped):
