@@ -15,6 +15,7 @@ namespace {
 constexpr int kSelThreads = 1024;
 constexpr int kSelWaves = kSelThreads / MTS_WAVE;
 constexpr int kUnroll = 4;
+constexpr int kParts = 4;      // blocks per expert
 constexpr int kRegKeys = 32;   // segments of up to 32768 routes keep their keys in registers
 
 // float -> unsigned key with the same order; -0 and +0 get the same key
@@ -34,7 +35,7 @@ __device__ __forceinline__ void count_digit(uint32_t* hist, bool count, uint32_t
         const uint64_t todo = __ballot(count);
         if (!todo) break;
         const int leader = __ffsll((unsigned long long)todo) - 1;
-        const uint32_t dl = (uint32_t)__shfl((int)d, leader, MTS_WAVE);
+        const uint32_t dl = (uint32_t)__builtin_amdgcn_readlane((int)d, leader);
         const uint64_t same = __ballot(count && d == dl);
         if (lane == leader) atomicAdd(&hist[dl], (uint32_t)__popcll(same));
         count = count && d != dl;
@@ -60,13 +61,15 @@ struct CompactOut {
     int32_t* s_scatter;
     int32_t* s_reverse;
     int32_t* x_gather;
-    int first, K;          // first row of the expert's kept entries
+    int first;             // first row of the expert's kept entries
+    uint32_t K, inverse;   // routes per token, floor((2^32 - 1) / K)
     __device__ __forceinline__ void put(int32_t entry, bool kept, uint32_t rank) const {
         const int row = first + (int)rank;
         s_reverse[entry] = kept ? row : -1;
         if (kept) {
             s_scatter[row] = entry;
-            x_gather[row] = entry / K;
+            const uint32_t q = __umulhi((uint32_t)entry, inverse);   // the quotient or one less
+            x_gather[row] = (int32_t)((uint32_t)entry - q * K >= K ? q + 1 : q);
         }
     }
 };
@@ -80,13 +83,7 @@ __device__ __forceinline__ void scan_table(uint32_t* table, int lane) {
         v[j] = table[lane * PER_LANE + j];
         sum += v[j];
     }
-    uint32_t incl = sum;
-#pragma unroll
-    for (int o = 1; o < MTS_WAVE; o <<= 1) {
-        const uint32_t up = __shfl_up(incl, o, MTS_WAVE);
-        if (lane >= o) incl += up;
-    }
-    uint32_t run = incl - sum;
+    uint32_t run = (uint32_t)wave_scan((int)sum) - sum;
 #pragma unroll
     for (int j = 0; j < PER_LANE; ++j) {
         table[lane * PER_LANE + j] = run;
@@ -101,7 +98,7 @@ template <bool REGS, class Out>
 __device__ __forceinline__ void select_segment(const float* __restrict__ w, const int32_t* __restrict__ seg,
                                                uint32_t* __restrict__ kseg, int n, uint32_t capacity, const Out& out,
                                                uint32_t* hist, uint32_t* chosen, uint32_t* wave_ties,
-                                               uint32_t* tie_table, uint32_t* kept_table) {
+                                               uint32_t* tie_table, uint32_t* kept_table, int part) {
     const int tid = threadIdx.x, lane = tid % MTS_WAVE, wave = tid / MTS_WAVE;
     uint32_t kr[REGS ? kRegKeys : 1];
     if (REGS) {
@@ -170,13 +167,9 @@ __device__ __forceinline__ void select_segment(const float* __restrict__ w, cons
             const uint32_t h0 = hist[4 * lane], h1 = hist[4 * lane + 1], h2 = hist[4 * lane + 2],
                            h3 = hist[4 * lane + 3];
             const uint32_t mine = h0 + h1 + h2 + h3;
-            uint32_t suffix = mine;
-#pragma unroll
-            for (int o = 1; o < MTS_WAVE; o <<= 1) {
-                const uint32_t up = __shfl_down(suffix, o, MTS_WAVE);
-                if (lane + o < MTS_WAVE) suffix += up;
-            }
-            uint32_t above = suffix - mine;   // matching keys in the bins of higher lanes
+            const int upto = wave_scan((int)mine);
+            uint32_t above = (uint32_t)(__builtin_amdgcn_readlane(upto, MTS_WAVE - 1) - upto);   // matching keys in the bins of higher lanes
+            const uint32_t suffix = above + mine;
             if (above < need && need <= suffix) {
                 int d;
                 if (above + h3 >= need) d = 3;
@@ -240,10 +233,11 @@ __device__ __forceinline__ void select_segment(const float* __restrict__ w, cons
             if (wave == 0) scan_table(kept_table, lane);
             __syncthreads();
         }
-        constexpr int BATCH = 8;
+        constexpr int BATCH = 4;
 #pragma unroll
         for (int u0 = 0; u0 < kRegKeys; u0 += BATCH) {
-            if (u0 * kSelThreads >= n) break;   // block-uniform
+            if (u0 * kSelThreads >= n) break;   // block-uniform, as the next
+            if (u0 / BATCH % kParts != part) continue;
             int32_t entry[BATCH];
 #pragma unroll
             for (int j = 0; j < BATCH; ++j) {
@@ -290,10 +284,11 @@ __device__ __forceinline__ void select_segment(const float* __restrict__ w, cons
     }
 }
 
-// one expert's segment: everything, nothing, or the selection
+// One expert's segment: everything, nothing, or the selection.  kParts blocks select, all of them the same (on CUs that would
+// idle), and each writes a part of the answer: its scattered stores were a third of the time.
 template <class Out>
 __device__ __forceinline__ void select_expert(const float* __restrict__ w, const int32_t* __restrict__ seg, uint32_t* __restrict__ keys, int n,
-                                              int64_t capacity, const Out& out) {
+                                              int64_t capacity, const Out& out, int part) {
     __shared__ uint32_t hist[256];
     __shared__ uint32_t chosen[2];          // prefix, number still to take inside it
     __shared__ uint32_t wave_ties[kSelWaves];
@@ -301,13 +296,13 @@ __device__ __forceinline__ void select_expert(const float* __restrict__ w, const
     __shared__ uint32_t kept_table[Out::kRanked ? kRegKeys * kSelWaves : 1];
     const bool all = (int64_t)n <= capacity, none = capacity <= 0;
     if (all || none) {   // block-uniform
-        for (int i = threadIdx.x; i < n; i += kSelThreads) out.put(seg[i], !none, (uint32_t)i);
+        for (int i = part * kSelThreads + threadIdx.x; i < n; i += kParts * kSelThreads) out.put(seg[i], !none, (uint32_t)i);
         return;
     }
     if (n <= kRegKeys * kSelThreads)
-        select_segment<true>(w, seg, (uint32_t*)nullptr, n, (uint32_t)capacity, out, hist, chosen, wave_ties, tie_table, kept_table);
-    else
-        select_segment<false>(w, seg, keys, n, (uint32_t)capacity, out, hist, chosen, wave_ties, tie_table, kept_table);
+        select_segment<true>(w, seg, (uint32_t*)nullptr, n, (uint32_t)capacity, out, hist, chosen, wave_ties, tie_table, kept_table, part);
+    else if (part == 0)   // its keys are in memory
+        select_segment<false>(w, seg, keys, n, (uint32_t)capacity, out, hist, chosen, wave_ties, tie_table, kept_table, part);
 }
 
 __device__ __forceinline__ int32_t accepted_of(int n, int64_t capacity) { return capacity <= 0 ? 0 : ((int64_t)n <= capacity ? n : (int32_t)capacity); }
@@ -318,14 +313,14 @@ __global__ __launch_bounds__(kSelThreads) void capacity_select_kernel(
     uint32_t* __restrict__ keys, uint8_t* __restrict__ keep, int32_t* __restrict__ kept_index,
     int32_t* __restrict__ accepted) {
     const int e = blockIdx.x, n = counts[e], first = expert_start[e];
-    if (threadIdx.x == 0) accepted[e] = accepted_of(n, capacity);
-    select_expert(w, s_scatter + first, keys + first, n, capacity, MaskOut{keep, kept_index, e});
+    if (blockIdx.y == 0 && threadIdx.x == 0) accepted[e] = accepted_of(n, capacity);
+    select_expert(w, s_scatter + first, keys + first, n, capacity, MaskOut{keep, kept_index, e}, blockIdx.y);
 }
 
 // The same selection as a compacted permutation: how many routes every expert accepts is known from the counts alone, so
-// every block knows where its expert's kept rows start.  24 576 x 2 routes over 8 experts, half of them over the limit: 31 to 33 us
-// on eight blocks (four counting passes over up to 12 000 keys, then scattered stores), in place of the
-// routing metadata twice (25 us), the mask (34 us) and its application.
+// every block knows where its expert's kept rows start.  24 576 x 2 routes over 8 experts, the fullest with 11 000: 21 us (26 with one
+// block an expert and shuffles through LDS; three passes of 11 bits: 24), four counting passes over an expert's keys
+// and its scattered stores, in place of the routing metadata twice (25 us), the mask (34 us) and its application.
 __global__ __launch_bounds__(kSelThreads) void capacity_compact_kernel(
     const float* __restrict__ w, const int32_t* __restrict__ s_scatter, const int32_t* __restrict__ counts,
     const int32_t* __restrict__ expert_start, int E, int K, int64_t capacity, uint32_t* __restrict__ keys, int32_t* __restrict__ accepted,
@@ -339,13 +334,13 @@ __global__ __launch_bounds__(kSelThreads) void capacity_compact_kernel(
     int32_t kept_first = 0;
 #pragma unroll
     for (int j = 0; j < kSelWaves; ++j) kept_first += in_front[j];
-    if (tid == 0) {
+    if (blockIdx.y == 0 && tid == 0) {
         const int32_t a = accepted_of(n, capacity);
         accepted[e] = a;
         kept_start[e] = kept_first;
         if (e == E - 1) kept_start[E] = kept_first + a;
     }
-    select_expert(w, s_scatter + first, keys + first, n, capacity, CompactOut{kept_scatter, kept_reverse, kept_gather, kept_first, K});
+    select_expert(w, s_scatter + first, keys + first, n, capacity, CompactOut{kept_scatter, kept_reverse, kept_gather, kept_first, (uint32_t)K, 0xffffffffu / (uint32_t)K}, blockIdx.y);
 }
 
 // Weights under a capacity limit: those of dropped routes become zero, a token's others are renormalised (a token may lose
@@ -459,7 +454,7 @@ extern "C" int mts_moe_capacity_mask(const int32_t* top_k_index, const float* to
     capacity_init_kernel<<<(int)(init_blocks < 2048 ? init_blocks : 2048), 256, 0, (hipStream_t)stream>>>(
         TK, keep, kept_index);
     MTS_CHECK_LAUNCH();
-    capacity_select_kernel<<<E, kSelThreads, 0, (hipStream_t)stream>>>(
+    capacity_select_kernel<<<dim3((unsigned)E, kParts), kSelThreads, 0, (hipStream_t)stream>>>(
         top_k_weights, s_scatter, counts, expert_start, capacity, keys, keep, kept_index, accepted_counts);
     MTS_CHECK_LAUNCH();
     return MTS_OK;
@@ -476,7 +471,7 @@ extern "C" int mts_moe_capacity_compact(const float* top_k_weights, const int32_
         return MTS_ERR_NULL;
     if (T <= 0 || K < 1 || E < 1 || E > MTS_MAX_EXPERTS || T * (int64_t)K > 0x7fffffffLL) return MTS_ERR_SHAPE;
     if (workspace_bytes < mts_moe_capacity_compact_workspace_bytes(T, K)) return MTS_ERR_WORKSPACE;
-    capacity_compact_kernel<<<E, kSelThreads, 0, (hipStream_t)stream>>>(top_k_weights, s_scatter, counts, expert_start, E, K, capacity,
+    capacity_compact_kernel<<<dim3((unsigned)E, kParts), kSelThreads, 0, (hipStream_t)stream>>>(top_k_weights, s_scatter, counts, expert_start, E, K, capacity,
                                                                         (uint32_t*)workspace, accepted_counts, kept_start, kept_scatter,
                                                                         kept_reverse, kept_gather);
     MTS_CHECK_LAUNCH();

@@ -48,6 +48,14 @@ def test_mask_matches_oracle(T, K, E, capacity, levels, zipf):
     _check_mask(idx, w, E, capacity)
 
 
+@pytest.mark.parametrize("T", [4095, 4097, 16384, 16385, 20481, 32768, 32769])
+def test_parts_of_a_segment(T):
+    """The answer for one expert's segment is written by several blocks, 4096 positions at a time, each in turn; above 32 768 by one."""
+    print(f"capacity mask, one segment of {T}", flush=True)
+    idx, w = _mask_case(T, T, 1, 1, 50)
+    _check_mask(idx, w, 1, T // 3)
+
+
 def test_mask_on_router_output_with_exact_ties():
     """Weights as the router makes them: K=1 normalised gives 1.0 everywhere, so the whole
     decision rests on the entry order; K=2 on tied logits gives pairs of equal weights."""
