@@ -22,6 +22,7 @@
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/utils/pybind.h>
 
+#include <array>
 #include <cmath>
 #include <map>
 #include <mutex>
@@ -96,7 +97,51 @@ template <typename... Ts>
 bool on_one_gpu(const Tensor& first, const Ts&... others) {
     return first.is_cuda() && ((others.device() == first.device()) && ...);
 }
-int64_t round4(int64_t n) { return (n + 3) / 4 * 4; }
+
+// Contiguous elements of `base`, a dense allocation of bytes, as a tensor of their own.  No view: the parts of an allocation do not overlap, and
+// none of those made this way is handed to a caller who could differentiate through it.
+Tensor part_of(const Tensor& base, int64_t first_byte, at::IntArrayRef size, at::ScalarType type) {
+    auto impl = c10::make_intrusive<c10::TensorImpl>(c10::Storage(base.storage()), base.key_set(), c10::scalarTypeToTypeMeta(type));
+    impl->set_storage_offset(base.storage_offset() + first_byte / (int64_t)c10::elementSize(type));
+    impl->set_sizes_contiguous(size);
+    return Tensor(std::move(impl));
+}
+
+// Tensors of one call that come and go together, in one allocation where that is small: a call of few tokens is bound by the host, which
+// spends about a microsecond on each allocation and on each view (16 tokens 768/1024: a call without gradients 48 -> 36 us, 512 tokens with them 165 -> 137).  Above the limit each
+// has its own, so that no block grows with the sum of the large ones.
+class Together {
+    static constexpr int64_t kMostBytes = 32 << 20;
+    struct Job {
+        Tensor* out;
+        std::array<int64_t, 2> size;
+        int dims;
+        at::ScalarType type;
+        int64_t bytes() const { return (size[0] * (dims > 1 ? size[1] : 1) * (int64_t)c10::elementSize(type) + 255) / 256 * 256; }
+        at::IntArrayRef sizes() const { return at::IntArrayRef(size.data(), (size_t)dims); }
+    };
+    c10::SmallVector<Job, 12> jobs_;
+    const Tensor& like_;
+
+public:
+    explicit Together(const Tensor& like) : like_(like) {}
+    void add(Tensor& out, int64_t rows, int64_t columns, at::ScalarType type) { jobs_.push_back({&out, {rows, columns}, 2, type}); }
+    void add(Tensor& out, int64_t count, at::ScalarType type) { jobs_.push_back({&out, {count, 1}, 1, type}); }
+    void make() {
+        int64_t total = 0;
+        for (const Job& j : jobs_) total += j.bytes();
+        if (total > kMostBytes || jobs_.size() < 2) {
+            for (const Job& j : jobs_) *j.out = at::empty(j.sizes(), like_.options().dtype(j.type));
+            return;
+        }
+        const Tensor base = at::empty({total}, like_.options().dtype(at::kByte));
+        int64_t at_byte = 0;
+        for (const Job& j : jobs_) {
+            *j.out = part_of(base, at_byte, j.sizes(), j.type);
+            at_byte += j.bytes();
+        }
+    }
+};
 
 // ---- contracts ---------------------------------------------------------------------------------------------------------------
 // The first requirement that the arguments miss, or NULL.
@@ -244,18 +289,19 @@ struct Routing {
     Tensor expert_start, x_gather, s_scatter, s_reverse;
 };
 
-// Routing metadata of given expert indices, in one int32 allocation (the per-row arrays start on 16-byte boundaries).
+// Routing metadata of given expert indices (the per-row arrays start on 16-byte boundaries).
 Routing route(const Tensor& index, int64_t E) {
-    const int64_t T = index.size(0), K = index.size(1), TK = T * K, pad = round4(2 * E + 1);
-    Tensor buf = i32({pad + 3 * round4(TK)}, index);
+    const int64_t T = index.size(0), K = index.size(1), TK = T * K, ws_bytes = mts_moe_route_workspace_bytes(T, K, E);
+    Tensor counts, ws;
     Routing r;
-    Tensor counts = buf.narrow(0, 0, E);
-    r.expert_start = buf.narrow(0, E, E + 1);
-    r.s_scatter = buf.narrow(0, pad, TK);
-    r.s_reverse = buf.narrow(0, pad + round4(TK), TK);
-    r.x_gather = buf.narrow(0, pad + 2 * round4(TK), TK);
-    const int64_t ws_bytes = mts_moe_route_workspace_bytes(T, K, E);
-    Tensor ws = bytes(ws_bytes, index);
+    Together together(index);
+    together.add(counts, E, at::kInt);
+    together.add(r.expert_start, E + 1, at::kInt);
+    together.add(r.s_scatter, TK, at::kInt);
+    together.add(r.s_reverse, TK, at::kInt);
+    together.add(r.x_gather, TK, at::kInt);
+    together.add(ws, std::max<int64_t>(ws_bytes, 4), at::kByte);
+    together.make();
     check(mts_moe_route(ptr_as<int32_t>(index), T, K, E, 64, ptr_as<int32_t>(counts), ptr_as<int32_t>(r.expert_start), ptr_as<int32_t>(r.s_scatter),
                         ptr_as<int32_t>(r.s_reverse), ptr_as<int32_t>(r.x_gather), nullptr, nullptr, nullptr, ptr(ws), ws_bytes, stream_of(index)),
           "mts_moe_route");
@@ -288,7 +334,9 @@ struct Saved {
 };
 
 // Gate/up + SwiGLU, down projection and combine for routes that are already sorted.  `weights`: flat, activation dtype.
-Tensor experts_forward(const Tensor& x, const Tensor& w1_in, const Tensor& w2_in, const Tensor& weights, const Routing& r, const Options& opt, Saved& s) {
+// `post_act` [TK,I] and `y` [TK,H]: scratch that the caller has, or undefined
+Tensor experts_forward(const Tensor& x, const Tensor& w1_in, const Tensor& w2_in, const Tensor& weights, const Routing& r, const Options& opt, Saved& s,
+                       Tensor post_act = Tensor(), Tensor y = Tensor()) {
     const int64_t T = x.size(0), H = x.size(1), E = w1_in.size(0), I = w1_in.size(1) / 2, TK = weights.numel(), K = TK / T;
     const auto dtype = x.scalar_type();
     const int act = dtype_code(dtype);
@@ -315,7 +363,9 @@ Tensor experts_forward(const Tensor& x, const Tensor& w1_in, const Tensor& w2_in
     // The routing weight is applied where the activation is formed: post_act = s * silu(g) * u.  The down projection then
     // yields s * y, the combine is a plain sum, and post_act is at the same time the operand of the dW2 GEMM, so it is kept
     // for the backward pass instead of being written again there.
-    Tensor pre_act, post_act = at::empty({TK, I}, x.options()), y = at::empty({TK, H}, x.options());
+    Tensor pre_act;
+    if (!post_act.defined()) post_act = at::empty({TK, I}, x.options());
+    if (!y.defined()) y = at::empty({TK, H}, x.options());
     if (!opt.on(NO_BACKWARD) || dtype == at::kFloat) pre_act = at::empty({TK, 2 * I}, x.options());
     void* route_w = weighted ? ptr(weights) : nullptr;
     int32_t* route_entry = weighted ? ptr_as<int32_t>(r.s_scatter) : nullptr;
@@ -431,6 +481,7 @@ ExpertGrads experts_backward(const Saved& s, Tensor dO, const Needs& need, const
     auto side = [&](int i) { return overlap ? side_stream(device, i) : main; };
     ExpertGrads g;
     Tensor w1_bwd, w2_bwd, d_pre_act, weighted_act, ds_part, ws1, ws2, schedule, dx_expanded;
+    Together temporaries(s.x);
     Forked forked(main);   // behind everything that the side streams touch: joined first
 
     // The ring kernels (16-bit types, widths of whole 64-wide k-tiles or of at least 256) and the fp32 kernels read the
@@ -448,9 +499,7 @@ ExpertGrads experts_backward(const Saved& s, Tensor dO, const Needs& need, const
     w2_bwd = layout && s.staged2.defined() ? s.staged2 : stage(s.w2, !layout, dtype, main);
 
     const bool weighted = s.post_act.defined();
-    d_pre_act = at::empty({TK, 2 * I}, s.x.options());
     weighted_act = weighted ? s.post_act : at::empty({TK, I}, s.x.options());   // s * silu(g) * u
-    ds_part = f32({TK, mts_moe_ds_partials(I)}, s.x);
     // When every gradient is wanted, dW1, dW2, dX and the dS reduction go out as ONE launch whose block order starts the long
     // weight-gradient tiles first; which XCD runs which of its units and dX tiles follows a table that the dO * W2 launch
     // writes on the side (uneven routing).
@@ -464,7 +513,20 @@ ExpertGrads experts_backward(const Saved& s, Tensor dO, const Needs& need, const
     ws2 = dw_workspace(2, need.w2);
     const int64_t ws1_bytes = ws1.defined() ? ws1.numel() : 0, ws2_bytes = ws2.defined() ? ws2.numel() : 0;
     if (joint && opt.on(JOINT_SCHEDULE) && ws1.defined() && ws2.defined() && mts_moe_bwd_schedule_bytes(E) > 0)
-        schedule = i32({mts_moe_bwd_schedule_bytes(E) / 4}, s.x);
+        temporaries.add(schedule, mts_moe_bwd_schedule_bytes(E) / 4, at::kInt);
+    temporaries.add(d_pre_act, TK, 2 * I, dtype);
+    temporaries.add(ds_part, TK, mts_moe_ds_partials(I), at::kFloat);
+    if (need.x) temporaries.add(dx_expanded, TK, H, dtype);
+    // the router's backward rides in the joint launch: it needs nothing the launch writes
+    const bool tail_in_joint = joint && tail && opt.on(TAIL_IN_JOINT) && mts_moe_bwd_joint_router_supported(act, T, H, I, E);
+    const int64_t tail_bytes = tail_in_joint ? mts_moe_head_bwd_workspace_bytes(T, H, E) : 0;
+    Tensor tail_ws;
+    if (tail_in_joint) {
+        temporaries.add(g.ds, T, K, s.weights.scalar_type());
+        temporaries.add(tail->dx_r, T, H, dtype);
+        temporaries.add(tail_ws, std::max<int64_t>(tail_bytes, 4), at::kByte);
+    }
+    temporaries.make();
     check(mts_moe_bwd_dy1(ptr(dO), ptr(w2_bwd), layout, ptr(s.pre_act), ptr(s.weights), ptr_as<int32_t>(s.x_gather), ptr_as<int32_t>(s.s_scatter),
                           ptr_as<int32_t>(s.expert_start), T, K, E, H, I, act, ptr(d_pre_act), weighted ? nullptr : ptr(weighted_act),
                           ptr_as<float>(ds_part), ptr_as<int32_t>(schedule), main),
@@ -480,16 +542,11 @@ ExpertGrads experts_backward(const Saved& s, Tensor dO, const Needs& need, const
     if (joint) {
         g.dw1 = at::empty_like(s.w1);
         g.dw2 = at::empty_like(s.w2);
-        g.ds = at::empty({T, K}, s.weights.options());
-        dx_expanded = at::empty({TK, H}, s.x.options());
+        if (!g.ds.defined()) g.ds = at::empty({T, K}, s.weights.options());
         const int grad = dtype_code(s.w1);
-        if (tail && opt.on(TAIL_IN_JOINT) && mts_moe_bwd_joint_router_supported(act, T, H, I, E)) {
-            // the router's backward as trailing blocks of the same launch: it needs nothing the launch writes
-            tail->dx_r = at::empty_like(s.x);
+        if (tail_in_joint) {
             tail->dw_r = at::empty_like(tail->w_r);
             if (opt.on(COMBINE_IN_TAIL)) g.dx = at::empty_like(s.x);
-            const int64_t ws_bytes = mts_moe_head_bwd_workspace_bytes(T, H, E);
-            Tensor ws = bytes(ws_bytes, s.x);
             check(mts_moe_bwd_joint_router(ptr(dO), ptr(weighted_act), ptr(d_pre_act), ptr(s.x), ptr(w1_bwd), ptr_as<int32_t>(s.x_gather),
                                            ptr_as<int32_t>(s.expert_start), ptr_as<int32_t>(s.s_reverse), ptr_as<float>(ds_part), T, K, E, H, I, act, grad,
                                            ptr(dx_expanded), ptr(g.dw1), ptr(g.dw2), ptr(g.ds), ptr(ws1), ws1_bytes, ptr(ws2), ws2_bytes,
@@ -497,7 +554,7 @@ ExpertGrads experts_backward(const Saved& s, Tensor dO, const Needs& need, const
                                            ptr_as<int32_t>(tail->indices), ptr_as<int32_t>(tail->counts), ptr_as<float>(tail->g_prob_mean),
                                            ptr_as<float>(tail->g_z_loss), ptr_as<float>(tail->g_load_balance),
                                            (tail->normalize ? 1 : 0) | (tail->kept_reverse.defined() ? MTS_NORMALIZE_KEPT : 0), ptr(tail->dx_r), ptr(g.dx),
-                                           ptr_as<float>(tail->dw_r), ptr(ws), ws_bytes, ptr_as<int32_t>(schedule), main),
+                                           ptr_as<float>(tail->dw_r), ptr(tail_ws), tail_bytes, ptr_as<int32_t>(schedule), main),
                   "mts_moe_bwd_joint_router");
             if (!g.dx.defined()) combine_dx();
             return g;
@@ -534,7 +591,6 @@ ExpertGrads experts_backward(const Saved& s, Tensor dO, const Needs& need, const
     }
     if (need.x) {
         if (!layout) order_after(main, side0);   // W1's transposed copy
-        dx_expanded = at::empty({TK, H}, s.x.options());
         check(mts_moe_bwd_dx(ptr(d_pre_act), ptr(w1_bwd), layout, ptr_as<int32_t>(s.expert_start), TK, E, H, I, act, ptr(dx_expanded), main), "mts_moe_bwd_dx");
         combine_dx();
     }
@@ -572,76 +628,109 @@ struct FusedMoE : torch::autograd::Function<FusedMoE> {
 };
 
 // The whole MoE layer (router projection, post-process, routing metadata, experts, combine) as one node.
+struct LayerForward {
+    Tensor out, load_balance, z_loss, prob_mean, entropy, counts, load_stats, indices, weights;   // results
+    Tensor w_r, logits;
+    Saved s;
+};
+
+// capacity >= 0: an expert accepts at most that many routes; the others get no row
+LayerForward layer_forward(const Tensor& x_, const Tensor& w_r_, const Tensor& w1_, const Tensor& w2_, int64_t K, bool normalize, int64_t capacity,
+                           const Options& opt) {
+    LayerForward f;
+    const Tensor x = dense_router_operand(x_, w_r_.size(0)), w_r = dense_router_operand(w_r_, w_r_.size(0));
+    const Tensor w1 = w1_.contiguous(), w2 = w2_.contiguous();
+    const int64_t T = x.size(0), H = x.size(1), E = w_r.size(0), TK = T * K, I = w1.size(1) / 2;
+    const auto dtype = x.scalar_type();
+    const bool narrow = dtype != at::kFloat, limited = capacity >= 0, alone = opt.on(NO_BACKWARD), few = E <= kFewExperts;
+    const int64_t ws_bytes = few ? mts_moe_head_workspace_bytes(T, K, E) : mts_router_workspace_bytes(T, E);
+    f.w_r = w_r;
+    f.weights = f32({T, K}, x), f.indices = i32({T, K}, x);
+    Tensor weights_act, ws, post_act, y;
+    Routing r;
+    // what the backward pass keeps, and what this call alone needs
+    Together kept(x), scratch(x);
+    Together& own = alone ? scratch : kept;
+    own.add(f.logits, T, E, at::kFloat);
+    if (narrow || limited) own.add(weights_act, T, K, dtype);
+    else weights_act = f.weights;
+    auto add_rows = [&](Routing& to) {
+        own.add(to.expert_start, E + 1, at::kInt);
+        own.add(to.s_scatter, TK, at::kInt);
+        own.add(to.s_reverse, TK, at::kInt);
+        own.add(to.x_gather, TK, at::kInt);
+    };
+    if (few) add_rows(r);
+    scratch.add(ws, std::max<int64_t>(ws_bytes, 4), at::kByte);
+    scratch.add(y, TK, H, dtype);
+    if (alone) scratch.add(post_act, TK, I, dtype);
+    scratch.make();
+    if (!alone) kept.make();
+    // E mean probabilities, z, entropy, load-balancing term, E + 7 load statistics; the counts behind them
+    const int64_t floats = 2 * E + 10;
+    Tensor stats = f32({floats + E}, x);
+    if (alone) {   // nobody differentiates: parts instead of views
+        auto floats_at = [&](int64_t first, at::IntArrayRef size) { return part_of(stats, first * 4, size, at::kFloat); };
+        f.prob_mean = floats_at(0, {E}), f.z_loss = floats_at(E, {}), f.entropy = floats_at(E + 1, {}), f.load_balance = floats_at(E + 2, {});
+        f.load_stats = floats_at(E + 3, {E + 7});
+    } else {
+        f.prob_mean = stats.narrow(0, 0, E), f.z_loss = stats.select(0, E), f.entropy = stats.select(0, E + 1), f.load_balance = stats.select(0, E + 2);
+        f.load_stats = stats.narrow(0, E + 3, E + 7);
+    }
+    f.counts = part_of(stats, floats * 4, {E}, at::kInt);
+    void* load_stats = limited ? nullptr : ptr(f.load_stats);
+    void* cast_weights = narrow && !limited ? ptr(weights_act) : nullptr;
+    if (few) {
+        check(mts_moe_head_fwd(ptr(x), ptr_as<float>(w_r), T, H, E, K, normalize, dtype_code(x), ptr_as<float>(f.logits), ptr_as<float>(f.weights),
+                               ptr_as<int32_t>(f.indices), cast_weights, ptr_as<float>(f.prob_mean), ptr_as<float>(f.z_loss), ptr_as<float>(f.entropy),
+                               ptr_as<int32_t>(f.counts), ptr_as<float>(f.load_balance), static_cast<float*>(load_stats), ptr_as<int32_t>(r.expert_start),
+                               ptr_as<int32_t>(r.s_scatter), ptr_as<int32_t>(r.s_reverse), ptr_as<int32_t>(r.x_gather), ptr(ws), ws_bytes, stream_of(x)),
+              "mts_moe_head_fwd");
+    } else {   // the chained head is written for few experts
+        router_projection_forward(x, w_r, f.logits);
+        check(mts_router_fwd(ptr_as<float>(f.logits), T, E, K, normalize, ptr_as<float>(f.weights), ptr_as<int32_t>(f.indices), ptr_as<float>(f.prob_mean),
+                             ptr_as<float>(f.z_loss), ptr_as<float>(f.entropy), ptr_as<int32_t>(f.counts), ptr_as<float>(f.load_balance),
+                             static_cast<float*>(load_stats), cast_weights, narrow ? dtype_code(x) : 0, ptr(ws), ws_bytes, stream_of(x)),
+              "mts_router_fwd");
+        r = route(f.indices, E);
+    }
+    if (limited) {
+        const Routing every = r;
+        Tensor accepted, keys;
+        const int64_t keys_bytes = mts_moe_capacity_compact_workspace_bytes(T, K);
+        Together rows(x);
+        rows.add(r.expert_start, E + 1, at::kInt);
+        rows.add(r.s_scatter, TK, at::kInt);
+        rows.add(r.s_reverse, TK, at::kInt);
+        rows.add(r.x_gather, TK, at::kInt);
+        rows.add(accepted, E, at::kInt);
+        rows.add(keys, std::max<int64_t>(keys_bytes, 4), at::kByte);
+        rows.make();
+        check(mts_moe_capacity_compact(ptr_as<float>(f.weights), ptr_as<int32_t>(f.counts), ptr_as<int32_t>(every.expert_start),
+                                       ptr_as<int32_t>(every.s_scatter), T, K, E, capacity, ptr_as<int32_t>(accepted), ptr_as<int32_t>(r.expert_start),
+                                       ptr_as<int32_t>(r.s_scatter), ptr_as<int32_t>(r.s_reverse), ptr_as<int32_t>(r.x_gather), ptr(keys), keys_bytes,
+                                       stream_of(x)),
+              "mts_moe_capacity_compact");
+        check(mts_moe_capacity_weights_fwd(ptr_as<float>(f.weights), ptr_as<int32_t>(r.s_reverse), ptr_as<int32_t>(accepted), ptr_as<float>(f.entropy), T, K,
+                                           E, normalize, dtype_code(x), ptr(weights_act), ptr_as<float>(f.load_stats), stream_of(x)),
+              "mts_moe_capacity_weights_fwd");
+    }
+    f.out = experts_forward(x, w1, w2, weights_act, r, opt, f.s, post_act, y);
+    return f;
+}
+
 struct MoELayer : torch::autograd::Function<MoELayer> {
-    // capacity >= 0: an expert accepts at most that many routes; the others get no row
-    static variable_list forward(AutogradContext* ctx, const Tensor& x_, const Tensor& w_r_, const Tensor& w1_, const Tensor& w2_, int64_t K, bool normalize,
+    static variable_list forward(AutogradContext* ctx, const Tensor& x, const Tensor& w_r, const Tensor& w1, const Tensor& w2, int64_t K, bool normalize,
                                  int64_t capacity, int64_t switches, int64_t limit) {
-        const Options opt{switches, limit};
-        const Tensor x = dense_router_operand(x_, w_r_.size(0)), w_r = dense_router_operand(w_r_, w_r_.size(0));
-        const Tensor w1 = w1_.contiguous(), w2 = w2_.contiguous();
-        const int64_t T = x.size(0), H = x.size(1), E = w_r.size(0), TK = T * K;
-        const bool narrow = x.scalar_type() != at::kFloat, limited = capacity >= 0;
-        Tensor logits = f32({T, E}, x), weights = f32({T, K}, x), indices = i32({T, K}, x);
-        Tensor weights_act = narrow || limited ? at::empty({T, K}, x.options()) : weights;
-        Tensor stats = f32({2 * E + 10}, x);   // E mean probabilities, z, entropy, load-balancing term, E + 7 load statistics
-        Tensor prob_mean = stats.narrow(0, 0, E), z_loss = stats.select(0, E), entropy = stats.select(0, E + 1), load_balance = stats.select(0, E + 2),
-               load_stats = stats.narrow(0, E + 3, E + 7);
-        // counts, expert_start and the three permutation arrays in one allocation, each 16-byte aligned
-        const int64_t o1 = round4(E), o2 = o1 + round4(E + 1);
-        Tensor meta = i32({o2 + 3 * round4(TK)}, x);
-        Tensor counts = meta.narrow(0, 0, E);
-        Routing r;
-        r.expert_start = meta.narrow(0, o1, E + 1);
-        r.s_scatter = meta.narrow(0, o2, TK);
-        r.s_reverse = meta.narrow(0, o2 + round4(TK), TK);
-        r.x_gather = meta.narrow(0, o2 + 2 * round4(TK), TK);
-        if (E > kFewExperts) {   // the chained head is written for few experts
-            router_projection_forward(x, w_r, logits);
-            const int64_t ws_bytes = mts_router_workspace_bytes(T, E);
-            Tensor ws = bytes(ws_bytes, x);
-            check(mts_router_fwd(ptr_as<float>(logits), T, E, K, normalize, ptr_as<float>(weights), ptr_as<int32_t>(indices), ptr_as<float>(prob_mean),
-                                 ptr_as<float>(z_loss), ptr_as<float>(entropy), ptr_as<int32_t>(counts), ptr_as<float>(load_balance),
-                                 limited ? nullptr : ptr_as<float>(load_stats), narrow && !limited ? ptr(weights_act) : nullptr, narrow ? dtype_code(x) : 0,
-                                 ptr(ws), ws_bytes, stream_of(x)),
-                  "mts_router_fwd");
-            r = route(indices, E);
-        } else {
-            const int64_t ws_bytes = mts_moe_head_workspace_bytes(T, K, E);
-            Tensor ws = bytes(ws_bytes, x);
-            check(mts_moe_head_fwd(ptr(x), ptr_as<float>(w_r), T, H, E, K, normalize, dtype_code(x), ptr_as<float>(logits), ptr_as<float>(weights),
-                                   ptr_as<int32_t>(indices), narrow && !limited ? ptr(weights_act) : nullptr, ptr_as<float>(prob_mean), ptr_as<float>(z_loss),
-                                   ptr_as<float>(entropy), ptr_as<int32_t>(counts), ptr_as<float>(load_balance), limited ? nullptr : ptr_as<float>(load_stats),
-                                   ptr_as<int32_t>(r.expert_start), ptr_as<int32_t>(r.s_scatter), ptr_as<int32_t>(r.s_reverse), ptr_as<int32_t>(r.x_gather),
-                                   ptr(ws), ws_bytes, stream_of(x)),
-                  "mts_moe_head_fwd");
-        }
-        if (limited) {
-            const Routing every = r;
-            Tensor kept = i32({o2 + 3 * round4(TK)}, x), accepted = kept.narrow(0, 0, E);
-            r.expert_start = kept.narrow(0, o1, E + 1);
-            r.s_scatter = kept.narrow(0, o2, TK);
-            r.s_reverse = kept.narrow(0, o2 + round4(TK), TK);
-            r.x_gather = kept.narrow(0, o2 + 2 * round4(TK), TK);
-            const int64_t keys_bytes = mts_moe_capacity_compact_workspace_bytes(T, K);
-            Tensor keys = bytes(keys_bytes, x);
-            check(mts_moe_capacity_compact(ptr_as<float>(weights), ptr_as<int32_t>(counts), ptr_as<int32_t>(every.expert_start), ptr_as<int32_t>(every.s_scatter),
-                                           T, K, E, capacity, ptr_as<int32_t>(accepted), ptr_as<int32_t>(r.expert_start), ptr_as<int32_t>(r.s_scatter),
-                                           ptr_as<int32_t>(r.s_reverse), ptr_as<int32_t>(r.x_gather), ptr(keys), keys_bytes, stream_of(x)),
-                  "mts_moe_capacity_compact");
-            check(mts_moe_capacity_weights_fwd(ptr_as<float>(weights), ptr_as<int32_t>(r.s_reverse), ptr_as<int32_t>(accepted), ptr_as<float>(entropy), T, K, E,
-                                               normalize, dtype_code(x), ptr(weights_act), ptr_as<float>(load_stats), stream_of(x)),
-                  "mts_moe_capacity_weights_fwd");
-        }
-        Saved s;
-        Tensor out = experts_forward(x, w1, w2, weights_act.view(-1), r, opt, s);
+        const LayerForward f = layer_forward(x, w_r, w1, w2, K, normalize, capacity, {switches, limit});
         variable_list keep;
-        s.append_to(keep);
-        keep.insert(keep.end(), {w_r, logits, weights, indices, counts});
+        f.s.append_to(keep);
+        keep.insert(keep.end(), {f.w_r, f.logits, f.weights, f.indices, f.counts});
         ctx->save_for_backward(std::move(keep));
-        ctx->saved_data["options"] = std::vector<int64_t>{switches, limit, normalize, limited};
-        ctx->mark_non_differentiable({entropy, counts, load_stats, indices, weights});
+        ctx->saved_data["options"] = std::vector<int64_t>{switches, limit, normalize, capacity >= 0};
+        ctx->mark_non_differentiable({f.entropy, f.counts, f.load_stats, f.indices, f.weights});
         ctx->set_materialize_grads(false);
-        return {out, load_balance, z_loss, prob_mean, entropy, counts, load_stats, indices, weights};
+        return {f.out, f.load_balance, f.z_loss, f.prob_mean, f.entropy, f.counts, f.load_stats, f.indices, f.weights};
     }
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
         const auto o = ctx->saved_data["options"].toIntVector();
@@ -1114,7 +1203,12 @@ PYBIND11_MODULE(_host, m) {
     m.def("moe_layer", [](const Tensor& x, const Tensor& w_r, const Tensor& w1, const Tensor& w2, int64_t top_k, bool normalize, int64_t capacity, int64_t switches,
                           int64_t limit) {
         c10::OptionalDeviceGuard guard(x.device());
-        const variable_list v = MoELayer::apply(x, w_r, w1, w2, top_k, normalize, capacity, switches | no_backward(x, w_r, w1, w2), limit);
+        const int64_t without = no_backward(x, w_r, w1, w2);
+        if (without && all_plain(x, w_r, w1, w2)) {   // no node
+            const LayerForward f = layer_forward(x, w_r, w1, w2, top_k, normalize, capacity, {switches | without, limit});
+            return std::make_tuple(f.out, f.load_balance, f.z_loss, f.prob_mean, f.entropy, f.counts, f.load_stats, f.indices, f.weights);
+        }
+        const variable_list v = MoELayer::apply(x, w_r, w1, w2, top_k, normalize, capacity, switches | without, limit);
         return std::make_tuple(v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], v[8]);
     });
     m.def("router_postprocess", [](const Tensor& logits, int64_t top_k, bool normalize, int64_t act_dtype) {

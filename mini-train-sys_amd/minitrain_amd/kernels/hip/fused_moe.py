@@ -79,7 +79,7 @@ def compute_routing_metadata(topk_indices: torch.Tensor, E: int, block_m_token: 
 
 def routing_for_experts(topk_indices: torch.Tensor, E: int):
     """``(expert_start, x_gather, s_scatter, s_reverse)``: what the operator itself needs of the routing
-    metadata, in one int32 allocation (the tile list of the reference's kernels is not produced)."""
+    metadata (the tile list of the reference's kernels is not produced)."""
     return _lib.host().route(topk_indices, E)
 
 

@@ -359,3 +359,30 @@ def test_side_streams_are_joined_where_the_backward_pass_raises():
         out = ops.fused_moe(x, w1, w2, index, weights)
         with pytest.raises(RuntimeError, match="aligned"):
             torch.autograd.grad(out, (x, w1, w2), seed)
+
+
+@pytest.mark.parametrize("T,H,E,I,K,dtype,capacity", [
+    (1, 64, 4, 40, 1, torch.bfloat16, None), (16, 256, 8, 128, 2, torch.float16, None), (40, 64, 24, 64, 4, torch.bfloat16, None),
+    (33, 64, 8, 64, 2, torch.float32, 5), (300, 128, 8, 128, 2, torch.bfloat16, 60), (12000, 256, 8, 512, 2, torch.bfloat16, None)])
+def test_layer_without_gradients_equals_the_node(T, H, E, I, K, dtype, capacity):
+    """The same results without the node, whose buffers share an allocation where they are small together; results of one call stay as
+    they are through the next, and through changes of each other."""
+    print(f"layer without gradients T={T} H={H} E={E} I={I} K={K} {dtype} capacity={capacity}", flush=True)
+    ops = hip_backend()
+    x, w_r, w1, w2, _ = (t.cuda() for t in O.make_inputs(T + E, T, H, E, I))
+    x, w1, w2 = x.to(dtype), w1.to(dtype), w2.to(dtype)
+    leaves = [t.clone().requires_grad_(True) for t in (x, w_r, w1, w2)]
+    want = [t.detach().clone() for t in ops.moe_layer(*leaves, K, normalize=True, capacity=capacity)]
+    with torch.no_grad():
+        first = ops.moe_layer(x, w_r, w1, w2, K, normalize=True, capacity=capacity)
+        again = ops.moe_layer(x.flip(0).contiguous(), w_r, w1, w2, K, normalize=True, capacity=capacity)
+    outside = ops.moe_layer(x, w_r, w1, w2, K, normalize=True, capacity=capacity)   # nothing requires a gradient
+    with torch.inference_mode():
+        inference = ops.moe_layer(x, w_r, w1, w2, K, normalize=True, capacity=capacity)
+    for got in (first, outside, inference):
+        for a, b in zip(got, want):
+            assert a.dtype == b.dtype and a.shape == b.shape and not a.requires_grad and torch.equal(a, b)
+    for i, t in enumerate(first):
+        t.fill_(3)
+        assert all(torch.equal(a, b) for a, b in zip(first[i + 1:], want[i + 1:]))
+    assert again[0].shape == want[0].shape and torch.equal(outside[0], want[0])
