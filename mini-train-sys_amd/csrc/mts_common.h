@@ -167,6 +167,15 @@ void mts_router_bwd_shape(int64_t T, int H, int E, MtsRouterBwdShape* shape);
 int mts_launch_router_dw_reduce(const float* part, int row_blocks, int64_t EH, float* d_w_r, hipStream_t s);
 int mts_router_head_group(int H, int E, int act_dtype);   // rows a wave of the chained forward kernel finishes together
 void mts_router_head_geometry(int64_t T, int group, int* blocks, int* rows_per_wave);
+// What the launch behind the head writes from partial and cnt.  Where the head is one block (up to 64 tokens) the block writes it itself:
+// *finished is 1 then, and partial and cnt are left as they are.
+struct MtsHeadFinish {
+    float inv_t, inv_routes;
+    float *prob_mean, *z_loss, *entropy;
+    int32_t* counts;
+    float *load_balance, *load_stats;
+    int32_t *expert_start, *s_scatter, *s_reverse, *x_gather;
+};
 int mts_launch_router_head(const void* x, const float* w_r, int64_t T, int H, int E, int K, int normalize, int act_dtype,
                            float* logits, float* weights, int32_t* indices, void* weights_act, float* partial,
-                           int32_t* cnt, hipStream_t s);
+                           int32_t* cnt, MtsHeadFinish finish, int* finished, hipStream_t s);

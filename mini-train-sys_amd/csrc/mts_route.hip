@@ -14,22 +14,18 @@
 // counted, gets no row, and its s_reverse entry is -1.  expert_start[E] is the number
 // of routes that were kept.
 #include "mts_common.h"
+#include "mts_route_scatter.h"
 #include "mts_router_row.h"
 
 #include <mutex>
 
 namespace {
 
+using namespace mts_route;
+
 typedef __attribute__((ext_vector_type(4))) int32_t i32x4;
 constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / MTS_WAVE;
-constexpr int kChunk = 256;   // entries per wave
-constexpr int kSteps = kChunk / MTS_WAVE;
-constexpr int kFewExperts = 8;   // windows up to this many experts are ranked with one ballot per expert
-
-// Expert ids >= E are a caller error; they are clamped so that no address derived from
-// them can leave the output arrays.  Negative ids (dropped routes) stay negative.
-__device__ __forceinline__ int clamp_expert(int e, int E) { return e >= E ? E - 1 : e; }
 
 // Experts are handled in windows of at most MTS_MAX_EXPERTS ids, [e0, e0 + EW): one pass of the
 // three kernels per window, so that the per-wave counters fit LDS whatever E is.  A pass counts and
@@ -157,111 +153,6 @@ __global__ __launch_bounds__(1024) void route_scan_kernel(
     route_scan_block(cnt, n_chunks, E, block_m, counts, expert_start, tile_row_start, tile_expert, tile_count, e0);
 }
 
-// The stable scatter of one chunk (entries [cbeg, cend)) by one wave; next[e] is the next free row
-// of window expert e for this chunk (LDS, private to the wave).
-// E: all experts; [e0, e0 + EW): the window of this pass.
-// scatter_load fetches the window-relative expert ids of kSteps x 64 entries starting at `base`
-// (-1: dropped route, whose -1 goes to s_reverse in the first pass; -2: not this pass);
-// scatter_place ranks and writes them.
-__device__ __forceinline__ void scatter_load(int (&ev)[kSteps], const int32_t* __restrict__ idx, int E, int e0, int EW,
-                                             int64_t base, int64_t cend) {
-    const int lane = threadIdx.x % MTS_WAVE;
-#pragma unroll
-    for (int s = 0; s < kSteps; ++s) {  // these loads are in flight together
-        const int64_t n = base + s * MTS_WAVE + lane;
-        const int e = n < cend ? clamp_expert(idx[n], E) : -1;
-        ev[s] = e < 0 ? (e0 == 0 && n < cend ? -1 : -2) : (e >= e0 && e < e0 + EW ? e - e0 : -2);
-    }
-}
-
-// Division of an entry (below 2^31) by the routes per token: a multiplication and a correction for each, one division for all
-struct TokenOf {
-    uint32_t K, inverse;
-    __device__ __forceinline__ explicit TokenOf(int k) : K((uint32_t)k), inverse(0xffffffffu / (uint32_t)k) {}
-    __device__ __forceinline__ uint32_t operator()(uint32_t n) const {
-        const uint32_t q = __umulhi(n, inverse);   // the quotient or one less
-        return n - q * K >= K ? q + 1 : q;
-    }
-};
-
-// LDS the compiler knows as LDS: through a generic pointer every access would wait for the global ones in flight
-typedef volatile __attribute__((address_space(3))) int32_t* LdsRows;
-
-__device__ __forceinline__ void scatter_place(const int (&ev)[kSteps], int K, int EW, int64_t base, int64_t cend,
-                                              LdsRows next, int32_t* __restrict__ s_scatter,
-                                              int32_t* __restrict__ s_reverse, int32_t* __restrict__ x_gather) {
-    const int lane = threadIdx.x % MTS_WAVE;
-    const uint64_t lt = lanemask_lt();
-    const TokenOf by_K(K);
-    if (EW <= kFewExperts) {   // wave-uniform
-        // A window of few experts: one ballot per expert ranks the 64 entries of a step, and the next free rows
-        // stay in registers from step to step (the same positions as below: entries of one expert in lane order).
-        int32_t nx[kFewExperts];
-#pragma unroll
-        for (int x = 0; x < kFewExperts; ++x) nx[x] = x < EW ? next[x] : 0;
-#pragma unroll
-        for (int s = 0; s < kSteps; ++s) {
-            const int64_t n = base + s * MTS_WAVE + lane;
-            if (base + s * MTS_WAVE >= cend) break;   // wave-uniform
-            const int e = ev[s];
-            int pos = -1;
-#pragma unroll
-            for (int x = 0; x < kFewExperts; ++x) {
-                const uint64_t same = __ballot(e == x);
-                if (e == x) pos = nx[x] + __popcll(same & lt);
-                nx[x] += __popcll(same);
-            }
-            if (e >= -1 && n < cend) s_reverse[n] = pos;
-            if (e >= 0) {
-                s_scatter[pos] = (int32_t)n;
-                x_gather[pos] = (int32_t)by_K((uint32_t)n);
-            }
-        }
-#pragma unroll
-        for (int x = 0; x < kFewExperts; ++x)
-            if (lane == x && x < EW) next[x] = nx[x];
-        return;
-    }
-#pragma unroll
-    for (int s = 0; s < kSteps; ++s) {
-        const int64_t n = base + s * MTS_WAVE + lane;
-        if (base + s * MTS_WAVE >= cend) break;   // wave-uniform
-        const int e = ev[s];
-        const bool valid = e >= 0;
-        int pos = -1;
-        // the lanes with the same expert: one ballot per bit of the id
-        uint64_t same = __ballot(valid);
-#pragma unroll 1
-        for (int bit = 0; (1 << bit) < EW; ++bit) {
-            const uint64_t set = __ballot((e >> bit) & 1);
-            same &= ((e >> bit) & 1) ? set : ~set;
-        }
-        if (valid) {
-            const int first = next[e];   // every lane reads before the first of its group updates
-            pos = first + __popcll(same & lt);
-            if ((same & lt) == 0) next[e] = first + __popcll(same);
-        }
-        if (e >= -1 && n < cend) s_reverse[n] = pos;
-        if (valid) {
-            s_scatter[pos] = (int32_t)n;
-            x_gather[pos] = (int32_t)by_K((uint32_t)n);
-        }
-    }
-}
-
-// `first` holds the ids of the chunk's first kSteps x 64 entries already (scatter_load at cbeg)
-__device__ __forceinline__ void scatter_chunk(int (&first)[kSteps], const int32_t* __restrict__ idx, int K, int E, int e0,
-                                              int EW, int64_t cbeg, int64_t cend, LdsRows next,
-                                              int32_t* __restrict__ s_scatter, int32_t* __restrict__ s_reverse,
-                                              int32_t* __restrict__ x_gather) {
-    scatter_place(first, K, EW, cbeg, cend, next, s_scatter, s_reverse, x_gather);
-    for (int64_t base = cbeg + kChunk; base < cend; base += kChunk) {
-        int ev[kSteps];
-        scatter_load(ev, idx, E, e0, EW, base, cend);
-        scatter_place(ev, K, EW, base, cend, next, s_scatter, s_reverse, x_gather);
-    }
-}
-
 // chunk_len entries per wave (a multiple of 64 is not required); the chunks are the ones the
 // counters in cnt were taken over
 // E: all experts; [e0, e0 + EW): the window of this pass (cnt is [chunk][EW], expert_start points at expert e0)
@@ -290,6 +181,7 @@ __global__ __launch_bounds__(kThreads) void route_scatter_kernel(
 // chunks before its own take.  One launch and one dependent round trip less than scan-then-scatter.
 constexpr int kFinishChunks = MTS_HEAD_MAX_CHUNKS;
 constexpr int kFinishMaxE = 16;
+static_assert(kFinishMaxE == mts_route::kHeadExperts, "as the head kernel has it");
 __global__ __launch_bounds__(kThreads) void head_scatter_kernel(
     const float* __restrict__ partial, const int32_t* __restrict__ cnt, int n_chunks, int E, float inv_t,
     float inv_routes, float* __restrict__ prob_mean, float* __restrict__ z_loss, float* __restrict__ entropy,
@@ -539,9 +431,13 @@ extern "C" int mts_moe_head_fwd(const void* x, const float* w_r, int64_t T, int 
     hipStream_t s = (hipStream_t)stream;
     float* partial = (float*)workspace;
     int32_t* cnt = (int32_t*)(partial + (int64_t)MTS_HEAD_MAX_CHUNKS * (E + 2));
+    // the rows of one block are scattered, and its statistics completed, by the block itself
+    const MtsHeadFinish finish = {1.0f / (float)T, 1.0f / ((float)T * (float)K), prob_mean, z_loss, entropy, counts, load_balance, load_stats,
+                                  expert_start, s_scatter, s_reverse, x_gather};
+    int finished = 0;
     const int rc = mts_launch_router_head(x, w_r, T, H, E, K, normalize, act_dtype, logits, weights, indices, weights_act,
-                                          partial, cnt, s);
-    if (rc) return rc;
+                                          partial, cnt, finish, &finished, s);
+    if (rc || finished) return rc;
     int blocks, rows_per_wave;
     mts_router_head_geometry(T, mts_router_head_group(H, E, act_dtype), &blocks, &rows_per_wave);
     const int64_t rows_per_chunk = (int64_t)rows_per_wave * 4;

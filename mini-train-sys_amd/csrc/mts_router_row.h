@@ -177,15 +177,18 @@ __device__ __forceinline__ void row_logit_gradient(const RowState<EP, G>& r, con
 // ---- reduction of the routing statistics (one block) ----------------------------------------
 // Column i < E of the per-block partials is the probability mass of expert i, column E the sum
 // of squared log-partitions, column E+1 the entropy sum.  Sums run in a fixed order (bit-stable).
-struct StatsShared {
-    float prod[MTS_MAX_EXPERTS];    // fraction of routes x mean probability, per expert
-    float share[MTS_MAX_EXPERTS];   // fraction of routes, per expert
-    int routes_of[MTS_MAX_EXPERTS];
+template <int EXPERTS>
+struct StatsOf {
+    float prod[EXPERTS];    // fraction of routes x mean probability, per expert
+    float share[EXPERTS];   // fraction of routes, per expert
+    int routes_of[EXPERTS];
     float entropy_s;
 };
+typedef StatsOf<MTS_MAX_EXPERTS> StatsShared;
 
 // what one thread does with the mean `v` of column i and, for i < E, the routes `c` of expert i
-__device__ __forceinline__ void stats_column(StatsShared& sh, int i, float v, int c, int E, float inv_routes,
+template <class Stats>
+__device__ __forceinline__ void stats_column(Stats& sh, int i, float v, int c, int E, float inv_routes,
                                              float* __restrict__ prob_mean, float* __restrict__ z_loss,
                                              float* __restrict__ entropy, int32_t* __restrict__ counts) {
     if (i < E) {
@@ -208,7 +211,8 @@ __device__ __forceinline__ void stats_column(StatsShared& sh, int i, float v, in
 // largest and smallest route count, the coefficient of variation (population standard deviation x E),
 // largest fraction x E, the number of experts without a route, a zero (the dropped-route fraction of
 // dropless routing) and the entropy over log E.  Either output may be NULL.
-__device__ __forceinline__ void stats_finalize(const StatsShared& sh, int wave, int lb_wave, int ls_wave, int E,
+template <class Stats>
+__device__ __forceinline__ void stats_finalize(const Stats& sh, int wave, int lb_wave, int ls_wave, int E,
                                                float* __restrict__ load_balance, float* __restrict__ load_stats) {
     const int lane = threadIdx.x % MTS_WAVE;
     if (wave == lb_wave && load_balance) {

@@ -80,6 +80,15 @@ def test_chained_head_equals_the_three_operators(T, H, E, K, dtype, normalize):
 
 
 @pytest.mark.parametrize("T,H,E,K,dtype", [
+    (16, 768, 8, 2, torch.bfloat16), (63, 768, 8, 1, torch.bfloat16), (64, 256, 8, 8, torch.bfloat16), (65, 256, 8, 8, torch.bfloat16),
+    (64, 72, 3, 3, torch.bfloat16), (16, 100, 16, 8, torch.float32), (32, 64, 12, 5, torch.float16), (33, 64, 12, 5, torch.float16)])
+def test_head_of_one_block_finishes_the_routing_itself(T, H, E, K, dtype):
+    """The last counts of tokens that one block takes and the first that it does not, more routes than one round of the scatter, few and
+    many experts."""
+    test_chained_head_equals_the_three_operators(T, H, E, K, dtype, True)
+
+
+@pytest.mark.parametrize("T,H,E,K,dtype", [
     (1500, 768, 8, 2, torch.bfloat16),    # projection on the matrix pipe
     (1500, 256, 8, 3, torch.float16),     # 16-bit rows the matrix-pipe projection does not take: vector pipe
     (700, 192, 12, 4, torch.float32),     # more than 8 experts: several lanes per row in the post-process
