@@ -585,3 +585,20 @@ def test_moe_block_end_to_end():
     assert_close_scaled(block.down_proj.grad, leaves[3].grad, BF16_TOL, "dW2")
     for key in ("moe/router_entropy", "moe/dropped_route_fraction", "moe/max_expert_load", "moe/min_expert_load"):
         assert key in out.router_metrics
+
+
+@pytest.mark.parametrize("counts", [(1153, 1152, 1281, 1280, 1409, 1, 128, 129), (3072, 3200, 3201, 3199, 2945, 127, 0, 2944)])
+@pytest.mark.parametrize("H,I", [(512, 512), (768, 1024)])
+def test_last_tiles_of_few_rows(counts, H, I):
+    """The last tile of an expert takes half the height up to 128 rows: one row less and one more, an expert of only such a tile, and none."""
+    print(f"last tiles {counts} {H}/{I}", flush=True)
+    T = sum(counts)
+    idx = torch.repeat_interleave(torch.arange(len(counts)), torch.tensor(counts))[torch.randperm(T, generator=torch.Generator().manual_seed(T))]
+    x, _, w1, w2, g = O.make_inputs(T, T, H, len(counts), I)
+    x, w1, w2, g = (t.bfloat16() for t in (x, w1, w2, g))
+    w = torch.rand(T, 1, generator=torch.Generator().manual_seed(1)).bfloat16()
+    case = (x, w1, w2, idx.int().unsqueeze(1), w, g)
+    out, grads = hip_moe_grads(*case)
+    want, want_grads = oracle_moe_grads(*case, device="cuda")
+    for got, ref, what in zip((out, *grads), (want, *want_grads), ("out", "dx", "dw1", "dw2", "dweights")):
+        assert_close_scaled(got, ref, BF16_TOL, what)
