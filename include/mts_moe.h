@@ -177,6 +177,15 @@ int mts_moe_route(const int32_t* top_k_index, int64_t T, int K, int E, int block
                   int32_t* tile_expert, int32_t* tile_count, void* workspace,
                   int64_t workspace_bytes, void* stream);
 
+/* mts_router_fwd and mts_moe_route (E up to MTS_MAX_EXPERTS) as one chain, with the results of both; the
+ * statistics are reduced beside the routing metadata instead of in front of it.             */
+int64_t mts_moe_router_route_workspace_bytes(int64_t T, int K, int E);
+int mts_moe_router_route(const float* logits, int64_t T, int E, int K, int normalize, float* weights,
+                         int32_t* indices, float* prob_mean, float* z_loss, float* entropy,
+                         int32_t* counts, float* load_balance, float* load_stats, void* weights_act,
+                         int act_dtype, int32_t* expert_start, int32_t* s_scatter, int32_t* s_reverse,
+                         int32_t* x_gather, void* workspace, int64_t workspace_bytes, void* stream);
+
 /* mts_moe_route without a workspace argument, for callers that cannot allocate device memory
  * (code under HIP graph capture, serving loops and harnesses that forbid hipMalloc).  It has no
  * counterpart in the reference.  The chunk counters live in an array inside the library's device

@@ -643,7 +643,7 @@ LayerForward layer_forward(const Tensor& x_, const Tensor& w_r_, const Tensor& w
     const int64_t T = x.size(0), H = x.size(1), E = w_r.size(0), TK = T * K, I = w1.size(1) / 2;
     const auto dtype = x.scalar_type();
     const bool narrow = dtype != at::kFloat, limited = capacity >= 0, alone = opt.on(NO_BACKWARD), few = E <= kFewExperts;
-    const int64_t ws_bytes = few ? mts_moe_head_workspace_bytes(T, K, E) : mts_router_workspace_bytes(T, E);
+    const int64_t ws_bytes = few ? mts_moe_head_workspace_bytes(T, K, E) : mts_moe_router_route_workspace_bytes(T, K, E);
     f.w_r = w_r;
     f.weights = f32({T, K}, x), f.indices = i32({T, K}, x);
     Tensor weights_act, ws, post_act, y;
@@ -660,7 +660,7 @@ LayerForward layer_forward(const Tensor& x_, const Tensor& w_r_, const Tensor& w
         own.add(to.s_reverse, TK, at::kInt);
         own.add(to.x_gather, TK, at::kInt);
     };
-    if (few) add_rows(r);
+    add_rows(r);
     scratch.add(ws, std::max<int64_t>(ws_bytes, 4), at::kByte);
     scratch.add(y, TK, H, dtype);
     if (alone) scratch.add(post_act, TK, I, dtype);
@@ -688,11 +688,11 @@ LayerForward layer_forward(const Tensor& x_, const Tensor& w_r_, const Tensor& w
               "mts_moe_head_fwd");
     } else {   // the chained head is written for few experts
         router_projection_forward(x, w_r, f.logits);
-        check(mts_router_fwd(ptr_as<float>(f.logits), T, E, K, normalize, ptr_as<float>(f.weights), ptr_as<int32_t>(f.indices), ptr_as<float>(f.prob_mean),
-                             ptr_as<float>(f.z_loss), ptr_as<float>(f.entropy), ptr_as<int32_t>(f.counts), ptr_as<float>(f.load_balance),
-                             static_cast<float*>(load_stats), cast_weights, narrow ? dtype_code(x) : 0, ptr(ws), ws_bytes, stream_of(x)),
-              "mts_router_fwd");
-        r = route(f.indices, E);
+        check(mts_moe_router_route(ptr_as<float>(f.logits), T, E, K, normalize, ptr_as<float>(f.weights), ptr_as<int32_t>(f.indices), ptr_as<float>(f.prob_mean),
+                                   ptr_as<float>(f.z_loss), ptr_as<float>(f.entropy), ptr_as<int32_t>(f.counts), ptr_as<float>(f.load_balance),
+                                   static_cast<float*>(load_stats), cast_weights, narrow ? dtype_code(x) : 0, ptr_as<int32_t>(r.expert_start),
+                                   ptr_as<int32_t>(r.s_scatter), ptr_as<int32_t>(r.s_reverse), ptr_as<int32_t>(r.x_gather), ptr(ws), ws_bytes, stream_of(x)),
+              "mts_moe_router_route");
     }
     if (limited) {
         const Routing every = r;

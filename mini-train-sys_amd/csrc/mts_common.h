@@ -167,6 +167,20 @@ void mts_router_bwd_shape(int64_t T, int H, int E, MtsRouterBwdShape* shape);
 int mts_launch_router_dw_reduce(const float* part, int row_blocks, int64_t EH, float* d_w_r, hipStream_t s);
 int mts_router_head_group(int H, int E, int act_dtype);   // rows a wave of the chained forward kernel finishes together
 void mts_router_head_geometry(int64_t T, int group, int* blocks, int* rows_per_wave);
+// Routing statistics that are still to be reduced from the partial sums of a router launch's blocks: arguments of mts_router::stats_block
+struct MtsRouterStats {
+    const float* partial;
+    const int32_t* partial_counts;
+    int blocks, E;
+    float inv_t, inv_routes;
+    float *prob_mean, *z_loss, *entropy;
+    int32_t* counts;
+    float *load_balance, *load_stats;
+};
+// mts_router_fwd without that reduction
+int mts_launch_router_fwd(const float* logits, int64_t T, int E, int K, int normalize, float* weights, int32_t* indices, float* prob_mean, float* z_loss,
+                          float* entropy, int32_t* counts, float* load_balance, float* load_stats, void* weights_act, int act_dtype, void* workspace,
+                          int64_t workspace_bytes, MtsRouterStats* stats, hipStream_t s);
 // What the launch behind the head writes from partial and cnt.  Where the head is one block (up to 64 tokens) the block writes it itself:
 // *finished is 1 then, and partial and cnt are left as they are.
 struct MtsHeadFinish {

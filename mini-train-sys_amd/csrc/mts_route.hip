@@ -144,12 +144,18 @@ __device__ __forceinline__ void route_scan_block(
     }
 }
 
-__global__ __launch_bounds__(1024) void route_scan_kernel(
-    int32_t* __restrict__ cnt, int64_t n_chunks, int E, int64_t TK, int block_m,
+// The second block, where there is one, reduces the router's statistics meanwhile, which nothing in the chain waits for.
+constexpr int kScanThreads = 1024;
+__global__ __launch_bounds__(kScanThreads) void route_scan_kernel(
+    int32_t* __restrict__ cnt, int64_t n_chunks, int E, int block_m,
     int32_t* __restrict__ counts, int32_t* __restrict__ expert_start,
     int32_t* __restrict__ tile_row_start, int32_t* __restrict__ tile_expert,
-    int32_t* __restrict__ tile_count, int e0) {
-    (void)TK;
+    int32_t* __restrict__ tile_count, int e0, MtsRouterStats stats) {
+    if (blockIdx.x == 1) {
+        mts_router::stats_block<kScanThreads>(stats.partial, stats.partial_counts, stats.blocks, stats.E, stats.inv_t, stats.inv_routes, stats.prob_mean,
+                                              stats.z_loss, stats.entropy, stats.counts, stats.load_balance, stats.load_stats, threadIdx.x / MTS_WAVE);
+        return;
+    }
     route_scan_block(cnt, n_chunks, E, block_m, counts, expert_start, tile_row_start, tile_expert, tile_count, e0);
 }
 
@@ -321,7 +327,7 @@ namespace {
 int route_launch(const int32_t* top_k_index, int64_t T, int K, int E, int block_m, int32_t* counts,
                  int32_t* expert_start, int32_t* s_scatter, int32_t* s_reverse, int32_t* x_gather,
                  int32_t* tile_row_start, int32_t* tile_expert, int32_t* tile_count, int32_t* cnt,
-                 hipStream_t s) {
+                 hipStream_t s, const MtsRouterStats* stats = nullptr) {
     const bool permute = s_scatter != nullptr;
     const int64_t TK = T * K;
     const int64_t n_chunks = (TK + kChunk - 1) / kChunk;
@@ -331,8 +337,9 @@ int route_launch(const int32_t* top_k_index, int64_t T, int K, int E, int block_
         const size_t lds = (size_t)kWaves * EW * sizeof(int32_t);
         route_hist_kernel<<<grid, kThreads, lds, s>>>(top_k_index, TK, E, e0, EW, cnt);
         MTS_CHECK_LAUNCH();
-        route_scan_kernel<<<1, 1024, 0, s>>>(cnt, n_chunks, EW, TK, block_m, counts + e0, expert_start + e0,
-                                             tile_row_start, tile_expert, tile_count, e0);
+        route_scan_kernel<<<stats ? 2 : 1, kScanThreads, 0, s>>>(cnt, n_chunks, EW, block_m, counts + e0, expert_start + e0, tile_row_start, tile_expert,
+                                                                 tile_count, e0, stats ? *stats : MtsRouterStats{});
+        stats = nullptr;
         MTS_CHECK_LAUNCH();
         if (!permute) continue;
         route_scatter_kernel<<<grid, kThreads, lds, s>>>(top_k_index, TK, K, E, e0, EW, kChunk, cnt, expert_start + e0,
@@ -409,6 +416,28 @@ extern "C" int mts_moe_route_static(const int32_t* top_k_index, int64_t T, int K
     if (err) return err;
     return route_launch(top_k_index, T, K, E, block_m, counts, expert_start, s_scatter, s_reverse, x_gather,
                         tile_row_start, tile_expert, tile_count, cnt, (hipStream_t)stream);
+}
+
+extern "C" int64_t mts_moe_router_route_workspace_bytes(int64_t T, int K, int E) {
+    const int64_t router = (mts_router_workspace_bytes(T, E) + 15) / 16 * 16;
+    return router + (int64_t)(E + 3) / 4 * 16 + mts_moe_route_workspace_bytes(T, K, E);   // the scan's own counts
+}
+
+extern "C" int mts_moe_router_route(const float* logits, int64_t T, int E, int K, int normalize, float* weights, int32_t* indices, float* prob_mean, float* z_loss,
+                                    float* entropy, int32_t* counts, float* load_balance, float* load_stats, void* weights_act, int act_dtype,
+                                    int32_t* expert_start, int32_t* s_scatter, int32_t* s_reverse, int32_t* x_gather, void* workspace,
+                                    int64_t workspace_bytes, void* stream) {
+    if (!workspace || !expert_start || !s_scatter || !s_reverse || !x_gather) return MTS_ERR_NULL;
+    if (T <= 0 || K < 1 || E < 1 || E > MTS_MAX_EXPERTS || T * (int64_t)K > 0x7fffffffLL) return MTS_ERR_SHAPE;
+    if (workspace_bytes < mts_moe_router_route_workspace_bytes(T, K, E)) return MTS_ERR_WORKSPACE;
+    const int64_t router = (mts_router_workspace_bytes(T, E) + 15) / 16 * 16;
+    int32_t* scan_counts = (int32_t*)((char*)workspace + router);
+    int32_t* cnt = scan_counts + (E + 3) / 4 * 4;
+    MtsRouterStats stats;
+    const int rc = mts_launch_router_fwd(logits, T, E, K, normalize, weights, indices, prob_mean, z_loss, entropy, counts, load_balance, load_stats, weights_act,
+                                         act_dtype, workspace, router, &stats, (hipStream_t)stream);
+    if (rc) return rc;
+    return route_launch(indices, T, K, E, 64, scan_counts, expert_start, s_scatter, s_reverse, x_gather, nullptr, nullptr, nullptr, cnt, (hipStream_t)stream, &stats);
 }
 
 extern "C" int64_t mts_moe_head_workspace_bytes(int64_t T, int K, int E) {

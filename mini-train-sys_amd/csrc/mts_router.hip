@@ -116,13 +116,9 @@ __global__ __launch_bounds__(kThreads) void router_fwd_kernel(
 }
 
 constexpr int kStatsThreads = 1024;
-__global__ __launch_bounds__(kStatsThreads) void router_stats_kernel(
-    const float* __restrict__ partial, const int32_t* __restrict__ partial_counts, int nblocks, int E,
-    float inv_t, float inv_routes, float* __restrict__ prob_mean, float* __restrict__ z_loss,
-    float* __restrict__ entropy, int32_t* __restrict__ counts, float* __restrict__ load_balance,
-    float* __restrict__ load_stats) {
-    stats_block<kStatsThreads>(partial, partial_counts, nblocks, E, inv_t, inv_routes, prob_mean, z_loss, entropy,
-                                     counts, load_balance, load_stats, threadIdx.x / MTS_WAVE);
+__global__ __launch_bounds__(kStatsThreads) void router_stats_kernel(MtsRouterStats s) {
+    stats_block<kStatsThreads>(s.partial, s.partial_counts, s.blocks, s.E, s.inv_t, s.inv_routes, s.prob_mean, s.z_loss, s.entropy, s.counts,
+                               s.load_balance, s.load_stats, threadIdx.x / MTS_WAVE);
 }
 
 template <int EP, int G>
@@ -222,18 +218,15 @@ extern "C" int64_t mts_router_workspace_bytes(int64_t T, int E) {
     return (int64_t)kMaxBlocks * (2 * E + 2) * (int64_t)sizeof(float);   // float partials, then int32 route counts
 }
 
-extern "C" int mts_router_fwd(const float* logits, int64_t T, int E, int K, int normalize,
-                              float* weights, int32_t* indices, float* prob_mean, float* z_loss,
-                              float* entropy, int32_t* counts, float* load_balance, float* load_stats,
-                              void* weights_act, int act_dtype, void* workspace, int64_t workspace_bytes,
-                              void* stream) {
+int mts_launch_router_fwd(const float* logits, int64_t T, int E, int K, int normalize, float* weights, int32_t* indices, float* prob_mean, float* z_loss,
+                          float* entropy, int32_t* counts, float* load_balance, float* load_stats, void* weights_act, int act_dtype, void* workspace,
+                          int64_t workspace_bytes, MtsRouterStats* stats, hipStream_t s) {
     int rc = check_router(logits, T, E, K);
     if (rc) return rc;
     if (weights_act && act_dtype != MTS_BF16 && act_dtype != MTS_F16) return MTS_ERR_DTYPE;
     if (!weights || !indices || !prob_mean || !z_loss || !entropy || !workspace) return MTS_ERR_NULL;
     if ((counts || load_balance || load_stats) && T * (int64_t)K > 0x7fffffffLL) return MTS_ERR_SHAPE;   // int32 route counts
     if (workspace_bytes < mts_router_workspace_bytes(T, E)) return MTS_ERR_WORKSPACE;
-    hipStream_t s = (hipStream_t)stream;
     float* partial = (float*)workspace;
     int32_t* partial_counts = (int32_t*)(partial + (int64_t)kMaxBlocks * (E + 2));
     int G = E > 512 ? 64 : lanes_for(E);
@@ -241,9 +234,20 @@ extern "C" int mts_router_fwd(const float* logits, int64_t T, int E, int K, int 
     MTS_ROUTER_DISPATCH(router_fwd_kernel, <<<grid, kThreads, 0, s>>>(logits, T, E, K, normalize, weights, indices,
                                                                       partial, partial_counts, weights_act, act_dtype));
     MTS_CHECK_LAUNCH();
-    router_stats_kernel<<<1, kStatsThreads, 0, s>>>(partial, partial_counts, grid, E, 1.0f / (float)T,
-                                               1.0f / ((float)T * (float)K), prob_mean, z_loss, entropy, counts,
-                                               load_balance, load_stats);
+    *stats = {partial, partial_counts, grid, E, 1.0f / (float)T, 1.0f / ((float)T * (float)K), prob_mean, z_loss, entropy, counts, load_balance, load_stats};
+    return MTS_OK;
+}
+
+extern "C" int mts_router_fwd(const float* logits, int64_t T, int E, int K, int normalize,
+                              float* weights, int32_t* indices, float* prob_mean, float* z_loss,
+                              float* entropy, int32_t* counts, float* load_balance, float* load_stats,
+                              void* weights_act, int act_dtype, void* workspace, int64_t workspace_bytes,
+                              void* stream) {
+    MtsRouterStats stats;
+    const int rc = mts_launch_router_fwd(logits, T, E, K, normalize, weights, indices, prob_mean, z_loss, entropy, counts, load_balance, load_stats, weights_act,
+                                         act_dtype, workspace, workspace_bytes, &stats, (hipStream_t)stream);
+    if (rc) return rc;
+    router_stats_kernel<<<1, kStatsThreads, 0, (hipStream_t)stream>>>(stats);
     MTS_CHECK_LAUNCH();
     return MTS_OK;
 }

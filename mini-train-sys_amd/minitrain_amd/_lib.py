@@ -40,6 +40,8 @@ SIGNATURES = {
     "mts_router_wide_bwd_workspace_bytes": (_l, [_l, _i, _i]),
     "mts_router_wide_bwd": (_i, [_p, _p, _p, _l, _i, _i, _i, _p, _p, _p, _l, _p]),
     "mts_moe_route_workspace_bytes": (_l, [_l, _i, _i]),
+    "mts_moe_router_route_workspace_bytes": (_l, [_l, _i, _i]),
+    "mts_moe_router_route": (_i, [_p, _l, _i, _i, _i, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i, _p, _p, _p, _p, _p, _l, _p]),
     "mts_moe_route": (_i, [_p, _l, _i, _i, _i, _p, _p, _p, _p, _p, _p, _p, _p, _p, _l, _p]),
     "mts_moe_route_static": (_i, [_p, _l, _i, _i, _i, _p, _p, _p, _p, _p, _p, _p, _p, _p]),
     "mts_moe_capacity_workspace_bytes": (_l, [_l, _i, _i]),

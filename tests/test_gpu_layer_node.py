@@ -395,3 +395,32 @@ def test_layer_without_gradients_equals_the_node(T, H, E, I, K, dtype, capacity)
         t.fill_(3)
         assert all(torch.equal(a, b) for a, b in zip(first[i + 1:], want[i + 1:]))
     assert again[0].shape == want[0].shape and torch.equal(outside[0], want[0])
+
+
+@pytest.mark.parametrize("T,E,K", [(1, 17, 1), (40, 24, 4), (3000, 64, 8), (700, 1000, 2)])
+def test_router_and_routing_of_many_experts_as_one_chain(T, E, K):
+    """Statistics that a second block reduces beside the scan, and the permutation: those of the two calls, bit for bit."""
+    print(f"router and routing T={T} E={E} K={K}", flush=True)
+    from minitrain_amd import _lib
+    from minitrain_amd.kernels.hip.fused_moe import compute_routing_metadata
+    from minitrain_amd.kernels.hip.router import router_postprocess
+
+    lib = _lib.load()
+    logits = torch.randn(T, E, generator=torch.Generator().manual_seed(T)).cuda()
+    f32, i32 = dict(dtype=torch.float32, device="cuda"), dict(dtype=torch.int32, device="cuda")
+    o = dict(weights=torch.empty(T, K, **f32), indices=torch.empty(T, K, **i32), prob_mean=torch.empty(E, **f32), z_loss=torch.empty(1, **f32),
+             entropy=torch.empty(1, **f32), counts=torch.empty(E, **i32), load_balance=torch.empty(1, **f32), load_stats=torch.empty(E + 7, **f32))
+    rows = [torch.full((n,), -9, **i32) for n in (E + 1, T * K, T * K, T * K)]
+    ws_bytes = lib.mts_moe_router_route_workspace_bytes(T, K, E)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device="cuda")
+    args = (logits.data_ptr(), T, E, K, 1, *[t.data_ptr() for t in o.values()], None, 0, *[t.data_ptr() for t in rows], ws.data_ptr())
+    assert lib.mts_moe_router_route(*args, ws_bytes - 1, _lib.stream_of(logits)) != 0
+    _lib.check(lib.mts_moe_router_route(*args, ws_bytes, _lib.stream_of(logits)), "mts_moe_router_route")
+    torch.cuda.synchronize()
+    route = router_postprocess(logits, K, normalize=True, weights_dtype=None)
+    for name, want in (("weights", route.expert_weights), ("indices", route.expert_indices), ("prob_mean", route.probability_per_expert), ("z_loss", route.z_loss),
+                       ("entropy", route.entropy), ("counts", route.expert_counts), ("load_balance", route.load_balance_loss), ("load_stats", route.load_stats)):
+        assert torch.equal(o[name].flatten(), want.flatten()), name
+    _, start, gather, scatter, reverse, *_ = compute_routing_metadata(o["indices"], E)
+    for got, want in zip(rows, (start, scatter, reverse, gather)):
+        assert torch.equal(got, want)
