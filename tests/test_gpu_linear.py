@@ -75,6 +75,46 @@ def test_gradients_in_other_layouts_in_rounds(layout, N):
         assert float((got.double() - want).abs().max()) <= ULP[torch.bfloat16] * float(want.abs().max())
 
 
+@pytest.mark.parametrize("layout", ["sequence first", "part of a wider row", "misaligned", "weight by columns"])
+def test_operands_in_other_layouts_in_rounds(layout):
+    """Inputs that are not dense or not aligned and a weight that is not: the same gradients."""
+    print(f"linear in rounds, {layout}", flush=True)
+    g = torch.Generator().manual_seed(7)
+    r = lambda *shape: torch.randn(*shape, generator=g).bfloat16().cuda()
+    x = {"sequence first": lambda: r(100, 2, 16).transpose(0, 1), "part of a wider row": lambda: r(2, 100, 48)[..., 16:32], "misaligned": lambda: r(2, 100, 17)[..., 1:],
+         "weight by columns": lambda: r(2, 100, 16)}[layout]().detach().requires_grad_(True)
+    w = torch.randn(16, 136, generator=g).cuda().t() if layout == "weight by columns" else torch.randn(136, 16, generator=g).cuda()
+    w = w.detach().requires_grad_(True)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        y = hip_backend().linear(x, w)
+    grad = r(2, 100, 136)
+    y.backward(grad)
+    wide, rows = w.detach().bfloat16().double(), grad.double().reshape(-1, 136)
+    for got, want, tol in ((y.detach(), x.detach().double() @ wide.T, ULP[torch.bfloat16]), (x.grad, grad.double() @ wide, ULP[torch.bfloat16]),
+                           (w.grad, rows.T @ x.detach().double().reshape(-1, 16), 1e-5)):
+        assert got.shape == want.shape and float((got.double() - want).abs().max()) <= tol * float(want.abs().max())
+
+
+@pytest.mark.parametrize("create_graph", [False, True])
+def test_vocabulary_weight_changed_before_the_backward_pass(create_graph):
+    """The gradients are those of the weight of the forward pass, and can be differentiated again."""
+    print(f"linear in rounds, weight changed in place, create_graph={create_graph}", flush=True)
+    g = torch.Generator().manual_seed(8)
+    x, w = torch.randn(2, 100, 16, generator=g).bfloat16().cuda().requires_grad_(True), torch.randn(136, 16, generator=g).cuda().requires_grad_(True)
+    grad = torch.randn(2, 100, 136, generator=g).bfloat16().cuda()
+    got = []
+    for f in (lambda: hip_backend().linear(x, w), lambda: torch.nn.functional.linear(x, w)):
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            y = f()
+        with torch.no_grad():
+            w.mul_(2)
+        got.append(torch.autograd.grad(y, (x, w), grad, create_graph=create_graph))
+        with torch.no_grad():
+            w.div_(2)
+    for a, b in zip(*got):
+        assert a.dtype == b.dtype and a.requires_grad == create_graph and float((a.detach().float() - b.detach().float()).abs().max()) <= ULP[torch.bfloat16] * float(b.detach().abs().max())
+
+
 @pytest.mark.parametrize("rows,V", [(130, 64), (200, 1003), (129, 50257)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_loss_on_a_projection(rows, V, dtype):
