@@ -1475,6 +1475,130 @@ __device__ __forceinline__ void rows_gemm_ws_tile(const RowsParams& p, bf16_t* s
     rows_epilogue<T, EPI>(p, acc, smem, row0, rend, n0, wm, wn, srow);
 }
 
+// ---------------------------------------------------------------------------
+// Gate/up over `span` column tiles of one m-tile, one after the other in the same block: the loads run on across the border of two tiles, so that
+// the first k-tile of the next lands while the epilogue of the last is on its way, and rows, offsets and routing weights are found once.
+// The k loop's buffers stay its own; the epilogue stages 32 x 64 results of a wave at a time in 4 KiB behind them (160 KiB in all).
+// Whole k-tiles and whole column tiles only.  Bound by the matrix units' clock and by what the two ends of a tile still cost: of 26 us a tile of
+// 768 k spends 16 in its loop, 4.3 in the epilogue and, alone, 6 in front of the loop and between blocks, of which the second tile saves all.
+// 24 576 tokens of 768/1024, 8 experts: the step 843 -> 825 us.
+// ---------------------------------------------------------------------------
+template <class T>
+constexpr int stream_lds_elems() { return 2 * T::STAGE + T::NWAVES * 32 * (T::WN / 2); }
+
+// 32 x 64 values of a wave (element i of fragment f as value(f, i)) through its staging buffer to rows rowg0.. and columns col..
+template <class T, class Value>
+__device__ __forceinline__ void stream_flush(bf16_t* buf, __amdgpu_buffer_rsrc_t rs, uint32_t ldc, uint32_t col, int rowg0, int rrel, Value value) {
+    static_assert(T::WN == 128, "64 columns a half");
+    int lane = threadIdx.x % MTS_WAVE;
+    asm volatile("" : "+v"(lane));   // addresses are worked out here: kept over the k loop they would not fit the registers
+    const int ml = lane % 32;
+#pragma unroll
+    for (int f = 0; f < 2; ++f)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            stage4(buf + ml * 64 + (((4 * f + j) ^ (ml & 7)) << 3) + lane / 32 * 4, value(f, 4 * j), value(f, 4 * j + 1), value(f, 4 * j + 2), value(f, 4 * j + 3));
+#pragma unroll
+    for (int it = 0; it < 4; ++it) {
+        const int r = it * 8 + lane / 8, c = lane % 8;
+        const u32x4 v = *reinterpret_cast<const u32x4*>(buf + r * 64 + ((c ^ (r & 7)) << 3));
+        const uint32_t off = rowg0 + r < rrel ? ((uint32_t)(rowg0 + r) * ldc + col + (uint32_t)c * 8) * 2u : kInvalid;
+        __builtin_amdgcn_raw_buffer_store_b128(v, rs, (int)off, 0, 0);
+    }
+}
+
+template <class T>
+__device__ __forceinline__ void gateup_stream(const RowsParams& p, bf16_t* smem, int e, int row0, int rend, int ntile, int span) {
+    static_assert(T::STAGES == 2 && T::CHUNKS == 8, "two buffers of 64-wide k-tiles");
+    constexpr int TN = T::BN / 2;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / MTS_WAVE), lane = threadIdx.x % MTS_WAVE;
+    const int nk = p.Kdim / T::BKS, n0 = ntile * TN, total = nk * span;
+    if (wave >= T::NWAVES) {
+        const int pw = wave - T::NWAVES;
+        const __amdgpu_buffer_rsrc_t rs_a = p.a_gather ? make_rsrc(p.A, p.a_rows * p.lda * 2)
+                                                       : make_rsrc(p.A + (int64_t)row0 * p.lda, (int64_t)(rend - row0) * p.lda * 2);
+        const __amdgpu_buffer_rsrc_t rs_b = make_rsrc(p.B + (int64_t)e * p.b_rows * p.Kdim, (int64_t)p.b_rows * p.Kdim * 2);
+        uint32_t voff_a[T::A_INSTR], voff_b[T::B_INSTR];
+        const int slot = lane % T::CHUNKS, rin = lane / T::CHUNKS;
+        int row[T::A_INSTR], src[T::A_INSTR];
+#pragma unroll
+        for (int j = 0; j < T::A_INSTR; ++j) row[j] = row0 + (pw * T::A_INSTR + j) * T::RPI + rin;
+        gather_rows(p.a_gather, row0, rend, row, src);
+#pragma unroll
+        for (int j = 0; j < T::B_INSTR; ++j) {
+            const int br = (pw * T::B_INSTR + j) * T::RPI + rin;
+            voff_b[j] = ((uint32_t)(br / TN * p.N + n0 + br % TN) * (uint32_t)p.Kdim + (slot ^ ((br >> 1) & 7)) * 8) * 2u;
+        }
+        auto tile_a = [&](int stage, int kt) {
+            bf16_t* sa = smem + stage * T::STAGE + pw * T::A_INSTR * 512;
+            const int soff = kt * T::BKS * 2;
+#pragma unroll
+            for (int j = 0; j < T::A_INSTR; ++j) __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_a, MTS_LDS_PTR(sa + j * 512), 16, (int)voff_a[j], soff, 0, 0);
+        };
+        auto tile_b = [&](int stage, int kt, int tile) {
+            bf16_t* sb = smem + stage * T::STAGE + T::BM * T::BKS + pw * T::B_INSTR * 512;
+            const int soff = (kt * T::BKS + tile * TN * p.Kdim) * 2;
+#pragma unroll
+            for (int j = 0; j < T::B_INSTR; ++j) __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_b, MTS_LDS_PTR(sb + j * 512), 16, (int)voff_b[j], soff, 0, 0);
+        };
+        tile_b(0, 0, 0);
+#pragma unroll
+        for (int j = 0; j < T::A_INSTR; ++j) {
+            const int tr = row[j] - row0;
+            voff_a[j] = row[j] < rend ? ((uint32_t)src[j] * (uint32_t)p.lda + (slot ^ ((tr >> 1) & 7)) * 8) * 2u : kInvalid;
+        }
+        tile_a(0, 0);
+        int kt = 1, tile = 0;   // the k-tile that follows
+        for (int g = 0; g < total; ++g) {
+            wait_vmcnt<0>();
+            __builtin_amdgcn_s_barrier();   // k-tile g has landed, the one before is consumed
+            if (g + 1 < total) {
+                if (kt == nk) kt = 0, ++tile;
+                tile_a((g + 1) & 1, kt);
+                tile_b((g + 1) & 1, kt, tile);
+                ++kt;
+            }
+        }
+        return;
+    }
+    const int wm = wave / T::WAVES_N, wn = wave % T::WAVES_N;
+    float srow[T::MF];
+    load_row_weights<T, EPI_SWIGLU>(p, row0, rend, wm, srow);
+    FragPipe<T, true, T::BKS, false> pipe;
+    pipe.init(wm, wn);
+    bf16_t* buf = smem + 2 * T::STAGE + wave * 32 * 64;
+    const int rrel = rend - row0;
+    const uint32_t N = (uint32_t)p.N;
+    const __amdgpu_buffer_rsrc_t rs_c = make_rsrc(p.C ? p.C + (int64_t)row0 * 2 * N : nullptr, p.C ? (int64_t)rrel * 2 * N * 2 : 0);
+    const __amdgpu_buffer_rsrc_t rs_c2 = make_rsrc(p.C2 + (int64_t)row0 * N, (int64_t)rrel * N * 2);
+    int g = 0;
+    for (int tile = 0; tile < span; ++tile) {
+        f32x16 acc[T::MF][T::NF];
+        zero_acc<T>(acc);
+        for (int kt = 0; kt < nk; ++kt, ++g) {
+            __builtin_amdgcn_s_barrier();
+            const bf16_t* cur = smem + (g & 1) * T::STAGE;
+            pipe.prime(cur);
+#pragma unroll
+            for (int ks = 0; ks < T::BKS / 16 - 1; ++ks) pipe.step(ks, acc, cur, ks + 1);
+            pipe.template step<false>(T::BKS / 16 - 1, acc, cur, 0);
+        }
+        const uint32_t col = (uint32_t)(n0 + tile * TN + wn * 64);
+#pragma unroll
+        for (int mf = 0; mf < T::MF; ++mf) {
+            const int rowg0 = wm * T::WM + mf * 32;
+            if (p.C) {
+                stream_flush<T>(buf, rs_c, 2 * N, col, rowg0, rrel, [&](int f, int i) { return acc[mf][f][i]; });
+                stream_flush<T>(buf, rs_c, 2 * N, N + col, rowg0, rrel, [&](int f, int i) { return acc[mf][2 + f][i]; });
+            }
+            stream_flush<T>(buf, rs_c2, N, col, rowg0, rrel, [&](int f, int i) {
+                const float v = acc[mf][f][i];
+                return v * sigmoidf_(v) * acc[mf][2 + f][i] * srow[mf];
+            });
+        }
+    }
+}
+
 // the work of block `block` of a launch; `smem` holds ws_lds_elems<T, EPI>() elements, 1 KiB aligned.
 // TH (same block shape and columns, half the rows) runs the halves of the tiles that a launch with tail_slots cuts up.
 // A located tile, whole (T) or one of `parts` = 2 halves (TH).  The last tile of an expert is a half as well where it has no more rows than
@@ -2384,6 +2508,7 @@ __global__ __launch_bounds__(WsLarge::NT, WsLarge::WAVES_PER_EU) void bwd_joint_
 struct FwdJointParams {
     RowsParams gu, down;
     int n_gu;                  // blocks of the gate/up part (the down part's follow)
+    int span;                  // column tiles a gate/up block takes one after the other
     int32_t* ready;            // [max m-tiles]
     int32_t* done;             // [max m-tiles]
     int32_t* status;           // one word, sticky: FWD_JOINT_TIMEOUT | FWD_JOINT_PLACEMENT
@@ -2443,17 +2568,20 @@ __global__ __launch_bounds__(FwdGuTile::NT, FwdGuTile::WAVES_PER_EU) void fwd_jo
     constexpr int GU_LDS = ws_lds_elems<FwdGuTile, EPI_SWIGLU>(), DOWN_LDS = ws_lds_elems<FwdDownTile, EPI_PLAIN>();
     constexpr int LDS_ELEMS = GU_LDS > DOWN_LDS ? GU_LDS : DOWN_LDS;
     static_assert(LDS_ELEMS * 2 <= 160 * 1024, "LDS capacity");
+    static_assert(stream_lds_elems<FwdGuTile>() <= LDS_ELEMS && stream_lds_elems<FwdGuHalf>() <= LDS_ELEMS, "LDS of streamed tiles");
     __shared__ __attribute__((aligned(1024))) bf16_t smem[LDS_ELEMS];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / MTS_WAVE), lane = threadIdx.x % MTS_WAVE;
     int b = blockIdx.x;
     int e, row0, rend, ntile, parts, mtile;
     if (b < q.n_gu) {
         if (!locate_rows_tile<FwdGuTile::BM>(q.gu, b, e, row0, rend, ntile, parts, mtile)) return;   // whole tiles only
-        rows_gemm_ws_run<FwdGuTile, EPI_SWIGLU, false, FwdGuHalf>(q.gu, smem, e, row0, rend, ntile, 1);
+        if (q.span == 1) rows_gemm_ws_run<FwdGuTile, EPI_SWIGLU, false, FwdGuHalf>(q.gu, smem, e, row0, rend, ntile, 1);
+        else if (rend - row0 <= FwdGuHalf::BM) gateup_stream<FwdGuHalf>(q.gu, smem, e, row0, rend, ntile * q.span, q.span);
+        else gateup_stream<FwdGuTile>(q.gu, smem, e, row0, rend, ntile * q.span, q.span);
         if (wave < FwdGuTile::NWAVES) {
             wait_vmcnt<0>();   // this wave's rows of pre_act and post_act are in the L2
             if (lane == 0)
-                __hip_atomic_fetch_add(q.ready + mtile, 1 + (xcc_id() << kReadyCountBits), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_fetch_add(q.ready + mtile, q.span * (1 + (xcc_id() << kReadyCountBits)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         return;
     }
@@ -2740,11 +2868,27 @@ bool fwd_joint_pays(int64_t TK, int E, int I) {
     return m_tiles<FwdGuTile>(TK, E) * n_tiles_gu >= 2 * kXcds * kCusPerXcd;
 }
 
+// Two column tiles a gate/up block (gateup_stream) from four rounds of tiles on: below that the down tiles do not fill what longer blocks leave.
+// The pass forward, us, one tile / two: 12 288 tokens of 768/1024, 8 experts (3 rounds) 161 / 166, 16 384 (4) 198 / 188, 32 768 361 / 349; the launch
+// at other shapes of 6 to 9 rounds: 1024/1024 325 / 316, 512/1024 197 / 178, 64 experts of 1024/512 467 / 451.  Beyond 1024 of k a tile's loop hides its
+// ends (2048/768: 600 / 603).  Four tiles: 844 -> 868 for the step of 24 576 tokens (an XCD's blocks then hold twice the rows its L2 does).
+int stream_span(const RowsParams& gu, int64_t TK) {
+    const bool whole = gu.Kdim % FwdGuTile::BKS == 0 && gu.N % (FwdGuTile::BN / 2) == 0 && gu.n_tiles % 2 == 0;
+    return whole && gu.Kdim <= 1024 && TK / FwdGuTile::BM * gu.n_tiles >= 4 * kXcds * kCusPerXcd ? 2 : 1;
+}
 int launch_fwd_joint(RowsParams gu, RowsParams down, int64_t TK, int32_t* workspace, hipStream_t s) {
     FwdJointParams q = {};
     gu.reverse = down.reverse = 0;   // the down part follows the gate/up part through the range, oldest rows first
     gu.tail_slots = down.tail_slots = 0;
     q.n_gu = (int)rows_grid<FwdGuTile, EPI_SWIGLU>(gu, TK).x;
+    q.ready_count = FwdGuTile::NWAVES * gu.n_tiles;
+    q.span = stream_span(gu, TK);
+    if (q.span > 1) {   // the walk of the column tiles, in steps of span
+        gu.n_tiles /= q.span;
+        if (gu.n_tiles % gu.n_groups) gu.n_groups = 1;
+        set_dividers(gu);
+        q.n_gu /= q.span;
+    }
     // Only the end of the down part is ragged: its last m-tiles (per XCD) are cut into tiles of half the height, as many
     // as make about 3/8 of a round of whole tiles (measured at 768/1024: 2, 4 and 6 m-tiles of 3 tiles each give 276, 272
     // and 281 us; none 277).
@@ -2762,7 +2906,6 @@ int launch_fwd_joint(RowsParams gu, RowsParams down, int64_t TK, int32_t* worksp
     q.status = workspace;           // word 0; the counters start 16 bytes in
     q.ready = workspace + 4;
     q.done = q.ready + n;
-    q.ready_count = FwdGuTile::NWAVES * gu.n_tiles;
     q.spin_ticks = mts_tuning().fwd_joint_spin_us * 100;   // the wall clock counts at 100 MHz
     fwd_joint_kernel<FwdGuTile><<<dim3((unsigned)(q.n_gu + n_down)), FwdGuTile::NT, 0, s>>>(q);
     MTS_CHECK_LAUNCH();

@@ -602,3 +602,25 @@ def test_last_tiles_of_few_rows(counts, H, I):
     want, want_grads = oracle_moe_grads(*case, device="cuda")
     for got, ref, what in zip((out, *grads), (want, *want_grads), ("out", "dx", "dw1", "dw2", "dweights")):
         assert_close_scaled(got, ref, BF16_TOL, what)
+
+
+@pytest.mark.parametrize("H,I,T,dtype", [(64, 2048, 16500, torch.bfloat16), (192, 1024, 33100, torch.float16), (1024, 768, 44000, torch.bfloat16), (256, 1152, 36700, torch.bfloat16)])
+def test_gate_up_of_two_column_tiles_a_block(H, I, T, dtype):
+    """From four rounds of gate/up tiles on a block takes two of them in turn: one k-tile and many, last tiles of any height, an odd number of
+    column tiles (one a block); forward alone writes the same rows."""
+    print(f"two column tiles {H}/{I} T={T} {dtype}", flush=True)
+    E = 8
+    g = torch.Generator().manual_seed(T)
+    share = torch.tensor([0.21, 0.02, 0.15, 0.11, 0.0, 0.17, 0.13, 0.21])
+    idx = torch.multinomial(share, T, replacement=True, generator=g)
+    x, _, w1, w2, grad = O.make_inputs(T, T, H, E, I)
+    x, w1, w2, grad = (t.to(dtype) for t in (x, w1, w2, grad))
+    w = torch.rand(T, 1, generator=g).to(dtype)
+    case = (x, w1, w2, idx.int().unsqueeze(1), w, grad)
+    out, grads = hip_moe_grads(*case)
+    want, want_grads = oracle_moe_grads(*case, device="cuda")
+    for got, ref, what in zip((out, *grads), (want, *want_grads), ("out", "dx", "dw1", "dw2", "dweights")):
+        assert_close_scaled(got, ref, BF16_TOL, what)
+    with torch.no_grad():
+        alone = hip_backend().fused_moe(*(t.cuda() for t in (x, w1, w2, case[3], w)))
+    assert torch.equal(alone, out)
