@@ -49,9 +49,9 @@ RIDGE_FLOP_PER_BYTE = PEAK_BF16_TFLOPS * 1e12 / (PEAK_HBM_GBS * 1e9)   # 312.5: 
 # line names the file that holds the runs' commands and tables.
 TRAFFIC_SOURCE = "profiles/moe_layer_24x1024_hbm_traffic.txt"
 MEASURED_TRAFFIC_BYTES = {
-    "fwd_gateup_down": 783.4e6,   # gate/up and down as one launch; as two launches: 546.9 and 224.1
-    "fwd_gateup_swiglu": 546.9e6, "fwd_down": 224.1e6, "bwd_dy1": 531.4e6,
-    "bwd_joint": 1243.7e6,   # the joint launch (1078.8) and the launch of partial sums with the dX combine behind it (164.9)
+    "fwd_gateup_down": 915.9e6,   # gate/up and down as one launch; as two launches: 546.9 and 224.1
+    "fwd_gateup_swiglu": 546.9e6, "fwd_down": 224.1e6, "bwd_dy1": 531.6e6,
+    "bwd_joint": 1241.5e6,   # the joint launch (1076.5) and the launch of partial sums with the dX combine behind it (165.0)
     "combine": 114.4e6,
 }
 
