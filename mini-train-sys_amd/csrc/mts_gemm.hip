@@ -162,6 +162,7 @@ struct RowsParams {
                                // fill at most half of them, each of those is cut into two tiles of half the height (0: never)
     int tail_tiles;            // with xcd_ranges: this many tiles at the end of every XCD's list are cut in two whatever the rounds
                                // come to (a launch whose blocks start behind another part's: its rounds are not aligned)
+    int pairs;                 // with xcd_ranges: the tiles of an XCD's whole pairs of rounds go two a block (neighbouring columns): parts == kPair
     const int32_t* sched;      // with xcd_ranges: the m-tile range of every XCD (first[8], count[8]) from the schedule of the joint
                                // backward launch, or NULL: equal ranges
     int32_t* sched_out;        // dO*W2 launch: one more block writes the schedule of the joint backward launch here (NULL: none)
@@ -618,6 +619,11 @@ __device__ __forceinline__ void rows_epilogue(const RowsParams& p, f32x16 (&acc)
 // same time and each of them again for every group of m-tiles.
 // ---------------------------------------------------------------------------
 constexpr int kXcds = 8, kCusPerXcd = 32;
+constexpr int kPair = 0;   // pieces of a tile that is one of two
+// tiles of an XCD's list (an even number) that go two a block: all from four rounds on, below that those of whole pairs of rounds
+__host__ __device__ __forceinline__ int paired_tiles(int tiles) {
+    return tiles >= 4 * kCusPerXcd ? tiles : tiles / (2 * kCusPerXcd) * (2 * kCusPerXcd);
+}
 
 // The expert that owns m-tile `tile` is found with one vector load: lane l reads
 // expert_start[l] and [l+1], a wave scan turns tile counts into tile offsets, and a
@@ -672,6 +678,12 @@ __device__ __forceinline__ bool find_rows_tile(const RowsParams& p, int b, int& 
                 j = whole + (j - whole) / 2;
                 k = p.by_n_tiles.quotient(j, ntile);
             }
+        }
+        if (p.pairs) {
+            const int paired = paired_tiles(my * p.n_tiles);
+            if (2 * j < paired) parts = kPair, j *= 2;
+            else j += paired / 2;
+            k = p.by_n_tiles.quotient(j, ntile);
         }
         if (p.n_groups > 1 && my > 0) {
             // group g of the columns, m-tile k of the range, column r of the group: j = (g * my + k) * npg + r
@@ -2508,7 +2520,6 @@ __global__ __launch_bounds__(WsLarge::NT, WsLarge::WAVES_PER_EU) void bwd_joint_
 struct FwdJointParams {
     RowsParams gu, down;
     int n_gu;                  // blocks of the gate/up part (the down part's follow)
-    int span;                  // column tiles a gate/up block takes one after the other
     int32_t* ready;            // [max m-tiles]
     int32_t* done;             // [max m-tiles]
     int32_t* status;           // one word, sticky: FWD_JOINT_TIMEOUT | FWD_JOINT_PLACEMENT
@@ -2575,13 +2586,14 @@ __global__ __launch_bounds__(FwdGuTile::NT, FwdGuTile::WAVES_PER_EU) void fwd_jo
     int e, row0, rend, ntile, parts, mtile;
     if (b < q.n_gu) {
         if (!locate_rows_tile<FwdGuTile::BM>(q.gu, b, e, row0, rend, ntile, parts, mtile)) return;   // whole tiles only
-        if (q.span == 1) rows_gemm_ws_run<FwdGuTile, EPI_SWIGLU, false, FwdGuHalf>(q.gu, smem, e, row0, rend, ntile, 1);
-        else if (rend - row0 <= FwdGuHalf::BM) gateup_stream<FwdGuHalf>(q.gu, smem, e, row0, rend, ntile * q.span, q.span);
-        else gateup_stream<FwdGuTile>(q.gu, smem, e, row0, rend, ntile * q.span, q.span);
+        const int span = parts == kPair ? 2 : 1;
+        if (span == 1) rows_gemm_ws_run<FwdGuTile, EPI_SWIGLU, false, FwdGuHalf>(q.gu, smem, e, row0, rend, ntile, 1);
+        else if (rend - row0 <= FwdGuHalf::BM) gateup_stream<FwdGuHalf>(q.gu, smem, e, row0, rend, ntile, span);
+        else gateup_stream<FwdGuTile>(q.gu, smem, e, row0, rend, ntile, span);
         if (wave < FwdGuTile::NWAVES) {
             wait_vmcnt<0>();   // this wave's rows of pre_act and post_act are in the L2
             if (lane == 0)
-                __hip_atomic_fetch_add(q.ready + mtile, q.span * (1 + (xcc_id() << kReadyCountBits)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_fetch_add(q.ready + mtile, span * (1 + (xcc_id() << kReadyCountBits)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         return;
     }
@@ -2868,13 +2880,14 @@ bool fwd_joint_pays(int64_t TK, int E, int I) {
     return m_tiles<FwdGuTile>(TK, E) * n_tiles_gu >= 2 * kXcds * kCusPerXcd;
 }
 
-// Two column tiles a gate/up block (gateup_stream) from four rounds of tiles on: below that the down tiles do not fill what longer blocks leave.
-// The pass forward, us, one tile / two: 12 288 tokens of 768/1024, 8 experts (3 rounds) 161 / 166, 16 384 (4) 198 / 188, 32 768 361 / 349; the launch
-// at other shapes of 6 to 9 rounds: 1024/1024 325 / 316, 512/1024 197 / 178, 64 experts of 1024/512 467 / 451.  Beyond 1024 of k a tile's loop hides its
-// ends (2048/768: 600 / 603).  Four tiles: 844 -> 868 for the step of 24 576 tokens (an XCD's blocks then hold twice the rows its L2 does).
-int stream_span(const RowsParams& gu, int64_t TK) {
-    const bool whole = gu.Kdim % FwdGuTile::BKS == 0 && gu.N % (FwdGuTile::BN / 2) == 0 && gu.n_tiles % 2 == 0;
-    return whole && gu.Kdim <= 1024 && TK / FwdGuTile::BM * gu.n_tiles >= 4 * kXcds * kCusPerXcd ? 2 : 1;
+// Two column tiles a gate/up block (gateup_stream): all tiles of an XCD that has four rounds of them, below that those of whole pairs of rounds, the
+// others one a block behind them (all in pairs leaves CUs idle that the down tiles do not fill: 12 288 tokens of 768/1024, three rounds, 161 us one
+// a block, 166 in pairs, 152 -> 149 so).  The pass forward, us, before and now: 8192 tokens (2.1 rounds) 120 -> 113, 14 000 166 -> 162, 16 384
+// 198 -> 182, 32 768 361 -> 349; the launch at other shapes of 6 to 9 rounds: 1024/1024 325 -> 316, 512/1024 197 -> 178, 64 experts of 1024/512
+// 467 -> 451.  Beyond 1024 of k a tile's loop hides its ends (2048/768: 600 / 603).  Four tiles a block: the step of 24 576 tokens 844 -> 868 (an
+// XCD's blocks then hold twice the rows its L2 does).
+int stream_pairs(const RowsParams& gu) {
+    return gu.xcd_ranges && gu.Kdim % FwdGuTile::BKS == 0 && gu.Kdim <= 1024 && gu.N % FwdGuTile::BN == 0 && gu.n_tiles / gu.n_groups % 2 == 0;
 }
 int launch_fwd_joint(RowsParams gu, RowsParams down, int64_t TK, int32_t* workspace, hipStream_t s) {
     FwdJointParams q = {};
@@ -2882,12 +2895,11 @@ int launch_fwd_joint(RowsParams gu, RowsParams down, int64_t TK, int32_t* worksp
     gu.tail_slots = down.tail_slots = 0;
     q.n_gu = (int)rows_grid<FwdGuTile, EPI_SWIGLU>(gu, TK).x;
     q.ready_count = FwdGuTile::NWAVES * gu.n_tiles;
-    q.span = stream_span(gu, TK);
-    if (q.span > 1) {   // the walk of the column tiles, in steps of span
-        gu.n_tiles /= q.span;
-        if (gu.n_tiles % gu.n_groups) gu.n_groups = 1;
-        set_dividers(gu);
-        q.n_gu /= q.span;
+    gu.pairs = stream_pairs(gu);
+    if (gu.pairs) {   // as many blocks as the longest list of an XCD makes, whatever its length comes to
+        int blocks = 0;
+        for (int tiles = 0; tiles <= q.n_gu / kXcds; tiles += gu.n_tiles) blocks = tiles - paired_tiles(tiles) / 2 > blocks ? tiles - paired_tiles(tiles) / 2 : blocks;
+        q.n_gu = blocks * kXcds;
     }
     // Only the end of the down part is ragged: its last m-tiles (per XCD) are cut into tiles of half the height, as many
     // as make about 3/8 of a round of whole tiles (measured at 768/1024: 2, 4 and 6 m-tiles of 3 tiles each give 276, 272

@@ -604,10 +604,10 @@ def test_last_tiles_of_few_rows(counts, H, I):
         assert_close_scaled(got, ref, BF16_TOL, what)
 
 
-@pytest.mark.parametrize("H,I,T,dtype", [(64, 2048, 16500, torch.bfloat16), (192, 1024, 33100, torch.float16), (1024, 768, 44000, torch.bfloat16), (256, 1152, 36700, torch.bfloat16)])
+@pytest.mark.parametrize("H,I,T,dtype", [(256, 1024, 17300, torch.bfloat16), (64, 2048, 16500, torch.bfloat16), (192, 1024, 33100, torch.float16), (1024, 768, 44000, torch.bfloat16), (256, 1152, 36700, torch.bfloat16)])
 def test_gate_up_of_two_column_tiles_a_block(H, I, T, dtype):
-    """From four rounds of gate/up tiles on a block takes two of them in turn: one k-tile and many, last tiles of any height, an odd number of
-    column tiles (one a block); forward alone writes the same rows."""
+    """From two rounds of gate/up tiles on blocks take two of them in turn, from four on all of them: one k-tile and many, last tiles of any
+    height, an odd number of column tiles (one a block); forward alone writes the same rows."""
     print(f"two column tiles {H}/{I} T={T} {dtype}", flush=True)
     E = 8
     g = torch.Generator().manual_seed(T)
