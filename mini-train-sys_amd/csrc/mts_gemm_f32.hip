@@ -4,8 +4,10 @@
 // An fp32 value is the exact sum of three bf16 ones (x = x0 + x1 + x2, each the rest rounded to nearest: mts_split3.h), a
 // product of two bf16 values is exact in fp32, and the bf16 matrix instruction adds in fp32 at 16 times the rate of the fp32
 // one.  A product is therefore taken as x0*y0 + x0*y1 + x1*y0 + x1*y1 + x0*y2 + x2*y0; the three terms left out are below
-// 2^-26 of it, a quarter of an fp32 rounding.  k-tiles that hold a value whose split is not exact (infinite, NaN, below 2^-60 or
-// from 2^127 on, but not zero) are multiplied by the fp32 instruction instead.
+// 2^-26 of it, a quarter of an fp32 rounding, and a sum of three and more products still comes out closer than from the fp32
+// instruction, which rounds more often.  Shorter sums (the weight gradient of an expert with one or two rows) are left to
+// that instruction, and so are k-tiles that hold a value whose split is not exact (infinite, NaN, below 2^-60 or
+// from 2^127 on, but not zero).
 //
 // What bounds it: on paper the matrix pipes (six instructions of 32 cycles for a 32 x 32 x 16 product: 417 TFLOP/s at 2.4 GHz, 2.7 times the fp32
 // instruction), in fact the vector unit that splits: a value costs about 8 vector instructions, each 4.9 cycles of a SIMD, and a wave alone
@@ -14,7 +16,7 @@
 // loads that never depend on a branch.  2048 tokens, 768/1024, 8 experts, top-2, us before (fp32 instruction) and now: gate/up 178 -> 112, down
 // 90 -> 60, dO*W2 95 -> 90, dX 167 -> 96, dW1 146 -> 87, dW2 76 -> 57; 8192 tokens: 588 -> 397, 282 -> 172, 298 -> 227, 498 -> 324, 512 -> 303, 266 -> 177.
 // Relative error against fp64 over all five results of the operator: 4.1e-7..1.02e-6 where the fp32 instruction had 4.3e-7..1.18e-6,
-// smaller for each at every size (fewer roundings of a sum: 6 per 16 products instead of 8).
+// smaller for each at every size; by the length of the sum: mts_split3.h.
 #include "mts_split3.h"
 
 #include <type_traits>
@@ -107,7 +109,6 @@ __global__ __launch_bounds__(kThreads, 4) void rows_gemm_f32_kernel(Rows32 p) {
         if (threadIdx.x < BM) row_weight[threadIdx.x] = p.route_w && r < rend ? p.route_w[p.s_scatter[r]] : 1.f;
     }
     if (threadIdx.x == 0) special = 0;
-    const int tiles = (p.Kdim + TK - 1) / TK;
     f32x16 acc[MF][NF] = {};
     const int wave = threadIdx.x / MTS_WAVE, wm = wave / WAVES_N, wn = wave % WAVES_N, lane = threadIdx.x % MTS_WAVE;
     auto a_at = [&](int mf) { return wm * (BM / WAVES_M) + mf * 32; };
@@ -142,7 +143,7 @@ __global__ __launch_bounds__(kThreads, 4) void rows_gemm_f32_kernel(Rows32 p) {
             } else b.fetch(set, t * TK, p.Kdim);
         };
         load_k_tiles(p.Kdim, a, b, As, Bs, (LdsWord*)&special, fetch);
-    } else multiply_k_tiles<ATile, BTile>(tiles, As, Bs, (LdsWord*)&special, acc, a_at, b_at);
+    } else multiply_k_tiles<ATile, BTile>(p.Kdim, As, Bs, (LdsWord*)&special, acc, a_at, b_at);
 
     if (threadIdx.x < kLoaders) {
 #pragma unroll
@@ -254,7 +255,6 @@ __global__ __launch_bounds__(kThreads, 4) void dw_gemm_f32_kernel(Dw32 p) {
     const int rbeg = p.expert_start[e], rend = p.expert_start[e + 1];
 
     if (threadIdx.x == 0) special = 0;
-    const int tiles = (rend - rbeg + TK - 1) / TK;
     const int wave = threadIdx.x / MTS_WAVE, wm = wave / 2, wn = wave % 2, lane = threadIdx.x % MTS_WAVE;
     auto a_at = [&](int mf) { return wm * (BM / 2) + mf * 32; };
     auto b_at = [&](int nf) { return wn * (BN / 2) + nf * 32; };
@@ -291,7 +291,7 @@ __global__ __launch_bounds__(kThreads, 4) void dw_gemm_f32_kernel(Dw32 p) {
         load_k_tiles(rend - rbeg, a, b, Ps, Qs, (LdsWord*)&special, fetch);
         return;
     }
-    multiply_k_tiles<PT, QT>(tiles, Ps, Qs, (LdsWord*)&special, acc, a_at, b_at);
+    multiply_k_tiles<PT, QT>(rend - rbeg, Ps, Qs, (LdsWord*)&special, acc, a_at, b_at);
 
     OutT* C = reinterpret_cast<OutT*>(p.C) + (int64_t)e * p.M * p.N;
 #pragma unroll

@@ -22,6 +22,13 @@ constexpr uint32_t kSmallest = 0x21800000u;   // 2^-60
 constexpr uint32_t kBeyond = 0x7f000000u;     // 2^127
 constexpr uint32_t kMarker = 0x7fffu;         // third plane of a value kept as its bits: a NaN, which no split gives
 
+// Sums of so few terms are left to the fp32 instruction, which rounds once for each: six bf16 products a term and the three left out come to more
+// than that.  Relative error against fp64 (norm, and the worst of 512 x 512 sums over the sum of the terms' sizes), fp32 instruction / six products:
+// 1 term 2.5e-8 / 3.5e-8, 0.6e-7 / 1.5e-7; 2 terms 3.1e-8 / 3.3e-8, 1.1e-7 / 1.2e-7; 3 terms 3.6e-8 / 3.3e-8, 1.5e-7 / 1.2e-7; 16 terms 7.4e-8 / 3.4e-8,
+// 2.3e-7 / 1.0e-7; 17 terms (the second k-tile) 7.5e-8 / 6.3e-8, 2.2e-7 / 2.1e-7; 1024 terms 5.7e-7 / 4.9e-7, 2.5e-7 / 2.4e-7.  All nine products: 1 term
+// 3.4e-8, 1.2e-7, and a fifth more time.
+constexpr int kFewTerms = 2;
+
 // The loads of the loops below are unconditional: a load that a lane or a pass may skip makes the compiler wait for all loads in flight at the
 // next use of any.  What lies outside an operand is read from its last element instead, and set to zero where it would be added.
 
@@ -248,12 +255,13 @@ __device__ __forceinline__ void load_k_tiles(int Kdim, AT& a, BT& b, bf16_t* As,
     __syncthreads();
 }
 template <class AT, class BT, int MF, int NF, class AAt, class BAt>
-__device__ __forceinline__ void multiply_k_tiles(int tiles, const bf16_t* As, const bf16_t* Bs, LdsWord* special, f32x16 (&acc)[MF][NF], AAt a_at,
+__device__ __forceinline__ void multiply_k_tiles(int Kdim, const bf16_t* As, const bf16_t* Bs, LdsWord* special, f32x16 (&acc)[MF][NF], AAt a_at,
                                                  BAt b_at) {
+    const int tiles = (Kdim + TK - 1) / TK;
     __syncthreads();
     int t = 0;
     __syncthreads();   // k-tile 0 has landed
-    for (; t < tiles; ++t) {
+    for (; t < tiles && Kdim > kFewTerms; ++t) {
         const int first = __builtin_amdgcn_readfirstlane(*special);
         if (first && t + 1 >= first) break;
         mma_tile<AT, BT>(As + t % 2 * AT::SIZE, Bs + t % 2 * BT::SIZE, acc, a_at, b_at);

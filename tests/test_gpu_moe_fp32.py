@@ -87,3 +87,24 @@ def test_values_that_three_bf16_terms_do_not_hold(R, H, I):
             assert torch.equal(dw[e, h].isnan(), want[h].isnan()), h
             if want[h].isfinite().all():
                 assert_close_scaled(dw[e, h], want[h], 1e-5, f"column {h}")
+
+
+@pytest.mark.parametrize("R", [1, 2, 3, 17])
+@pytest.mark.parametrize("M,N", [(72, 100), (1100, 2100)])   # both tile sizes
+def test_sums_of_few_terms(R, M, N):
+    """A sum of one term is that product rounded once; sums of up to n terms err by no more than a rounding of the running sum for
+    each (n * 2^-24 of the terms' sizes), as the fp32 instruction's do."""
+    print(f"few fp32 terms R={R} M={M} N={N}", flush=True)
+    torch.manual_seed(R + M)
+
+    def check(got, want, size, name):
+        if R == 1:
+            assert torch.equal(got, want.float()), name
+        assert ((got.double() - want).abs() <= R * 2.0 ** -24 * size).all(), name
+
+    d_out, act = torch.randn(R, M), torch.randn(R, N)
+    dw = _dw2(d_out.cuda(), act.cuda(), [0, R])[0]
+    check(dw, d_out.double().t() @ act.double(), d_out.double().abs().t() @ act.double().abs(), "weight gradient")
+    act, w2 = torch.randn(M, R), torch.randn(1, N, R)
+    y = _down(act.cuda(), w2.cuda(), [0, M])
+    check(y, act.double() @ w2[0].double().t(), act.double().abs() @ w2[0].double().abs().t(), "rows")
