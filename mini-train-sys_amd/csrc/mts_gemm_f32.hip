@@ -7,7 +7,7 @@
 // 2^-26 of it, a quarter of an fp32 rounding, and a sum of three and more products still comes out closer than from the fp32
 // instruction, which rounds more often.  Shorter sums (the weight gradient of an expert with one or two rows) are left to
 // that instruction, and so are k-tiles that hold a value whose split is not exact (infinite, NaN, below 2^-60 or
-// from 2^127 on, but not zero).
+// from 2^50 on, but not zero).
 //
 // What bounds it: on paper the matrix pipes (six instructions of 32 cycles for a 32 x 32 x 16 product: 417 TFLOP/s at 2.4 GHz, 2.7 times the fp32
 // instruction), in fact the vector unit that splits: a value costs about 8 vector instructions, each 4.9 cycles of a SIMD, and a wave alone

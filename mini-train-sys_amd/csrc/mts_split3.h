@@ -2,9 +2,11 @@
 // bf16 planes on their way into LDS, fragment reads and the k loop of a block of four waves.
 //
 // x0 = bf16(x), x1 = bf16(x - x0), x2 = x - x0 - x1, each rounded to nearest: the differences are exact, x1 is at most 2^-9 of x
-// and x2 at most 2^-18, and x2 fits 8 bits, so x = x0 + x1 + x2 for every x in [2^-60, 2^127) and for zero.  Any other value (the
-// planes could overflow, or lose bits below the smallest normal number in a product) goes into the planes as its own bits
-// with a marker, and its k-tile and the ones behind it are multiplied by the fp32 instruction from the values put together again.
+// and x2 at most 2^-18, and x2 fits 8 bits, so x = x0 + x1 + x2 (the splitting of Henry, Tang and Heinecke, "Leveraging the bfloat16
+// Artificial Intelligence Datatype For Higher-Precision Computations", 2019).  Values in [2^-60, 2^50) and zero are split so.  Below, a
+// product could lose bits under the smallest number there is; above, a sum could leave the range of fp32 where the values' own does
+// not, because x0 may be rounded up: sums of fewer than 2^27 products below 2^100 cannot.  Any other value goes into the planes as its
+// own bits with a marker, and its k-tile and the ones behind it are multiplied by the fp32 instruction from the values put together again.
 #pragma once
 
 #include "mts_common.h"
@@ -19,7 +21,7 @@ constexpr int kDepth = 2;                // k-tiles in flight in registers, and 
 typedef volatile __attribute__((address_space(3))) int LdsWord;
 
 constexpr uint32_t kSmallest = 0x21800000u;   // 2^-60
-constexpr uint32_t kBeyond = 0x7f000000u;     // 2^127
+constexpr uint32_t kBeyond = 0x58800000u;     // 2^50
 constexpr uint32_t kMarker = 0x7fffu;         // third plane of a value kept as its bits: a NaN, which no split gives
 
 // Sums of so few terms are left to the fp32 instruction, which rounds once for each: six bf16 products a term and the three left out come to more

@@ -108,3 +108,30 @@ def test_sums_of_few_terms(R, M, N):
     act, w2 = torch.randn(M, R), torch.randn(1, N, R)
     y = _down(act.cuda(), w2.cuda(), [0, M])
     check(y, act.double() @ w2[0].double().t(), act.double().abs() @ w2[0].double().abs().t(), "rows")
+
+
+@pytest.mark.parametrize("R,H,I", [(90, 72, 100), (2700, 1100, 260)])   # both tile sizes
+def test_products_at_the_ends_of_the_range(R, H, I):
+    """Products just below the largest number, alone and in a sum, are finite although a value rounded to fewer bits would not be; products
+    of two numbers near 2^-60 keep all their bits, the smallest of which lie below the smallest normal number.  1e-5 as above."""
+    print(f"ends of the range R={R} H={H} I={I}", flush=True)
+    torch.manual_seed(R)
+    starts = [0, R]
+    below = torch.tensor(1.0 - 2.0 ** -24)
+    act, w2 = torch.zeros(R, I), torch.zeros(1, H, I)
+    act[0, 7], w2[0, :, 7] = below * 2.0 ** 127, below * 2.0
+    act[1, 20:24], w2[0, :, 20:24] = 0.999 * 2.0 ** 64, 0.999 * 2.0 ** 62
+    act[2, 40:], w2[0, :, 40:] = torch.randn(I - 40), torch.randn(H, I - 40)
+    y = _down(act.cuda(), w2.cuda(), starts)
+    want = act.double() @ w2[0].double().t()
+    assert want[:3].float().isfinite().all()
+    for r in range(4):
+        assert_close_scaled(y[r].double(), want[r], 1e-5, f"row {r}")
+    near = 2.0 ** -60
+    act, w2 = (1 + torch.rand(R, I)) * near, (1 + torch.rand(1, H, I)) * torch.randn(1, H, I).sign() * near
+    y = _down(act.cuda(), w2.cuda(), starts)
+    assert_close_scaled(y.double() / near / near, (act.double() @ w2[0].double().t()) / near / near, 1e-5, "small products")
+    d_out, act = torch.zeros(R, H), torch.zeros(R, I)
+    d_out[3:7, 1], act[3:7, 2] = 0.999 * 2.0 ** 64, 0.999 * 2.0 ** 62
+    dw = _dw2(d_out.cuda(), act.cuda(), starts)[0]
+    assert_close_scaled(dw.double(), d_out.double().t() @ act.double(), 1e-5, "weight gradient")
