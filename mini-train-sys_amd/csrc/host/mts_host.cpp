@@ -666,9 +666,10 @@ LayerForward layer_forward(const Tensor& x_, const Tensor& w_r_, const Tensor& w
     if (alone) scratch.add(post_act, TK, I, dtype);
     scratch.make();
     if (!alone) kept.make();
-    // E mean probabilities, z, entropy, load-balancing term, E + 7 load statistics; the counts behind them
-    const int64_t floats = 2 * E + 10;
-    Tensor stats = f32({floats + E}, x);
+    // E mean probabilities, z, entropy, load-balancing term, E + 7 load statistics.  The counts are integers and have an allocation of
+    // their own: a caller may save all results together, which torch refuses for one storage under two types.
+    Tensor stats = f32({2 * E + 10}, x);
+    f.counts = i32({E}, x);
     if (alone) {   // nobody differentiates: parts instead of views
         auto floats_at = [&](int64_t first, at::IntArrayRef size) { return part_of(stats, first * 4, size, at::kFloat); };
         f.prob_mean = floats_at(0, {E}), f.z_loss = floats_at(E, {}), f.entropy = floats_at(E + 1, {}), f.load_balance = floats_at(E + 2, {});
@@ -677,7 +678,6 @@ LayerForward layer_forward(const Tensor& x_, const Tensor& w_r_, const Tensor& w
         f.prob_mean = stats.narrow(0, 0, E), f.z_loss = stats.select(0, E), f.entropy = stats.select(0, E + 1), f.load_balance = stats.select(0, E + 2);
         f.load_stats = stats.narrow(0, E + 3, E + 7);
     }
-    f.counts = part_of(stats, floats * 4, {E}, at::kInt);
     void* load_stats = limited ? nullptr : ptr(f.load_stats);
     void* cast_weights = narrow && !limited ? ptr(weights_act) : nullptr;
     if (few) {

@@ -397,6 +397,25 @@ def test_layer_without_gradients_equals_the_node(T, H, E, I, K, dtype, capacity)
     assert again[0].shape == want[0].shape and torch.equal(outside[0], want[0])
 
 
+@pytest.mark.parametrize("gradients", [False, True])
+@pytest.mark.parametrize("E,capacity", [(8, None), (8, 40), (24, None)])
+def test_results_of_the_layer_are_saved_together(gradients, E, capacity):
+    """Counts are integers and statistics are not: one storage under two types could not be saved."""
+    import io
+
+    print(f"saving the layer's results E={E} capacity={capacity} gradients={gradients}", flush=True)
+    x, w_r, w1, w2, _ = O.make_inputs(41, 100, 64, E, 32)
+    args = [x.bfloat16().cuda(), w_r.cuda(), w1.bfloat16().cuda(), w2.bfloat16().cuda()]
+    for t in args if gradients else ():
+        t.requires_grad_(True)
+    results = [t.detach() for t in hip_backend().moe_layer(*args, 2, normalize=True, capacity=capacity)]
+    file = io.BytesIO()
+    torch.save(results, file)
+    file.seek(0)
+    for a, b in zip(torch.load(file, weights_only=True), results):
+        assert a.dtype == b.dtype and torch.equal(a, b)
+
+
 @pytest.mark.parametrize("T,E,K", [(1, 17, 1), (40, 24, 4), (3000, 64, 8), (700, 1000, 2)])
 def test_router_and_routing_of_many_experts_as_one_chain(T, E, K):
     """Statistics that a second block reduces beside the scan, and the permutation: those of the two calls, bit for bit."""
