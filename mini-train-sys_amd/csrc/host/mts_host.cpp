@@ -20,6 +20,7 @@
 #include <pybind11/pybind11.h>
 #include <pybind11/stl.h>
 #include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/graph_task.h>
 #include <torch/csrc/utils/pybind.h>
 
 #include <array>
@@ -985,8 +986,9 @@ struct QkvRope : torch::autograd::Function<QkvRope> {
 // 279 / 555 and 278 / 375, 512 rows 69 / 197 and 58 / 67; 1024 rows of 8192 31 / 44 and 26 / 25), and dX no longer where a projection
 // is less than eight times as wide as its input (12 288 rows of 2304 48 / 45, 8192 rows of 4096 -> 12 288 612 / 594).
 constexpr int64_t kLinearRoundsRows = 128;
+int64_t row_pitch(int64_t N) { return (N + 63) / 64 * 64; }   // 16-bit rows that start on 128 bytes
 bool linear_in_rounds(const Tensor& x, int64_t T, int64_t N, int64_t K) {
-    return T >= kLinearRoundsRows && N >= 8 * K && N < k2GiB && mts_linear_rounds_supported(dtype_code(x), T, N, K, (N + 7) / 8 * 8);
+    return T >= kLinearRoundsRows && N >= 8 * K && N < k2GiB && mts_linear_rounds_supported(dtype_code(x), T, N, K, row_pitch(N));
 }
 // rows that mts_linear_dx_rounds and mts_linear_dw_rounds read in place
 bool rows_fit(const Tensor& g) { return g.stride(1) == 1 && g.stride(0) >= g.size(1) && g.stride(0) % 8 == 0 && aligned16(g); }
@@ -1044,14 +1046,12 @@ struct Linear : torch::autograd::Function<Linear> {
             return {dx, at::matmul(g.to(at::kFloat).t().contiguous(), x.reshape({T, K}).to(at::kFloat))};
         }
         if (rounds) {
-            const Tensor g = grads[0].reshape({T, N});
-            if (rows_fit(g) && mts_linear_rounds_supported(dtype_code(x), T, N, K, g.stride(0))) return in_rounds(ctx, g, x, rounded, T, N, K);
-            if (!mts_linear_dw_supported(dtype_code(x), T, N, K)) {   // rows at odd places: a copy costs more than it gives
-                Tensor dx, dw;
-                if (ctx->needs_input_grad(0)) dx = at::matmul(g, rounded).view(x.sizes());
-                if (ctx->needs_input_grad(1)) dw = at::matmul(g.t(), x.reshape({T, K})).to(at::kFloat);
-                return {dx, dw};
-            }
+            // Rows at odd places are copied.  us, copy and both gradients / the library's products, 50 257 columns, 768 wide: 24 576 rows 3909 / 4712,
+            // 8192 1390 / 1375, 2048 403 / 597, 512 180 / 325, 128 116 / 305; 1024 rows of 8193 66 / 76.
+            Tensor g = grads[0].reshape({T, N});
+            if (!rows_fit(g) || !mts_linear_rounds_supported(dtype_code(x), T, N, K, g.stride(0)))
+                g = at::empty({T, row_pitch(N)}, g.options()).narrow(1, 0, N).copy_(g);
+            return in_rounds(ctx, g, x, rounded, T, N, K);
         }
         const Tensor g = dense16(grads[0].reshape({T, N})), in = dense16(x.reshape({T, K}));
         Tensor dx, dw;
@@ -1124,24 +1124,28 @@ bool cross_entropy_supported(const Tensor& logits, const Tensor& targets) {
            logits.size(1) < k2GiB;
 }
 
-// Whether the logits come, through views at most, from a projection whose gradients read rows of any pitch (Linear::in_rounds)
-bool logits_of_rounds(const Tensor& logits) {
-    if (!at::GradMode::is_enabled() || !logits.requires_grad() || logits.scalar_type() == at::kFloat) return false;
-    std::shared_ptr<torch::autograd::Node> fn = logits.grad_fn();
+// Whether the gradient that `self` returns goes, through views at most, to a projection whose gradients read rows of any pitch
+// (Linear::in_rounds), and nobody sees it on the way: no hook, no retained gradient, no result of autograd.grad.  Whoever does gets it dense.
+bool goes_to_rounds(torch::autograd::Node* self) {
+    const auto* execution = torch::autograd::get_current_graph_task_exec_info();
+    if (!self || !execution || !self->post_hooks().empty()) return false;
+    torch::autograd::Node* fn = self->next_edge(0).function.get();
     for (int depth = 0; fn && depth < 4; ++depth) {
-        if (dynamic_cast<torch::autograd::CppNode<Linear>*>(fn.get())) return true;
+        if (!fn->pre_hooks().empty() || !fn->tensor_pre_hooks().empty() || !fn->retains_grad_hooks().empty() || !fn->post_hooks().empty()) return false;
+        const auto found = execution->find(fn);
+        if (found != execution->end() && found->second.captures_) return false;
+        if (dynamic_cast<torch::autograd::CppNode<Linear>*>(fn)) return true;
         const std::string name = fn->name();
         if ((name != "ViewBackward0" && name != "UnsafeViewBackward0" && name != "ReshapeAliasBackward0") || fn->num_outputs() != 1) return false;
-        fn = fn->next_edge(0).function;
+        fn = fn->next_edge(0).function.get();
     }
     return false;
 }
 
 // mean cross-entropy without an fp32 copy of the logits
 struct CrossEntropy : torch::autograd::Function<CrossEntropy> {
-    // dense16, dense; `pitched`: the rows of the gradient start on 128 bytes
-    static Tensor forward(AutogradContext* ctx, const Tensor& logits, const Tensor& targets, bool pitched) {
-        ctx->saved_data["pitched"] = pitched;
+    // dense16, dense
+    static Tensor forward(AutogradContext* ctx, const Tensor& logits, const Tensor& targets) {
         const int64_t N = logits.size(0), V = logits.size(1);
         // per row: maximum, log of the sum, loss; then 1 / count.  The loss is a tensor of its own, which the caller may change
         // (no view) and which is not kept.
@@ -1163,23 +1167,23 @@ struct CrossEntropy : torch::autograd::Function<CrossEntropy> {
             const Tensor p = at::softmax(s[0].to(at::kFloat), 1) - hit.to(at::kFloat), none = at::zeros({}, p.options());
             const Tensor ignored = t.eq(kIgnoreIndex), outside = t.lt(0).logical_or(t.ge(V)).logical_and(ignored.logical_not());
             const Tensor scale = g * s[2].select(0, 3 * N) + at::where(outside, at::full({}, NAN, p.options()), none);
-            return {at::where(ignored, none, p * scale).to(s[0].scalar_type()), Tensor(), Tensor()};
+            return {at::where(ignored, none, p * scale).to(s[0].scalar_type()), Tensor()};
         }
         const Tensor g = like_f32(grads[0]);
         const float* row = ptr_as<float>(s[2]);
-        if (ctx->saved_data["pitched"].toBool() && V % 8) {
-            const int64_t pitch = (V + 63) / 64 * 64;
+        if (V % 8 && s[0].scalar_type() != at::kFloat && goes_to_rounds(torch::autograd::get_current_node().get())) {
+            const int64_t pitch = row_pitch(V);
             Tensor rows = at::empty({N, pitch}, s[0].options());
             check(mts_cross_entropy_bwd_pitched(ptr(s[0]), ptr_as<int64_t>(s[1]), N, V, kIgnoreIndex, dtype_code(s[0]), row, row + N, ptr_as<float>(g),
                                                 row + 3 * N, ptr(rows), pitch, stream_of(s[0])),
                   "mts_cross_entropy_bwd_pitched");
-            return {rows.narrow(1, 0, V), Tensor(), Tensor()};
+            return {rows.narrow(1, 0, V), Tensor()};
         }
         Tensor d = at::empty_like(s[0]);
         check(mts_cross_entropy_bwd(ptr(s[0]), ptr_as<int64_t>(s[1]), N, V, kIgnoreIndex, dtype_code(s[0]), row, row + N, ptr_as<float>(g),
                                     row + 3 * N, ptr(d), stream_of(s[0])),
               "mts_cross_entropy_bwd");
-        return {d, Tensor(), Tensor()};
+        return {d, Tensor()};
     }
 };
 
@@ -1255,6 +1259,6 @@ PYBIND11_MODULE(_host, m) {
     m.def("cross_entropy", [](const Tensor& logits, const Tensor& targets) {
         c10::OptionalDeviceGuard guard(logits.device());
         const Tensor dense = dense16(logits);
-        return CrossEntropy::apply(dense, targets.contiguous(), logits_of_rounds(dense));
+        return CrossEntropy::apply(dense, targets.contiguous());
     });
 }

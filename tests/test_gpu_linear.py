@@ -61,7 +61,7 @@ def test_linear_in_rounds(T, N, K, pad, dtype):
 @pytest.mark.parametrize("N", [64, 67])
 @pytest.mark.parametrize("layout", ["dense", "every other column", "misaligned", "gradient of one value"])
 def test_gradients_in_other_layouts_in_rounds(layout, N):
-    """What the kernels read in place and what they do not: the same products (those of the library are rounded to 16 bits)."""
+    """What the kernels read in place and what is copied for them: the same products."""
     print(f"linear in rounds, {layout}, {N} columns", flush=True)
     g = torch.Generator().manual_seed(6)
     r = lambda *shape: torch.randn(*shape, generator=g).bfloat16().cuda()
@@ -118,7 +118,7 @@ def test_vocabulary_weight_changed_before_the_backward_pass(create_graph):
 @pytest.mark.parametrize("rows,V", [(130, 64), (200, 1003), (129, 50257)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_loss_on_a_projection(rows, V, dtype):
-    """The gradient of the logits of a projection has rows that start on 16 bytes, with the values that a leaf's has."""
+    """The gradient of the logits of a projection has the values that a leaf's has, and is dense where somebody sees it."""
     print(f"loss on a projection {rows}x{V} {dtype}", flush=True)
     g = torch.Generator().manual_seed(V)
     x, w = torch.randn(1, rows, 8, generator=g).to(dtype).cuda().requires_grad_(True), torch.randn(V, 8, generator=g).cuda().requires_grad_(True)
@@ -133,8 +133,59 @@ def test_loss_on_a_projection(rows, V, dtype):
     leaf = logits.detach().view(-1, V).requires_grad_(True)
     ops.cross_entropy(leaf, targets).backward()
     assert torch.equal(seen[0].view(-1, V), leaf.grad) and leaf.grad.is_contiguous()
-    assert seen[0].stride(1) % 8 == 0 and logits.is_contiguous()
+    assert seen[0].is_contiguous() and logits.is_contiguous()
     for got, want, tol in ((x.grad[0], leaf.grad.double() @ w.detach().to(dtype).double(), ULP[dtype]), (w.grad, leaf.grad.double().T @ x.detach()[0].double(), 1e-5)):
+        assert float((got.double() - want).abs().max()) <= tol * float(want.abs().max())
+
+
+@pytest.mark.parametrize("who", ["hook of the logits", "hook of their view", "retain_grad", "autograd.grad", "hook before the node", "hook behind the node",
+                                 "hook behind the loss", "module hook", "nobody"])
+def test_who_sees_the_gradient_of_the_logits_sees_it_dense(who):
+    """Rows of an odd vocabulary are pitched on their way from the loss to the projection only where nobody can see them; the gradients of
+    the projection are the same."""
+    print(f"gradient of the logits seen by {who}", flush=True)
+    rows, V = 256, 8193
+    g = torch.Generator().manual_seed(9)
+    x, w = torch.randn(2, rows // 2, 8, generator=g).bfloat16().cuda().requires_grad_(True), torch.randn(V, 8, generator=g).cuda().requires_grad_(True)
+    targets = torch.randint(0, V, (rows,), generator=g).cuda()
+    ops, seen = hip_backend(), []
+
+    class Head(torch.nn.Module):
+        def forward(self, x):
+            return ops.linear(x, w)
+
+    head = Head()
+    if who == "module hook":
+        head.register_full_backward_hook(lambda module, into, out: seen.append(out[0]))
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        logits = head(x)
+        flat = logits.view(-1, V)
+        loss = ops.cross_entropy(flat, targets)
+    node = logits.grad_fn
+    {"hook of the logits": lambda: logits.register_hook(seen.append), "hook of their view": lambda: flat.register_hook(seen.append), "retain_grad": logits.retain_grad,
+     "hook before the node": lambda: node.register_prehook(lambda out: seen.append(out[0])),
+     "hook behind the node": lambda: node.register_hook(lambda into, out: seen.append(out[0])),
+     "hook behind the loss": lambda: loss.grad_fn.register_hook(lambda into, out: seen.append(into[0]))}.get(who, lambda: None)()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    if who == "autograd.grad":
+        *grads, d = torch.autograd.grad(loss, (x, w, logits))
+        seen.append(d)
+    else:
+        loss.backward()
+        grads = [x.grad, w.grad]
+    if who == "retain_grad":
+        seen.append(logits.grad)
+    leaf = flat.detach().requires_grad_(True)
+    peak = torch.cuda.max_memory_allocated() - before
+    ops.cross_entropy(leaf, targets).backward()
+    assert len(seen) == (who != "nobody")
+    for d in seen:
+        assert d.is_contiguous() and torch.equal(d.view(-1), leaf.grad.view(-1))
+    # a dense gradient is copied on its way
+    assert (peak < 2 * leaf.numel() * 2) == (who == "nobody"), peak
+    for got, want, tol in ((grads[0].view(-1, 8), leaf.grad.double() @ w.detach().bfloat16().double(), ULP[torch.bfloat16]),
+                           (grads[1], leaf.grad.double().T @ x.detach().double().view(-1, 8), 1e-5)):
         assert float((got.double() - want).abs().max()) <= tol * float(want.abs().max())
 
 
