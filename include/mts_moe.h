@@ -512,7 +512,8 @@ int mts_linear_dw(const void* g, const void* x, int64_t T, int N, int K, int act
                   void* workspace, int64_t workspace_bytes, void* stream);
 /* Both gradients where they have tiles for whole rounds of the chip: dw as above, and
  * dx [T,K] = g W of act_dtype, w [N,K] the rounded weight.  Rows of g are ldg elements apart (a multiple
- * of 8, at least N; what lies between them is not used), N is any number, K a multiple of 8.
+ * of 8, at least N), N is any number, K a multiple of 8.  A row is read in pieces of eight elements: up to
+ * seven behind its N are read and not used, behind the last row as well, where g has to hold them.
  * which: 0 dx, 1 dw.                                                                        */
 int mts_linear_rounds_supported(int act_dtype, int64_t T, int N, int K, int64_t ldg);
 int64_t mts_linear_rounds_workspace_bytes(int which, int64_t T, int N, int K);

@@ -990,8 +990,11 @@ int64_t row_pitch(int64_t N) { return (N + 63) / 64 * 64; }   // 16-bit rows tha
 bool linear_in_rounds(const Tensor& x, int64_t T, int64_t N, int64_t K) {
     return T >= kLinearRoundsRows && N >= 8 * K && N < k2GiB && mts_linear_rounds_supported(dtype_code(x), T, N, K, row_pitch(N));
 }
-// rows that mts_linear_dx_rounds and mts_linear_dw_rounds read in place
-bool rows_fit(const Tensor& g) { return g.stride(1) == 1 && g.stride(0) >= g.size(1) && g.stride(0) % 8 == 0 && aligned16(g); }
+// Rows that mts_linear_dx_rounds and mts_linear_dw_rounds read in place, in whole pieces of eight elements: the storage holds the last one too.
+bool rows_fit(const Tensor& g) {
+    const int64_t end = g.storage_offset() + (g.size(0) - 1) * g.stride(0) + (g.size(1) + 7) / 8 * 8;
+    return g.stride(1) == 1 && g.stride(0) >= g.size(1) && g.stride(0) % 8 == 0 && aligned16(g) && end * g.element_size() <= (int64_t)g.storage().nbytes();
+}
 
 // A projection under autocast: the product is the library's, the gradient of its fp32 weight is summed in fp32 here.
 bool linear_supported(const Tensor& x, const Tensor& w) {
@@ -1246,6 +1249,7 @@ PYBIND11_MODULE(_host, m) {
         return std::make_tuple(v[0], v[1], v[2]);
     });
     m.def("linear_supported", &linear_supported);
+    m.def("linear_rows_fit", &rows_fit);
     m.def("linear", [](const Tensor& x, const Tensor& w) {
         c10::OptionalDeviceGuard guard(x.device());
         return Linear::apply(x, w);

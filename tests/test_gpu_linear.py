@@ -59,14 +59,15 @@ def test_linear_in_rounds(T, N, K, pad, dtype):
 
 
 @pytest.mark.parametrize("N", [64, 67])
-@pytest.mark.parametrize("layout", ["dense", "every other column", "misaligned", "gradient of one value"])
+@pytest.mark.parametrize("layout", ["dense", "every other column", "misaligned", "gradient of one value", "nothing behind the last row"])
 def test_gradients_in_other_layouts_in_rounds(layout, N):
     """What the kernels read in place and what is copied for them: the same products."""
     print(f"linear in rounds, {layout}, {N} columns", flush=True)
     g = torch.Generator().manual_seed(6)
     r = lambda *shape: torch.randn(*shape, generator=g).bfloat16().cuda()
     grad = {"dense": lambda: r(200, N), "every other column": lambda: r(200, 2 * N)[:, ::2], "misaligned": lambda: r(200, 80)[:, 1:N + 1],
-            "gradient of one value": lambda: torch.ones((), device="cuda", dtype=torch.bfloat16).expand(200, N)}[layout]()
+            "gradient of one value": lambda: torch.ones((), device="cuda", dtype=torch.bfloat16).expand(200, N),
+            "nothing behind the last row": lambda: r(199 * 72 + N).as_strided((200, N), (72, 1))}[layout]()
     x, w = r(200, 8).requires_grad_(True), torch.randn(N, 8, generator=g).cuda().requires_grad_(True)
     with torch.autocast("cuda", dtype=torch.bfloat16):
         y = hip_backend().linear(x, w)
