@@ -2628,7 +2628,7 @@ constexpr int K_COUNT = MTS_K_COUNT;
 // it leaves of the power budget shows in the kernels around it.  Gate/up on 256x256 tiles with specialised
 // waves moves a third less data from L2 to LDS per FLOP than on two co-resident 256x128 ring blocks and makes
 // the step 2-3.5 % shorter, although the kernel alone is at best as fast; dO*W2 with the SwiGLU backward in
-// its epilogue is better off with three co-resident 4-wave blocks per CU.  The forward GEMMs take their
+// its epilogue is better off with three co-resident 4-wave blocks per CU where they are one round (launch_rows_any).  The forward GEMMs take their
 // k-tiles 64 wide (two buffers instead of four stages, the same time for a tile to land): a row then contributes
 // a whole 128-byte line per load instruction, which the CU's vector cache serves at twice the rate of two
 // half lines (gate/up -2.4 %, down -1 %); so does dX, inside the joint backward launch and on its own.
@@ -2731,14 +2731,15 @@ int launch_rows_any(int kind, RowsParams p, int64_t TK, hipStream_t s, bool b_km
     if (!tile_forced(kind) && small_tiles_pay(kind, TK, p.E, p.N)) choice = 5;
     // three blocks per CU hold two stages each: for short reductions, and for the epilogue that fits beside them
     if (choice == 3 && (EPI != EPI_DY1N || !b_kmajor)) choice = 1;
-    // longer ones, and launches of more than about a round of 256 x 256 tiles, go to the specialised waves: a third less L2 traffic per product and
-    // pre-activations that land during the k loop.  The kernel, three blocks per CU / this, us (tiles): 24 576 tokens of 768/1024 150.0 / 140.6
-    // (800), 8192 of 1024/512 with 64 experts, top-4, 64.0 / 54.4 (320), 24 576 of 2048/1024 266 / 226 (WsLarge 240), 5003 of 768/1024 31.7 / 33.2
-    // (172), 6001 of 1000/1368 with even experts 61.5 / 66.0 (306), uneven ones the operator's call 553 / 533.  In the layer step, which the power limit
-    // holds, what it gains is 1 % at 20 000 and 40 000 tokens and nothing at 24 576.
+    // Longer ones, and launches that three blocks per CU cannot hold in one round however the routes are spread, go to the specialised waves: a third
+    // less L2 traffic per product and pre-activations that land during the k loop.  The kernel, three blocks per CU / this, us: 24 576 tokens of
+    // 768/1024 150 / 141, 24 576 of 2048/1024 266 / 226 (WsLarge 240), 1795 of it 43 / 36 (53).  At the border, evenly spread routes (which fit that round
+    // longest), random ones, a few experts much longer: 768/1024 9216 tokens 59 / 65, 71 / 66, 72 / 67, 9492 69 / 65, 71 / 65, 72 / 67; 512/2048 4608 52 / 54,
+    // 63 / 55, 63 / 57, 4746 58 / 57, 62 / 57, 63 / 57; 1024/512 with 64 experts, top-4, 8192 63 / 57, 65 / 71, 76 / 67, 9492 89 / 72, 83 / 72, 82 / 76;
+    // 1000/1368 5898 71 / 74, 72 / 75, 91 / 78, 6904 95 / 82, 94 / 82, 94 / 82.  Above it the worst of 90 calls is 4 % slower (256 wide) and the others at most 2 %.
     if (choice == 3 && !tile_forced(kind)) {
-        const int64_t tiles = (TK / WsWide::BM + p.E / 2) * ((p.N + WsWide::BN - 1) / WsWide::BN);
-        if (p.Kdim > 1024 || tiles >= 300) choice = 4;
+        const int64_t blocks = (TK + RingThreePerCu::BM - 1) / RingThreePerCu::BM * ((p.N + RingThreePerCu::BN - 1) / RingThreePerCu::BN);
+        if (p.Kdim > 1024 || blocks > 3 * kXcds * kCusPerXcd) choice = 4;
     }
     // the 64-wide variant exists for the GEMMs with a plain or SwiGLU epilogue
     if (choice == 4 && epi_is_dy1(EPI) && (EPI != EPI_DY1N || !b_kmajor)) choice = 2;
