@@ -85,6 +85,8 @@ def _case(seed, T, H, E, I, K, dtype, skew=0.0, empty_expert=None):
     (4096, 64, 1, 64, 1, torch.bfloat16, 0.0, True),        # one expert, one k-tile per GEMM, one column tile each
     (9000, 512, 16, 1984, 2, torch.bfloat16, 0.2, True),    # 15.5 column tiles of gate/up: the last one half empty
     (3000, 320, 130, 64, 2, torch.float16, 0.0, True),      # more experts than a wave holds: the search walks two groups
+    (16384, 128, 128, 512, 2, torch.bfloat16, 0.0, True),   # the same with two column tiles a block: whole pairs of rounds ...
+    (13000, 64, 200, 1024, 2, torch.float16, 0.1, True),    # ... and all of them
     # an expert's W1 of 8 and 6 MiB: gate/up walks its column tiles in two groups; the down part of 2048 columns would alone, here it does not
     (3000, 2048, 4, 1024, 2, torch.bfloat16, 0.3, True),
     (2100, 1024, 6, 1536, 2, torch.float16, 0.0, True),

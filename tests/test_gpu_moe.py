@@ -624,3 +624,27 @@ def test_gate_up_of_two_column_tiles_a_block(H, I, T, dtype):
     with torch.no_grad():
         alone = hip_backend().fused_moe(*(t.cuda() for t in (x, w1, w2, case[3], w)))
     assert torch.equal(alone, out)
+
+
+@pytest.mark.parametrize("H,I,T,E,dtype", [(256, 512, 16384, 128, torch.bfloat16), (64, 1024, 20000, 100, torch.float16), (1024, 256, 30000, 300, torch.bfloat16)])
+def test_pairs_and_half_tiles_of_more_experts_than_a_wave_holds(H, I, T, E, dtype):
+    """Two column tiles a gate/up block (whole pairs of rounds and all of them) and last tiles of half the height, in the forward launch, dO*W2
+    and dX, where the search for a tile takes more than one round of 64 experts."""
+    print(f"pairs and half tiles {H}/{I} T={T} E={E} {dtype}", flush=True)
+    g = torch.Generator().manual_seed(T)
+    share = torch.arange(1, E + 1, dtype=torch.float64)[torch.randperm(E, generator=g)] ** -0.5
+    counts = torch.bincount(torch.multinomial(share, T, replacement=True, generator=g), minlength=E)
+    counts[[3, 62, 63, 64, 65, 66, E - 1]] = torch.tensor([128, 0, 129, 1, 384, 385, 256])
+    T = int(counts.sum())
+    idx = torch.repeat_interleave(torch.arange(E), counts)[torch.randperm(T, generator=g)]
+    x, _, w1, w2, grad = O.make_inputs(T, T, H, E, I)
+    x, w1, w2, grad = (t.to(dtype) for t in (x, w1, w2, grad))
+    w = torch.rand(T, 1, generator=g).to(dtype)
+    case = (x, w1, w2, idx.int().unsqueeze(1), w, grad)
+    out, grads = hip_moe_grads(*case)
+    want, want_grads = oracle_moe_grads(*case, device="cuda")
+    for got, ref, what in zip((out, *grads), (want, *want_grads), ("out", "dx", "dw1", "dw2", "dweights")):
+        assert_close_scaled(got, ref, BF16_TOL, what)
+    with torch.no_grad():
+        alone = hip_backend().fused_moe(*(t.cuda() for t in (x, w1, w2, case[3], w)))
+    assert torch.equal(alone, out)
