@@ -646,7 +646,12 @@ LayerForward layer_forward(const Tensor& x_, const Tensor& w_r_, const Tensor& w
     const bool narrow = dtype != at::kFloat, limited = capacity >= 0, alone = opt.on(NO_BACKWARD), few = E <= kFewExperts;
     const int64_t ws_bytes = few ? mts_moe_head_workspace_bytes(T, K, E) : mts_moe_router_route_workspace_bytes(T, K, E);
     f.w_r = w_r;
-    f.weights = f32({T, K}, x), f.indices = i32({T, K}, x);
+    f.weights = f32({T, K}, x);
+    // The integer results in one allocation and the fp32 statistics in another: a caller may save all results together, which torch refuses
+    // for one storage under two types.
+    const int64_t counts_bytes = (E + 3) / 4 * 16;
+    const Tensor integers = i32({counts_bytes / 4 + TK}, x);
+    f.counts = part_of(integers, 0, {E}, at::kInt), f.indices = part_of(integers, counts_bytes, {T, K}, at::kInt);
     Tensor weights_act, ws, post_act, y;
     Routing r;
     // what the backward pass keeps, and what this call alone needs
@@ -667,10 +672,8 @@ LayerForward layer_forward(const Tensor& x_, const Tensor& w_r_, const Tensor& w
     if (alone) scratch.add(post_act, TK, I, dtype);
     scratch.make();
     if (!alone) kept.make();
-    // E mean probabilities, z, entropy, load-balancing term, E + 7 load statistics.  The counts are integers and have an allocation of
-    // their own: a caller may save all results together, which torch refuses for one storage under two types.
+    // E mean probabilities, z, entropy, load-balancing term, E + 7 load statistics
     Tensor stats = f32({2 * E + 10}, x);
-    f.counts = i32({E}, x);
     if (alone) {   // nobody differentiates: parts instead of views
         auto floats_at = [&](int64_t first, at::IntArrayRef size) { return part_of(stats, first * 4, size, at::kFloat); };
         f.prob_mean = floats_at(0, {E}), f.z_loss = floats_at(E, {}), f.entropy = floats_at(E + 1, {}), f.load_balance = floats_at(E + 2, {});
