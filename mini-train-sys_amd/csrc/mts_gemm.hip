@@ -2736,10 +2736,13 @@ int launch_rows_any(int kind, RowsParams p, int64_t TK, hipStream_t s, bool b_km
     // 768/1024 150 / 141, 24 576 of 2048/1024 266 / 226 (WsLarge 240), 1795 of it 43 / 36 (53).  At the border, evenly spread routes (which fit that round
     // longest), random ones, a few experts much longer: 768/1024 9216 tokens 59 / 65, 71 / 66, 72 / 67, 9492 69 / 65, 71 / 65, 72 / 67; 512/2048 4608 52 / 54,
     // 63 / 55, 63 / 57, 4746 58 / 57, 62 / 57, 63 / 57; 1024/512 with 64 experts, top-4, 8192 63 / 57, 65 / 71, 76 / 67, 9492 89 / 72, 83 / 72, 82 / 76;
-    // 1000/1368 5898 71 / 74, 72 / 75, 91 / 78, 6904 95 / 82, 94 / 82, 94 / 82.  Above it the worst of 90 calls is 4 % slower (256 wide) and the others at most 2 %.
+    // 1000/1368 5898 71 / 74, 72 / 75, 91 / 78, 6904 95 / 82, 94 / 82, 94 / 82.  Widths whose last 256 columns are half empty stay where that adds more than an
+    // eighth to the columns (128 columns of 768 above the border 1.01 to 1.18 times as long, 384 0.97 to 1.13, 640 of 256 to 1024 0.91 to 1.07, 896
+    // 0.90 to 1.11; 1152 0.87 to 1.01).  Of 300 calls above the border some of 2432 columns are 3 to 7 % slower, some of 256 of k 3 %, the others at most 2 %.
     if (choice == 3 && !tile_forced(kind)) {
-        const int64_t blocks = (TK + RingThreePerCu::BM - 1) / RingThreePerCu::BM * ((p.N + RingThreePerCu::BN - 1) / RingThreePerCu::BN);
-        if (p.Kdim > 1024 || blocks > 3 * kXcds * kCusPerXcd) choice = 4;
+        const int64_t narrow = (p.N + RingThreePerCu::BN - 1) / RingThreePerCu::BN, wide = (p.N + WsWide::BN - 1) / WsWide::BN * (WsWide::BN / RingThreePerCu::BN);
+        const int64_t blocks = (TK + RingThreePerCu::BM - 1) / RingThreePerCu::BM * narrow;
+        if (p.Kdim > 1024 || (blocks > 3 * kXcds * kCusPerXcd && 8 * wide <= 9 * narrow)) choice = 4;
     }
     // the 64-wide variant exists for the GEMMs with a plain or SwiGLU epilogue
     if (choice == 4 && epi_is_dy1(EPI) && (EPI != EPI_DY1N || !b_kmajor)) choice = 2;
