@@ -541,6 +541,37 @@ int mts_attention_bwd(const MtsHeads* q, const MtsHeads* k, const MtsHeads* v, c
                       int causal, int act_dtype, const MtsHeads* dq, const MtsHeads* dk,
                       const MtsHeads* dv, float* delta, void* stream);
 
+/* ---- optimizer update (minitrain/train/trainer.py:85-159, minitrain/train/optim.py:30-47) ----
+ * All tables are host arrays; the kernels take tensors of any size and alignment.
+ *
+ * mts_grad_norm: result[0] = 2-norm of all gradients together, result[1] = min(1, max_norm / (norm + 1e-6))
+ * (1 without gradients), result[2] = 1 where the norm or *loss (may be NULL) is not finite, else 0.      */
+typedef struct {
+    const float* data;
+    int64_t n;
+} MtsGradSpan;
+int64_t mts_grad_norm_workspace_bytes(const MtsGradSpan* grads, int count);
+int mts_grad_norm(const MtsGradSpan* grads, int count, float max_norm, const float* loss,
+                  float* result, void* workspace, int64_t workspace_bytes, void* stream);
+
+/* AdamW: step += 1, then the moments and the parameter, with gradients multiplied by *clip (NULL: 1).
+ * Nothing is written where *skip (may be NULL) is not zero.  keep_grad: the gradient as it was used is
+ * written back.                                                                              */
+#define MTS_ADAM_GROUPS 4
+typedef struct {
+    double lr, beta1, beta2, eps, weight_decay;
+} MtsAdamGroup;
+typedef struct {
+    float *param, *grad, *exp_avg, *exp_avg_sq;
+    float* step;   /* one value */
+    int64_t n;
+    int group, keep_grad;
+} MtsAdamTensor;
+int64_t mts_adamw_workspace_bytes(int count);
+int mts_adamw(const MtsAdamTensor* tensors, int count, const MtsAdamGroup* groups, int n_groups,
+              const float* clip, const float* skip, void* workspace, int64_t workspace_bytes,
+              void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1193,6 +1193,62 @@ struct CrossEntropy : torch::autograd::Function<CrossEntropy> {
     }
 };
 
+// ---- optimizer update ------------------------------------------------------------------------------------------------------------
+
+// Whether one update may be taken by the kernels: fp32 parameters, dense gradients and moments on one GPU, a step count on it for each.
+bool adamw_supported(const std::vector<Tensor>& params, const std::vector<Tensor>& exp_avgs, const std::vector<Tensor>& exp_avg_sqs,
+                     const std::vector<Tensor>& steps) {
+    if (params.empty() || exp_avgs.size() != params.size() || exp_avg_sqs.size() != params.size() || steps.size() != params.size() ||
+        params.size() >= (1u << 20) || !nobody_dispatches())
+        return false;
+    auto fits = [&](const Tensor& t, const Tensor& p) {
+        return t.defined() && is_plain(t) && t.layout() == at::kStrided && t.scalar_type() == at::kFloat && t.device() == params[0].device() &&
+               t.is_contiguous() && t.sizes() == p.sizes();
+    };
+    for (size_t i = 0; i < params.size(); ++i) {
+        const Tensor &p = params[i], &step = steps[i];
+        if (!p.is_cuda() || !fits(p, p) || !fits(p.grad(), p) || !fits(exp_avgs[i], p) || !fits(exp_avg_sqs[i], p) || p.numel() >= (1LL << 30)) return false;
+        if (!is_plain(step) || step.layout() != at::kStrided || step.device() != p.device() || step.scalar_type() != at::kFloat || step.numel() != 1) return false;
+    }
+    return true;
+}
+
+// norm of the gradients, clipping coefficient, and whether norm or loss are not finite; max_norm < 0: the gradients stay out of it
+Tensor grad_norm(const std::vector<Tensor>& params, double max_norm, const Tensor& loss) {
+    std::vector<MtsGradSpan> spans;
+    if (max_norm >= 0)
+        for (const Tensor& p : params) spans.push_back({ptr_as<float>(p.grad()), p.numel()});
+    Tensor result = f32({3}, params[0]);
+    const int64_t ws_bytes = mts_grad_norm_workspace_bytes(spans.data(), (int)spans.size());
+    Tensor ws = bytes(ws_bytes, params[0]);
+    check(mts_grad_norm(spans.data(), (int)spans.size(), (float)max_norm, ptr_as<float>(loss), ptr_as<float>(result), ptr(ws), ws.numel(), stream_of(params[0])),
+          "mts_grad_norm");
+    return result;
+}
+
+// groups: of each tensor; settings: lr, beta1, beta2, eps and weight decay of each group; scale: what grad_norm returned
+void adamw(const std::vector<Tensor>& params, const std::vector<Tensor>& exp_avgs, const std::vector<Tensor>& exp_avg_sqs, const std::vector<Tensor>& steps,
+           const std::vector<int64_t>& groups, const std::vector<std::array<double, 5>>& settings, const Tensor& scale, bool skip_if_not_finite) {
+    std::vector<MtsAdamTensor> tensors;
+    for (size_t i = 0; i < params.size(); ++i) {
+        const Tensor& g = params[i].grad();
+        // a gradient that somebody else holds is left clipped, as stock clipping leaves it
+        const bool held = g.use_count() > 1 || g.storage().use_count() > 1;
+        tensors.push_back({ptr_as<float>(params[i]), ptr_as<float>(g), ptr_as<float>(exp_avgs[i]), ptr_as<float>(exp_avg_sqs[i]), ptr_as<float>(steps[i]),
+                           params[i].numel(), (int)groups[i], held});
+    }
+    std::vector<MtsAdamGroup> of;
+    for (const auto& s : settings) of.push_back({s[0], s[1], s[2], s[3], s[4]});
+    Tensor ws = bytes(mts_adamw_workspace_bytes((int)tensors.size()), params[0]);
+    const float* result = ptr_as<float>(scale);
+    check(mts_adamw(tensors.data(), (int)tensors.size(), of.data(), (int)of.size(), result + 1, skip_if_not_finite ? result + 2 : nullptr, ptr(ws), ws.numel(),
+                    stream_of(params[0])),
+          "mts_adamw");
+    for (const auto* written : {&params, &exp_avgs, &exp_avg_sqs, &steps})
+        for (const Tensor& t : *written)
+            if (!t.is_inference()) t.unsafeGetTensorImpl()->bump_version();
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_host, m) {
@@ -1261,6 +1317,18 @@ PYBIND11_MODULE(_host, m) {
     m.def("attention", [](const Tensor& q, const Tensor& k, const Tensor& v, bool causal) {
         c10::OptionalDeviceGuard guard(q.device());
         return Attention::apply(q, k, v, causal);
+    });
+    m.attr("ADAM_GROUPS") = MTS_ADAM_GROUPS;
+    m.def("adamw_supported", &adamw_supported);
+    m.def("grad_norm", [](const std::vector<Tensor>& params, double max_norm, const Tensor& loss) {
+        c10::OptionalDeviceGuard guard(params.at(0).device());
+        return grad_norm(params, max_norm, loss);
+    });
+    m.def("adamw", [](const std::vector<Tensor>& params, const std::vector<Tensor>& exp_avgs, const std::vector<Tensor>& exp_avg_sqs,
+                      const std::vector<Tensor>& steps, const std::vector<int64_t>& groups, const std::vector<std::array<double, 5>>& settings, const Tensor& scale,
+                      bool skip_if_not_finite) {
+        c10::OptionalDeviceGuard guard(params.at(0).device());
+        adamw(params, exp_avgs, exp_avg_sqs, steps, groups, settings, scale, skip_if_not_finite);
     });
     m.def("cross_entropy_supported", &cross_entropy_supported);
     m.def("cross_entropy", [](const Tensor& logits, const Tensor& targets) {

@@ -8,6 +8,8 @@ import contextlib
 
 import torch
 
+from minitrain_amd.train.update import plan
+
 
 def build_optimizer(model: torch.nn.Module, *, lr: float = 3e-4, weight_decay: float = 0.1, betas=(0.9, 0.95),
                     eps: float = 1e-8) -> torch.optim.Optimizer:
@@ -23,8 +25,8 @@ def train_step(model: torch.nn.Module, optimizer: torch.optim.Optimizer, batch: 
                use_fused_loss: bool = False, check_finite: bool = True) -> torch.Tensor:
     """Forward, backward, clipping and the optimizer update, exactly once; returns the loss.
 
-    A non-finite loss or gradient norm raises ``FloatingPointError`` from the host before the optimizer
-    runs (the conditions the reference tests, minitrain/train/trainer.py:77-78,101-106).  The test is one flag
+    A non-finite loss or gradient norm raises ``FloatingPointError`` from the host, and parameters and optimizer state stay
+    as they were (the conditions the reference tests, minitrain/train/trainer.py:77-78,101-106).  The test is one flag
     computed on the device and read once per step; nothing on the device asserts or traps.
     ``check_finite=False`` skips the read (and its synchronisation) for callers that check at their own
     interval."""
@@ -39,8 +41,24 @@ def train_step(model: torch.nn.Module, optimizer: torch.optim.Optimizer, batch: 
     )
     with ctx:
         loss, _ = model(input_ids, targets=targets, use_fused_loss=use_fused_loss)
-    finite = torch.isfinite(loss.detach())
     loss.backward()
+    update = plan(model, optimizer, loss.detach(), grad_clip_norm)
+    if update is not None:
+        # The update is enqueued before the flag is read and looks at it by itself: the next step's first launches then come
+        # while it runs, where a read in front of it leaves the GPU without work until they arrive.
+        norm = update.norm(grad_clip_norm, loss.detach())
+        if check_finite:
+            flag = torch.empty((), dtype=torch.float32, pin_memory=True).copy_(norm[2], non_blocking=True)
+            copied = torch.cuda.Event()
+            copied.record()
+        update.apply(norm, skip_if_not_finite=check_finite)
+        if check_finite:
+            copied.synchronize()
+        optimizer.zero_grad(set_to_none=True)
+        if check_finite and float(flag) != 0:
+            raise FloatingPointError("non-finite training loss or global gradient norm")
+        return loss.detach()
+    finite = torch.isfinite(loss.detach())
     if grad_clip_norm is not None:
         norm = torch.nn.utils.clip_grad_norm_(model.parameters(), grad_clip_norm)
         finite = finite & torch.isfinite(norm)
