@@ -522,6 +522,18 @@ int mts_linear_dw_rounds(const void* g, int64_t ldg, const void* x, int64_t T, i
 int mts_linear_dx_rounds(const void* g, int64_t ldg, const void* w, int64_t T, int N, int K, int act_dtype,
                          void* dx, void* workspace, int64_t workspace_bytes, void* stream);
 
+/* Means over the layers of a model: out[g][i] = mean over l of src[first[g] + l][i], l < first[g+1] - first[g], i < n[g], summed in
+ * that order.  src: pointers to f32, or int64 where whole[g] != 0.  All tables are host arrays.     */
+#define MTS_MEAN_GROUPS 16
+#define MTS_MEAN_TENSORS 384
+int mts_layer_means(const void* const* src, const int* first, const int* n, const int* whole,
+                    int groups, float* const* out, void* stream);
+
+/* Up to four sums of up to four numbers: out[j] = (sum of weight[4*j + i] * in[i] over the i whose bit is set in terms[j]) /
+ * divisor[j], the products rounded and added in that order.  Host arrays; in and out hold device pointers.  */
+int mts_scalar_sums(const float* const* in, int inputs, const float* weight, const int* terms,
+                    const float* divisor, float* const* out, int outputs, void* stream);
+
 /* Scaled dot-product attention of heads of 64 elements, bf16 or fp16, queries and keys of the
  * same length; causal != 0: query i sees keys 0..i.  Tensors are [B,heads,S,64], dense in the last
  * dimension, 16-byte aligned, other strides multiples of 8 elements.  fp32 scores, sums and

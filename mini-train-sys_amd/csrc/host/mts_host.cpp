@@ -1193,6 +1193,125 @@ struct CrossEntropy : torch::autograd::Function<CrossEntropy> {
     }
 };
 
+// ---- numbers of a model's layers -----------------------------------------------------------------------------------------------
+
+typedef std::vector<std::vector<Tensor>> Groups;   // tensors of one quantity, one a layer
+
+// `differentiable` groups come first; the others carry no gradient
+bool layer_means_supported(const Groups& groups, int64_t differentiable) {
+    if (groups.empty() || groups.size() > MTS_MEAN_GROUPS || groups[0].empty() || !nobody_dispatches() || at::impl::torch_function_mode_enabled()) return false;
+    size_t tensors = 0;
+    const at::Device device = groups[0][0].device();
+    for (size_t g = 0; g < groups.size(); ++g) {
+        if (groups[g].empty()) return false;
+        const Tensor& first = groups[g][0];
+        const bool tracked = (int64_t)g < differentiable;
+        if (tracked ? first.dim() != 0 : first.dim() > 1) return false;
+        if (first.numel() < 1 || !(first.scalar_type() == at::kFloat || (first.scalar_type() == at::kLong && first.dim() == 0 && !tracked))) return false;
+        for (const Tensor& t : groups[g])
+            if (!is_plain(t) || !t.is_cuda() || t.device() != device || t.scalar_type() != first.scalar_type() || t.sizes() != first.sizes() || !t.is_contiguous() ||
+                (!tracked && t.requires_grad()))
+                return false;
+        tensors += groups[g].size();
+    }
+    return tensors <= MTS_MEAN_TENSORS;
+}
+
+void scalar_sums(std::initializer_list<Tensor> in, const float (&weight)[4][4], const int (&terms)[4], const float (&divisor)[4],
+                 std::initializer_list<Tensor> out) {
+    const float* sources[4] = {};
+    float* results[4] = {};
+    int inputs = 0, outputs = 0;
+    for (const Tensor& t : in) sources[inputs++] = ptr_as<float>(t);
+    for (const Tensor& t : out) results[outputs++] = ptr_as<float>(t);
+    check(mts_scalar_sums(sources, inputs, &weight[0][0], terms, divisor, results, outputs, stream_of(*out.begin())), "mts_scalar_sums");
+}
+
+// The mean of every group, fp32.  `tracked`: the tensors of the differentiable groups, for autograd.
+struct LayerMeans : torch::autograd::Function<LayerMeans> {
+    static variable_list means(const Groups& groups, int64_t differentiable) {
+        const void* src[MTS_MEAN_TENSORS];
+        int first[MTS_MEAN_GROUPS + 1] = {}, n[MTS_MEAN_GROUPS], whole[MTS_MEAN_GROUPS];
+        float* out[MTS_MEAN_GROUPS];
+        int64_t total = 0;
+        for (size_t g = differentiable; g < groups.size(); ++g) total += groups[g][0].numel();
+        const Tensor& like = groups[0][0];
+        const Tensor records = f32({std::max<int64_t>(total, 1)}, like);
+        variable_list result;
+        int64_t at_element = 0;
+        for (size_t g = 0; g < groups.size(); ++g) {
+            const Tensor& t = groups[g][0];
+            if ((int64_t)g < differentiable) result.push_back(f32({}, like));
+            else {
+                result.push_back(part_of(records, at_element * 4, t.sizes(), at::kFloat));
+                at_element += t.numel();
+            }
+            first[g + 1] = first[g] + (int)groups[g].size(), n[g] = (int)t.numel(), whole[g] = t.scalar_type() == at::kLong, out[g] = ptr_as<float>(result.back());
+            for (size_t l = 0; l < groups[g].size(); ++l) src[first[g] + l] = ptr(groups[g][l]);
+        }
+        check(mts_layer_means(src, first, n, whole, (int)groups.size(), out, stream_of(like)), "mts_layer_means");
+        return result;
+    }
+    static variable_list forward(AutogradContext* ctx, at::TensorList tracked, const Groups& groups, int64_t differentiable) {
+        variable_list result = means(groups, differentiable);
+        std::vector<int64_t> counts;
+        for (int64_t g = 0; g < differentiable; ++g) counts.push_back((int64_t)groups[g].size());
+        ctx->saved_data["counts"] = counts;
+        ctx->mark_non_differentiable(variable_list(result.begin() + differentiable, result.end()));
+        ctx->set_materialize_grads(false);
+        return result;
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        const auto counts = ctx->saved_data["counts"].toIntVector();
+        const bool stock = written_out(grads);
+        variable_list result;
+        Tensor share[2];
+        if (!stock && counts.size() == 2 && grads[0].defined() && grads[1].defined()) {
+            c10::OptionalDeviceGuard guard(grads[0].device());
+            for (Tensor& t : share) t = f32({}, grads[0]);
+            const Tensor a = grads[0].to(at::kFloat), b = grads[1].to(at::kFloat);
+            scalar_sums({a, b}, {{1.f, 0.f}, {0.f, 1.f}}, {1, 2}, {(float)counts[0], (float)counts[1]}, {share[0], share[1]});
+        }
+        for (size_t g = 0; g < counts.size(); ++g) {
+            const Tensor one = !grads[g].defined() ? Tensor() : g < 2 && share[g].defined() ? share[g] : grads[g] / (double)counts[g];
+            result.insert(result.end(), (size_t)counts[g], one);
+        }
+        result.resize(result.size() + 2);
+        return result;
+    }
+};
+
+bool total_loss_supported(const Tensor& loss, const Tensor& aux, const Tensor& z) {
+    auto number = [](const Tensor& t) { return t.dim() == 0 && t.scalar_type() == at::kFloat; };
+    return all_plain(loss, aux, z) && on_one_gpu(loss, aux, z) && number(loss) && number(aux) && number(z);
+}
+
+// loss + a * aux + b * z; and without a gradient a * aux, b * z and the sum of the two
+struct TotalLoss : torch::autograd::Function<TotalLoss> {
+    static variable_list forward(AutogradContext* ctx, const Tensor& loss, const Tensor& aux, const Tensor& z, double a, double b) {
+        Tensor total = f32({}, loss), parts = f32({3}, loss);
+        auto part = [&](int i) { return part_of(parts, i * 4, {}, at::kFloat); };
+        const variable_list out{total, part(0), part(1), part(2)};
+        const float fa = (float)a, fb = (float)b;
+        scalar_sums({loss, aux, z}, {{1.f, fa, fb}, {0.f, fa, 0.f}, {0.f, 0.f, fb}, {0.f, fa, fb}}, {7, 2, 4, 6}, {1.f, 1.f, 1.f, 1.f}, {out[0], out[1], out[2], out[3]});
+        ctx->saved_data["a"] = a;
+        ctx->saved_data["b"] = b;
+        ctx->mark_non_differentiable({out[1], out[2], out[3]});
+        ctx->set_materialize_grads(false);
+        return out;
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        const Tensor& g = grads[0];
+        const double a = ctx->saved_data["a"].toDouble(), b = ctx->saved_data["b"].toDouble();
+        if (!g.defined()) return variable_list(5);
+        if (written_out(grads) || g.scalar_type() != at::kFloat) return {g, g * a, g * b, Tensor(), Tensor()};
+        c10::OptionalDeviceGuard guard(g.device());
+        Tensor d_aux = f32({}, g), d_z = f32({}, g);
+        scalar_sums({g}, {{(float)a}, {(float)b}}, {1, 1}, {1.f, 1.f}, {d_aux, d_z});
+        return {g, d_aux, d_z, Tensor(), Tensor()};
+    }
+};
+
 // ---- optimizer update ------------------------------------------------------------------------------------------------------------
 
 // Whether one update may be taken by the kernels: fp32 parameters, dense gradients and moments on one GPU, a step count on it for each.
@@ -1317,6 +1436,25 @@ PYBIND11_MODULE(_host, m) {
     m.def("attention", [](const Tensor& q, const Tensor& k, const Tensor& v, bool causal) {
         c10::OptionalDeviceGuard guard(q.device());
         return Attention::apply(q, k, v, causal);
+    });
+    m.def("layer_means_supported", &layer_means_supported);
+    m.def("layer_means", [](const Groups& groups, int64_t differentiable) {
+        c10::OptionalDeviceGuard guard(groups.at(0).at(0).device());
+        variable_list tracked;
+        bool wanted = false;
+        for (int64_t g = 0; g < differentiable; ++g)
+            for (const Tensor& t : groups.at(g)) {
+                tracked.push_back(t);
+                wanted |= t.requires_grad();
+            }
+        if (!wanted || !at::GradMode::is_enabled()) return LayerMeans::means(groups, differentiable);
+        return LayerMeans::apply(at::TensorList(tracked), groups, differentiable);
+    });
+    m.def("total_loss_supported", &total_loss_supported);
+    m.def("total_loss", [](const Tensor& loss, const Tensor& aux, const Tensor& z, double a, double b) {
+        c10::OptionalDeviceGuard guard(loss.device());
+        const variable_list v = TotalLoss::apply(loss, aux, z, a, b);
+        return std::make_tuple(v[0], v[1], v[2], v[3]);
     });
     m.attr("ADAM_GROUPS") = MTS_ADAM_GROUPS;
     m.def("adamw_supported", &adamw_supported);

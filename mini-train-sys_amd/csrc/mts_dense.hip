@@ -516,6 +516,49 @@ __global__ __launch_bounds__(kCeThreads) void cross_entropy_bwd_kernel(const ET*
 
 bool dense_dtype_ok(int dtype) { return dtype == MTS_BF16 || dtype == MTS_F32 || dtype == MTS_F16; }
 
+// ---------------------------------------------------------------------------
+// Numbers of a model's layers: the means of its routers' losses and monitoring records, and the loss as their sum.  A launch
+// each where stock operators take two a quantity (12 layers: 29 launches of 2 to 5 us; a pass of 640 tokens through two layers is
+// bound by the host that makes them).
+// ---------------------------------------------------------------------------
+
+struct MeanTable {
+    const void* src[MTS_MEAN_TENSORS];
+    float* out[MTS_MEAN_GROUPS];
+    int n[MTS_MEAN_GROUPS];
+    uint16_t first[MTS_MEAN_GROUPS + 1];
+    uint8_t whole[MTS_MEAN_GROUPS];
+};
+static_assert(sizeof(MeanTable) <= 4096, "kernel arguments");
+
+constexpr int kMeanThreads = 64;
+template <typename T>
+__device__ __forceinline__ float mean_at(const void* const* src, int count, int i) {
+    float sum = 0.f;
+    for (int l = 0; l < count; ++l) sum += (float)static_cast<const T*>(src[l])[i];
+    return sum / (float)count;
+}
+__global__ __launch_bounds__(kMeanThreads) void layer_means_kernel(MeanTable t) {
+    const int g = blockIdx.x, first = t.first[g], count = t.first[g + 1] - first;
+    for (int i = threadIdx.x; i < t.n[g]; i += kMeanThreads)
+        t.out[g][i] = t.whole[g] ? mean_at<int64_t>(t.src + first, count, i) : mean_at<float>(t.src + first, count, i);
+}
+
+struct ScalarSums {
+    const float* in[4];
+    float* out[4];
+    float weight[4][4], divisor[4];
+    int inputs, terms[4];
+};
+__global__ void scalar_sums_kernel(ScalarSums p) {
+#pragma clang fp contract(off)
+    const int j = threadIdx.x;
+    float sum = 0.f;
+    for (int i = 0; i < p.inputs; ++i)
+        if (p.terms[j] >> i & 1) sum += p.weight[j][i] * *p.in[i];
+    *p.out[j] = sum / p.divisor[j];
+}
+
 }  // namespace
 
 extern "C" int mts_rmsnorm_supported(int H) { return H > 0 && H % 4 == 0 && norm_groups(H) > 0; }
@@ -622,4 +665,40 @@ extern "C" int mts_cross_entropy_bwd(const void* logits, const int64_t* targets,
 extern "C" int mts_cross_entropy_bwd_pitched(const void* logits, const int64_t* targets, int64_t N, int V, int64_t ignore_index, int dtype, const float* row_max,
                                              const float* row_log_sum, const float* g_loss, const float* inv_count, void* d_logits, int64_t pitch, void* stream) {
     return cross_entropy_bwd<true>(logits, targets, N, V, ignore_index, dtype, row_max, row_log_sum, g_loss, inv_count, d_logits, pitch, stream);
+}
+
+extern "C" int mts_layer_means(const void* const* src, const int* first, const int* n, const int* whole, int groups, float* const* out, void* stream) {
+    if (!src || !first || !n || !whole || !out) return MTS_ERR_NULL;
+    if (groups < 1 || groups > MTS_MEAN_GROUPS || first[0] != 0 || first[groups] > MTS_MEAN_TENSORS) return MTS_ERR_SHAPE;
+    MeanTable t = {};
+    for (int g = 0; g < groups; ++g) {
+        if (first[g + 1] <= first[g] || n[g] < 1) return MTS_ERR_SHAPE;
+        if (!out[g]) return MTS_ERR_NULL;
+        t.out[g] = out[g], t.n[g] = n[g], t.whole[g] = whole[g] != 0, t.first[g + 1] = (uint16_t)first[g + 1];
+    }
+    for (int i = 0; i < first[groups]; ++i) {
+        if (!src[i]) return MTS_ERR_NULL;
+        t.src[i] = src[i];
+    }
+    layer_means_kernel<<<dim3((unsigned)groups), kMeanThreads, 0, (hipStream_t)stream>>>(t);
+    MTS_CHECK_LAUNCH();
+    return MTS_OK;
+}
+
+extern "C" int mts_scalar_sums(const float* const* in, int inputs, const float* weight, const int* terms, const float* divisor, float* const* out, int outputs,
+                               void* stream) {
+    if (!in || !weight || !terms || !divisor || !out) return MTS_ERR_NULL;
+    if (inputs < 1 || inputs > 4 || outputs < 1 || outputs > 4) return MTS_ERR_SHAPE;
+    ScalarSums p = {};
+    p.inputs = inputs;
+    for (int i = 0; i < inputs; ++i)
+        if (!(p.in[i] = in[i])) return MTS_ERR_NULL;
+    for (int j = 0; j < outputs; ++j) {
+        if (!(p.out[j] = out[j])) return MTS_ERR_NULL;
+        p.divisor[j] = divisor[j], p.terms[j] = terms[j];
+        for (int i = 0; i < 4; ++i) p.weight[j][i] = weight[4 * j + i];
+    }
+    scalar_sums_kernel<<<1, outputs, 0, (hipStream_t)stream>>>(p);
+    MTS_CHECK_LAUNCH();
+    return MTS_OK;
 }

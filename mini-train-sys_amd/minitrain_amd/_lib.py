@@ -100,6 +100,8 @@ SIGNATURES = {
     "mts_attention_fwd": (_i, [_p, _p, _p, _l, _i, _l, _i, _i, _p, _p, _p]),
     "mts_attention_bwd": (_i, [_p, _p, _p, _p, _p, _p, _l, _i, _l, _i, _i, _p, _p, _p, _p, _p]),
     "mts_cross_entropy_bwd": (_i, [_p, _p, _l, _i, _l, _i, _p, _p, _p, _p, _p, _p]),
+    "mts_layer_means": (_i, [_p, _p, _p, _p, _i, _p, _p]),
+    "mts_scalar_sums": (_i, [_p, _i, _p, _p, _p, _p, _i, _p]),
     "mts_grad_norm_workspace_bytes": (_l, [_p, _i]),
     "mts_grad_norm": (_i, [_p, _i, _c.c_float, _p, _p, _p, _l, _p]),
     "mts_adamw_workspace_bytes": (_l, [_i]),

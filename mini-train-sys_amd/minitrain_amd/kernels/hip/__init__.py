@@ -91,6 +91,20 @@ class HipOpsBackend(DenseTorchOps):
         logits = self.linear(x, weight)
         return self.cross_entropy(F.linear(x, weight) if logits is None else logits, targets)
 
+    def layer_means(self, groups, differentiable):
+        """Extension: the mean over the layers of every group of tensors in one launch (the first ``differentiable`` groups
+        are single numbers that carry gradients), or None when the kernel does not take them."""
+        if not dense.is_layer_means_supported(groups, differentiable):
+            return None
+        return dense.layer_means(groups, differentiable)
+
+    def total_loss(self, loss, aux, z, aux_coef, z_coef):
+        """Extension: ``(loss + aux_coef * aux + z_coef * z, aux_coef * aux, z_coef * z, their sum)``, the last three without
+        gradients, or None when the kernel does not take them."""
+        if not dense.is_total_loss_supported(loss, aux, z):
+            return None
+        return dense.total_loss(loss, aux, z, aux_coef, z_coef)
+
     def expert_counts(self, expert_indices, num_experts):
         """Extension: routes per expert (int32 ``[E]``) without a host synchronisation."""
         return expert_counts(expert_indices, num_experts)

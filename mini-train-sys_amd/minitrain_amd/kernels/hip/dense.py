@@ -74,3 +74,22 @@ def is_cross_entropy_supported(logits, targets) -> bool:
 def cross_entropy(logits, targets):
     """``F.cross_entropy(logits.float(), targets)`` without the fp32 copy of the logits"""
     return _lib.host().cross_entropy(logits, targets)
+
+
+def is_layer_means_supported(groups, differentiable: int) -> bool:
+    flat = [t for group in groups for t in group]
+    return all(isinstance(t, torch.Tensor) for t in flat) and _may_replace(*flat) and _lib.host().layer_means_supported(groups, differentiable)
+
+
+def layer_means(groups, differentiable: int):
+    """``torch.stack(group).float().mean(0)`` of every group of tensors; gradients go to the first ``differentiable`` ones"""
+    return _lib.host().layer_means(groups, differentiable)
+
+
+def is_total_loss_supported(loss, aux, z) -> bool:
+    return _may_replace(loss, aux, z) and _lib.host().total_loss_supported(loss, aux, z)
+
+
+def total_loss(loss, aux, z, aux_coef: float, z_coef: float):
+    """``loss + aux_coef * aux + z_coef * z``, and without gradients its two last terms and their sum"""
+    return _lib.host().total_loss(loss, aux, z, aux_coef, z_coef)

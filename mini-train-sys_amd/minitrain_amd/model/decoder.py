@@ -66,6 +66,28 @@ def project(linear: nn.Linear, x: torch.Tensor, ops: OpsBackend) -> torch.Tensor
     return linear(x) if y is None else y
 
 
+def layer_means(losses: list, records: list, ops: OpsBackend) -> list:
+    """The means over the layers of the losses and of the records (numbers, or one per expert), in one launch where the
+    backend offers it."""
+    fused = getattr(ops, "layer_means", None)
+    means = fused([*losses, *records], len(losses)) if fused is not None else None
+    if means is None:
+        stacked = [torch.stack(values) for values in records]
+        means = [torch.stack(values).mean() for values in losses]
+        means += [s.float().mean() if s.ndim == 1 else s.detach().mean(dim=0) for s in stacked]
+    return means
+
+
+def total_loss(loss, aux, z, aux_coef: float, z_coef: float, ops: OpsBackend):
+    """``loss`` with the weighted losses of the routers, those two and their sum."""
+    fused = getattr(ops, "total_loss", None)
+    sums = fused(loss, aux, z, aux_coef, z_coef) if fused is not None else None
+    if sums is None:
+        weighted_aux, weighted_z = aux_coef * aux, z_coef * z
+        sums = loss + weighted_aux + weighted_z, weighted_aux, weighted_z, weighted_aux + weighted_z
+    return sums
+
+
 class CausalSelfAttention(nn.Module):
     def __init__(self, cfg: ModelConfig) -> None:
         super().__init__()
@@ -154,15 +176,13 @@ class MiniTransformer(nn.Module):
             for name, value in ffn.router_metrics.items():
                 per_layer.setdefault(name, []).append(value)
         metrics = {}
-        for name, values in per_layer.items():
-            stacked = torch.stack(values)
-            if stacked.ndim == 1:
-                metrics[name] = stacked.float().mean()
+        self._router_aux, self._router_z, *means = layer_means([aux, z], list(per_layer.values()), self.ops)
+        for name, mean in zip(per_layer, means):
+            if mean.ndim == 0:
+                metrics[name] = mean
             else:   # per-expert vectors: one entry per expert, averaged over layers
-                for i, v in enumerate(stacked.detach().mean(dim=0)):
+                for i, v in enumerate(mean.unbind()):
                     metrics[f"{name}/expert_{i:02d}"] = v
-        self._router_aux = torch.stack(aux).mean()
-        self._router_z = torch.stack(z).mean()
         metrics["moe/aux_loss"] = self._router_aux.detach()
         metrics["moe/z_loss"] = self._router_z.detach()
         self.last_training_metrics = metrics
@@ -180,13 +200,13 @@ class MiniTransformer(nn.Module):
         else:
             output = project(self.lm_head, hidden, self.ops)
             lm_loss = self.ops.cross_entropy(output.reshape(-1, output.size(-1)), targets.reshape(-1))
-        weighted_aux = self.cfg.router_aux_loss_coef * self._router_aux
-        weighted_z = self.cfg.router_z_loss_coef * self._router_z
-        loss = lm_loss + weighted_aux + weighted_z
+        loss, weighted_aux, weighted_z, regularization = total_loss(
+            lm_loss, self._router_aux, self._router_z, self.cfg.router_aux_loss_coef, self.cfg.router_z_loss_coef, self.ops
+        )
         m = self.last_training_metrics
         m["loss/lm_cross_entropy"] = lm_loss.detach()
         m["loss/moe_aux_weighted"] = weighted_aux.detach()
         m["loss/moe_z_weighted"] = weighted_z.detach()
-        m["loss/moe_regularization_total"] = (weighted_aux + weighted_z).detach()
+        m["loss/moe_regularization_total"] = regularization.detach()
         m["loss/total"] = loss.detach()
         return loss, output
