@@ -503,6 +503,13 @@ int mts_cross_entropy_bwd_pitched(const void* logits, const int64_t* targets, in
                                   const float* row_log_sum, const float* g_loss, const float* inv_count,
                                   void* d_logits, int64_t pitch, void* stream);
 
+/* Gradient of an embedding table: dw [V,H] f32, row r the sum of the rows of g [T,H] (act_dtype) whose id is r, in ascending order.
+ * H a multiple of 4 up to 4096, T up to 2^18, V up to 2^20 (mts_embedding_bwd_supported).            */
+int mts_embedding_bwd_supported(int64_t T, int64_t V, int64_t H);
+int64_t mts_embedding_bwd_workspace_bytes(int64_t T, int64_t V);
+int mts_embedding_bwd(const void* g, const int64_t* ids, int64_t T, int V, int H, int act_dtype, float* dw,
+                      void* workspace, int64_t workspace_bytes, void* stream);
+
 /* Weight gradient of a dense projection y = x W^T: dw [N,K] f32 = g^T x, g [T,N] and x [T,K] dense
  * bf16 or fp16, fp32 sums in a fixed order.  N and K multiples of 8, at most 32 tiles of 256 x 256,
  * T at least 1024 (mts_linear_dw_supported).                                               */

@@ -1072,6 +1072,31 @@ struct Linear : torch::autograd::Function<Linear> {
     }
 };
 
+// The stock lookup; the table's gradient is summed here, from the gradient as it arrives in the activation dtype.
+bool embedding_supported(const Tensor& ids, const Tensor& w, at::ScalarType type) {
+    return at::GradMode::is_enabled() && w.requires_grad() && all_plain(ids, w) && on_one_gpu(ids, w) && ids.scalar_type() == at::kLong && w.dim() == 2 &&
+           w.scalar_type() == at::kFloat && is_activation_type(type) && mts_embedding_bwd_supported(ids.numel(), w.size(0), w.size(1));
+}
+
+struct Embedding : torch::autograd::Function<Embedding> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& ids, const Tensor& w, at::ScalarType type) {
+        ctx->save_for_backward({ids});
+        ctx->saved_data["rows"] = w.size(0);
+        return at::embedding(w, ids).to(type);
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        const Tensor ids = ctx->get_saved_variables()[0].contiguous();
+        c10::OptionalDeviceGuard guard(ids.device());
+        const int64_t V = ctx->saved_data["rows"].toInt(), T = ids.numel(), H = grads[0].size(-1);
+        if (written_out(grads)) return {Tensor(), at::embedding_dense_backward(grads[0].to(at::kFloat), ids, V, -1, false), Tensor()};
+        const Tensor g = dense16(grads[0]);
+        const int64_t ws_bytes = mts_embedding_bwd_workspace_bytes(T, V);
+        Tensor dw = f32({V, H}, g), ws = bytes(ws_bytes, g);
+        check(mts_embedding_bwd(ptr(g), ptr_as<int64_t>(ids), T, V, H, dtype_code(g), ptr_as<float>(dw), ptr(ws), ws_bytes, stream_of(g)), "mts_embedding_bwd");
+        return {Tensor(), dw, Tensor()};
+    }
+};
+
 bool heads_fit(const Tensor& t) {   // as the kernels read them
     return t.stride(3) == 1 && t.stride(0) % 8 == 0 && t.stride(1) % 8 == 0 && t.stride(2) % 8 == 0 && aligned16(t);
 }
@@ -1431,6 +1456,11 @@ PYBIND11_MODULE(_host, m) {
     m.def("linear", [](const Tensor& x, const Tensor& w) {
         c10::OptionalDeviceGuard guard(x.device());
         return Linear::apply(x, w);
+    });
+    m.def("embedding_supported", &embedding_supported);
+    m.def("embedding", [](const Tensor& ids, const Tensor& w, at::ScalarType type) {
+        c10::OptionalDeviceGuard guard(w.device());
+        return Embedding::apply(ids, w, type);
     });
     m.def("attention_supported", &attention_supported);
     m.def("attention", [](const Tensor& q, const Tensor& k, const Tensor& v, bool causal) {

@@ -77,6 +77,12 @@ class HipOpsBackend(DenseTorchOps):
             return None
         return dense.linear(x, weight)
 
+    def embedding(self, ids, weight, dtype):
+        """Extension: ``F.embedding(ids, weight).to(dtype)`` whose gradient is this backend's, or None where the caller's own does as well."""
+        if not dense.is_embedding_supported(ids, weight, dtype):
+            return None
+        return dense.embedding(ids, weight, dtype)
+
     def attention(self, q, k, v, *, is_causal, dropout_p):
         if not dropout_p and dense.is_attention_supported(q, k, v):
             return dense.attention(q, k, v, is_causal)

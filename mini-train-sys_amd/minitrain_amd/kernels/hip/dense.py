@@ -58,6 +58,15 @@ def linear(x, weight):
     return _lib.host().linear(x, weight)
 
 
+def is_embedding_supported(ids, weight, dtype) -> bool:
+    return _may_replace(ids, weight) and _lib.host().embedding_supported(ids, weight, dtype)
+
+
+def embedding(ids, weight, dtype):
+    """``F.embedding(ids, weight).to(dtype)`` with the gradient of ``weight`` summed from the gradient in ``dtype``"""
+    return _lib.host().embedding(ids, weight, dtype)
+
+
 def is_attention_supported(q, k, v) -> bool:
     return _may_replace(q, k, v) and _lib.host().attention_supported(q, k, v)
 

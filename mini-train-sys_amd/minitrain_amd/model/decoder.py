@@ -66,6 +66,14 @@ def project(linear: nn.Linear, x: torch.Tensor, ops: OpsBackend) -> torch.Tensor
     return linear(x) if y is None else y
 
 
+def embed(table: nn.Embedding, ids: torch.Tensor, dtype: torch.dtype, ops: OpsBackend) -> torch.Tensor:
+    """``table(ids).to(dtype)``, by the backend's own operator where it has one for these operands."""
+    own = getattr(ops, "embedding", None)
+    plain = table.padding_idx is None and table.max_norm is None and not table.scale_grad_by_freq and not table.sparse
+    x = own(ids, table.weight, dtype) if own is not None and plain and runs_as_written(table, nn.Embedding) else None
+    return table(ids).to(dtype) if x is None else x
+
+
 def layer_means(losses: list, records: list, ops: OpsBackend) -> list:
     """The means over the layers of the losses and of the records (numbers, or one per expert), in one launch where the
     backend offers it."""
@@ -158,7 +166,7 @@ class MiniTransformer(nn.Module):
         self._router_z = None
 
     def hidden_states(self, input_ids: torch.Tensor) -> torch.Tensor:
-        hidden = self.dropout(self.embed(input_ids).to(self.activation_dtype))
+        hidden = self.dropout(embed(self.embed, input_ids, self.activation_dtype, self.ops))
         cos, sin = self.rotary(hidden.size(1))
         if cos.device != hidden.device or cos.dtype != hidden.dtype:
             raise RuntimeError("RoPE cache must match the residual device and dtype")
