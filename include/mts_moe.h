@@ -503,6 +503,18 @@ int mts_cross_entropy_bwd_pitched(const void* logits, const int64_t* targets, in
                                   const float* row_log_sum, const float* g_loss, const float* inv_count,
                                   void* d_logits, int64_t pitch, void* stream);
 
+/* Both at once for g_loss = 1: loss, what the backward pass keeps, and d_logits (rows pitch elements apart, a multiple of 8).  bf16 and fp16,
+ * V from 8 to 65 536 (mts_cross_entropy_both_supported).  mts_cross_entropy_bwd_unless_one: as mts_cross_entropy_bwd_pitched, but where
+ * *g_loss is 1 d_logits stays as it is.                                                          */
+int mts_cross_entropy_both_supported(int V, int dtype);
+int mts_cross_entropy_both(const void* logits, const int64_t* targets, int64_t N, int V, int64_t ignore_index, int dtype,
+                           float* row_max, float* row_log_sum, float* row_loss, float* loss, float* inv_count,
+                           void* d_logits, int64_t pitch, void* stream);
+int mts_cross_entropy_bwd_unless_one(const void* logits, const int64_t* targets, int64_t N, int V,
+                                     int64_t ignore_index, int dtype, const float* row_max,
+                                     const float* row_log_sum, const float* g_loss, const float* inv_count,
+                                     void* d_logits, int64_t pitch, void* stream);
+
 /* Gradient of an embedding table: dw [V,H] f32, row r the sum of the rows of g [T,H] (act_dtype) whose id is r, in ascending order.
  * H a multiple of 4 up to 4096, T up to 2^18, V up to 2^20 (mts_embedding_bwd_supported).            */
 int mts_embedding_bwd_supported(int64_t T, int64_t V, int64_t H);

@@ -11,6 +11,7 @@
 // the operator forks two side streams for kernels that do not depend on one another and joins them before it returns.
 #include <ATen/ATen.h>
 #include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/SavedTensorHooks.h>
 #include <ATen/autocast_mode.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
@@ -1155,16 +1156,15 @@ bool cross_entropy_supported(const Tensor& logits, const Tensor& targets) {
            logits.size(1) < k2GiB;
 }
 
-// Whether the gradient that `self` returns goes, through views at most, to a projection whose gradients read rows of any pitch
-// (Linear::in_rounds), and nobody sees it on the way: no hook, no retained gradient, no result of autograd.grad.  Whoever does gets it dense.
-bool goes_to_rounds(torch::autograd::Node* self) {
-    const auto* execution = torch::autograd::get_current_graph_task_exec_info();
-    if (!self || !execution || !self->post_hooks().empty()) return false;
-    torch::autograd::Node* fn = self->next_edge(0).function.get();
+// Whether gradients of what `fn` made go, through views at most, to a projection whose gradients read rows of any pitch (Linear::in_rounds).  With
+// `execution`, the backward pass that is under way: and nobody sees them on the way, by a hook, a retained gradient or as a result of autograd.grad.
+bool goes_to_rounds(torch::autograd::Node* fn, const std::unordered_map<torch::autograd::Node*, torch::autograd::GraphTask::ExecInfo>* execution) {
     for (int depth = 0; fn && depth < 4; ++depth) {
         if (!fn->pre_hooks().empty() || !fn->tensor_pre_hooks().empty() || !fn->retains_grad_hooks().empty() || !fn->post_hooks().empty()) return false;
-        const auto found = execution->find(fn);
-        if (found != execution->end() && found->second.captures_) return false;
+        if (execution) {
+            const auto found = execution->find(fn);
+            if (found != execution->end() && found->second.captures_) return false;
+        }
         if (dynamic_cast<torch::autograd::CppNode<Linear>*>(fn)) return true;
         const std::string name = fn->name();
         if ((name != "ViewBackward0" && name != "UnsafeViewBackward0" && name != "ReshapeAliasBackward0") || fn->num_outputs() != 1) return false;
@@ -1172,19 +1172,41 @@ bool goes_to_rounds(torch::autograd::Node* self) {
     }
     return false;
 }
+// the same of the gradient that the node `self` returns in this backward pass; whoever sees it gets it dense
+bool goes_to_rounds_unseen(torch::autograd::Node* self) {
+    const auto* execution = torch::autograd::get_current_graph_task_exec_info();
+    return self && execution && self->post_hooks().empty() && goes_to_rounds(self->next_edge(0).function.get(), execution);
+}
 
 // mean cross-entropy without an fp32 copy of the logits
 struct CrossEntropy : torch::autograd::Function<CrossEntropy> {
+    // Whether the gradient is formed with the loss, for a caller who says that the loss is the root of its backward pass (its own gradient is
+    // then 1; where it is not after all, the backward pass forms it anew): from logits that are in registers anyway.  Rows as the backward
+    // pass will return them, so far as that is known; not where saved tensors are to go elsewhere, and this one would stay.
+    static bool formed_ahead(const Tensor& logits) {
+        const int64_t V = logits.size(1);
+        return at::GradMode::is_enabled() && logits.requires_grad() && mts_cross_entropy_both_supported((int)V, dtype_code(logits)) &&
+               !at::SavedTensorDefaultHooks::get_hooks() && (V % 8 == 0 || goes_to_rounds(logits.grad_fn().get(), nullptr));
+    }
     // dense16, dense
-    static Tensor forward(AutogradContext* ctx, const Tensor& logits, const Tensor& targets) {
+    static Tensor forward(AutogradContext* ctx, const Tensor& logits, const Tensor& targets, bool ahead) {
         const int64_t N = logits.size(0), V = logits.size(1);
         // per row: maximum, log of the sum, loss; then 1 / count.  The loss is a tensor of its own, which the caller may change
         // (no view) and which is not kept.
         Tensor rows = f32({3 * N + 1}, logits), loss = f32({}, logits);
         float* row = ptr_as<float>(rows);
-        check(mts_cross_entropy_fwd(ptr(logits), ptr_as<int64_t>(targets), N, V, kIgnoreIndex, dtype_code(logits), row, row + N, row + 2 * N,
-                                    ptr_as<float>(loss), row + 3 * N, stream_of(logits)),
-              "mts_cross_entropy_fwd");
+        if (ahead) {
+            const int64_t pitch = V % 8 ? row_pitch(V) : V;
+            Tensor d = at::empty({N, pitch}, logits.options());
+            check(mts_cross_entropy_both(ptr(logits), ptr_as<int64_t>(targets), N, V, kIgnoreIndex, dtype_code(logits), row, row + N, row + 2 * N, ptr_as<float>(loss),
+                                         row + 3 * N, ptr(d), pitch, stream_of(logits)),
+                  "mts_cross_entropy_both");
+            ctx->saved_data["ahead"] = d;
+        } else {
+            check(mts_cross_entropy_fwd(ptr(logits), ptr_as<int64_t>(targets), N, V, kIgnoreIndex, dtype_code(logits), row, row + N, row + 2 * N,
+                                        ptr_as<float>(loss), row + 3 * N, stream_of(logits)),
+                  "mts_cross_entropy_fwd");
+        }
         ctx->save_for_backward({logits, targets, rows});
         return loss;
     }
@@ -1198,23 +1220,35 @@ struct CrossEntropy : torch::autograd::Function<CrossEntropy> {
             const Tensor p = at::softmax(s[0].to(at::kFloat), 1) - hit.to(at::kFloat), none = at::zeros({}, p.options());
             const Tensor ignored = t.eq(kIgnoreIndex), outside = t.lt(0).logical_or(t.ge(V)).logical_and(ignored.logical_not());
             const Tensor scale = g * s[2].select(0, 3 * N) + at::where(outside, at::full({}, NAN, p.options()), none);
-            return {at::where(ignored, none, p * scale).to(s[0].scalar_type()), Tensor()};
+            return {at::where(ignored, none, p * scale).to(s[0].scalar_type()), Tensor(), Tensor()};
         }
         const Tensor g = like_f32(grads[0]);
         const float* row = ptr_as<float>(s[2]);
-        if (V % 8 && s[0].scalar_type() != at::kFloat && goes_to_rounds(torch::autograd::get_current_node().get())) {
+        const bool pitched = V % 8 && s[0].scalar_type() != at::kFloat && goes_to_rounds_unseen(torch::autograd::get_current_node().get());
+        const auto ahead = ctx->saved_data.find("ahead");
+        if (ahead != ctx->saved_data.end()) {
+            const Tensor rows = ahead->second.toTensor();
+            ctx->saved_data.erase(ahead);   // whoever gets it may write to it; a second pass forms its own
+            if (V % 8 == 0 || pitched) {
+                check(mts_cross_entropy_bwd_unless_one(ptr(s[0]), ptr_as<int64_t>(s[1]), N, V, kIgnoreIndex, dtype_code(s[0]), row, row + N, ptr_as<float>(g),
+                                                       row + 3 * N, ptr(rows), rows.size(1), stream_of(s[0])),
+                      "mts_cross_entropy_bwd_unless_one");
+                return {V % 8 ? rows.narrow(1, 0, V) : rows, Tensor(), Tensor()};
+            }
+        }
+        if (pitched) {
             const int64_t pitch = row_pitch(V);
             Tensor rows = at::empty({N, pitch}, s[0].options());
             check(mts_cross_entropy_bwd_pitched(ptr(s[0]), ptr_as<int64_t>(s[1]), N, V, kIgnoreIndex, dtype_code(s[0]), row, row + N, ptr_as<float>(g),
                                                 row + 3 * N, ptr(rows), pitch, stream_of(s[0])),
                   "mts_cross_entropy_bwd_pitched");
-            return {rows.narrow(1, 0, V), Tensor()};
+            return {rows.narrow(1, 0, V), Tensor(), Tensor()};
         }
         Tensor d = at::empty_like(s[0]);
         check(mts_cross_entropy_bwd(ptr(s[0]), ptr_as<int64_t>(s[1]), N, V, kIgnoreIndex, dtype_code(s[0]), row, row + N, ptr_as<float>(g),
                                     row + 3 * N, ptr(d), stream_of(s[0])),
               "mts_cross_entropy_bwd");
-        return {d, Tensor()};
+        return {d, Tensor(), Tensor()};
     }
 };
 
@@ -1499,9 +1533,9 @@ PYBIND11_MODULE(_host, m) {
         adamw(params, exp_avgs, exp_avg_sqs, steps, groups, settings, scale, skip_if_not_finite);
     });
     m.def("cross_entropy_supported", &cross_entropy_supported);
-    m.def("cross_entropy", [](const Tensor& logits, const Tensor& targets) {
+    m.def("cross_entropy", [](const Tensor& logits, const Tensor& targets, bool is_root) {
         c10::OptionalDeviceGuard guard(logits.device());
         const Tensor dense = dense16(logits);
-        return CrossEntropy::apply(dense, targets.contiguous());
+        return CrossEntropy::apply(dense, targets.contiguous(), is_root && CrossEntropy::formed_ahead(dense));
     });
 }

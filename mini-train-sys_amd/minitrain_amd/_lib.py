@@ -89,6 +89,9 @@ SIGNATURES = {
     "mts_rmsnorm_bwd": (_i, [_p, _p, _p, _p, _p, _l, _i, _i, _p, _p, _p, _l, _p]),
     "mts_rope": (_i, [_p, _i, _p, _p, _l, _l, _i, _i, _i, _p]),
     "mts_cross_entropy_fwd": (_i, [_p, _p, _l, _i, _l, _i, _p, _p, _p, _p, _p, _p]),
+    "mts_cross_entropy_both_supported": (_i, [_i, _i]),
+    "mts_cross_entropy_both": (_i, [_p, _p, _l, _i, _l, _i, _p, _p, _p, _p, _p, _p, _l, _p]),
+    "mts_cross_entropy_bwd_unless_one": (_i, [_p, _p, _l, _i, _l, _i, _p, _p, _p, _p, _p, _l, _p]),
     "mts_embedding_bwd_supported": (_i, [_l, _l, _l]),
     "mts_embedding_bwd_workspace_bytes": (_l, [_l, _l]),
     "mts_embedding_bwd": (_i, [_p, _p, _l, _i, _i, _i, _p, _p, _l, _p]),

@@ -8,6 +8,9 @@ everything else (CPU tensors, other dtypes or layouts) to the stock operators.  
 are native (``csrc/host/mts_host.cpp``).
 """
 
+import contextlib
+import threading
+
 import torch
 from torch.overrides import has_torch_function
 
@@ -80,9 +83,23 @@ def is_cross_entropy_supported(logits, targets) -> bool:
     return _may_replace(logits, targets) and _lib.host().cross_entropy_supported(logits, targets)
 
 
+_root = threading.local()
+
+
+@contextlib.contextmanager
+def loss_is_root():
+    """Losses formed inside, by this thread, are the root of the caller's backward pass, unscaled: their gradient may be formed with them."""
+    before = getattr(_root, "is_loss", False)
+    _root.is_loss = True
+    try:
+        yield
+    finally:
+        _root.is_loss = before
+
+
 def cross_entropy(logits, targets):
     """``F.cross_entropy(logits.float(), targets)`` without the fp32 copy of the logits"""
-    return _lib.host().cross_entropy(logits, targets)
+    return _lib.host().cross_entropy(logits, targets, getattr(_root, "is_loss", False))
 
 
 def is_layer_means_supported(groups, differentiable: int) -> bool:

@@ -8,6 +8,7 @@ import contextlib
 
 import torch
 
+from minitrain_amd.kernels.hip.dense import loss_is_root
 from minitrain_amd.train.update import plan
 
 
@@ -39,7 +40,7 @@ def train_step(model: torch.nn.Module, optimizer: torch.optim.Optimizer, batch: 
         if autocast_dtype is not None and device.type == "cuda"
         else contextlib.nullcontext()
     )
-    with ctx:
+    with ctx, loss_is_root():
         loss, _ = model(input_ids, targets=targets, use_fused_loss=use_fused_loss)
     loss.backward()
     update = plan(model, optimizer, loss.detach(), grad_clip_norm)
