@@ -122,6 +122,16 @@ int mts_router_wide_bwd(const float* dlogits, const void* x, const float* w_r, i
                         int act_dtype, void* dx, float* d_w_r, void* workspace,
                         int64_t workspace_bytes, void* stream);
 
+/* The head of a layer with 17 to 64 experts in three launches: projection chained to the post-process, scan, scatter.  As mts_router_wide_fwd
+ * followed by mts_moe_router_route; T up to 32 768 (mts_moe_wide_head_supported).                 */
+int mts_moe_wide_head_supported(int64_t T, int H, int E, int K);
+int64_t mts_moe_wide_head_workspace_bytes(int64_t T, int E);
+int mts_moe_wide_head_fwd(const void* x, const float* w_r, int64_t T, int H, int E, int K, int normalize,
+                          int act_dtype, float* logits, float* weights, int32_t* indices, void* weights_act,
+                          float* prob_mean, float* z_loss, float* entropy, int32_t* counts, float* load_balance,
+                          float* load_stats, int32_t* expert_start, int32_t* s_scatter, int32_t* s_reverse,
+                          int32_t* x_gather, void* workspace, int64_t workspace_bytes, void* stream);
+
 /* ---- the layer's head in two launches ---------------------------------------
  * mts_router_logits_fwd + mts_router_fwd + mts_moe_route as one chain (router projection,
  * post-process and routing metadata of minitrain/model/moe_router.py:64-90 and

@@ -645,7 +645,8 @@ LayerForward layer_forward(const Tensor& x_, const Tensor& w_r_, const Tensor& w
     const int64_t T = x.size(0), H = x.size(1), E = w_r.size(0), TK = T * K, I = w1.size(1) / 2;
     const auto dtype = x.scalar_type();
     const bool narrow = dtype != at::kFloat, limited = capacity >= 0, alone = opt.on(NO_BACKWARD), few = E <= kFewExperts;
-    const int64_t ws_bytes = few ? mts_moe_head_workspace_bytes(T, K, E) : mts_moe_router_route_workspace_bytes(T, K, E);
+    const bool chained = few || mts_moe_wide_head_supported(T, H, E, K);   // projection, post-process and routing metadata behind one entry point
+    const int64_t ws_bytes = few ? mts_moe_head_workspace_bytes(T, K, E) : chained ? mts_moe_wide_head_workspace_bytes(T, E) : mts_moe_router_route_workspace_bytes(T, K, E);
     f.w_r = w_r;
     f.weights = f32({T, K}, x);
     // The integer results in one allocation and the fp32 statistics in another: a caller may save all results together, which torch refuses
@@ -685,13 +686,13 @@ LayerForward layer_forward(const Tensor& x_, const Tensor& w_r_, const Tensor& w
     }
     void* load_stats = limited ? nullptr : ptr(f.load_stats);
     void* cast_weights = narrow && !limited ? ptr(weights_act) : nullptr;
-    if (few) {
-        check(mts_moe_head_fwd(ptr(x), ptr_as<float>(w_r), T, H, E, K, normalize, dtype_code(x), ptr_as<float>(f.logits), ptr_as<float>(f.weights),
+    if (chained) {
+        check((few ? mts_moe_head_fwd : mts_moe_wide_head_fwd)(ptr(x), ptr_as<float>(w_r), T, H, E, K, normalize, dtype_code(x), ptr_as<float>(f.logits), ptr_as<float>(f.weights),
                                ptr_as<int32_t>(f.indices), cast_weights, ptr_as<float>(f.prob_mean), ptr_as<float>(f.z_loss), ptr_as<float>(f.entropy),
                                ptr_as<int32_t>(f.counts), ptr_as<float>(f.load_balance), static_cast<float*>(load_stats), ptr_as<int32_t>(r.expert_start),
                                ptr_as<int32_t>(r.s_scatter), ptr_as<int32_t>(r.s_reverse), ptr_as<int32_t>(r.x_gather), ptr(ws), ws_bytes, stream_of(x)),
-              "mts_moe_head_fwd");
-    } else {   // the chained head is written for few experts
+              few ? "mts_moe_head_fwd" : "mts_moe_wide_head_fwd");
+    } else {
         router_projection_forward(x, w_r, f.logits);
         check(mts_moe_router_route(ptr_as<float>(f.logits), T, E, K, normalize, ptr_as<float>(f.weights), ptr_as<int32_t>(f.indices), ptr_as<float>(f.prob_mean),
                                    ptr_as<float>(f.z_loss), ptr_as<float>(f.entropy), ptr_as<int32_t>(f.counts), ptr_as<float>(f.load_balance),

@@ -181,6 +181,11 @@ struct MtsRouterStats {
 int mts_launch_router_fwd(const float* logits, int64_t T, int E, int K, int normalize, float* weights, int32_t* indices, float* prob_mean, float* z_loss,
                           float* entropy, int32_t* counts, float* load_balance, float* load_stats, void* weights_act, int act_dtype, void* workspace,
                           int64_t workspace_bytes, MtsRouterStats* stats, hipStream_t s);
+// rows of a block of the chained head of 17 to 64 experts (mts_router_wide.hip), which are a chunk of its routing metadata, and the most of them
+#define MTS_WIDE_HEAD_ROWS 32
+#define MTS_WIDE_HEAD_CHUNKS 1024
+int mts_launch_wide_head(const void* x, const float* w_r, int64_t T, int H, int E, int K, int normalize, int act_dtype, float* logits, float* weights, int32_t* indices,
+                         void* weights_act, float* partial, int32_t* partial_counts, int32_t* cnt, hipStream_t s);
 // What the launch behind the head writes from partial and cnt.  Where the head is one block (up to 64 tokens) the block writes it itself:
 // *finished is 1 then, and partial and cnt are left as they are.
 struct MtsHeadFinish {

@@ -440,6 +440,43 @@ extern "C" int mts_moe_router_route(const float* logits, int64_t T, int E, int K
     return route_launch(indices, T, K, E, 64, scan_counts, expert_start, s_scatter, s_reverse, x_gather, nullptr, nullptr, nullptr, cnt, (hipStream_t)stream, &stats);
 }
 
+// The routing metadata of more than MTS_WIDE_HEAD_CHUNKS chunks of the chained kernel takes longer than what the chain saves; below 17 experts the head
+// of few experts is ahead.
+extern "C" int mts_moe_wide_head_supported(int64_t T, int H, int E, int K) {
+    return T > 0 && (T + MTS_WIDE_HEAD_ROWS - 1) / MTS_WIDE_HEAD_ROWS <= MTS_WIDE_HEAD_CHUNKS && E > 16 && E <= 64 && K >= 1 && K <= MTS_MAX_TOP_K &&
+           mts_router_wide_supported(H, E) ? 1 : 0;
+}
+
+extern "C" int64_t mts_moe_wide_head_workspace_bytes(int64_t T, int E) {
+    const int64_t chunks = (T + MTS_WIDE_HEAD_ROWS - 1) / MTS_WIDE_HEAD_ROWS;
+    return (chunks * (3 * E + 2) + E) * (int64_t)sizeof(int32_t);   // statistics, routes for them, routes for the scan; the scan's totals
+}
+
+extern "C" int mts_moe_wide_head_fwd(const void* x, const float* w_r, int64_t T, int H, int E, int K, int normalize, int act_dtype, float* logits, float* weights,
+                                     int32_t* indices, void* weights_act, float* prob_mean, float* z_loss, float* entropy, int32_t* counts, float* load_balance,
+                                     float* load_stats, int32_t* expert_start, int32_t* s_scatter, int32_t* s_reverse, int32_t* x_gather, void* workspace,
+                                     int64_t workspace_bytes, void* stream) {
+    if (!prob_mean || !z_loss || !entropy || !counts || !expert_start || !s_scatter || !s_reverse || !x_gather || !workspace) return MTS_ERR_NULL;
+    if (weights_act && act_dtype == MTS_F32) return MTS_ERR_DTYPE;
+    if (!mts_moe_wide_head_supported(T, H, E, K)) return MTS_ERR_SHAPE;
+    if (workspace_bytes < mts_moe_wide_head_workspace_bytes(T, E)) return MTS_ERR_WORKSPACE;
+    if (!mts_aligned16(workspace)) return MTS_ERR_ALIGN;
+    hipStream_t s = (hipStream_t)stream;
+    const int64_t chunks = (T + MTS_WIDE_HEAD_ROWS - 1) / MTS_WIDE_HEAD_ROWS;
+    float* partial = (float*)workspace;
+    int32_t *partial_counts = (int32_t*)(partial + chunks * (E + 2)), *cnt = partial_counts + chunks * E, *totals = cnt + chunks * E;
+    const int rc = mts_launch_wide_head(x, w_r, T, H, E, K, normalize, act_dtype, logits, weights, indices, weights_act, partial, partial_counts, cnt, s);
+    if (rc) return rc;
+    const MtsRouterStats stats = {partial, partial_counts, (int)chunks, E, 1.0f / (float)T, 1.0f / ((float)T * (float)K), prob_mean, z_loss, entropy, counts,
+                                  load_balance, load_stats};
+    route_scan_kernel<<<2, kScanThreads, 0, s>>>(cnt, chunks, E, 64, totals, expert_start, nullptr, nullptr, nullptr, 0, stats);
+    MTS_CHECK_LAUNCH();
+    route_scatter_kernel<<<dim3((unsigned)((chunks + kWaves - 1) / kWaves)), kThreads, (size_t)kWaves * E * sizeof(int32_t), s>>>(
+        indices, T * K, K, E, 0, E, MTS_WIDE_HEAD_ROWS * K, cnt, expert_start, s_scatter, s_reverse, x_gather);
+    MTS_CHECK_LAUNCH();
+    return MTS_OK;
+}
+
 extern "C" int64_t mts_moe_head_workspace_bytes(int64_t T, int K, int E) {
     (void)T;
     (void)K;

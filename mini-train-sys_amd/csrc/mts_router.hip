@@ -21,96 +21,29 @@ __global__ __launch_bounds__(kThreads) void router_fwd_kernel(
     const float* __restrict__ logits, int64_t T, int E, int K, int normalize,
     float* __restrict__ weights, int32_t* __restrict__ indices, float* __restrict__ partial,
     int32_t* __restrict__ partial_counts, void* __restrict__ weights_act, int act_dtype) {
-    constexpr int ROWS = kThreads / G;
+    constexpr int ROWS = kThreads / G, WAVES = kThreads / MTS_WAVE;
     const int g = threadIdx.x % G;
     const int rl = threadIdx.x / G;
-    float psum[EP];
-    int csum[EP];   // routes to the experts this lane owns (slot j is expert j*G + g)
-#pragma unroll
-    for (int j = 0; j < EP; ++j) {
-        psum[j] = 0.f;
-        csum[j] = 0;
-    }
-    float zsum = 0.f, hsum = 0.f;
-
+    RowTotals<EP, G> totals;
     for (int64_t row0 = (int64_t)blockIdx.x * ROWS; row0 < T; row0 += (int64_t)gridDim.x * ROWS) {
         int64_t row = row0 + rl;
         bool live = row < T;
         RowState<EP, G> r;
         load_row<EP, G>(logits, live ? row : 0, E, g, r);
-
-        float sel_p[MTS_MAX_TOP_K];
-        int sel_e[MTS_MAX_TOP_K];
-        float mass;
-        select_top_k<EP, G>(r, E, K, g, sel_p, sel_e, mass);
-#pragma unroll
-        for (int k = 0; k < MTS_MAX_TOP_K; ++k)
-#pragma unroll
-            for (int j = 0; j < EP; ++j) csum[j] += (live && k < K && j * G + g == sel_e[k]) ? 1 : 0;
-        if (live && g == 0) {
-            float inv = normalize ? 1.0f / fmaxf(mass, 1.1920928955078125e-07f) : 1.0f;
-#pragma unroll
-            for (int k = 0; k < MTS_MAX_TOP_K; ++k) {
-                if (k < K) {
-                    const float wk = sel_p[k] * inv;
-                    weights[row * K + k] = wk;
-                    indices[row * K + k] = sel_e[k];
-                    // the copy the MoE block hands to fused_moe: rounded once, as tensor.to() rounds
-                    if (weights_act) {
-                        if (act_dtype == MTS_BF16) reinterpret_cast<bf16_t*>(weights_act)[row * K + k] = (bf16_t)wk;
-                        else reinterpret_cast<mts_f16_t*>(weights_act)[row * K + k] = (mts_f16_t)wk;
-                    }
-                }
-            }
-        }
-        if (live) {
-#pragma unroll
-            for (int j = 0; j < EP; ++j) {
-                psum[j] += r.p[j];
-                // p * log(max(p, 1e-9)); p == 0 (padding or underflow) contributes 0
-                float lp = fmaxf(r.l[j] - r.L, kLogFloor);
-                hsum -= (r.p[j] > 0.f) ? r.p[j] * lp : 0.f;
-            }
-            if (g == 0) zsum += r.L * r.L;
-        }
+        totals.take(r, live, row, E, K, normalize, g, weights, indices, weights_act, act_dtype);
     }
 
-    // wave: sum lanes that hold the same experts (same g)
-#pragma unroll
-    for (int j = 0; j < EP; ++j) psum[j] = lane_reduce<32, G>(psum[j], LaneSum());
-    zsum = wave_sum(zsum);
-    hsum = wave_sum(hsum);
-#pragma unroll
-    for (int j = 0; j < EP; ++j) csum[j] = lane_reduce<32, G>(csum[j], LaneSum());
-
-    __shared__ float red[kThreads / MTS_WAVE][EP * G + 2];
-    __shared__ int32_t cred[kThreads / MTS_WAVE][EP * G];
-    const int wave = threadIdx.x / MTS_WAVE, lane = threadIdx.x % MTS_WAVE;
-    if (lane < G) {
-#pragma unroll
-        for (int j = 0; j < EP; ++j) {
-            red[wave][j * G + lane] = psum[j];
-            cred[wave][j * G + lane] = csum[j];
-        }
-    }
-    if (lane == 0) {
-        red[wave][EP * G] = zsum;
-        red[wave][EP * G + 1] = hsum;
-    }
+    __shared__ float red[WAVES][EP * G + 2];
+    __shared__ int32_t cred[WAVES][EP * G];
+    totals.to_lds(red[threadIdx.x / MTS_WAVE], cred[threadIdx.x / MTS_WAVE]);
     __syncthreads();
     float* out = partial + (int64_t)blockIdx.x * (E + 2);
-    for (int i = threadIdx.x; i < E + 2; i += kThreads) {
-        int src = i < E ? i : EP * G + (i - E);
-        float v = 0.f;
-#pragma unroll
-        for (int w = 0; w < kThreads / MTS_WAVE; ++w) v += red[w][src];
-        out[i] = v;
-    }
+    for (int i = threadIdx.x; i < E + 2; i += kThreads) out[i] = block_column<EP, G, WAVES>(red, i, E);
     int32_t* cout = partial_counts + (int64_t)blockIdx.x * E;
     for (int i = threadIdx.x; i < E; i += kThreads) {
         int32_t v = 0;
 #pragma unroll
-        for (int w = 0; w < kThreads / MTS_WAVE; ++w) v += cred[w][i];
+        for (int w = 0; w < WAVES; ++w) v += cred[w][i];
         cout[i] = v;
     }
 }

@@ -137,6 +137,86 @@ __device__ __forceinline__ void select_top_k(const RowState<EP, G>& r, int E, in
     }
 }
 
+// What a lane has summed over its rows, G lanes a row: probability mass and routes of its experts (slot j is expert j*G + g), squared
+// log-partitions, entropies.
+template <int EP, int G>
+struct RowTotals {
+    float psum[EP] = {};
+    int csum[EP] = {};
+    float zsum = 0.f, hsum = 0.f;
+
+    // top-k of a row: its weights and indices go out, its statistics to the sums (rows that are not `live`: neither)
+    __device__ __forceinline__ void take(const RowState<EP, G>& r, bool live, int64_t row, int E, int K, int normalize, int g, float* __restrict__ weights,
+                                         int32_t* __restrict__ indices, void* __restrict__ weights_act, int act_dtype) {
+        float sel_p[MTS_MAX_TOP_K];
+        int sel_e[MTS_MAX_TOP_K];
+        float mass;
+        select_top_k<EP, G>(r, E, K, g, sel_p, sel_e, mass);
+#pragma unroll
+        for (int k = 0; k < MTS_MAX_TOP_K; ++k)
+#pragma unroll
+            for (int j = 0; j < EP; ++j) csum[j] += (live && k < K && j * G + g == sel_e[k]) ? 1 : 0;
+        if (live && g == 0) {
+            float inv = normalize ? 1.0f / fmaxf(mass, 1.1920928955078125e-07f) : 1.0f;
+#pragma unroll
+            for (int k = 0; k < MTS_MAX_TOP_K; ++k) {
+                if (k < K) {
+                    const float wk = sel_p[k] * inv;
+                    weights[row * K + k] = wk;
+                    indices[row * K + k] = sel_e[k];
+                    // the copy the MoE block hands to fused_moe: rounded once, as tensor.to() rounds
+                    if (weights_act) {
+                        if (act_dtype == MTS_BF16) reinterpret_cast<bf16_t*>(weights_act)[row * K + k] = (bf16_t)wk;
+                        else reinterpret_cast<mts_f16_t*>(weights_act)[row * K + k] = (mts_f16_t)wk;
+                    }
+                }
+            }
+        }
+        if (live) {
+#pragma unroll
+            for (int j = 0; j < EP; ++j) {
+                psum[j] += r.p[j];
+                // p * log(max(p, 1e-9)); p == 0 (padding or underflow) contributes 0
+                float lp = fmaxf(r.l[j] - r.L, kLogFloor);
+                hsum -= (r.p[j] > 0.f) ? r.p[j] * lp : 0.f;
+            }
+            if (g == 0) zsum += r.L * r.L;
+        }
+    }
+
+    // the sums of a wave's lanes to the wave's row of LDS
+    __device__ __forceinline__ void to_lds(float* red, int32_t* cred) {
+        const int lane = threadIdx.x % MTS_WAVE;
+#pragma unroll
+        for (int j = 0; j < EP; ++j) psum[j] = lane_reduce<32, G>(psum[j], LaneSum());   // lanes that hold the same experts
+        zsum = wave_sum(zsum);
+        hsum = wave_sum(hsum);
+#pragma unroll
+        for (int j = 0; j < EP; ++j) csum[j] = lane_reduce<32, G>(csum[j], LaneSum());
+        if (lane < G) {
+#pragma unroll
+            for (int j = 0; j < EP; ++j) {
+                red[j * G + lane] = psum[j];
+                cred[j * G + lane] = csum[j];
+            }
+        }
+        if (lane == 0) {
+            red[EP * G] = zsum;
+            red[EP * G + 1] = hsum;
+        }
+    }
+};
+
+// column i < E + 2 of a block's statistics, and for i < E its routes, from its waves' rows
+template <int EP, int G, int WAVES>
+__device__ __forceinline__ float block_column(const float (&red)[WAVES][EP * G + 2], int i, int E) {
+    const int src = i < E ? i : EP * G + (i - E);
+    float v = 0.f;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) v += red[w][src];
+    return v;
+}
+
 // Gradient of a row's logits.  dp: gradient that reaches the row's probabilities through the mean
 // probability (and the load-balancing term), per slot of this lane; gz: gradient of the z-loss
 // times 2/T; weights / indices / grad_w(k): the row's selected weights, experts and weight gradients.

@@ -10,6 +10,7 @@
 // 8192 x 1024, 64 experts, bf16: 15.8 us forward, 29 + 5.5 backward; 22 and 19 + 17 + 6 with branches at the loads, four waves, 2-byte stores
 // of dx and a launch each.  16 384 x 2048, 128 experts: 124 -> 95 and 210 -> 188.
 #include "mts_f32_tiles.h"
+#include "mts_router_row.h"
 
 #include <type_traits>
 
@@ -23,66 +24,122 @@ constexpr int kBwdLds = 2 * (64 * 20 + 16 * 72);   // floats: the two buffers of
 // 32 rows x 64 experts; wave w multiplies k-step w of every 64-wide k-tile, the eight sums meet in LDS.  Two waves of a SIMD: one reads its
 // fragments while the other multiplies (four waves of two k-steps each: 19.9 us for 8192 x 1024 x 64 where this takes 15.8).
 template <typename XT>
-__global__ __launch_bounds__(kLogitsThreads) void wide_logits_kernel(const XT* __restrict__ x, const float* __restrict__ w, int64_t T, int H, int E,
-                                                                     float* __restrict__ logits) {
-    constexpr int BM = 32, BN = 64, TKS = 64, WAVES = kLogitsThreads / MTS_WAVE, STEPS = TKS / 8 / WAVES;
+struct WideTile {
+    static constexpr int BM = 32, BN = 64, TKS = 64, WAVES = kLogitsThreads / MTS_WAVE, STEPS = TKS / 8 / WAVES;
     typedef RowTile<XT, BM, TKS, true, kLogitsThreads> AT;
     typedef RowTile<float, BN, TKS, true, kLogitsThreads> BT;
-    constexpr int TILES = 2 * (AT::SIZE + BT::SIZE), SUMS = WAVES * BM * BN;
-    __shared__ __attribute__((aligned(16))) float lds[TILES > SUMS ? TILES : SUMS];
-    float(*As)[AT::SIZE] = reinterpret_cast<float(*)[AT::SIZE]>(lds);
-    float(*Bs)[BT::SIZE] = reinterpret_cast<float(*)[BT::SIZE]>(lds + 2 * AT::SIZE);
-    const int64_t row0 = (int64_t)blockIdx.x * BM;
-    const int e0 = blockIdx.y * BN;
-    AT a;
-    BT b;
-#pragma unroll
-    for (int q = 0; q < AT::LOADS; ++q) {
-        const int64_t r = row0 + AT::row(q);
-        a.ptr[q] = x + (r < T ? r : T - 1) * H;
-    }
-#pragma unroll
-    for (int q = 0; q < BT::LOADS; ++q) {
-        const int e = e0 + BT::row(q);
-        b.ptr[q] = w + (int64_t)(e < E ? e : E - 1) * H;
-    }
-    const int wave = threadIdx.x / MTS_WAVE, lane = threadIdx.x % MTS_WAVE;
-    f32x16 acc[1][2] = {};
-    auto fetch = [&](int set, int t) {
-        a.fetch(set, t * TKS, H);
-        b.fetch(set, t * TKS, H);
-    };
-    run_k_tiles<AT, BT, TKS, STEPS, 1, 2, true>(H, a, b, As, Bs, acc, [](int) { return 0; }, [](int nf) { return nf * 32; }, fetch, wave * STEPS);
-    // a lane holds runs of four experts of row lane % 32; the groups of four of a row are dealt by the row
-    const int ml = lane % 32;
-    float* mine = lds + wave * BM * BN + ml * BN;
-#pragma unroll
-    for (int nf = 0; nf < 2; ++nf)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const f32x4 v = {acc[0][nf][4 * j], acc[0][nf][4 * j + 1], acc[0][nf][4 * j + 2], acc[0][nf][4 * j + 3]};
-            *reinterpret_cast<f32x4*>(mine + (((nf * 8 + 2 * j + lane / 32) ^ (ml & 15)) << 2)) = v;
-        }
-    __syncthreads();
+    static constexpr int TILES = 2 * (AT::SIZE + BT::SIZE), SUMS = WAVES * BM * BN, LDS = TILES > SUMS ? TILES : SUMS;   // floats
     static_assert(BM * BN / 4 == kLogitsThreads, "four sums a thread");
-    const int m = threadIdx.x / (BN / 4), g = threadIdx.x % (BN / 4);
-    const int64_t r = row0 + m;
-    const float* part = lds + m * BN + ((g ^ (m & 15)) << 2);
-    f32x4 sum = *reinterpret_cast<const f32x4*>(part);
+    static __device__ __forceinline__ int row() { return threadIdx.x / (BN / 4); }
+    static __device__ __forceinline__ int first_expert() { return threadIdx.x % (BN / 4) * 4; }
+
+    // logits of row row0 + row(), experts e0 + first_expert() .. + 3
+    static __device__ __forceinline__ f32x4 logits(const XT* __restrict__ x, const float* __restrict__ w, int64_t T, int H, int E, int64_t row0, int e0, float* lds) {
+        float(*As)[AT::SIZE] = reinterpret_cast<float(*)[AT::SIZE]>(lds);
+        float(*Bs)[BT::SIZE] = reinterpret_cast<float(*)[BT::SIZE]>(lds + 2 * AT::SIZE);
+        AT a;
+        BT b;
 #pragma unroll
-    for (int k = 1; k < WAVES; ++k) {   // in wave order
-        const f32x4 v = *reinterpret_cast<const f32x4*>(part + k * BM * BN);
+        for (int q = 0; q < AT::LOADS; ++q) {
+            const int64_t r = row0 + AT::row(q);
+            a.ptr[q] = x + (r < T ? r : T - 1) * H;
+        }
 #pragma unroll
-        for (int j = 0; j < 4; ++j) sum[j] += v[j];
+        for (int q = 0; q < BT::LOADS; ++q) {
+            const int e = e0 + BT::row(q);
+            b.ptr[q] = w + (int64_t)(e < E ? e : E - 1) * H;
+        }
+        const int wave = threadIdx.x / MTS_WAVE, lane = threadIdx.x % MTS_WAVE;
+        f32x16 acc[1][2] = {};
+        auto fetch = [&](int set, int t) {
+            a.fetch(set, t * TKS, H);
+            b.fetch(set, t * TKS, H);
+        };
+        run_k_tiles<AT, BT, TKS, STEPS, 1, 2, true>(H, a, b, As, Bs, acc, [](int) { return 0; }, [](int nf) { return nf * 32; }, fetch, wave * STEPS);
+        // a lane holds runs of four experts of row lane % 32; the groups of four of a row are dealt by the row
+        const int ml = lane % 32;
+        float* mine = lds + wave * BM * BN + ml * BN;
+#pragma unroll
+        for (int nf = 0; nf < 2; ++nf)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const f32x4 v = {acc[0][nf][4 * j], acc[0][nf][4 * j + 1], acc[0][nf][4 * j + 2], acc[0][nf][4 * j + 3]};
+                *reinterpret_cast<f32x4*>(mine + (((nf * 8 + 2 * j + lane / 32) ^ (ml & 15)) << 2)) = v;
+            }
+        __syncthreads();
+        const float* part = lds + row() * BN + ((first_expert() / 4 ^ (row() & 15)) << 2);
+        f32x4 sum = *reinterpret_cast<const f32x4*>(part);
+#pragma unroll
+        for (int k = 1; k < WAVES; ++k) {   // in wave order
+            const f32x4 v = *reinterpret_cast<const f32x4*>(part + k * BM * BN);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) sum[j] += v[j];
+        }
+        return sum;
     }
-    if (r >= T) return;
-    float* out = logits + r * E + e0 + 4 * g;
-    if (E % 4 == 0) {
-        if (e0 + 4 * g < E) *reinterpret_cast<f32x4*>(out) = sum;
-    } else {
+    static __device__ __forceinline__ void store(f32x4 sum, float* __restrict__ logits, int64_t r, int64_t T, int E, int e) {
+        if (r >= T) return;
+        float* out = logits + r * E + e;
+        if (E % 4 == 0) {
+            if (e < E) *reinterpret_cast<f32x4*>(out) = sum;
+        } else {
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-            if (e0 + 4 * g + j < E) out[j] = sum[j];
+            for (int j = 0; j < 4; ++j)
+                if (e + j < E) out[j] = sum[j];
+        }
+    }
+};
+template <typename XT>
+__global__ __launch_bounds__(kLogitsThreads) void wide_logits_kernel(const XT* __restrict__ x, const float* __restrict__ w, int64_t T, int H, int E,
+                                                                     float* __restrict__ logits) {
+    typedef WideTile<XT> Tile;
+    __shared__ __attribute__((aligned(16))) float lds[Tile::LDS];
+    const int64_t row0 = (int64_t)blockIdx.x * Tile::BM;
+    const int e0 = blockIdx.y * Tile::BN;
+    const f32x4 sum = Tile::logits(x, w, T, H, E, row0, e0, lds);
+    Tile::store(sum, logits, row0 + Tile::row(), T, E, e0 + Tile::first_expert());
+}
+
+// The same chained to the post-process, for up to 64 experts: a block holds all logits of its rows, so that its first waves go on with
+// G lanes a row, as the post-process kernel does (the same results), and leave its routes per expert, which are the counters of the routing
+// metadata's chunks.
+template <typename XT, int G>
+__global__ __launch_bounds__(kLogitsThreads) void wide_head_kernel(const XT* __restrict__ x, const float* __restrict__ w, int64_t T, int H, int E, int K, int normalize,
+                                                                   float* __restrict__ logits, float* __restrict__ weights, int32_t* __restrict__ indices,
+                                                                   void* __restrict__ weights_act, int act_dtype, float* __restrict__ partial,
+                                                                   int32_t* __restrict__ partial_counts, int32_t* __restrict__ cnt) {
+    using namespace mts_router;
+    typedef WideTile<XT> Tile;
+    constexpr int EP = 8, WAVES = Tile::BM * G / MTS_WAVE, LROW = 72;   // a row's lanes and the rows of a wave fall on different banks
+    __shared__ __attribute__((aligned(16))) float lds[Tile::LDS];
+    __shared__ __attribute__((aligned(16))) float rows[Tile::BM][LROW];
+    __shared__ float red[WAVES][EP * G + 2];
+    __shared__ int32_t cred[WAVES][EP * G];
+    const int64_t row0 = (int64_t)blockIdx.x * Tile::BM;
+    const f32x4 sum = Tile::logits(x, w, T, H, E, row0, 0, lds);
+    *reinterpret_cast<f32x4*>(&rows[Tile::row()][Tile::first_expert()]) = sum;
+    Tile::store(sum, logits, row0 + Tile::row(), T, E, Tile::first_expert());
+    __syncthreads();
+    const int wave = threadIdx.x / MTS_WAVE;
+    if (wave < WAVES) {
+        const int g = threadIdx.x % G, rl = threadIdx.x / G;
+        RowState<EP, G> r;
+#pragma unroll
+        for (int j = 0; j < EP; ++j) r.l[j] = j * G + g < E ? rows[rl][j * G + g] : -INFINITY;
+        softmax_row<EP, G>(r);
+        RowTotals<EP, G> totals;
+        totals.take(r, row0 + rl < T, row0 + rl, E, K, normalize, g, weights, indices, weights_act, act_dtype);
+        totals.to_lds(red[wave], cred[wave]);
+    }
+    __syncthreads();
+    const int i = threadIdx.x;
+    if (i < E + 2) partial[(int64_t)blockIdx.x * (E + 2) + i] = block_column<EP, G, WAVES>(red, i, E);
+    if (i < E) {
+        int32_t v = 0;
+#pragma unroll
+        for (int k = 0; k < WAVES; ++k) v += cred[k][i];
+        partial_counts[(int64_t)blockIdx.x * E + i] = v;
+        cnt[(int64_t)blockIdx.x * E + i] = v;
     }
 }
 
@@ -226,6 +283,28 @@ extern "C" int mts_router_wide_fwd(const void* x, const float* w_r, int64_t T, i
     if (act_dtype == MTS_BF16) wide_logits_kernel<bf16_t><<<grid, kLogitsThreads, 0, s>>>((const bf16_t*)x, w_r, T, H, E, logits);
     else if (act_dtype == MTS_F16) wide_logits_kernel<mts_f16_t><<<grid, kLogitsThreads, 0, s>>>((const mts_f16_t*)x, w_r, T, H, E, logits);
     else wide_logits_kernel<float><<<grid, kLogitsThreads, 0, s>>>((const float*)x, w_r, T, H, E, logits);
+    MTS_CHECK_LAUNCH();
+    return MTS_OK;
+}
+
+int mts_launch_wide_head(const void* x, const float* w_r, int64_t T, int H, int E, int K, int normalize, int act_dtype, float* logits, float* weights, int32_t* indices,
+                         void* weights_act, float* partial, int32_t* partial_counts, int32_t* cnt, hipStream_t s) {
+    const int rc = wide_check(x, w_r, T, H, E, act_dtype);
+    if (rc) return rc;
+    if (!logits || !weights || !indices) return MTS_ERR_NULL;
+    if (E > 64 || K < 1 || K > E || K > MTS_MAX_TOP_K) return MTS_ERR_SHAPE;
+    if (!mts_aligned16(logits)) return MTS_ERR_ALIGN;
+    const dim3 grid((unsigned)((T + MTS_WIDE_HEAD_ROWS - 1) / MTS_WIDE_HEAD_ROWS));
+    auto launch = [&](auto* kind) {
+        typedef typename std::remove_pointer<decltype(kind)>::type XT;
+        static_assert(WideTile<XT>::BM == MTS_WIDE_HEAD_ROWS, "rows of a chunk");
+        // as many lanes a row as the post-process kernel takes for as many experts
+        if (E > 32) wide_head_kernel<XT, 8><<<grid, kLogitsThreads, 0, s>>>((const XT*)x, w_r, T, H, E, K, normalize, logits, weights, indices, weights_act, act_dtype, partial, partial_counts, cnt);
+        else wide_head_kernel<XT, 4><<<grid, kLogitsThreads, 0, s>>>((const XT*)x, w_r, T, H, E, K, normalize, logits, weights, indices, weights_act, act_dtype, partial, partial_counts, cnt);
+    };
+    if (act_dtype == MTS_BF16) launch((bf16_t*)nullptr);
+    else if (act_dtype == MTS_F16) launch((mts_f16_t*)nullptr);
+    else launch((float*)nullptr);
     MTS_CHECK_LAUNCH();
     return MTS_OK;
 }

@@ -62,6 +62,9 @@ SIGNATURES = {
     "mts_moe_fwd_few_rows_preferred": (_i, [_i, _i, _l, _l, _i, _i, _i]),
     "mts_moe_fwd_few_rows": (_i, [_p, _p, _p, _i, _p, _p, _p, _p, _l, _i, _i, _i, _i, _i, _p, _p, _p, _p]),
     "mts_moe_combine": (_i, [_p, _p, _p, _p, _l, _i, _i, _i, _p, _p]),
+    "mts_moe_wide_head_supported": (_i, [_l, _i, _i, _i]),
+    "mts_moe_wide_head_workspace_bytes": (_l, [_l, _i]),
+    "mts_moe_wide_head_fwd": (_i, [_p, _p, _l, _i, _i, _i, _i, _i] + [_p] * 15 + [_l, _p]),
     "mts_moe_head_workspace_bytes": (_l, [_l, _i, _i]),
     "mts_moe_head_fwd": (_i, [_p, _p, _l, _i, _i, _i, _i, _i] + [_p] * 14 + [_p, _l, _p]),
     "mts_moe_head_bwd_workspace_bytes": (_l, [_l, _i, _i]),
