@@ -167,19 +167,19 @@ struct RowsParams {
                                // backward launch, or NULL: equal ranges
     int32_t* sched_out;        // dO*W2 launch: one more block writes the schedule of the joint backward launch here (NULL: none)
     float* part;               // EPI_SPLIT: the tile's place among the partial results
-    int sched_slots, sched_dx_cap;
+    int sched_slots, sched_dx_cap, sched_least;
 };
 
 // the schedule of the joint backward launch (defined with the weight-gradient GEMMs below)
 __device__ __forceinline__ void joint_schedule_wave(const int32_t* __restrict__ expert_start, int E, int slots, int dx_bm,
-                                                    int dx_cap, int32_t* __restrict__ sched);
+                                                    int dx_cap, int least, int32_t* __restrict__ sched);
 constexpr int kSchedDxRows = 256;   // rows of a dX tile of that launch (JointDxTile::BM)
 
 // The last block of a dO*W2 launch that was given a table writes the schedule: it needs nothing but expert_start,
 // and inside this launch it costs no time of its own.
 __device__ __forceinline__ bool schedule_block(const RowsParams& p) {
     if (p.sched_out == nullptr || blockIdx.x != gridDim.x - 1) return false;
-    if (threadIdx.x < MTS_WAVE) joint_schedule_wave(p.expert_start, p.E, p.sched_slots, kSchedDxRows, p.sched_dx_cap, p.sched_out);
+    if (threadIdx.x < MTS_WAVE) joint_schedule_wave(p.expert_start, p.E, p.sched_slots, kSchedDxRows, p.sched_dx_cap, p.sched_least, p.sched_out);
     return true;
 }
 
@@ -1663,6 +1663,7 @@ struct DwParams {
     Divider by_n_tiles, by_tiles;      // by n_tiles and tiles_per_expert
     const int32_t* sched;   // the unit table of the joint backward launch's schedule (which units an XCD runs), or NULL:
     int sched_slots;        // unit u runs on XCD u % 8; sched_slots: table entries per XCD
+    int least_share;        // the least rows that an expert is cut by (kLeastShare)
     int segment_rows;       // not 0: no experts, E segments of this many of the TK rows
     int p_pad;              // elements between the rows of P (0: dense), with a P that is read in place
 };
@@ -1671,7 +1672,7 @@ struct DwParams {
 // Row chunks of over-full experts.  A weight-gradient tile reduces over all rows of its
 // expert, so with skewed routing the tiles of the fullest expert set the kernel's time.
 // When the caller supplies a workspace, an expert with more than 1.15 times the balanced
-// share of rows (share = ceil(kept routes / E), rounded up to 32) is cut into
+// share of rows (share = ceil(kept routes / E), rounded up to 32; see dw_least_share) is cut into
 // ceil(count / share) chunks of equal length (a multiple of 32 rows).  A (expert, chunk)
 // pair is a unit; the units of an expert that was cut write fp32 tiles to the workspace,
 // slot by slot, and a second kernel adds the chunks of a tile in chunk order, so the result
@@ -1682,11 +1683,13 @@ struct DwUnit {
     int slot;            // index of the unit's partial tiles in the workspace, -1: writes C itself
 };
 
-__device__ __forceinline__ int dw_share_of(const int32_t* expert_start, int E) {
+__device__ __forceinline__ int dw_share_of(const int32_t* expert_start, int E, int least) {
     const int total = expert_start[E] - expert_start[0];   // the caller may pass a sub-range of the experts
-    return ((total + E - 1) / E + 31) / 32 * 32;
+    const int share = ((total + E - 1) / E + 31) / 32 * 32;
+    return share > least ? share : least;
 }
-__device__ __forceinline__ int dw_share(const DwParams& p) { return dw_share_of(p.expert_start, p.E); }
+constexpr int kSchedShare = 24;   // where the schedule of the joint backward launch keeps the share it was made with
+__device__ __forceinline__ int dw_share(const DwParams& p) { return p.sched ? p.sched[kSchedShare] : dw_share_of(p.expert_start, p.E, p.least_share); }
 
 // 1.15 shares: uniform routing stays far below it (the counts of 24576 tokens scatter by about 1 %), and at the uneven
 // routing of a trained router it beats 1.25 by 2-3 % of the layer step where an expert falls between the two
@@ -1753,7 +1756,7 @@ __device__ __forceinline__ bool locate_dw_unit(const DwParams& p, int unit, DwUn
 // weight-gradient unit 6 H I FLOPs (dW1 and dW2) and a dX tile 4 H I.  Which XCD computes a tile has no
 // influence on the tile's value: results are the same as with the round-robin deal, bit for bit.
 // Table (int32): [0,8) first dX m-tile of every XCD, [8,16) its number of m-tiles, [16,24) its number of
-// units, from kSchedUnits on (e, first row, end row, workspace slot) of unit k of XCD x at (x * slots + k) * 4.
+// units, [24] the share that experts were cut by, from kSchedUnits on (e, first row, end row, workspace slot) of unit k of XCD x at (x * slots + k) * 4.
 // ---------------------------------------------------------------------------
 constexpr int kSchedCounts = 16, kSchedUnits = 32;
 constexpr int kSchedMaxExperts = 32;          // one unit per lane: 2 E <= 64
@@ -1761,9 +1764,9 @@ constexpr int64_t kSchedBytes = 4096;         // (32 + 8 * 8 * 4) * 4 bytes are 
 // Called by one whole wave (lane = threadIdx.x % 64); E <= kSchedMaxExperts.  Units are cut as locate_dw_unit cuts
 // them when it has a workspace for the chunk partials.
 __device__ __forceinline__ void joint_schedule_wave(const int32_t* __restrict__ expert_start, int E, int slots, int dx_bm,
-                                                    int dx_cap, int32_t* __restrict__ sched) {
+                                                    int dx_cap, int least, int32_t* __restrict__ sched) {
     const int lane = threadIdx.x % MTS_WAVE;
-    const int share = dw_share_of(expert_start, E);
+    const int share = dw_share_of(expert_start, E, least);
     const int s0 = lane < E ? expert_start[lane] : 0, s1 = lane < E ? expert_start[lane + 1] : 0;
     const int nc = lane < E ? dw_chunks_cut(s1 - s0, share) : 0;
     const int ns = nc > 1 ? nc : 0;
@@ -1881,13 +1884,14 @@ __device__ __forceinline__ void joint_schedule_wave(const int32_t* __restrict__ 
             sched[kSchedCounts + x] = held[x];
             first += count[x];
         }
+        sched[kSchedShare] = share;
     }
 }
 
 // the schedule in a launch of its own (for a caller whose dO*W2 GEMM is not this library's)
 __global__ __launch_bounds__(MTS_WAVE) void joint_schedule_kernel(const int32_t* expert_start, int E, int slots, int dx_bm, int dx_cap,
                                                                     int32_t* sched) {
-    joint_schedule_wave(expert_start, E, slots, dx_bm, dx_cap, sched);
+    joint_schedule_wave(expert_start, E, slots, dx_bm, dx_cap, 0, sched);
 }
 
 // Adds the chunk partials of the experts that were cut: block `block` of `blocks`.  Only cut experts have pieces (a sixteenth of a tile, four
@@ -2834,6 +2838,23 @@ dim3 dw_grid(DwParams& p, int E, int units) {
     return dim3((unsigned)(((units + kXcds - 1) / kXcds) * kXcds * p.tiles_per_expert));
 }
 
+// Where the tiles of all experts are rounds of the chip anyway, none is cut by fewer than 256 rows: a tile costs 7.4 us besides 1.7 for 64 rows, so
+// that shorter chunks are more work and not less, and each writes and reads fp32 partial tiles on top.  (The layer's step of 64 experts of 1024/512, uneven routing, with
+// chunks from 1.15 shares on and now: 600 tokens 302 -> 235 us, 2500 tokens 494 -> 411; 24 of 2048/768, 1000 tokens 343 -> 284.)  With less than three rounds the longest tile is the launch's time, and chunks of any
+// length shorten it.
+constexpr int kLeastShare = 256;
+int dw_least_share(int E, int64_t H, int64_t I) {
+    typedef DwWsLarge T;
+    auto tiles = [](int64_t M, int64_t N) { return ((M + T::BM - 1) / T::BM) * ((N + T::BN - 1) / T::BN); };
+    return E * (tiles(2 * I, H) + tiles(H, I)) >= 3 * kXcds * kCusPerXcd ? kLeastShare : 0;
+}
+// Units of a launch that may cut: an expert of c rows makes at most c / share more of them than one, and one that is cut has more rows than a share.
+int dw_units(const DwParams& p, int E) {
+    if (!p.part) return E;
+    const int64_t more = p.least_share ? (p.TK + p.least_share - 1) / p.least_share : E;
+    return E + (int)(more < E ? more : E);
+}
+
 // fp32 tile partials of up to 2E row-chunk units (see DwUnit)
 int64_t dw_chunk_workspace_bytes(int E, int M, int N) {
     typedef DwWsLarge T;
@@ -2861,7 +2882,8 @@ int launch_dw_any(int kind, DwParams p, int E, int grad_dtype, void* workspace, 
             if (!mts_aligned16(workspace)) return MTS_ERR_ALIGN;
             p.part = (float*)workspace;
         }
-        const dim3 grid = dw_grid<T>(p, E, p.part ? 2 * E : E);
+        p.least_share = kind == K_DW1 ? dw_least_share(E, p.N, p.M / 2) : dw_least_share(E, p.M, p.N);
+        const dim3 grid = dw_grid<T>(p, E, dw_units(p, E));
         if (choice == 4) {
             if (grad_dtype == MTS_GEMM_DTYPE) dw_gemm_ws_kernel<DwWsWide, bf16_t><<<grid, T::NT, 0, s>>>(p);
             else dw_gemm_ws_kernel<DwWsWide, float><<<grid, T::NT, 0, s>>>(p);
@@ -2983,9 +3005,12 @@ int launch_bwd_joint(BwdJointParams q, int E, int grad_dtype, void* ws1, int64_t
         if (!mts_aligned16(ws2)) return MTS_ERR_ALIGN;
         q.dw2.part = (float*)ws2;
     }
-    q.n_dw1 = (int)dw_grid<T>(q.dw1, E, q.dw1.part ? 2 * E : E).x;
-    q.n_dw2 = (int)dw_grid<T>(q.dw2, E, q.dw2.part ? 2 * E : E).x;
     const bool own_dw2 = q.dw2.C != nullptr;
+    const bool scheduled = schedule && own_dw2 && q.dw1.part && q.dw2.part && E <= kSchedMaxExperts && mts_tuning().joint_schedule;
+    q.dw1.least_share = q.dw2.least_share = dw_least_share(E, q.dw1.N, q.dw1.M / 2);
+    // an XCD of the schedule is given up to twice its share of the units
+    q.n_dw1 = (int)dw_grid<T>(q.dw1, E, scheduled ? 2 * E : dw_units(q.dw1, E)).x;
+    q.n_dw2 = (int)dw_grid<T>(q.dw2, E, scheduled ? 2 * E : dw_units(q.dw2, E)).x;
     if (!own_dw2) {
         q.n_dw2 = 0;
         q.dw2.E = 0;
@@ -2996,7 +3021,7 @@ int launch_bwd_joint(BwdJointParams q, int E, int grad_dtype, void* ws1, int64_t
     q.n_dx = (int)(small_dx ? rows_grid<WsSmall, EPI_PLAIN>(q.dx, q.dx.TK) : rows_grid<JointDxTile, EPI_PLAIN>(q.dx, q.dx.TK)).x;
     // With both workspaces (row chunks on) and a schedule from the caller (written by the dO*W2 launch), units and dX
     // tiles go to the XCDs as the table says.
-    if (schedule && own_dw2 && q.dw1.part && q.dw2.part && E <= kSchedMaxExperts && mts_tuning().joint_schedule) {
+    if (scheduled) {
         if (!mts_aligned16(schedule)) return MTS_ERR_ALIGN;
         int slots, cap;
         schedule_shape(q.dx.TK, E, slots, cap);
@@ -3196,6 +3221,7 @@ extern "C" int MTS_GEMM_ENTRY(mts_moe_bwd_dy1)(const void* d_out, const void* w2
         if (!mts_aligned16(schedule)) return MTS_ERR_ALIGN;
         p.sched_out = schedule;
         schedule_shape(T * K, E, p.sched_slots, p.sched_dx_cap);
+        p.sched_least = dw_least_share(E, H, I);
     }
     if (!weighted_act) return launch_rows_any<EPI_DY1N>(K_DY1, p, T * K, (hipStream_t)stream, w2_as_stored != 0);
     return launch_rows_any<EPI_DY1>(K_DY1, p, T * K, (hipStream_t)stream, w2_as_stored != 0);
