@@ -582,6 +582,18 @@ int mts_attention_bwd(const MtsHeads* q, const MtsHeads* k, const MtsHeads* v, c
                       int causal, int act_dtype, const MtsHeads* dq, const MtsHeads* dk,
                       const MtsHeads* dv, float* delta, void* stream);
 
+/* The same between rotary encodings (mts_rope): the forward pass takes queries as they are and turned keys, turns the queries by the angles
+ * cos, sin [S,64] as it reads them and writes them to q_turned (NULL: nowhere); the backward pass takes both turned and returns gradients of what
+ * they were turned from, rounded once.                                                          */
+int mts_attention_turned_fwd(const MtsHeads* q, const MtsHeads* k_turned, const MtsHeads* v, const void* cos,
+                             const void* sin, int64_t B, int heads, int64_t S, int causal, int act_dtype,
+                             const MtsHeads* q_turned, const MtsHeads* out, float* lse, void* stream);
+int mts_attention_turned_bwd(const MtsHeads* q_turned, const MtsHeads* k_turned, const MtsHeads* v,
+                             const MtsHeads* out, const MtsHeads* d_out, const float* lse, const void* cos,
+                             const void* sin, int64_t B, int heads, int64_t S, int causal, int act_dtype,
+                             const MtsHeads* dq, const MtsHeads* dk, const MtsHeads* dv, float* delta,
+                             void* stream);
+
 /* ---- optimizer update (minitrain/train/trainer.py:85-159, minitrain/train/optim.py:30-47) ----
  * All tables are host arrays; the kernels take tensors of any size and alignment.
  *

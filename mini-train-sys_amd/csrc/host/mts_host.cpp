@@ -1149,6 +1149,76 @@ struct Attention : torch::autograd::Function<Attention> {
     }
 };
 
+// Rotary encoding and attention of a packed projection [B, S, 3 * heads * 64] as one node: the keys are turned by a launch of their own, the queries
+// where the attention reads them, and the gradients are turned back where it writes them, in place in the gradient of the projection.
+bool qkv_attention_supported(const Tensor& qkv, const Tensor& cos, const Tensor& sin, int64_t heads) {
+    if (!qkv_rope_supported(qkv, cos, sin, heads) || (qkv.scalar_type() != at::kBFloat16 && qkv.scalar_type() != at::kHalf)) return false;
+    if (!mts_attention_supported(qkv.size(0), heads, qkv.size(1), qkv.size(2) / (3 * heads)) || !aligned16(cos) || !aligned16(sin)) return false;
+    if (at::autocast::is_autocast_enabled(at::kCUDA) && at::autocast::get_autocast_dtype(at::kCUDA) != qkv.scalar_type()) return false;
+    return at::globalContext().userEnabledFlashSDP();
+}
+
+struct QkvAttention : torch::autograd::Function<QkvAttention> {
+    static MtsHeads view(const Tensor& t) { return {ptr(t), t.stride(0), t.stride(1), t.stride(2)}; }
+    // [B, heads, S, D] of queries, keys or values inside a packed projection
+    static MtsHeads part(const Tensor& packed, int which, int64_t heads, int64_t D) {
+        const int64_t S = packed.size(1), row = packed.size(2);
+        return {static_cast<char*>(ptr(packed)) + which * heads * D * packed.element_size(), S * row, D, row};
+    }
+    static Tensor forward(AutogradContext* ctx, const Tensor& qkv, const Tensor& cos, const Tensor& sin, int64_t heads, bool causal, bool backward) {   // dense16
+        const int64_t B = qkv.size(0), S = qkv.size(1), D = qkv.size(2) / (3 * heads);
+        Tensor k = heads_inside(qkv, B, heads, S, D), q = backward ? heads_inside(qkv, B, heads, S, D) : Tensor();
+        Tensor out = at::empty({B, S, heads * D}, qkv.options()), lse = f32({B * heads * S}, qkv);
+        launch_rope({{qkv.view({B, S, 3, heads, D}).select(2, 1).transpose(1, 2), k, TURN}}, cos, sin);
+        const MtsHeads vq = part(qkv, 0, heads, D), vk = view(k), vv = part(qkv, 2, heads, D), vo = {ptr(out), S * heads * D, D, heads * D};
+        const MtsHeads turned = backward ? view(q) : MtsHeads{};
+        check(mts_attention_turned_fwd(&vq, &vk, &vv, ptr(cos), ptr(sin), B, heads, S, causal, dtype_code(qkv), backward ? &turned : nullptr, &vo,
+                                       ptr_as<float>(lse), stream_of(qkv)),
+              "mts_attention_turned_fwd");
+        if (backward) {
+            ctx->save_for_backward({qkv, q, k, out, lse, cos, sin});
+            ctx->saved_data["heads"] = heads;
+            ctx->saved_data["causal"] = causal;
+        }
+        return out;
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        const variable_list s = ctx->get_saved_variables();
+        const Tensor &qkv = s[0], &q = s[1], &k = s[2], &cos = s[5], &sin = s[6];
+        c10::OptionalDeviceGuard guard(qkv.device());
+        const int64_t heads = ctx->saved_data["heads"].toInt(), B = qkv.size(0), S = qkv.size(1), D = qkv.size(2) / (3 * heads);
+        const bool causal = ctx->saved_data["causal"].toBool();
+        if (written_out(grads)) {   // attention in fp32, as its own node has it
+            auto head = [&](const Tensor& t) { return t.view({B, S, heads, D}).transpose(1, 2); };
+            const variable_list parts = qkv.chunk(3, -1);
+            auto turned = [&](const Tensor& t) {
+                const variable_list h = t.chunk(2, -1);
+                return t * cos + at::cat({-h[1], h[0]}, -1) * sin;
+            };
+            const double scale = 1.0 / std::sqrt((double)D);
+            const Tensor qf = turned(head(parts[0])).to(at::kFloat), kf = turned(head(parts[1])).to(at::kFloat), vf = head(parts[2]).to(at::kFloat);
+            const Tensor g = head(grads[0].contiguous()).to(at::kFloat);
+            Tensor score = at::matmul(qf, kf.transpose(2, 3).contiguous()) * scale;
+            if (causal) score = score.masked_fill(at::ones({S, S}, qkv.options().dtype(at::kBool)).triu(1), -INFINITY);
+            const Tensor p = at::softmax(score, -1), dp = at::matmul(g, vf.transpose(2, 3).contiguous());
+            const Tensor ds = p * (dp - (dp * p).sum(-1, true)) * scale;
+            auto back = [&](const Tensor& t, bool turn) { return (turn ? turned_back(t.to(qkv.scalar_type()), cos, sin) : t.to(qkv.scalar_type())).transpose(1, 2); };
+            const Tensor d = at::stack({back(at::matmul(ds, kf), true), back(at::matmul(ds.transpose(2, 3).contiguous(), qf), true),
+                                        back(at::matmul(p.transpose(2, 3).contiguous(), g), false)}, 2);
+            return {d.reshape(qkv.sizes()), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+        }
+        const Tensor g = dense16(grads[0]), d = at::empty_like(qkv);
+        Tensor delta = at::empty_like(s[4]);
+        const MtsHeads vq = view(q), vk = view(k), vv = part(qkv, 2, heads, D), rows = {ptr(s[3]), S * heads * D, D, heads * D};
+        const MtsHeads vg = {ptr(g), rows.batch_stride, rows.head_stride, rows.row_stride};
+        const MtsHeads dq = part(d, 0, heads, D), dk = part(d, 1, heads, D), dv = part(d, 2, heads, D);
+        check(mts_attention_turned_bwd(&vq, &vk, &vv, &rows, &vg, ptr_as<float>(s[4]), ptr(cos), ptr(sin), B, heads, S, causal, dtype_code(qkv), &dq, &dk, &dv,
+                                       ptr_as<float>(delta), stream_of(qkv)),
+              "mts_attention_turned_bwd");
+        return {d, Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+    }
+};
+
 constexpr int64_t kIgnoreIndex = -100;   // torch's default
 
 bool cross_entropy_supported(const Tensor& logits, const Tensor& targets) {
@@ -1501,6 +1571,11 @@ PYBIND11_MODULE(_host, m) {
     m.def("attention", [](const Tensor& q, const Tensor& k, const Tensor& v, bool causal) {
         c10::OptionalDeviceGuard guard(q.device());
         return Attention::apply(q, k, v, causal);
+    });
+    m.def("qkv_attention_supported", &qkv_attention_supported);
+    m.def("qkv_attention", [](const Tensor& qkv, const Tensor& cos, const Tensor& sin, int64_t heads, bool causal) {
+        c10::OptionalDeviceGuard guard(qkv.device());
+        return QkvAttention::apply(dense16(qkv), cos, sin, heads, causal, at::GradMode::is_enabled() && qkv.requires_grad());
     });
     m.def("layer_means_supported", &layer_means_supported);
     m.def("layer_means", [](const Groups& groups, int64_t differentiable) {

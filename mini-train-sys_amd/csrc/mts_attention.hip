@@ -13,6 +13,13 @@
 // batch 8: 31 us forward (79) and 121 backward (308); batch 24: 72 us (534 TFLOP/s; 168) and 304 (445 TFLOP/s of the seven
 // products that two separate kernels form, so that each gradient is summed by one block in a fixed order; 844).
 //
+// Between rotary encodings (the decoder's case) the queries are turned as they are read and the gradients turned back as they are written, straight into the
+// gradient of the packed projection: a launch that turned queries and one that turned gradients and copied those of the values go (24 x 12 heads x
+// 1024: 38 + 38 us), the keys keep theirs (20).  In turn the forward kernel takes 92 us where it took 78 (it leaves the turned queries for the
+// backward pass; 32 for 31 without, batch 8), dQ 102 for 100, dK/dV 127 for 130.  Results leave through LDS, a line by eight lanes: with 8-byte
+// pieces of 32 rows an instruction forward, dQ and dK/dV took 95, 116 and 144 us.  Training step of four layers 14.41 -> 14.27 ms, validation
+// pass of 8 x 1024 tokens through twelve 3.92 -> 3.90; passes of 800 tokens, which wait for the host, 512 -> 470 us, training steps 1.81 -> 1.69 ms.
+//
 // Error against fp64 (2-norm, bf16, 24 heads x 1024): output 2.0e-3, dQ 2.5e-3, dK 2.4e-3, dV 2.3e-3, the stock operator's to
 // three digits; likewise at 200 and 777 rows, for scores three times as far apart, and in fp16.
 #include "mts_common.h"
@@ -115,19 +122,91 @@ __device__ __forceinline__ typename Mma<ET>::frag narrowed(const f32x16& v, int 
     return f;
 }
 
-// transposed accumulators (64 x 32: two tiles) to the row of this lane's column
+// Four elements of a row in two registers.  A lane of a transposed accumulator holds elements 8 * i + 4 * (lane / 32) + 0..3 of the row of its column, the
+// lane 32 from it the other four of every eight; memory is asked in pieces of 16 bytes, of which a lane takes 16 * k + 8 * (lane / 32) + 0..7: twice
+// the bytes an instruction.
+typedef uint2 Quad;
+__device__ __forceinline__ void load_quads(const void* row, Quad (&q)[8]) {
+    const int lane = threadIdx.x % MTS_WAVE;
+    u32x4 v[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = *reinterpret_cast<const u32x4*>(static_cast<const char*>(row) + 32 * k + 16 * (lane / 32));
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {   // each half hands the other the quad that it has a place for
+        const auto x = __builtin_amdgcn_permlane32_swap(v[k][0], v[k][2], false, false), y = __builtin_amdgcn_permlane32_swap(v[k][1], v[k][3], false, false);
+        q[2 * k] = {x[0], y[0]}, q[2 * k + 1] = {x[1], y[1]};
+    }
+}
+
+// The 32 x 64 results of a wave go out through a tile of its own in LDS, where nothing is read any more: eight lanes then write a row, a whole line.
 template <typename ET>
-__device__ __forceinline__ void store_row(ET* row, const f32x16 (&acc)[2], float scale) {
+__device__ __forceinline__ void flush_rows(const ET* tile, ET* head, int64_t stride, int first, int S) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
     const int lane = threadIdx.x % MTS_WAVE;
 #pragma unroll
-    for (int dt = 0; dt < 2; ++dt)
+    for (int i = 0; i < 4; ++i) {
+        const int r = 8 * i + lane / 8;
+        if (first + r < S) *reinterpret_cast<u32x4*>(head + (first + r) * stride + lane % 8 * 8) = *reinterpret_cast<const u32x4*>(tile + chunk_off(r, lane % 8));
+    }
+}
+template <typename ET>
+__device__ __forceinline__ void put_quad(ET* tile, int i, typename Mma<ET>::quad v) {
+    const int lane = threadIdx.x % MTS_WAVE;
+    *reinterpret_cast<typename Mma<ET>::quad*>(tile + chunk_off(lane % 32, i) + 4 * (lane / 32)) = v;
+}
+// transposed accumulators (64 x 32: two tiles)
+template <typename ET>
+__device__ __forceinline__ void store_rows(ET* tile, ET* head, int64_t stride, int first, int S, const f32x16 (&acc)[2], float scale) {
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            typename Mma<ET>::quad o;
+    for (int i = 0; i < 8; ++i) {
+        typename Mma<ET>::quad o;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) o[r] = (ET)(acc[dt][4 * g + r] * scale);
-            *reinterpret_cast<typename Mma<ET>::quad*>(row + 32 * dt + 8 * g + 4 * (lane / 32)) = o;
+        for (int r = 0; r < 4; ++r) o[r] = (ET)(acc[i / 4][i % 4 * 4 + r] * scale);
+        put_quad<ET>(tile, i, o);
+    }
+    flush_rows(tile, head, stride, first, S);
+}
+
+// Rotary encoding (rope_kernel's pairs (d, d + 32) and its arithmetic) of a row that a lane holds as an operand: both elements of a pair are its own.
+// cos, sin: the row's angles.
+template <typename ET>
+__device__ __forceinline__ void turn(typename Mma<ET>::frag (&f)[4], const ET* cos, const ET* sin) {
+    typename Mma<ET>::frag c[4], s[4];
+    own_frags<ET>(cos, c);
+    own_frags<ET>(sin, s);
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const float x1 = (float)f[ks][j], x2 = (float)f[ks + 2][j];
+            f[ks][j] = difference_of_rounded_products<ET>(x1, (float)c[ks][j], x2, (float)s[ks][j]);
+            f[ks + 2][j] = sum_of_rounded_products<ET>(x2, (float)c[ks + 2][j], x1, (float)s[ks + 2][j]);
         }
+}
+// The same of a gradient turned back: in fp32, rounded once, on its way out.  cos, sin: the angles of the row of this lane's column.
+template <typename ET>
+__device__ __forceinline__ void store_rows_turned_back(ET* tile, ET* head, int64_t stride, int first, int S, const f32x16 (&acc)[2], float scale, const ET* cos,
+                                                       const ET* sin) {
+    typedef typename Mma<ET>::quad quad;
+    Quad c[8], s[8];
+    load_quads(cos, c);
+    load_quads(sin, s);
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+        const quad c1 = __builtin_bit_cast(quad, c[g]), c2 = __builtin_bit_cast(quad, c[g + 4]);
+        const quad s1 = __builtin_bit_cast(quad, s[g]), s2 = __builtin_bit_cast(quad, s[g + 4]);
+        quad o1, o2;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const float g1 = acc[0][4 * g + r] * scale, g2 = acc[1][4 * g + r] * scale;
+            o1[r] = (ET)fmaf(g1, (float)c1[r], g2 * (float)s2[r]);
+            o2[r] = (ET)fmaf(g2, (float)c2[r], -(g1 * (float)s1[r]));
+        }
+        put_quad<ET>(tile, g, o1);
+        put_quad<ET>(tile, g + 4, o2);
+    }
+    flush_rows(tile, head, stride, first, S);
 }
 
 // Blocks of one head on one XCD (its keys and values, or queries and gradients, are read by all of them); `order` counts the
@@ -151,13 +230,18 @@ template <typename ET>
 struct AttnArgs {
     Heads<const ET> q, k, v, o, dO;
     Heads<ET> out, dq, dk, dv;
+    // Rotary angles [S, 64], or NULL: the forward kernel then turns the queries on their way in (and leaves them in q_turned, where that is
+    // given), the backward kernels turn the gradients of queries and keys back on their way out.
+    const ET *cos, *sin;
+    Heads<ET> q_turned;
     float *lse, *delta;   // [BH, S]: log2 of the row's sum of exponentials; sum of dO * O
     int64_t BH;
     int heads, S, blocks;
     float scale;
 };
 
-template <typename ET, bool CAUSAL>
+// TURN: with rotary angles (AttnArgs::cos)
+template <typename ET, bool CAUSAL, bool TURN>
 __global__ __launch_bounds__(kThreads, 3) void attention_fwd_kernel(AttnArgs<ET> a) {
     typedef typename Mma<ET>::frag frag;
     __shared__ __align__(16) ET lds[2][2][kTileElems];
@@ -166,15 +250,19 @@ __global__ __launch_bounds__(kThreads, 3) void attention_fwd_kernel(AttnArgs<ET>
     const int lane = threadIdx.x % MTS_WAVE, wave = threadIdx.x / MTS_WAVE, half = lane / 32;
     const int S = a.S, q0 = (CAUSAL ? a.blocks - 1 - at.order : at.order) * kOwn, first = q0 + 32 * wave, row = first + lane % 32;
     const ET *k = a.k.row0(at.bh, a.heads), *v = a.v.row0(at.bh, a.heads);
+    TileCopy<ET> kc, vc;   // on their way before the queries are waited for
+    kc.fetch(k, a.k.s, 0, S);
+    vc.fetch(v, a.v.s, 0, S);
     frag q[4];
     own_frags<ET>(a.q.row0(at.bh, a.heads) + min(row, S - 1) * a.q.s, q);
+    if constexpr (TURN) {
+        const int64_t angle = (int64_t)min(row, S - 1) * kHead;
+        turn<ET>(q, a.cos + angle, a.sin + angle);
+    }
     const float sc = a.scale * kLog2e;
     float top = -INFINITY, sum = 0.f;
     f32x16 acc[2] = {};
     const int end = CAUSAL ? min(S, q0 + kOwn) : S, tiles = (end + kTile - 1) / kTile;
-    TileCopy<ET> kc, vc;
-    kc.fetch(k, a.k.s, 0, S);
-    vc.fetch(v, a.v.s, 0, S);
     kc.commit(lds[0][0]);
     vc.commit(lds[0][1]);
     __syncthreads();
@@ -236,14 +324,22 @@ __global__ __launch_bounds__(kThreads, 3) void attention_fwd_kernel(AttnArgs<ET>
         __syncthreads();
     }
     sum = lane_pair<32>(sum, LaneSum());
-    if (row >= S) return;
-    store_row(a.out.row0(at.bh, a.heads) + row * a.out.s, acc, 1.f / sum);
-    if (half == 0) a.lse[at.bh * S + row] = top * sc + log2f(sum);
+    ET* tile = &lds[0][0][0] + wave * 32 * kHead;   // the loop has ended with a barrier
+    store_rows(tile, a.out.row0(at.bh, a.heads), a.out.s, first, S, acc, 1.f / sum);
+    if constexpr (TURN) {   // here and not where they are turned: a tile's loads would be waited for behind these stores
+        if (a.q_turned.p) {
+            tile += kOwn * kHead;
+#pragma unroll
+            for (int ks = 0; ks < 4; ++ks) *reinterpret_cast<frag*>(tile + chunk_off(lane % 32, 2 * ks + half)) = q[ks];
+            flush_rows(tile, a.q_turned.row0(at.bh, a.heads), a.q_turned.s, first, S);
+        }
+    }
+    if (half == 0 && row < S) a.lse[at.bh * S + row] = top * sc + log2f(sum);
 }
 
-// dQ of 128 queries; also delta, which the other kernel reads.
-template <typename ET, bool CAUSAL>
-__global__ __launch_bounds__(kThreads, 2) void attention_dq_kernel(AttnArgs<ET> a) {
+// dQ of 128 queries; also delta, which the other kernel reads.  Three blocks a CU (at 171 registers and two of them 116 us for 102).
+template <typename ET, bool CAUSAL, bool TURN>
+__global__ __launch_bounds__(kThreads, 3) void attention_dq_kernel(AttnArgs<ET> a) {
     typedef typename Mma<ET>::frag frag;
     __shared__ __align__(16) ET lds[2][2][kTileElems];
     const Where at(a.BH);
@@ -315,11 +411,13 @@ __global__ __launch_bounds__(kThreads, 2) void attention_dq_kernel(AttnArgs<ET> 
         }
         __syncthreads();
     }
-    if (row < S) store_row(a.dq.row0(at.bh, a.heads) + row * a.dq.s, acc, a.scale);
+    ET *tile = &lds[0][0][0] + wave * 32 * kHead, *dq = a.dq.row0(at.bh, a.heads);
+    if constexpr (TURN) store_rows_turned_back(tile, dq, a.dq.s, first, S, acc, a.scale, a.cos + from * kHead, a.sin + from * kHead);
+    else store_rows(tile, dq, a.dq.s, first, S, acc, a.scale);
 }
 
 // dK and dV of 128 keys.
-template <typename ET, bool CAUSAL>
+template <typename ET, bool CAUSAL, bool TURN>
 __global__ __launch_bounds__(kThreads, 2) void attention_dkdv_kernel(AttnArgs<ET> a) {
     typedef typename Mma<ET>::frag frag;
     __shared__ __align__(16) ET lds[2][2][kTileElems];
@@ -402,9 +500,11 @@ __global__ __launch_bounds__(kThreads, 2) void attention_dkdv_kernel(AttnArgs<ET
         if (t + 1 < tiles) commit((t + 1) & 1);
         __syncthreads();
     }
-    if (row >= S) return;
-    store_row(a.dk.row0(at.bh, a.heads) + row * a.dk.s, dk, a.scale);
-    store_row(a.dv.row0(at.bh, a.heads) + row * a.dv.s, dv, 1.f);
+    ET *tile = &lds[0][0][0] + wave * 32 * kHead, *to = a.dk.row0(at.bh, a.heads);
+    store_rows(tile, a.dv.row0(at.bh, a.heads), a.dv.s, first, S, dv, 1.f);
+    tile += kOwn * kHead;
+    if constexpr (TURN) store_rows_turned_back(tile, to, a.dk.s, first, S, dk, a.scale, a.cos + from * kHead, a.sin + from * kHead);
+    else store_rows(tile, to, a.dk.s, first, S, dk, a.scale);
 }
 
 template <typename T>
@@ -438,29 +538,36 @@ AttnArgs<ET> attention_args(const MtsHeads* q, const MtsHeads* k, const MtsHeads
 template <typename ET>
 dim3 attention_grid(const AttnArgs<ET>& a) { return dim3((unsigned)((a.BH + 7) / 8 * 8 * a.blocks)); }
 
+#define MTS_ATTENTION_LAUNCH(KERNEL)                                                                  \
+    if (a.cos && causal) KERNEL<ET, true, true><<<attention_grid(a), kThreads, 0, st>>>(a);           \
+    else if (a.cos) KERNEL<ET, false, true><<<attention_grid(a), kThreads, 0, st>>>(a);               \
+    else if (causal) KERNEL<ET, true, false><<<attention_grid(a), kThreads, 0, st>>>(a);              \
+    else KERNEL<ET, false, false><<<attention_grid(a), kThreads, 0, st>>>(a);
+
 template <typename ET>
 int attention_fwd(const MtsHeads* q, const MtsHeads* k, const MtsHeads* v, int64_t B, int heads, int64_t S, int causal, const MtsHeads* out, float* lse,
-                  hipStream_t st) {
+                  const void* cos, const void* sin, const MtsHeads* q_turned, hipStream_t st) {
     AttnArgs<ET> a = attention_args<ET>(q, k, v, B, heads, S);
     a.out = heads_of<ET>(*out), a.lse = lse;
-    if (causal) attention_fwd_kernel<ET, true><<<attention_grid(a), kThreads, 0, st>>>(a);
-    else attention_fwd_kernel<ET, false><<<attention_grid(a), kThreads, 0, st>>>(a);
+    a.cos = (const ET*)cos, a.sin = (const ET*)sin;
+    if (q_turned) a.q_turned = heads_of<ET>(*q_turned);
+    MTS_ATTENTION_LAUNCH(attention_fwd_kernel)
     MTS_CHECK_LAUNCH();
     return MTS_OK;
 }
 
 template <typename ET>
 int attention_bwd(const MtsHeads* q, const MtsHeads* k, const MtsHeads* v, const MtsHeads* out, const MtsHeads* d_out, const float* lse, int64_t B,
-                  int heads, int64_t S, int causal, const MtsHeads* dq, const MtsHeads* dk, const MtsHeads* dv, float* delta, hipStream_t st) {
+                  int heads, int64_t S, int causal, const MtsHeads* dq, const MtsHeads* dk, const MtsHeads* dv, float* delta,
+                  const void* cos, const void* sin, hipStream_t st) {
     AttnArgs<ET> a = attention_args<ET>(q, k, v, B, heads, S);
+    a.cos = (const ET*)cos, a.sin = (const ET*)sin;
     a.o = heads_of<const ET>(*out), a.dO = heads_of<const ET>(*d_out);
     a.dq = heads_of<ET>(*dq), a.dk = heads_of<ET>(*dk), a.dv = heads_of<ET>(*dv);
     a.lse = const_cast<float*>(lse), a.delta = delta;
-    if (causal) attention_dq_kernel<ET, true><<<attention_grid(a), kThreads, 0, st>>>(a);
-    else attention_dq_kernel<ET, false><<<attention_grid(a), kThreads, 0, st>>>(a);
+    MTS_ATTENTION_LAUNCH(attention_dq_kernel)
     MTS_CHECK_LAUNCH();
-    if (causal) attention_dkdv_kernel<ET, true><<<attention_grid(a), kThreads, 0, st>>>(a);
-    else attention_dkdv_kernel<ET, false><<<attention_grid(a), kThreads, 0, st>>>(a);
+    MTS_ATTENTION_LAUNCH(attention_dkdv_kernel)
     MTS_CHECK_LAUNCH();
     return MTS_OK;
 }
@@ -472,21 +579,46 @@ extern "C" int mts_attention_supported(int64_t B, int heads, int64_t S, int head
     return (B * heads + 7) / 8 * 8 * ((S + kOwn - 1) / kOwn) * kThreads < (1LL << 32);
 }
 
+static int attention_fwd_any(const MtsHeads* q, const MtsHeads* k, const MtsHeads* v, int64_t B, int heads, int64_t S, int causal, int act_dtype, const MtsHeads* out,
+                             float* lse, const void* cos, const void* sin, const MtsHeads* q_turned, void* stream) {
+    const MtsHeads* all[] = {q, k, v, out, q_turned};
+    if (!lse) return MTS_ERR_NULL;
+    if (int e = attention_shape(all, q_turned ? 5 : 4, B, heads, S, act_dtype)) return e;
+    if (!mts_aligned16(cos) || !mts_aligned16(sin)) return MTS_ERR_ALIGN;
+    if (act_dtype == MTS_BF16) return attention_fwd<bf16_t>(q, k, v, B, heads, S, causal, out, lse, cos, sin, q_turned, (hipStream_t)stream);
+    return attention_fwd<mts_f16_t>(q, k, v, B, heads, S, causal, out, lse, cos, sin, q_turned, (hipStream_t)stream);
+}
+static int attention_bwd_any(const MtsHeads* q, const MtsHeads* k, const MtsHeads* v, const MtsHeads* out, const MtsHeads* d_out, const float* lse, int64_t B, int heads,
+                             int64_t S, int causal, int act_dtype, const MtsHeads* dq, const MtsHeads* dk, const MtsHeads* dv, float* delta, const void* cos,
+                             const void* sin, void* stream) {
+    const MtsHeads* all[] = {q, k, v, out, d_out, dq, dk, dv};
+    if (!lse || !delta) return MTS_ERR_NULL;
+    if (int e = attention_shape(all, 8, B, heads, S, act_dtype)) return e;
+    if (!mts_aligned16(cos) || !mts_aligned16(sin)) return MTS_ERR_ALIGN;
+    if (act_dtype == MTS_BF16) return attention_bwd<bf16_t>(q, k, v, out, d_out, lse, B, heads, S, causal, dq, dk, dv, delta, cos, sin, (hipStream_t)stream);
+    return attention_bwd<mts_f16_t>(q, k, v, out, d_out, lse, B, heads, S, causal, dq, dk, dv, delta, cos, sin, (hipStream_t)stream);
+}
+
 extern "C" int mts_attention_fwd(const MtsHeads* q, const MtsHeads* k, const MtsHeads* v, int64_t B, int heads, int64_t S, int causal, int act_dtype,
                                  const MtsHeads* out, float* lse, void* stream) {
-    const MtsHeads* all[] = {q, k, v, out};
-    if (!lse) return MTS_ERR_NULL;
-    if (int e = attention_shape(all, 4, B, heads, S, act_dtype)) return e;
-    if (act_dtype == MTS_BF16) return attention_fwd<bf16_t>(q, k, v, B, heads, S, causal, out, lse, (hipStream_t)stream);
-    return attention_fwd<mts_f16_t>(q, k, v, B, heads, S, causal, out, lse, (hipStream_t)stream);
+    return attention_fwd_any(q, k, v, B, heads, S, causal, act_dtype, out, lse, nullptr, nullptr, nullptr, stream);
 }
 
 extern "C" int mts_attention_bwd(const MtsHeads* q, const MtsHeads* k, const MtsHeads* v, const MtsHeads* out, const MtsHeads* d_out, const float* lse,
                                  int64_t B, int heads, int64_t S, int causal, int act_dtype, const MtsHeads* dq, const MtsHeads* dk, const MtsHeads* dv,
                                  float* delta, void* stream) {
-    const MtsHeads* all[] = {q, k, v, out, d_out, dq, dk, dv};
-    if (!lse || !delta) return MTS_ERR_NULL;
-    if (int e = attention_shape(all, 8, B, heads, S, act_dtype)) return e;
-    if (act_dtype == MTS_BF16) return attention_bwd<bf16_t>(q, k, v, out, d_out, lse, B, heads, S, causal, dq, dk, dv, delta, (hipStream_t)stream);
-    return attention_bwd<mts_f16_t>(q, k, v, out, d_out, lse, B, heads, S, causal, dq, dk, dv, delta, (hipStream_t)stream);
+    return attention_bwd_any(q, k, v, out, d_out, lse, B, heads, S, causal, act_dtype, dq, dk, dv, delta, nullptr, nullptr, stream);
+}
+
+extern "C" int mts_attention_turned_fwd(const MtsHeads* q, const MtsHeads* k_turned, const MtsHeads* v, const void* cos, const void* sin, int64_t B, int heads,
+                                        int64_t S, int causal, int act_dtype, const MtsHeads* q_turned, const MtsHeads* out, float* lse, void* stream) {
+    if (!cos || !sin) return MTS_ERR_NULL;
+    return attention_fwd_any(q, k_turned, v, B, heads, S, causal, act_dtype, out, lse, cos, sin, q_turned, stream);
+}
+
+extern "C" int mts_attention_turned_bwd(const MtsHeads* q_turned, const MtsHeads* k_turned, const MtsHeads* v, const MtsHeads* out, const MtsHeads* d_out,
+                                        const float* lse, const void* cos, const void* sin, int64_t B, int heads, int64_t S, int causal, int act_dtype,
+                                        const MtsHeads* dq, const MtsHeads* dk, const MtsHeads* dv, float* delta, void* stream) {
+    if (!cos || !sin) return MTS_ERR_NULL;
+    return attention_bwd_any(q_turned, k_turned, v, out, d_out, lse, B, heads, S, causal, act_dtype, dq, dk, dv, delta, cos, sin, stream);
 }

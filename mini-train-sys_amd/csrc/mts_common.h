@@ -100,6 +100,21 @@ __device__ __forceinline__ uint64_t lanemask_lt() {
     return (1ull << (threadIdx.x & 63)) - 1ull;
 }
 
+// round(a * b) + round(c * d), rounded, as separate elementwise operators leave them (contraction would drop the two conversions in between)
+template <typename ET>
+__device__ __forceinline__ ET sum_of_rounded_products(float a, float b, float c, float d) {
+#pragma clang fp contract(off)
+    const ET p = (ET)(a * b), q = (ET)(c * d);
+    return (ET)((float)p + (float)q);
+}
+
+template <typename ET>
+__device__ __forceinline__ ET difference_of_rounded_products(float a, float b, float c, float d) {
+#pragma clang fp contract(off)
+    const ET p = (ET)(a * b), q = (ET)(c * d);
+    return (ET)((float)p - (float)q);
+}
+
 static inline bool mts_aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 // fp16 instantiation of the grouped GEMMs (mts_gemm_f16.hip); the public entry points forward to it

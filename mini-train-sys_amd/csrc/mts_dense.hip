@@ -33,14 +33,6 @@ __device__ __forceinline__ ET rounded_sum(ET a, ET b) {
 #pragma clang fp contract(off)
     return (ET)((float)a + (float)b);
 }
-// round(a * b) + round(c * d)
-template <typename ET>
-__device__ __forceinline__ ET sum_of_rounded_products(float a, float b, float c, float d) {
-#pragma clang fp contract(off)
-    const ET p = (ET)(a * b), q = (ET)(c * d);
-    return (ET)((float)p + (float)q);
-}
-
 constexpr int kNormWaves = 4;
 constexpr int kNormThreads = kNormWaves * MTS_WAVE;
 

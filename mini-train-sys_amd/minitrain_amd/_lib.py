@@ -108,6 +108,8 @@ SIGNATURES = {
     "mts_attention_supported": (_i, [_l, _i, _l, _i]),
     "mts_attention_fwd": (_i, [_p, _p, _p, _l, _i, _l, _i, _i, _p, _p, _p]),
     "mts_attention_bwd": (_i, [_p, _p, _p, _p, _p, _p, _l, _i, _l, _i, _i, _p, _p, _p, _p, _p]),
+    "mts_attention_turned_fwd": (_i, [_p, _p, _p, _p, _p, _l, _i, _l, _i, _i, _p, _p, _p, _p]),
+    "mts_attention_turned_bwd": (_i, [_p, _p, _p, _p, _p, _p, _p, _p, _l, _i, _l, _i, _i, _p, _p, _p, _p, _p]),
     "mts_cross_entropy_bwd": (_i, [_p, _p, _l, _i, _l, _i, _p, _p, _p, _p, _p, _p]),
     "mts_layer_means": (_i, [_p, _p, _p, _p, _i, _p, _p]),
     "mts_scalar_sums": (_i, [_p, _i, _p, _p, _p, _p, _i, _p]),

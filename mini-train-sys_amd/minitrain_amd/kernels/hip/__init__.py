@@ -88,6 +88,13 @@ class HipOpsBackend(DenseTorchOps):
             return dense.attention(q, k, v, is_causal)
         return super().attention(q, k, v, is_causal=is_causal, dropout_p=dropout_p)
 
+    def qkv_attention(self, qkv, cos, sin, heads, *, is_causal, dropout_p):
+        """Extension: ``attention`` of what ``qkv_rope`` returns, as ``[B, S, heads * D]``, or None when the kernels do not take it or one of
+        the operators that it stands for is overridden."""
+        if dropout_p or not self._are_own(("rope", "qkv_rope", "attention")) or not dense.is_qkv_attention_supported(qkv, cos, sin, heads):
+            return None
+        return dense.qkv_attention(qkv, cos, sin, heads, is_causal)
+
     def cross_entropy(self, logits, targets):
         if dense.is_cross_entropy_supported(logits, targets):
             return dense.cross_entropy(logits, targets)
@@ -150,7 +157,7 @@ class HipOpsBackend(DenseTorchOps):
 
 _OF_LAYER = ("router_logits", "router_postprocess", "fused_moe")
 _OF_LIMITED_LAYER = (*_OF_LAYER, "capacity_mask")
-_OWN = {name: getattr(HipOpsBackend, name) for name in ("rmsnorm", "rope", *_OF_LIMITED_LAYER)}
+_OWN = {name: getattr(HipOpsBackend, name) for name in ("rmsnorm", "rope", "qkv_rope", "attention", *_OF_LIMITED_LAYER)}
 
 __all__ = [
     "HipOpsBackend",

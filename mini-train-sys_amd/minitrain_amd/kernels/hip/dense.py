@@ -79,6 +79,15 @@ def attention(q, k, v, is_causal: bool):
     return _lib.host().attention(q, k, v, is_causal)
 
 
+def is_qkv_attention_supported(qkv, cos, sin, heads: int) -> bool:
+    return _may_replace(qkv, cos, sin) and _lib.host().qkv_attention_supported(qkv, cos, sin, heads)
+
+
+def qkv_attention(qkv, cos, sin, heads: int, is_causal: bool):
+    """``attention(*qkv_rope(qkv, cos, sin, heads), is_causal)`` as ``[B, S, heads * D]``"""
+    return _lib.host().qkv_attention(qkv, cos, sin, heads, is_causal)
+
+
 def is_cross_entropy_supported(logits, targets) -> bool:
     return _may_replace(logits, targets) and _lib.host().cross_entropy_supported(logits, targets)
 

@@ -109,6 +109,11 @@ class CausalSelfAttention(nn.Module):
     def forward(self, x, ops: OpsBackend, rope_cos, rope_sin):
         B, S, H = x.shape
         qkv = project(self.qkv, x, ops)
+        dropout_p = self.p_drop if self.training else 0.0
+        whole = getattr(ops, "qkv_attention", None)
+        ctx = whole(qkv, rope_cos, rope_sin, self.n_heads, is_causal=True, dropout_p=dropout_p) if whole is not None else None
+        if ctx is not None:
+            return self.resid_dropout(project(self.out, ctx, ops))
         packed = getattr(ops, "qkv_rope", None)   # a backend may take the packed projection as it is
         turned = packed(qkv, rope_cos, rope_sin, self.n_heads) if packed is not None else None
         if turned is not None:
@@ -116,7 +121,7 @@ class CausalSelfAttention(nn.Module):
         else:
             q, k, v = (t.view(B, S, self.n_heads, self.head_dim).transpose(1, 2) for t in qkv.chunk(3, dim=-1))
             q, k = ops.rope(q, k, rope_cos, rope_sin)
-        ctx = ops.attention(q, k, v, is_causal=True, dropout_p=self.p_drop if self.training else 0.0)
+        ctx = ops.attention(q, k, v, is_causal=True, dropout_p=dropout_p)
         return self.resid_dropout(project(self.out, ctx.transpose(1, 2).reshape(B, S, H), ops))
 
 
