@@ -122,6 +122,13 @@ int mts_router_wide_bwd(const float* dlogits, const void* x, const float* w_r, i
                         int act_dtype, void* dx, float* d_w_r, void* workspace,
                         int64_t workspace_bytes, void* stream);
 
+/* n fp32 values of src rounded to a 16-bit activation dtype; n a multiple of 8, both 16-byte aligned. */
+typedef struct MtsCast {
+    const float* src;
+    void* dst;
+    int64_t n;
+} MtsCast;
+
 /* The head of a layer with 17 to 64 experts in three launches: projection chained to the post-process, scan, scatter.  As mts_router_wide_fwd
  * followed by mts_moe_router_route; T up to 32 768 (mts_moe_wide_head_supported).                 */
 int mts_moe_wide_head_supported(int64_t T, int H, int E, int K);
@@ -131,6 +138,11 @@ int mts_moe_wide_head_fwd(const void* x, const float* w_r, int64_t T, int H, int
                           float* prob_mean, float* z_loss, float* entropy, int32_t* counts, float* load_balance,
                           float* load_stats, int32_t* expert_start, int32_t* s_scatter, int32_t* s_reverse,
                           int32_t* x_gather, void* workspace, int64_t workspace_bytes, void* stream);
+int mts_moe_wide_head_cast_fwd(const void* x, const float* w_r, int64_t T, int H, int E, int K, int normalize,
+                          int act_dtype, float* logits, float* weights, int32_t* indices, void* weights_act,
+                          float* prob_mean, float* z_loss, float* entropy, int32_t* counts, float* load_balance,
+                          float* load_stats, int32_t* expert_start, int32_t* s_scatter, int32_t* s_reverse,
+                          int32_t* x_gather, void* workspace, int64_t workspace_bytes, const MtsCast* casts, void* stream);
 
 /* ---- the layer's head in two launches ---------------------------------------
  * mts_router_logits_fwd + mts_router_fwd + mts_moe_route as one chain (router projection,
@@ -150,6 +162,14 @@ int mts_moe_head_fwd(const void* x, const float* w_r, int64_t T, int H, int E, i
                      float* load_balance, float* load_stats, int32_t* expert_start, int32_t* s_scatter,
                      int32_t* s_reverse, int32_t* x_gather, void* workspace, int64_t workspace_bytes,
                      void* stream);
+/* With casts (two, or NULL), as mts_moe_cast_weights_pair: the first is made by further blocks of the first launch, the second by
+ * further blocks of the last, whose own blocks wait for memory most of their time.  act_dtype then is a 16-bit type.                  */
+int mts_moe_head_cast_fwd(const void* x, const float* w_r, int64_t T, int H, int E, int K, int normalize,
+                          int act_dtype, float* logits, float* weights, int32_t* indices, void* weights_act,
+                          float* prob_mean, float* z_loss, float* entropy, int32_t* counts,
+                          float* load_balance, float* load_stats, int32_t* expert_start, int32_t* s_scatter,
+                          int32_t* s_reverse, int32_t* x_gather, void* workspace, int64_t workspace_bytes,
+                          const MtsCast* casts, void* stream);
 
 /* mts_router_bwd chained into mts_router_logits_bwd: every block of the projection's backward
  * kernel first forms the logit gradients of its rows from the post-process's saved tensors

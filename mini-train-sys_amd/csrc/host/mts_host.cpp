@@ -335,25 +335,33 @@ struct Saved {
     Saved() = default;
 };
 
+// with few rows the kernels read the weights once and round fp32 ones themselves; a backward pass wants the rounded copies
+bool reads_masters(const Tensor& x, const Tensor& w1, const Tensor& w2, int64_t TK, const Options& opt) {
+    return w1.scalar_type() == at::kFloat && w2.scalar_type() == at::kFloat && x.scalar_type() != at::kFloat && opt.on(NO_BACKWARD) &&
+           mts_moe_fwd_few_rows_preferred(dtype_code(x), MTS_F32, x.size(0), TK, w1.size(0), x.size(1), w1.size(1) / 2);
+}
+// fp32 master weights are rounded together (the backward pass reuses the copies)
+bool copies_masters(const Tensor& x, const Tensor& w1, const Tensor& w2, int64_t TK, const Options& opt) {
+    return w1.scalar_type() == at::kFloat && w2.scalar_type() == at::kFloat && x.scalar_type() != at::kFloat && w1.numel() % 8 == 0 && w2.numel() % 8 == 0 &&
+           !reads_masters(x, w1, w2, TK, opt);
+}
+
 // Gate/up + SwiGLU, down projection and combine for routes that are already sorted.  `weights`: flat, activation dtype.
-// `post_act` [TK,I] and `y` [TK,H]: scratch that the caller has, or undefined
+// `post_act` [TK,I] and `y` [TK,H]: scratch that the caller has, or undefined; `w1`, `w2`: copies of master weights that the caller has made
 Tensor experts_forward(const Tensor& x, const Tensor& w1_in, const Tensor& w2_in, const Tensor& weights, const Routing& r, const Options& opt, Saved& s,
-                       Tensor post_act = Tensor(), Tensor y = Tensor()) {
+                       Tensor post_act = Tensor(), Tensor y = Tensor(), Tensor w1 = Tensor(), Tensor w2 = Tensor()) {
     const int64_t T = x.size(0), H = x.size(1), E = w1_in.size(0), I = w1_in.size(1) / 2, TK = weights.numel(), K = TK / T;
     const auto dtype = x.scalar_type();
     const int act = dtype_code(dtype);
     void* stream = stream_of(x);
     const bool weighted = opt.on(WEIGHTED_POST);
-    Tensor w1, w2;
-    // with few rows the kernels read the weights once and round fp32 ones themselves; a backward pass wants the rounded copies
-    const bool masters = w1_in.scalar_type() == at::kFloat && w2_in.scalar_type() == at::kFloat && dtype != at::kFloat;
-    const bool few_masters = masters && opt.on(NO_BACKWARD) && mts_moe_fwd_few_rows_preferred(act, MTS_F32, T, TK, E, H, I);
+    const bool few_masters = reads_masters(x, w1_in, w2_in, TK, opt);
     const bool few = few_masters || mts_moe_fwd_few_rows_preferred(act, act, T, TK, E, H, I);
     if (few_masters) {
         w1 = w1_in;
         w2 = w2_in;
-    } else if (masters && w1_in.numel() % 8 == 0 && w2_in.numel() % 8 == 0) {
-        // fp32 master weights: both casts in one launch (the backward pass reuses the copies)
+    } else if (w1.defined()) {
+    } else if (copies_masters(x, w1_in, w2_in, TK, opt)) {
         w1 = at::empty(w1_in.sizes(), x.options());
         w2 = at::empty(w2_in.sizes(), x.options());
         check(mts_moe_cast_weights_pair(ptr_as<float>(w1_in), ptr(w1), w1_in.numel(), ptr_as<float>(w2_in), ptr(w2), w2_in.numel(), act, stream),
@@ -686,12 +694,20 @@ LayerForward layer_forward(const Tensor& x_, const Tensor& w_r_, const Tensor& w
     }
     void* load_stats = limited ? nullptr : ptr(f.load_stats);
     void* cast_weights = narrow && !limited ? ptr(weights_act) : nullptr;
+    Tensor copy1, copy2;   // of master weights: made beside the head
     if (chained) {
-        check((few ? mts_moe_head_fwd : mts_moe_wide_head_fwd)(ptr(x), ptr_as<float>(w_r), T, H, E, K, normalize, dtype_code(x), ptr_as<float>(f.logits), ptr_as<float>(f.weights),
+        MtsCast casts[2];
+        const bool copied = copies_masters(x, w1, w2, TK, opt);
+        if (copied) {
+            copy1 = at::empty(w1.sizes(), x.options()), copy2 = at::empty(w2.sizes(), x.options());
+            casts[0] = {ptr_as<float>(w1), ptr(copy1), w1.numel()}, casts[1] = {ptr_as<float>(w2), ptr(copy2), w2.numel()};
+        }
+        check((few ? mts_moe_head_cast_fwd : mts_moe_wide_head_cast_fwd)(ptr(x), ptr_as<float>(w_r), T, H, E, K, normalize, dtype_code(x), ptr_as<float>(f.logits), ptr_as<float>(f.weights),
                                ptr_as<int32_t>(f.indices), cast_weights, ptr_as<float>(f.prob_mean), ptr_as<float>(f.z_loss), ptr_as<float>(f.entropy),
                                ptr_as<int32_t>(f.counts), ptr_as<float>(f.load_balance), static_cast<float*>(load_stats), ptr_as<int32_t>(r.expert_start),
-                               ptr_as<int32_t>(r.s_scatter), ptr_as<int32_t>(r.s_reverse), ptr_as<int32_t>(r.x_gather), ptr(ws), ws_bytes, stream_of(x)),
-              few ? "mts_moe_head_fwd" : "mts_moe_wide_head_fwd");
+                               ptr_as<int32_t>(r.s_scatter), ptr_as<int32_t>(r.s_reverse), ptr_as<int32_t>(r.x_gather), ptr(ws), ws_bytes,
+                               copied ? casts : nullptr, stream_of(x)),
+              few ? "mts_moe_head_cast_fwd" : "mts_moe_wide_head_cast_fwd");
     } else {
         router_projection_forward(x, w_r, f.logits);
         check(mts_moe_router_route(ptr_as<float>(f.logits), T, E, K, normalize, ptr_as<float>(f.weights), ptr_as<int32_t>(f.indices), ptr_as<float>(f.prob_mean),
@@ -721,7 +737,7 @@ LayerForward layer_forward(const Tensor& x_, const Tensor& w_r_, const Tensor& w
                                            E, normalize, dtype_code(x), ptr(weights_act), ptr_as<float>(f.load_stats), stream_of(x)),
               "mts_moe_capacity_weights_fwd");
     }
-    f.out = experts_forward(x, w1, w2, weights_act, r, opt, f.s, post_act, y);
+    f.out = experts_forward(x, w1, w2, weights_act, r, opt, f.s, post_act, y, copy1, copy2);
     return f;
 }
 

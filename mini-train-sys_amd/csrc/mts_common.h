@@ -200,7 +200,7 @@ int mts_launch_router_fwd(const float* logits, int64_t T, int E, int K, int norm
 #define MTS_WIDE_HEAD_ROWS 32
 #define MTS_WIDE_HEAD_CHUNKS 1024
 int mts_launch_wide_head(const void* x, const float* w_r, int64_t T, int H, int E, int K, int normalize, int act_dtype, float* logits, float* weights, int32_t* indices,
-                         void* weights_act, float* partial, int32_t* partial_counts, int32_t* cnt, hipStream_t s);
+                         void* weights_act, float* partial, int32_t* partial_counts, int32_t* cnt, const MtsCast* cast, hipStream_t s);
 // What the launch behind the head writes from partial and cnt.  Where the head is one block (up to 64 tokens) the block writes it itself:
 // *finished is 1 then, and partial and cnt are left as they are.
 struct MtsHeadFinish {
@@ -212,4 +212,4 @@ struct MtsHeadFinish {
 };
 int mts_launch_router_head(const void* x, const float* w_r, int64_t T, int H, int E, int K, int normalize, int act_dtype,
                            float* logits, float* weights, int32_t* indices, void* weights_act, float* partial,
-                           int32_t* cnt, MtsHeadFinish finish, int* finished, hipStream_t s);
+                           int32_t* cnt, MtsHeadFinish finish, int* finished, const MtsCast* cast, hipStream_t s);   // cast: more blocks of the launch, or NULL

@@ -13,6 +13,7 @@
 // A negative expert id marks a dropped route (capacity-limited dispatch): it is not
 // counted, gets no row, and its s_reverse entry is -1.  expert_start[E] is the number
 // of routes that were kept.
+#include "mts_cast_block.h"
 #include "mts_common.h"
 #include "mts_route_scatter.h"
 #include "mts_router_row.h"
@@ -159,13 +160,20 @@ __global__ __launch_bounds__(kScanThreads) void route_scan_kernel(
     route_scan_block(cnt, n_chunks, E, block_m, counts, expert_start, tile_row_start, tile_expert, tile_count, e0);
 }
 
+// a copy that rides in a launch of kThreads
+__device__ __forceinline__ void ride(const MtsCastJob& copy, int dtype) {
+    if (dtype == MTS_BF16) mts_cast::cast_block<bf16_t, kThreads>(copy.cast, blockIdx.x - copy.own_blocks);
+    else mts_cast::cast_block<mts_f16_t, kThreads>(copy.cast, blockIdx.x - copy.own_blocks);
+}
+
 // chunk_len entries per wave (a multiple of 64 is not required); the chunks are the ones the
 // counters in cnt were taken over
 // E: all experts; [e0, e0 + EW): the window of this pass (cnt is [chunk][EW], expert_start points at expert e0)
 __global__ __launch_bounds__(kThreads) void route_scatter_kernel(
     const int32_t* __restrict__ idx, int64_t TK, int K, int E, int e0, int EW, int chunk_len,
     const int32_t* __restrict__ cnt, const int32_t* __restrict__ expert_start, int32_t* __restrict__ s_scatter,
-    int32_t* __restrict__ s_reverse, int32_t* __restrict__ x_gather) {
+    int32_t* __restrict__ s_reverse, int32_t* __restrict__ x_gather, MtsCastJob copy, int cast_dtype) {
+    if (blockIdx.x >= copy.own_blocks) return ride(copy, cast_dtype);
     extern __shared__ int32_t lds[];  // [kWaves][E] next free row per expert
     const int wave = threadIdx.x / MTS_WAVE, lane = threadIdx.x % MTS_WAVE;
     const int64_t chunk = (int64_t)blockIdx.x * kWaves + wave;
@@ -193,9 +201,10 @@ __global__ __launch_bounds__(kThreads) void head_scatter_kernel(
     float inv_routes, float* __restrict__ prob_mean, float* __restrict__ z_loss, float* __restrict__ entropy,
     int32_t* __restrict__ counts, float* __restrict__ load_balance, float* __restrict__ load_stats,
     int32_t* __restrict__ expert_start, const int32_t* __restrict__ idx, int64_t TK, int K, int chunk_len,
-    int32_t* __restrict__ s_scatter, int32_t* __restrict__ s_reverse, int32_t* __restrict__ x_gather) {
+    int32_t* __restrict__ s_scatter, int32_t* __restrict__ s_reverse, int32_t* __restrict__ x_gather, MtsCastJob copy, int cast_dtype) {
+    if (blockIdx.x >= copy.own_blocks) return ride(copy, cast_dtype);
     const int wave = threadIdx.x / MTS_WAVE, lane = threadIdx.x % MTS_WAVE;
-    if (blockIdx.x + 1 < gridDim.x) {
+    if (blockIdx.x + 1 < copy.own_blocks) {
         __shared__ int32_t next_rows[kWaves][kFinishMaxE];
         __shared__ int32_t sums[kWaves][2 * kFinishMaxE];
         static_assert(kFinishChunks == 2 * kThreads, "two chunks per thread");
@@ -343,7 +352,7 @@ int route_launch(const int32_t* top_k_index, int64_t T, int K, int E, int block_
         MTS_CHECK_LAUNCH();
         if (!permute) continue;
         route_scatter_kernel<<<grid, kThreads, lds, s>>>(top_k_index, TK, K, E, e0, EW, kChunk, cnt, expert_start + e0,
-                                                         s_scatter, s_reverse, x_gather);
+                                                         s_scatter, s_reverse, x_gather, mts_cast::job(nullptr, (unsigned)grid), 0);
         MTS_CHECK_LAUNCH();
     }
     return MTS_OK;
@@ -452,29 +461,51 @@ extern "C" int64_t mts_moe_wide_head_workspace_bytes(int64_t T, int E) {
     return (chunks * (3 * E + 2) + E) * (int64_t)sizeof(int32_t);   // statistics, routes for them, routes for the scan; the scan's totals
 }
 
-extern "C" int mts_moe_wide_head_fwd(const void* x, const float* w_r, int64_t T, int H, int E, int K, int normalize, int act_dtype, float* logits, float* weights,
+static int check_casts(const MtsCast* casts, int act_dtype) {
+    if (!casts) return MTS_OK;
+    if (act_dtype == MTS_F32) return MTS_ERR_DTYPE;
+    for (int i = 0; i < 2; ++i) {
+        if (!casts[i].src || !casts[i].dst) return MTS_ERR_NULL;
+        if (casts[i].n < 8 || casts[i].n % 8 || casts[i].n >= (1LL << 36)) return MTS_ERR_SHAPE;   // 2^36 values: 2^31 threads
+        if (!mts_aligned16(casts[i].src) || !mts_aligned16(casts[i].dst)) return MTS_ERR_ALIGN;
+    }
+    return MTS_OK;
+}
+
+extern "C" int mts_moe_wide_head_cast_fwd(const void* x, const float* w_r, int64_t T, int H, int E, int K, int normalize, int act_dtype, float* logits, float* weights,
                                      int32_t* indices, void* weights_act, float* prob_mean, float* z_loss, float* entropy, int32_t* counts, float* load_balance,
                                      float* load_stats, int32_t* expert_start, int32_t* s_scatter, int32_t* s_reverse, int32_t* x_gather, void* workspace,
-                                     int64_t workspace_bytes, void* stream) {
+                                     int64_t workspace_bytes, const MtsCast* casts, void* stream) {
     if (!prob_mean || !z_loss || !entropy || !counts || !expert_start || !s_scatter || !s_reverse || !x_gather || !workspace) return MTS_ERR_NULL;
     if (weights_act && act_dtype == MTS_F32) return MTS_ERR_DTYPE;
     if (!mts_moe_wide_head_supported(T, H, E, K)) return MTS_ERR_SHAPE;
     if (workspace_bytes < mts_moe_wide_head_workspace_bytes(T, E)) return MTS_ERR_WORKSPACE;
     if (!mts_aligned16(workspace)) return MTS_ERR_ALIGN;
+    if (const int rc = check_casts(casts, act_dtype)) return rc;
     hipStream_t s = (hipStream_t)stream;
     const int64_t chunks = (T + MTS_WIDE_HEAD_ROWS - 1) / MTS_WIDE_HEAD_ROWS;
     float* partial = (float*)workspace;
     int32_t *partial_counts = (int32_t*)(partial + chunks * (E + 2)), *cnt = partial_counts + chunks * E, *totals = cnt + chunks * E;
-    const int rc = mts_launch_wide_head(x, w_r, T, H, E, K, normalize, act_dtype, logits, weights, indices, weights_act, partial, partial_counts, cnt, s);
+    const int rc = mts_launch_wide_head(x, w_r, T, H, E, K, normalize, act_dtype, logits, weights, indices, weights_act, partial, partial_counts, cnt, casts, s);
     if (rc) return rc;
     const MtsRouterStats stats = {partial, partial_counts, (int)chunks, E, 1.0f / (float)T, 1.0f / ((float)T * (float)K), prob_mean, z_loss, entropy, counts,
                                   load_balance, load_stats};
     route_scan_kernel<<<2, kScanThreads, 0, s>>>(cnt, chunks, E, 64, totals, expert_start, nullptr, nullptr, nullptr, 0, stats);
     MTS_CHECK_LAUNCH();
-    route_scatter_kernel<<<dim3((unsigned)((chunks + kWaves - 1) / kWaves)), kThreads, (size_t)kWaves * E * sizeof(int32_t), s>>>(
-        indices, T * K, K, E, 0, E, MTS_WIDE_HEAD_ROWS * K, cnt, expert_start, s_scatter, s_reverse, x_gather);
+    const MtsCast* second = casts ? casts + 1 : nullptr;
+    const unsigned blocks = (unsigned)((chunks + kWaves - 1) / kWaves);
+    route_scatter_kernel<<<dim3((unsigned)(blocks + mts_cast::blocks(second, kThreads))), kThreads, (size_t)kWaves * E * sizeof(int32_t), s>>>(
+        indices, T * K, K, E, 0, E, MTS_WIDE_HEAD_ROWS * K, cnt, expert_start, s_scatter, s_reverse, x_gather, mts_cast::job(second, blocks), act_dtype);
     MTS_CHECK_LAUNCH();
     return MTS_OK;
+}
+
+extern "C" int mts_moe_wide_head_fwd(const void* x, const float* w_r, int64_t T, int H, int E, int K, int normalize, int act_dtype, float* logits, float* weights,
+                                     int32_t* indices, void* weights_act, float* prob_mean, float* z_loss, float* entropy, int32_t* counts, float* load_balance,
+                                     float* load_stats, int32_t* expert_start, int32_t* s_scatter, int32_t* s_reverse, int32_t* x_gather, void* workspace,
+                                     int64_t workspace_bytes, void* stream) {
+    return mts_moe_wide_head_cast_fwd(x, w_r, T, H, E, K, normalize, act_dtype, logits, weights, indices, weights_act, prob_mean, z_loss, entropy, counts, load_balance,
+                                      load_stats, expert_start, s_scatter, s_reverse, x_gather, workspace, workspace_bytes, nullptr, stream);
 }
 
 extern "C" int64_t mts_moe_head_workspace_bytes(int64_t T, int K, int E) {
@@ -483,37 +514,53 @@ extern "C" int64_t mts_moe_head_workspace_bytes(int64_t T, int K, int E) {
     return (int64_t)MTS_HEAD_MAX_CHUNKS * (2 * E + 2) * (int64_t)sizeof(float);   // statistics partials, then route counts
 }
 
-extern "C" int mts_moe_head_fwd(const void* x, const float* w_r, int64_t T, int H, int E, int K, int normalize,
+extern "C" int mts_moe_head_cast_fwd(const void* x, const float* w_r, int64_t T, int H, int E, int K, int normalize,
                                 int act_dtype, float* logits, float* weights, int32_t* indices, void* weights_act,
                                 float* prob_mean, float* z_loss, float* entropy, int32_t* counts, float* load_balance,
                                 float* load_stats, int32_t* expert_start, int32_t* s_scatter, int32_t* s_reverse,
-                                int32_t* x_gather, void* workspace, int64_t workspace_bytes, void* stream) {
+                                int32_t* x_gather, void* workspace, int64_t workspace_bytes, const MtsCast* casts, void* stream) {
     if (!prob_mean || !z_loss || !entropy || !counts || !expert_start || !s_scatter || !s_reverse || !x_gather || !workspace)
         return MTS_ERR_NULL;
     if (weights_act && act_dtype == MTS_F32) return MTS_ERR_DTYPE;
     if (T <= 0 || K < 1 || T * (int64_t)K > 0x7fffffffLL) return MTS_ERR_SHAPE;
     if (workspace_bytes < mts_moe_head_workspace_bytes(T, K, E)) return MTS_ERR_WORKSPACE;
     if (!mts_aligned16(workspace)) return MTS_ERR_ALIGN;
+    if (const int rc = check_casts(casts, act_dtype)) return rc;
     hipStream_t s = (hipStream_t)stream;
     float* partial = (float*)workspace;
     int32_t* cnt = (int32_t*)(partial + (int64_t)MTS_HEAD_MAX_CHUNKS * (E + 2));
     // the rows of one block are scattered, and its statistics completed, by the block itself
     const MtsHeadFinish finish = {1.0f / (float)T, 1.0f / ((float)T * (float)K), prob_mean, z_loss, entropy, counts, load_balance, load_stats,
                                   expert_start, s_scatter, s_reverse, x_gather};
-    int finished = 0;
-    const int rc = mts_launch_router_head(x, w_r, T, H, E, K, normalize, act_dtype, logits, weights, indices, weights_act,
-                                          partial, cnt, finish, &finished, s);
-    if (rc || finished) return rc;
     int blocks, rows_per_wave;
     mts_router_head_geometry(T, mts_router_head_group(H, E, act_dtype), &blocks, &rows_per_wave);
+    if (casts && blocks == 1) {   // no second launch to ride in
+        const int rc = mts_moe_cast_weights_pair(casts[0].src, casts[0].dst, casts[0].n, casts[1].src, casts[1].dst, casts[1].n, act_dtype, stream);
+        if (rc) return rc;
+        casts = nullptr;
+    }
+    int finished = 0;
+    const int rc = mts_launch_router_head(x, w_r, T, H, E, K, normalize, act_dtype, logits, weights, indices, weights_act,
+                                          partial, cnt, finish, &finished, casts, s);
+    if (rc || finished) return rc;
     const int64_t rows_per_chunk = (int64_t)rows_per_wave * 4;
     const int64_t n_chunks = (T + rows_per_chunk - 1) / rows_per_chunk;
     if (n_chunks > kFinishChunks || E > kFinishMaxE) return MTS_ERR_SHAPE;   // cannot happen: the geometry caps the chunks, the projection E
     const int grid = (int)((n_chunks + kWaves - 1) / kWaves) + 1;   // scatter blocks, then the block that reduces
-    head_scatter_kernel<<<grid, kThreads, 0, s>>>(partial, cnt, (int)n_chunks, E, 1.0f / (float)T,
+    const MtsCast* second = casts ? casts + 1 : nullptr;
+    head_scatter_kernel<<<dim3((unsigned)(grid + mts_cast::blocks(second, kThreads))), kThreads, 0, s>>>(partial, cnt, (int)n_chunks, E, 1.0f / (float)T,
                                                   1.0f / ((float)T * (float)K), prob_mean, z_loss, entropy, counts,
                                                   load_balance, load_stats, expert_start, indices, T * (int64_t)K, K,
-                                                  (int)(rows_per_chunk * K), s_scatter, s_reverse, x_gather);
+                                                  (int)(rows_per_chunk * K), s_scatter, s_reverse, x_gather, mts_cast::job(second, (unsigned)grid), act_dtype);
     MTS_CHECK_LAUNCH();
     return MTS_OK;
+}
+
+extern "C" int mts_moe_head_fwd(const void* x, const float* w_r, int64_t T, int H, int E, int K, int normalize,
+                                int act_dtype, float* logits, float* weights, int32_t* indices, void* weights_act,
+                                float* prob_mean, float* z_loss, float* entropy, int32_t* counts, float* load_balance,
+                                float* load_stats, int32_t* expert_start, int32_t* s_scatter, int32_t* s_reverse,
+                                int32_t* x_gather, void* workspace, int64_t workspace_bytes, void* stream) {
+    return mts_moe_head_cast_fwd(x, w_r, T, H, E, K, normalize, act_dtype, logits, weights, indices, weights_act, prob_mean, z_loss, entropy, counts, load_balance,
+                                 load_stats, expert_start, s_scatter, s_reverse, x_gather, workspace, workspace_bytes, nullptr, stream);
 }

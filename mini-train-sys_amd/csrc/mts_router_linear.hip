@@ -3,6 +3,7 @@
 // copy of the activations is made; every sum runs in a fixed order (no float atomics).
 // 2*T*H*E FLOP forward, twice that backward: the backward kernels and the forward ones for fp16 / fp32 rows
 // run them on the vector pipe; bf16 rows with up to 8 experts take the forward product to the matrix pipe.
+#include "mts_cast_block.h"
 #include "mts_common.h"
 #include "mts_route_scatter.h"
 #include "mts_router_row.h"
@@ -401,8 +402,11 @@ template <typename XT, int EP, int PASSES, bool CHUNKED = false, bool MMA = fals
 __global__ __launch_bounds__(kFwdThreads, MMA ? 2 : 1) void router_head_kernel(
     const XT* __restrict__ x, const float* __restrict__ w, int64_t T, int H, int E, int K, int normalize,
     int rows_per_wave, int n_chunks, float* __restrict__ logits, float* __restrict__ weights, int32_t* __restrict__ indices,
-    void* __restrict__ weights_act, int act_dtype, float* __restrict__ partial, int32_t* __restrict__ cnt, MtsHeadFinish finish) {
+    void* __restrict__ weights_act, int act_dtype, float* __restrict__ partial, int32_t* __restrict__ cnt, MtsHeadFinish finish, MtsCastJob copy) {
     using namespace mts_router;
+    if constexpr (sizeof(XT) == 2) {
+        if (blockIdx.x >= copy.own_blocks) return mts_cast::cast_block<XT, kFwdThreads>(copy.cast, blockIdx.x - copy.own_blocks);
+    }
     static_assert(!MMA || (EP == 8 && sizeof(XT) == 2 && !CHUNKED), "the matrix-pipe projection: bf16 rows, up to 8 experts");
     extern __shared__ __attribute__((aligned(16))) float w_lds[];   // [E][H] fp32, or the bf16 terms of the matrix-pipe path
     constexpr int WAVES = kFwdThreads / MTS_WAVE;
@@ -752,14 +756,15 @@ void mts_router_head_geometry(int64_t T, int group, int* blocks, int* rows_per_w
 
 int mts_launch_router_head(const void* x, const float* w_r, int64_t T, int H, int E, int K, int normalize, int act_dtype,
                            float* logits, float* weights, int32_t* indices, void* weights_act, float* partial,
-                           int32_t* cnt, MtsHeadFinish finish, int* finished, hipStream_t s) {
+                           int32_t* cnt, MtsHeadFinish finish, int* finished, const MtsCast* cast, hipStream_t s) {
     const int rc = check(x, w_r, T, H, E, act_dtype);
     if (rc != MTS_OK) return rc;
     if (!logits || !weights || !indices || !partial || !cnt) return MTS_ERR_NULL;
     if (K < 1 || K > E || K > MTS_MAX_TOP_K) return MTS_ERR_SHAPE;
     int blocks, rows_per_wave;
     mts_router_head_geometry(T, mts_router_head_group(H, E, act_dtype), &blocks, &rows_per_wave);
-    const dim3 grid((unsigned)blocks);
+    const dim3 grid((unsigned)(blocks + mts_cast::blocks(cast, kFwdThreads)));
+    const MtsCastJob copy = mts_cast::job(cast, (unsigned)blocks);
     *finished = blocks == 1;
     if (blocks != 1) finish.expert_start = nullptr;
     if (mma_projection_ok(H, E, act_dtype)) {
@@ -767,7 +772,7 @@ int mts_launch_router_head(const void* x, const float* w_r, int64_t T, int H, in
         if (allow_lds(router_head_kernel<bf16_t, 8, 1, false, true>, bytes, 20 * 1024) != hipSuccess) return MTS_ERR_SHAPE;
         router_head_kernel<bf16_t, 8, 1, false, true><<<grid, kFwdThreads, bytes, s>>>(
             (const bf16_t*)x, w_r, T, H, E, K, normalize, rows_per_wave, 1, logits, weights, indices, weights_act, MTS_BF16,
-            partial, cnt, finish);
+            partial, cnt, finish, copy);
         MTS_CHECK_LAUNCH();
         return MTS_OK;
     }
@@ -780,7 +785,7 @@ int mts_launch_router_head(const void* x, const float* w_r, int64_t T, int H, in
         if (allow_lds(router_head_kernel<XT, EP, PS, CH>, lds, 20 * 1024) != hipSuccess) return MTS_ERR_SHAPE;                   \
         router_head_kernel<XT, EP, PS, CH><<<grid, kFwdThreads, lds, s>>>((const XT*)x, w_r, T, H, E, K, normalize,   \
                                                                           rows_per_wave, n_chunks, logits, weights, indices, \
-                                                                          weights_act, wa_dtype, partial, cnt, finish); \
+                                                                          weights_act, wa_dtype, partial, cnt, finish, copy); \
     } while (0)
 #define MTS_HEAD_PASSES(XT, EP)                           \
     do {                                                  \

@@ -9,6 +9,7 @@
 // the blocks of either fill the CUs that the other leaves.  Loads never depend on a branch (mts_f32_tiles.h).
 // 8192 x 1024, 64 experts, bf16: 15.8 us forward, 29 + 5.5 backward; 22 and 19 + 17 + 6 with branches at the loads, four waves, 2-byte stores
 // of dx and a launch each.  16 384 x 2048, 128 experts: 124 -> 95 and 210 -> 188.
+#include "mts_cast_block.h"
 #include "mts_f32_tiles.h"
 #include "mts_router_row.h"
 
@@ -107,8 +108,11 @@ template <typename XT, int G>
 __global__ __launch_bounds__(kLogitsThreads) void wide_head_kernel(const XT* __restrict__ x, const float* __restrict__ w, int64_t T, int H, int E, int K, int normalize,
                                                                    float* __restrict__ logits, float* __restrict__ weights, int32_t* __restrict__ indices,
                                                                    void* __restrict__ weights_act, int act_dtype, float* __restrict__ partial,
-                                                                   int32_t* __restrict__ partial_counts, int32_t* __restrict__ cnt) {
+                                                                   int32_t* __restrict__ partial_counts, int32_t* __restrict__ cnt, MtsCastJob copy) {
     using namespace mts_router;
+    if constexpr (sizeof(XT) == 2) {
+        if (blockIdx.x >= copy.own_blocks) return mts_cast::cast_block<XT, kLogitsThreads>(copy.cast, blockIdx.x - copy.own_blocks);
+    }
     typedef WideTile<XT> Tile;
     constexpr int EP = 8, WAVES = Tile::BM * G / MTS_WAVE, LROW = 72;   // a row's lanes and the rows of a wave fall on different banks
     __shared__ __attribute__((aligned(16))) float lds[Tile::LDS];
@@ -288,19 +292,21 @@ extern "C" int mts_router_wide_fwd(const void* x, const float* w_r, int64_t T, i
 }
 
 int mts_launch_wide_head(const void* x, const float* w_r, int64_t T, int H, int E, int K, int normalize, int act_dtype, float* logits, float* weights, int32_t* indices,
-                         void* weights_act, float* partial, int32_t* partial_counts, int32_t* cnt, hipStream_t s) {
+                         void* weights_act, float* partial, int32_t* partial_counts, int32_t* cnt, const MtsCast* cast, hipStream_t s) {
     const int rc = wide_check(x, w_r, T, H, E, act_dtype);
     if (rc) return rc;
     if (!logits || !weights || !indices) return MTS_ERR_NULL;
     if (E > 64 || K < 1 || K > E || K > MTS_MAX_TOP_K) return MTS_ERR_SHAPE;
     if (!mts_aligned16(logits)) return MTS_ERR_ALIGN;
-    const dim3 grid((unsigned)((T + MTS_WIDE_HEAD_ROWS - 1) / MTS_WIDE_HEAD_ROWS));
+    const unsigned blocks = (unsigned)((T + MTS_WIDE_HEAD_ROWS - 1) / MTS_WIDE_HEAD_ROWS);
+    const dim3 grid((unsigned)(blocks + mts_cast::blocks(cast, kLogitsThreads)));
+    const MtsCastJob copy = mts_cast::job(cast, blocks);
     auto launch = [&](auto* kind) {
         typedef typename std::remove_pointer<decltype(kind)>::type XT;
         static_assert(WideTile<XT>::BM == MTS_WIDE_HEAD_ROWS, "rows of a chunk");
         // as many lanes a row as the post-process kernel takes for as many experts
-        if (E > 32) wide_head_kernel<XT, 8><<<grid, kLogitsThreads, 0, s>>>((const XT*)x, w_r, T, H, E, K, normalize, logits, weights, indices, weights_act, act_dtype, partial, partial_counts, cnt);
-        else wide_head_kernel<XT, 4><<<grid, kLogitsThreads, 0, s>>>((const XT*)x, w_r, T, H, E, K, normalize, logits, weights, indices, weights_act, act_dtype, partial, partial_counts, cnt);
+        if (E > 32) wide_head_kernel<XT, 8><<<grid, kLogitsThreads, 0, s>>>((const XT*)x, w_r, T, H, E, K, normalize, logits, weights, indices, weights_act, act_dtype, partial, partial_counts, cnt, copy);
+        else wide_head_kernel<XT, 4><<<grid, kLogitsThreads, 0, s>>>((const XT*)x, w_r, T, H, E, K, normalize, logits, weights, indices, weights_act, act_dtype, partial, partial_counts, cnt, copy);
     };
     if (act_dtype == MTS_BF16) launch((bf16_t*)nullptr);
     else if (act_dtype == MTS_F16) launch((mts_f16_t*)nullptr);

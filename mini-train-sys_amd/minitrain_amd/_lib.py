@@ -65,8 +65,10 @@ SIGNATURES = {
     "mts_moe_wide_head_supported": (_i, [_l, _i, _i, _i]),
     "mts_moe_wide_head_workspace_bytes": (_l, [_l, _i]),
     "mts_moe_wide_head_fwd": (_i, [_p, _p, _l, _i, _i, _i, _i, _i] + [_p] * 15 + [_l, _p]),
+    "mts_moe_wide_head_cast_fwd": (_i, [_p, _p, _l, _i, _i, _i, _i, _i] + [_p] * 15 + [_l, _p, _p]),
     "mts_moe_head_workspace_bytes": (_l, [_l, _i, _i]),
     "mts_moe_head_fwd": (_i, [_p, _p, _l, _i, _i, _i, _i, _i] + [_p] * 14 + [_p, _l, _p]),
+    "mts_moe_head_cast_fwd": (_i, [_p, _p, _l, _i, _i, _i, _i, _i] + [_p] * 14 + [_p, _l, _p, _p]),
     "mts_moe_head_bwd_workspace_bytes": (_l, [_l, _i, _i]),
     "mts_moe_head_bwd": (_i, [_p] * 11 + [_l, _i, _i, _i, _i, _i, _p, _p, _p, _l, _p]),
     "mts_moe_ds_partials": (_i, [_i]),
