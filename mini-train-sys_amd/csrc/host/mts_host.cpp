@@ -1108,7 +1108,7 @@ struct Embedding : torch::autograd::Function<Embedding> {
         const int64_t V = ctx->saved_data["rows"].toInt(), T = ids.numel(), H = grads[0].size(-1);
         if (written_out(grads)) return {Tensor(), at::embedding_dense_backward(grads[0].to(at::kFloat), ids, V, -1, false), Tensor()};
         const Tensor g = dense16(grads[0]);
-        const int64_t ws_bytes = mts_embedding_bwd_workspace_bytes(T, V);
+        const int64_t ws_bytes = mts_embedding_bwd_workspace_bytes(T, V, H);
         Tensor dw = f32({V, H}, g), ws = bytes(ws_bytes, g);
         check(mts_embedding_bwd(ptr(g), ptr_as<int64_t>(ids), T, V, H, dtype_code(g), ptr_as<float>(dw), ptr(ws), ws_bytes, stream_of(g)), "mts_embedding_bwd");
         return {Tensor(), dw, Tensor()};

@@ -12,12 +12,15 @@ def _ids(T, V, spread, g):
         return torch.full((T,), V - 1)
     if spread == "few":   # some rows of more tokens than a wave sums alone
         return torch.randint(0, min(V, 5), (T,), generator=g) * (V // min(V, 5)) % V
-    return torch.randint(0, V, (T,), generator=g)
+    ids = torch.randint(0, V, (T,), generator=g)
+    return torch.where(torch.rand(T, generator=g) < 0.5, V // 3, ids) if spread == "half" else ids
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("T,V,H,spread", [(1, 1, 4, "one"), (63, 7, 256, "even"), (65, 257, 260, "even"), (1025, 1000, 768, "few"), (1000, 513, 1024, "one"),
-                                          (5003, 50257, 768, "even"), (4099, 8192, 1536, "few"), (300, 33, 4096, "few")])
+                                          (5003, 50257, 768, "even"), (4099, 8192, 1536, "few"), (300, 33, 4096, "few"),
+                                          # rows of whole segments of 128 places, alone and with others in front and behind; ranges of ids at their longest
+                                          (127, 9, 512, "one"), (128, 9, 512, "one"), (8193, 3, 260, "even"), (20000, 50257, 768, "half"), (3000, 300001, 4, "even")])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 def test_gradient_of_the_table(T, V, H, spread, dtype):
     print(f"embedding T={T} V={V} H={H} {spread} {dtype}", flush=True)
