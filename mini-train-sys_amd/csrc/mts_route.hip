@@ -160,6 +160,61 @@ __global__ __launch_bounds__(kScanThreads) void route_scan_kernel(
     route_scan_block(cnt, n_chunks, E, block_m, counts, expert_start, tile_row_start, tile_expert, tile_count, e0);
 }
 
+// Few entries: counters, scan and scatter by one block, whose waves take a contiguous share each (the same rows: entries of one expert in their order) and hold
+// it in registers from the first part to the last.  The three launches wait for one another and for memory most of their 12 us; up to a chunk a wave the
+// block takes 6 (8 to 128 experts).  From there on its ids would come a second time and its stores are one CU's: 8192 entries 10 to 13 us, 16 384 17 to 23, where
+// the launches still take 12.
+constexpr int kOneWaves = kScanThreads / MTS_WAVE;
+constexpr int64_t kOneEntries = kOneWaves * kChunk;
+constexpr int kOneExperts = 256;   // whose counters are in LDS for every wave
+__global__ __launch_bounds__(kScanThreads) void route_one_kernel(const int32_t* __restrict__ idx, int TK, int K, int E, int32_t* __restrict__ counts,
+                                                                 int32_t* __restrict__ expert_start, int32_t* __restrict__ s_scatter,
+                                                                 int32_t* __restrict__ s_reverse, int32_t* __restrict__ x_gather, MtsRouterStats stats) {
+    if (blockIdx.x == 1) {
+        mts_router::stats_block<kScanThreads>(stats.partial, stats.partial_counts, stats.blocks, stats.E, stats.inv_t, stats.inv_routes, stats.prob_mean,
+                                              stats.z_loss, stats.entropy, stats.counts, stats.load_balance, stats.load_stats, threadIdx.x / MTS_WAVE);
+        return;
+    }
+    extern __shared__ int32_t lds[];   // [kOneWaves][E] the waves' counters, then [E] over all of them
+    const int wave = threadIdx.x / MTS_WAVE, lane = threadIdx.x % MTS_WAVE;
+    const int share = (TK + kScanThreads - 1) / kScanThreads * MTS_WAVE;
+    const int cbeg = min(wave * share, TK), cend = min(cbeg + share, TK);
+    int32_t *mine = lds + wave * E, *all = lds + kOneWaves * E;
+    int first[kSteps];
+    scatter_load(first, idx, E, 0, E, cbeg, cend);
+    for (int e = lane; e < E; e += MTS_WAVE) mine[e] = 0;
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s)
+        if (first[s] >= 0) atomicAdd(&mine[first[s]], 1);
+    __syncthreads();
+    for (int e = threadIdx.x; e < E; e += kScanThreads) {
+        int32_t before = 0;
+#pragma unroll
+        for (int w = 0; w < kOneWaves; ++w) {
+            const int32_t n = lds[w * E + e];
+            lds[w * E + e] = before;
+            before += n;
+        }
+        all[e] = counts[e] = before;
+    }
+    __syncthreads();
+    if (wave == 0) {
+        int32_t carry = 0;
+        for (int eb = 0; eb < E; eb += MTS_WAVE) {
+            const int e = eb + lane;
+            const int32_t n = e < E ? all[e] : 0, incl = wave_scan(n);
+            if (e < E) all[e] = expert_start[e] = carry + incl - n;
+            carry += __builtin_amdgcn_readlane(incl, MTS_WAVE - 1);
+        }
+        if (lane == 0) expert_start[E] = carry;
+    }
+    __syncthreads();
+    if (!s_scatter || cbeg >= cend) return;
+    LdsRows next = (LdsRows)mine;
+    for (int e = lane; e < E; e += MTS_WAVE) next[e] = next[e] + all[e];
+    scatter_place(first, K, E, cbeg, cend, next, s_scatter, s_reverse, x_gather);
+}
+
 // a copy that rides in a launch of kThreads
 __device__ __forceinline__ void ride(const MtsCastJob& copy, int dtype) {
     if (dtype == MTS_BF16) mts_cast::cast_block<bf16_t, kThreads>(copy.cast, blockIdx.x - copy.own_blocks);
@@ -331,7 +386,7 @@ extern "C" int64_t mts_moe_route_workspace_bytes(int64_t T, int K, int E) {
 
 namespace {
 
-// the three launches; cnt holds n_chunks * E counters, every one of which is written by the
+// the launches; cnt holds n_chunks * E counters, every one of which is written by the
 // histogram kernel before the scan reads it (nothing has to start at zero)
 int route_launch(const int32_t* top_k_index, int64_t T, int K, int E, int block_m, int32_t* counts,
                  int32_t* expert_start, int32_t* s_scatter, int32_t* s_reverse, int32_t* x_gather,
@@ -339,6 +394,12 @@ int route_launch(const int32_t* top_k_index, int64_t T, int K, int E, int block_
                  hipStream_t s, const MtsRouterStats* stats = nullptr) {
     const bool permute = s_scatter != nullptr;
     const int64_t TK = T * K;
+    if (TK <= kOneEntries && E <= kOneExperts && !tile_row_start && !tile_expert && !tile_count) {
+        route_one_kernel<<<stats ? 2 : 1, kScanThreads, (size_t)(kOneWaves + 1) * E * sizeof(int32_t), s>>>(top_k_index, (int)TK, K, E, counts, expert_start, s_scatter,
+                                                                                                            s_reverse, x_gather, stats ? *stats : MtsRouterStats{});
+        MTS_CHECK_LAUNCH();
+        return MTS_OK;
+    }
     const int64_t n_chunks = (TK + kChunk - 1) / kChunk;
     const int grid = (int)((n_chunks + kWaves - 1) / kWaves);
     for (int e0 = 0; e0 < E; e0 += MTS_MAX_EXPERTS) {   // one pass per window of experts
