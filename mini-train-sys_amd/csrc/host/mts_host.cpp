@@ -357,16 +357,16 @@ Tensor experts_forward(const Tensor& x, const Tensor& w1_in, const Tensor& w2_in
     const bool weighted = opt.on(WEIGHTED_POST);
     const bool few_masters = reads_masters(x, w1_in, w2_in, TK, opt);
     const bool few = few_masters || mts_moe_fwd_few_rows_preferred(act, act, T, TK, E, H, I);
+    const bool given = w1.defined();
     if (few_masters) {
         w1 = w1_in;
         w2 = w2_in;
-    } else if (w1.defined()) {
-    } else if (copies_masters(x, w1_in, w2_in, TK, opt)) {
+    } else if (!given && copies_masters(x, w1_in, w2_in, TK, opt)) {
         w1 = at::empty(w1_in.sizes(), x.options());
         w2 = at::empty(w2_in.sizes(), x.options());
         check(mts_moe_cast_weights_pair(ptr_as<float>(w1_in), ptr(w1), w1_in.numel(), ptr_as<float>(w2_in), ptr(w2), w2_in.numel(), act, stream),
               "mts_moe_cast_weights_pair");
-    } else {
+    } else if (!given) {
         w1 = stage(w1_in, false, dtype, stream);
         w2 = stage(w2_in, false, dtype, stream);
     }
