@@ -10,6 +10,8 @@
 #include "mts_router_bwd_block.h"
 #include "mts_tuning.h"
 
+#include <type_traits>
+
 namespace {
 
 using namespace mts_rl;
@@ -398,13 +400,14 @@ __global__ __launch_bounds__(kFwdThreads) void router_logits_fwd_kernel(const XT
 // statistics (fixed order) and the routes per expert, which are at the same time the chunk
 // histogram of the routing metadata (chunk = the entries of the block's rows).
 // ---------------------------------------------------------------------------
-template <typename XT, int EP, int PASSES, bool CHUNKED = false, bool MMA = false>
+// COPY: further blocks may copy weights (a launch without them is 0.2 us of 10 shorter where the code is not there, 16 tokens).
+template <typename XT, int EP, int PASSES, bool CHUNKED = false, bool MMA = false, bool COPY = sizeof(XT) == 2>
 __global__ __launch_bounds__(kFwdThreads, MMA ? 2 : 1) void router_head_kernel(
     const XT* __restrict__ x, const float* __restrict__ w, int64_t T, int H, int E, int K, int normalize,
     int rows_per_wave, int n_chunks, float* __restrict__ logits, float* __restrict__ weights, int32_t* __restrict__ indices,
     void* __restrict__ weights_act, int act_dtype, float* __restrict__ partial, int32_t* __restrict__ cnt, MtsHeadFinish finish, MtsCastJob copy) {
     using namespace mts_router;
-    if constexpr (sizeof(XT) == 2) {
+    if constexpr (COPY) {
         if (blockIdx.x >= copy.own_blocks) return mts_cast::cast_block<XT, kFwdThreads>(copy.cast, blockIdx.x - copy.own_blocks);
     }
     static_assert(!MMA || (EP == 8 && sizeof(XT) == 2 && !CHUNKED), "the matrix-pipe projection: bf16 rows, up to 8 experts");
@@ -769,10 +772,15 @@ int mts_launch_router_head(const void* x, const float* w_r, int64_t T, int H, in
     if (blocks != 1) finish.expert_start = nullptr;
     if (mma_projection_ok(H, E, act_dtype)) {
         const size_t bytes = mma_lds_bytes(H);
-        if (allow_lds(router_head_kernel<bf16_t, 8, 1, false, true>, bytes, 20 * 1024) != hipSuccess) return MTS_ERR_SHAPE;
-        router_head_kernel<bf16_t, 8, 1, false, true><<<grid, kFwdThreads, bytes, s>>>(
-            (const bf16_t*)x, w_r, T, H, E, K, normalize, rows_per_wave, 1, logits, weights, indices, weights_act, MTS_BF16,
-            partial, cnt, finish, copy);
+        auto launch = [&](auto with) {
+            constexpr bool COPY = decltype(with)::value;
+            if (allow_lds(router_head_kernel<bf16_t, 8, 1, false, true, COPY>, bytes, 20 * 1024) != hipSuccess) return false;
+            router_head_kernel<bf16_t, 8, 1, false, true, COPY><<<grid, kFwdThreads, bytes, s>>>(
+                (const bf16_t*)x, w_r, T, H, E, K, normalize, rows_per_wave, 1, logits, weights, indices, weights_act, MTS_BF16,
+                partial, cnt, finish, copy);
+            return true;
+        };
+        if (!(cast ? launch(std::true_type()) : launch(std::false_type()))) return MTS_ERR_SHAPE;
         MTS_CHECK_LAUNCH();
         return MTS_OK;
     }
