@@ -51,7 +51,7 @@ def train_step(model: torch.nn.Module, optimizer: torch.optim.Optimizer, batch: 
         if check_finite:
             flag = torch.empty((), dtype=torch.float32, pin_memory=True).copy_(norm[2], non_blocking=True)
             copied = torch.cuda.Event()
-            copied.record()
+            copied.record(torch.cuda.current_stream(norm.device))   # the copy's, whatever device is the current one
         update.apply(norm, skip_if_not_finite=check_finite)
         if check_finite:
             copied.synchronize()
