@@ -102,7 +102,9 @@ __device__ __forceinline__ void best_of_lanes(float& bv, int& be) {
 
 // K rounds of arg-max over the logits of a row (ties to the lower expert index).  `taken` has a
 // bit per slot j of this lane (expert j*G + g); sel_e / sel_p get the expert and its softmax
-// probability per rank, mass the sum of the selected probabilities.
+// probability per rank, mass the sum of the selected probabilities.  A NaN counts as -infinity: such
+// a row's weights are NaN, but its routes are K different experts as any row's are, which the counters,
+// the scan and the scatter of the routing metadata rely on.
 template <int EP, int G>
 __device__ __forceinline__ void select_top_k(const RowState<EP, G>& r, int E, int K, int g,
                                              float (&sel_p)[MTS_MAX_TOP_K], int (&sel_e)[MTS_MAX_TOP_K], float& mass) {
@@ -122,8 +124,8 @@ __device__ __forceinline__ void select_top_k(const RowState<EP, G>& r, int E, in
             for (int j = 0; j < EP; ++j) {
                 int e = j * G + g;
                 bool free_slot = !((taken >> j) & 1u);
-                if (free_slot && (r.l[j] > bv || (r.l[j] == bv && e < be))) {
-                    bv = r.l[j];
+                if (free_slot && (r.l[j] > bv || be == 0x7fffffff)) {   // the lane's experts ascend: an equal one stays behind
+                    bv = fmaxf(r.l[j], bv);
                     be = e;
                 }
             }
