@@ -163,7 +163,9 @@ int mts_moe_head_fwd(const void* x, const float* w_r, int64_t T, int H, int E, i
                      int32_t* s_reverse, int32_t* x_gather, void* workspace, int64_t workspace_bytes,
                      void* stream);
 /* With casts (two, or NULL), as mts_moe_cast_weights_pair: the first is made by further blocks of the first launch, the second by
- * further blocks of the last, whose own blocks wait for memory most of their time.  act_dtype then is a 16-bit type.                  */
+ * further blocks of the last, whose own blocks wait for memory most of their time; both by a launch of their own where
+ * mts_moe_head_casts_ride is 0 (n1, n2: the lengths).  act_dtype then is a 16-bit type.          */
+int mts_moe_head_casts_ride(int64_t T, int H, int E, int act_dtype, int64_t n1, int64_t n2);
 int mts_moe_head_cast_fwd(const void* x, const float* w_r, int64_t T, int H, int E, int K, int normalize,
                           int act_dtype, float* logits, float* weights, int32_t* indices, void* weights_act,
                           float* prob_mean, float* z_loss, float* entropy, int32_t* counts,

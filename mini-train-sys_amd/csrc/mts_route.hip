@@ -527,10 +527,28 @@ static int check_casts(const MtsCast* casts, int act_dtype) {
     if (act_dtype == MTS_F32) return MTS_ERR_DTYPE;
     for (int i = 0; i < 2; ++i) {
         if (!casts[i].src || !casts[i].dst) return MTS_ERR_NULL;
-        if (casts[i].n < 8 || casts[i].n % 8 || casts[i].n >= (1LL << 36)) return MTS_ERR_SHAPE;   // 2^36 values: 2^31 threads
+        if (casts[i].n < 8 || casts[i].n % 8) return MTS_ERR_SHAPE;
         if (!mts_aligned16(casts[i].src) || !mts_aligned16(casts[i].dst)) return MTS_ERR_ALIGN;
     }
     return MTS_OK;
+}
+
+extern "C" int mts_moe_head_casts_ride(int64_t T, int H, int E, int act_dtype, int64_t n1, int64_t n2) {
+    constexpr int64_t kMost = 1LL << 34;   // values: 2^30 threads, of fewer than 2^32 that a launch holds
+    if (n1 > kMost || n2 > kMost) return 0;
+    if (E > kFinishMaxE) return 1;
+    int blocks, rows_per_wave;
+    mts_router_head_geometry(T, mts_router_head_group(H, E, act_dtype), &blocks, &rows_per_wave);
+    return blocks > 1 ? 1 : 0;   // one block: no second launch to ride in
+}
+
+// The copies that the head's launches are to carry; those that they do not are made here.
+static int carried_casts(const MtsCast** casts, int64_t T, int H, int E, int act_dtype, void* stream) {
+    if (const int rc = check_casts(*casts, act_dtype)) return rc;
+    const MtsCast* c = *casts;
+    if (!c || mts_moe_head_casts_ride(T, H, E, act_dtype, c[0].n, c[1].n)) return MTS_OK;
+    *casts = nullptr;
+    return mts_moe_cast_weights_pair(c[0].src, c[0].dst, c[0].n, c[1].src, c[1].dst, c[1].n, act_dtype, stream);
 }
 
 extern "C" int mts_moe_wide_head_cast_fwd(const void* x, const float* w_r, int64_t T, int H, int E, int K, int normalize, int act_dtype, float* logits, float* weights,
@@ -542,7 +560,7 @@ extern "C" int mts_moe_wide_head_cast_fwd(const void* x, const float* w_r, int64
     if (!mts_moe_wide_head_supported(T, H, E, K)) return MTS_ERR_SHAPE;
     if (workspace_bytes < mts_moe_wide_head_workspace_bytes(T, E)) return MTS_ERR_WORKSPACE;
     if (!mts_aligned16(workspace)) return MTS_ERR_ALIGN;
-    if (const int rc = check_casts(casts, act_dtype)) return rc;
+    if (const int rc = carried_casts(&casts, T, H, E, act_dtype, stream)) return rc;
     hipStream_t s = (hipStream_t)stream;
     const int64_t chunks = (T + MTS_WIDE_HEAD_ROWS - 1) / MTS_WIDE_HEAD_ROWS;
     float* partial = (float*)workspace;
@@ -586,7 +604,7 @@ extern "C" int mts_moe_head_cast_fwd(const void* x, const float* w_r, int64_t T,
     if (T <= 0 || K < 1 || T * (int64_t)K > 0x7fffffffLL) return MTS_ERR_SHAPE;
     if (workspace_bytes < mts_moe_head_workspace_bytes(T, K, E)) return MTS_ERR_WORKSPACE;
     if (!mts_aligned16(workspace)) return MTS_ERR_ALIGN;
-    if (const int rc = check_casts(casts, act_dtype)) return rc;
+    if (const int rc = carried_casts(&casts, T, H, E, act_dtype, stream)) return rc;
     hipStream_t s = (hipStream_t)stream;
     float* partial = (float*)workspace;
     int32_t* cnt = (int32_t*)(partial + (int64_t)MTS_HEAD_MAX_CHUNKS * (E + 2));
@@ -595,11 +613,6 @@ extern "C" int mts_moe_head_cast_fwd(const void* x, const float* w_r, int64_t T,
                                   expert_start, s_scatter, s_reverse, x_gather};
     int blocks, rows_per_wave;
     mts_router_head_geometry(T, mts_router_head_group(H, E, act_dtype), &blocks, &rows_per_wave);
-    if (casts && blocks == 1) {   // no second launch to ride in
-        const int rc = mts_moe_cast_weights_pair(casts[0].src, casts[0].dst, casts[0].n, casts[1].src, casts[1].dst, casts[1].n, act_dtype, stream);
-        if (rc) return rc;
-        casts = nullptr;
-    }
     int finished = 0;
     const int rc = mts_launch_router_head(x, w_r, T, H, E, K, normalize, act_dtype, logits, weights, indices, weights_act,
                                           partial, cnt, finish, &finished, casts, s);

@@ -68,6 +68,7 @@ SIGNATURES = {
     "mts_moe_wide_head_cast_fwd": (_i, [_p, _p, _l, _i, _i, _i, _i, _i] + [_p] * 15 + [_l, _p, _p]),
     "mts_moe_head_workspace_bytes": (_l, [_l, _i, _i]),
     "mts_moe_head_fwd": (_i, [_p, _p, _l, _i, _i, _i, _i, _i] + [_p] * 14 + [_p, _l, _p]),
+    "mts_moe_head_casts_ride": (_i, [_l, _i, _i, _i, _l, _l]),
     "mts_moe_head_cast_fwd": (_i, [_p, _p, _l, _i, _i, _i, _i, _i] + [_p] * 14 + [_p, _l, _p, _p]),
     "mts_moe_head_bwd_workspace_bytes": (_l, [_l, _i, _i]),
     "mts_moe_head_bwd": (_i, [_p] * 11 + [_l, _i, _i, _i, _i, _i, _p, _p, _p, _l, _p]),
