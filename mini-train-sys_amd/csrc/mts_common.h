@@ -210,6 +210,7 @@ struct MtsHeadFinish {
     float *load_balance, *load_stats;
     int32_t *expert_start, *s_scatter, *s_reverse, *x_gather;
 };
+bool mts_router_head_carries(int64_t T, int H, int E, int act_dtype);   // whether copies of weights gain as further blocks of it
 int mts_launch_router_head(const void* x, const float* w_r, int64_t T, int H, int E, int K, int normalize, int act_dtype,
                            float* logits, float* weights, int32_t* indices, void* weights_act, float* partial,
                            int32_t* cnt, MtsHeadFinish finish, int* finished, const MtsCast* cast, hipStream_t s);   // cast: more blocks of the launch, or NULL

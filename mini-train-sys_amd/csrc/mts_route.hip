@@ -536,10 +536,10 @@ static int check_casts(const MtsCast* casts, int act_dtype) {
 extern "C" int mts_moe_head_casts_ride(int64_t T, int H, int E, int act_dtype, int64_t n1, int64_t n2) {
     constexpr int64_t kMost = 1LL << 34;   // values: 2^30 threads, of fewer than 2^32 that a launch holds
     if (n1 > kMost || n2 > kMost) return 0;
-    if (E > kFinishMaxE) return 1;
+    if (E > kFinishMaxE) return 1;   // room for two blocks a CU at any width
     int blocks, rows_per_wave;
     mts_router_head_geometry(T, mts_router_head_group(H, E, act_dtype), &blocks, &rows_per_wave);
-    return blocks > 1 ? 1 : 0;   // one block: no second launch to ride in
+    return blocks > 1 && mts_router_head_carries(T, H, E, act_dtype) ? 1 : 0;   // one block: no second launch to ride in
 }
 
 // The copies that the head's launches are to carry; those that they do not are made here.

@@ -757,6 +757,22 @@ void mts_router_head_geometry(int64_t T, int group, int* blocks, int* rows_per_w
     *rows_per_wave = (int)per_wave;
 }
 
+// Copies beside the head (mts_cast_block.h) are blocks of the head's kernel and hold as much LDS as its own.  Where a CU has room for two of them they gain at
+// every size (768 wide, 16 384 to 65 536 tokens: the layer's pass 210 -> 204, 287 -> 280, 525 -> 516, 689 -> 684 us; 12 experts of 1024, 2048 tokens of
+// fp16: 103 -> 86).  Where it has room for one, the copies wait for the CUs that the head's last round leaves: a launch of their own against the ride with
+// 63 blocks 250 / 251 us, 125 294 / 292, 128 538 / 537 and 119.6 / 119.7, 188 310 / 319 and 697 / 706 and 131 / 133, 256 393 / 411 and 156 / 162, 256 + 119
+// 188 / 185, 512 595 / 604 (1024 to 4096 wide).  They ride where at least half of the CUs are left.
+bool mts_router_head_carries(int64_t T, int H, int E, int act_dtype) {
+    constexpr int kCus = 256, kCuLds = 160 * 1024;
+    const size_t parked = (E <= 8 ? 10 : 19) * 1024;   // the kernel's own arrays
+    const size_t lds = (mma_projection_ok(H, E, act_dtype) ? mma_lds_bytes(H) : (size_t)E * H * sizeof(float)) + parked;
+    if (2 * lds <= kCuLds) return true;
+    int blocks, rows_per_wave;
+    mts_router_head_geometry(T, mts_router_head_group(H, E, act_dtype), &blocks, &rows_per_wave);
+    const int last = blocks % kCus;
+    return last != 0 && last <= kCus / 2;
+}
+
 int mts_launch_router_head(const void* x, const float* w_r, int64_t T, int H, int E, int K, int normalize, int act_dtype,
                            float* logits, float* weights, int32_t* indices, void* weights_act, float* partial,
                            int32_t* cnt, MtsHeadFinish finish, int* finished, const MtsCast* cast, hipStream_t s) {

@@ -37,11 +37,12 @@ def _weights(n, seed):
     return w.cuda()
 
 
-# lengths around the values of a block of 256 and of 512 threads; one block of the head (which has no second launch), a few, and all that it has
+# lengths around the values of a block of 256 and of 512 threads; one block of the head (which has no second launch), a few, and all that it has;
+# a head that fills the CUs one by one (129 blocks: the copies have their own launch, 257: they ride)
 @pytest.mark.parametrize("T,H,E,K,n1,n2,dtype", [
     (1, 64, 8, 2, 8, 8192, torch.bfloat16), (64, 768, 8, 2, 8200, 8, torch.bfloat16), (65, 768, 8, 2, 8184, 8192, torch.bfloat16),
     (65, 760, 16, 1, 8192, 8200, torch.float16), (1000, 64, 8, 2, 40008, 3 * 8192, torch.float16), (20000, 768, 8, 2, 1 << 20, 1 << 19, torch.bfloat16),
-    (40000, 64, 4, 2, 8, 8, torch.bfloat16), (1, 64, 17, 1, 8, 8, torch.float16), (300, 768, 64, 4, 16384, 16376, torch.bfloat16), (5000, 132, 33, 8, 16392, 8, torch.bfloat16)])
+    (40000, 64, 4, 2, 8, 8, torch.bfloat16), (2064, 1024, 16, 2, 8200, 8192, torch.float16), (4112, 1024, 16, 2, 8192, 8200, torch.bfloat16), (1, 64, 17, 1, 8, 8, torch.float16), (300, 768, 64, 4, 16384, 16376, torch.bfloat16), (5000, 132, 33, 8, 16392, 8, torch.bfloat16)])
 def test_copies_beside_the_head(T, H, E, K, n1, n2, dtype):
     print(f"head with copies T={T} H={H} E={E} K={K} n={n1},{n2} {dtype}", flush=True)
     g = torch.Generator().manual_seed(T)
