@@ -1491,16 +1491,17 @@ Tensor grad_norm(const std::vector<Tensor>& params, double max_norm, const Tenso
     return result;
 }
 
-// groups: of each tensor; settings: lr, beta1, beta2, eps and weight decay of each group; scale: what grad_norm returned
+// groups: of each tensor; settings: lr, beta1, beta2, eps and weight decay of each group; scale: what grad_norm returned, clipped: from the gradients
 void adamw(const std::vector<Tensor>& params, const std::vector<Tensor>& exp_avgs, const std::vector<Tensor>& exp_avg_sqs, const std::vector<Tensor>& steps,
-           const std::vector<int64_t>& groups, const std::vector<std::array<double, 5>>& settings, const Tensor& scale, bool skip_if_not_finite) {
+           const std::vector<int64_t>& groups, const std::vector<std::array<double, 5>>& settings, const Tensor& scale, bool clipped, bool skip_if_not_finite) {
     std::vector<MtsAdamTensor> tensors;
+    std::vector<Tensor> held;   // gradients that somebody else holds: left clipped, and marked as written, as stock clipping leaves them
     for (size_t i = 0; i < params.size(); ++i) {
         const Tensor& g = params[i].grad();
-        // a gradient that somebody else holds is left clipped, as stock clipping leaves it
-        const bool held = g.use_count() > 1 || g.storage().use_count() > 1;
+        const bool keep = clipped && (g.use_count() > 1 || g.storage().use_count() > 1);
         tensors.push_back({ptr_as<float>(params[i]), ptr_as<float>(g), ptr_as<float>(exp_avgs[i]), ptr_as<float>(exp_avg_sqs[i]), ptr_as<float>(steps[i]),
-                           params[i].numel(), (int)groups[i], held});
+                           params[i].numel(), (int)groups[i], keep});
+        if (keep) held.push_back(g);
     }
     std::vector<MtsAdamGroup> of;
     for (const auto& s : settings) of.push_back({s[0], s[1], s[2], s[3], s[4]});
@@ -1509,7 +1510,7 @@ void adamw(const std::vector<Tensor>& params, const std::vector<Tensor>& exp_avg
     check(mts_adamw(tensors.data(), (int)tensors.size(), of.data(), (int)of.size(), result + 1, skip_if_not_finite ? result + 2 : nullptr, ptr(ws), ws.numel(),
                     stream_of(params[0])),
           "mts_adamw");
-    for (const auto* written : {&params, &exp_avgs, &exp_avg_sqs, &steps})
+    for (const auto* written : {&params, &exp_avgs, &exp_avg_sqs, &steps, &std::as_const(held)})
         for (const Tensor& t : *written)
             if (!t.is_inference()) t.unsafeGetTensorImpl()->bump_version();
 }
@@ -1620,9 +1621,9 @@ PYBIND11_MODULE(_host, m) {
     });
     m.def("adamw", [](const std::vector<Tensor>& params, const std::vector<Tensor>& exp_avgs, const std::vector<Tensor>& exp_avg_sqs,
                       const std::vector<Tensor>& steps, const std::vector<int64_t>& groups, const std::vector<std::array<double, 5>>& settings, const Tensor& scale,
-                      bool skip_if_not_finite) {
+                      bool clipped, bool skip_if_not_finite) {
         c10::OptionalDeviceGuard guard(params.at(0).device());
-        adamw(params, exp_avgs, exp_avg_sqs, steps, groups, settings, scale, skip_if_not_finite);
+        adamw(params, exp_avgs, exp_avg_sqs, steps, groups, settings, scale, clipped, skip_if_not_finite);
     });
     m.def("cross_entropy_supported", &cross_entropy_supported);
     m.def("cross_entropy", [](const Tensor& logits, const Tensor& targets, bool is_root) {

@@ -29,6 +29,7 @@ class Update:
     def __init__(self, optimizer):
         self.optimizer = optimizer
         self.params, self.exp_avgs, self.exp_avg_sqs, self.steps, self.groups, self.settings = [], [], [], [], [], []
+        self.clipped = False
 
     def add_group(self, group) -> bool:
         if not group["fused"] or group["amsgrad"] or group["maximize"] or group["capturable"] or group["differentiable"] or group["foreach"]:
@@ -52,10 +53,12 @@ class Update:
 
     def norm(self, max_norm: float | None, loss: torch.Tensor) -> torch.Tensor:
         """``[norm, clipping coefficient, whether norm or loss are not finite]``"""
+        self.clipped = max_norm is not None
         return _lib.host().grad_norm(self.params, -1.0 if max_norm is None else max_norm, loss)
 
     def apply(self, norm: torch.Tensor, skip_if_not_finite: bool) -> None:
-        _lib.host().adamw(self.params, self.exp_avgs, self.exp_avg_sqs, self.steps, self.groups, self.settings, norm, skip_if_not_finite)
+        _lib.host().adamw(self.params, self.exp_avgs, self.exp_avg_sqs, self.steps, self.groups, self.settings, norm, self.clipped,
+                           skip_if_not_finite)
         if "step" in self.optimizer.__dict__:
             self.optimizer._opt_called = True
 

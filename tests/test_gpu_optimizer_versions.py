@@ -1,0 +1,47 @@
+"""What the optimizer update marks as written, against stock clipping and fused AdamW."""
+
+import pytest
+import torch
+
+from tests.test_gpu_optimizer import Bag, _optimizer
+
+pytestmark = pytest.mark.gpu
+
+
+def _step(bag, opt, limit, own):
+    """A second step (the first makes the state), with graphs that have saved a gradient and a parameter: whether they notice."""
+    from minitrain_amd.train.update import plan
+
+    for p, g in zip(bag.p, bag.grads):
+        p.grad = g.clone()
+    opt.step()
+    for p, g in zip(bag.p, bag.grads):
+        p.grad = g.clone()
+    x = torch.ones_like(bag.p[0], requires_grad=True)
+    of_gradient, of_parameter = (x * bag.p[0].grad).sum(), (x * bag.p[0].detach()).sum()
+    loss = torch.ones((), device="cuda")
+    if own:
+        update = plan(bag, opt, loss, limit)
+        update.apply(update.norm(limit, loss), True)
+    else:
+        if limit is not None:
+            torch.nn.utils.clip_grad_norm_(bag.parameters(), limit)
+        opt.step()
+    noticed = []
+    for result in (of_gradient, of_parameter):
+        try:
+            result.backward()
+            noticed.append(False)
+        except RuntimeError as e:
+            assert "modified by an inplace operation" in str(e)
+            noticed.append(True)
+    return noticed
+
+
+@pytest.mark.parametrize("limit", [None, 1e-3, 1e9])
+def test_a_graph_that_saved_a_gradient_notices_the_clipping(limit):
+    runs = []
+    for own in (True, False):
+        bag = Bag([5, 4097])
+        runs.append(_step(bag, _optimizer(bag), limit, own))
+    assert runs[0][0] == runs[1][0] == (limit is not None)
