@@ -1510,9 +1510,9 @@ void adamw(const std::vector<Tensor>& params, const std::vector<Tensor>& exp_avg
     check(mts_adamw(tensors.data(), (int)tensors.size(), of.data(), (int)of.size(), result + 1, skip_if_not_finite ? result + 2 : nullptr, ptr(ws), ws.numel(),
                     stream_of(params[0])),
           "mts_adamw");
-    for (const auto* written : {&params, &exp_avgs, &exp_avg_sqs, &steps, &std::as_const(held)})
-        for (const Tensor& t : *written)
-            if (!t.is_inference()) t.unsafeGetTensorImpl()->bump_version();
+    // The stock fused operator marks neither parameters nor state as written: graphs that have saved one go on.
+    for (const Tensor& g : held)
+        if (!g.is_inference()) g.unsafeGetTensorImpl()->bump_version();
 }
 
 }  // namespace

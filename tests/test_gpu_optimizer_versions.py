@@ -45,3 +45,12 @@ def test_a_graph_that_saved_a_gradient_notices_the_clipping(limit):
         bag = Bag([5, 4097])
         runs.append(_step(bag, _optimizer(bag), limit, own))
     assert runs[0][0] == runs[1][0] == (limit is not None)
+
+
+@pytest.mark.parametrize("limit", [None, 1e-3])
+def test_a_graph_that_saved_a_parameter_goes_on_as_after_a_stock_step(limit):
+    runs = []
+    for own in (True, False):
+        bag = Bag([5, 4097])
+        runs.append(_step(bag, _optimizer(bag), limit, own)[1])
+    assert runs[0] == runs[1]
