@@ -11,6 +11,18 @@ from torch.optim import optimizer as _optimizer
 from minitrain_amd import _lib
 
 
+_TORCH_OWN = ("torch.optim.optimizer", "torch.optim.adam", "torch.optim.adamw")
+
+
+def _is_torch_own(function) -> bool:
+    """Whether ``function`` and all that it wraps are written in the modules of torch's AdamW."""
+    while function is not None:
+        if getattr(function, "__globals__", {}).get("__name__") not in _TORCH_OWN:
+            return False
+        function = getattr(function, "__wrapped__", None)
+    return True
+
+
 def _runs_as_written(optimizer) -> bool:
     """Whether ``optimizer.step()`` is AdamW's and nobody looks on."""
     if type(optimizer) is not torch.optim.AdamW or hasattr(optimizer, "grad_scale") or hasattr(optimizer, "found_inf"):
@@ -18,6 +30,8 @@ def _runs_as_written(optimizer) -> bool:
     if optimizer._optimizer_step_pre_hooks or optimizer._optimizer_step_post_hooks:
         return False
     if _optimizer._global_optimizer_pre_hooks or _optimizer._global_optimizer_post_hooks:
+        return False
+    if not _is_torch_own(torch.optim.AdamW.step):   # replaced on the class
         return False
     step = optimizer.__dict__.get("step")   # a learning-rate scheduler wraps it to note that it has run
     return step is None or (getattr(step, "_wrapped_by_lr_sched", False) and getattr(step, "__wrapped__", None) is torch.optim.AdamW.step)

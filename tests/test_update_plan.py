@@ -1,0 +1,31 @@
+"""Which optimizers the update in the kernels stands in for (host code: no GPU)."""
+
+import functools
+
+import torch
+
+from minitrain_amd.train import update
+
+
+def _optimizer():
+    return torch.optim.AdamW([torch.nn.Parameter(torch.ones(3))], lr=1e-3)
+
+
+def test_a_step_replaced_on_the_class_is_called(monkeypatch):
+    opt = _optimizer()
+    assert update._runs_as_written(opt)
+    torch.optim.lr_scheduler.LambdaLR(opt, lambda _: 1.0)
+    assert update._runs_as_written(opt)
+    known = torch.optim.AdamW.step
+
+    def step(self, closure=None):
+        return known(self, closure)
+
+    for replaced in (step, functools.wraps(known)(step)):
+        with monkeypatch.context() as m:
+            m.setattr(torch.optim.AdamW, "step", replaced)
+            fresh = _optimizer()
+            assert not update._runs_as_written(fresh) and not update._runs_as_written(opt)
+            torch.optim.lr_scheduler.LambdaLR(fresh, lambda _: 1.0)
+            assert not update._runs_as_written(fresh)
+        assert update._runs_as_written(opt)
