@@ -48,6 +48,8 @@ class Update:
     def add_group(self, group) -> bool:
         if not group["fused"] or group["amsgrad"] or group["maximize"] or group["capturable"] or group["differentiable"] or group["foreach"]:
             return False
+        if not group.get("decoupled_weight_decay", True):   # Adam's decay, by the gradient
+            return False
         numbers = (group["lr"], *group["betas"], group["eps"], group["weight_decay"])
         if any(isinstance(n, torch.Tensor) for n in numbers):
             return False

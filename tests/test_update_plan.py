@@ -29,3 +29,10 @@ def test_a_step_replaced_on_the_class_is_called(monkeypatch):
             torch.optim.lr_scheduler.LambdaLR(fresh, lambda _: 1.0)
             assert not update._runs_as_written(fresh)
         assert update._runs_as_written(opt)
+
+
+def test_decay_by_the_gradient_stays_stock():
+    opt = torch.optim.AdamW([torch.nn.Parameter(torch.ones(3))], lr=1e-3)
+    group = {**opt.param_groups[0], "fused": True}
+    assert update.Update(opt).add_group(group)
+    assert not update.Update(opt).add_group({**group, "decoupled_weight_decay": False})
