@@ -1614,6 +1614,8 @@ PYBIND11_MODULE(_host, m) {
         return std::make_tuple(v[0], v[1], v[2], v[3]);
     });
     m.attr("ADAM_GROUPS") = MTS_ADAM_GROUPS;
+    // not by way of Python's `grad`, whose object counts as a holder of the gradient from then on
+    m.def("has_gradient", [](const Tensor& p) { return p.grad().defined(); });
     m.def("adamw_supported", &adamw_supported);
     m.def("grad_norm", [](const std::vector<Tensor>& params, double max_norm, const Tensor& loss) {
         c10::OptionalDeviceGuard guard(params.at(0).device());

@@ -54,7 +54,7 @@ class Update:
         if any(isinstance(n, torch.Tensor) for n in numbers):
             return False
         for p in group["params"]:
-            if p.grad is None:
+            if not _lib.host().has_gradient(p):
                 continue
             state = self.optimizer.state.get(p)
             if not state:   # the first step makes it
@@ -89,7 +89,7 @@ def plan(model: torch.nn.Module, optimizer: torch.optim.Optimizer, loss: torch.T
     if len(optimizer.param_groups) > _lib.host().ADAM_GROUPS or not all(update.add_group(g) for g in optimizer.param_groups):
         return None
     # clipping looks at the model's gradients, the update at the optimizer's: the same ones
-    if {id(p) for p in model.parameters() if p.grad is not None} != {id(p) for p in update.params}:
+    if {id(p) for p in model.parameters() if _lib.host().has_gradient(p)} != {id(p) for p in update.params}:
         return None
     if not _lib.host().adamw_supported(update.params, update.exp_avgs, update.exp_avg_sqs, update.steps) or loss.device != update.params[0].device:
         return None

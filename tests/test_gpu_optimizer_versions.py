@@ -1,4 +1,4 @@
-"""What the optimizer update marks as written, against stock clipping and fused AdamW."""
+"""What the optimizer update writes besides parameters and state, and what it marks as written, against stock clipping and fused AdamW."""
 
 import pytest
 import torch
@@ -54,3 +54,24 @@ def test_a_graph_that_saved_a_parameter_goes_on_as_after_a_stock_step(limit):
         bag = Bag([5, 4097])
         runs.append(_step(bag, _optimizer(bag), limit, own)[1])
     assert runs[0] == runs[1]
+
+
+def test_only_held_gradients_are_written():
+    from minitrain_amd.train.update import plan
+
+    bag = Bag([4097, 4097])
+    opt = _optimizer(bag)
+
+    def backward():
+        sum((p * g).sum() for p, g in zip(bag.p, bag.grads)).backward()
+
+    backward()
+    opt.step()
+    opt.zero_grad(set_to_none=True)
+    backward()
+    held = bag.p[0].grad
+    update = plan(bag, opt, torch.ones((), device="cuda"), 1.0)
+    norm = update.norm(1.0, torch.ones((), device="cuda"))
+    update.apply(norm, True)
+    torch.testing.assert_close(held, bag.grads[0] * norm[1], rtol=1e-6, atol=0)   # a rounding of the product
+    assert torch.equal(bag.p[1].grad, bag.grads[1])
