@@ -66,11 +66,12 @@ def project(linear: nn.Linear, x: torch.Tensor, ops: OpsBackend) -> torch.Tensor
     return linear(x) if y is None else y
 
 
-def embed(table: nn.Embedding, ids: torch.Tensor, dtype: torch.dtype, ops: OpsBackend) -> torch.Tensor:
+def embed(table: nn.Module, ids: torch.Tensor, dtype: torch.dtype, ops: OpsBackend) -> torch.Tensor:
     """``table(ids).to(dtype)``, by the backend's own operator where it has one for these operands."""
-    own = getattr(ops, "embedding", None)
-    plain = table.padding_idx is None and table.max_norm is None and not table.scale_grad_by_freq and not table.sparse
-    x = own(ids, table.weight, dtype) if own is not None and plain and runs_as_written(table, nn.Embedding) else None
+    own = getattr(ops, "embedding", None) if runs_as_written(table, nn.Embedding) else None   # another module may stand in its place
+    if own is not None and (table.padding_idx is not None or table.max_norm is not None or table.scale_grad_by_freq or table.sparse):
+        own = None
+    x = own(ids, table.weight, dtype) if own is not None else None
     return table(ids).to(dtype) if x is None else x
 
 
