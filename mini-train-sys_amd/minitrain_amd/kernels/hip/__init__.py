@@ -114,7 +114,7 @@ class HipOpsBackend(DenseTorchOps):
     def total_loss(self, loss, aux, z, aux_coef, z_coef):
         """Extension: ``(loss + aux_coef * aux + z_coef * z, aux_coef * aux, z_coef * z, their sum)``, the last three without
         gradients, or None when the kernel does not take them."""
-        if not dense.is_total_loss_supported(loss, aux, z):
+        if not (isinstance(aux_coef, (int, float)) and isinstance(z_coef, (int, float)) and dense.is_total_loss_supported(loss, aux, z)):
             return None
         return dense.total_loss(loss, aux, z, aux_coef, z_coef)
 

@@ -66,3 +66,14 @@ def test_what_the_kernels_do_not_take():
     assert ops.layer_means([*losses, [t.clone().requires_grad_(True) for t in records[0]]], 2) is None   # records carry no gradient
     assert ops.layer_means([*losses, [records[1][0], records[1][0][:2]]], 2) is None             # of different sizes
     assert ops.total_loss(losses[0][0].double(), losses[0][1], losses[1][0], 1.0, 1.0) is None
+
+
+def test_coefficients_that_are_tensors_keep_their_gradients():
+    """A coefficient may be learned or changed in place: the stock operators, on the GPU, with its gradient."""
+    from minitrain_amd.model.decoder import total_loss
+
+    loss, aux, z = (torch.full((), v, device="cuda") for v in (3.0, 2.0, 0.5))
+    a = torch.tensor(0.25, device="cuda", requires_grad=True)
+    total, weighted, *_ = total_loss(loss, aux, z, a, 2, hip_backend())
+    total.backward()
+    assert float(total) == 4.5 and float(weighted) == 0.5 and float(a.grad) == 2.0
