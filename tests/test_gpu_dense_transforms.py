@@ -7,6 +7,7 @@ from torch.utils._python_dispatch import TorchDispatchMode
 
 from minitrain_amd.kernels.dense_ops import DenseTorchOps
 from minitrain_amd.kernels.hip import HipOpsBackend, dense
+from minitrain_amd.model.decoder import layer_means, total_loss
 from tests.helpers import hip_backend
 
 pytestmark = pytest.mark.gpu
@@ -30,6 +31,17 @@ def _operands(name):
     if name == "cross_entropy":
         targets = torch.tensor([1, 0, -100, 6, 3, 3], device="cuda")
         return (r(6, 7),), lambda ops, x: ops.cross_entropy(x, targets)
+    if name == "embedding":
+        ids = torch.tensor([[1, 0, 4, 1], [2, 1, 4, 4]], device="cuda")
+
+        def lookup(ops, table):
+            x = ops.embedding(ids, table, torch.float32) if hasattr(ops, "embedding") else None
+            return torch.nn.functional.embedding(ids, table) if x is None else x
+        return (r(5, 8),), lookup
+    if name == "layer_means":
+        return (r(1)[0], r(1)[0], r(1)[0], r(1)[0]), lambda ops, a, b, c, d: torch.stack(layer_means([[a, b], [c, d]], [], ops))
+    if name == "total_loss":
+        return (r(1)[0], r(1)[0], r(1)[0]), lambda ops, *a: total_loss(*a, 0.25, 0.5, ops)[0]
     angle = r(5, 8)
     cos, sin = angle.cos(), angle.sin()
     if name == "rope":
@@ -45,7 +57,7 @@ def _operands(name):
     return (r(2, 5, 72),), packed
 
 
-NAMES = ["rmsnorm", "add_rmsnorm", "cross_entropy", "rope", "qkv_rope"]
+NAMES = ["rmsnorm", "add_rmsnorm", "cross_entropy", "rope", "qkv_rope", "embedding", "layer_means", "total_loss"]
 
 
 @pytest.mark.parametrize("name", NAMES)
@@ -134,6 +146,10 @@ def _more_operands(name):
     r = lambda *shape: torch.randn(*shape, generator=g).cuda()
     if name == "attention":
         return tuple(r(2, 3, 9, 64).bfloat16() for _ in range(3)), lambda ops, q, k, v: ops.attention(q, k, v, is_causal=True, dropout_p=0.0)
+    if name == "qkv_attention":
+        angle = r(9, 64)
+        cos, sin = angle.cos().bfloat16(), angle.sin().bfloat16()
+        return (r(2, 9, 3 * 3 * 64).bfloat16(),), lambda ops, qkv: ops.qkv_attention(qkv, cos, sin, 3, is_causal=True, dropout_p=0.0)
     if name == "linear":
         def project(ops, x, w):
             with torch.autocast("cuda", dtype=torch.bfloat16):
@@ -147,7 +163,7 @@ def _more_operands(name):
 SCALED_TOL = {torch.float32: 2e-5, torch.bfloat16: 2.0 ** -6}
 
 
-@pytest.mark.parametrize("name", [*NAMES, "attention", "linear", "router_logits"])
+@pytest.mark.parametrize("name", [*NAMES, "attention", "qkv_attention", "linear", "router_logits"])
 @pytest.mark.parametrize("how", ["is_grads_batched", "vmap"])
 def test_batched_gradients(name, how):
     """Several gradients of one result in a call, as a vectorised jacobian takes them, against one call for each."""
@@ -189,9 +205,15 @@ def _predicates():
     yield "linear", linear, [r(2, 520, 64).bfloat16(), r(72, 64).requires_grad_(True)]
     yield "router_logits", is_router_logits_supported, [r(37, 64), r(24, 64)]
     yield "moe_layer", layer, [r(4, 64), r(37, 64), r(4, 128, 64), r(4, 64, 64)]
+    ids = torch.tensor([1, 0, 4], device="cuda")
+    yield "embedding", lambda table: dense.is_embedding_supported(ids, table, torch.bfloat16), [r(5, 8).requires_grad_(True)]
+    cos, sin = r(9, 64).bfloat16(), r(9, 64).bfloat16()
+    yield "qkv_attention", lambda qkv: dense.is_qkv_attention_supported(qkv, cos, sin, 3), [r(2, 9, 3 * 3 * 64).bfloat16()]
+    yield "layer_means", lambda a, b, c: dense.is_layer_means_supported([[a, b], [c]], 1), [r(1)[0], r(1)[0], r(1)[0]]
+    yield "total_loss", dense.is_total_loss_supported, [r(1)[0], r(1)[0], r(1)[0]]
 
 
-@pytest.mark.parametrize("which", range(4))
+@pytest.mark.parametrize("which", range(8))
 def test_kernels_stay_out_where_somebody_looks(which):
     """The operators that take 16-bit operands only and the layer as one node: not under a transform, a mode or with duals."""
     import torch.autograd.forward_ad as fwd

@@ -145,3 +145,41 @@ def test_who_looks_on_gets_the_stock_calls(monkeypatch):
     assert steps(lambda m, o: o.param_groups[0].update(amsgrad=True) or [s.update(max_exp_avg_sq=torch.zeros_like(s["exp_avg"])) for s in o.state.values()]) == 0
     assert steps(lambda m, o: o.param_groups[0].update(lr=torch.tensor(1e-3, device="cuda"))) == 0
     assert steps(lambda m, o: o.param_groups[1]["params"].pop()) == 0
+
+
+class _Linear(Bag):
+    """A model whose gradients are given numbers, whatever the parameters are."""
+
+    def forward(self, input_ids, *, targets, use_fused_loss):
+        return sum((p * g).sum() for p, g in zip(self.p, self.grads)) * input_ids.float().mean(), None
+
+
+@pytest.mark.parametrize("clip,check,poison", [(None, True, None), (None, True, "inf"), (None, True, "nan"), (1.0, True, None), (1.0, False, None), (1.0, False, "inf"),
+                                               (1.0, False, "nan"), (None, False, "nan")])
+def test_steps_without_clipping_and_without_the_check(monkeypatch, clip, check, poison):
+    """Against the stock calls. Without clipping nobody looks at the norm, so that a gradient that is not finite passes with a finite loss; without
+    the check everything passes."""
+    from minitrain_amd.train import step, update
+
+    print(f"clip={clip} check={check} poison={poison}", flush=True)
+    taken = []
+    apply = update.Update.apply
+    monkeypatch.setattr(update.Update, "apply", lambda self, *a, **k: (taken.append(1), apply(self, *a, **k))[1])
+    batch = {"input_ids": torch.ones(2, 3, dtype=torch.long), "targets": torch.ones(2, 3, dtype=torch.long)}
+    sides = []
+    for own in (True, False):
+        if not own:
+            monkeypatch.setattr(step, "plan", lambda *a: None)
+        model = _Linear([5, 4097, 20000])
+        opt = _optimizer(model)
+        for i in range(3):
+            hook = model.p[1].register_hook(lambda g: g * float(poison)) if poison and i == 2 else None
+            loss = step.train_step(model, opt, batch, autocast_dtype=None, grad_clip_norm=clip, check_finite=check)
+            if hook:
+                hook.remove()
+            assert loss.isfinite()
+        sides.append([t for p in model.p for t in (p.detach(), *opt.state[p].values())])
+        assert len(taken) == 2   # the first step makes the state
+    assert not poison or sides[0][4].isnan().any()
+    for a, b in zip(*sides):   # three updates, a few roundings each
+        torch.testing.assert_close(a, b, rtol=2e-6, atol=1e-9, equal_nan=True)

@@ -28,6 +28,13 @@ def _int(dtype, *shape):
     return lambda index: _labelled(index, *shape, dtype=dtype)
 
 
+def _update_supported(h, *tensors):
+    """Of tensors that are each a parameter, two moments and a step; a gradient is where its parameter is, or cannot be set."""
+    for param, *_ in tensors:
+        param.grad = _labelled(param.device.index, *param.shape)
+    return h.adamw_supported(*map(list, zip(*tensors)))
+
+
 CALLS = {
     "rmsnorm": ([_bf16(3, 8), _fp32(8)], lambda h, x, w: h.rmsnorm_supported(x, w, None)),
     "add_rmsnorm": ([_bf16(3, 8), _fp32(8), _bf16(3, 8)], lambda h, x, w, r: h.rmsnorm_supported(x, w, r)),
@@ -35,6 +42,11 @@ CALLS = {
     "qkv_rope": ([_bf16(1, 3, 24), _bf16(3, 4), _bf16(3, 4)], lambda h, *a: h.qkv_rope_supported(*a, 2)),
     "attention": ([_bf16(1, 1, 3, 64)] * 3, lambda h, *a: h.attention_supported(*a)),
     "cross_entropy": ([_bf16(3, 8), _int(torch.int64, 3)], lambda h, *a: h.cross_entropy_supported(*a)),
+    "embedding": ([_int(torch.int64, 1, 3), _fp32(5, 8)], lambda h, ids, w: h.embedding_supported(ids, w.requires_grad_(True), torch.bfloat16)),
+    "qkv_attention": ([_bf16(1, 3, 192), _bf16(3, 64), _bf16(3, 64)], lambda h, *a: h.qkv_attention_supported(*a, 1)),
+    "layer_means": ([_fp32(), _fp32(), _fp32(4), _fp32(4)], lambda h, a, b, c, d: h.layer_means_supported([[a, b], [c, d]], 1)),
+    "total_loss": ([_fp32()] * 3, lambda h, *a: h.total_loss_supported(*a)),
+    "adamw": ([_fp32(8)] * 3 + [_fp32()] + [_fp32(4)] * 3 + [_fp32()], lambda h, *a: _update_supported(h, a[:4], a[4:])),
     "router_logits": ([_bf16(3, 8), _fp32(4, 8)], lambda h, *a: h.router_logits_supported(*a)),
     "router_logits, many experts": ([_bf16(3, 8), _fp32(20, 8)], lambda h, *a: h.router_logits_supported(*a)),
     "moe_layer": ([_bf16(3, 8), _fp32(4, 8), _bf16(4, 16, 8), _bf16(4, 8, 8)], lambda h, *a: h.layer_violation(*a, 2) is None),
