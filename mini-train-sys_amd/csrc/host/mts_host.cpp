@@ -1093,7 +1093,7 @@ struct Linear : torch::autograd::Function<Linear> {
 // The stock lookup; the table's gradient is summed here, from the gradient as it arrives in the activation dtype.
 bool embedding_supported(const Tensor& ids, const Tensor& w, at::ScalarType type) {
     return at::GradMode::is_enabled() && w.requires_grad() && all_plain(ids, w) && on_one_gpu(ids, w) && ids.scalar_type() == at::kLong && w.dim() == 2 &&
-           w.scalar_type() == at::kFloat && is_activation_type(type) && mts_embedding_bwd_supported(ids.numel(), w.size(0), w.size(1));
+           w.scalar_type() == at::kFloat && is_activation_type(type) && mts_embedding_bwd_preferred(ids.numel(), w.size(0), w.size(1));
 }
 
 struct Embedding : torch::autograd::Function<Embedding> {

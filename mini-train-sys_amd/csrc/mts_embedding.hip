@@ -280,6 +280,17 @@ extern "C" int mts_embedding_bwd_supported(int64_t T, int64_t V, int64_t H) {
     return T > 0 && T <= kMostTokens && V > 0 && V <= kMostIds && H > 0 && H % 4 == 0 && H <= 16 * 4 * MTS_WAVE ? 1 : 0;
 }
 
+// Against the stock operators (conversion, sort, sums): ahead from 64 tokens on with tables of up to 65 536 rows (64 tokens 38 us, stock 45; 512 39 / 58).  More rows
+// are more blocks that each read all tokens, and a launch over all rows, while the stock sums walk the tokens; us here / stock, 768 wide: 128 256 rows, 64 tokens
+// 77 / 70; 262 144 rows, 64 tokens 172 / 130, 512 175 / 169, 4096 183 / 209; 300 001, 1024 tokens 204 / 230 (4 wide 63 / 62), 3000 209 / 401; 393 216, 4096 tokens
+// 272 / 267, 65 536 411 / 757; 524 288, 65 536 tokens of 512 361 / 549, of 128 187 / 187; 2^20, 4096 tokens 728 / 560, 65 536 950 / 1062, 262 144 of 256 825 / 971,
+// of 128 677 / 563.
+extern "C" int mts_embedding_bwd_preferred(int64_t T, int64_t V, int64_t H) {
+    if (!mts_embedding_bwd_supported(T, V, H)) return 0;
+    if (V <= 65536) return 1;
+    return V <= 327680 ? T >= V / 256 : T * H >= 64 * V;
+}
+
 extern "C" int64_t mts_embedding_bwd_workspace_bytes(int64_t T, int64_t V, int64_t H) {
     return (segments(T) * H + V + 1 + T) * (int64_t)sizeof(int32_t);   // sums of the segments first, on 16 bytes
 }

@@ -99,6 +99,7 @@ SIGNATURES = {
     "mts_cross_entropy_both": (_i, [_p, _p, _l, _i, _l, _i, _p, _p, _p, _p, _p, _p, _l, _p]),
     "mts_cross_entropy_bwd_unless_one": (_i, [_p, _p, _l, _i, _l, _i, _p, _p, _p, _p, _p, _l, _p]),
     "mts_embedding_bwd_supported": (_i, [_l, _l, _l]),
+    "mts_embedding_bwd_preferred": (_i, [_l, _l, _l]),
     "mts_embedding_bwd_workspace_bytes": (_l, [_l, _l, _l]),
     "mts_embedding_bwd": (_i, [_p, _p, _l, _i, _i, _i, _p, _p, _l, _p]),
     "mts_linear_dw_supported": (_i, [_i, _l, _i, _i]),
