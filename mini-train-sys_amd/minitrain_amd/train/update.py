@@ -11,11 +11,11 @@ from torch.optim import optimizer as _optimizer
 from minitrain_amd import _lib
 
 
-_TORCH_OWN = ("torch.optim.optimizer", "torch.optim.adam", "torch.optim.adamw")
+_TORCH_OWN = ("torch.optim.optimizer", "torch.optim.adam", "torch.optim.adamw", "torch.nn.utils.clip_grad")
 
 
 def _is_torch_own(function) -> bool:
-    """Whether ``function`` and all that it wraps are written in the modules of torch's AdamW."""
+    """Whether ``function`` and all that it wraps are written in the modules of torch's AdamW and clipping."""
     while function is not None:
         if getattr(function, "__globals__", {}).get("__name__") not in _TORCH_OWN:
             return False
@@ -35,6 +35,11 @@ def _runs_as_written(optimizer) -> bool:
         return False
     step = optimizer.__dict__.get("step")   # a learning-rate scheduler wraps it to note that it has run
     return step is None or (getattr(step, "_wrapped_by_lr_sched", False) and getattr(step, "__wrapped__", None) is torch.optim.AdamW.step)
+
+
+def _clips_as_written() -> bool:
+    """Whether the clipping that a step calls is torch's: another may stand in its place."""
+    return _is_torch_own(torch.nn.utils.clip_grad_norm_)
 
 
 class Update:
@@ -83,7 +88,7 @@ def plan(model: torch.nn.Module, optimizer: torch.optim.Optimizer, loss: torch.T
     """The update that the kernels can take in the place of clipping and ``optimizer.step()``, or None."""
     if not loss.is_cuda or loss.dtype != torch.float32 or loss.numel() != 1 or torch.compiler.is_compiling() or torch.cuda.is_current_stream_capturing():
         return None
-    if not _runs_as_written(optimizer) or (grad_clip_norm is not None and not grad_clip_norm >= 0):
+    if not _runs_as_written(optimizer) or (grad_clip_norm is not None and not (grad_clip_norm >= 0 and _clips_as_written())):
         return None
     update = Update(optimizer)
     if len(optimizer.param_groups) > _lib.host().ADAM_GROUPS or not all(update.add_group(g) for g in optimizer.param_groups):

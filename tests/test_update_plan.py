@@ -36,3 +36,17 @@ def test_decay_by_the_gradient_stays_stock():
     group = {**opt.param_groups[0], "fused": True}
     assert update.Update(opt).add_group(group)
     assert not update.Update(opt).add_group({**group, "decoupled_weight_decay": False})
+
+
+def test_clipping_that_was_replaced_is_called(monkeypatch):
+    assert update._clips_as_written()
+    known = torch.nn.utils.clip_grad_norm_
+
+    def clip(parameters, max_norm, *args, **kwargs):
+        return known(parameters, max_norm, *args, **kwargs)
+
+    for replaced in (clip, functools.wraps(known)(clip), functools.partial(known, norm_type=1.0)):
+        with monkeypatch.context() as m:
+            m.setattr(torch.nn.utils, "clip_grad_norm_", replaced)
+            assert not update._clips_as_written()
+    assert update._clips_as_written()
