@@ -33,6 +33,8 @@ def _runs_as_written(optimizer) -> bool:
         return False
     if not _is_torch_own(torch.optim.AdamW.step):   # replaced on the class
         return False
+    if "zero_grad" in optimizer.__dict__ or not _is_torch_own(torch.optim.AdamW.zero_grad):   # may keep the gradients, which are to be clipped ones then
+        return False
     step = optimizer.__dict__.get("step")   # a learning-rate scheduler wraps it to note that it has run
     return step is None or (getattr(step, "_wrapped_by_lr_sched", False) and getattr(step, "__wrapped__", None) is torch.optim.AdamW.step)
 

@@ -50,3 +50,13 @@ def test_clipping_that_was_replaced_is_called(monkeypatch):
             m.setattr(torch.nn.utils, "clip_grad_norm_", replaced)
             assert not update._clips_as_written()
     assert update._clips_as_written()
+
+
+def test_gradients_that_another_zero_grad_may_keep_are_clipped_by_the_stock_calls(monkeypatch):
+    opt = _optimizer()
+    with monkeypatch.context() as m:
+        m.setattr(torch.optim.AdamW, "zero_grad", lambda self, set_to_none=True: None)
+        assert not update._runs_as_written(opt)
+    assert update._runs_as_written(opt)
+    opt.zero_grad = lambda set_to_none=True: None
+    assert not update._runs_as_written(opt)
