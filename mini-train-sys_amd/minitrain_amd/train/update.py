@@ -11,7 +11,8 @@ from torch.optim import optimizer as _optimizer
 from minitrain_amd import _lib
 
 
-_TORCH_OWN = ("torch.optim.optimizer", "torch.optim.adam", "torch.optim.adamw", "torch.nn.utils.clip_grad")
+# torch._compile: wraps zero_grad, for the compiler to leave it alone
+_TORCH_OWN = ("torch.optim.optimizer", "torch.optim.adam", "torch.optim.adamw", "torch.nn.utils.clip_grad", "torch._compile")
 
 
 def _is_torch_own(function) -> bool:
