@@ -547,9 +547,9 @@ int mts_cross_entropy_bwd_unless_one(const void* logits, const int64_t* targets,
                                      const float* row_log_sum, const float* g_loss, const float* inv_count,
                                      void* d_logits, int64_t pitch, void* stream);
 
-/* Gradient of an embedding table: dw [V,H] f32, row r the sum of the rows of g [T,H] (act_dtype) whose id is r, in ascending order.
- * H a multiple of 4 up to 4096, T up to 2^18, V up to 2^20 (mts_embedding_bwd_supported); mts_embedding_bwd_preferred: where it is also
- * ahead of sorting the tokens.                                                              */
+/* Gradient of an embedding table: dw [V,H] f32, row r the sum of the rows of g [T,H] (act_dtype) whose id is r: up to 32 of them
+ * in ascending order, more in groups whose order depends on the ids alone.  H a multiple of 4 up to 4096, T up to 2^18, V up to
+ * 2^20 (mts_embedding_bwd_supported); mts_embedding_bwd_preferred: where it is also ahead of sorting the tokens.     */
 int mts_embedding_bwd_supported(int64_t T, int64_t V, int64_t H);
 int mts_embedding_bwd_preferred(int64_t T, int64_t V, int64_t H);
 int64_t mts_embedding_bwd_workspace_bytes(int64_t T, int64_t V, int64_t H);

@@ -1,5 +1,6 @@
-// The gradient of an embedding table: row r of dw is the fp32 sum, in token order, of the rows of g whose id is r, and zero where
-// there is none.
+// The gradient of an embedding table: row r of dw is the fp32 sum of the rows of g whose id is r, and zero where there is none.  Up to
+// kLongRow tokens are added in token order.  Of more, each wave adds a share of those in front of the whole segments (below), one of those behind them
+// and one of the segments' sums, and the waves' sums are added in turn: a fixed order for the same ids, which goes by where the row lies in the order.
 //
 // Bound by HBM at the table's size (50 257 x 768: 154 MB written, 38 MB of bf16 gradients read for 24 576 tokens), as long as the
 // tokens are sorted by id cheaply: a block owns a range of ids and looks through all of them (200 KB out of an L2, two passes), so that
