@@ -4,9 +4,9 @@
 // Bound by HBM: the norm reads every gradient once, the update reads parameter, gradient and both moments once and writes three of
 // them.  The coefficient is applied where the update reads the gradient, so no pass of its own scales the gradients, and the
 // parameters of a model share one launch: a block finds its tensor from the launch's table (a step of a small model is otherwise a
-// few hundred microseconds of launches).  162 M parameters of fp32 (a four-layer decoder with 50 257 words): norm 149 us (4.4 TB/s), update
-// 946 us (4.8 TB/s), where stock clipping and fused AdamW took 200 + 277 and 1129 us, and some 60 us in small kernels; with them the
-// step of 24 576 tokens 15.53 -> 14.62 ms, the rest of it from enqueuing the update ahead of the host's look at the flag.
+// few hundred microseconds of launches).  162 M parameters of fp32 (a four-layer decoder with 50 257 words): norm 151 us (4.3 TB/s), update
+// 824 us (5.5 TB/s; 946 where every gradient is written back), where stock clipping and fused AdamW took 200 + 277 and 1129 us, and some 60 us in small kernels; with them the
+// step of 24 576 tokens 15.53 -> 14.62 ms with all gradients written back and another 0.12 less without, the rest of it from enqueuing the update ahead of the host's look at the flag.
 #include "mts_common.h"
 
 namespace {
