@@ -5,7 +5,7 @@ reference's ``MiniTransformer`` (minitrain/model/transformer.py:10-170) with its
 (minitrain/model/blocks.py:19-60, 105-135) and rotary cache (minitrain/model/rotary.py), so a
 state dict of one loads into the other.  Every operator goes through the ``ops`` backend: the
 ``hip`` backend supplies the two MoE operators (and the router projection and route counts the
-router module asks for), the other six stay on stock PyTorch-ROCm.
+router module asks for) and takes the other operators where its kernels do; what they do not take stays on stock PyTorch-ROCm.
 """
 
 import math
