@@ -354,6 +354,19 @@ int mts_moe_fwd_few_rows(const void* x, const void* w1, const void* w2, int weig
                          int H, int I, int act_dtype, void* pre_act, void* post_act, void* y,
                          void* stream);
 
+/* The whole forward pass of the layer for few tokens (up to 32; up to 16 experts, 8 with fp32 weights; 16-bit activations) in two launches: outputs as
+ * mts_moe_head_fwd, then mts_moe_fwd_few_rows with the routing weights and mts_moe_combine without them, all of them written;
+ * weight_dtype as there.  pre_act, load_balance and load_stats may be NULL; arrived: H / 32 words, rounded up, of scratch.  */
+int mts_moe_few_tokens_supported(int act_dtype, int weight_dtype, int64_t T, int K, int E, int H, int I);
+int mts_moe_few_tokens_preferred(int act_dtype, int weight_dtype, int64_t T, int K, int E, int H, int I);
+int mts_moe_few_tokens_fwd(const void* x, const float* w_r, const void* w1, const void* w2, int weight_dtype,
+                           int64_t T, int H, int E, int I, int K, int normalize, int act_dtype,
+                           float* logits, float* weights, int32_t* indices, void* weights_act,
+                           float* prob_mean, float* z_loss, float* entropy, int32_t* counts,
+                           float* load_balance, float* load_stats, int32_t* expert_start, int32_t* s_scatter,
+                           int32_t* s_reverse, int32_t* x_gather, void* pre_act, void* post_act, void* y,
+                           int32_t* arrived, void* out, void* stream);
+
 /* Replaces _token_gather_weighted_sum_kernel (fused_moe_kernels.py:451-498):
  * out[t] = addend[t] + sum_k w[t,k] * y[s_reverse[t*K+k]]  (fp32 sum, one rounding);
  * weights == NULL gives the unweighted sum used for dx; addend [T,H] (act_dtype) may be NULL

@@ -346,6 +346,28 @@ bool copies_masters(const Tensor& x, const Tensor& w1, const Tensor& w2, int64_t
            !reads_masters(x, w1, w2, TK, opt);
 }
 
+// The expert weights as the forward kernels read them: as they are, or copies in the activation dtype.
+std::pair<Tensor, Tensor> forward_weights(const Tensor& x, const Tensor& w1, const Tensor& w2, int64_t TK, const Options& opt) {
+    if (reads_masters(x, w1, w2, TK, opt)) return {w1, w2};
+    void* stream = stream_of(x);
+    if (!copies_masters(x, w1, w2, TK, opt)) return {stage(w1, false, x.scalar_type(), stream), stage(w2, false, x.scalar_type(), stream)};
+    Tensor copy1 = at::empty(w1.sizes(), x.options()), copy2 = at::empty(w2.sizes(), x.options());
+    check(mts_moe_cast_weights_pair(ptr_as<float>(w1), ptr(copy1), w1.numel(), ptr_as<float>(w2), ptr(copy2), w2.numel(), dtype_code(x), stream),
+          "mts_moe_cast_weights_pair");
+    return {copy1, copy2};
+}
+
+// What the backward pass of a forward pass needs; `w1`, `w2`: the weights that the kernels read, kept where they are copies that the backward GEMMs take.
+void keep(Saved& s, const Tensor& x, const Tensor& w1_in, const Tensor& w2_in, const Tensor& w1, const Tensor& w2, const Tensor& pre_act, const Tensor& post_act,
+          const Tensor& weights, const Routing& r) {
+    s.x = x, s.w1 = w1_in, s.w2 = w2_in, s.pre_act = pre_act, s.post_act = post_act, s.weights = weights;
+    s.expert_start = r.expert_start, s.x_gather = r.x_gather, s.s_scatter = r.s_scatter, s.s_reverse = r.s_reverse;
+    if (stored_layout(dtype_code(x), x.size(1), w1_in.size(1) / 2)) {   // the backward GEMMs read the weights as stored: they reuse casts made here
+        if (!w1.is_same(w1_in)) s.staged1 = w1;
+        if (!w2.is_same(w2_in)) s.staged2 = w2;
+    }
+}
+
 // Gate/up + SwiGLU, down projection and combine for routes that are already sorted.  `weights`: flat, activation dtype.
 // `post_act` [TK,I] and `y` [TK,H]: scratch that the caller has, or undefined; `w1`, `w2`: copies of master weights that the caller has made
 Tensor experts_forward(const Tensor& x, const Tensor& w1_in, const Tensor& w2_in, const Tensor& weights, const Routing& r, const Options& opt, Saved& s,
@@ -355,21 +377,8 @@ Tensor experts_forward(const Tensor& x, const Tensor& w1_in, const Tensor& w2_in
     const int act = dtype_code(dtype);
     void* stream = stream_of(x);
     const bool weighted = opt.on(WEIGHTED_POST);
-    const bool few_masters = reads_masters(x, w1_in, w2_in, TK, opt);
-    const bool few = few_masters || mts_moe_fwd_few_rows_preferred(act, act, T, TK, E, H, I);
-    const bool given = w1.defined();
-    if (few_masters) {
-        w1 = w1_in;
-        w2 = w2_in;
-    } else if (!given && copies_masters(x, w1_in, w2_in, TK, opt)) {
-        w1 = at::empty(w1_in.sizes(), x.options());
-        w2 = at::empty(w2_in.sizes(), x.options());
-        check(mts_moe_cast_weights_pair(ptr_as<float>(w1_in), ptr(w1), w1_in.numel(), ptr_as<float>(w2_in), ptr(w2), w2_in.numel(), act, stream),
-              "mts_moe_cast_weights_pair");
-    } else if (!given) {
-        w1 = stage(w1_in, false, dtype, stream);
-        w2 = stage(w2_in, false, dtype, stream);
-    }
+    const bool few = reads_masters(x, w1_in, w2_in, TK, opt) || mts_moe_fwd_few_rows_preferred(act, act, T, TK, E, H, I);
+    if (!w1.defined()) std::tie(w1, w2) = forward_weights(x, w1_in, w2_in, TK, opt);
     // The routing weight is applied where the activation is formed: post_act = s * silu(g) * u.  The down projection then
     // yields s * y, the combine is a plain sum, and post_act is at the same time the operand of the dW2 GEMM, so it is kept
     // for the backward pass instead of being written again there.
@@ -401,13 +410,7 @@ Tensor experts_forward(const Tensor& x, const Tensor& w1_in, const Tensor& w2_in
     }
     Tensor out = at::empty({T, H}, x.options());
     check(mts_moe_combine(ptr(y), weighted ? nullptr : ptr(weights), nullptr, ptr_as<int32_t>(r.s_reverse), T, K, H, act, ptr(out), stream), "mts_moe_combine");
-    s.x = x, s.w1 = w1_in, s.w2 = w2_in, s.pre_act = pre_act, s.weights = weights;
-    s.expert_start = r.expert_start, s.x_gather = r.x_gather, s.s_scatter = r.s_scatter, s.s_reverse = r.s_reverse;
-    if (weighted) s.post_act = post_act;
-    if (stored_layout(act, H, I)) {   // the backward GEMMs read the weights as stored: they reuse casts made here
-        if (!w1.is_same(w1_in)) s.staged1 = w1;
-        if (!w2.is_same(w2_in)) s.staged2 = w2;
-    }
+    keep(s, x, w1_in, w2_in, w1, w2, pre_act, weighted ? post_act : Tensor(), weights, r);
     return out;
 }
 
@@ -653,8 +656,11 @@ LayerForward layer_forward(const Tensor& x_, const Tensor& w_r_, const Tensor& w
     const int64_t T = x.size(0), H = x.size(1), E = w_r.size(0), TK = T * K, I = w1.size(1) / 2;
     const auto dtype = x.scalar_type();
     const bool narrow = dtype != at::kFloat, limited = capacity >= 0, alone = opt.on(NO_BACKWARD), few = E <= kFewExperts;
+    // few tokens: all of it behind one entry point, in two launches
+    const bool whole = narrow && !limited && opt.on(WEIGHTED_POST) &&
+                       mts_moe_few_tokens_preferred(dtype_code(dtype), reads_masters(x, w1, w2, TK, opt) ? MTS_F32 : dtype_code(dtype), T, K, E, H, I);
     const bool chained = few || mts_moe_wide_head_supported(T, H, E, K);   // projection, post-process and routing metadata behind one entry point
-    const int64_t ws_bytes = few ? mts_moe_head_workspace_bytes(T, K, E) : chained ? mts_moe_wide_head_workspace_bytes(T, E) : mts_moe_router_route_workspace_bytes(T, K, E);
+    const int64_t ws_bytes = whole ? (H + 31) / 32 * 4 : few ? mts_moe_head_workspace_bytes(T, K, E) : chained ? mts_moe_wide_head_workspace_bytes(T, E) : mts_moe_router_route_workspace_bytes(T, K, E);
     f.w_r = w_r;
     f.weights = f32({T, K}, x);
     // The integer results in one allocation and the fp32 statistics in another: a caller may save all results together, which torch refuses
@@ -694,6 +700,20 @@ LayerForward layer_forward(const Tensor& x_, const Tensor& w_r_, const Tensor& w
     }
     void* load_stats = limited ? nullptr : ptr(f.load_stats);
     void* cast_weights = narrow && !limited ? ptr(weights_act) : nullptr;
+    if (whole) {
+        const auto [w1_read, w2_read] = forward_weights(x, w1, w2, TK, opt);
+        Tensor pre_act;
+        if (!alone) pre_act = at::empty({TK, 2 * I}, x.options()), post_act = at::empty({TK, I}, x.options());
+        f.out = at::empty({T, H}, x.options());
+        check(mts_moe_few_tokens_fwd(ptr(x), ptr_as<float>(w_r), ptr(w1_read), ptr(w2_read), dtype_code(w1_read), T, H, E, I, K, normalize, dtype_code(dtype),
+                                     ptr_as<float>(f.logits), ptr_as<float>(f.weights), ptr_as<int32_t>(f.indices), cast_weights, ptr_as<float>(f.prob_mean),
+                                     ptr_as<float>(f.z_loss), ptr_as<float>(f.entropy), ptr_as<int32_t>(f.counts), ptr_as<float>(f.load_balance),
+                                     static_cast<float*>(load_stats), ptr_as<int32_t>(r.expert_start), ptr_as<int32_t>(r.s_scatter), ptr_as<int32_t>(r.s_reverse),
+                                     ptr_as<int32_t>(r.x_gather), ptr(pre_act), ptr(post_act), ptr(y), ptr_as<int32_t>(ws), ptr(f.out), stream_of(x)),
+              "mts_moe_few_tokens_fwd");
+        keep(f.s, x, w1, w2, w1_read, w2_read, pre_act, post_act, weights_act, r);
+        return f;
+    }
     Tensor copy1, copy2;   // of master weights: made beside the head
     if (chained) {
         MtsCast casts[2];

@@ -8,59 +8,11 @@
 // steps of 64 k are in flight before the first product.  fp32 weights are rounded on the way, as the cast in front of the
 // large tiles does.  16 tokens, top-2 of 8 experts: gate/up 17.3 -> 11.6 us, down 14.6 -> 5.5; with fp32 weights 17.9 and 8.3,
 // and no cast (20 us) in front.
-#include "mts_common.h"
+#include "mts_few_block.h"
 
 namespace {
 
-template <typename ET>
-struct Few;
-template <>
-struct Few<bf16_t> {
-    typedef bf16x8 frag;
-    typedef bf16x4 quad;
-    static __device__ __forceinline__ f32x4 mul(frag a, frag b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
-};
-template <>
-struct Few<mts_f16_t> {
-    typedef mts_f16x8 frag;
-    typedef mts_f16x4 quad;
-    static __device__ __forceinline__ f32x4 mul(frag a, frag b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
-};
-
-constexpr int kWaves = 4, kThreads = kWaves * MTS_WAVE;
-constexpr int kCols = 32;
-constexpr uint32_t kOutside = 0x80000000u;   // behind the end of every operand (smaller than 2 GiB): reads as zero
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t operand(const void* p, int64_t bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)(uint32_t)bytes, 0x00020000);
-}
-
-// eight consecutive k of a row as they lie in memory, and as a fragment
-template <typename ET, typename WT>
-struct Chunk;
-template <typename ET>
-struct Chunk<ET, ET> {
-    u32x4 v;
-    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t r, uint32_t element) {
-        v = __builtin_amdgcn_raw_buffer_load_b128(r, (int)(element == kOutside ? kOutside : element * 2), 0, 0);
-    }
-    __device__ __forceinline__ typename Few<ET>::frag frag() const { return __builtin_bit_cast(typename Few<ET>::frag, v); }
-};
-template <typename ET>
-struct Chunk<ET, float> {
-    f32x4 a, b;
-    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t r, uint32_t element) {
-        const uint32_t at = element == kOutside ? kOutside : element * 4;
-        a = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)at, 0, 0));
-        b = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)at, 16, 0));
-    }
-    __device__ __forceinline__ typename Few<ET>::frag frag() const {
-        typename Few<ET>::frag f;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) f[j] = (ET)a[j], f[4 + j] = (ET)b[j];
-        return f;
-    }
-};
+using namespace mts_few;
 
 struct FewRows {
     const void *A, *W;

@@ -61,6 +61,9 @@ SIGNATURES = {
     "mts_moe_fwd_few_rows_supported": (_i, [_i, _i, _l, _l, _i, _i, _i]),
     "mts_moe_fwd_few_rows_preferred": (_i, [_i, _i, _l, _l, _i, _i, _i]),
     "mts_moe_fwd_few_rows": (_i, [_p, _p, _p, _i, _p, _p, _p, _p, _l, _i, _i, _i, _i, _i, _p, _p, _p, _p]),
+    "mts_moe_few_tokens_supported": (_i, [_i, _i, _l, _i, _i, _i, _i]),
+    "mts_moe_few_tokens_preferred": (_i, [_i, _i, _l, _i, _i, _i, _i]),
+    "mts_moe_few_tokens_fwd": (_i, [_p, _p, _p, _p, _i, _l, _i, _i, _i, _i, _i, _i] + [_p] * 20),
     "mts_moe_combine": (_i, [_p, _p, _p, _p, _l, _i, _i, _i, _p, _p]),
     "mts_moe_wide_head_supported": (_i, [_l, _i, _i, _i]),
     "mts_moe_wide_head_workspace_bytes": (_l, [_l, _i]),

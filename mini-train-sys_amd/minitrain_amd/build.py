@@ -23,7 +23,7 @@ LIB_DIR = os.path.join(PKG_DIR, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libmts_moe.so")
 HOST_SOURCE = os.path.join(CSRC, "host", "mts_host.cpp")
 HOST_PATH = os.path.join(LIB_DIR, "_host.so")
-SOURCES = ("mts_router.hip", "mts_router_linear.hip", "mts_router_wide.hip", "mts_route.hip", "mts_capacity.hip", "mts_combine.hip", "mts_dense.hip", "mts_attention.hip", "mts_optim.hip", "mts_embedding.hip", "mts_few_rows.hip", "mts_gemm.hip", "mts_gemm_f16.hip", "mts_gemm_f32.hip", "mts_probe.hip", "mts_tuning.hip")
+SOURCES = ("mts_router.hip", "mts_router_linear.hip", "mts_router_wide.hip", "mts_route.hip", "mts_capacity.hip", "mts_combine.hip", "mts_dense.hip", "mts_attention.hip", "mts_optim.hip", "mts_embedding.hip", "mts_few_rows.hip", "mts_few_tokens.hip", "mts_gemm.hip", "mts_gemm_f16.hip", "mts_gemm_f32.hip", "mts_probe.hip", "mts_tuning.hip")
 
 FLAGS = [
     "-O3",
