@@ -569,9 +569,17 @@ int64_t mts_embedding_bwd_workspace_bytes(int64_t T, int64_t V, int64_t H);
 int mts_embedding_bwd(const void* g, const int64_t* ids, int64_t T, int V, int H, int act_dtype, float* dw,
                       void* workspace, int64_t workspace_bytes, void* stream);
 
+/* A dense projection y [T,N] = x W^T, x [T,K] and w [N,K] dense bf16 or fp16 (w rounded by the caller), and the gradient
+ * dx [T,K] = g W, by the kernels of mts_moe_fwd_down and mts_moe_bwd_dx.  N and K multiples of 8 that are multiples of 64
+ * or at least 256.  _preferred: where they are ahead of the library's product.                    */
+int mts_linear_rows_supported(int act_dtype, int64_t T, int N, int K);
+int mts_linear_fwd_preferred(int act_dtype, int64_t T, int N, int K);
+int mts_linear_fwd(const void* x, const void* w, int64_t T, int N, int K, int act_dtype, void* y, void* stream);
+int mts_linear_dx_preferred(int act_dtype, int64_t T, int N, int K);
+int mts_linear_dx(const void* g, const void* w, int64_t T, int N, int K, int act_dtype, void* dx, void* stream);
 /* Weight gradient of a dense projection y = x W^T: dw [N,K] f32 = g^T x, g [T,N] and x [T,K] dense
  * bf16 or fp16, fp32 sums in a fixed order.  N and K multiples of 8, at most 32 tiles of 256 x 256,
- * T at least 1024 (mts_linear_dw_supported).                                               */
+ * T at least 128 (mts_linear_dw_supported).                                               */
 int mts_linear_dw_supported(int act_dtype, int64_t T, int N, int K);
 int64_t mts_linear_dw_workspace_bytes(int64_t T, int N, int K);
 int mts_linear_dw(const void* g, const void* x, int64_t T, int N, int K, int act_dtype, float* dw,

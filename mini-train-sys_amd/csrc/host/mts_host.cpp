@@ -1037,15 +1037,37 @@ bool rows_fit(const Tensor& g) {
     return g.stride(1) == 1 && g.stride(0) >= g.size(1) && g.stride(0) % 8 == 0 && aligned16(g) && end * g.element_size() <= (int64_t)g.storage().nbytes();
 }
 
-// A projection under autocast: the product is the library's, the gradient of its fp32 weight is summed in fp32 here.
+// Operands of a projection under autocast.
+bool projection_operands(const Tensor& x, const Tensor& w) {
+    return all_plain(x, w) && on_one_gpu(x, w) && x.dim() >= 2 && w.dim() == 2 && w.scalar_type() == at::kFloat &&
+           (x.scalar_type() == at::kBFloat16 || x.scalar_type() == at::kHalf) && x.size(-1) == w.size(1) && x.numel() > 0 &&
+           at::autocast::is_autocast_enabled(at::kCUDA) && at::autocast::get_autocast_dtype(at::kCUDA) == x.scalar_type();
+}
+// The product, where its kernel is ahead of the library's and takes the activations as they lie; else undefined.
+Tensor own_product(const Tensor& x, const Tensor& rounded) {
+    const int64_t N = rounded.size(0), K = rounded.size(1), T = x.numel() / K;
+    if (!mts_linear_fwd_preferred(dtype_code(x), T, N, K) || !x.is_contiguous() || !aligned16(x)) return {};
+    const Tensor w = dense16(rounded);
+    c10::SmallVector<int64_t, 4> size(x.sizes());
+    size.back() = N;
+    Tensor y = at::empty(size, x.options());
+    check(mts_linear_fwd(ptr(x), ptr(w), T, N, K, dtype_code(x), ptr(y), stream_of(x)), "mts_linear_fwd");
+    return y;
+}
+
+// A projection whose fp32 weight wants a gradient, which is summed in fp32 here; the products are the library's or ours.
 bool linear_supported(const Tensor& x, const Tensor& w) {
-    if (!(at::GradMode::is_enabled() && w.requires_grad() && all_plain(x, w) && on_one_gpu(x, w) && x.dim() >= 2 && w.dim() == 2 &&
-          w.scalar_type() == at::kFloat && (x.scalar_type() == at::kBFloat16 || x.scalar_type() == at::kHalf) && x.size(-1) == w.size(1) && x.numel() > 0))
-        return false;
-    if (!at::autocast::is_autocast_enabled(at::kCUDA) || at::autocast::get_autocast_dtype(at::kCUDA) != x.scalar_type()) return false;
+    if (!(at::GradMode::is_enabled() && w.requires_grad() && projection_operands(x, w))) return false;
     const int64_t T = x.numel() / x.size(-1), N = w.size(0), K = w.size(1);
     return linear_in_rounds(x, T, N, K) || mts_linear_dw_supported(dtype_code(x), T, N, K);
 }
+
+// One that wants none: the weight rounded as autocast does it, and kept by it for as long.
+bool linear_alone_supported(const Tensor& x, const Tensor& w) {
+    if ((at::GradMode::is_enabled() && (x.requires_grad() || w.requires_grad())) || !projection_operands(x, w)) return false;
+    return x.is_contiguous() && aligned16(x) && mts_linear_fwd_preferred(dtype_code(x), x.numel() / x.size(-1), w.size(0), w.size(1));
+}
+Tensor linear_alone(const Tensor& x, const Tensor& w) { return own_product(x, at::autocast::cached_cast(x.scalar_type(), w, c10::DeviceType::CUDA)); }
 
 struct Linear : torch::autograd::Function<Linear> {
     static variable_list in_rounds(AutogradContext* ctx, const Tensor& g, const Tensor& x, const Tensor& rounded, int64_t T, int64_t N, int64_t K) {
@@ -1073,7 +1095,8 @@ struct Linear : torch::autograd::Function<Linear> {
         const Tensor rounded = w.to(x.scalar_type());
         ctx->save_for_backward({x, rounded});
         ctx->saved_data["weight"] = w;   // not kept as it is now: the caller may change it before the backward pass, as under stock autocast
-        return at::linear(x, rounded);
+        const Tensor own = own_product(x, rounded);
+        return own.defined() ? own : at::linear(x, rounded);
     }
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
         const variable_list s = ctx->get_saved_variables();
@@ -1099,7 +1122,13 @@ struct Linear : torch::autograd::Function<Linear> {
         }
         const Tensor g = dense16(grads[0].reshape({T, N})), in = dense16(x.reshape({T, K}));
         Tensor dx, dw;
-        if (ctx->needs_input_grad(0)) dx = at::matmul(g, rounded).view(x.sizes());
+        if (ctx->needs_input_grad(0)) {
+            if (mts_linear_dx_preferred(dtype_code(x), T, N, K)) {
+                const Tensor w = dense16(rounded);
+                dx = at::empty(x.sizes(), x.options());
+                check(mts_linear_dx(ptr(g), ptr(w), T, N, K, dtype_code(x), ptr(dx), stream_of(x)), "mts_linear_dx");
+            } else dx = at::matmul(g, rounded).view(x.sizes());
+        }
         if (ctx->needs_input_grad(1)) {
             dw = f32({N, K}, x);
             const int64_t ws_bytes = mts_linear_dw_workspace_bytes(T, N, K);
@@ -1598,6 +1627,11 @@ PYBIND11_MODULE(_host, m) {
     m.def("linear", [](const Tensor& x, const Tensor& w) {
         c10::OptionalDeviceGuard guard(x.device());
         return Linear::apply(x, w);
+    });
+    m.def("linear_alone_supported", &linear_alone_supported);
+    m.def("linear_alone", [](const Tensor& x, const Tensor& w) {
+        c10::OptionalDeviceGuard guard(x.device());
+        return linear_alone(x, w);
     });
     m.def("embedding_supported", &embedding_supported);
     m.def("embedding", [](const Tensor& ids, const Tensor& w, at::ScalarType type) {

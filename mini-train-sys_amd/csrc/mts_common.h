@@ -137,6 +137,8 @@ int mts_moe_bwd_dx_f16(const void* d_pre_act, const void* w1, int w1_as_stored, 
 int mts_moe_bwd_dw2_f16(const void* d_out, const void* weighted_act, const int32_t* x_gather,
                         const int32_t* expert_start, int64_t T, int K, int E, int H, int I, int act_dtype,
                         int grad_dtype, void* d_w2, void* workspace, int64_t workspace_bytes, void* stream);
+int mts_linear_fwd_f16(const void* x, const void* w, int64_t T, int N, int K, int act_dtype, void* y, void* stream);
+int mts_linear_dx_f16(const void* g, const void* w, int64_t T, int N, int K, int act_dtype, void* dx, void* stream);
 int mts_linear_dw_tiles_f16(const void* g, const void* x, int64_t T, int N, int K, float* part, void* stream);
 int mts_linear_dw_rounds_f16(const void* g, int64_t ldg, const void* x, int64_t T, int N, int K, float* dw, float* part, void* stream);
 int mts_linear_dx_rounds_f16(const void* g, int64_t ldg, const void* w, int64_t T, int N, int K, void* dx, float* part, void* stream);

@@ -143,7 +143,7 @@ struct RowsParams {
     int b_rows;
     int N;                     // output columns (SwiGLU: I, B holds 2I rows)
     int Kdim;
-    const int32_t* expert_start;
+    const int32_t* expert_start;   // NULL: one expert, all TK rows are its own
     int E;
     bf16_t* C;                 // plain: [TK,N]; SwiGLU: pre_act [TK,2N]; DY1: d_pre_act [TK,2N]
     bf16_t* C2;                // SwiGLU: post_act [TK,N]; DY1: weighted_act [TK,N]
@@ -155,7 +155,8 @@ struct RowsParams {
     int64_t TK;                // rows of every output
     int n_tiles;               // column tiles per m-tile (set by the launcher, like by_n_tiles and by_group)
     Divider by_n_tiles, by_group;   // by n_tiles and by the tiles of a group
-    int xcd_ranges;            // block -> tile mapping: 1 = every XCD takes a contiguous range of m-tiles
+    int flat;                  // block -> tile mapping: tiles in their order, columns fastest (one expert, no more tiles than the chip has CUs)
+    int xcd_ranges;            // else: 1 = every XCD takes a contiguous range of m-tiles
     int n_groups;              // with xcd_ranges: the n-tiles are walked in this many groups, all m-tiles of the range per group
     int reverse;               // with xcd_ranges: the range's m-tiles are walked from the last to the first
     int tail_slots;            // with xcd_ranges: blocks an XCD runs at a time; when the tiles behind its last whole round
@@ -640,7 +641,8 @@ __device__ __forceinline__ bool find_rows_tile(const RowsParams& p, int b, int& 
     // up to 64 experts: lane l reads expert_start[l] and [l + 1] once, for the count of m-tiles and for the search
     const bool in_regs = p.E <= MTS_WAVE;
     const int lane = threadIdx.x % MTS_WAVE;
-    const int w0 = p.expert_start[min(lane, p.E)], w1 = p.expert_start[min(lane + 1, p.E)];   // equal behind the last expert
+    int w0 = lane ? (int)p.TK : 0, w1 = (int)p.TK;   // no table: one expert has all rows
+    if (p.expert_start) w0 = p.expert_start[min(lane, p.E)], w1 = p.expert_start[min(lane + 1, p.E)];   // equal behind the last expert
     const int wnt = (w1 - w0 + BM - 1) / BM, wincl = wave_scan(wnt);   // in_regs: the lane's m-tiles, and those up to its last one
     const int xcd = b % kXcds;
     int j = b / kXcds;
@@ -648,7 +650,9 @@ __device__ __forceinline__ bool find_rows_tile(const RowsParams& p, int b, int& 
     int tile = xcd + kXcds * k;
     parts = 1;      // pieces the tile is cut into: this block computes piece `part`
     int part = 0;
-    if (p.xcd_ranges && p.sched) {
+    if (p.flat) {
+        tile = p.by_n_tiles.quotient(b, ntile);
+    } else if (p.xcd_ranges && p.sched) {
         // the XCD's range of m-tiles comes from the table (n-tile groups and cut tiles are not combined with it); a block
         // the table leaves without work finds that out with one load
         const int my = p.sched[kXcds + xcd];
@@ -2713,6 +2717,12 @@ dim3 rows_grid(RowsParams& p, int64_t TK) {
         while (weight_bytes / p.n_groups > kL2Bytes / 2 && p.n_tiles % (2 * p.n_groups) == 0 && p.n_tiles / (2 * p.n_groups) >= 4)
             p.n_groups *= 2;
     set_dividers(p);
+    // Without a table the tiles are known: ranges of whole m-tiles would leave some XCDs with more than their CUs hold and others with CUs idle (1500 rows
+    // of 768 to 2304: 18.3 -> 10.2 us)
+    if (!p.expert_start && std::is_same<T, WsSmall>::value && m_tiles<T>(TK, 1) * p.n_tiles <= kXcds * kCusPerXcd) {
+        p.flat = 1;
+        return dim3((unsigned)(m_tiles<T>(TK, 1) * p.n_tiles));
+    }
     const int64_t m_groups = (m_tiles<T>(TK, p.E) + kXcds - 1) / kXcds;
     if (!p.xcd_ranges) p.tail_slots = 0;
     // tiles that are cut in two add at most tail_slots / 2 blocks per XCD; one more block writes the schedule (dO*W2 only)
@@ -3316,7 +3326,7 @@ extern "C" int MTS_GEMM_ENTRY(mts_moe_bwd_dw1)(const void* d_pre_act, const void
 // an XCD's 32 CUs in one round; a segment's tiles run on one XCD, and a second kernel adds the segments' partial results
 // in their order.  24 576 rows: 768 x 768 166 -> 46 us (36 and the sum), 2304 x 768 194 -> 97 us against the library's products, which
 // the widening of their 16-bit results follows; both gradients of the projection 193 -> 83 and 288 -> 206, and no slower
-// down to 1024 rows (89 -> 70), the least that is measured.
+// down to 1024 rows (89 -> 70).  Fewer rows wait for the host, which spends 20 us on each of the library's launches and 4 on these.
 // ---------------------------------------------------------------------------
 namespace {
 constexpr int kLinearTiles = 32;   // CUs of an XCD
@@ -3327,7 +3337,10 @@ LinearSplit linear_split(int64_t T, int N, int K) {
     LinearSplit s;
     s.tiles = ((N + DwWsWide::BM - 1) / DwWsWide::BM) * ((K + DwWsWide::BN - 1) / DwWsWide::BN);
     const int64_t most = kXcds * (kLinearTiles / s.tiles > 0 ? kLinearTiles / s.tiles : 1);
-    const int64_t rows = ((T + most - 1) / most + DwWsWide::BKS - 1) / DwWsWide::BKS * DwWsWide::BKS;
+    int64_t rows = ((T + most - 1) / most + DwWsWide::BKS - 1) / DwWsWide::BKS * DwWsWide::BKS;
+    // A segment's fp32 tiles are written and read again: not for fewer than 256 rows (us, 64 / 128 / 256 / 512: 768 x 768 512 rows 18.6 / 14.4 / 14.5 / 15.8,
+    // 1024 24.7 / 19.3 / 17.0 / 18.9, 2048 24.7 / 25.0 / 22.1 / 21.5; 2304 x 768 512 29.6 / 24.9 / 20.4 / 19.3, 1024 28.5 / 30.3 / 28.0 / 24.7).
+    if (rows < 256) rows = 256;
     s.rows = (int)rows;
     s.segments = (int)((T + rows - 1) / rows);
     return s;
@@ -3508,9 +3521,60 @@ static int linear_dw_tiles(const void* g, const void* x, int64_t T, int N, int K
     return MTS_OK;
 }
 
+// y = x W^T and dx = g W by the tiles of the expert GEMMs, one expert with all rows
+static int linear_rows(int kind, const void* a, int64_t lda, const void* w, int64_t T, int N, int Kdim, bool b_kmajor, void* c, void* stream) {
+    RowsParams p = {};
+    p.A = (const bf16_t*)a; p.a_rows = T; p.lda = (int)lda;
+    p.B = (const bf16_t*)w; p.b_rows = N;
+    p.N = N; p.Kdim = Kdim; p.E = 1;
+    p.C = (bf16_t*)c; p.TK = T;
+    return launch_rows_any<EPI_PLAIN>(kind, p, T, (hipStream_t)stream, b_kmajor);
+}
+extern "C" int MTS_GEMM_ENTRY(mts_linear_fwd)(const void* x, const void* w, int64_t T, int N, int K, int act_dtype, void* y, void* stream) {
 #ifndef MTS_GEMM_F16
+    if (act_dtype == MTS_F16) return mts_linear_fwd_f16(x, w, T, N, K, act_dtype, y, stream);
+#endif
+    if (!x || !w || !y) return MTS_ERR_NULL;
+    if (act_dtype != MTS_GEMM_DTYPE) return MTS_ERR_DTYPE;
+    if (!mts_linear_rows_supported(act_dtype, T, N, K)) return MTS_ERR_SHAPE;
+    if (!mts_aligned16(x) || !mts_aligned16(w) || !mts_aligned16(y)) return MTS_ERR_ALIGN;
+    return linear_rows(K_DOWN, x, K, w, T, N, K, false, y, stream);
+}
+extern "C" int MTS_GEMM_ENTRY(mts_linear_dx)(const void* g, const void* w, int64_t T, int N, int K, int act_dtype, void* dx, void* stream) {
+#ifndef MTS_GEMM_F16
+    if (act_dtype == MTS_F16) return mts_linear_dx_f16(g, w, T, N, K, act_dtype, dx, stream);
+#endif
+    if (!g || !w || !dx) return MTS_ERR_NULL;
+    if (act_dtype != MTS_GEMM_DTYPE) return MTS_ERR_DTYPE;
+    if (!mts_linear_rows_supported(act_dtype, T, N, K)) return MTS_ERR_SHAPE;
+    if (!mts_aligned16(g) || !mts_aligned16(w) || !mts_aligned16(dx)) return MTS_ERR_ALIGN;
+    return linear_rows(K_DX, g, N, w, T, K, N, true, dx, stream);
+}
+
+#ifndef MTS_GEMM_F16
+extern "C" int mts_linear_rows_supported(int act_dtype, int64_t T, int N, int K) {
+    return (act_dtype == MTS_BF16 || act_dtype == MTS_F16) && rows_pipelined(K) && rows_kmajor_ok(K_DX, N) && check_common(T, 1, N, K, 0) == MTS_OK;
+}
+// Against the library's product, us of the GPU, library / here.  Where a CU has at most one small tile: 768 to 2304 1024 rows 11.1 / 9.4, 1500 11.2 / 10.2, 1792
+// 11.6 / 11.8; 768 to 768 512 rows 5.8 / 8.0, 2048 8.3 / 8.1, 4096 11.3 / 9.5.  (The host spends 20 us on a call of the library and 4 on this: a decoder with
+// so few rows waits for it, and the evaluation of 1024 tokens by two layers takes 311 us for 478.)  Narrow ones up to 8192 rows: 768 to 768 6144 12.5 / 12.9,
+// 8192 15.2 / 14.5; 768 to 1000 6144 18.7 / 14.3; 1024 to 1024 6144 16.6 / 16.8, 8192 19.8 / 19.3.  And from a whole round of large tiles on: 768 to 768
+// 24 576 49.4 / 36.3, 32 768 42.9 / 39.1, 49 152 58.2 / 59.3; 768 to 1000 24 576 51.6 / 42.9; 512 to 768 24 576 33.2 / 26.6.  Not between the two (768 to
+// 768 11 000 17.9 / 20.8, 21 000 23.7 / 35.4), where half of a round would be idle (768 to 512 32 768 24.1 / 27.2), with longer sums (1024 to 1024 24 576
+// 46.1 / 48.6) and where it is wide (768 to 2304 4096 19.3 / 21.6, 24 576 83.3 / 87.9).
+extern "C" int mts_linear_fwd_preferred(int act_dtype, int64_t T, int N, int K) {
+    if (!mts_linear_rows_supported(act_dtype, T, N, K) || K > 1024) return 0;
+    if (small_tiles_pay(K_DOWN, T, 1, N)) return 1;
+    if (N > 1024) return 0;
+    const int64_t tiles = (T + WsWide::BM - 1) / WsWide::BM * ((N + WsWide::BN - 1) / WsWide::BN);
+    return T <= 8192 || (K < 1024 && N > 512 && tiles > kXcds * kCusPerXcd);
+}
+// (768 to 2304: 1024 rows 14.3 / 16.4, 2048 22.5 / 17.0, 4096 26.9 / 42.6; 768 to 768: 1024 rows 7.9 / 8.2, 2048 10.7 / 8.5, 4096 13.4 / 18.2)
+extern "C" int mts_linear_dx_preferred(int act_dtype, int64_t T, int N, int K) {
+    return mts_linear_rows_supported(act_dtype, T, N, K) && N <= 3072 && small_tiles_pay(K_DX, T, 1, K);
+}
 extern "C" int mts_linear_dw_supported(int act_dtype, int64_t T, int N, int K) {
-    if ((act_dtype != MTS_BF16 && act_dtype != MTS_F16) || N < 8 || K < 8 || N % 8 || K % 8 || T < 1024 || T > 0x7fffffffLL) return 0;
+    if ((act_dtype != MTS_BF16 && act_dtype != MTS_F16) || N < 8 || K < 8 || N % 8 || K % 8 || T < 128 || T > 0x7fffffffLL) return 0;
     return (int64_t)N * K < (1LL << 30) && linear_split(T, N, K).tiles <= kLinearTiles;
 }
 extern "C" int64_t mts_linear_dw_workspace_bytes(int64_t T, int N, int K) {

@@ -105,6 +105,11 @@ SIGNATURES = {
     "mts_embedding_bwd_preferred": (_i, [_l, _l, _l]),
     "mts_embedding_bwd_workspace_bytes": (_l, [_l, _l, _l]),
     "mts_embedding_bwd": (_i, [_p, _p, _l, _i, _i, _i, _p, _p, _l, _p]),
+    "mts_linear_rows_supported": (_i, [_i, _l, _i, _i]),
+    "mts_linear_fwd_preferred": (_i, [_i, _l, _i, _i]),
+    "mts_linear_fwd": (_i, [_p, _p, _l, _i, _i, _i, _p, _p]),
+    "mts_linear_dx_preferred": (_i, [_i, _l, _i, _i]),
+    "mts_linear_dx": (_i, [_p, _p, _l, _i, _i, _i, _p, _p]),
     "mts_linear_dw_supported": (_i, [_i, _l, _i, _i]),
     "mts_linear_dw_workspace_bytes": (_l, [_l, _i, _i]),
     "mts_linear_dw": (_i, [_p, _p, _l, _i, _i, _i, _p, _p, _l, _p]),

@@ -73,9 +73,11 @@ class HipOpsBackend(DenseTorchOps):
 
     def linear(self, x, weight):
         """Extension: ``F.linear(x, weight)``, or None where the caller's own does as well."""
-        if not dense.is_linear_supported(x, weight):
-            return None
-        return dense.linear(x, weight)
+        if dense.is_linear_supported(x, weight):
+            return dense.linear(x, weight)
+        if dense.is_linear_alone_supported(x, weight):
+            return dense.linear_alone(x, weight)
+        return None
 
     def embedding(self, ids, weight, dtype):
         """Extension: ``F.embedding(ids, weight).to(dtype)`` whose gradient is this backend's, or None where the caller's own does as well."""

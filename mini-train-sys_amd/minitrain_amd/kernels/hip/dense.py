@@ -61,6 +61,15 @@ def linear(x, weight):
     return _lib.host().linear(x, weight)
 
 
+def is_linear_alone_supported(x, weight) -> bool:
+    return _may_replace(x, weight) and _lib.host().linear_alone_supported(x, weight)
+
+
+def linear_alone(x, weight):
+    """``F.linear(x, weight)`` under autocast, where no gradient is wanted"""
+    return _lib.host().linear_alone(x, weight)
+
+
 def is_embedding_supported(ids, weight, dtype) -> bool:
     return _may_replace(ids, weight) and _lib.host().embedding_supported(ids, weight, dtype)
 

@@ -259,3 +259,44 @@ def test_other_calls_stay_stock():
             assert not dense.is_linear_supported(x, w)
     with torch.autocast("cuda", dtype=torch.float16):
         assert not dense.is_linear_supported(x, w)
+
+
+@pytest.mark.parametrize("T,N,K", [(1, 64, 64), (2, 2304, 768), (127, 320, 256), (128, 128, 320), (129, 1000, 264), (1500, 2304, 768), (1792, 2304, 768), (8191, 768, 768),
+                                   (300, 16384, 128), (22100, 776, 512)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_products(T, N, K, dtype):
+    """The products alone: a row, tiles and one row more or less, a round of small tiles and its last, rounds of large ones, sums of whole k-tiles and others."""
+    from minitrain_amd import _lib
+
+    print(f"linear products T={T} N={N} K={K} {dtype}", flush=True)
+    lib, act, stream = _lib.load(), _lib.dtype_code(dtype), torch.cuda.current_stream().cuda_stream
+    g = torch.Generator().manual_seed(T + N)
+    x, w, grad = (torch.randn(*s, generator=g).to(dtype).cuda() for s in ((T, K), (N, K), (T, N)))
+    y, dx = torch.full((T, N), float("nan"), dtype=dtype, device="cuda"), torch.full((T, K), float("nan"), dtype=dtype, device="cuda")
+    _lib.check(lib.mts_linear_fwd(x.data_ptr(), w.data_ptr(), T, N, K, act, y.data_ptr(), stream), "mts_linear_fwd")
+    _lib.check(lib.mts_linear_dx(grad.data_ptr(), w.data_ptr(), T, N, K, act, dx.data_ptr(), stream), "mts_linear_dx")
+    for got, want in ((y, x.double() @ w.double().T), (dx, grad.double() @ w.double())):
+        assert float((got.double() - want).abs().max()) <= ULP[dtype] * float(want.abs().max())
+
+
+@pytest.mark.parametrize("T,N,K", [(16, 768, 768), (1000, 2304, 768), (300, 1000, 264)])
+def test_projection_without_gradients(T, N, K):
+    """Evaluation under autocast: the product that the stock operator gives, its cached rounding of the weight, and no graph."""
+    g = torch.Generator().manual_seed(T)
+    x, w = torch.randn(1, T, K, generator=g).bfloat16().cuda(), torch.randn(N, K, generator=g).cuda().requires_grad_(True)
+    ops = hip_backend()
+    for context in (torch.no_grad, torch.inference_mode):
+        with context(), torch.autocast("cuda", dtype=torch.bfloat16):
+            y, stock = ops.linear(x, w), torch.nn.functional.linear(x, w)
+            w_before = w.detach().clone()
+            if context is torch.no_grad:   # a weight changed inside the context: autocast goes on with its copy
+                w.mul_(2)
+                assert torch.equal(ops.linear(x, w), y) and torch.equal(torch.nn.functional.linear(x, w), stock)
+                w.copy_(w_before)
+        assert not y.requires_grad and y.shape == (1, T, N)
+        want = x.double() @ w.detach().bfloat16().double().T
+        assert float((y.double() - want).abs().max()) <= ULP[torch.bfloat16] * float(want.abs().max())
+    with torch.no_grad():
+        assert ops.linear(x, w) is None   # no autocast
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            assert ops.linear(x[..., 1:], w[:, 1:]) is None and ops.linear(x.transpose(1, 2), torch.zeros(8, T, device="cuda")) is None
