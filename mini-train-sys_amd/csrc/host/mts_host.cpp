@@ -1669,7 +1669,14 @@ PYBIND11_MODULE(_host, m) {
     });
     m.attr("ADAM_GROUPS") = MTS_ADAM_GROUPS;
     // not by way of Python's `grad`, whose object counts as a holder of the gradient from then on
-    m.def("has_gradient", [](const Tensor& p) { return p.grad().defined(); });
+    m.def("gradients_defined", [](const std::vector<Tensor>& params) {
+        std::vector<bool> defined;
+        for (const Tensor& p : params) defined.push_back(p.grad().defined());
+        return defined;
+    });
+    m.def("drop_gradients", [](const std::vector<Tensor>& params) {
+        for (const Tensor& p : params) p.mutable_grad().reset();
+    });
     m.def("adamw_supported", &adamw_supported);
     m.def("grad_norm", [](const std::vector<Tensor>& params, double max_norm, const Tensor& loss) {
         c10::OptionalDeviceGuard guard(params.at(0).device());

@@ -9,7 +9,8 @@ import contextlib
 import torch
 
 from minitrain_amd.kernels.hip.dense import loss_is_root
-from minitrain_amd.train.update import plan
+from minitrain_amd.train.modules import plain_modules, set_training
+from minitrain_amd.train.update import Update, plan
 
 
 def build_optimizer(model: torch.nn.Module, *, lr: float = 3e-4, weight_decay: float = 0.1, betas=(0.9, 0.95),
@@ -31,7 +32,7 @@ def train_step(model: torch.nn.Module, optimizer: torch.optim.Optimizer, batch: 
     computed on the device and read once per step; nothing on the device asserts or traps.
     ``check_finite=False`` skips the read (and its synchronisation) for callers that check at their own
     interval."""
-    model.train()
+    set_training(model, plain_modules(model))
     device = next(model.parameters()).device
     input_ids = batch["input_ids"].to(device, non_blocking=True)
     targets = batch["targets"].to(device, non_blocking=True)
@@ -55,7 +56,10 @@ def train_step(model: torch.nn.Module, optimizer: torch.optim.Optimizer, batch: 
         update.apply(norm, skip_if_not_finite=check_finite)
         if check_finite:
             copied.synchronize()
-        optimizer.zero_grad(set_to_none=True)
+        if isinstance(update, Update):
+            update.drop_gradients()
+        else:
+            optimizer.zero_grad(set_to_none=True)
         if check_finite and float(flag) != 0:
             raise FloatingPointError("non-finite training loss or global gradient norm")
         return loss.detach()

@@ -9,6 +9,7 @@ import torch
 from torch.optim import optimizer as _optimizer
 
 from minitrain_amd import _lib
+from minitrain_amd.train.modules import parameters_of, plain_modules
 
 
 # torch._compile: wraps zero_grad, for the compiler to leave it alone
@@ -61,8 +62,8 @@ class Update:
         numbers = (group["lr"], *group["betas"], group["eps"], group["weight_decay"])
         if any(isinstance(n, torch.Tensor) for n in numbers):
             return False
-        for p in group["params"]:
-            if not _lib.host().has_gradient(p):
+        for p, defined in zip(group["params"], _lib.host().gradients_defined(group["params"])):
+            if not defined:
                 continue
             state = self.optimizer.state.get(p)
             if not state:   # the first step makes it
@@ -86,6 +87,10 @@ class Update:
         if "step" in self.optimizer.__dict__:
             self.optimizer._opt_called = True
 
+    def drop_gradients(self) -> None:
+        """``optimizer.zero_grad(set_to_none=True)``: no other parameter of the optimizer has a gradient"""
+        _lib.host().drop_gradients(self.params)
+
 
 def plan(model: torch.nn.Module, optimizer: torch.optim.Optimizer, loss: torch.Tensor, grad_clip_norm: float | None) -> Update | None:
     """The update that the kernels can take in the place of clipping and ``optimizer.step()``, or None."""
@@ -97,7 +102,8 @@ def plan(model: torch.nn.Module, optimizer: torch.optim.Optimizer, loss: torch.T
     if len(optimizer.param_groups) > _lib.host().ADAM_GROUPS or not all(update.add_group(g) for g in optimizer.param_groups):
         return None
     # clipping looks at the model's gradients, the update at the optimizer's: the same ones
-    if {id(p) for p in model.parameters() if _lib.host().has_gradient(p)} != {id(p) for p in update.params}:
+    of_model = parameters_of(model, plain_modules(model))
+    if {id(p) for p, defined in zip(of_model, _lib.host().gradients_defined(of_model)) if defined} != {id(p) for p in update.params}:
         return None
     if not _lib.host().adamw_supported(update.params, update.exp_avgs, update.exp_avg_sqs, update.steps) or loss.device != update.params[0].device:
         return None

@@ -1,0 +1,51 @@
+"""The short walk through a model's modules, against the calls that it stands for (host code: no GPU)."""
+
+import pytest
+import torch
+from torch import nn
+
+from minitrain_amd.train.modules import parameters_of, plain_modules, set_training
+
+
+def _model():
+    shared = nn.Linear(3, 3)
+    return nn.Sequential(shared, nn.Sequential(nn.Dropout(0.1), shared, nn.ModuleList([nn.Linear(3, 2, bias=False)])), nn.Identity())
+
+
+def test_modules_and_parameters_are_those_of_the_model():
+    model = _model()
+    modules = plain_modules(model)
+    assert {id(m) for m in modules} == {id(m) for m in model.modules()} and len(modules) == len(list(model.modules()))
+    assert {id(p) for p in parameters_of(model, modules)} == {id(p) for p in model.parameters()}
+    assert [id(p) for p in parameters_of(model, None)] == [id(p) for p in model.parameters()]
+
+
+def test_modules_that_are_not_in_training_are_put_there():
+    model = _model()
+    model[1][0].eval()
+    set_training(model, plain_modules(model))
+    assert all(m.training for m in model.modules())
+
+
+@pytest.mark.parametrize("name", ["train", "named_parameters", "children"])
+@pytest.mark.parametrize("how", ["class", "instance"])
+def test_a_module_with_an_answer_of_its_own_is_asked(name, how):
+    calls = []
+
+    def answer(self, *args, **kwargs):
+        calls.append(name)
+        return getattr(nn.Linear, name)(self, *args, **kwargs)
+
+    model = _model()
+    if how == "class":
+        model[1].append(type("Own", (nn.Linear,), {name: answer})(3, 3))
+    else:
+        model[1].append(nn.Linear(3, 3))
+        model[1][-1].__dict__[name] = answer.__get__(model[1][-1])
+    assert plain_modules(model) is None
+    set_training(model, plain_modules(model))
+    if name == "train":
+        assert calls == ["train"]
+    assert {id(p) for p in parameters_of(model, plain_modules(model))} == {id(p) for p in model.parameters()}
+    model[1][-1].__dict__.pop(name, None)
+    assert torch.is_tensor(model[1][-1].weight)
