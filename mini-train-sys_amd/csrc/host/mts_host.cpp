@@ -516,6 +516,8 @@ ExpertGrads experts_backward(const Saved& s, Tensor dO, const Needs& need, const
     // When every gradient is wanted, dW1, dW2, dX and the dS reduction go out as ONE launch whose block order starts the long
     // weight-gradient tiles first; which XCD runs which of its units and dX tiles follows a table that the dO * W2 launch
     // writes on the side (uneven routing).
+    const bool joint_f32 = opt.on(JOINT_BWD) && need.x && need.w1 && need.w2 && need.s && dtype == at::kFloat && s.w1.scalar_type() == at::kFloat &&
+                           s.w2.scalar_type() == at::kFloat && mts_moe_bwd_joint_f32_supported(H, I) && aligned16(dO) && aligned16(s.x) && aligned16(w1_bwd);
     const bool joint = opt.on(JOINT_BWD) && need.x && need.w1 && need.w2 && need.s && layout && s.w1.scalar_type() == s.w2.scalar_type() &&
                        mts_moe_bwd_joint_supported(act, H, I);
     auto dw_workspace = [&](int which, bool wanted) {
@@ -576,6 +578,18 @@ ExpertGrads experts_backward(const Saved& s, Tensor dO, const Needs& need, const
                                 ptr_as<int32_t>(s.expert_start), ptr_as<int32_t>(s.s_reverse), ptr_as<float>(ds_part), T, K, E, H, I, act, grad,
                                 ptr(dx_expanded), ptr(g.dw1), ptr(g.dw2), ptr(g.ds), ptr(ws1), ws1_bytes, ptr(ws2), ws2_bytes, ptr_as<int32_t>(schedule), main),
               "mts_moe_bwd_joint");
+        combine_dx();
+        return g;
+    }
+
+    if (joint_f32) {
+        g.dw1 = at::empty_like(s.w1);
+        g.dw2 = at::empty_like(s.w2);
+        g.ds = at::empty({T, K}, s.weights.options());
+        check(mts_moe_bwd_joint_f32(ptr_as<float>(dO), ptr_as<float>(weighted_act), ptr_as<float>(d_pre_act), ptr_as<float>(s.x), ptr_as<float>(w1_bwd),
+                                    ptr_as<int32_t>(s.x_gather), ptr_as<int32_t>(s.expert_start), ptr_as<int32_t>(s.s_reverse), ptr_as<float>(ds_part), T, K, E, H, I,
+                                    ptr_as<float>(dx_expanded), ptr_as<float>(g.dw1), ptr_as<float>(g.dw2), ptr_as<float>(g.ds), main),
+              "mts_moe_bwd_joint_f32");
         combine_dx();
         return g;
     }

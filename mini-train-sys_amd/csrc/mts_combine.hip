@@ -3,6 +3,7 @@
 // (cast / transpose) of expert weights to bf16.
 #include "mts_common.h"
 #include "mts_combine_block.h"
+#include "mts_ds_block.h"
 
 namespace {
 
@@ -75,28 +76,9 @@ __global__ __launch_bounds__(kThreads) void combine_f32_kernel(
 
 // ---- routing-weight gradient ---------------------------------------------
 template <typename OutT>
-__global__ __launch_bounds__(kThreads) void ds_reduce_kernel(const float* __restrict__ part,
-                                                             const int32_t* __restrict__ s_rev,
-                                                             int64_t TK, int np,
+__global__ __launch_bounds__(kThreads) void ds_reduce_kernel(const float* __restrict__ part, const int32_t* __restrict__ s_rev, int64_t TK, int np,
                                                              OutT* __restrict__ d_w) {
-    for (int64_t n = (int64_t)blockIdx.x * kThreads + threadIdx.x; n < TK;
-         n += (int64_t)gridDim.x * kThreads) {
-        const int32_t r = s_rev[n];   // negative: dropped route, no gradient
-        float v = 0.f;
-        if (r >= 0) {
-            // one add after the other (a fixed order), but 16 loads in flight at a time
-            const float* p = part + (int64_t)r * np;
-            for (int j0 = 0; j0 < np; j0 += 16) {
-                float t[16];
-#pragma unroll
-                for (int j = 0; j < 16; ++j) t[j] = j0 + j < np ? p[j0 + j] : 0.f;
-#pragma unroll
-                for (int j = 0; j < 16; ++j)
-                    if (j0 + j < np) v += t[j];
-            }
-        }
-        d_w[n] = (OutT)v;
-    }
+    mts_ds::sum_block<OutT, kThreads>(part, s_rev, TK, np, d_w, blockIdx.x, gridDim.x);
 }
 
 // ---- weight staging --------------------------------------------------------

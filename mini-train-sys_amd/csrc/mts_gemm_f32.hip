@@ -17,6 +17,7 @@
 // 90 -> 60, dO*W2 95 -> 90, dX 167 -> 96, dW1 146 -> 87, dW2 76 -> 57; 8192 tokens: 588 -> 397, 282 -> 172, 298 -> 227, 498 -> 324, 512 -> 303, 266 -> 177.
 // Relative error against fp64 over all five results of the operator: 4.1e-7..1.02e-6 where the fp32 instruction had 4.3e-7..1.18e-6,
 // smaller for each at every size; by the length of the sum: mts_split3.h.
+#include "mts_ds_block.h"
 #include "mts_split3.h"
 
 #include <type_traits>
@@ -81,25 +82,40 @@ __device__ __forceinline__ int find_m_tile(const int32_t* __restrict__ expert_st
 
 // BN counts the columns of the B tile (SwiGLU: gate and up columns side by side, half the outputs)
 template <int BM, int BN, int EPI, bool BKM, bool VEC>
-__global__ __launch_bounds__(kThreads, 4) void rows_gemm_f32_kernel(Rows32 p) {
-    constexpr int WAVES_M = 2, WAVES_N = 2;
-    constexpr int MF = BM / WAVES_M / 32, NF = BN / WAVES_N / 32;
-    constexpr int OUT_N = EPI == E32_SWIGLU ? BN / 2 : BN, SLOT = 64, SLOTS = OUT_N / SLOT;
-    static_assert(OUT_N % SLOT == 0, "partial row sums cover 64 columns each");
+struct RowsTile {
+    static constexpr int WAVES_M = 2, WAVES_N = 2;
     typedef RowPlanes<BM, VEC> ATile;
     typedef typename std::conditional<BKM, KPlanes<BN, VEC>, RowPlanes<BN, VEC>>::type BTile;
-    __shared__ __attribute__((aligned(16))) bf16_t As[2 * ATile::SIZE];
-    __shared__ __attribute__((aligned(16))) bf16_t Bs[2 * BTile::SIZE];
-    __shared__ float ds_sum[EPI == E32_DY1 ? WAVES_N : 1][BM];
-    __shared__ float row_weight[EPI == E32_PLAIN ? 1 : BM];
-    __shared__ int special;
+    struct Lds {
+        __attribute__((aligned(16))) bf16_t As[2 * ATile::SIZE];
+        __attribute__((aligned(16))) bf16_t Bs[2 * BTile::SIZE];
+        float ds_sum[EPI == E32_DY1 ? WAVES_N : 1][BM];
+        float row_weight[EPI == E32_PLAIN ? 1 : BM];
+        int special;
+    };
+};
+
+// the work of block `block`
+template <int BM, int BN, int EPI, bool BKM, bool VEC>
+__device__ __forceinline__ void rows_block(const Rows32& p, int block, typename RowsTile<BM, BN, EPI, BKM, VEC>::Lds& lds) {
+    typedef RowsTile<BM, BN, EPI, BKM, VEC> Tile;
+    typedef typename Tile::ATile ATile;
+    typedef typename Tile::BTile BTile;
+    constexpr int WAVES_M = Tile::WAVES_M, WAVES_N = Tile::WAVES_N;
+    constexpr int MF = BM / WAVES_M / 32, NF = BN / WAVES_N / 32;
+    constexpr int OUT_N = EPI == E32_SWIGLU ? BN / 2 : BN, SLOT = 64, SLOTS = OUT_N / SLOT, HALF = NF > 1 ? NF / 2 : 1;
+    static_assert(OUT_N % SLOT == 0, "partial row sums cover 64 columns each");
+    bf16_t *As = lds.As, *Bs = lds.Bs;
+    auto& ds_sum = lds.ds_sum;
+    auto& row_weight = lds.row_weight;
+    int& special = lds.special;
 
     // block b runs on XCD b % 8: every XCD takes an equal contiguous run of the tiles, columns fastest, so that an expert's
     // weights stream through one L2 and the blocks that share activation rows are neighbours in time
     int e = 0, row0 = 0, rend = 0;
     const int total = find_m_tile<BM>(p.expert_start, p.E, -1, e, row0, rend) * p.n_tiles;
-    const int per_xcd = (total + kXcds - 1) / kXcds, slot = blockIdx.x / kXcds;
-    const int tile = (blockIdx.x % kXcds) * per_xcd + slot;
+    const int per_xcd = (total + kXcds - 1) / kXcds, slot = block / kXcds;
+    const int tile = (block % kXcds) * per_xcd + slot;
     if (slot >= per_xcd || tile >= total) return;
     find_m_tile<BM>(p.expert_start, p.E, tile / p.n_tiles, e, row0, rend);
     const int ny = tile % p.n_tiles, n0 = ny * OUT_N;
@@ -112,7 +128,7 @@ __global__ __launch_bounds__(kThreads, 4) void rows_gemm_f32_kernel(Rows32 p) {
     f32x16 acc[MF][NF] = {};
     const int wave = threadIdx.x / MTS_WAVE, wm = wave / WAVES_N, wn = wave % WAVES_N, lane = threadIdx.x % MTS_WAVE;
     auto a_at = [&](int mf) { return wm * (BM / WAVES_M) + mf * 32; };
-    auto b_at = [&](int nf) { return EPI == E32_SWIGLU ? nf / (NF / 2) * OUT_N + wn * (OUT_N / WAVES_N) + nf % (NF / 2) * 32 : wn * (BN / WAVES_N) + nf * 32; };
+    auto b_at = [&](int nf) { return EPI == E32_SWIGLU ? nf / HALF * OUT_N + wn * (OUT_N / WAVES_N) + nf % HALF * 32 : wn * (BN / WAVES_N) + nf * 32; };
     if (threadIdx.x >= kLoaders) {
         ATile a;
 #pragma unroll
@@ -224,6 +240,12 @@ __global__ __launch_bounds__(kThreads, 4) void rows_gemm_f32_kernel(Rows32 p) {
     }
 }
 
+template <int BM, int BN, int EPI, bool BKM, bool VEC>
+__global__ __launch_bounds__(kThreads, 4) void rows_gemm_f32_kernel(Rows32 p) {
+    __shared__ typename RowsTile<BM, BN, EPI, BKM, VEC>::Lds lds;
+    rows_block<BM, BN, EPI, BKM, VEC>(p, blockIdx.x, lds);
+}
+
 struct Dw32 {
     const float* P;
     const int32_t* p_gather;
@@ -236,21 +258,45 @@ struct Dw32 {
     int m_tiles, n_tiles;
 };
 
-// BM x BN outputs; the reduction runs over the expert's rows, both operands k-major
-template <int BM, int BN, typename OutT, bool VEC>
-__global__ __launch_bounds__(kThreads, 4) void dw_gemm_f32_kernel(Dw32 p) {
-    constexpr int MF = BM / 64, NF = BN / 64;
+// The expert with the `n`-th most rows: the longest sums start first.  More experts than a wave has lanes: as they come.
+__device__ __forceinline__ int longest_expert(const int32_t* __restrict__ expert_start, int E, int n) {
+    if (E > MTS_WAVE) return n;
+    const int lane = threadIdx.x % MTS_WAVE;
+    const int rows = lane < E ? expert_start[lane + 1] - expert_start[lane] : -1;
+    int before = 0;
+    for (int f = 0; f < E; ++f) {
+        const int other = __builtin_amdgcn_readlane(rows, f);
+        before += other > rows || (other == rows && f < lane) ? 1 : 0;
+    }
+    return __ffsll((unsigned long long)__ballot(lane < E && before == n)) - 1;
+}
+
+template <int BM, int BN, bool VEC>
+struct DwTile {
     typedef KPlanes<BM, VEC> PT;
     typedef KPlanes<BN, VEC> QT;
-    __shared__ __attribute__((aligned(16))) bf16_t Ps[2 * PT::SIZE];
-    __shared__ __attribute__((aligned(16))) bf16_t Qs[2 * QT::SIZE];
-    __shared__ int special;
+    struct Lds {
+        __attribute__((aligned(16))) bf16_t Ps[2 * PT::SIZE];
+        __attribute__((aligned(16))) bf16_t Qs[2 * QT::SIZE];
+        int special;
+    };
+};
+
+// BM x BN outputs; the reduction runs over the expert's rows, both operands k-major
+template <int BM, int BN, typename OutT, bool VEC>
+__device__ __forceinline__ void dw_block(const Dw32& p, int block, typename DwTile<BM, BN, VEC>::Lds& lds) {
+    constexpr int MF = BM / 64, NF = BN / 64;
+    typedef typename DwTile<BM, BN, VEC>::PT PT;
+    typedef typename DwTile<BM, BN, VEC>::QT QT;
+    bf16_t *Ps = lds.Ps, *Qs = lds.Qs;
+    int& special = lds.special;
     // an XCD takes an equal contiguous run of every expert's tiles, columns fastest: an equal share of the work however
     // uneven the experts are, and about an eighth of P through its L2
     const int per_expert = p.m_tiles * p.n_tiles, per_xcd = (per_expert + kXcds - 1) / kXcds;
-    const int slot = blockIdx.x / kXcds, e = slot / per_xcd;
-    const int tile = (blockIdx.x % kXcds) * per_xcd + slot % per_xcd;
-    if (tile >= per_expert || e >= p.E) return;
+    const int slot = block / kXcds;
+    const int tile = (block % kXcds) * per_xcd + slot % per_xcd;
+    if (tile >= per_expert || slot / per_xcd >= p.E) return;
+    const int e = longest_expert(p.expert_start, p.E, slot / per_xcd);
     const int m0 = tile / p.n_tiles * BM, n0 = tile % p.n_tiles * BN;
     const int rbeg = p.expert_start[e], rend = p.expert_start[e + 1];
 
@@ -307,6 +353,61 @@ __global__ __launch_bounds__(kThreads, 4) void dw_gemm_f32_kernel(Dw32 p) {
         }
 }
 
+template <int BM, int BN, typename OutT, bool VEC>
+__global__ __launch_bounds__(kThreads, 4) void dw_gemm_f32_kernel(Dw32 p) {
+    __shared__ typename DwTile<BM, BN, VEC>::Lds lds;
+    dw_block<BM, BN, OutT, VEC>(p, blockIdx.x, lds);
+}
+
+// the experts with more than `rows` rows; more experts than a wave has lanes: all of them where one has
+__device__ __forceinline__ int longer_experts(const int32_t* __restrict__ expert_start, int E, int rows) {
+    int longer = 0;
+    for (int e0 = 0; e0 < E; e0 += MTS_WAVE) {
+        const int e = e0 + threadIdx.x % MTS_WAVE;
+        longer += (int)__popcll(__ballot(e < E && expert_start[min(e, E - 1) + 1] - expert_start[min(e, E - 1)] > rows));
+    }
+    return E > MTS_WAVE && longer ? E : longer;
+}
+
+// dX, dW1, dW2 and the routing weights' gradient in one launch: blocks of one part take the CUs as those in front leave them, and nothing is forked onto
+// other streams and joined again (four events, for which the host takes 20 us and the stream some 5 each).  In front of dX, whose sums have 2I terms, come the
+// weight gradients of experts with more than two thirds as many rows, the longest first; behind it those of the others.  Whole operators, us, as launches
+// side by side and so: 64 tokens of 256/256 210 / 125; 256 of 768/1024 202 / 171; 2048 477 / 456, a few experts popular 476 / 470; 4096 of 1024/1024 1066 /
+// 1045 and 1052 / 1048; 8192 of 768/1024 1493 / 1465 and 1490 / 1488.  With all of dX in front 4096 tokens and popular experts took 1060 for 1019, with all of
+// it behind 2048 even ones 478 for 442; with both weight gradients of an expert side by side 2048 tokens of 16 popular experts 530 for 498.
+struct Bwd32 {
+    Rows32 dx;
+    Dw32 dw1, dw2;
+    int n_dx, n_dw1, n_dw2, per_dw1, per_dw2;   // blocks, multiples of the XCDs; blocks an expert and XCD
+    const float* ds_part;
+    const int32_t* s_reverse;
+    int64_t entries;
+    int np, n_ds;
+    float* d_weights;
+};
+template <int DX, int DW>
+__global__ __launch_bounds__(kThreads, 4) void bwd_joint_f32_kernel(Bwd32 q) {
+    __shared__ union {
+        typename RowsTile<DX, DX, E32_PLAIN, true, true>::Lds dx;
+        typename DwTile<DW, DW, true>::Lds dw;
+    } lds;
+    const int front = longer_experts(q.dx.expert_start, q.dx.E, 2 * q.dx.Kdim / 3) * kXcds, front1 = front * q.per_dw1, front2 = front * q.per_dw2;
+    int b = blockIdx.x;
+    if (b < front1) return dw_block<DW, DW, float, true>(q.dw1, b, lds.dw);
+    b -= front1;
+    if (b < front2) return dw_block<DW, DW, float, true>(q.dw2, b, lds.dw);
+    b -= front2;
+    if (b < q.n_dx) return rows_block<DX, DX, E32_PLAIN, true, true>(q.dx, b, lds.dx);
+    b -= q.n_dx;
+    if (b < q.n_dw1 - front1) return dw_block<DW, DW, float, true>(q.dw1, front1 + b, lds.dw);
+    b -= q.n_dw1 - front1;
+    if (b < q.n_dw2 - front2) return dw_block<DW, DW, float, true>(q.dw2, front2 + b, lds.dw);
+    b -= q.n_dw2 - front2;
+    mts_ds::sum_block<float, kThreads>(q.ds_part, q.s_reverse, q.entries, q.np, q.d_weights, b, q.n_ds);
+}
+
+int64_t dw_blocks(const Dw32& p) { return ((int64_t)p.m_tiles * p.n_tiles + kXcds - 1) / kXcds * kXcds * p.E; }
+
 int64_t m_tiles32(int64_t rows, int E, int bm) {
     const int64_t a = (rows + bm - 1) / bm + E - 1;
     return a < rows ? a : rows;
@@ -353,7 +454,7 @@ int mts_f32_dw(const float* P, const int32_t* p_gather, const float* Q, const in
     const int bt = large ? 128 : 64;
     Dw32 p = {P, p_gather, Q, q_gather, M, N, expert_start, E, C, (M + bt - 1) / bt, (N + bt - 1) / bt};
     const bool vec = M % 4 == 0 && N % 4 == 0 && mts_aligned16(P) && mts_aligned16(Q);
-    const int64_t blocks = ((int64_t)p.m_tiles * p.n_tiles + kXcds - 1) / kXcds * kXcds * E;
+    const int64_t blocks = dw_blocks(p);
     if (blocks >= (1LL << 31)) return MTS_ERR_SHAPE;
     const dim3 grid((unsigned)blocks);
     auto launch = [&](auto* kind) {
@@ -367,6 +468,39 @@ int mts_f32_dw(const float* P, const int32_t* p_gather, const float* Q, const in
     else if (grad_dtype == MTS_BF16) launch((bf16_t*)nullptr);
     else if (grad_dtype == MTS_F16) launch((mts_f16_t*)nullptr);
     else return MTS_ERR_DTYPE;
+    MTS_CHECK_LAUNCH();
+    return MTS_OK;
+}
+
+extern "C" int mts_moe_bwd_joint_f32_supported(int H, int I) { return H >= 4 && I >= 4 && H % 4 == 0 && I % 4 == 0; }
+
+extern "C" int mts_moe_bwd_joint_f32(const float* d_out, const float* weighted_act, const float* d_pre_act, const float* x, const float* w1, const int32_t* x_gather,
+                                     const int32_t* expert_start, const int32_t* s_reverse, const float* ds_partial, int64_t T, int K, int E, int H, int I,
+                                     float* dx_expanded, float* d_w1, float* d_w2, float* d_weights, void* stream) {
+    if (!d_out || !weighted_act || !d_pre_act || !x || !w1 || !x_gather || !expert_start || !s_reverse || !ds_partial || !dx_expanded || !d_w1 || !d_w2 || !d_weights)
+        return MTS_ERR_NULL;
+    if (T <= 0 || K < 1 || T * K > 0x7fffffffLL || E < 1 || E > MTS_MAX_MOE_EXPERTS || !mts_moe_bwd_joint_f32_supported(H, I)) return MTS_ERR_SHAPE;
+    if (!mts_aligned16(d_out) || !mts_aligned16(weighted_act) || !mts_aligned16(d_pre_act) || !mts_aligned16(x) || !mts_aligned16(w1)) return MTS_ERR_ALIGN;
+    const int64_t TK = T * K;
+    const bool large_dx = large_tiles(TK, H, E), large_dw = large_tiles((int64_t)E * 2 * I, H, 0);   // dW2's tiles follow dW1's
+    const int bx = large_dx ? 128 : 64, bw = large_dw ? 128 : 64;
+    Bwd32 q = {};
+    q.dx = {d_pre_act, 2 * I, nullptr, w1, H, H, 2 * I, expert_start, E, dx_expanded, nullptr, nullptr, nullptr, nullptr, nullptr, 0, (H + bx - 1) / bx};
+    q.dw1 = {d_pre_act, nullptr, x, x_gather, 2 * I, H, expert_start, E, d_w1, (2 * I + bw - 1) / bw, (H + bw - 1) / bw};
+    q.dw2 = {d_out, x_gather, weighted_act, nullptr, H, I, expert_start, E, d_w2, (H + bw - 1) / bw, (I + bw - 1) / bw};
+    const int64_t n_dx = (m_tiles32(TK, E, bx) * q.dx.n_tiles + kXcds - 1) / kXcds * kXcds, n_dw1 = dw_blocks(q.dw1), n_dw2 = dw_blocks(q.dw2);
+    const int64_t want = (TK + kThreads - 1) / kThreads;
+    q.n_ds = (int)(want < 64 ? want : 64);
+    const int64_t blocks = n_dx + n_dw1 + n_dw2 + q.n_ds;
+    if (blocks >= (1LL << 31)) return MTS_ERR_SHAPE;
+    q.n_dx = (int)n_dx, q.n_dw1 = (int)n_dw1, q.n_dw2 = (int)n_dw2, q.per_dw1 = (int)(n_dw1 / E / kXcds), q.per_dw2 = (int)(n_dw2 / E / kXcds);
+    q.ds_part = ds_partial, q.s_reverse = s_reverse, q.entries = TK, q.np = mts_moe_ds_partials(I), q.d_weights = d_weights;
+    const dim3 grid((unsigned)blocks);
+    hipStream_t s = (hipStream_t)stream;
+    if (large_dx && large_dw) bwd_joint_f32_kernel<128, 128><<<grid, kThreads, 0, s>>>(q);
+    else if (large_dx) bwd_joint_f32_kernel<128, 64><<<grid, kThreads, 0, s>>>(q);
+    else if (large_dw) bwd_joint_f32_kernel<64, 128><<<grid, kThreads, 0, s>>>(q);
+    else bwd_joint_f32_kernel<64, 64><<<grid, kThreads, 0, s>>>(q);
     MTS_CHECK_LAUNCH();
     return MTS_OK;
 }

@@ -87,6 +87,8 @@ SIGNATURES = {
     "mts_moe_bwd_dw_workspace_bytes": (_l, [_i, _i, _i, _i]),
     "mts_moe_bwd_dw2": (_i, [_p, _p, _p, _p, _l, _i, _i, _i, _i, _i, _i, _p, _p, _l, _p]),
     "mts_moe_bwd_dw1": (_i, [_p, _p, _p, _p, _l, _i, _i, _i, _i, _i, _i, _p, _p, _l, _p]),
+    "mts_moe_bwd_joint_f32_supported": (_i, [_i, _i]),
+    "mts_moe_bwd_joint_f32": (_i, [_p] * 9 + [_l, _i, _i, _i, _i] + [_p] * 5),
     "mts_moe_bwd_joint_supported": (_i, [_i, _i, _i]),
     "mts_moe_bwd_joint": (_i, [_p, _p, _p, _p, _p, _p, _p, _p, _p, _l, _i, _i, _i, _i, _i, _i, _p, _p, _p, _p, _p, _l, _p, _l, _p, _p]),
     "mts_moe_bwd_joint_router_supported": (_i, [_i, _l, _i, _i, _i]),

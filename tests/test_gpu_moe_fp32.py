@@ -135,3 +135,24 @@ def test_products_at_the_ends_of_the_range(R, H, I):
     d_out[3:7, 1], act[3:7, 2] = 0.999 * 2.0 ** 64, 0.999 * 2.0 ** 62
     dw = _dw2(d_out.cuda(), act.cuda(), starts)[0]
     assert_close_scaled(dw.double(), d_out.double().t() @ act.double(), 1e-5, "weight gradient")
+
+
+@pytest.mark.parametrize("T,H,E,I,K,popular", [
+    (1, 4, 1, 4, 1, 0.0), (33, 64, 2, 64, 1, 0.0), (257, 64, 4, 132, 2, 3.0), (129, 36, 70, 24, 2, 0.0), (512, 132, 8, 200, 2, 6.0),
+    (1500, 520, 3, 1032, 2, 0.0), (2000, 256, 5, 64, 2, 2.0), (40, 260, 64, 516, 3, 0.0)])
+def test_gradients_of_one_launch_are_those_of_separate_ones(T, H, E, I, K, popular, monkeypatch):
+    """Both tile sizes for either part, experts without rows and with most of them, dX in front of all, some and none of the weight gradients, more experts
+    than a wave has lanes, dropped routes: the same sums in the same order."""
+    from minitrain_amd.kernels.hip.switches import SWITCHES
+
+    print(f"fp32 gradients in one launch T={T} H={H} E={E} I={I} K={K} popular={popular}", flush=True)
+    case = routed_case(50 + T, T, H, E, I, K, dtype=torch.float32, bias=popular * torch.linspace(-1, 1, E))
+    idx = case["idx"].clone()
+    if T > 1:
+        idx[T // 2, 0] = -1
+    one = hip_moe_grads(case["x"], case["w1"], case["w2"], idx, case["w"], case["g"])
+    monkeypatch.setattr(SWITCHES, "joint_bwd", False)
+    several = hip_moe_grads(case["x"], case["w1"], case["w2"], idx, case["w"], case["g"])
+    assert torch.equal(one[0], several[0])
+    for name, a, b in zip(("dx", "dW1", "dW2", "dS"), one[1], several[1]):
+        assert a.isfinite().all() and torch.equal(a, b), name
