@@ -2753,6 +2753,21 @@ bool small_tiles_pay(int kind, int64_t TK, int E, int N) {
 // does launch_rows_any take B in the weights' stored layout for this kind and reduction length?
 bool rows_kmajor_ok(int kind, int Kdim) { return tile_choice(kind) >= 1 && rows_pipelined(Kdim); }
 
+// m-tiles of the XCD that has most: routes spread evenly over the experts, or half a tile more than whole ones for each
+int64_t m_tiles_of_xcd(int64_t TK, int E, int bm, bool even) {
+    const int64_t experts = TK < E ? TK : E;
+    const int64_t tiles2 = even ? 2 * experts * (((TK + experts - 1) / experts + bm - 1) / bm) : 2 * ((TK + bm - 1) / bm) + experts;   // twice as many
+    return (tiles2 + 2 * kXcds - 1) / (2 * kXcds);
+}
+// whether dO*W2 on large tiles (`wide` columns of them) is ahead of three narrow blocks a CU that fit their round
+bool large_tiles_ahead(int64_t TK, int E, int64_t narrow, int64_t wide) {
+    for (const bool even : {true, false}) {
+        const int64_t a_cu = (m_tiles_of_xcd(TK, E, RingThreePerCu::BM, even) * narrow + kCusPerXcd - 1) / kCusPerXcd, large = m_tiles_of_xcd(TK, E, WsWide::BM, even) * wide;
+        if (a_cu < 2 || 2 * large > (a_cu == 2 ? kCusPerXcd : 2 * kCusPerXcd)) return false;
+    }
+    return true;
+}
+
 // b_kmajor: B is [E][Kdim][N] (the weights as stored) instead of the transposed copy [E][N][Kdim];
 // only the ring and specialised kernels read it that way
 template <int EPI>
@@ -2771,10 +2786,14 @@ int launch_rows_any(int kind, RowsParams p, int64_t TK, hipStream_t s, bool b_km
     // 1000/1368 5898 71 / 74, 72 / 75, 91 / 78, 6904 95 / 82, 94 / 82, 94 / 82.  Widths whose last 256 columns are half empty stay where that adds more than an
     // eighth to the columns (128 columns of 768 above the border 1.01 to 1.18 times as long, 384 0.97 to 1.13, 640 of 256 to 1024 0.91 to 1.07, 896
     // 0.90 to 1.11; 1152 0.87 to 1.01).  Of 300 calls above the border some of 2432 columns are 3 to 7 % slower, some of 256 of k 3 %, the others at most 2 %.
+    // Within that round a CU holds one, two or three of the narrow blocks (768/1024: 23, 29 and 41 us), and where the large tiles are a round of one block a CU
+    // they are ahead of three (35), and of two where they are half a round and cut (24).  Asked for routes spread evenly and for half a tile more an expert, and
+    // changed where both say so.  Of 360 calls, even, random and with popular experts, 108 changed: 2946 tokens of 768/1024 29.1 / 24.2, 6544 of 776/1024 46.4 /
+    // 39.3, 4195 of 1000/1368 53.0 / 44.1, 8261 of 768/768 43.1 / 37.6, 5122 of 1000/680 with 16 experts, top-3, 55.7 / 40.1; none more than the noise slower.
     if (choice == 3 && !tile_forced(kind)) {
         const int64_t narrow = (p.N + RingThreePerCu::BN - 1) / RingThreePerCu::BN, wide = (p.N + WsWide::BN - 1) / WsWide::BN * (WsWide::BN / RingThreePerCu::BN);
         const int64_t blocks = (TK + RingThreePerCu::BM - 1) / RingThreePerCu::BM * narrow;
-        if (p.Kdim > 1024 || (blocks > 3 * kXcds * kCusPerXcd && 8 * wide <= 9 * narrow)) choice = 4;
+        if (p.Kdim > 1024 || (8 * wide <= 9 * narrow && (blocks > 3 * kXcds * kCusPerXcd || large_tiles_ahead(TK, p.E, narrow, wide / 2)))) choice = 4;
     }
     // the 64-wide variant exists for the GEMMs with a plain or SwiGLU epilogue
     if (choice == 4 && epi_is_dy1(EPI) && (EPI != EPI_DY1N || !b_kmajor)) choice = 2;

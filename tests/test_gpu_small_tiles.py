@@ -7,6 +7,7 @@ import pytest
 import torch
 
 from minitrain_amd.kernels.hip.fused_moe import fused_moe
+from tests.helpers import BF16_TOL, assert_close_scaled, hip_moe_grads, oracle_moe_grads, routed_case
 
 pytestmark = pytest.mark.gpu
 
@@ -43,3 +44,15 @@ def test_small_tiles(rows, E, H, I, dtype, params):
     for what, got, ref in [("out", out.detach(), want.detach())] + [(n, a.grad, b.grad) for n, a, b in zip(("dx", "dw1", "dw2", "ds"), leaves, wide)]:
         err, scale = float((got.double() - ref).abs().max()), float(ref.abs().max())
         assert err <= TOL[dtype] * scale, (what, err, scale)
+
+
+@pytest.mark.parametrize("T,H,E,I,K", [(2946, 128, 8, 1024, 2), (3400, 72, 16, 1000, 1), (6544, 128, 8, 768, 2), (5122, 64, 16, 680, 3), (5200, 64, 8, 1024, 2)])
+def test_gradient_on_large_tiles_within_the_round_of_narrow_ones(T, H, E, I, K):
+    """dO*W2 where a CU would hold two or three narrow blocks and the large tiles are half a round, cut in two, or a whole one; and one call that
+    stays: the gradients that pass through it."""
+    print(f"dO*W2 on large tiles T={T} H={H} E={E} I={I} K={K}", flush=True)
+    case = routed_case(31 + T, T, H, E, I, K, bias=torch.linspace(-0.5, 0.5, E))
+    _, grads = hip_moe_grads(case["x"], case["w1"], case["w2"], case["idx"], case["w"], case["g"])
+    _, ref = oracle_moe_grads(case["x"], case["w1"], case["w2"], case["idx"], case["w"], case["g"], device="cuda")
+    for name, a, b in zip(("dx", "dW1", "dW2", "dS"), grads, ref):
+        assert_close_scaled(a, b, BF16_TOL, name)
