@@ -2437,7 +2437,8 @@ typedef DwWsWide JointDwTile;                             // the weight-gradient
 // hardware queues interleave them, and the long weight-gradient tiles (one tile reduces
 // over all rows of an expert) tend to start last and finish last.  Here the block index
 // fixes the order: the dW1 tiles first, then dW2, then the dX tiles, which are a third as
-// long and fill the CUs as they come free, then a few blocks that add up dS.
+// long at 24 576 tokens and fill the CUs as they come free, then a few blocks that add up dS;
+// with few rows an expert the dX tiles are the long ones and go in front (dx_in_front).
 // Every part starts at a multiple of the XCD count, so block % 8 is still the part's own
 // XCD index.
 // ---------------------------------------------------------------------------
@@ -2446,6 +2447,7 @@ struct BwdJointParams {
     DwParams dw1, dw2;
     RowsParams dx;
     int n_dw1, n_dw2, n_dx;        // blocks per part, in launch order
+    int dx_first;                  // dX's blocks in front of the weight gradients' (dx_in_front)
     const float* ds_part;          // [entries rows][np]
     const int32_t* s_reverse;      // entry -> row, negative for a dropped route
     bf16_t* d_weights;             // [entries]
@@ -2477,22 +2479,27 @@ __global__ __launch_bounds__(WsLarge::NT, WsLarge::WAVES_PER_EU) void bwd_joint_
     constexpr int LDS_ELEMS = ROWS_LDS > JointDwTile::LDS_ELEMS ? ROWS_LDS : JointDwTile::LDS_ELEMS;
     static_assert(LDS_ELEMS * 2 <= 160 * 1024, "LDS capacity");
     __shared__ __attribute__((aligned(1024))) bf16_t smem[LDS_ELEMS];
-    int b = blockIdx.x;
-    if (b < q.n_dw1) {
+    int b = blockIdx.x, x = b - q.n_dw1 - q.n_dw2;   // x: the block of dX
+    const bool lead = !std::is_same<DxTile, WsSmall>::value && q.dx_first;
+    if (lead) {
+        x = b;
+        b -= q.n_dx;
+    }
+    if (b >= 0 && b < q.n_dw1) {
         dw_gemm_ws_block<JointDwTile, OutT>(q.dw1, smem, b);
         return;
     }
     b -= q.n_dw1;
-    if (b < q.n_dw2) {
+    if (b >= 0 && b < q.n_dw2) {
         dw_gemm_ws_block<JointDwTile, OutT>(q.dw2, smem, b);
         return;
     }
     b -= q.n_dw2;
-    if (b < q.n_dx) {
-        rows_gemm_ws_block<DxTile, EPI_PLAIN, true, DxHalf>(q.dx, smem, b);   // W1 as stored: [E][2I][H]
+    if (x < q.n_dx) {
+        rows_gemm_ws_block<DxTile, EPI_PLAIN, true, DxHalf>(q.dx, smem, x);   // W1 as stored: [E][2I][H]
         return;
     }
-    b -= q.n_dx;
+    if (!lead) b -= q.n_dx;
     if (b < q.n_ds) {
         for (int64_t n = (int64_t)b * WsLarge::NT + threadIdx.x; n < q.entries; n += (int64_t)q.n_ds * WsLarge::NT) {
             const int32_t r = q.s_reverse[n];
@@ -2741,13 +2748,31 @@ bool rows_pipelined(int Kdim) { return Kdim % 64 == 0 || Kdim >= 256; }
 //   gate/up  512 tokens 19.4 / 14.8 (192), 1024 tokens 21.9 / 23.5 (320);   down  2048 tokens 17.6 / 13.2 (216), 4096 tokens 20.5 / 23.1 (408);
 //   dO*W2 (192 x 128 ring blocks there)  1024 tokens 25.6 / 16.0 (160), 2048 tokens 27.2 / 28.1 (288);
 //   joint backward launch  192 tokens 49 / 27, 512 tokens 58 / 37, 1024 tokens 65 / 52 (120), 2048 tokens 62 / 68 (216): dX shares the CUs
-//   with the weight gradients (in front of them instead of behind: 512 tokens 44).
+//   with the weight gradients (in front of them instead of behind: 512 tokens 44).  Where the large ones go in front (dx_in_front) the small ones
+//   are ahead up to 192 of them if the reduction is long (large in front / small behind: 1600 tokens 44.5 / 37.8, 1000 of 1024/1536 with 16
+//   experts 90 / 78, 2100 47 / 56), and no further than 160 if not (1000 of 768/512 with 24 experts 28 / 31).
 // The count is that of routes spread evenly: half a tile more per expert than whole ones.
-bool small_tiles_pay(int kind, int64_t TK, int E, int N) {
+bool small_tiles_pay(int kind, int64_t TK, int E, int N, bool long_dx = false) {
     const int per_block = kind == K_GATEUP ? WsSmall::BN / 2 : WsSmall::BN;
     const int64_t present = TK < E ? TK : E, spread = TK / WsSmall::BM + E / 2;
     const int64_t tiles = (spread > present ? spread : present) * ((N + per_block - 1) / per_block);
-    return tiles <= (kind == K_DX ? 160 : 256);
+    return tiles <= (kind != K_DX ? 256 : long_dx ? 192 : 160);
+}
+
+// whether one of dX's tiles takes long beside one of the weight gradients': it reduces over 2I, that one over an expert's rows
+bool long_tiles(const RowsParams& dx, int E) { return dx.Kdim >= 1536 && dx.Kdim / 2 >= dx.TK / E; }
+
+// Whether the large dX tiles of the joint backward launch go in front of the weight gradients'.  They are the longer ones there while an expert's rows
+// are fewer than I, and where they are two thirds of a round they start at once, on CUs of their own, while the short ones come one after the
+// other on the rest; behind them they start when the first round of the weight gradients ends.  More of them leave too few CUs to those, and longer
+// weight-gradient tiles are the ones to begin with.  The launch behind / in front, us, random routing and (popular experts): 768/1024 1700 tokens 61 / 49
+// (76 / 61), 2900 65 / 50 (77 / 63), 4358 77 / 74, 4681 79 / 82, 24 576 344 / 395; 1024/1536, 16 experts 1800 125 / 101 (207 / 171), 4178
+// 168 / 167 (294 / 257), 5439 183 / 196; 1000/1368 2100 98 / 78 (122 / 96), 4096 125 / 128 (181 / 154); 768/512, 24 experts 1778 44 / 32 (69 / 58), 4512
+// 55 / 46, 10 821 87 / 88; 2048/512 2100 64 / 56 (81 / 69).
+bool dx_in_front(const RowsParams& dx, int E) {
+    const int64_t present = dx.TK < E ? dx.TK : E, spread = dx.TK / WsWide::BM + E / 2;
+    const int64_t tiles = (spread > present ? spread : present) * ((dx.N + WsWide::BN - 1) / WsWide::BN);
+    return dx.Kdim / 2 >= dx.TK / E && 3 * tiles <= 2 * kXcds * kCusPerXcd;
 }
 
 // does launch_rows_any take B in the weights' stored layout for this kind and reduction length?
@@ -3046,7 +3071,8 @@ int launch_bwd_joint(BwdJointParams q, int E, int grad_dtype, void* ws1, int64_t
         q.dw2.part = nullptr;
     }
     q.dx.reverse = (tile_order_mask() & ORDER_DX) ? 1 : 0;
-    const bool small_dx = tile_forced(K_DX) ? tile_choice(K_DX) == 5 : small_tiles_pay(K_DX, q.dx.TK, E, q.dx.N);
+    const bool small_dx = tile_forced(K_DX) ? tile_choice(K_DX) == 5 : small_tiles_pay(K_DX, q.dx.TK, E, q.dx.N, long_tiles(q.dx, E));
+    q.dx_first = !small_dx && dx_in_front(q.dx, E);
     q.n_dx = (int)(small_dx ? rows_grid<WsSmall, EPI_PLAIN>(q.dx, q.dx.TK) : rows_grid<JointDxTile, EPI_PLAIN>(q.dx, q.dx.TK)).x;
     // With both workspaces (row chunks on) and a schedule from the caller (written by the dO*W2 launch), units and dX
     // tiles go to the XCDs as the table says.

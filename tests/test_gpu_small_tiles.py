@@ -56,3 +56,19 @@ def test_gradient_on_large_tiles_within_the_round_of_narrow_ones(T, H, E, I, K):
     _, ref = oracle_moe_grads(case["x"], case["w1"], case["w2"], case["idx"], case["w"], case["g"], device="cuda")
     for name, a, b in zip(("dx", "dW1", "dW2", "dS"), grads, ref):
         assert_close_scaled(a, b, BF16_TOL, name)
+
+
+@pytest.mark.parametrize("T,H,E,I,K", [(1600, 768, 8, 1024, 2), (1810, 776, 8, 1024, 2), (5400, 256, 8, 1400, 2), (5700, 256, 8, 1400, 2), (700, 512, 24, 520, 3)])
+@pytest.mark.parametrize("fp32_weights", [False, True])
+def test_dx_in_front_of_the_weight_gradients(T, H, E, I, K, fp32_weights):
+    """The joint backward launch with its dX tiles in front: on both sides of the line to small tiles behind, on both sides of I rows an expert, and
+    with ragged widths; an expert without routes, popular ones."""
+    print(f"dX in front T={T} H={H} E={E} I={I} K={K} fp32_weights={fp32_weights}", flush=True)
+    bias = torch.linspace(-1.0, 1.0, E)
+    bias[1] = -100.0
+    case = routed_case(37 + T, T, H, E, I, K, bias=bias)
+    w1, w2 = ((case[n].float() if fp32_weights else case[n]) for n in ("w1", "w2"))
+    _, grads = hip_moe_grads(case["x"], w1, w2, case["idx"], case["w"], case["g"])
+    _, ref = oracle_moe_grads(case["x"], case["w1"], case["w2"], case["idx"], case["w"], case["g"], device="cuda")
+    for name, a, b in zip(("dx", "dW1", "dW2", "dS"), grads, ref):
+        assert_close_scaled(a, b, BF16_TOL, name)
