@@ -296,8 +296,8 @@ struct Two {   // as one access
 };
 
 // 32 columns of one expert's down projection; the block that arrives last at a range of columns, counted over the experts with rows, adds the tokens'
-// routes.  Rows and counter pass between the XCDs' L2s: both are written and read by agent-scope accesses, and the barrier in front of the counter waits
-// for the block's rows to be written.
+// routes.  Rows and counter pass between the XCDs' L2s: both are written and read by agent-scope accesses, and every wave waits for its rows to be
+// acknowledged before the barrier in front of the counter (which by itself waits for LDS alone).
 template <typename ET, typename WT, int MT>
 __global__ __launch_bounds__(kThreads) void few_tokens_down_kernel(FewTokens p) {
     constexpr int STEP_REGS = 8 * (2 * (int)(sizeof(WT) / sizeof(ET)) + MT);
@@ -368,6 +368,7 @@ __global__ __launch_bounds__(kThreads) void few_tokens_down_kernel(FewTokens p) 
             }
         }
     }
+    __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
     __syncthreads();
     if (threadIdx.x == 0) arrived = __hip_atomic_fetch_add(p.arrived + nt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
