@@ -7,11 +7,19 @@
 // so what matters is that every SIMD has a share: forward, 32 rows x 64 experts per block with k dealt to its eight waves;
 // dW_r, whose outputs fill 16 blocks only, the rows cut into chunks and the partial sums added in chunk order; dx in the same launch, so that
 // the blocks of either fill the CUs that the other leaves.  Loads never depend on a branch (mts_f32_tiles.h).
-// 8192 x 1024, 64 experts, bf16: 15.8 us forward, 29 + 5.5 backward; 22 and 19 + 17 + 6 with branches at the loads, four waves, 2-byte stores
+// 8192 x 1024, 64 experts: 15.8 us forward, 29 + 5.5 backward; 22 and 19 + 17 + 6 with branches at the loads, four waves, 2-byte stores
 // of dx and a launch each.  16 384 x 2048, 128 experts: 124 -> 95 and 210 -> 188.
+//
+// Backward of bf16 rows, from 1024 on (split_bwd_kernel): the fp32 operands as three bf16 terms each, which the bf16 instruction multiplies at 16 times the rate,
+// three products for dW_r and six for dx.  Two waves a SIMD and what they wait for bound it then, so operands go from memory into fragments without
+// LDS, except w_r's terms, which many rows share.  The launch, us: 8192 x 1024, 64 experts 26.4 -> 16.1; 8192 x 768, 24 17.6 -> 11.3; 16 384 x 2048, 128
+// 148 -> 100, 32 experts 66 -> 30.  Error against fp64: dW_r 1.6e-7 (3.0e-7), 3.6e-7 (8.1e-7) at 16 384 x 2048, 128; dx its rounding.  The forward pass so
+// split, fragments from memory: 14.6 -> 15.0 us and 83 -> 91 (32 experts 42 -> 38), as every 32 rows read and split w_r anew: not taken.  dW_r with three or four
+// steps in flight 10.3 -> 13.7 and 15.0 us alone: more code than a short kernel can fetch.
 #include "mts_cast_block.h"
 #include "mts_f32_tiles.h"
 #include "mts_router_row.h"
+#include "mts_split3.h"
 
 #include <type_traits>
 
@@ -21,6 +29,55 @@ using namespace mts_f32;
 
 constexpr int kThreads = 256, kLogitsThreads = 512;
 constexpr int kBwdLds = 2 * (64 * 20 + 16 * 72);   // floats: the two buffers of dx
+
+// bf16 activations: the fp32 operand as three bf16 terms (mts_split3.h), split in registers as they come from memory; x needs no splitting, so that three
+// bf16 products make one that nothing is left out of.
+struct Split8 {
+    bf16x8 term[3];
+    bool exact;   // every one of the values is the sum of its terms, in every lane of the wave
+};
+__device__ __forceinline__ bool in_range(uint32_t bf16_bits) { return mts_split3::splits_exactly(__uint_as_float(bf16_bits << 16)); }
+__device__ __forceinline__ Split8 split8(const float (&value)[8]) {
+    Split8 s;
+    float v[8];
+    uint32_t keys = 0;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = value[j];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+        u32x4 h;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            h[i] = mts_split3::round2(v[2 * i], v[2 * i + 1]);
+            if (q < 2) v[2 * i] -= __uint_as_float(h[i] << 16), v[2 * i + 1] -= __uint_as_float(h[i] & 0xffff0000u);
+            if (q == 0) {
+                const mts_split3::u16x2 k = mts_split3::range_keys(h[i]);
+                keys = i == 0 ? __builtin_bit_cast(uint32_t, k) : __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(mts_split3::u16x2, keys), k));
+            }
+        }
+        s.term[q] = __builtin_bit_cast(bf16x8, h);
+    }
+    s.exact = true;
+    if (__ballot(max(keys & 0xffffu, keys >> 16) >= mts_split3::kRange)) {   // zeros, or values that the split does not hold
+        bool any = false;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) any |= !mts_split3::splits_exactly(value[j]);
+        s.exact = !__ballot(any);
+    }
+    return s;
+}
+// whether no product with terms of the split can leave the range, in every lane of the wave
+__device__ __forceinline__ bool ordinary(bf16x8 x) {
+    const u32x4 u = __builtin_bit_cast(u32x4, x);
+    mts_split3::u16x2 keys = mts_split3::range_keys(u[0]);
+#pragma unroll
+    for (int i = 1; i < 4; ++i) keys = __builtin_elementwise_max(keys, mts_split3::range_keys(u[i]));
+    if (!__ballot(max(keys[0], keys[1]) >= mts_split3::kRange)) return true;
+    bool any = false;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) any |= !in_range(u[i] & 0xffffu) || !in_range(u[i] >> 16);
+    return !__ballot(any);
+}
 
 // 32 rows x 64 experts; wave w multiplies k-step w of every 64-wide k-tile, the eight sums meet in LDS.  Two waves of a SIMD: one reads its
 // fragments while the other multiplies (four waves of two k-steps each: 19.9 us for 8192 x 1024 x 64 where this takes 15.8).
@@ -252,6 +309,243 @@ __global__ __launch_bounds__(kThreads) void wide_bwd_kernel(const float* __restr
     else wide_dx_block<XT, VEC>(dl, w, T, H, E, dx, blockIdx.x - dw_blocks, lds);
 }
 
+// Both gradients for bf16 rows, up to 128 experts, on the split.
+constexpr int kSplitCols = 128;   // columns of a dW_r block
+constexpr int kSplitDwLds = 4 * 16 * MTS_WAVE * 4;   // floats: the sums of four waves
+
+// partial dW_r over one chunk of rows, 32 experts x 128 columns per block, steps of 16 rows dealt to the waves.  A lane loads an expert and four columns of
+// eight rows: with the columns of a fragment four apart these are the fragments, without LDS.  (64 experts a block would split and convert half as
+// often, in more registers than there are.)
+__device__ __forceinline__ void split_dw_block(const float* __restrict__ dl, const bf16_t* __restrict__ x, int64_t T, int H, int E, int64_t rows_per_chunk,
+                                               float* __restrict__ part, unsigned tile, unsigned chunk, float* lds) {
+    typedef __attribute__((ext_vector_type(2))) uint32_t Columns;
+    const unsigned n_tiles = (unsigned)((H + kSplitCols - 1) / kSplitCols);
+    const int wave = threadIdx.x / MTS_WAVE, lane = threadIdx.x % MTS_WAVE;
+    const int e0 = (int)(tile / n_tiles) * 32, h = (int)(tile % n_tiles) * kSplitCols + lane % 32 * 4;
+    const int64_t r0 = (int64_t)chunk * rows_per_chunk;
+    const int rows = (int)(r0 + rows_per_chunk < T ? rows_per_chunk : T - r0), steps = (rows + 15) / 16;
+    const float* dp = dl + r0 * E + min(e0 + lane % 32, E - 1);
+    const bf16_t* xp = x + r0 * H + min(h, H - 4);
+    float d[2][8];
+    Columns c[2][8];
+    auto fetch = [&](int set, int s) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int64_t r = min(s * 16 + lane / 32 * 8 + j, rows - 1);
+            d[set][j] = dp[r * E];
+            c[set][j] = *reinterpret_cast<const Columns*>(xp + r * H);
+        }
+    };
+    f32x16 acc[4] = {};
+    auto multiply = [&](int set, int s) {   // false: not this step
+        if (s * 16 + 16 > rows) {   // the last step: zeros on both sides
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                if (s * 16 + lane / 32 * 8 + j >= rows) d[set][j] = 0.f, c[set][j] = Columns{};
+        }
+        mts_split3::u16x2 keys = mts_split3::range_keys(c[set][0][0]);
+#pragma unroll
+        for (int i = 1; i < 16; ++i) keys = __builtin_elementwise_max(keys, mts_split3::range_keys(c[set][i / 2][i % 2]));
+        bool plain = true;
+        if (__ballot(max(keys[0], keys[1]) >= mts_split3::kRange)) {   // zeros, or values beyond the range of the split's
+            bool any = false;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) any |= !in_range(c[set][i / 2][i % 2] & 0xffffu) || !in_range(c[set][i / 2][i % 2] >> 16);
+            plain = !__ballot(any);
+        }
+        bf16x8 xv[4];
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            u32x4 u;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) u[i] = __builtin_amdgcn_perm(c[set][2 * i + 1][p / 2], c[set][2 * i][p / 2], p % 2 ? 0x07060302u : 0x05040100u);
+            xv[p] = __builtin_bit_cast(bf16x8, u);
+        }
+        const Split8 t = split8(d[set]);
+        if (!plain || !t.exact) return false;
+#pragma unroll
+        for (int q = 2; q >= 0; --q)
+#pragma unroll
+            for (int p = 0; p < 4; ++p) acc[p] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(t.term[q], xv[p], acc[p], 0, 0, 0);
+        return true;
+    };
+    int s = wave;
+    if (s < steps) fetch(0, s);
+    for (bool exact = true; exact && s < steps;) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            fetch(1 - u, s + 4);
+            __builtin_amdgcn_sched_barrier(0);   // the loads stay in front
+            if (!(exact = multiply(u, s)) || (s += 4) >= steps) break;
+        }
+    }
+#pragma unroll 1
+    for (; s < steps; s += 4)   // from a step on that holds a value the split does not: by the fp32 instruction, whose k is lane / 32
+#pragma unroll 1
+        for (int j = 0; j < 8; ++j) {
+            const int64_t r = s * 16 + lane / 32 * 8 + j;
+            const bool in = r < rows;
+            const float dv = in ? dp[r * E] : 0.f;
+            const Columns cv = in ? *reinterpret_cast<const Columns*>(xp + r * H) : Columns{};
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+                const float xf = __uint_as_float(p % 2 ? cv[p / 2] & 0xffff0000u : cv[p / 2] << 16);
+                acc[p] = __builtin_amdgcn_mfma_f32_32x32x2f32(dv, xf, acc[p], 0, 0, 0);
+            }
+        }
+    // the waves' sums in wave order; wave w adds and stores rows 8w .. 8w + 7
+    f32x4* sums = reinterpret_cast<f32x4*>(lds);
+    float* out = part + (int64_t)chunk * E * H;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) sums[(wave * 16 + i) * MTS_WAVE + lane] = f32x4{acc[0][i], acc[1][i], acc[2][i], acc[3][i]};
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        f32x4 v = sums[(4 * wave + i) * MTS_WAVE + lane];
+#pragma unroll
+        for (int k = 1; k < 4; ++k) v += sums[(k * 16 + 4 * wave + i) * MTS_WAVE + lane];
+        const int m = e0 + 8 * wave + 4 * (lane / 32) + i;
+        if (m < E && h < H) *reinterpret_cast<f32x4*>(out + (int64_t)m * H + h) = v;
+    }
+}
+
+// dx: a block keeps the terms of w_r for COLS columns and all experts in LDS and takes 32 rows a wave at a time, whose dlogits are split in registers.  The
+// columns of a fragment are dealt so that a lane ends with 16 consecutive ones.
+template <int KS>
+struct SplitDx {
+    static constexpr int COLS = KS > 4 ? 64 : 128, LD = KS * 16 + 8, PLANE = COLS * LD;   // bf16; rows of 16 bytes more than a multiple of 64: reads of eight lanes on all banks
+    static constexpr int LDS = 3 * PLANE / 2 + 4;   // floats, and the flag
+    static constexpr int column(int m) { return 16 * (m >> 2 & 1) + 4 * (m >> 3) + (m & 3); }
+
+    static __device__ __forceinline__ void block(const float* __restrict__ dl, const float* __restrict__ w, int64_t T, int H, int E, bf16_t* __restrict__ dx, unsigned block,
+                                                 unsigned row_blocks, float* lds) {
+        bf16_t* terms = reinterpret_cast<bf16_t*>(lds);
+        int* special = reinterpret_cast<int*>(lds + 3 * PLANE / 2);
+        const int n_tiles = (H + COLS - 1) / COLS, n0 = (int)(block % n_tiles) * COLS;
+        const int wave = threadIdx.x / MTS_WAVE, lane = threadIdx.x % MTS_WAVE;
+        if (threadIdx.x == 0) *special = 0;
+        const int64_t step = (int64_t)row_blocks * 128;
+        int64_t row0 = ((int64_t)(block / n_tiles) * 4 + wave) * 32;
+        f32x4 raw[KS][2];
+        auto fetch = [&](int64_t r) {
+            const float* dp = dl + (r < T ? r : T - 1) * E;
+#pragma unroll
+            for (int s = 0; s < KS; ++s)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) raw[s][h] = *reinterpret_cast<const f32x4*>(dp + min(16 * s + lane / 32 * 8, E - 8) + 4 * h);
+        };
+        fetch(row0 + lane % 32);
+        constexpr int PIECES = COLS * KS * 2 / kThreads;   // eight experts of a column
+        float v[PIECES][8];
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i) {
+            const int at = i * kThreads + threadIdx.x, col = min(n0 + at % COLS, H - 1);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[i][j] = w[(int64_t)min(at / COLS * 8 + j, E - 1) * H + col];
+        }
+        __builtin_amdgcn_sched_barrier(0);   // the loads stay together in front
+        __syncthreads();
+        bool exact = true;
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i) {
+            const int at = i * kThreads + threadIdx.x, c = at % COLS, k0 = at / COLS * 8;
+            if (k0 >= E) {
+#pragma unroll
+                for (int j = 0; j < 8; ++j) v[i][j] = 0.f;
+            }
+            const Split8 s = split8(v[i]);
+            exact &= s.exact;
+#pragma unroll
+            for (int q = 0; q < 3; ++q) *reinterpret_cast<bf16x8*>(terms + q * PLANE + c * LD + k0) = s.term[q];
+        }
+        if (!exact && lane == 0) *special = 1;
+        __syncthreads();
+        const bool plain = *special == 0;
+        const int cm = column(lane % 32);
+        for (; row0 < T; row0 += step) {
+            const int64_t r = row0 + lane % 32;
+            const float* dp = dl + (r < T ? r : T - 1) * E;
+            Split8 d[KS];
+            bool all = plain;
+#pragma unroll
+            for (int s = 0; s < KS; ++s) {
+                float v[8];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) v[j] = 16 * s + lane / 32 * 8 < E ? raw[s][j / 4][j % 4] : 0.f;
+                d[s] = split8(v);
+                all &= d[s].exact;
+            }
+            fetch(r + step);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int nf = 0; nf < COLS / 32; ++nf) {
+                f32x16 acc = {};
+                if (all) {
+#pragma unroll
+                    for (int s = 0; s < KS; ++s) {
+                        bf16x8 a[3];
+#pragma unroll
+                        for (int q = 0; q < 3; ++q) a[q] = *reinterpret_cast<const bf16x8*>(terms + q * PLANE + (nf * 32 + cm) * LD + 16 * s + lane / 32 * 8);
+                        constexpr int kTerms[6][2] = {{2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}, {0, 0}};   // small ones first
+#pragma unroll
+                        for (int t = 0; t < 6; ++t) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[kTerms[t][0]], d[s].term[kTerms[t][1]], acc, 0, 0, 0);
+                    }
+                } else {   // by the fp32 instruction, whose k is lane / 32
+                    const float* wp = w + min(n0 + nf * 32 + cm, H - 1);
+#pragma unroll 1
+                    for (int k = lane / 32; k < (E + 1) / 2 * 2; k += 2)
+                        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(k < E ? wp[(int64_t)k * H] : 0.f, k < E ? dp[k] : 0.f, acc, 0, 0, 0);
+                }
+                const int h = n0 + nf * 32 + 16 * (lane / 32);
+#pragma unroll
+                for (int g = 0; g < 2; ++g) {
+                    bf16x8 v;
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) v[j] = (bf16_t)acc[8 * g + j];
+                    if (r < T && h + 8 * g < H) *reinterpret_cast<bf16x8*>(dx + r * H + h + 8 * g) = v;
+                }
+            }
+        }
+    }
+};
+
+// KS: steps of 16 experts
+template <int KS>
+__global__ __launch_bounds__(kThreads, 2) void split_bwd_kernel(const float* __restrict__ dl, const bf16_t* __restrict__ x, const float* __restrict__ w, int64_t T, int H,
+                                                                int E, int64_t rows_per_chunk, unsigned dw_tiles, unsigned chunks, unsigned row_blocks,
+                                                                bf16_t* __restrict__ dx, float* __restrict__ part) {
+    constexpr int LDS = SplitDx<KS>::LDS > kSplitDwLds ? SplitDx<KS>::LDS : kSplitDwLds;
+    __shared__ __attribute__((aligned(16))) float lds[LDS];
+    const unsigned dw_blocks = dw_tiles * chunks;
+    if (blockIdx.x < dw_blocks) split_dw_block(dl, x, T, H, E, rows_per_chunk, part, blockIdx.x % dw_tiles, blockIdx.x / dw_tiles, lds);
+    else SplitDx<KS>::block(dl, w, T, H, E, dx, blockIdx.x - dw_blocks, row_blocks, lds);
+}
+
+// Whole pieces of eight experts and columns are what the loads take, and the terms of more than 128 experts do not fit.  Fewer rows leave the blocks a chain
+// of latencies either way: 256 of 768 and 24 experts 4.8 us / 4.8 here, 613 and 32 experts 5.2 / 5.6, 993 and 24 5.8 / 5.6; 2048 of 1024 and 64 13.9 / 8.7.
+bool split_bwd_takes(int64_t T, int H, int E, int act_dtype) {
+    return act_dtype == MTS_BF16 && H % 8 == 0 && E % 8 == 0 && E <= 128 && T >= 1024;
+}
+struct SplitGrid {
+    int64_t rows;
+    unsigned dw_tiles, chunks, col_tiles, row_blocks;
+};
+// A block of each kind per CU; chunks of 128 rows or more.
+SplitGrid split_grid(int64_t T, int H, int E) {
+    SplitGrid g;
+    g.dw_tiles = (unsigned)((E + 31) / 32 * ((H + kSplitCols - 1) / kSplitCols));
+    int64_t count = (256 + g.dw_tiles - 1) / g.dw_tiles;
+    const int64_t most = (T + 127) / 128;
+    if (count > most) count = most;
+    g.rows = ((T + count - 1) / count + 15) / 16 * 16;
+    g.chunks = (unsigned)((T + g.rows - 1) / g.rows);
+    const int cols = E > 64 ? SplitDx<8>::COLS : SplitDx<4>::COLS;
+    g.col_tiles = (unsigned)((H + cols - 1) / cols);
+    const int64_t want = (256 + g.col_tiles - 1) / g.col_tiles, need = (T + 127) / 128;
+    g.row_blocks = (unsigned)(want < need ? want : need);
+    return g;
+}
+
 // Rows are cut into as many chunks as make about two blocks per CU, of at least 64 rows.
 struct WideChunks {
     int64_t rows;
@@ -317,7 +611,8 @@ int mts_launch_wide_head(const void* x, const float* w_r, int64_t T, int H, int 
 
 extern "C" int64_t mts_router_wide_bwd_workspace_bytes(int64_t T, int H, int E) {
     if (T <= 0 || H <= 0 || E <= 0) return 0;
-    return (int64_t)wide_chunks(T, H, E).count * E * H * (int64_t)sizeof(float);
+    const int64_t chunks = wide_chunks(T, H, E).count, split = split_bwd_takes(T, H, E, MTS_BF16) ? split_grid(T, H, E).chunks : 0;
+    return (chunks > split ? chunks : split) * E * H * (int64_t)sizeof(float);
 }
 
 extern "C" int mts_router_wide_bwd(const float* dlogits, const void* x, const float* w_r, int64_t T, int H, int E, int act_dtype, void* dx,
@@ -328,6 +623,19 @@ extern "C" int mts_router_wide_bwd(const float* dlogits, const void* x, const fl
     if (workspace_bytes < mts_router_wide_bwd_workspace_bytes(T, H, E)) return MTS_ERR_WORKSPACE;
     if (!mts_aligned16(dlogits) || !mts_aligned16(dx) || !mts_aligned16(d_w_r) || !mts_aligned16(workspace)) return MTS_ERR_ALIGN;
     hipStream_t s = (hipStream_t)stream;
+    if (split_bwd_takes(T, H, E, act_dtype)) {
+        const SplitGrid g = split_grid(T, H, E);
+        const unsigned blocks = g.dw_tiles * g.chunks + g.col_tiles * g.row_blocks;
+        auto launch = [&](auto steps) {
+            split_bwd_kernel<decltype(steps)::value><<<blocks, kThreads, 0, s>>>(dlogits, (const bf16_t*)x, w_r, T, H, E, g.rows, g.dw_tiles, g.chunks, g.row_blocks,
+                                                                                 (bf16_t*)dx, (float*)workspace);
+        };
+        if (E <= 32) launch(std::integral_constant<int, 2>());
+        else if (E <= 64) launch(std::integral_constant<int, 4>());
+        else launch(std::integral_constant<int, 8>());
+        MTS_CHECK_LAUNCH();
+        return mts_launch_router_dw_reduce((const float*)workspace, (int)g.chunks, (int64_t)E * H, d_w_r, s);
+    }
     const bool vec = E % 4 == 0;
     const WideChunks c = wide_chunks(T, H, E);
     const unsigned dw_tiles = (unsigned)((H + 63) / 64 * ((E + 63) / 64));
