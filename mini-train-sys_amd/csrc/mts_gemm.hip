@@ -634,15 +634,18 @@ __host__ __device__ __forceinline__ int paired_tiles(int tiles) {
 // (a weight-gradient tile of two k-tiles 12.9 -> 11.1 us); the layer of 24 576 tokens 877 -> 868 us, 4096 tokens of 4096/14336 -1.4 %.
 // mtile: the m-tile's index in expert order, -1 where the block has none; a block that has the empty half of a cut tile
 // (the tile's rows end in the other half) gets the index and the answer false.
-template <int BM>
+// ONE: there may be no table, then one expert has all rows.  A kernel of its own form, as the choice costs the others up to 1 us a launch
+// (dO*W2 of 6001 tokens of 1000/1368 89.0 -> 90.2).
+template <int BM, bool ONE>
 __device__ __forceinline__ bool find_rows_tile(const RowsParams& p, int b, int& e, int& row0, int& rend, int& ntile, int& parts,
                                                int& mtile) {
     mtile = -1;
     // up to 64 experts: lane l reads expert_start[l] and [l + 1] once, for the count of m-tiles and for the search
     const bool in_regs = p.E <= MTS_WAVE;
     const int lane = threadIdx.x % MTS_WAVE;
-    int w0 = lane ? (int)p.TK : 0, w1 = (int)p.TK;   // no table: one expert has all rows
-    if (p.expert_start) w0 = p.expert_start[min(lane, p.E)], w1 = p.expert_start[min(lane + 1, p.E)];   // equal behind the last expert
+    const int32_t* table = ONE && !p.expert_start ? reinterpret_cast<const int32_t*>(p.B) : p.expert_start;   // a load that no branch is in front of
+    int w0 = table[min(lane, p.E)], w1 = table[min(lane + 1, p.E)];   // equal behind the last expert
+    if (ONE && !p.expert_start) w0 = lane ? (int)p.TK : 0, w1 = (int)p.TK;
     const int wnt = (w1 - w0 + BM - 1) / BM, wincl = wave_scan(wnt);   // in_regs: the lane's m-tiles, and those up to its last one
     const int xcd = b % kXcds;
     int j = b / kXcds;
@@ -650,7 +653,7 @@ __device__ __forceinline__ bool find_rows_tile(const RowsParams& p, int b, int& 
     int tile = xcd + kXcds * k;
     parts = 1;      // pieces the tile is cut into: this block computes piece `part`
     int part = 0;
-    if (p.flat) {
+    if (ONE && p.flat) {
         tile = p.by_n_tiles.quotient(b, ntile);
     } else if (p.xcd_ranges && p.sched) {
         // the XCD's range of m-tiles comes from the table (n-tile groups and cut tiles are not combined with it); a block
@@ -754,11 +757,11 @@ __device__ __forceinline__ void gather_rows(const int32_t* __restrict__ gather, 
 // The answer is the same in every lane, and the compiler is told so behind the search loop: descriptors
 // and LDS addresses built from these values then stay in scalar registers (a buffer instruction whose
 // descriptor sits in vector registers is wrapped in a loop over its distinct values).
-template <int BM>
+template <int BM, bool ONE = false>
 __device__ __forceinline__ bool locate_rows_tile(const RowsParams& p, int b, int& e, int& row0, int& rend, int& ntile, int& parts,
                                                  int& mtile) {
     int fe = 0, frow0 = 0, frend = 0, fn = 0, fh = 1, fm = -1;
-    const bool found = find_rows_tile<BM>(p, b, fe, frow0, frend, fn, fh, fm);
+    const bool found = find_rows_tile<BM, ONE>(p, b, fe, frow0, frend, fn, fh, fm);
     e = __builtin_amdgcn_readfirstlane(fe);
     row0 = __builtin_amdgcn_readfirstlane(frow0);
     rend = __builtin_amdgcn_readfirstlane(frend);
@@ -767,15 +770,15 @@ __device__ __forceinline__ bool locate_rows_tile(const RowsParams& p, int b, int
     mtile = __builtin_amdgcn_readfirstlane(fm);
     return __builtin_amdgcn_readfirstlane((int)found) != 0;
 }
-template <int BM>
+template <int BM, bool ONE = false>
 __device__ __forceinline__ bool locate_rows_tile(const RowsParams& p, int b, int& e, int& row0, int& rend, int& ntile, int& parts) {
     int mtile;
-    return locate_rows_tile<BM>(p, b, e, row0, rend, ntile, parts, mtile);
+    return locate_rows_tile<BM, ONE>(p, b, e, row0, rend, ntile, parts, mtile);
 }
-template <int BM>
+template <int BM, bool ONE = false>
 __device__ __forceinline__ bool locate_rows_tile(const RowsParams& p, int b, int& e, int& row0, int& rend, int& ntile) {
     int parts;   // a slice of a tile is a tile with fewer rows to a kernel that does not treat it specially
-    return locate_rows_tile<BM>(p, b, e, row0, rend, ntile, parts);
+    return locate_rows_tile<BM, ONE>(p, b, e, row0, rend, ntile, parts);
 }
 
 // ---------------------------------------------------------------------------
@@ -792,7 +795,7 @@ __global__ __launch_bounds__(T::NT) void rows_gemm_kernel(RowsParams p) {
         if (schedule_block(p)) return;
     }
     int e, row0, rend, ntile;
-    if (!locate_rows_tile<T::BM>(p, blockIdx.x, e, row0, rend, ntile)) return;
+    if (!locate_rows_tile<T::BM, EPI == EPI_PLAIN>(p, blockIdx.x, e, row0, rend, ntile)) return;
     const int n0 = ntile * (SWIGLU ? T::BN / 2 : T::BN);  // first output column of this block
 
     KMajorLoader<T::BM, T::NT> la;
@@ -937,7 +940,7 @@ __global__ __launch_bounds__(T::NT, T::WAVES_PER_EU) void rows_gemm_ring_kernel(
         if (schedule_block(p)) return;
     }
     int e, row0, rend, ntile;
-    if (!locate_rows_tile<T::BM>(p, blockIdx.x, e, row0, rend, ntile)) return;
+    if (!locate_rows_tile<T::BM, EPI == EPI_PLAIN>(p, blockIdx.x, e, row0, rend, ntile)) return;
     const int n0 = ntile * (SWIGLU ? T::BN / 2 : T::BN);
     const int wave = threadIdx.x / MTS_WAVE, lane = threadIdx.x % MTS_WAVE;
     const int wm = wave / T::WAVES_N, wn = wave % T::WAVES_N;
@@ -1628,13 +1631,13 @@ __device__ __forceinline__ void rows_gemm_ws_run(const RowsParams& p, bf16_t* sm
     rows_gemm_ws_tile<T, EPI, BKM>(p, smem, e, row0, rend, ntile, rows_ready);
 }
 
-template <class T, int EPI, bool BKM, class TH = T>
+template <class T, int EPI, bool BKM, class TH = T, bool ONE = false>
 __device__ __forceinline__ void rows_gemm_ws_block(const RowsParams& p, bf16_t* smem, int block) {
     static_assert(TH::NT == T::NT && TH::BN == T::BN && (TH::BM == T::BM || 2 * TH::BM == T::BM), "half tile shape");
     static_assert(ws_lds_elems<TH, EPI>() <= ws_lds_elems<T, EPI>(), "the half tile fits the same LDS");
     static_assert(EPI != EPI_DY1N || T::STAGES != 2 || 2 * TH::NWAVES * 4096 <= ws_lds_elems<T, EPI>(), "two slabs of the half tile fit it");
     int e, row0, rend, ntile, parts;
-    if (!locate_rows_tile<T::BM>(p, block, e, row0, rend, ntile, parts)) return;
+    if (!locate_rows_tile<T::BM, ONE>(p, block, e, row0, rend, ntile, parts)) return;
     rows_gemm_ws_run<T, EPI, BKM, TH>(p, smem, e, row0, rend, ntile, parts);
 }
 
@@ -1645,7 +1648,7 @@ __global__ __launch_bounds__(T::NT, T::WAVES_PER_EU) void rows_gemm_ws_kernel(Ro
     if constexpr (epi_is_dy1(EPI)) {
         if (schedule_block(p)) return;
     }
-    rows_gemm_ws_block<T, EPI, BKM, TH>(p, smem, blockIdx.x);
+    rows_gemm_ws_block<T, EPI, BKM, TH, EPI == EPI_PLAIN>(p, smem, blockIdx.x);
 }
 
 // ---------------------------------------------------------------------------
