@@ -186,17 +186,26 @@ extern "C" int mts_moe_fwd_few_rows_supported(int act_dtype, int weight_dtype, i
     return ((wide + kCols - 1) / kCols + 7) / 8 * 8 * (TK / 16 + E) * kThreads < (1LL << 32);
 }
 
-// Against the large tiles (a forward pass of the layer, us; here / there).  They lose to it where they are few: gate/up makes one
+// Against the tiles (a forward pass of the layer, us; here / there).  They lose to it where they are few: gate/up makes one
 // for every expert and 256 of its 2I columns, and the chip has 256 CUs.  768/1024, 8 experts (64 of them): 4 rows an expert
-// 48 / 52, 32 rows 46 / 56, 64 rows 59 / 57; 16 experts (128): 8 rows 52 / 63, 16 rows 56 / 64, 32 rows 66 / 64; 1024/512, 64
-// experts (256): 1 row 82 / 91, 8 rows 97 / 99, 16 rows 115 / 101.  fp32 weights need no rounded copies in front, which move
-// more bytes than the products: 768/1024, 8 experts: 4 rows 46 / 67, 64 rows 69 / 74, 128 rows 82 / 75; 1024/512, 64 experts:
-// 4 rows 140 / 217, 64 rows 222 / 227; 2048/768, 128 experts: 4 rows 490 / 1094, 64 rows 904 / 1162.
+// 34 / 36, 32 rows 47 / 42; 512/1024 24 rows 38 / 38, 64 rows 47 / 40; 512/2048 24 rows 43 / 46, 32 rows 49 / 46.  With more than 64 tokens the routing is
+// a second launch for both, which costs this path 6 and the tiles 3; there 768/1024 and 1024/1024 are behind from 12 rows on (12 rows 40 / 41 and 46 / 45,
+// 24 rows 44 / 41 and 49 / 44).
+// fp32 weights need no rounded copies in front.  With up to 64 tokens these are a launch of their own: 768/1024, 8 experts: 16 rows an expert 46 / 52, 32 rows
+// 53 / 54.  With more they are made beside the head and the routing, and what counts is how much there is to read and how many columns share it: 512/512
+// (6 M weights) 24 rows 33 / 36, 64 rows 37 / 37; 1024/512 (13 M) 24 rows 44 / 44, 64 rows 50 / 45; 768/1024 (19 M) 12 rows 48 / 43, 64 rows 65 / 44; 1024/1024
+// (25 M) 24 rows 58 / 50, 64 rows 71 / 51; 512/2048 (25 M) 24 rows 47 / 53, 64 rows 72 / 54; 1024/2048 (50 M) 48 rows 84 / 87, 64 rows 110 / 87; 16 experts of
+// 768/1024 (38 M) 8 rows 58 / 62, 12 rows 68 / 63; 64 of 1024/512 (100 M) 32 rows 149 / 168; 32 of 2048/768 (151 M) 64 rows 255 / 260.
 extern "C" int mts_moe_fwd_few_rows_preferred(int act_dtype, int weight_dtype, int64_t T, int64_t TK, int E, int H, int I) {
     if (!mts_moe_fwd_few_rows_supported(act_dtype, weight_dtype, T, TK, E, H, I)) return 0;
-    if (weight_dtype == MTS_F32) return TK <= 64LL * E;
-    const int64_t large = E * ((2LL * I + 255) / 256), rows = 2048 / large;
-    return TK <= (rows < 8 ? 8 : (rows > 48 ? 48 : rows)) * E;
+    const int64_t weights = 3LL * E * H * I;
+    const bool one_launch = T <= 64, broad = I >= 2 * H, light = weights <= 14LL << 20;
+    if (weight_dtype == MTS_F32) {
+        const int rows = one_launch || weights >= 90LL << 20 ? 64 : broad && weights >= 45LL << 20 ? 48 : broad || light ? 24 : 8;
+        return TK <= (int64_t)rows * E;
+    }
+    const int64_t large = E * ((2LL * I + 255) / 256), most = one_launch || broad || light ? 48 : 12, rows = 2048 / large;
+    return TK <= (rows < 8 ? 8 : (rows > most ? most : rows)) * E;
 }
 
 extern "C" int mts_moe_fwd_few_rows(const void* x, const void* w1, const void* w2, int weight_dtype, const int32_t* x_gather, const int32_t* expert_start,

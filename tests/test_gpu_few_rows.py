@@ -88,3 +88,19 @@ def test_layer_with_and_without_a_backward_pass(T, dtype):
     assert torch.equal(trained, read)
     trained.sum().backward()
     assert all(t.grad.isfinite().all() for t in (w_r, w1, w2))
+
+
+@pytest.mark.parametrize("T,K,E,H,I", [(64, 2, 8, 768, 1024), (65, 2, 8, 768, 1024), (65, 1, 8, 512, 512), (193, 1, 8, 1024, 512), (96, 2, 8, 512, 2048), (97, 2, 8, 512, 2048),
+                                       (192, 2, 8, 1024, 2048), (193, 2, 8, 1024, 2048), (64, 2, 16, 768, 1024), (65, 2, 16, 768, 1024)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_either_side_of_the_rule(T, K, E, H, I, dtype):
+    """fp32 master weights without a backward pass, read as they are or rounded first, on both sides of every line of the rule: as with weights that were rounded
+    before.  The two sum the same products in other orders, which moves a rounding of either expert row or of the output by one step at most."""
+    print(f"few rows rule T={T} K={K} E={E} H={H} I={I} {dtype}", flush=True)
+    g = torch.Generator().manual_seed(T + H)
+    x = torch.randn(T, H, generator=g).to(dtype).cuda()
+    w_r = torch.randn(E, H, generator=g).cuda()
+    w1, w2 = (torch.randn(E, 2 * I, H, generator=g) * H ** -0.5).cuda(), (torch.randn(E, H, I, generator=g) * I ** -0.5).cuda()
+    with torch.no_grad():
+        got, want = (moe_layer(x, w_r, a, b, K, normalize=True)[0] for a, b in ((w1, w2), (w1.to(dtype), w2.to(dtype))))
+    _close(got, want.double(), 4 * ULP[dtype], "out")
