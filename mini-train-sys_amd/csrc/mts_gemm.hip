@@ -2788,10 +2788,11 @@ int64_t m_tiles_of_xcd(int64_t TK, int E, int bm, bool even) {
     return (tiles2 + 2 * kXcds - 1) / (2 * kXcds);
 }
 // whether dO*W2 on large tiles (`wide` columns of them) is ahead of three narrow blocks a CU that fit their round
-bool large_tiles_ahead(int64_t TK, int E, int64_t narrow, int64_t wide) {
+bool large_tiles_ahead(int64_t TK, int E, int Kdim, int64_t narrow, int64_t wide) {
+    const int round = 2 * kCusPerXcd, most = Kdim > 768 ? round : round * 7 / 8;
     for (const bool even : {true, false}) {
         const int64_t a_cu = (m_tiles_of_xcd(TK, E, RingThreePerCu::BM, even) * narrow + kCusPerXcd - 1) / kCusPerXcd, large = m_tiles_of_xcd(TK, E, WsWide::BM, even) * wide;
-        if (a_cu < 2 || 2 * large > (a_cu == 2 ? kCusPerXcd : 2 * kCusPerXcd)) return false;
+        if (a_cu < 2 || 2 * large > (a_cu == 2 ? round / 2 : most)) return false;
     }
     return true;
 }
@@ -2817,11 +2818,14 @@ int launch_rows_any(int kind, RowsParams p, int64_t TK, hipStream_t s, bool b_km
     // Within that round a CU holds one, two or three of the narrow blocks (768/1024: 23, 29 and 41 us), and where the large tiles are a round of one block a CU
     // they are ahead of three (35), and of two where they are half a round and cut (24).  Asked for routes spread evenly and for half a tile more an expert, and
     // changed where both say so.  Of 360 calls, even, random and with popular experts, 108 changed: 2946 tokens of 768/1024 29.1 / 24.2, 6544 of 776/1024 46.4 /
-    // 39.3, 4195 of 1000/1368 53.0 / 44.1, 8261 of 768/768 43.1 / 37.6, 5122 of 1000/680 with 16 experts, top-3, 55.7 / 40.1; none more than the noise slower.
+    // 39.3, 4195 of 1000/1368 53.0 / 44.1, 8261 of 768/768 43.1 / 37.6, 5122 of 1000/680 with 16 experts, top-3, 55.7 / 40.1.
+    // A round that is nearly full is no better where sums are short and routes uneven: the whole pass of 3410 tokens of 512/1024, top-4, 231 / 237, 9202 of 768/768 with
+    // 16 experts 438 / 448; so up to 768 of k it is seven eighths of one at most.  Of 44 such passes none is then more than 1 % slower, and 1.6 % shorter on average
+    // (6406 of 776/1024 323 / 315, 3843 of 512/1536 240 / 221).
     if (choice == 3 && !tile_forced(kind)) {
         const int64_t narrow = (p.N + RingThreePerCu::BN - 1) / RingThreePerCu::BN, wide = (p.N + WsWide::BN - 1) / WsWide::BN * (WsWide::BN / RingThreePerCu::BN);
         const int64_t blocks = (TK + RingThreePerCu::BM - 1) / RingThreePerCu::BM * narrow;
-        if (p.Kdim > 1024 || (8 * wide <= 9 * narrow && (blocks > 3 * kXcds * kCusPerXcd || large_tiles_ahead(TK, p.E, narrow, wide / 2)))) choice = 4;
+        if (p.Kdim > 1024 || (8 * wide <= 9 * narrow && (blocks > 3 * kXcds * kCusPerXcd || large_tiles_ahead(TK, p.E, p.Kdim, narrow, wide / 2)))) choice = 4;
     }
     // the 64-wide variant exists for the GEMMs with a plain or SwiGLU epilogue
     if (choice == 4 && epi_is_dy1(EPI) && (EPI != EPI_DY1N || !b_kmajor)) choice = 2;
