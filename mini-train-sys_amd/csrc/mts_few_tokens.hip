@@ -10,7 +10,7 @@
 //  * a block of the second launch takes 16 columns of the down projection of every expert with rows, four waves an expert, and adds a token's routes from
 //    LDS, each rounded as a row of the down projection is.
 // The products are the same sums in the same order as those of mts_few_rows.hip; the logits are the fp32 instruction's in four parts.  16 tokens, 8 experts of
-// 768/1024, us of kernels: 9.2 + 11.0 + 5.0 + 3.1 in four launches, 14.1 + 7.2 in two (1.8 TB/s of weights in both); 31.5 -> 23.9 us a call.
+// 768/1024, us of kernels: 9.2 + 11.0 + 5.0 + 3.1 in four launches, 14.5 + 7.8 in two (1.8 TB/s of weights in both); 32.8 -> 24.7 us a call.
 #include "mts_few_block.h"
 #include "mts_router_row.h"
 
