@@ -11,7 +11,9 @@ _walked = attrgetter(*_WALKED)
 
 
 def plain_modules(model: nn.Module) -> list[nn.Module] | None:
-    """``list(model.modules())``, or None where a module answers one of the calls that the walk stands for in a way of its own."""
+    """``list(model.modules())``, or None where the model or a module in it answers one of the calls that the walk stands for in a way of its own."""
+    if not isinstance(model, nn.Module):   # anything with ``train()`` and ``parameters()``
+        return None
     modules, seen = [model], {model}
     for module in modules:   # grows on the way
         for child in module._modules.values():

@@ -5,6 +5,7 @@ import torch
 from torch import nn
 
 from minitrain_amd.train.modules import parameters_of, plain_modules, set_training
+from minitrain_amd.train.step import train_step
 
 
 def _model():
@@ -49,3 +50,34 @@ def test_a_module_with_an_answer_of_its_own_is_asked(name, how):
     assert {id(p) for p in parameters_of(model, plain_modules(model))} == {id(p) for p in model.parameters()}
     model[1][-1].__dict__.pop(name, None)
     assert torch.is_tensor(model[1][-1].weight)
+
+
+class _Head(nn.Linear):
+    def forward(self, ids, *, targets, use_fused_loss):
+        return (super().forward(ids) - targets).square().mean(), None
+
+
+class _Wrapper:
+    """No module, but all that a step calls."""
+
+    def __init__(self, model):
+        self.model, self.asked = model, 0
+
+    def train(self):
+        self.asked += 1
+        return self.model.train()
+
+    def parameters(self):
+        return self.model.parameters()
+
+    def __call__(self, *args, **kwargs):
+        return self.model(*args, **kwargs)
+
+
+def test_a_model_that_is_no_module_is_asked():
+    model = _Wrapper(_Head(2, 1).eval())
+    before = [p.detach().clone() for p in model.parameters()]
+    train_step(model, torch.optim.SGD(model.parameters(), lr=0.1), {"input_ids": torch.ones(1, 2), "targets": torch.full((1, 1), 5.0)})
+    assert model.asked == 1 and model.model.training
+    assert not any(torch.equal(a, b) for a, b in zip(before, model.parameters()))
+    assert plain_modules(model) is None and [id(p) for p in parameters_of(model, None)] == [id(p) for p in model.parameters()]
