@@ -6,7 +6,7 @@ from operator import attrgetter
 from torch import nn
 
 # what ``train()`` and ``parameters()`` go through, of every module on the way
-_WALKED = ("train", "parameters", "named_parameters", "_named_members", "named_modules", "children", "named_children")
+_WALKED = ("train", "parameters", "named_parameters", "_named_members", "named_modules", "children", "named_children", "__setattr__")
 _walked = attrgetter(*_WALKED)
 
 
@@ -21,8 +21,10 @@ def plain_modules(model: nn.Module) -> list[nn.Module] | None:
                 seen.add(child)
                 modules.append(child)
     stock = _walked(nn.Module)
+    if any(getattr(call, "__globals__", {}).get("__name__") != nn.Module.__module__ for call in stock):   # replaced for all modules
+        return None
     for cls in {type(m) for m in modules}:
-        if _walked(cls) != stock:
+        if _walked(cls) != stock or hasattr(cls, "training"):
             return None
     for module in modules:
         own = module.__dict__

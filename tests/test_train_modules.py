@@ -81,3 +81,43 @@ def test_a_model_that_is_no_module_is_asked():
     assert model.asked == 1 and model.model.training
     assert not any(torch.equal(a, b) for a, b in zip(before, model.parameters()))
     assert plain_modules(model) is None and [id(p) for p in parameters_of(model, None)] == [id(p) for p in model.parameters()]
+
+
+@pytest.mark.parametrize("name", ["train", "parameters", "_named_members"])
+def test_a_call_that_was_replaced_on_the_class_of_all_modules_is_made(monkeypatch, name):
+    calls, stock = [], getattr(nn.Module, name)
+
+    def answer(self, *args, **kwargs):
+        calls.append(name)
+        return stock(self, *args, **kwargs)
+
+    model = _model()
+    monkeypatch.setattr(nn.Module, name, answer)
+    set_training(model, plain_modules(model))
+    list(parameters_of(model, plain_modules(model)))
+    assert calls
+
+
+def test_a_class_that_watches_its_mode_is_told():
+    told = []
+
+    class Watching(nn.Linear):
+        def __setattr__(self, name, value):
+            if name == "training":
+                told.append(value)
+            super().__setattr__(name, value)
+
+    class Property(nn.Linear):
+        @property
+        def training(self):
+            return True
+
+        @training.setter
+        def training(self, value):
+            told.append(value)
+
+    for cls in (Watching, Property):
+        model = nn.Sequential(cls(3, 3))
+        told.clear()
+        set_training(model, plain_modules(model))
+        assert told == [True]
