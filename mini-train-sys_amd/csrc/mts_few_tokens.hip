@@ -368,7 +368,7 @@ __global__ __launch_bounds__(kThreads) void few_tokens_down_kernel(FewTokens p) 
             }
         }
     }
-    __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the rows' stores stay in front of it, the counter behind
     __syncthreads();
     if (threadIdx.x == 0) arrived = __hip_atomic_fetch_add(p.arrived + nt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
