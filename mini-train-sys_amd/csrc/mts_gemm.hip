@@ -2450,7 +2450,6 @@ struct BwdJointParams {
     DwParams dw1, dw2;
     RowsParams dx;
     int n_dw1, n_dw2, n_dx;        // blocks per part, in launch order
-    int dx_first;                  // dX's blocks in front of the weight gradients' (dx_in_front)
     const float* ds_part;          // [entries rows][np]
     const int32_t* s_reverse;      // entry -> row, negative for a dropped route
     bf16_t* d_weights;             // [entries]
@@ -2475,34 +2474,40 @@ struct BwdJointParams {
 
 static_assert(WsWide::BM == kSchedDxRows, "the schedule counts dX tiles of this height");
 typedef WsWide JointDxTile;   // dX reads d_pre_act row-major: whole lines per row with 64-wide k-tiles (a third buffer gains nothing here)
-template <typename OutT, class DxTile, class DxHalf>
+// LEAD: dX's blocks in front of the weight gradients' (dx_in_front).  A form of its own, as the choice at run time costs the order behind them half a per cent
+// of the launch (6001 tokens of 1000/1368, fp16: 241.0 -> 242.3 us).
+template <typename OutT, class DxTile, class DxHalf, bool LEAD = false>
 __global__ __launch_bounds__(WsLarge::NT, WsLarge::WAVES_PER_EU) void bwd_joint_kernel(BwdJointParams q) {
     static_assert(WsLarge::NT == JointDwTile::NT && DxTile::NT == WsLarge::NT, "one block shape");
     constexpr int ROWS_LDS = ws_lds_elems<DxTile, EPI_PLAIN>();
     constexpr int LDS_ELEMS = ROWS_LDS > JointDwTile::LDS_ELEMS ? ROWS_LDS : JointDwTile::LDS_ELEMS;
     static_assert(LDS_ELEMS * 2 <= 160 * 1024, "LDS capacity");
     __shared__ __attribute__((aligned(1024))) bf16_t smem[LDS_ELEMS];
-    int b = blockIdx.x, x = b - q.n_dw1 - q.n_dw2;   // x: the block of dX
-    const bool lead = !std::is_same<DxTile, WsSmall>::value && q.dx_first;
-    if (lead) {
-        x = b;
+    int b = blockIdx.x;
+    if (LEAD) {
+        if (b < q.n_dx) {
+            rows_gemm_ws_block<DxTile, EPI_PLAIN, true, DxHalf>(q.dx, smem, b);   // W1 as stored: [E][2I][H]
+            return;
+        }
         b -= q.n_dx;
     }
-    if (b >= 0 && b < q.n_dw1) {
+    if (b < q.n_dw1) {
         dw_gemm_ws_block<JointDwTile, OutT>(q.dw1, smem, b);
         return;
     }
     b -= q.n_dw1;
-    if (b >= 0 && b < q.n_dw2) {
+    if (b < q.n_dw2) {
         dw_gemm_ws_block<JointDwTile, OutT>(q.dw2, smem, b);
         return;
     }
     b -= q.n_dw2;
-    if (x < q.n_dx) {
-        rows_gemm_ws_block<DxTile, EPI_PLAIN, true, DxHalf>(q.dx, smem, x);   // W1 as stored: [E][2I][H]
-        return;
+    if (!LEAD) {
+        if (b < q.n_dx) {
+            rows_gemm_ws_block<DxTile, EPI_PLAIN, true, DxHalf>(q.dx, smem, b);
+            return;
+        }
+        b -= q.n_dx;
     }
-    if (!lead) b -= q.n_dx;
     if (b < q.n_ds) {
         for (int64_t n = (int64_t)b * WsLarge::NT + threadIdx.x; n < q.entries; n += (int64_t)q.n_ds * WsLarge::NT) {
             const int32_t r = q.s_reverse[n];
@@ -3079,7 +3084,7 @@ int launch_bwd_joint(BwdJointParams q, int E, int grad_dtype, void* ws1, int64_t
     }
     q.dx.reverse = (tile_order_mask() & ORDER_DX) ? 1 : 0;
     const bool small_dx = tile_forced(K_DX) ? tile_choice(K_DX) == 5 : small_tiles_pay(K_DX, q.dx.TK, E, q.dx.N, long_tiles(q.dx, E));
-    q.dx_first = !small_dx && dx_in_front(q.dx, E);
+    const bool dx_first = !small_dx && dx_in_front(q.dx, E);
     q.n_dx = (int)(small_dx ? rows_grid<WsSmall, EPI_PLAIN>(q.dx, q.dx.TK) : rows_grid<JointDxTile, EPI_PLAIN>(q.dx, q.dx.TK)).x;
     // With both workspaces (row chunks on) and a schedule from the caller (written by the dO*W2 launch), units and dX
     // tiles go to the XCDs as the table says.
@@ -3101,6 +3106,9 @@ int launch_bwd_joint(BwdJointParams q, int E, int grad_dtype, void* ws1, int64_t
     if (small_dx) {
         if (grad_dtype == MTS_GEMM_DTYPE) bwd_joint_kernel<bf16_t, WsSmall, WsSmall><<<grid, WsLarge::NT, 0, s>>>(q);
         else bwd_joint_kernel<float, WsSmall, WsSmall><<<grid, WsLarge::NT, 0, s>>>(q);
+    } else if (dx_first) {
+        if (grad_dtype == MTS_GEMM_DTYPE) bwd_joint_kernel<bf16_t, JointDxTile, WsWideHalf, true><<<grid, WsLarge::NT, 0, s>>>(q);
+        else bwd_joint_kernel<float, JointDxTile, WsWideHalf, true><<<grid, WsLarge::NT, 0, s>>>(q);
     } else {
         if (grad_dtype == MTS_GEMM_DTYPE) bwd_joint_kernel<bf16_t, JointDxTile, WsWideHalf><<<grid, WsLarge::NT, 0, s>>>(q);
         else bwd_joint_kernel<float, JointDxTile, WsWideHalf><<<grid, WsLarge::NT, 0, s>>>(q);
