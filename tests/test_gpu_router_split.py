@@ -79,3 +79,66 @@ def test_router_split_of_values_that_do_not_split(T, H, E, where, value):
         assert bool(((got.double() - want).abs() <= bound)[finite].all()), name
         assert torch.equal(got.isnan(), want.isnan()), name
         assert bool((got.double() == want)[want.isinf()].all()) and bool((got.isinf() | (got.abs() > 3e38))[over].all()), name
+
+
+def _confident(T, E, std, g):
+    """dlogits as a router leaves them whose logits have this spread: p * (something of its own)"""
+    p = torch.softmax(torch.randn(T, E, generator=g).cuda() * std, dim=-1)
+    return (p * torch.randn(T, E, generator=g).cuda() * 1e-4).contiguous()
+
+
+@pytest.mark.parametrize("std", [5, 12, 40])
+@pytest.mark.parametrize("T,H,E", [(1024, 264, 64), (1041, 72, 24), (2050, 136, 128), (1300, 520, 32)])
+def test_router_split_of_confident_routers(T, H, E, std):
+    """dlogits over the whole range of fp32, down to zeros.  Beside the bound of the sums: up to 2^10 roundings to a multiple of the
+    smallest number, 2^-149, in dw."""
+    print(f"router split T={T} H={H} E={E} std={std}", flush=True)
+    lib = _lib.load()
+    g = torch.Generator().manual_seed(T + std)
+    x, w, dl = torch.randn(T, H, generator=g).bfloat16().cuda(), (torch.randn(E, H, generator=g) * 0.05).cuda(), _confident(T, E, std, g)
+    dl[:, 3] *= 2.0 ** -90   # an expert that hardly any token hears of
+    dx, dw = _backward(lib, dl, x, w)
+    _check(dx, dl, w, 2.0 ** -8)
+    want, sizes = dl.double().T @ x.double(), dl.double().abs().T @ x.double().abs()
+    assert bool(((dw.double() - want).abs() <= 2.0 ** -20 * sizes + 2.0 ** -139).all())
+
+
+@pytest.mark.parametrize("where,border", [("x", 2.0 ** 50), ("w", 2.0 ** 26), ("dl", 4.0)])
+@pytest.mark.parametrize("below", [True, False])
+def test_router_split_up_to_the_largest_values_that_it_takes(where, border, below):
+    """Operands that are as large as the split takes them throughout, and one value beyond."""
+    lib = _lib.load()
+    g = torch.Generator().manual_seed(11)
+    T, H, E = 1041, 136, 64
+    t = dict(x=torch.rand(T, H, generator=g) - 0.5, w=torch.rand(E, H, generator=g) - 0.5, dl=torch.rand(T, E, generator=g) - 0.5)
+    t[where] *= 2 * border * (1 - 2.0 ** -8)
+    if not below:
+        t[where][t[where].shape[0] // 2, 5] = border
+    x, w, dl = t["x"].bfloat16().cuda(), t["w"].cuda(), t["dl"].cuda()
+    dx, dw = _backward(lib, dl, x, w)
+    _check(dx, dl, w, 2.0 ** -8)
+    _check(dw, dl.T, x)
+
+
+@pytest.mark.parametrize("T,H,E", [(8192, 1024, 64), (16384, 2048, 128)])
+def test_router_split_is_as_fast_for_confident_routers(T, H, E):
+    """The split takes values of all sizes below its border: the same work for any dlogits, and a quarter of its time for noise."""
+    lib = _lib.load()
+    g = torch.Generator().manual_seed(3)
+    x, w = torch.randn(T, H, generator=g).bfloat16().cuda(), (torch.randn(E, H, generator=g) * 0.05).cuda()
+
+    def time_of(dl):
+        times = []
+        for _ in range(7):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            for _ in range(10):
+                _backward(lib, dl, x, w)
+            end.record()
+            torch.cuda.synchronize()
+            times.append(start.elapsed_time(end))
+        return min(times)
+
+    ordinary, tiny = _confident(T, E, 1, g), _confident(T, E, 12, g)
+    time_of(ordinary)
+    assert time_of(tiny) <= 1.25 * time_of(ordinary)
