@@ -346,8 +346,11 @@ int mts_moe_fwd_gateup_down(const void* x, const void* w1, const void* w2, const
  * mts_moe_fwd_gateup_swiglu and mts_moe_fwd_down; any number of rows is correct.           */
 int mts_moe_fwd_few_rows_supported(int act_dtype, int weight_dtype, int64_t T, int64_t TK, int E,
                                    int H, int I);
+/* Whether that is ahead of the tiles, in front of which MTS_F32 weights are rounded in a launch of their own (_preferred) or
+ * beside the head (_preferred_to_ride, where mts_moe_head_casts_ride).                       */
 int mts_moe_fwd_few_rows_preferred(int act_dtype, int weight_dtype, int64_t T, int64_t TK, int E,
                                    int H, int I);
+int mts_moe_fwd_few_rows_preferred_to_ride(int act_dtype, int64_t T, int64_t TK, int E, int H, int I);
 int mts_moe_fwd_few_rows(const void* x, const void* w1, const void* w2, int weight_dtype,
                          const int32_t* x_gather, const int32_t* expert_start,
                          const void* weights, const int32_t* s_scatter, int64_t T, int K, int E,

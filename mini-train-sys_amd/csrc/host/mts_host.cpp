@@ -335,22 +335,25 @@ struct Saved {
     Saved() = default;
 };
 
-// with few rows the kernels read the weights once and round fp32 ones themselves; a backward pass wants the rounded copies
-bool reads_masters(const Tensor& x, const Tensor& w1, const Tensor& w2, int64_t TK, const Options& opt) {
-    return w1.scalar_type() == at::kFloat && w2.scalar_type() == at::kFloat && x.scalar_type() != at::kFloat && opt.on(NO_BACKWARD) &&
-           mts_moe_fwd_few_rows_preferred(dtype_code(x), MTS_F32, x.size(0), TK, w1.size(0), x.size(1), w1.size(1) / 2);
+bool masters(const Tensor& x, const Tensor& w1, const Tensor& w2) {
+    return w1.scalar_type() == at::kFloat && w2.scalar_type() == at::kFloat && x.scalar_type() != at::kFloat;
 }
-// fp32 master weights are rounded together (the backward pass reuses the copies)
-bool copies_masters(const Tensor& x, const Tensor& w1, const Tensor& w2, int64_t TK, const Options& opt) {
-    return w1.scalar_type() == at::kFloat && w2.scalar_type() == at::kFloat && x.scalar_type() != at::kFloat && w1.numel() % 8 == 0 && w2.numel() % 8 == 0 &&
-           !reads_masters(x, w1, w2, TK, opt);
+// With few rows the kernels read the weights once and round fp32 ones themselves; a backward pass wants the rounded copies.  `ride`: these would be made
+// beside the head.
+bool reads_masters(const Tensor& x, const Tensor& w1, const Tensor& w2, int64_t TK, const Options& opt, bool ride = false) {
+    if (!masters(x, w1, w2) || !opt.on(NO_BACKWARD)) return false;
+    const int act = dtype_code(x);
+    const int64_t T = x.size(0), E = w1.size(0), H = x.size(1), I = w1.size(1) / 2;
+    return ride ? mts_moe_fwd_few_rows_preferred_to_ride(act, T, TK, E, H, I) : mts_moe_fwd_few_rows_preferred(act, MTS_F32, T, TK, E, H, I);
 }
+// fp32 master weights that can be rounded together (the backward pass reuses the copies)
+bool copies_masters(const Tensor& x, const Tensor& w1, const Tensor& w2) { return masters(x, w1, w2) && w1.numel() % 8 == 0 && w2.numel() % 8 == 0; }
 
 // The expert weights as the forward kernels read them: as they are, or copies in the activation dtype.
 std::pair<Tensor, Tensor> forward_weights(const Tensor& x, const Tensor& w1, const Tensor& w2, int64_t TK, const Options& opt) {
     if (reads_masters(x, w1, w2, TK, opt)) return {w1, w2};
     void* stream = stream_of(x);
-    if (!copies_masters(x, w1, w2, TK, opt)) return {stage(w1, false, x.scalar_type(), stream), stage(w2, false, x.scalar_type(), stream)};
+    if (!copies_masters(x, w1, w2)) return {stage(w1, false, x.scalar_type(), stream), stage(w2, false, x.scalar_type(), stream)};
     Tensor copy1 = at::empty(w1.sizes(), x.options()), copy2 = at::empty(w2.sizes(), x.options());
     check(mts_moe_cast_weights_pair(ptr_as<float>(w1), ptr(copy1), w1.numel(), ptr_as<float>(w2), ptr(copy2), w2.numel(), dtype_code(x), stream),
           "mts_moe_cast_weights_pair");
@@ -377,8 +380,8 @@ Tensor experts_forward(const Tensor& x, const Tensor& w1_in, const Tensor& w2_in
     const int act = dtype_code(dtype);
     void* stream = stream_of(x);
     const bool weighted = opt.on(WEIGHTED_POST);
-    const bool few = reads_masters(x, w1_in, w2_in, TK, opt) || mts_moe_fwd_few_rows_preferred(act, act, T, TK, E, H, I);
     if (!w1.defined()) std::tie(w1, w2) = forward_weights(x, w1_in, w2_in, TK, opt);
+    const bool few = (dtype != at::kFloat && dtype_code(w1) == MTS_F32) || mts_moe_fwd_few_rows_preferred(act, act, T, TK, E, H, I);
     // The routing weight is applied where the activation is formed: post_act = s * silu(g) * u.  The down projection then
     // yields s * y, the combine is a plain sum, and post_act is at the same time the operand of the dW2 GEMM, so it is kept
     // for the backward pass instead of being written again there.
@@ -731,7 +734,8 @@ LayerForward layer_forward(const Tensor& x_, const Tensor& w_r_, const Tensor& w
     Tensor copy1, copy2;   // of master weights: made beside the head
     if (chained) {
         MtsCast casts[2];
-        const bool copied = copies_masters(x, w1, w2, TK, opt);
+        const bool ride = copies_masters(x, w1, w2) && mts_moe_head_casts_ride(T, H, E, dtype_code(x), w1.numel(), w2.numel());
+        const bool copied = copies_masters(x, w1, w2) && !reads_masters(x, w1, w2, TK, opt, ride);
         if (copied) {
             copy1 = at::empty(w1.sizes(), x.options()), copy2 = at::empty(w2.sizes(), x.options());
             casts[0] = {ptr_as<float>(w1), ptr(copy1), w1.numel()}, casts[1] = {ptr_as<float>(w2), ptr(copy2), w2.numel()};

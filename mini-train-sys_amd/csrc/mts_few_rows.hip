@@ -186,26 +186,31 @@ extern "C" int mts_moe_fwd_few_rows_supported(int act_dtype, int weight_dtype, i
     return ((wide + kCols - 1) / kCols + 7) / 8 * 8 * (TK / 16 + E) * kThreads < (1LL << 32);
 }
 
-// Against the tiles (a forward pass of the layer, us; here / there).  They lose to it where they are few: gate/up makes one
-// for every expert and 256 of its 2I columns, and the chip has 256 CUs.  768/1024, 8 experts (64 of them): 4 rows an expert
-// 34 / 36, 32 rows 47 / 42; 512/1024 24 rows 38 / 38, 64 rows 47 / 40; 512/2048 24 rows 43 / 46, 32 rows 49 / 46.  With more than 64 tokens the routing is
-// a second launch for both, which costs this path 6 and the tiles 3; there 768/1024 and 1024/1024 are behind from 12 rows on (12 rows 40 / 41 and 46 / 45,
-// 24 rows 44 / 41 and 49 / 44).
-// fp32 weights need no rounded copies in front.  With up to 64 tokens these are a launch of their own: 768/1024, 8 experts: 16 rows an expert 46 / 52, 32 rows
-// 53 / 54.  With more they are made beside the head and the routing, and what counts is how much there is to read and how many columns share it: 512/512
-// (6 M weights) 24 rows 33 / 36, 64 rows 37 / 37; 1024/512 (13 M) 24 rows 44 / 44, 64 rows 50 / 45; 768/1024 (19 M) 12 rows 48 / 43, 64 rows 65 / 44; 1024/1024
-// (25 M) 24 rows 58 / 50, 64 rows 71 / 51; 512/2048 (25 M) 24 rows 47 / 53, 64 rows 72 / 54; 1024/2048 (50 M) 48 rows 84 / 87, 64 rows 110 / 87; 16 experts of
-// 768/1024 (38 M) 8 rows 58 / 62, 12 rows 68 / 63; 64 of 1024/512 (100 M) 32 rows 149 / 168; 32 of 2048/768 (151 M) 64 rows 255 / 260.
+// Against the tiles, in us.  What this path does more, for 2^20 weights: every 16 rows of an expert behind the first 16 (half of them, on average) read the
+// activations again for every 32 columns, 0.2; and more blocks start, 0.025.  What it does less: the tiles' down projection is one chain over I where four
+// waves share it here, 1 for 256 of I; and a routing of up to 64 tokens is one launch, behind which this path has the shorter start, 1.  With fp32 weights the
+// tiles want rounded copies as well: a launch in front, 6, and the time that more than 27 M weights take at the rate of memory, 1 a M.  Beside the head they
+// are made while it runs: its launches cover 6 of that with up to 16 experts, 20 with more.
+// Placed on 140 shapes and tried on 60 others (512 to 2048 by 256 to 2048, 3 to 128 experts, 3 to 200 M weights, 2 to 80 rows an expert, the operator and the
+// layer, weights not in the caches): on those the call is behind the better path by 0.2 % (fp32), 0.4 % (16 bits, layer) and 1.0 % (operator) on average; furthest
+// with 80 experts and 2 rows, of whom many have none (776/640, 16 bits 72 / 95).  Here / there:
+// operator, fp32, 768/1024, 8 experts, 16 rows 40 / 45, 32 rows 45 / 45, 64 rows 59 / 46; 128 experts of 768/256, 8 rows 86 / 135, 32 rows 130 / 138, 64 rows
+// 176 / 148; layer, fp32, 64 experts of 1024/512 32 rows 153 / 168, 64 rows 192 / 170; 8 of 768/1024, 16 rows 49 / 57 (64 tokens), 32 rows 59 / 51; 32 of 768/256
+// 8 rows 54 / 53, 16 rows 62 / 54; 16 bits, 8 of 768/1024 16 rows 39 / 42, 32 rows 48 / 44; 512/2048 32 rows 51 / 51, 64 rows 67 / 52.
+enum { MASTERS_NONE, MASTERS_COPIED_IN_FRONT, MASTERS_COPIED_BESIDE_HEAD };
+static int few_rows_ahead(int masters, int64_t T, int64_t TK, int E, int H, int I) {
+    const double weights = 3.0 * E * H * I / (1 << 20), rows = (double)TK / E, again = rows > 8 ? rows / 16 - 0.5 : 0.0;
+    double there = I / 256.0 + (T <= 64 ? 1.0 : 0.0);
+    if (masters != MASTERS_NONE) there += weights > 33.0 ? weights - 27.0 : 6.0;
+    if (masters == MASTERS_COPIED_BESIDE_HEAD) there -= E <= 16 ? 6.0 : 20.0;
+    return rows <= 64.0 && weights * (0.2 * again + 0.025) <= there;   // more rows: not measured
+}
 extern "C" int mts_moe_fwd_few_rows_preferred(int act_dtype, int weight_dtype, int64_t T, int64_t TK, int E, int H, int I) {
-    if (!mts_moe_fwd_few_rows_supported(act_dtype, weight_dtype, T, TK, E, H, I)) return 0;
-    const int64_t weights = 3LL * E * H * I;
-    const bool one_launch = T <= 64, broad = I >= 2 * H, light = weights <= 14LL << 20;
-    if (weight_dtype == MTS_F32) {
-        const int rows = one_launch || weights >= 90LL << 20 ? 64 : broad && weights >= 45LL << 20 ? 48 : broad || light ? 24 : 8;
-        return TK <= (int64_t)rows * E;
-    }
-    const int64_t large = E * ((2LL * I + 255) / 256), most = one_launch || broad || light ? 48 : 12, rows = 2048 / large;
-    return TK <= (rows < 8 ? 8 : (rows > most ? most : rows)) * E;
+    return mts_moe_fwd_few_rows_supported(act_dtype, weight_dtype, T, TK, E, H, I) &&
+           few_rows_ahead(weight_dtype == MTS_F32 ? MASTERS_COPIED_IN_FRONT : MASTERS_NONE, T, TK, E, H, I);
+}
+extern "C" int mts_moe_fwd_few_rows_preferred_to_ride(int act_dtype, int64_t T, int64_t TK, int E, int H, int I) {
+    return mts_moe_fwd_few_rows_supported(act_dtype, MTS_F32, T, TK, E, H, I) && few_rows_ahead(MASTERS_COPIED_BESIDE_HEAD, T, TK, E, H, I);
 }
 
 extern "C" int mts_moe_fwd_few_rows(const void* x, const void* w1, const void* w2, int weight_dtype, const int32_t* x_gather, const int32_t* expert_start,

@@ -60,6 +60,7 @@ SIGNATURES = {
     "mts_moe_fwd_gateup_down": (_i, [_p] * 7 + [_l, _i, _i, _i, _i, _i, _p, _p, _p, _p, _l, _p]),
     "mts_moe_fwd_few_rows_supported": (_i, [_i, _i, _l, _l, _i, _i, _i]),
     "mts_moe_fwd_few_rows_preferred": (_i, [_i, _i, _l, _l, _i, _i, _i]),
+    "mts_moe_fwd_few_rows_preferred_to_ride": (_i, [_i, _l, _l, _i, _i, _i]),
     "mts_moe_fwd_few_rows": (_i, [_p, _p, _p, _i, _p, _p, _p, _p, _l, _i, _i, _i, _i, _i, _p, _p, _p, _p]),
     "mts_moe_few_tokens_supported": (_i, [_i, _i, _l, _i, _i, _i, _i]),
     "mts_moe_few_tokens_preferred": (_i, [_i, _i, _l, _i, _i, _i, _i]),

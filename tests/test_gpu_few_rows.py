@@ -9,6 +9,7 @@ import torch
 from minitrain_amd import _lib
 from minitrain_amd.kernels.hip.fused_moe import routing_for_experts
 from minitrain_amd.kernels.hip.moe_layer import moe_layer
+from minitrain_amd.model.ops import get_ops_backend
 
 pytestmark = pytest.mark.gpu
 
@@ -104,3 +105,29 @@ def test_either_side_of_the_rule(T, K, E, H, I, dtype):
     with torch.no_grad():
         got, want = (moe_layer(x, w_r, a, b, K, normalize=True)[0] for a, b in ((w1, w2), (w1.to(dtype), w2.to(dtype))))
     _close(got, want.double(), 4 * ULP[dtype], "out")
+
+
+@pytest.mark.parametrize("call", ["operator", "layer"])
+def test_masters_of_many_experts_are_not_copied(call):
+    """Without a backward pass: no rounded copies of 75 M weights for 9 rows an expert, where they would be a launch of their own (the operator, and a layer of
+    more experts than the head's launches carry copies for)."""
+    T, K, E, H, I = 300, 4, 128, 768, 256
+    g = torch.Generator(device="cuda").manual_seed(1)
+    x = torch.randn(T, H, generator=g, device="cuda").bfloat16()
+    w1, w2 = torch.randn(E, 2 * I, H, generator=g, device="cuda") * H ** -0.5, torch.randn(E, H, I, generator=g, device="cuda") * I ** -0.5
+    w_r = torch.randn(E, H, generator=g, device="cuda")
+    ops = get_ops_backend("hip")
+
+    def run(a, b):
+        if call == "layer":
+            return moe_layer(x, w_r, a, b, K, normalize=True)[0]
+        route = ops.router_postprocess(x.float() @ w_r.T, K, normalize=True)
+        return ops.fused_moe(x, a, b, route.expert_indices, route.expert_weights.bfloat16())
+
+    with torch.no_grad():
+        want = run(w1.bfloat16(), w2.bfloat16())
+        before = torch.cuda.memory_allocated()
+        torch.cuda.reset_peak_memory_stats()
+        got = run(w1, w2)
+    assert torch.cuda.max_memory_allocated() - before < w1.numel()   # the copies: three bytes for each of these
+    _close(got, want.double(), 4 * ULP[torch.bfloat16], "out")
