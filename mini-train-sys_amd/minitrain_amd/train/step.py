@@ -10,7 +10,7 @@ import torch
 
 from minitrain_amd.kernels.hip.dense import loss_is_root
 from minitrain_amd.train.modules import plain_modules, set_training
-from minitrain_amd.train.update import Update, plan
+from minitrain_amd.train.update import plan
 
 
 def build_optimizer(model: torch.nn.Module, *, lr: float = 3e-4, weight_decay: float = 0.1, betas=(0.9, 0.95),
@@ -56,10 +56,7 @@ def train_step(model: torch.nn.Module, optimizer: torch.optim.Optimizer, batch: 
         update.apply(norm, skip_if_not_finite=check_finite)
         if check_finite:
             copied.synchronize()
-        if isinstance(update, Update):
-            update.drop_gradients()
-        else:
-            optimizer.zero_grad(set_to_none=True)
+        update.drop_gradients()
         if check_finite and float(flag) != 0:
             raise FloatingPointError("non-finite training loss or global gradient norm")
         return loss.detach()

@@ -45,6 +45,9 @@ def test_event_is_recorded_where_the_flag_is_copied(monkeypatch, value):
         def apply(self, norm, skip_if_not_finite):
             calls.append("apply")
 
+        def drop_gradients(self):
+            calls.append("drop")
+
     model = _Model(2, 1)
     optimizer = torch.optim.SGD(model.parameters(), lr=0.0)
     batch = {"input_ids": torch.ones(1, 2), "targets": torch.ones(1)}
@@ -57,4 +60,4 @@ def test_event_is_recorded_where_the_flag_is_copied(monkeypatch, value):
             step.train_step(model, optimizer, batch)
     else:
         step.train_step(model, optimizer, batch)
-    assert calls == [("record", ("stream of", _Flag.device)), "apply", "synchronize"]
+    assert calls == [("record", ("stream of", _Flag.device)), "apply", "synchronize", "drop"]
