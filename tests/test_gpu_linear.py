@@ -6,6 +6,7 @@ of the largest value for the lengths here.  The other results carry one 16-bit r
 import pytest
 import torch
 
+from minitrain_amd import _lib
 from minitrain_amd.kernels.hip import dense
 from tests.helpers import hip_backend
 
@@ -33,6 +34,22 @@ def test_linear(T, N, K, dtype):
         err, scale = float((got.double() - want).abs().max()), float(want.abs().max())
         assert err <= tol * scale, (what, err, scale)
     assert w.grad.dtype == torch.float32
+
+
+@pytest.mark.parametrize("T", [128, 129, 255, 256, 257, 511, 513, 1023])
+@pytest.mark.parametrize("N,K", [(264, 248), (768, 768), (2304, 768)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_linear_of_few_rows(T, N, K, dtype):
+    """One segment, whose tiles are the result, and two; products of either kind beside it."""
+    test_linear(T, N, K, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_linear_of_fewer_rows_is_the_callers(dtype):
+    x, w = torch.randn(127, 768, device="cuda", dtype=dtype, requires_grad=True), torch.randn(768, 768, device="cuda", requires_grad=True)
+    assert not _lib.load().mts_linear_dw_supported(_lib.dtype_code(dtype), 127, 768, 768)
+    with torch.autocast("cuda", dtype=dtype):
+        assert hip_backend().linear(x, w) is None
 
 
 @pytest.mark.parametrize("T,N,K,pad", [(128, 64, 8, 0), (131, 67, 8, 5), (300, 1003, 120, 21), (1025, 2112, 264, 0), (520, 9001, 1000, 7), (66000, 67, 8, 61), (66000, 64, 8, 8),
