@@ -8,6 +8,8 @@ import torch
 
 from minitrain_amd import _lib
 from oracle import moe_oracle as O
+from tests.helpers import BF16_TOL, assert_close_scaled, hip_backend
+from tests.test_gpu_layer_node import _layer_grads
 
 pytestmark = pytest.mark.gpu
 
@@ -97,3 +99,61 @@ def test_few_tokens_of_ties_and_of_no_number():
     assert len(set(o["indices"][7].tolist())) == K and bool(o["out"][7].isnan().all())
     others = [t for t in range(T) if t != 7]
     assert torch.equal(o["out"][others], clean["out"][others]) and torch.equal(o["indices"][others], clean["indices"][others])
+
+
+@pytest.mark.parametrize("T,K,E,H,I", [(2, 2, 8, 768, 1024), (5, 1, 4, 64, 40), (16, 2, 8, 256, 128), (17, 2, 8, 776, 264), (31, 4, 8, 128, 512), (32, 2, 16, 512, 256)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("masters", [False, True])
+def test_layer_of_few_tokens_and_its_gradients(T, K, E, H, I, dtype, masters):
+    """The layer node, which takes the two launches, against the oracle in fp32 on the same rounded values."""
+    print(f"layer of few tokens T={T} K={K} E={E} H={H} I={I} {dtype} masters={masters}", flush=True)
+    act = _lib.dtype_code(dtype)
+    assert _lib.load().mts_moe_few_tokens_preferred(act, act, T, K, E, H, I)   # a backward pass follows: the weights are rounded first
+    x, w_r, w1, w2, g = O.make_inputs(70 + T, T, H, E, I)
+    res, grads = _layer_grads(hip_backend(), dict(x=x, w_r=w_r, w1=w1, w2=w2, g=g), K, True, dtype, masters)
+    kept = torch.float32 if masters else dtype
+    leaves = [x.to(dtype).float().requires_grad_(True), w_r.clone().requires_grad_(True), w1.to(kept).float().requires_grad_(True), w2.to(kept).float().requires_grad_(True)]
+    hidden, r = O.moe_feed_forward(leaves[0].to(dtype), leaves[1], leaves[2].to(kept), leaves[3].to(kept), K, normalize=True, compute_dtype=torch.float32)
+    ((hidden * g.to(dtype).float()).sum() + 0.01 * r.auxiliary_loss + 0.001 * r.z_loss).backward()
+    assert torch.equal(res[7].cpu(), r.expert_indices)
+    assert_close_scaled(res[0], hidden, BF16_TOL, "hidden")
+    torch.testing.assert_close(res[1].cpu(), r.auxiliary_loss, rtol=1e-4, atol=1e-6)
+    torch.testing.assert_close(res[2].cpu(), r.z_loss, rtol=1e-4, atol=1e-6)
+    for name, got, leaf in zip(("dx", "dW_r", "dW1", "dW2"), grads, leaves):
+        assert_close_scaled(got, leaf.grad, BF16_TOL, name)
+
+
+@pytest.mark.parametrize("T,masters", [(1, False), (16, False), (32, True)])
+def test_few_tokens_in_a_graph_and_on_two_streams(T, masters):
+    """Replays of a graph with other tokens and eager calls between them, and calls on two streams at a time, each with its own tokens: the counters of
+    the second launch are a call's own and cleared by its first, so all give what calls one after the other give."""
+    print(f"few tokens in a graph and on two streams T={T} masters={masters}", flush=True)
+    ops, K, E, H, I = hip_backend(), 2, 8, 768, 1024
+    _, w_r, w1, w2, _ = (t.cuda() for t in O.make_inputs(5, T, H, E, I))
+    if not masters:
+        w1, w2 = w1.bfloat16(), w2.bfloat16()
+    g = torch.Generator().manual_seed(4)
+    tokens = [torch.randn(T, H, generator=g).bfloat16().cuda() for _ in range(8)]
+    with torch.no_grad():
+        want = [ops.moe_layer(x, w_r, w1, w2, K, normalize=True)[0].clone() for x in tokens]
+        x = tokens[0].clone()
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = ops.moe_layer(x, w_r, w1, w2, K, normalize=True)[0]
+        for t, w in zip(tokens, want):
+            x.copy_(t)
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, w)
+            assert torch.equal(ops.moe_layer(t, w_r, w1, w2, K, normalize=True)[0], w)
+        streams = [torch.cuda.Stream() for _ in range(2)]
+        for s in streams:
+            s.wait_stream(torch.cuda.current_stream())
+        got = {}
+        for repeat in range(10):
+            for i, t in enumerate(tokens):
+                with torch.cuda.stream(streams[i % 2]):
+                    got[repeat, i] = ops.moe_layer(t, w_r, w1, w2, K, normalize=True)[0]
+        torch.cuda.synchronize()
+        assert all(torch.equal(o, want[i]) for (_, i), o in got.items())
