@@ -36,23 +36,25 @@ constexpr int kBwdLds = 2 * (64 * 20 + 16 * 72);   // floats: the two buffers of
 // Split as they come, values below 2^-60 had to be left to the fp32 instruction, and a softmax over logits 28 apart leaves such gradients behind a mean over
 // 8192 tokens: both gradients of 8192 x 1024, 64 experts, took 81 us for 24 at logits of standard deviation 5 and 87 at 10 (16 384 x 2048, 128: 559 and 564 for
 // 122); 24 and 124 at any now.  dW_r against fp64 there 1.55e-7 and 1.40e-7 (the fp32 instruction 1.96e-7 and 1.48e-7; 24 experts at 10: 1.81e-7 and 1.71e-7).
-constexpr float kDlScale = 0x1p48f, kWeightScale = 0x1p24f;   // of dlogits below 4 and weights below 2^26
-constexpr uint16_t kTooLarge = (uint16_t)(mts_split3::kBeyond >> 15);
+// Terms and products under 2^-126 are worth less than 2^-150 at 2^24 times their size.  Sums of fewer than 2^27 products below 2^100 stay in range: dlogits up
+// to 2^36, weights up to 2^16 and rows up to 2^40; a gradient of a sum over wide rows passes 4, and one that is scaled passes 2^16.
+constexpr float kScale = 0x1p24f;
+constexpr uint16_t kLargestDl = 2 * ((127 + 60) << 7), kLargestOther = 2 * ((127 + 40) << 7);   // 2^60 and 2^40 in the order of sizes()
 // two bf16 values without their signs, as numbers in the order of their size, infinities and NaN behind all others
 __device__ __forceinline__ mts_split3::u16x2 sizes(uint32_t pair) { return __builtin_bit_cast(mts_split3::u16x2, pair) << 1; }
 // in every lane of the wave
-__device__ __forceinline__ bool not_too_large(mts_split3::u16x2 largest) { return !__ballot(max(largest[0], largest[1]) >= kTooLarge); }
+__device__ __forceinline__ bool below(mts_split3::u16x2 largest, uint16_t bound) { return !__ballot(max(largest[0], largest[1]) >= bound); }
 
 struct Split8 {
     bf16x8 term[3];
     bool holds;   // every one of the scaled values is the sum of its terms, and sums of products stay in range, in every lane of the wave
 };
-__device__ __forceinline__ Split8 split8(const float (&value)[8], float scale) {
+__device__ __forceinline__ Split8 split8(const float (&value)[8], uint16_t bound) {
     Split8 s;
     float v[8];
     mts_split3::u16x2 largest = {};
 #pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = value[j] * scale;
+    for (int j = 0; j < 8; ++j) v[j] = value[j] * kScale;
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
         u32x4 h;
@@ -64,7 +66,7 @@ __device__ __forceinline__ Split8 split8(const float (&value)[8], float scale) {
         }
         s.term[q] = __builtin_bit_cast(bf16x8, h);
     }
-    s.holds = not_too_large(largest);
+    s.holds = below(largest, bound);
     return s;
 }
 
@@ -343,8 +345,8 @@ __device__ __forceinline__ void split_dw_block(const float* __restrict__ dl, con
             for (int i = 0; i < 4; ++i) u[i] = __builtin_amdgcn_perm(c[set][2 * i + 1][p / 2], c[set][2 * i][p / 2], p % 2 ? 0x07060302u : 0x05040100u);
             xv[p] = __builtin_bit_cast(bf16x8, u);
         }
-        const Split8 t = split8(d[set], kDlScale);
-        if (!not_too_large(largest) || !t.holds) return false;
+        const Split8 t = split8(d[set], kLargestDl);
+        if (!below(largest, kLargestOther) || !t.holds) return false;
 #pragma unroll
         for (int q = 2; q >= 0; --q)
 #pragma unroll
@@ -362,7 +364,7 @@ __device__ __forceinline__ void split_dw_block(const float* __restrict__ dl, con
         }
     }
 #pragma unroll
-    for (int p = 0; p < 4; ++p) acc[p] *= 1.f / kDlScale;
+    for (int p = 0; p < 4; ++p) acc[p] *= 1.f / kScale;
 #pragma unroll 1
     for (; s < steps; s += 4)   // from a step on that holds a value which is too large: by the fp32 instruction, whose k is lane / 32
 #pragma unroll 1
@@ -437,7 +439,7 @@ struct SplitDx {
 #pragma unroll
                 for (int j = 0; j < 8; ++j) v[i][j] = 0.f;
             }
-            const Split8 s = split8(v[i], kWeightScale);
+            const Split8 s = split8(v[i], kLargestOther);
             holds &= s.holds;
 #pragma unroll
             for (int q = 0; q < 3; ++q) *reinterpret_cast<bf16x8*>(terms + q * PLANE + c * LD + k0) = s.term[q];
@@ -456,7 +458,7 @@ struct SplitDx {
                 float v[8];
 #pragma unroll
                 for (int j = 0; j < 8; ++j) v[j] = 16 * s + lane / 32 * 8 < E ? raw[s][j / 4][j % 4] : 0.f;
-                d[s] = split8(v, kDlScale);
+                d[s] = split8(v, kLargestDl);
                 all &= d[s].holds;
             }
             fetch(r + step);
@@ -474,7 +476,7 @@ struct SplitDx {
 #pragma unroll
                         for (int t = 0; t < 6; ++t) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[kTerms[t][0]], d[s].term[kTerms[t][1]], acc, 0, 0, 0);
                     }
-                    acc *= 1.f / kDlScale / kWeightScale;
+                    acc *= 1.f / kScale / kScale;
                 } else {   // by the fp32 instruction, whose k is lane / 32
                     const float* wp = w + min(n0 + nf * 32 + cm, H - 1);
 #pragma unroll 1
