@@ -155,8 +155,7 @@ struct RowsParams {
     int64_t TK;                // rows of every output
     int n_tiles;               // column tiles per m-tile (set by the launcher, like by_n_tiles and by_group)
     Divider by_n_tiles, by_group;   // by n_tiles and by the tiles of a group
-    int flat;                  // block -> tile mapping: tiles in their order, columns fastest (one expert, no more tiles than the chip has CUs)
-    int xcd_ranges;            // else: 1 = every XCD takes a contiguous range of m-tiles
+    int xcd_ranges;            // block -> tile mapping: 1 = every XCD takes a contiguous range of m-tiles
     int n_groups;              // with xcd_ranges: the n-tiles are walked in this many groups, all m-tiles of the range per group
     int reverse;               // with xcd_ranges: the range's m-tiles are walked from the last to the first
     int tail_slots;            // with xcd_ranges: blocks an XCD runs at a time; when the tiles behind its last whole round
@@ -169,6 +168,8 @@ struct RowsParams {
     int32_t* sched_out;        // dO*W2 launch: one more block writes the schedule of the joint backward launch here (NULL: none)
     float* part;               // EPI_SPLIT: the tile's place among the partial results
     int sched_slots, sched_dx_cap, sched_least;
+    int flat;                  // without a table: tiles in their order, columns fastest (one expert, no more tiles than the chip has CUs).  Last, as in front
+                               // of the numbers of the mapping it moves these off the places from which one load takes several
 };
 
 // the schedule of the joint backward launch (defined with the weight-gradient GEMMs below)
@@ -634,18 +635,17 @@ __host__ __device__ __forceinline__ int paired_tiles(int tiles) {
 // (a weight-gradient tile of two k-tiles 12.9 -> 11.1 us); the layer of 24 576 tokens 877 -> 868 us, 4096 tokens of 4096/14336 -1.4 %.
 // mtile: the m-tile's index in expert order, -1 where the block has none; a block that has the empty half of a cut tile
 // (the tile's rows end in the other half) gets the index and the answer false.
-// ONE: there may be no table, then one expert has all rows.  A kernel of its own form, as the choice costs the others up to 1 us a launch
-// (dO*W2 of 6001 tokens of 1000/1368 89.0 -> 90.2).
+// ONE: there is no table, one expert has all rows.  Kernels of their own form, as the choice at run time costs the others up to 1 us a launch (dO*W2 of 6001
+// tokens of 1000/1368 89.0 -> 90.2, its down projection 42.9 -> 43.3).
 template <int BM, bool ONE>
 __device__ __forceinline__ bool find_rows_tile(const RowsParams& p, int b, int& e, int& row0, int& rend, int& ntile, int& parts,
                                                int& mtile) {
     mtile = -1;
     // up to 64 experts: lane l reads expert_start[l] and [l + 1] once, for the count of m-tiles and for the search
-    const bool in_regs = p.E <= MTS_WAVE;
+    const bool in_regs = ONE || p.E <= MTS_WAVE;
     const int lane = threadIdx.x % MTS_WAVE;
-    const int32_t* table = ONE && !p.expert_start ? reinterpret_cast<const int32_t*>(p.B) : p.expert_start;   // a load that no branch is in front of
-    int w0 = table[min(lane, p.E)], w1 = table[min(lane + 1, p.E)];   // equal behind the last expert
-    if (ONE && !p.expert_start) w0 = lane ? (int)p.TK : 0, w1 = (int)p.TK;
+    const int w0 = ONE ? (lane ? (int)p.TK : 0) : p.expert_start[min(lane, p.E)];   // equal to w1 behind the last expert
+    const int w1 = ONE ? (int)p.TK : p.expert_start[min(lane + 1, p.E)];
     const int wnt = (w1 - w0 + BM - 1) / BM, wincl = wave_scan(wnt);   // in_regs: the lane's m-tiles, and those up to its last one
     const int xcd = b % kXcds;
     int j = b / kXcds;
@@ -784,7 +784,7 @@ __device__ __forceinline__ bool locate_rows_tile(const RowsParams& p, int b, int
 // ---------------------------------------------------------------------------
 // rows_gemm
 // ---------------------------------------------------------------------------
-template <class T, int EPI>
+template <class T, int EPI, bool ONE = false>
 __global__ __launch_bounds__(T::NT) void rows_gemm_kernel(RowsParams p) {
     constexpr int LDS_ELEMS = T::LDS_ELEMS > EpiShape<T, EPI>::ELEMS ? T::LDS_ELEMS : EpiShape<T, EPI>::ELEMS;
     static_assert(LDS_ELEMS * 2 <= 160 * 1024, "LDS capacity");
@@ -795,7 +795,7 @@ __global__ __launch_bounds__(T::NT) void rows_gemm_kernel(RowsParams p) {
         if (schedule_block(p)) return;
     }
     int e, row0, rend, ntile;
-    if (!locate_rows_tile<T::BM, EPI == EPI_PLAIN>(p, blockIdx.x, e, row0, rend, ntile)) return;
+    if (!locate_rows_tile<T::BM, ONE>(p, blockIdx.x, e, row0, rend, ntile)) return;
     const int n0 = ntile * (SWIGLU ? T::BN / 2 : T::BN);  // first output column of this block
 
     KMajorLoader<T::BM, T::NT> la;
@@ -928,7 +928,7 @@ __device__ __forceinline__ void wait_vmcnt() {
 // BKM: B is read in the weights' stored layout [E][Kdim][N] (a row is one k) instead of the
 // transposed copy [E][N][Kdim]; its tiles land in LDS as [BKS k][BN] like the operands of the
 // weight-gradient GEMMs.
-template <class T, int EPI, bool BKM = false>
+template <class T, int EPI, bool BKM = false, bool ONE = false>
 __global__ __launch_bounds__(T::NT, T::WAVES_PER_EU) void rows_gemm_ring_kernel(RowsParams p) {
     constexpr int LDS_ELEMS = T::LDS_ELEMS > EpiShape<T, EPI>::ELEMS ? T::LDS_ELEMS : EpiShape<T, EPI>::ELEMS;
     static_assert(LDS_ELEMS * 2 <= 160 * 1024, "LDS capacity");
@@ -940,7 +940,7 @@ __global__ __launch_bounds__(T::NT, T::WAVES_PER_EU) void rows_gemm_ring_kernel(
         if (schedule_block(p)) return;
     }
     int e, row0, rend, ntile;
-    if (!locate_rows_tile<T::BM, EPI == EPI_PLAIN>(p, blockIdx.x, e, row0, rend, ntile)) return;
+    if (!locate_rows_tile<T::BM, ONE>(p, blockIdx.x, e, row0, rend, ntile)) return;
     const int n0 = ntile * (SWIGLU ? T::BN / 2 : T::BN);
     const int wave = threadIdx.x / MTS_WAVE, lane = threadIdx.x % MTS_WAVE;
     const int wm = wave / T::WAVES_N, wn = wave % T::WAVES_N;
@@ -1641,14 +1641,14 @@ __device__ __forceinline__ void rows_gemm_ws_block(const RowsParams& p, bf16_t* 
     rows_gemm_ws_run<T, EPI, BKM, TH>(p, smem, e, row0, rend, ntile, parts);
 }
 
-template <class T, int EPI, bool BKM = false, class TH = T>
+template <class T, int EPI, bool BKM = false, class TH = T, bool ONE = false>
 __global__ __launch_bounds__(T::NT, T::WAVES_PER_EU) void rows_gemm_ws_kernel(RowsParams p) {
     static_assert(ws_lds_elems<T, EPI>() * 2 <= 160 * 1024, "LDS capacity");
     __shared__ __attribute__((aligned(1024))) bf16_t smem[ws_lds_elems<T, EPI>()];
     if constexpr (epi_is_dy1(EPI)) {
         if (schedule_block(p)) return;
     }
-    rows_gemm_ws_block<T, EPI, BKM, TH, EPI == EPI_PLAIN>(p, smem, blockIdx.x);
+    rows_gemm_ws_block<T, EPI, BKM, TH, ONE>(p, smem, blockIdx.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -2803,8 +2803,8 @@ bool large_tiles_ahead(int64_t TK, int E, int Kdim, int64_t narrow, int64_t wide
 }
 
 // b_kmajor: B is [E][Kdim][N] (the weights as stored) instead of the transposed copy [E][N][Kdim];
-// only the ring and specialised kernels read it that way
-template <int EPI>
+// only the ring and specialised kernels read it that way.  ONE: p has no table of experts
+template <int EPI, bool ONE = false>
 int launch_rows_any(int kind, RowsParams p, int64_t TK, hipStream_t s, bool b_kmajor = false) {
     p.reverse = ((kind == K_DOWN && (tile_order_mask() & ORDER_DOWN)) || (kind == K_DY1 && (tile_order_mask() & ORDER_DY1)) ||
                  (kind == K_DX && (tile_order_mask() & ORDER_DX))) ? 1 : 0;
@@ -2844,16 +2844,16 @@ int launch_rows_any(int kind, RowsParams p, int64_t TK, hipStream_t s, bool b_km
     } else if (choice == 5) {
         const dim3 grid = rows_grid<WsSmall, EPI>(p, TK);
         if constexpr (EPI != EPI_SWIGLU) {
-            if (b_kmajor) rows_gemm_ws_kernel<WsSmall, EPI, true><<<grid, WsSmall::NT, 0, s>>>(p);
-            else rows_gemm_ws_kernel<WsSmall, EPI><<<grid, WsSmall::NT, 0, s>>>(p);
+            if (b_kmajor) rows_gemm_ws_kernel<WsSmall, EPI, true, WsSmall, ONE><<<grid, WsSmall::NT, 0, s>>>(p);
+            else rows_gemm_ws_kernel<WsSmall, EPI, false, WsSmall, ONE><<<grid, WsSmall::NT, 0, s>>>(p);
         } else {
             rows_gemm_ws_kernel<WsSmall, EPI><<<grid, WsSmall::NT, 0, s>>>(p);
         }
     } else if (choice == 1) {
         const dim3 grid = rows_grid<RingTwoPerCu, EPI>(p, TK);
         if constexpr (EPI != EPI_SWIGLU) {
-            if (b_kmajor) rows_gemm_ring_kernel<RingTwoPerCu, EPI, true><<<grid, RingTwoPerCu::NT, 0, s>>>(p);
-            else rows_gemm_ring_kernel<RingTwoPerCu, EPI><<<grid, RingTwoPerCu::NT, 0, s>>>(p);
+            if (b_kmajor) rows_gemm_ring_kernel<RingTwoPerCu, EPI, true, ONE><<<grid, RingTwoPerCu::NT, 0, s>>>(p);
+            else rows_gemm_ring_kernel<RingTwoPerCu, EPI, false, ONE><<<grid, RingTwoPerCu::NT, 0, s>>>(p);
         } else {
             rows_gemm_ring_kernel<RingTwoPerCu, EPI><<<grid, RingTwoPerCu::NT, 0, s>>>(p);
         }
@@ -2869,8 +2869,8 @@ int launch_rows_any(int kind, RowsParams p, int64_t TK, hipStream_t s, bool b_km
             if (!b_kmajor && tail_split_on()) p.tail_slots = kCusPerXcd;
             const dim3 grid = rows_grid<WsWide, EPI>(p, TK);
             if constexpr (EPI != EPI_SWIGLU) {
-                if (b_kmajor) rows_gemm_ws_kernel<WsWide, EPI, true, WsWideHalf><<<grid, WsWide::NT, 0, s>>>(p);
-                else rows_gemm_ws_kernel<WsDeep, EPI, false, WsDeepHalf><<<grid, WsWide::NT, 0, s>>>(p);
+                if (b_kmajor) rows_gemm_ws_kernel<WsWide, EPI, true, WsWideHalf, ONE><<<grid, WsWide::NT, 0, s>>>(p);
+                else rows_gemm_ws_kernel<WsDeep, EPI, false, WsDeepHalf, ONE><<<grid, WsWide::NT, 0, s>>>(p);
             } else {
                 // same tile, waves of 64x128: a wave's 32-row slab of g, u and a is 64 columns wide, i.e. whole 128-byte
                 // lines per row and store (with 128x64 waves it is 32 columns: gate/up +2.5 %)
@@ -2881,14 +2881,14 @@ int launch_rows_any(int kind, RowsParams p, int64_t TK, hipStream_t s, bool b_km
     } else if (choice == 2) {
         const dim3 grid = rows_grid<WsLarge, EPI>(p, TK);
         if constexpr (EPI != EPI_SWIGLU) {
-            if (b_kmajor) rows_gemm_ws_kernel<WsLarge, EPI, true><<<grid, WsLarge::NT, 0, s>>>(p);
-            else rows_gemm_ws_kernel<WsLarge, EPI><<<grid, WsLarge::NT, 0, s>>>(p);
+            if (b_kmajor) rows_gemm_ws_kernel<WsLarge, EPI, true, WsLarge, ONE><<<grid, WsLarge::NT, 0, s>>>(p);
+            else rows_gemm_ws_kernel<WsLarge, EPI, false, WsLarge, ONE><<<grid, WsLarge::NT, 0, s>>>(p);
         } else {
             rows_gemm_ws_kernel<WsLarge, EPI><<<grid, WsLarge::NT, 0, s>>>(p);
         }
     } else {
         const dim3 grid = rows_grid<StagedSmall, EPI>(p, TK);
-        rows_gemm_kernel<StagedSmall, EPI><<<grid, StagedSmall::NT, 0, s>>>(p);
+        rows_gemm_kernel<StagedSmall, EPI, ONE><<<grid, StagedSmall::NT, 0, s>>>(p);
     }
     MTS_CHECK_LAUNCH();
     return MTS_OK;
@@ -3588,7 +3588,7 @@ static int linear_rows(int kind, const void* a, int64_t lda, const void* w, int6
     p.B = (const bf16_t*)w; p.b_rows = N;
     p.N = N; p.Kdim = Kdim; p.E = 1;
     p.C = (bf16_t*)c; p.TK = T;
-    return launch_rows_any<EPI_PLAIN>(kind, p, T, (hipStream_t)stream, b_kmajor);
+    return launch_rows_any<EPI_PLAIN, true>(kind, p, T, (hipStream_t)stream, b_kmajor);
 }
 extern "C" int MTS_GEMM_ENTRY(mts_linear_fwd)(const void* x, const void* w, int64_t T, int N, int K, int act_dtype, void* y, void* stream) {
 #ifndef MTS_GEMM_F16
