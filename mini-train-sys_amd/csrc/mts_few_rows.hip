@@ -186,31 +186,32 @@ extern "C" int mts_moe_fwd_few_rows_supported(int act_dtype, int weight_dtype, i
     return ((wide + kCols - 1) / kCols + 7) / 8 * 8 * (TK / 16 + E) * kThreads < (1LL << 32);
 }
 
-// Against the tiles, in us.  What this path does more, for 2^20 weights: every 16 rows of an expert behind the first 16 (half of them, on average) read the
-// activations again for every 32 columns, 0.2; and more blocks start, 0.025.  What it does less: the tiles' down projection is one chain over I where four
-// waves share it here, 1 for 256 of I; and a routing of up to 64 tokens is one launch, behind which this path has the shorter start, 1.  With fp32 weights the
-// tiles want rounded copies as well: a launch in front, 6, and the time that more than 27 M weights take at the rate of memory, 1 a M.  Beside the head they
-// are made while it runs: its launches cover 6 of that with up to 16 experts, 20 with more.
-// Placed on 140 shapes and tried on 60 others (512 to 2048 by 256 to 2048, 3 to 128 experts, 3 to 200 M weights, 2 to 80 rows an expert, the operator and the
-// layer, weights not in the caches): on those the call is behind the better path by 0.2 % (fp32), 0.4 % (16 bits, layer) and 1.0 % (operator) on average; furthest
-// with 80 experts and 2 rows, of whom many have none (776/640, 16 bits 72 / 95).  Here / there:
-// operator, fp32, 768/1024, 8 experts, 16 rows 40 / 45, 32 rows 45 / 45, 64 rows 59 / 46; 128 experts of 768/256, 8 rows 86 / 135, 32 rows 130 / 138, 64 rows
-// 176 / 148; layer, fp32, 64 experts of 1024/512 32 rows 153 / 168, 64 rows 192 / 170; 8 of 768/1024, 16 rows 49 / 57 (64 tokens), 32 rows 59 / 51; 32 of 768/256
-// 8 rows 54 / 53, 16 rows 62 / 54; 16 bits, 8 of 768/1024 16 rows 39 / 42, 32 rows 48 / 44; 512/2048 32 rows 51 / 51, 64 rows 67 / 52.
+// Against the tiles, in us.  What this path does more: for 2^20 weights an expert's first 8 rows read the activations for every 32 columns, 0.2, and so does every further
+// 16 of them.  What it does less: the tiles' down projection is one chain over I where four waves share it here, 1 for 256 of I; and their rounds behind
+// the first, of 256 CUs with 128 columns of gate and up or 256 of the down projection each, cost 6 for 256 of k.  With fp32 weights the tiles want rounded copies as well: a
+// launch in front, 7, and the time that more than 21 M weights take at the rate of memory, 1 a M.  Beside the head they are made while it runs, which hides 9 more of them.
+// Placed on 1800 calls, each with three sets of weights in turn and with as many as the caches do not hold (512 to 2048 by 256 to 2048, 4 to 128 experts, 3 to 210 M
+// weights, 1.4 to 64 rows an expert, routes evenly spread and not, the operator and the layer): behind the better path by 0.6 % on average (copies in front 0.5 %), furthest
+// by 15 to 19 %.  On 500 calls that had no part in it 0.4 to 1.2 %, up to 30 %.  Here / there: layer, fp32, 8 experts of 768/1024 with one
+// route a token, 65 tokens 43.9 / 44.7, 80 47.5 / 44.4, 128 48.2 / 45.0; 16 of 1024/768 10 rows 60.5 / 71.9; 128 of 512/1024 9 rows 193 / 371; 64 of 768/512
+// 39 rows 121 / 124; operator, fp32, 8 of 768/768 36 rows 29 / 38; 16 of 1024/1536 50 rows 105 / 134; 16 of 512/512 57 rows 38 / 35; 16 bits, 16 of 1024/768 11 rows
+// 54 / 45 (layer), 64 of 768/1000 2 rows 73 / 84, 16 of 2048/1024 5 rows 57 / 49 (operator), 4 of 1024/1024 23 rows 35 / 37 (layer).
 enum { MASTERS_NONE, MASTERS_COPIED_IN_FRONT, MASTERS_COPIED_BESIDE_HEAD };
-static int few_rows_ahead(int masters, int64_t T, int64_t TK, int E, int H, int I) {
-    const double weights = 3.0 * E * H * I / (1 << 20), rows = (double)TK / E, again = rows > 8 ? rows / 16 - 0.5 : 0.0;
-    double there = I / 256.0 + (T <= 64 ? 1.0 : 0.0);
-    if (masters != MASTERS_NONE) there += weights > 33.0 ? weights - 27.0 : 6.0;
-    if (masters == MASTERS_COPIED_BESIDE_HEAD) there -= E <= 16 ? 6.0 : 20.0;
-    return rows <= 64.0 && weights * (0.2 * again + 0.025) <= there;   // more rows: not measured
+static int few_rows_ahead(int masters, int64_t TK, int E, int H, int I) {
+    auto beyond = [](double value, double border) { return value > border ? value - border : 0.0; };
+    const double weights = 3.0 * E * H * I / (1 << 20), rows = (double)TK / E, chain = I / 256.0;
+    double there = 0.0;
+    if (masters == MASTERS_NONE) there = 2.0 + chain + 6.0 * (beyond(E * (I / 128.0) / 256, 1.0) * H / 256 + beyond(E * (H / 256.0) / 256, 1.0) * chain);
+    if (masters == MASTERS_COPIED_IN_FRONT) there = 7.0 + chain + beyond(weights, 21.0);
+    if (masters == MASTERS_COPIED_BESIDE_HEAD) there = 0.75 + 0.75 * chain + beyond(weights, 30.0);
+    return rows <= 64.0 && weights * 0.2 * ((rows < 8.0 ? rows : 8.0) / 8 + beyond(rows, 8.0) / 16) <= there;   // more rows: not measured
 }
 extern "C" int mts_moe_fwd_few_rows_preferred(int act_dtype, int weight_dtype, int64_t T, int64_t TK, int E, int H, int I) {
     return mts_moe_fwd_few_rows_supported(act_dtype, weight_dtype, T, TK, E, H, I) &&
-           few_rows_ahead(weight_dtype == MTS_F32 ? MASTERS_COPIED_IN_FRONT : MASTERS_NONE, T, TK, E, H, I);
+           few_rows_ahead(weight_dtype == MTS_F32 ? MASTERS_COPIED_IN_FRONT : MASTERS_NONE, TK, E, H, I);
 }
 extern "C" int mts_moe_fwd_few_rows_preferred_to_ride(int act_dtype, int64_t T, int64_t TK, int E, int H, int I) {
-    return mts_moe_fwd_few_rows_supported(act_dtype, MTS_F32, T, TK, E, H, I) && few_rows_ahead(MASTERS_COPIED_BESIDE_HEAD, T, TK, E, H, I);
+    return mts_moe_fwd_few_rows_supported(act_dtype, MTS_F32, T, TK, E, H, I) && few_rows_ahead(MASTERS_COPIED_BESIDE_HEAD, TK, E, H, I);
 }
 
 extern "C" int mts_moe_fwd_few_rows(const void* x, const void* w1, const void* w2, int weight_dtype, const int32_t* x_gather, const int32_t* expert_start,

@@ -428,8 +428,7 @@ extern "C" int mts_moe_few_tokens_supported(int act_dtype, int weight_dtype, int
 // 2048/2048, 12 experts (288) 42.4 / 65.8 / 90.0 / 102 and 44.9 / 74.1 / 102 / 123; 4096/14336, 8 experts (2688) 159 / 476 / 563 / 597 and 340 / 551 / 680 / 825.
 extern "C" int mts_moe_few_tokens_preferred(int act_dtype, int weight_dtype, int64_t T, int K, int E, int H, int I) {
     constexpr int64_t kMostBytes = 192LL << 20;
-    return mts_moe_few_tokens_supported(act_dtype, weight_dtype, T, K, E, H, I) && mts_moe_fwd_few_rows_preferred(act_dtype, weight_dtype, T, T * K, E, H, I) &&
-           3LL * E * H * I * (weight_dtype == MTS_F32 ? 4 : 2) <= kMostBytes;
+    return mts_moe_few_tokens_supported(act_dtype, weight_dtype, T, K, E, H, I) && 3LL * E * H * I * (weight_dtype == MTS_F32 ? 4 : 2) <= kMostBytes;
 }
 
 extern "C" int mts_moe_few_tokens_fwd(const void* x, const float* w_r, const void* w1, const void* w2, int weight_dtype, int64_t T, int H, int E, int I, int K,
