@@ -462,11 +462,6 @@ int mts_moe_bwd_dw1(const void* d_pre_act, const void* x, const int32_t* x_gathe
  * changes which block computes a tile, not the tile: results are bit-identical with and without.
  * mts_moe_bwd_dy1 writes it as a by-product; mts_moe_bwd_schedule does in a launch of its own.
  * mts_moe_bwd_schedule_bytes(E): bytes of the table, 0 when E is beyond what it covers (32). */
-int mts_moe_bwd_joint_f32_supported(int H, int I);   /* the same for fp32 operands and gradients, w1 as stored: H and I multiples of 4 */
-int mts_moe_bwd_joint_f32(const float* d_out, const float* weighted_act, const float* d_pre_act, const float* x,
-                          const float* w1, const int32_t* x_gather, const int32_t* expert_start,
-                          const int32_t* s_reverse, const float* ds_partial, int64_t T, int K, int E, int H, int I,
-                          float* dx_expanded, float* d_w1, float* d_w2, float* d_weights, void* stream);
 int mts_moe_bwd_joint_supported(int act_dtype, int H, int I);
 int64_t mts_moe_bwd_schedule_bytes(int E);
 int mts_moe_bwd_schedule(const int32_t* expert_start, int64_t TK, int E, int32_t* schedule, void* stream);
@@ -477,6 +472,13 @@ int mts_moe_bwd_joint(const void* d_out, const void* weighted_act, const void* d
                       int act_dtype, int grad_dtype, void* dx_expanded, void* d_w1, void* d_w2,
                       void* d_weights, void* workspace1, int64_t workspace1_bytes,
                       void* workspace2, int64_t workspace2_bytes, const int32_t* schedule, void* stream);
+
+/* mts_moe_bwd_joint for fp32 operands and gradients, w1 as stored; H and I multiples of 4.      */
+int mts_moe_bwd_joint_f32_supported(int H, int I);
+int mts_moe_bwd_joint_f32(const float* d_out, const float* weighted_act, const float* d_pre_act, const float* x,
+                          const float* w1, const int32_t* x_gather, const int32_t* expert_start,
+                          const int32_t* s_reverse, const float* ds_partial, int64_t T, int K, int E, int H, int I,
+                          float* dx_expanded, float* d_w1, float* d_w2, float* d_weights, void* stream);
 
 /* mts_moe_bwd_joint with the router's backward in the same launch: what mts_moe_head_bwd computes
  * (the autograd backward of minitrain/model/moe_router.py:64-90 given the routing-weight gradient

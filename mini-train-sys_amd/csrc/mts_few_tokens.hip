@@ -1,16 +1,17 @@
 // Forward pass of the whole layer for few tokens (decoding): two launches, the second summing a token's routes.
 //
 // Such a call is a chain of latencies.  As head, gate/up, down and combine (mts_router_linear.hip, mts_few_rows.hip, mts_combine.hip) it was four launches of
-// 9.5, 10.4, 5.3 and 3.0 us (16 tokens, 8 experts of 768/1024), each of two or three trips to memory, the weights waiting for the routing; and the host
+// 9.3, 10.4, 5.4 and 3.0 us (16 tokens, 8 experts of 768/1024), each of two or three trips to memory, the weights waiting for the routing; and the host
 // spends as long on four launches.  Here
 //  * a block of the first launch belongs to an expert and 32 columns of its gate and up, whatever the routing: its weights are on their way while it works
-//    the routing out for itself (the projection of up to 32 tokens is some 50 fp32 matrix instructions a wave, its operands lie in the L2s), and they are
+//    the routing out for itself (48 fp32 matrix instructions a wave for a tile of 16 tokens at 768 columns, whose operands lie in the L2s), and they are
 //    multiplied with all tokens, 16 a tile, as a tile of fewer costs the same.  The routing says which of the products are stored, and where.  One
-//    block leaves the router's results and the routing metadata;
-//  * a block of the second launch takes 16 columns of the down projection of every expert with rows, four waves an expert, and adds a token's routes from
-//    LDS, each rounded as a row of the down projection is.
+//    block leaves the router's results and the routing metadata, and clears the counters of the second launch;
+//  * a block of the second launch takes 32 columns of the down projection of ONE expert and writes its rows of y to memory.  It then counts itself at its range of
+//    columns; the block that arrives there last, of those of the experts with rows, reads the rows again and adds the tokens' routes, each rounded as a row
+//    of the down projection is.  Rows and counter pass between the XCDs, which few_tokens_down_kernel says how they may.
 // The products are the same sums in the same order as those of mts_few_rows.hip; the logits are the fp32 instruction's in four parts.  16 tokens, 8 experts of
-// 768/1024, us of kernels: 9.2 + 11.0 + 5.0 + 3.1 in four launches, 14.5 + 7.8 in two (1.8 TB/s of weights in both); 32.8 -> 24.7 us a call.
+// 768/1024: 28.1 us of kernels in four launches, 13.9 + 7.7 in two (1.8 TB/s of weights in both); 31.6 -> 23.9 us a call.
 #include "mts_few_block.h"
 #include "mts_router_row.h"
 

@@ -12,8 +12,8 @@
 //
 // Backward of bf16 rows, from 1024 on (split_bwd_kernel): the fp32 operands as three bf16 terms each, which the bf16 instruction multiplies at 16 times the rate,
 // three products for dW_r and six for dx.  Two waves a SIMD and what they wait for bound it then, so operands go from memory into fragments without
-// LDS, except w_r's terms, which many rows share.  The launch, us: 8192 x 1024, 64 experts 26.4 -> 16.1; 8192 x 768, 24 17.6 -> 11.3; 16 384 x 2048, 128
-// 148 -> 100, 32 experts 66 -> 30.  Error against fp64: dW_r 1.6e-7 (3.0e-7), 3.6e-7 (8.1e-7) at 16 384 x 2048, 128; dx its rounding.  The forward pass so
+// LDS, except w_r's terms, which many rows share.  The launch and the sum of its partial dW_r, us: 8192 x 1024, 64 experts 35.3 -> 24.1; 8192 x 768, 24 23.7 -> 16.5;
+// 16 384 x 2048, 128 173 -> 116, 32 experts 78 -> 43.  Error against fp64: dW_r 1.6e-7 (3.0e-7), 3.6e-7 (8.1e-7) at 16 384 x 2048, 128; dx its rounding.  The forward pass so
 // split, fragments from memory: 14.6 -> 15.0 us and 83 -> 91 (32 experts 42 -> 38), as every 32 rows read and split w_r anew: not taken.  dW_r with three or four
 // steps in flight 10.3 -> 13.7 and 15.0 us alone: more code than a short kernel can fetch.
 #include "mts_cast_block.h"
