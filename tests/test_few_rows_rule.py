@@ -62,3 +62,11 @@ def test_rounded_weights_on_either_side(T, K, E, H, I, taken):
 def test_reading_them_beside_the_head_is_never_all_there_is(E, H, I):
     """what is taken in spite of copies beside the head is taken in front of a launch of them: the caller that makes no copies asks a second time"""
     assert all(_in_front(T, 2, E, H, I) for T in range(1, 40 * E, 3) if _beside(T, 2, E, H, I))
+
+
+# us, two launches / tiles, 16 bits: 29 tokens, top-4, 8 experts of 2048/1536 67 / 71; 15, top-1, 16 of 2048/1024 59 / 62; 1, top-2, 16 of 768/2048 36 / 40
+@pytest.mark.parametrize("T,K,E,H,I,weights,taken", [(29, 4, 8, 2048, 1536, BF16, True), (15, 1, 16, 2048, 1024, BF16, True), (1, 2, 16, 768, 2048, BF16, True),
+                                                     (32, 2, 8, 1024, 2048, F32, True), (32, 2, 8, 1024, 2056, F32, False), (32, 2, 12, 2048, 2048, BF16, False),
+                                                     (33, 2, 8, 768, 1024, BF16, False), (4, 2, 9, 768, 1024, F32, False)])
+def test_few_tokens_take_two_launches_up_to_a_size_of_the_weights(T, K, E, H, I, weights, taken):
+    assert bool(_lib.load().mts_moe_few_tokens_preferred(BF16, weights, T, K, E, H, I)) == taken
